@@ -57,8 +57,8 @@ def compress_weight(weight: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor, t
                                  _np_ptr(words))
     if nw < 0:
         raise ValueError("compress_weight: weight has values outside {-1, 0, 1}")
-    return (torch.from_numpy(words[:nw].copy()), torch.from_numpy(tile_off), torch.from_numpy(median),
-            torch.from_numpy(bitmap))
+    words.resize(int(nw), refcheck=False)            # in place: the worst case's tail goes back, nothing is copied
+    return torch.from_numpy(words), torch.from_numpy(tile_off), torch.from_numpy(median), torch.from_numpy(bitmap)
 
 
 def quant_weight_int8(weight: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:

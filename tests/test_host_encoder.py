@@ -25,6 +25,17 @@ def test_compress_weight_matches_oracle(coracle, shape, p0, seed):
     assert (vals.dtype, off.dtype, med.dtype, bm.dtype) == (torch.uint32, torch.int32, torch.uint16, torch.uint64)
 
 
+@pytest.mark.parametrize("shape,p0", [((64 * 35, 64 * 17), 0.4), ((64 * 67, 64 * 31), 0.7), ((64 * 33, 64 * 32), 0.0)])
+def test_compress_weight_over_several_threads(coracle, monkeypatch, shape, p0):
+    """Two to six threads with unequal shares of the tile rows (a megaweight is a thread's least): the streams join."""
+    monkeypatch.setenv("OMP_NUM_THREADS", "6")
+    w = make_ternary(*shape, p0, 11)
+    _same(T.compress_weight(torch.from_numpy(w)), coracle.encode(w))
+    w[-1, -1] = 2
+    with pytest.raises(ValueError):
+        T.compress_weight(torch.from_numpy(w))
+
+
 def test_compress_weight_row_skewed_round_trip(coracle):
     w = make_row_skewed(256, 192, 9)
     vals, off, med, bm = [t.numpy() for t in T.compress_weight(torch.from_numpy(w))]
