@@ -197,6 +197,11 @@ void ternaspmm_rmsnorm_quant(const terna_bf16* x, const terna_bf16* residual, te
                              const terna_bf16* weight, float eps, terna_bf16* y_out, int8_t* xq_out,
                              terna_bf16* s_out, int M, int K, terna_stream stream);
 
+/* quant_input alone (model.py:120-123) for activations that no norm precedes: s and xq of x bf16 [M][K] as above, with y = x.
+ * K % 8 == 0, K <= 8192; x and xq_out 16-byte aligned.  Returns 0, or -1 when the shape is not
+ * supported and nothing was enqueued.  Only enqueues. */
+int ternaspmm_quant_input(const terna_bf16* x, int8_t* xq_out, terna_bf16* s_out, int M, int K, terna_stream stream);
+
 /* Which of the reference's evaluations of SpBitLinear.quant_input (model.py:120-123) the prologue kernels above and
  * below reproduce -- its two lines leave the intermediate precision to PyTorch, and the ways of running them differ on a
  * few percent of the int8 activations (by one step):

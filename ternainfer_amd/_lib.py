@@ -78,6 +78,7 @@ PROTOTYPES = {
     "ternaspmm_repack_cache_limit": ([ctypes.c_longlong], ctypes.c_longlong),
     "ternaspmm_repack_cache_stats": ([_vp], None),
     "ternaspmm_plan_reference_call": ([_ci] * 6 + [_vp, _ci, _vp], _ci),
+    "ternaspmm_quant_input": ([_vp, _vp, _vp, _ci, _ci, _vp], _ci),
     "ternaspmm_quant_mode": ([_ci], _ci),
     "ternaspmm_fused_linear": ([_vp, _vp], _ci),
     "ternaspmm_quant_from_stats": ([_vp, _vp, _ci, _vp, ctypes.c_float, _vp, _vp, _ci, _ci, _vp], _ci),
@@ -89,6 +90,21 @@ PROTOTYPES = {
 }
 
 _lib = None
+_native = None
+
+
+def native():
+    """The native host path (csrc/py_native.cpp), bound to the library that `load` opens.  Raises if it is missing."""
+    global _native
+    if _native is None:
+        load()
+        try:
+            from . import _native as module
+        except ImportError as e:
+            raise ImportError(f"ternainfer_amd._native not found or not loadable ({e}): build it with `bash kernels/compile.sh`") from e
+        module.init(LIB_PATH)
+        _native = module
+    return _native
 
 
 def load() -> ctypes.CDLL:

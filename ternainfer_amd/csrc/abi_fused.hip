@@ -63,6 +63,22 @@ void ternaspmm_relu2_mul_rmsnorm_quant(const terna_bf16* x13, const terna_bf16* 
     if (e != hipSuccess) die("ternaspmm_relu2_mul_rmsnorm_quant", e, __LINE__);
 }
 
+int ternaspmm_quant_input(const terna_bf16* x, int8_t* xq_out, terna_bf16* s_out, int M, int K, terna_stream stream)
+{
+    const bool aligned = ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(xq_out)) & 15) == 0;
+    if (M < 1 || K < 8 || (K & 7) || K > 8 * kNormThreads * kNormMaxVecs || !aligned) return -1;
+    const int nv = (K / 8 + kNormThreads - 1) / kNormThreads;
+    const dim3 grid(M), block(kNormThreads);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const int qm = quant_mode();
+    if (nv <= 1) terna_quant_input_kernel<1><<<grid, block, 0, st>>>(x, K, xq_out, s_out, qm);
+    else if (nv <= 2) terna_quant_input_kernel<2><<<grid, block, 0, st>>>(x, K, xq_out, s_out, qm);
+    else terna_quant_input_kernel<4><<<grid, block, 0, st>>>(x, K, xq_out, s_out, qm);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) die("ternaspmm_quant_input", e, __LINE__);
+    return 0;
+}
+
 // One band per workgroup repeats the prologue in every workgroup: only where one round of workgroups covers the matrix.
 static bool bands_fit_one_round(int N) { return N / 16 <= 256; }
 

@@ -95,6 +95,36 @@ __device__ __forceinline__ u32x4 pack_bf16x8(const float f[8])
 }
 __device__ __forceinline__ float round_bf16(float v) { return bf16_bits_to_float(float_to_bf16_bits(v)); }
 
+// The last two passes: the row's maximum from the threads' own (`amax`), then the scale and the int8 values.
+template <int NV>
+__device__ __forceinline__ void quant_pass(const float (&h)[NV][8], float amax, int K, size_t row, int8_t* __restrict__ xq_out,
+                                           uint16_t* __restrict__ s_out, int quant_mode)
+{
+    __shared__ float red[kNormThreads / 64];
+    const int tid = threadIdx.x;
+    const int nvec = K >> 3;
+    amax = wave_max(amax);
+    if ((tid & 63) == 0) red[tid >> 6] = amax;
+    __syncthreads();
+    amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    uint16_t s_bits;
+    const float s = quant_scale(amax, quant_mode, &s_bits);
+    if (tid == 0) s_out[row] = s_bits;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int v = tid + i * kNormThreads;
+        if (v < nvec) {
+            uint32_t q[2] = {0u, 0u};
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const float r = quant_value(h[i][j], s, quant_mode);
+                q[j >> 2] |= (static_cast<uint32_t>(static_cast<int>(r)) & 0xffu) << (8 * (j & 3));
+            }
+            *reinterpret_cast<u32x2*>(xq_out + row * K + 8 * v) = u32x2{q[0], q[1]};
+        }
+    }
+}
+
 // The passes behind the formation of a row, for every kernel that holds one in registers (h[i][j] = element
 // 8 (tid + kNormThreads i) + j, vectors past K / 8 unused; raw_w the norm weights of the same elements): sum of squares
 // -- per thread in element order, the lanes of a wave by group_reduce, the four waves pairwise -- then the norm, the row
@@ -104,7 +134,7 @@ __device__ __forceinline__ void norm_quant_passes(float (&h)[NV][8], const u32x4
                                                   uint16_t* __restrict__ y_out, int8_t* __restrict__ xq_out,
                                                   uint16_t* __restrict__ s_out, int quant_mode)
 {
-    __shared__ float red[2][kNormThreads / 64];
+    __shared__ float red[kNormThreads / 64];
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
     const int nvec = K >> 3;
@@ -117,9 +147,9 @@ __device__ __forceinline__ void norm_quant_passes(float (&h)[NV][8], const u32x4
         }
     }
     ssq = wave_sum(ssq);
-    if (lane == 0) red[0][wave] = ssq;
+    if (lane == 0) red[wave] = ssq;
     __syncthreads();
-    const float total = (red[0][0] + red[0][1]) + (red[0][2] + red[0][3]);
+    const float total = (red[0] + red[1]) + (red[2] + red[3]);
     const float rstd = rsqrtf(total / static_cast<float>(K) + eps);
 
     float amax = 0.0f;
@@ -139,26 +169,7 @@ __device__ __forceinline__ void norm_quant_passes(float (&h)[NV][8], const u32x4
     }
     if (xq_out == nullptr) return;
 
-    amax = wave_max(amax);
-    if (lane == 0) red[1][wave] = amax;
-    __syncthreads();
-    amax = fmaxf(fmaxf(red[1][0], red[1][1]), fmaxf(red[1][2], red[1][3]));
-    uint16_t s_bits;
-    const float s = quant_scale(amax, quant_mode, &s_bits);
-    if (tid == 0) s_out[row] = s_bits;
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-        const int v = tid + i * kNormThreads;
-        if (v < nvec) {
-            uint32_t q[2] = {0u, 0u};
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float r = quant_value(h[i][j], s, quant_mode);
-                q[j >> 2] |= (static_cast<uint32_t>(static_cast<int>(r)) & 0xffu) << (8 * (j & 3));
-            }
-            *reinterpret_cast<u32x2*>(xq_out + row * K + 8 * v) = u32x2{q[0], q[1]};
-        }
-    }
+    quant_pass<NV>(h, amax, K, row, xq_out, s_out, quant_mode);
 }
 
 // GLU = false: x [M][K], optional residual [M][K] and sum_out [M][K].
@@ -223,6 +234,32 @@ __global__ __launch_bounds__(kNormThreads) void terna_norm_quant_kernel(
         }
     }
     norm_quant_passes<NV>(h, raw_w, K, eps, row, y_out, xq_out, s_out, quant_mode);
+}
+
+// quant_input of rows that no norm precedes (SpBitLinear on its own): x [M][K] -> (xq, s), one workgroup per row.
+// Bound: HBM on many rows, the launch on few.  It stands for the eleven elementwise and reduction launches of the same
+// lines in PyTorch (5000 x 6912: 350 us there, 21 us here; one row: 75 us of host time there, 2 us).
+template <int NV>
+__global__ __launch_bounds__(kNormThreads) void terna_quant_input_kernel(const uint16_t* __restrict__ x, int K, int8_t* __restrict__ xq_out,
+                                                                         uint16_t* __restrict__ s_out, int quant_mode)
+{
+    const int tid = threadIdx.x;
+    const size_t row = blockIdx.x;
+    const int nvec = K >> 3;
+    u32x4 raw[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {              // all requests first, on clamped addresses
+        const int v = tid + i * kNormThreads;
+        raw[i] = *reinterpret_cast<const u32x4*>(x + row * K + 8 * (v < nvec ? v : nvec - 1));
+    }
+    float h[NV][8], amax = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {              // (a clamped vector is one of the row's: the maximum may see it twice)
+        unpack_bf16x8(raw[i], h[i]);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(h[i][j]));
+    }
+    quant_pass<NV>(h, amax, K, row, xq_out, s_out, quant_mode);
 }
 
 }  // namespace terna

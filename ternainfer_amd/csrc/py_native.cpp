@@ -1,0 +1,469 @@
+// ternainfer_amd._native: the host path of one library call as one native function -- checks, output tensors, current
+// stream, launch(es).  In Python (ctypes) that path costs 13 - 16 us a call, several times what a decode-sized launch
+// takes on the device; here 2 - 3 us.  PyTorch stays what it is elsewhere in the package: the owner of device memory
+// and streams.  The library is the one _lib.py loads; init() binds its entry points by name.
+//
+// Every function checks shapes and element counts before anything is enqueued (the C ABI takes pointers on trust) and
+// raises ValueError; the tensors' types and devices are the caller's business where linear.py does not state otherwise.
+#include <dlfcn.h>
+
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <ATen/ops/empty.h>
+#include <c10/hip/HIPStream.h>
+
+#include <algorithm>
+#include <cstdarg>
+
+#include "../../include/ternaspmm.h"
+
+namespace {
+
+#define TERNA_ENTRY_POINTS(X)                                                                                          \
+    X(bitlinear_TernaSpMM)                                                                                             \
+    X(bitlinear_TernaSpMM_bf16)                                                                                        \
+    X(bitlinear_TernaSpMM_bf16_decode)                                                                                 \
+    X(bitlinear_TernaSpMM_bf16_prefill)                                                                                \
+    X(bitlinear_TernaSpMM_packed_ws)                                                                                   \
+    X(bitlinear_TernaSpMM_bf16_packed_ws)                                                                              \
+    X(ternaspmm_quant_input)                                                                                           \
+    X(ternaspmm_rmsnorm_quant)                                                                                         \
+    X(ternaspmm_relu2_mul_rmsnorm_quant)                                                                               \
+    X(ternaspmm_fused_linear)                                                                                          \
+    X(ternaspmm_quant_from_stats)                                                                                      \
+    X(ternaspmm_rope_kv_store)                                                                                         \
+    X(ternaspmm_prefill_attention)
+struct Library {
+#define X(name) decltype(&::name) name = nullptr;
+    TERNA_ENTRY_POINTS(X)
+#undef X
+} lib;
+
+const at::Tensor* tensor(PyObject* o) { return o == Py_None ? nullptr : &THPVariable_Unpack(o); }
+
+struct Refused : std::exception {};            // a Python error is set
+[[noreturn]] void refuse(const char* format, ...)
+{
+    va_list args;
+    va_start(args, format);
+    PyErr_FormatV(PyExc_ValueError, format, args);
+    va_end(args);
+    throw Refused();
+}
+
+long long integer(PyObject* o)
+{
+    const long long v = PyLong_AsLongLong(o);
+    if (v == -1 && PyErr_Occurred()) throw Refused();
+    return v;
+}
+int integer32(PyObject* o)
+{
+    const long long v = integer(o);
+    if (v < INT32_MIN || v > INT32_MAX) refuse("integer argument %lld out of range", v);
+    return static_cast<int>(v);
+}
+float real(PyObject* o)
+{
+    const double v = PyFloat_AsDouble(o);
+    if (v == -1.0 && PyErr_Occurred()) throw Refused();
+    return static_cast<float>(v);
+}
+
+template <typename T = void>
+T* data(const at::Tensor* t) { return t == nullptr ? nullptr : static_cast<T*>(t->data_ptr()); }
+
+void check_matrix(const char* who, const at::Tensor& x)
+{
+    if (x.dim() != 2) refuse("%s: expected a [M, K] tensor, got %d dimensions", who, static_cast<int>(x.dim()));
+    if (x.size(0) > INT32_MAX || x.size(1) > INT32_MAX) refuse("%s: tensor too large", who);
+}
+void check_numel(const char* who, const char* name, const at::Tensor* t, int64_t want)
+{
+    if (t != nullptr && t->numel() != want)
+        refuse("%s: %s has %lld elements, expected %lld", who, name, static_cast<long long>(t->numel()), static_cast<long long>(want));
+}
+void check_weight(const char* who, const at::Tensor& packed, const at::Tensor& ws, int ws_num, int64_t n, int64_t k)
+{
+    if (static_cast<int64_t>(packed.numel() * packed.element_size()) < n * k / 4 || ws.numel() < ws_num)
+        refuse("%s: packed weight or weight scales too small for this shape", who);
+}
+
+at::Tensor make(at::IntArrayRef shape, at::ScalarType type, const at::Tensor& like)
+{
+    return at::empty(shape, at::TensorOptions(type).device(like.device()));
+}
+terna_stream stream() { return c10::hip::getCurrentHIPStream().stream(); }
+
+// int8 rows and their bf16 scales in one allocation: (rows [m][k], scales [m])
+struct QuantRows {
+    at::Tensor held;
+    int8_t* q;
+    terna_bf16* s;
+};
+QuantRows make_quant_rows(int64_t m, int64_t k, const at::Tensor& like)
+{
+    QuantRows r{make({m * k + 2 * m}, at::kChar, like), nullptr, nullptr};     // k is even: the scales are aligned
+    r.q = static_cast<int8_t*>(r.held.data_ptr());
+    r.s = reinterpret_cast<terna_bf16*>(r.q + m * k);
+    return r;
+}
+
+PyObject* wrap(at::Tensor t) { return THPVariable_Wrap(std::move(t)); }
+PyObject* wrap_or_none(at::Tensor t) { return t.defined() ? wrap(std::move(t)) : Py_NewRef(Py_None); }
+template <typename... Ts>
+PyObject* pack(Ts&&... items)
+{
+    PyObject* tuple = PyTuple_New(sizeof...(items));
+    Py_ssize_t i = 0;
+    (PyTuple_SET_ITEM(tuple, i++, wrap_or_none(std::forward<Ts>(items))), ...);
+    return tuple;
+}
+
+// A module's activations as the kernels read them: bf16 rows on the current device, in one piece.  False: something the
+// native path does not take (another type, an empty batch ...), linear.py goes on.
+bool bf16_rows(const at::Tensor& x, at::Tensor* rows, int64_t* m, int64_t* k)
+{
+    if (!x.is_cuda() || x.scalar_type() != at::kBFloat16 || x.dim() < 1) return false;
+    *k = x.size(-1);
+    if (*k < 64 || x.numel() == 0 || x.device().index() != c10::hip::current_device()) return false;
+    *m = x.numel() / *k;
+    *rows = x.is_contiguous() ? x : x.contiguous();
+    return *m <= INT32_MAX && *k <= INT32_MAX;
+}
+at::Tensor make_output(const at::Tensor& x, int64_t n)
+{
+    at::DimVector shape(x.sizes());
+    shape.back() = n;
+    return make(shape, at::kBFloat16, x);
+}
+void check_format(const char* who, const at::Tensor& bitmap, int64_t n, int64_t k)
+{
+    if (bitmap.numel() * 64 != n * k)
+        refuse("%s: the weight's bitmap does not belong to a [%lld, %lld] matrix", who, static_cast<long long>(n), static_cast<long long>(k));
+}
+
+#define TERNA_FUNCTION(name, count)                                                                                    \
+    PyObject* name##_body(PyObject* const* a);                                                                         \
+    PyObject* name(PyObject*, PyObject* const* a, Py_ssize_t n)                                                        \
+    {                                                                                                                  \
+        HANDLE_TH_ERRORS                                                                                               \
+        if (n != (count)) {                                                                                            \
+            PyErr_Format(PyExc_TypeError, #name ": %d arguments expected", (count));                                   \
+            return nullptr;                                                                                            \
+        }                                                                                                              \
+        try {                                                                                                          \
+            return name##_body(a);                                                                                     \
+        } catch (const Refused&) {                                                                                     \
+            return nullptr;                                                                                            \
+        }                                                                                                              \
+        END_HANDLE_TH_ERRORS                                                                                           \
+    }                                                                                                                  \
+    PyObject* name##_body(PyObject* const* a)
+
+// (x, packed | None, bitmap, tile offsets, median offsets, signs, ws, ws_num, out_features, workspace | None): SpBitLinear -- quantise
+// the rows, then the int8 linear on the repacked weight or on the reference format.  None: x is not for this path.
+TERNA_FUNCTION(bit_linear, 10)
+{
+    const at::Tensor &x = *tensor(a[0]), &bitmap = *tensor(a[2]), &ws = *tensor(a[6]);
+    const at::Tensor *packed = tensor(a[1]), *workspace = tensor(a[9]);
+    const int ws_num = integer32(a[7]);
+    const int64_t n = integer32(a[8]);
+    at::Tensor rows;
+    int64_t m, k;
+    if (!bf16_rows(x, &rows, &m, &k) || k > 8192) Py_RETURN_NONE;
+    if (packed != nullptr) check_weight("SpBitLinear", *packed, ws, ws_num, n, k);
+    else check_format("SpBitLinear", bitmap, n, k);
+    QuantRows q = make_quant_rows(m, k, x);
+    at::Tensor out = make_output(x, n);
+    const terna_stream st = stream();
+    if (lib.ternaspmm_quant_input(data<terna_bf16>(&rows), q.q, q.s, m, k, st) != 0) Py_RETURN_NONE;
+    if (packed != nullptr)
+        lib.bitlinear_TernaSpMM_packed_ws(q.q, data(packed), data<terna_bf16>(&out), q.s, data<terna_bf16>(&ws), ws_num, m, n, k, 0,
+                                          data(workspace), workspace != nullptr ? workspace->numel() : 0, st);
+    else
+        lib.bitlinear_TernaSpMM(q.q, data<uint64_t>(&bitmap), data<int>(tensor(a[3])), data<uint16_t>(tensor(a[4])), data<uint32_t>(tensor(a[5])),
+                                data<terna_bf16>(&out), q.s, data<terna_bf16>(&ws), ws_num, m, n, k, 7, data<int32_t>(workspace), st);
+    return wrap(std::move(out));
+}
+
+// (x, bitmap, tile offsets, median offsets, signs, scale, ws_num, out_features, route 0 auto / 1 decode / 2 prefill)
+TERNA_FUNCTION(bit_linear_bf16, 9)
+{
+    const at::Tensor &x = *tensor(a[0]), &bitmap = *tensor(a[1]);
+    const int ws_num = integer32(a[6]), route = integer32(a[8]);
+    const int64_t n = integer32(a[7]);
+    at::Tensor rows;
+    int64_t m, k;
+    if (!bf16_rows(x, &rows, &m, &k)) Py_RETURN_NONE;
+    check_format("TernaInfer_linear_bf16", bitmap, n, k);
+    at::Tensor out = make_output(x, n);
+    const auto fn = route == 1 ? lib.bitlinear_TernaSpMM_bf16_decode : route == 2 ? lib.bitlinear_TernaSpMM_bf16_prefill : lib.bitlinear_TernaSpMM_bf16;
+    fn(data<terna_bf16>(&rows), data<uint64_t>(&bitmap), data<int>(tensor(a[2])), data<uint16_t>(tensor(a[3])), data<uint32_t>(tensor(a[4])),
+       data<terna_bf16>(&out), data<float>(tensor(a[5])), ws_num, m, n, k, 1, nullptr, stream());
+    return wrap(std::move(out));
+}
+
+// (x bf16 [..., K]) -> (int8 [..., K], bf16 [..., 1]), or None
+TERNA_FUNCTION(quant_input, 1)
+{
+    const at::Tensor& x = *tensor(a[0]);
+    at::Tensor rows;
+    int64_t m, k;
+    if (!bf16_rows(x, &rows, &m, &k)) Py_RETURN_NONE;
+    at::DimVector shape(x.sizes());
+    at::Tensor q = make(shape, at::kChar, x);
+    shape.back() = 1;
+    at::Tensor s = make(shape, at::kBFloat16, x);
+    if (lib.ternaspmm_quant_input(data<terna_bf16>(&rows), data<int8_t>(&q), data<terna_bf16>(&s), m, k, stream()) != 0) Py_RETURN_NONE;
+    return pack(std::move(q), std::move(s));
+}
+
+// (x int8 [M, K], s, packed, ws, ws_num, out_features, workspace | None)
+TERNA_FUNCTION(linear_packed, 7)
+{
+    const char* who = "TernaInfer_linear_packed";
+    const at::Tensor &x = *tensor(a[0]), &s = *tensor(a[1]), &packed = *tensor(a[2]), &ws = *tensor(a[3]);
+    const at::Tensor* workspace = tensor(a[6]);
+    const int ws_num = integer32(a[4]);
+    const int64_t n = integer32(a[5]);
+    check_matrix(who, x);
+    const int64_t m = x.size(0), k = x.size(1);
+    check_numel(who, "s", &s, m);
+    check_weight(who, packed, ws, ws_num, n, k);
+    const at::Tensor rows = x.contiguous(), scales = s.contiguous();
+    at::Tensor out = make({m, n}, at::kBFloat16, x);
+    lib.bitlinear_TernaSpMM_packed_ws(data<int8_t>(&rows), data(&packed), data<terna_bf16>(&out), data<terna_bf16>(&scales), data<terna_bf16>(&ws),
+                                      ws_num, m, n, k, 0, data(workspace), workspace != nullptr ? workspace->numel() : 0, stream());
+    return wrap(std::move(out));
+}
+
+// (x bf16 [M, K], packed, scale fp32, ws_num, out_features, workspace | None)
+TERNA_FUNCTION(linear_bf16_packed, 6)
+{
+    const char* who = "bf16 linear on a packed weight";
+    const at::Tensor &x = *tensor(a[0]), &packed = *tensor(a[1]), &scale = *tensor(a[2]);
+    const at::Tensor* workspace = tensor(a[5]);
+    const int ws_num = integer32(a[3]);
+    const int64_t n = integer32(a[4]);
+    check_matrix(who, x);
+    const int64_t m = x.size(0), k = x.size(1);
+    check_weight(who, packed, scale, ws_num, n, k);
+    const at::Tensor rows = x.contiguous();
+    at::Tensor out = make({m, n}, at::kBFloat16, x);
+    lib.bitlinear_TernaSpMM_bf16_packed_ws(data<terna_bf16>(&rows), data(&packed), data<terna_bf16>(&out), data<float>(&scale), ws_num, m, n, k, 0,
+                                           data(workspace), workspace != nullptr ? workspace->numel() : 0, stream());
+    return wrap(std::move(out));
+}
+
+// (x, weight, eps, residual | None, quant) -> (xq, s, h) or (y, None, h)
+TERNA_FUNCTION(rmsnorm_quant, 5)
+{
+    const char* who = "rmsnorm_quant";
+    const at::Tensor &x = *tensor(a[0]), &weight = *tensor(a[1]);
+    const at::Tensor* residual = tensor(a[3]);
+    const float eps = real(a[2]);
+    check_matrix(who, x);
+    const int64_t m = x.size(0), k = x.size(1);
+    check_numel(who, "residual", residual, m * k);
+    check_numel(who, "weight", &weight, k);
+    const at::Tensor rows = x.contiguous();
+    at::Tensor added, h = rows, q, s;
+    if (residual != nullptr) {
+        added = residual->contiguous();
+        h = make({m, k}, at::kBFloat16, x);
+    }
+    const bool quant = PyObject_IsTrue(a[4]);
+    q = make({m, k}, quant ? at::kChar : at::kBFloat16, x);
+    if (quant) s = make({m}, at::kBFloat16, x);
+    lib.ternaspmm_rmsnorm_quant(data<terna_bf16>(&rows), residual != nullptr ? data<terna_bf16>(&added) : nullptr,
+                                residual != nullptr ? data<terna_bf16>(&h) : nullptr, data<terna_bf16>(&weight), eps,
+                                quant ? nullptr : data<terna_bf16>(&q), quant ? data<int8_t>(&q) : nullptr, quant ? data<terna_bf16>(&s) : nullptr, m, k,
+                                stream());
+    return pack(std::move(q), std::move(s), residual != nullptr ? std::move(h) : x.is_contiguous() ? x : rows);
+}
+
+// (x13, weight, eps, quant) -> (xq, s) or (y, None)
+TERNA_FUNCTION(relu2_mul_rmsnorm_quant, 4)
+{
+    const char* who = "relu2_mul_rmsnorm_quant";
+    const at::Tensor &x = *tensor(a[0]), &weight = *tensor(a[1]);
+    const float eps = real(a[2]);
+    check_matrix(who, x);
+    const int64_t m = x.size(0), f = x.size(1) / 2;
+    check_numel(who, "weight", &weight, f);
+    const at::Tensor rows = x.contiguous();
+    const bool quant = PyObject_IsTrue(a[3]);
+    at::Tensor q = make({m, f}, quant ? at::kChar : at::kBFloat16, x), s;
+    if (quant) s = make({m}, at::kBFloat16, x);
+    lib.ternaspmm_relu2_mul_rmsnorm_quant(data<terna_bf16>(&rows), data<terna_bf16>(&weight), eps, quant ? nullptr : data<terna_bf16>(&q),
+                                          quant ? data<int8_t>(&q) : nullptr, quant ? data<terna_bf16>(&s) : nullptr, m, f, stream());
+    return pack(std::move(q), std::move(s));
+}
+
+void check_stats(const char* who, const at::Tensor& stats, int64_t m)
+{
+    if (stats.scalar_type() != at::kFloat || stats.dim() != 3 || stats.size(0) != m || stats.size(2) != 2 || !stats.is_contiguous())
+        refuse("%s: stats must be a contiguous fp32 [M, count, 2] tensor", who);
+}
+
+// (h, stats, norm_weight, eps) -> (xq, s)
+TERNA_FUNCTION(quant_from_stats, 4)
+{
+    const char* who = "quant_from_stats";
+    const at::Tensor &h = *tensor(a[0]), &stats = *tensor(a[1]), &weight = *tensor(a[2]);
+    const float eps = real(a[3]);
+    check_matrix(who, h);
+    const int64_t m = h.size(0), k = h.size(1);
+    check_numel(who, "norm_weight", &weight, k);
+    check_stats(who, stats, m);
+    const at::Tensor rows = h.contiguous();
+    at::Tensor q = make({m, k}, at::kChar, h), s = make({m}, at::kBFloat16, h);
+    if (lib.ternaspmm_quant_from_stats(data<terna_bf16>(&rows), data<float>(&stats), stats.size(1), data<terna_bf16>(&weight), eps, data<int8_t>(&q),
+                                       data<terna_bf16>(&s), m, k, stream()) != 0)
+        refuse("%s: unsupported shape M=%d K=%d", who, static_cast<int>(m), static_cast<int>(k));
+    return pack(std::move(q), std::move(s));
+}
+
+// (x, norm_weight | None, eps, packed, ws, ws_num, out_features, in_features, stats | None, attention splits (0: none), head_dim,
+//  quantised | None, epilogue, residual | None, next_norm_weight | None, want_raw, publish) -> the five tensors of
+// linear.fused_linear, or None where the library does not take the combination
+TERNA_FUNCTION(fused_linear, 17)
+{
+    const char* who = "fused_linear";
+    const at::Tensor &x = *tensor(a[0]), &packed = *tensor(a[3]), &ws = *tensor(a[4]);
+    const at::Tensor *weight = tensor(a[1]), *stats = tensor(a[8]), *quantised = tensor(a[11]), *residual = tensor(a[13]), *next_weight = tensor(a[14]);
+    const int64_t n = integer32(a[6]), k = integer32(a[7]);
+    ternaspmm_fused_linear_desc d{};
+    d.eps = real(a[2]);
+    d.ws_num = integer32(a[5]);
+    d.attention_splits = integer32(a[9]);
+    d.head_dim = integer32(a[10]);
+    d.epilogue = integer32(a[12]);
+    at::Tensor rows = x, scales, stream_in, out, stats_out, raw, xq, s;
+    int64_t m = 1;
+    if (d.attention_splits > 0) {
+        d.prologue = TERNASPMM_PROLOGUE_ATTENTION;
+    } else {
+        check_matrix(who, x);
+        m = x.size(0);
+        if (x.size(1) != k) refuse("%s: expected a [M, %lld] tensor", who, static_cast<long long>(k));
+        rows = x.contiguous();
+        if (quantised != nullptr) {
+            d.prologue = TERNASPMM_PROLOGUE_QUANTISED;
+            check_numel(who, "s", quantised, m);
+            if (x.scalar_type() != at::kChar || quantised->scalar_type() != at::kBFloat16)
+                refuse("%s: quantised activations are int8 with bf16 scales", who);
+            scales = quantised->contiguous();
+            d.s_in = data<terna_bf16>(&scales);
+        } else {
+            d.prologue = stats != nullptr ? TERNASPMM_PROLOGUE_STATS : TERNASPMM_PROLOGUE_NORM;
+            check_numel(who, "norm_weight", weight, k);
+        }
+    }
+    check_weight(who, packed, ws, d.ws_num, n, k);
+    d.M = m, d.N = n, d.K = k;
+    d.x = data(&rows), d.packed = data(&packed), d.ws = data<terna_bf16>(&ws), d.norm_weight = data<terna_bf16>(weight);
+    if (stats != nullptr) {
+        check_stats(who, *stats, m);
+        d.stats_in = data<float>(stats), d.stats_count = stats->size(1);
+    }
+    const int64_t columns = d.epilogue == TERNASPMM_EPILOGUE_GATE ? n / 2 : n;
+    if (d.epilogue != TERNASPMM_EPILOGUE_STORE && (next_weight == nullptr || next_weight->numel() != columns))
+        refuse("%s: a producing epilogue needs the next norm's weights", who);
+    if (d.epilogue == TERNASPMM_EPILOGUE_RESIDUAL) {
+        if (residual == nullptr || residual->numel() != m * n || residual->scalar_type() != at::kBFloat16)
+            refuse("%s: the residual epilogue needs a bf16 [M, N] stream", who);
+        stream_in = residual->contiguous();
+        d.residual = data<terna_bf16>(&stream_in);
+        if (PyObject_IsTrue(a[15])) {
+            raw = make({m, n}, at::kBFloat16, packed);
+            d.raw_out = data<terna_bf16>(&raw);
+        }
+    }
+    out = make({m, columns}, at::kBFloat16, packed);
+    d.out = data<terna_bf16>(&out);
+    if (d.epilogue != TERNASPMM_EPILOGUE_STORE) {
+        stats_out = make({m, columns / 16, 2}, at::kFloat, packed);
+        d.next_norm_weight = data<terna_bf16>(next_weight), d.stats_out = data<float>(&stats_out);
+    }
+    if (PyObject_IsTrue(a[16])) {
+        xq = make({m, k}, at::kChar, packed), s = make({m}, at::kBFloat16, packed);
+        d.xq_out = data<int8_t>(&xq), d.s_out = data<terna_bf16>(&s);
+    }
+    if (lib.ternaspmm_fused_linear(&d, stream()) < 0) Py_RETURN_NONE;
+    return pack(std::move(out), std::move(stats_out), std::move(raw), std::move(xq), std::move(s));
+}
+
+void check_cache(const char* who, const at::Tensor& k, const at::Tensor& v, int64_t kv_heads, int64_t head_dim)
+{
+    if (k.dim() != 4 || k.sizes() != v.sizes() || k.size(1) != kv_heads || k.size(3) != head_dim || !k.is_contiguous() || !v.is_contiguous())
+        refuse("%s: the caches are contiguous [B, KV, S, D] tensors of one shape", who);
+}
+// Positions of the t new tokens: [t] for all sequences, or [batch, t]; cos / sin rows of the same tokens.
+bool check_positions(const char* who, const at::Tensor& pos, int64_t batch, int64_t t)
+{
+    const bool each = pos.dim() == 2;
+    if (pos.scalar_type() != at::kLong || pos.numel() != (each ? batch * t : t) || !pos.is_contiguous())
+        refuse("%s: positions are a contiguous int64 [T] or [B, T] tensor", who);
+    return each;
+}
+
+// (qkv bf16 [B * T, (H + 2 KV) D], cos, sin, pos, cache_k, cache_v, heads, head_dim, scale, adjacent, attention): RoPE and cache write
+// of T new tokens per sequence, and with `attention` the multi-token attention -> bf16 [B * T, H D]; without it the
+// rotated q [B, H, T, D]
+TERNA_FUNCTION(prompt_attention, 11)
+{
+    const char* who = "prompt_attention";
+    const at::Tensor &qkv = *tensor(a[0]), &cos = *tensor(a[1]), &sin = *tensor(a[2]), &pos = *tensor(a[3]), &ck = *tensor(a[4]), &cv = *tensor(a[5]);
+    const int64_t h = integer32(a[6]), d = integer32(a[7]);
+    check_matrix(who, qkv);
+    if (ck.dim() != 4) refuse("%s: the caches are [B, KV, S, D] tensors", who);
+    const int64_t batch = ck.size(0), kv = ck.size(1), slots = ck.size(2), t = qkv.size(0) / std::max<int64_t>(batch, 1);
+    check_cache(who, ck, cv, kv, d);
+    if (batch < 1 || qkv.size(0) != batch * t || qkv.size(1) != (h + 2 * kv) * d || !qkv.is_contiguous())
+        refuse("%s: qkv does not have the shape of its caches", who);
+    const bool each = check_positions(who, pos, batch, t);
+    const int64_t angles = (each ? batch * t : t) * (d / 2);
+    if (cos.numel() != angles || sin.numel() != angles || cos.scalar_type() != at::kFloat || sin.scalar_type() != at::kFloat || !cos.is_contiguous() || !sin.is_contiguous())
+        refuse("%s: cos / sin are contiguous fp32 rows of D / 2, one per position", who);
+    at::Tensor q = make({batch, h, t, d}, at::kBFloat16, qkv);
+    const terna_stream st = stream();
+    lib.ternaspmm_rope_kv_store(data<terna_bf16>(&qkv), data<float>(&cos), data<float>(&sin), data<long long>(&pos), each, data<terna_bf16>(&q),
+                                data<terna_bf16>(&ck), data<terna_bf16>(&cv), batch, t, h, kv, d, slots, integer32(a[9]), st);
+    if (!PyObject_IsTrue(a[10])) return wrap(std::move(q));
+    at::Tensor o = make({batch * t, h * d}, at::kBFloat16, qkv);
+    lib.ternaspmm_prefill_attention(data<terna_bf16>(&q), data<terna_bf16>(&ck), data<terna_bf16>(&cv), data<long long>(&pos), each, data<terna_bf16>(&o),
+                                    batch, t, h, kv, d, slots, real(a[8]), st);
+    return wrap(std::move(o));
+}
+
+// (path of libternaspmm.so)
+TERNA_FUNCTION(init, 1)
+{
+    const char* path = PyUnicode_AsUTF8(a[0]);
+    if (path == nullptr) throw Refused();
+    void* handle = dlopen(path, RTLD_NOW | RTLD_LOCAL);
+    if (handle == nullptr) {
+        PyErr_SetString(PyExc_ImportError, dlerror());
+        throw Refused();
+    }
+#define X(name)                                                                                                        \
+    if ((lib.name = reinterpret_cast<decltype(&::name)>(dlsym(handle, #name))) == nullptr) {                             \
+        PyErr_SetString(PyExc_ImportError, "libternaspmm.so does not export " #name);                                  \
+        throw Refused();                                                                                               \
+    }
+    TERNA_ENTRY_POINTS(X)
+#undef X
+    Py_RETURN_NONE;
+}
+
+#define METHOD(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(name)), METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {METHOD(init), METHOD(bit_linear), METHOD(bit_linear_bf16), METHOD(quant_input), METHOD(linear_packed),
+                         METHOD(linear_bf16_packed), METHOD(rmsnorm_quant), METHOD(relu2_mul_rmsnorm_quant), METHOD(quant_from_stats),
+                         METHOD(fused_linear), METHOD(prompt_attention), {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__native() { return PyModule_Create(&module); }

@@ -1,8 +1,9 @@
 """Call site of the TernaSpMM path: the host-side mirror of the reference's ``model.py:21-153``.
 
 ``TernaInfer_linear`` / ``SpBitLinear`` / ``BF16BitLinear`` / ``get_global_workspace`` keep the
-reference's names, arguments and behaviour (row padding to ``max(8, next_pow2(M))``,
-``SPLIT_K = 7``, raw device pointers and the current stream handed to the C ABI).
+reference's names, arguments and results (``SPLIT_K = 7``, raw device pointers and the current
+stream handed to the C ABI).  The calls that run once per linear or norm of a forward pass go through
+``ternainfer_amd._native`` (csrc/py_native.cpp): checks, outputs and launches in one native function.
 ``TernaInfer_linear_bf16`` / ``SpBitLinearBF16`` are the same call site for the
 bf16-activation entry points this build adds.  PyTorch is only the owner of device memory
 and streams here; all arithmetic happens in libternaspmm.so.
@@ -39,57 +40,36 @@ def _p(t: torch.Tensor):
 
 def TernaInfer_linear(input, compressed_val, TileOffsets_global, TileOffsets_median, bitmap,
                       workspace, s, ws, ws_num, out_features):
-    """int8 activations x compressed ternary weight -> bf16 (model.py:45-92)."""
-    lib = _lib.load()
-    out_shape = list(input.shape)
-    out_shape[-1] = out_features
-    stream = torch.cuda.current_stream()
-
-    M = input.shape[0]
-    if len(out_shape) == 3:
-        M *= input.shape[1]
-    N = out_features
+    """int8 activations x compressed ternary weight -> bf16 (model.py:45-92).  The reference pads the rows to a power of two
+    of at least 8, which its kernels need; these take any row count, and the padded and the true count select the same
+    epilogue rule (<= 64 rows or more), so nothing is padded or copied here."""
     K = input.shape[-1]
-    SPLIT_K = 7
-
-    M_padded = max(8, 1 << (M - 1).bit_length())
-    pad_rows = M_padded - M
-    if pad_rows > 0:
-        input_padded = torch.cat([
-            input.reshape(M, K),
-            torch.empty((pad_rows, K), dtype=input.dtype, device=input.device)], dim=0)
-        # the reference also reads s for the padding rows; give those reads memory to land in
-        s_padded = torch.cat([s.reshape(M), torch.ones(pad_rows, dtype=s.dtype, device=s.device)])
-    else:
-        input_padded = input.reshape(M, K).contiguous()
-        s_padded = s.reshape(M).contiguous()
-
-    ret_padded = torch.empty((M_padded, N), dtype=torch.bfloat16, device=input.device)
-    lib.bitlinear_TernaSpMM(
-        _p(input_padded), _p(bitmap), _p(TileOffsets_global), _p(TileOffsets_median), _p(compressed_val),
-        _p(ret_padded), _p(s_padded), _p(ws), ws_num, M_padded, N, K, SPLIT_K, _p(workspace),
-        ctypes.c_void_p(stream.cuda_stream))
-    return ret_padded[:M, :].reshape(*out_shape)
+    x = input.reshape(-1, K).contiguous()
+    M = x.shape[0]
+    out = torch.empty((M, out_features), dtype=torch.bfloat16, device=input.device)
+    if M > 0:
+        _lib.load().bitlinear_TernaSpMM(
+            _p(x), _p(bitmap), _p(TileOffsets_global), _p(TileOffsets_median), _p(compressed_val),
+            _p(out), _p(s.reshape(M).contiguous()), _p(ws), ws_num, M, out_features, K, 7, _p(workspace),
+            ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    return out.reshape(*input.shape[:-1], out_features)
 
 
 def TernaInfer_linear_bf16(input, compressed_val, TileOffsets_global, TileOffsets_median, bitmap,
                            scale, ws_num, out_features, route: str = "auto"):
     """bf16 activations x compressed ternary weight -> bf16, fp32 accumulate, fp32 scale[ws_num].
     No row padding: the entry point takes the true M."""
-    lib = _lib.load()
-    fn = {"auto": lib.bitlinear_TernaSpMM_bf16, "decode": lib.bitlinear_TernaSpMM_bf16_decode,
-          "prefill": lib.bitlinear_TernaSpMM_bf16_prefill}[route]
-    out_shape = list(input.shape)
-    out_shape[-1] = out_features
-    K = input.shape[-1]
-    x = input.reshape(-1, K).contiguous()
-    M = x.shape[0]
-    assert x.dtype == torch.bfloat16 and scale.dtype == torch.float32
-    out = torch.empty((M, out_features), dtype=torch.bfloat16, device=input.device)
-    stream = torch.cuda.current_stream()
-    fn(_p(x), _p(bitmap), _p(TileOffsets_global), _p(TileOffsets_median), _p(compressed_val), _p(out),
-       _p(scale), ws_num, M, out_features, K, 1, None, ctypes.c_void_p(stream.cuda_stream))
-    return out.reshape(*out_shape)
+    assert input.dtype == torch.bfloat16 and scale.dtype == torch.float32
+    out = _lib.native().bit_linear_bf16(input, bitmap, TileOffsets_global, TileOffsets_median, compressed_val, scale, ws_num,
+                                        out_features, _ROUTES[route])
+    if out is None:
+        if input.numel() == 0:
+            return torch.empty((*input.shape[:-1], out_features), dtype=torch.bfloat16, device=input.device)
+        raise ValueError(f"TernaInfer_linear_bf16: unsupported input {tuple(input.shape)} on {input.device}")
+    return out
+
+
+_ROUTES = {"auto": 0, "decode": 1, "prefill": 2}
 
 
 def repack_weight(compressed_val, TileOffsets_global, TileOffsets_median, bitmap, out_features, in_features):
@@ -119,22 +99,11 @@ def _check_rows(who, x, k=None, **others):
 def TernaInfer_linear_packed(input, packed, s, ws, ws_num, out_features):
     """int8 activations x P2-layout ternary weight -> bf16; the reference's epilogue rule by M
     (decode arithmetic for M <= 64, prefill arithmetic above).  No row padding needed."""
-    lib = _lib.load()
-    out_shape = list(input.shape)
-    out_shape[-1] = out_features
     K = input.shape[-1]
-    x = input.reshape(-1, K).contiguous()
-    M = x.shape[0]
-    _check_rows("TernaInfer_linear_packed", x, s=(s, M))
-    if packed.numel() * packed.element_size() < out_features * K // 4 or ws.numel() < ws_num:
-        raise ValueError("TernaInfer_linear_packed: packed weight or weight scales too small for this shape")
-    out = torch.empty((M, out_features), dtype=torch.bfloat16, device=input.device)
-    stream = torch.cuda.current_stream()
-    work = get_global_workspace(input.device) if M > 64 else None      # large M: room for split-K partial sums
-    lib.bitlinear_TernaSpMM_packed_ws(_p(x), _p(packed), _p(out), _p(s.reshape(M).contiguous()), _p(ws), ws_num,
-                                      M, out_features, K, 0, _p(work) if work is not None else None,
-                                      work.numel() if work is not None else 0, ctypes.c_void_p(stream.cuda_stream))
-    return out.reshape(*out_shape)
+    x = input.reshape(-1, K)
+    work = get_global_workspace(input.device) if x.shape[0] > 64 else None      # large M: room for split-K partial sums
+    out = _lib.native().linear_packed(x, s, packed, ws, ws_num, out_features, work)
+    return out.reshape(*input.shape[:-1], out_features)
 
 
 def rmsnorm_quant(x, weight, eps, residual=None, quant=True):
@@ -142,27 +111,8 @@ def rmsnorm_quant(x, weight, eps, residual=None, quant=True):
     (model.py:330/334 + the norm + model.py:120-123).  x, residual: bf16 [M, K]; weight: bf16 [K].
     Returns (xq int8 [M, K], s bf16 [M], h) when quant else (y bf16 [M, K], h); h is the bf16 sum
     x + residual (x itself when residual is None)."""
-    m, k = x.shape
-    _check_rows("rmsnorm_quant", x, residual=(residual, m * k), weight=(weight, k))
-    x = x.contiguous()
-    lib = _lib.load()
-    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-    h = x
-    if residual is not None:
-        residual = residual.contiguous()
-        h = torch.empty_like(x)
-    if quant:
-        xq = torch.empty((m, k), dtype=torch.int8, device=x.device)
-        s = torch.empty(m, dtype=torch.bfloat16, device=x.device)
-        lib.ternaspmm_rmsnorm_quant(_p(x), _p(residual) if residual is not None else None,
-                                    _p(h) if residual is not None else None, _p(weight), float(eps), None, _p(xq),
-                                    _p(s), m, k, stream)
-        return xq, s, h
-    y = torch.empty_like(x)
-    lib.ternaspmm_rmsnorm_quant(_p(x), _p(residual) if residual is not None else None,
-                                _p(h) if residual is not None else None, _p(weight), float(eps), _p(y), None, None,
-                                m, k, stream)
-    return y, h
+    q, s, h = _lib.native().rmsnorm_quant(x, weight, eps, residual, quant)
+    return (q, s, h) if quant else (q, h)
 
 
 def rmsnorm_linear_packed(x, norm_weight, eps, packed, ws, ws_num, out_features, residual=None):
@@ -266,20 +216,8 @@ def relu2_mul_rmsnorm_linear_packed(x13, norm_weight, eps, packed, ws, ws_num, o
 def relu2_mul_rmsnorm_quant(x13, weight, eps, quant=True):
     """Fused squared_relu(x1) * x3 -> ffn_sub_norm -> [quant_input] (model.py:279-281 + 120-123).
     x13: bf16 [M, 2F].  Returns (xq int8 [M, F], s bf16 [M]) when quant else y bf16 [M, F]."""
-    m, f2 = x13.shape
-    f = f2 // 2
-    _check_rows("relu2_mul_rmsnorm_quant", x13, weight=(weight, f))
-    x13 = x13.contiguous()
-    lib = _lib.load()
-    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-    if quant:
-        xq = torch.empty((m, f), dtype=torch.int8, device=x13.device)
-        s = torch.empty(m, dtype=torch.bfloat16, device=x13.device)
-        lib.ternaspmm_relu2_mul_rmsnorm_quant(_p(x13), _p(weight), float(eps), None, _p(xq), _p(s), m, f, stream)
-        return xq, s
-    y = torch.empty((m, f), dtype=torch.bfloat16, device=x13.device)
-    lib.ternaspmm_relu2_mul_rmsnorm_quant(_p(x13), _p(weight), float(eps), _p(y), None, None, m, f, stream)
-    return y
+    q, s = _lib.native().relu2_mul_rmsnorm_quant(x13, weight, eps, quant)
+    return (q, s) if quant else q
 
 
 class FusedLinearDesc(ctypes.Structure):
@@ -336,16 +274,7 @@ def step_inputs(tokens, pos, embedding, rope_table, norm_weight):
 def quant_from_stats(h, stats, norm_weight, eps):
     """Norm + quant_input of h bf16 [M, K] from the partials its producer left (ternaspmm_quant_from_stats):
     (xq int8 [M, K], s bf16 [M])."""
-    m, k = h.shape
-    _check_rows("quant_from_stats", h, norm_weight=(norm_weight, k))
-    if stats.dtype != torch.float32 or stats.dim() != 3 or stats.shape[0] != m or stats.shape[2] != 2 or not stats.is_contiguous():
-        raise ValueError("quant_from_stats: stats must be a contiguous fp32 [M, count, 2] tensor")
-    xq = torch.empty((m, k), dtype=torch.int8, device=h.device)
-    s = torch.empty(m, dtype=torch.bfloat16, device=h.device)
-    if _lib.load().ternaspmm_quant_from_stats(_p(h.contiguous()), _p(stats), stats.shape[1], _p(norm_weight), float(eps), _p(xq), _p(s),
-                                             m, k, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) != 0:
-        raise ValueError(f"quant_from_stats: unsupported shape M={m} K={k}")
-    return xq, s
+    return _lib.native().quant_from_stats(h, stats, norm_weight, eps)
 
 
 def interleave_gate_up(packed, out_features, in_features):
@@ -365,62 +294,9 @@ def fused_linear(x, norm_weight, eps, packed, ws, ws_num, out_features, in_featu
     `quantised` = s (bf16 [M]), int8 activations that are quantised already (norm_weight is then not used).
     Returns (out, stats_out, raw, xq, s) -- stats_out for the producing epilogues, raw with `want_raw`, (xq, s) with
     `publish`, None otherwise -- or None when the library does not support the combination (nothing was enqueued)."""
-    lib = _lib.load()
-    k, n = in_features, out_features
-    if attention is not None:
-        m, pro = 1, PROLOGUE_ATTENTION
-    elif quantised is not None:
-        m, pro = x.shape[0], PROLOGUE_QUANTISED
-        _check_rows("fused_linear", x, k, s=(quantised, m))
-        if x.dtype != torch.int8 or quantised.dtype != torch.bfloat16:
-            raise ValueError("fused_linear: quantised activations are int8 with bf16 scales")
-        x = x.contiguous()
-    else:
-        m = x.shape[0]
-        _check_rows("fused_linear", x, k, norm_weight=(norm_weight, k))
-        x = x.contiguous()
-        pro = PROLOGUE_STATS if stats is not None else PROLOGUE_NORM
-    if packed.numel() * packed.element_size() < n * k // 4 or ws.numel() < ws_num:
-        raise ValueError("fused_linear: packed weight or weight scales too small for this shape")
-    dev = packed.device
-    out_cols = n // 2 if epilogue == EPILOGUE_GATE else n
-    d = FusedLinearDesc()
-    d.prologue, d.epilogue, d.M, d.N, d.K, d.ws_num, d.eps = pro, epilogue, m, n, k, ws_num, float(eps)
-    d.x, d.packed, d.ws = x.data_ptr(), packed.data_ptr(), ws.data_ptr()
-    d.norm_weight = norm_weight.data_ptr() if norm_weight is not None else None
-    if quantised is not None:
-        quantised = quantised.contiguous()
-        d.s_in = quantised.data_ptr()
-    if stats is not None:
-        if stats.dtype != torch.float32 or stats.dim() != 3 or stats.shape[0] != m or stats.shape[2] != 2 or not stats.is_contiguous():
-            raise ValueError("fused_linear: stats must be a contiguous fp32 [M, count, 2] tensor")
-        d.stats_in, d.stats_count = stats.data_ptr(), stats.shape[1]
-    if attention is not None:
-        d.attention_splits, d.head_dim = attention
-    out = torch.empty((m, out_cols), dtype=torch.bfloat16, device=dev)
-    d.out = out.data_ptr()
-    stats_out = raw = xq = s = None
-    if epilogue != EPILOGUE_STORE:
-        if next_norm_weight is None or next_norm_weight.numel() != out_cols:
-            raise ValueError("fused_linear: a producing epilogue needs the next norm's weights")
-        stats_out = torch.empty((m, out_cols // 16, 2), dtype=torch.float32, device=dev)
-        d.next_norm_weight, d.stats_out = next_norm_weight.data_ptr(), stats_out.data_ptr()
-    if epilogue == EPILOGUE_RESIDUAL:
-        if residual is None or residual.numel() != m * n or residual.dtype != torch.bfloat16:
-            raise ValueError("fused_linear: the residual epilogue needs a bf16 [M, N] stream")
-        residual = residual.contiguous()
-        d.residual = residual.data_ptr()
-        if want_raw:
-            raw = torch.empty((m, n), dtype=torch.bfloat16, device=dev)
-            d.raw_out = raw.data_ptr()
-    if publish:
-        xq = torch.empty((m, k), dtype=torch.int8, device=dev)
-        s = torch.empty(m, dtype=torch.bfloat16, device=dev)
-        d.xq_out, d.s_out = xq.data_ptr(), s.data_ptr()
-    rc = lib.ternaspmm_fused_linear(ctypes.byref(d), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
-    if rc < 0:
-        return None
-    return out, stats_out, raw, xq, s
+    splits, head_dim = attention if attention is not None else (0, 0)
+    return _lib.native().fused_linear(x, norm_weight, eps, packed, ws, ws_num, out_features, in_features, stats, splits, head_dim,
+                                      quantised, epilogue, residual, next_norm_weight, want_raw, publish)
 
 
 def lm_head(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -495,6 +371,10 @@ def quant_input(input: torch.Tensor, mode: Optional[int] = None):
     Returns (x_q int8, s bf16 [..., 1])."""
     if mode is None:
         mode = _lib.load().ternaspmm_quant_mode(-1)
+    if input.is_cuda and input.dtype == torch.bfloat16 and mode == _lib.load().ternaspmm_quant_mode(-1):
+        done = _lib.native().quant_input(input)   # one launch; None: rows the kernel does not take
+        if done is not None:
+            return done
     if mode == QUANT_EAGER:                       # the reference's two lines as they stand, on the bf16 tensor
         x = input.to(torch.bfloat16)
         s = 127 / x.abs().max(dim=-1, keepdim=True).values.clamp_(min=1e-5)
@@ -545,7 +425,15 @@ class SpBitLinear(_CompressedWeight):
         return quant_input(input)
 
     def forward(self, input):
-        input, s = self.quant_input(input)
+        p = self._parameters
+        packed = p.get("weight_packed")
+        work = get_global_workspace() if packed is None or input.numel() > 64 * self.in_features else None
+        out = _lib.native().bit_linear(input, packed, p["weight_bitmap"], p["weight_TileOffsets_global"],
+                                       p["weight_TileOffsets_median"], p["weight_compressed_val"], p["weight_scale"], self.ws_num,
+                                       self.out_features, work)
+        if out is not None:
+            return out
+        input, s = self.quant_input(input)        # other activation types and row lengths
         if self.weight_packed is not None:
             return TernaInfer_linear_packed(input, self.weight_packed, s, self.weight_scale,
                                             self.ws_num, self.out_features)
@@ -562,9 +450,10 @@ class SpBitLinearBF16(_CompressedWeight):
         self.scale_f32 = torch.nn.Parameter(self.weight_scale.float(), requires_grad=False)
 
     def forward(self, input):
+        p = self._parameters
         return TernaInfer_linear_bf16(
-            input, self.weight_compressed_val, self.weight_TileOffsets_global, self.weight_TileOffsets_median,
-            self.weight_bitmap, self.scale_f32, self.ws_num, self.out_features)
+            input, p["weight_compressed_val"], p["weight_TileOffsets_global"], p["weight_TileOffsets_median"],
+            p["weight_bitmap"], p["scale_f32"], self.ws_num, self.out_features)
 
 
 class BF16BitLinear(nn.Module):

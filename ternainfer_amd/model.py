@@ -76,24 +76,13 @@ class TernaryLinear:
 
     def quantised(self, xq: torch.Tensor, s: torch.Tensor) -> torch.Tensor:
         """int8 activations [M, K] + per-row scale bf16 [M] (as the fused prologue kernels write them)."""
-        m = xq.shape[0]
-        out = torch.empty((m, self.n), dtype=torch.bfloat16, device=xq.device)
-        stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-        work = get_global_workspace(xq.device) if m > 64 else None              # large M: room for split-K partial sums
-        self.lib.bitlinear_TernaSpMM_packed_ws(_p(xq), _p(self.packed), _p(out), _p(s), _p(self.ws), self.ws_num,
-                                               m, self.n, self.k, 0, _p(work), work.numel() if work is not None else 0, stream)
-        return out
+        work = get_global_workspace(xq.device) if xq.shape[0] > 64 else None     # large M: room for split-K partial sums
+        return _lib.native().linear_packed(xq, s, self.packed, self.ws, self.ws_num, self.n, work)
 
     def dense(self, x: torch.Tensor) -> torch.Tensor:
         """bf16 activations [M, K]."""
-        m = x.shape[0]
-        out = torch.empty((m, self.n), dtype=torch.bfloat16, device=x.device)
-        stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-        work = get_global_workspace(x.device) if m > 64 else None
-        self.lib.bitlinear_TernaSpMM_bf16_packed_ws(_p(x.contiguous()), _p(self.packed), _p(out), _p(self.scale_f32),
-                                                    self.ws_num, m, self.n, self.k, 0, _p(work),
-                                                    work.numel() if work is not None else 0, stream)
-        return out
+        work = get_global_workspace(x.device) if x.shape[0] > 64 else None
+        return _lib.native().linear_bf16_packed(x, self.packed, self.scale_f32, self.ws_num, self.n, work)
 
     def __call__(self, x: torch.Tensor) -> torch.Tensor:
         if self.act == "int8":                # model.py:120-133
@@ -380,16 +369,9 @@ class Block:
                                                     bsz, a.n_heads, a.n_kv_heads, a.head_dim, cache_k.shape[2],
                                                     a.head_dim ** -0.5, int(a.rope_adjacent), _p(attn_ws), stream)
         elif self.fused:
-            lib = self.wqkv.lib
-            stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-            q = torch.empty((bsz, a.n_heads, t, a.head_dim), dtype=torch.bfloat16, device=x.device)
-            lib.ternaspmm_rope_kv_store(_p(qkv), _p(cos), _p(sin), _p(pos_idx), per_seq, _p(q), _p(cache_k), _p(cache_v),
-                                        bsz, t, a.n_heads, a.n_kv_heads, a.head_dim, cache_k.shape[2],
-                                        int(a.rope_adjacent), stream)
-            if mask is KERNEL_ATTENTION:    # the prompt pass: the library's multi-token attention over the cache
-                o = torch.empty((bsz * t, a.n_heads * a.head_dim), dtype=torch.bfloat16, device=x.device)
-                lib.ternaspmm_prefill_attention(_p(q), _p(cache_k), _p(cache_v), _p(pos_idx), per_seq, _p(o), bsz, t, a.n_heads,
-                                                a.n_kv_heads, a.head_dim, cache_k.shape[2], a.head_dim ** -0.5, stream)
+            # RoPE + cache write, and on the prompt pass the library's multi-token attention over the cache
+            q = o = _lib.native().prompt_attention(qkv, cos, sin, pos_idx, cache_k, cache_v, a.n_heads, a.head_dim, a.head_dim ** -0.5,
+                                                   int(a.rope_adjacent), mask is KERNEL_ATTENTION)
         else:
             qkv = qkv.view(bsz, t, a.n_heads + 2 * a.n_kv_heads, a.head_dim).transpose(1, 2)
             q, k, v = qkv[:, :a.n_heads], qkv[:, a.n_heads:a.n_heads + a.n_kv_heads], qkv[:, a.n_heads + a.n_kv_heads:]

@@ -1079,3 +1079,28 @@ def test_rope_decode_attention_partial_rotate_half(lib, b, h, kv, d, s_max, n, s
     tol = 2.0 ** -7 * np.abs(unsplit).max(axis=-1, keepdims=True) + 1e-6
     assert np.isfinite(got).all()
     assert (np.abs(got - unsplit) <= 2 * tol).all(), float((np.abs(got - unsplit) / tol).max())
+
+
+@pytest.mark.parametrize("mode", [O.QUANT_ROUNDED, O.QUANT_COMPILED, O.QUANT_EAGER])
+@pytest.mark.parametrize("m,k", [(1, 64), (3, 2048), (2, 2056), (5, 4096), (2, 4104), (300, 6912), (1, 8192)])
+def test_quant_input_kernel(lib, m, k, mode):
+    """ternaspmm_quant_input behind linear.quant_input, bit for bit, on both sides of every vectors-per-thread variant; an
+    all-zero row (the clamp); rows it does not take stay with the torch statement of the same lines."""
+    from ternainfer_amd import linear as L
+    x = make_bf16_activations(m, k, 900 + k + m, outlier_frac=0.01)
+    x[m // 2] = 0
+    want_q, want_s = O.quant_input(x, mode)
+    print(f"[case] quant_input M={m} K={k} mode={mode}", flush=True)
+    lib.ternaspmm_quant_mode(mode)
+    try:
+        xd = _dev(x).view(torch.bfloat16)
+        for got_q, got_s in (L.quant_input(xd), L.quant_input(xd.reshape(1, m, k)), L.quant_input(xd.reshape(-1)[1:1 + (k - 8) * m].reshape(m, k - 8))):
+            if got_q.shape[-1] == k - 8:           # an unaligned view: same definition, other rows
+                want_q, want_s = O.quant_input(x.reshape(-1)[1:1 + (k - 8) * m].reshape(m, k - 8), mode)
+            assert got_s.shape == got_q.shape[:-1] + (1,)
+            assert (got_q.cpu().numpy().reshape(want_q.shape) == want_q).all()
+            assert (got_s.view(torch.int16).cpu().numpy().view(np.uint16).reshape(-1) == want_s).all()
+        assert lib.ternaspmm_quant_input(_vp(xd), _vp(xd), _vp(xd), m, 8200, None) == -1
+        assert lib.ternaspmm_quant_input(_vp(xd), _vp(xd), _vp(xd), m, 60, None) == -1
+    finally:
+        lib.ternaspmm_quant_mode(O.QUANT_ROUNDED)
