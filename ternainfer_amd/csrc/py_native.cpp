@@ -32,7 +32,15 @@ namespace {
     X(ternaspmm_fused_linear)                                                                                          \
     X(ternaspmm_quant_from_stats)                                                                                      \
     X(ternaspmm_rope_kv_store)                                                                                         \
-    X(ternaspmm_prefill_attention)
+    X(ternaspmm_prefill_attention)                                                                                     \
+    X(ternaspmm_rope_decode_attention)                                                                                 \
+    X(ternaspmm_rope_decode_attention_stats)                                                                           \
+    X(ternaspmm_rope_decode_attention_partial)                                                                         \
+    X(ternaspmm_attention_partial_bytes)                                                                               \
+    X(ternaspmm_attention_workspace_bytes)                                                                             \
+    X(ternaspmm_attention_merge_rmsnorm_quant)                                                                         \
+    X(ternaspmm_row_stats_count)                                                                                       \
+    X(ternaspmm_step_inputs)
 struct Library {
 #define X(name) decltype(&::name) name = nullptr;
     TERNA_ENTRY_POINTS(X)
@@ -395,47 +403,129 @@ TERNA_FUNCTION(fused_linear, 17)
     return pack(std::move(out), std::move(stats_out), std::move(raw), std::move(xq), std::move(s));
 }
 
-void check_cache(const char* who, const at::Tensor& k, const at::Tensor& v, int64_t kv_heads, int64_t head_dim)
-{
-    if (k.dim() != 4 || k.sizes() != v.sizes() || k.size(1) != kv_heads || k.size(3) != head_dim || !k.is_contiguous() || !v.is_contiguous())
-        refuse("%s: the caches are contiguous [B, KV, S, D] tensors of one shape", who);
-}
-// Positions of the t new tokens: [t] for all sequences, or [batch, t]; cos / sin rows of the same tokens.
-bool check_positions(const char* who, const at::Tensor& pos, int64_t batch, int64_t t)
-{
-    const bool each = pos.dim() == 2;
-    if (pos.scalar_type() != at::kLong || pos.numel() != (each ? batch * t : t) || !pos.is_contiguous())
-        refuse("%s: positions are a contiguous int64 [T] or [B, T] tensor", who);
-    return each;
-}
+// What the attention entry points read of a block's new tokens, checked against each other.
+struct AttentionArgs {
+    const at::Tensor &qkv, &cos, &sin, &pos, &ck, &cv;
+    int64_t heads, head_dim, batch, kv, slots, t;
+    float scale;
+    int adjacent;
+    bool each;                     // every sequence has its own positions
 
-// (qkv bf16 [B * T, (H + 2 KV) D], cos, sin, pos, cache_k, cache_v, heads, head_dim, scale, adjacent, attention): RoPE and cache write
-// of T new tokens per sequence, and with `attention` the multi-token attention -> bf16 [B * T, H D]; without it the
-// rotated q [B, H, T, D]
+    // a: qkv bf16 [B * T, (H + 2 KV) D], cos, sin, pos, cache_k, cache_v, heads, head_dim, scale, adjacent
+    AttentionArgs(const char* who, PyObject* const* a)
+        : qkv(*tensor(a[0])), cos(*tensor(a[1])), sin(*tensor(a[2])), pos(*tensor(a[3])), ck(*tensor(a[4])), cv(*tensor(a[5])),
+          heads(integer32(a[6])), head_dim(integer32(a[7])), scale(real(a[8])), adjacent(integer32(a[9]))
+    {
+        check_matrix(who, qkv);
+        if (ck.dim() != 4 || ck.sizes() != cv.sizes() || ck.size(0) < 1 || ck.size(3) != head_dim || !ck.is_contiguous() || !cv.is_contiguous())
+            refuse("%s: the caches are contiguous [B, KV, S, D] tensors of one shape", who);
+        batch = ck.size(0), kv = ck.size(1), slots = ck.size(2), t = qkv.size(0) / batch;
+        if (qkv.size(0) != batch * t || qkv.size(1) != (heads + 2 * kv) * head_dim || !qkv.is_contiguous())
+            refuse("%s: qkv does not have the shape of its caches", who);
+        each = pos.dim() == 2;
+        const int64_t rows = each ? batch * t : t;
+        if (pos.scalar_type() != at::kLong || pos.numel() != rows || !pos.is_contiguous())
+            refuse("%s: positions are a contiguous int64 [T] or [B, T] tensor", who);
+        if (cos.numel() < rows * (head_dim / 2) || sin.numel() != cos.numel() || cos.scalar_type() != at::kFloat || sin.scalar_type() != at::kFloat ||
+            !cos.is_contiguous() || !sin.is_contiguous())
+            refuse("%s: cos / sin are contiguous fp32 rows of D / 2, one per position", who);
+    }
+};
+#define TERNA_ATTENTION_INPUTS(g)                                                                                      \
+    data<terna_bf16>(&(g).qkv), data<float>(&(g).cos), data<float>(&(g).sin), data<long long>(&(g).pos), (g).each
+
+// (the ten of AttentionArgs, attention): RoPE and cache write of T new tokens per sequence, and with `attention` the multi-token
+// attention -> bf16 [B * T, H D]; without it the rotated q [B, H, T, D]
 TERNA_FUNCTION(prompt_attention, 11)
 {
-    const char* who = "prompt_attention";
-    const at::Tensor &qkv = *tensor(a[0]), &cos = *tensor(a[1]), &sin = *tensor(a[2]), &pos = *tensor(a[3]), &ck = *tensor(a[4]), &cv = *tensor(a[5]);
-    const int64_t h = integer32(a[6]), d = integer32(a[7]);
-    check_matrix(who, qkv);
-    if (ck.dim() != 4) refuse("%s: the caches are [B, KV, S, D] tensors", who);
-    const int64_t batch = ck.size(0), kv = ck.size(1), slots = ck.size(2), t = qkv.size(0) / std::max<int64_t>(batch, 1);
-    check_cache(who, ck, cv, kv, d);
-    if (batch < 1 || qkv.size(0) != batch * t || qkv.size(1) != (h + 2 * kv) * d || !qkv.is_contiguous())
-        refuse("%s: qkv does not have the shape of its caches", who);
-    const bool each = check_positions(who, pos, batch, t);
-    const int64_t angles = (each ? batch * t : t) * (d / 2);
-    if (cos.numel() != angles || sin.numel() != angles || cos.scalar_type() != at::kFloat || sin.scalar_type() != at::kFloat || !cos.is_contiguous() || !sin.is_contiguous())
-        refuse("%s: cos / sin are contiguous fp32 rows of D / 2, one per position", who);
-    at::Tensor q = make({batch, h, t, d}, at::kBFloat16, qkv);
+    const AttentionArgs g("prompt_attention", a);
+    at::Tensor q = make({g.batch, g.heads, g.t, g.head_dim}, at::kBFloat16, g.qkv);
     const terna_stream st = stream();
-    lib.ternaspmm_rope_kv_store(data<terna_bf16>(&qkv), data<float>(&cos), data<float>(&sin), data<long long>(&pos), each, data<terna_bf16>(&q),
-                                data<terna_bf16>(&ck), data<terna_bf16>(&cv), batch, t, h, kv, d, slots, integer32(a[9]), st);
+    lib.ternaspmm_rope_kv_store(TERNA_ATTENTION_INPUTS(g), data<terna_bf16>(&q), data<terna_bf16>(&g.ck), data<terna_bf16>(&g.cv), g.batch, g.t, g.heads,
+                                g.kv, g.head_dim, g.slots, g.adjacent, st);
     if (!PyObject_IsTrue(a[10])) return wrap(std::move(q));
-    at::Tensor o = make({batch * t, h * d}, at::kBFloat16, qkv);
-    lib.ternaspmm_prefill_attention(data<terna_bf16>(&q), data<terna_bf16>(&ck), data<terna_bf16>(&cv), data<long long>(&pos), each, data<terna_bf16>(&o),
-                                    batch, t, h, kv, d, slots, real(a[8]), st);
+    at::Tensor o = make({g.batch * g.t, g.heads * g.head_dim}, at::kBFloat16, g.qkv);
+    lib.ternaspmm_prefill_attention(data<terna_bf16>(&q), data<terna_bf16>(&g.ck), data<terna_bf16>(&g.cv), data<long long>(&g.pos), g.each,
+                                    data<terna_bf16>(&o), g.batch, g.t, g.heads, g.kv, g.head_dim, g.slots, g.scale, st);
     return wrap(std::move(o));
+}
+
+// (the ten of AttentionArgs, workspace | None, norm_weight | None, partial | None, splits): RoPE, cache write and attention of one new
+// token per sequence -> (out bf16 [B, H D], None); with the norm's weights (out, its partial statistics [B, H, 2]); with a
+// buffer for partial results these are all that is written -> None
+TERNA_FUNCTION(decode_attention, 14)
+{
+    const char* who = "decode_attention";
+    const AttentionArgs g(who, a);
+    const at::Tensor *workspace = tensor(a[10]), *weight = tensor(a[11]), *partial = tensor(a[12]);
+    if (g.t != 1) refuse("%s: one new token per sequence", who);
+    const terna_stream st = stream();
+    terna_bf16 *ck = data<terna_bf16>(&g.ck), *cv = data<terna_bf16>(&g.cv);
+    if (partial != nullptr) {
+        const long long need = lib.ternaspmm_attention_partial_bytes(g.batch, g.heads, g.head_dim);
+        if (need < 0 || static_cast<long long>(partial->numel() * partial->element_size()) < need) refuse("%s: the partial buffer is too small", who);
+        lib.ternaspmm_rope_decode_attention_partial(TERNA_ATTENTION_INPUTS(g), ck, cv, data<float>(partial), integer32(a[13]), g.batch, g.heads, g.kv,
+                                                    g.head_dim, g.slots, g.scale, g.adjacent, nullptr, nullptr, nullptr, 0, st);
+        Py_RETURN_NONE;
+    }
+    at::Tensor o = make({g.batch, g.heads * g.head_dim}, at::kBFloat16, g.qkv), stats;
+    if (weight != nullptr) {
+        check_numel(who, "norm_weight", weight, g.heads * g.head_dim);
+        stats = make({g.batch, g.heads, 2}, at::kFloat, g.qkv);
+        if (lib.ternaspmm_rope_decode_attention_stats(TERNA_ATTENTION_INPUTS(g), ck, cv, data<terna_bf16>(&o), g.batch, g.heads, g.kv, g.head_dim, g.slots,
+                                                      g.scale, g.adjacent, data<terna_bf16>(weight), data<float>(&stats), st) != g.heads)
+            refuse("%s: ternaspmm_rope_decode_attention_stats refused the launch", who);
+    } else {
+        if (workspace != nullptr && static_cast<long long>(workspace->numel() * workspace->element_size()) <
+                                        lib.ternaspmm_attention_workspace_bytes(g.batch, g.heads, g.head_dim))
+            refuse("%s: the workspace is too small", who);
+        lib.ternaspmm_rope_decode_attention(TERNA_ATTENTION_INPUTS(g), ck, cv, data<terna_bf16>(&o), g.batch, g.heads, g.kv, g.head_dim, g.slots, g.scale,
+                                            g.adjacent, data(workspace), st);
+    }
+    return pack(std::move(o), std::move(stats));
+}
+
+// (partial, splits, heads, head_dim, norm_weight, eps, sequences, want_output) -> (xq, s, o | None), or None
+TERNA_FUNCTION(attention_merge_rmsnorm_quant, 8)
+{
+    const char* who = "attention_merge_rmsnorm_quant";
+    const at::Tensor &partial = *tensor(a[0]), &weight = *tensor(a[4]);
+    const int splits = integer32(a[1]), heads = integer32(a[2]), head_dim = integer32(a[3]), sequences = integer32(a[6]);
+    const float eps = real(a[5]);
+    const int64_t k = static_cast<int64_t>(heads) * head_dim;
+    const long long held = partial.numel() * partial.element_size(), need = lib.ternaspmm_attention_partial_bytes(sequences, heads, head_dim);
+    if (sequences < 1 || need < 0 || held < need) refuse("partial buffer of %lld bytes does not hold %d sequences", held, sequences);
+    if (weight.numel() != k || weight.scalar_type() != at::kBFloat16) refuse("%s: the norm weight is a bf16 vector of heads * head_dim elements", who);
+    at::Tensor q = make({sequences, k}, at::kChar, partial), s = make({sequences}, at::kBFloat16, partial), o;
+    if (PyObject_IsTrue(a[7])) o = make({sequences, k}, at::kBFloat16, partial);
+    if (lib.ternaspmm_attention_merge_rmsnorm_quant(data<float>(&partial), splits, data<terna_bf16>(&weight), eps, o.defined() ? data<terna_bf16>(&o) : nullptr,
+                                                    data<int8_t>(&q), data<terna_bf16>(&s), sequences, heads, head_dim, stream()) != 0)
+        Py_RETURN_NONE;
+    return pack(std::move(q), std::move(s), std::move(o));
+}
+
+// (tokens, pos, embedding, rope_table, norm_weight) -> (x, stats, rope [2, B, half]); tokens / pos contiguous int64 vectors
+TERNA_FUNCTION(step_inputs, 5)
+{
+    const char* who = "step_inputs";
+    const at::Tensor &tokens = *tensor(a[0]), &pos = *tensor(a[1]), &embedding = *tensor(a[2]), &table = *tensor(a[3]), &weight = *tensor(a[4]);
+    check_matrix(who, embedding);
+    const int64_t b = tokens.numel(), v = embedding.size(0), k = embedding.size(1);
+    if (table.dim() != 3 || table.size(1) != 2 || tokens.scalar_type() != at::kLong || pos.scalar_type() != at::kLong || (pos.numel() != 1 && pos.numel() != b) ||
+        table.scalar_type() != at::kFloat || embedding.scalar_type() != at::kBFloat16 || !embedding.is_contiguous() || !table.is_contiguous())
+        refuse("%s: tokens / pos int64, embedding bf16 [V, K] and rope_table fp32 [S, 2, half] contiguous", who);
+    check_numel(who, "norm_weight", &weight, k);
+    const int count = lib.ternaspmm_row_stats_count(k);
+    if (count < 1) refuse("%s: unsupported K=%d", who, static_cast<int>(k));
+    const at::Tensor ids = tokens.contiguous(), at_slot = pos.contiguous();         // (copies only where a caller passed a strided view)
+    const int64_t slots = table.size(0), half = table.size(2);
+    at::Tensor x = make({b, k}, at::kBFloat16, embedding), stats = make({b, count, 2}, at::kFloat, embedding), rope = make({2, b, half}, at::kFloat, embedding);
+    if (lib.ternaspmm_step_inputs(data<long long>(&ids), data<long long>(&at_slot), pos.numel() == b && b > 1, data<terna_bf16>(&embedding), v, k,
+                                  data<float>(&table), slots, half, data<terna_bf16>(&weight), data<terna_bf16>(&x), data<float>(&stats), data<float>(&rope), b,
+                                  stream()) != count)
+        refuse("%s: the library refused the launch (B=%d V=%d K=%d S=%d half=%d)", who, static_cast<int>(b), static_cast<int>(v), static_cast<int>(k),
+               static_cast<int>(slots), static_cast<int>(half));
+    return pack(std::move(x), std::move(stats), std::move(rope));
 }
 
 // (path of libternaspmm.so)
@@ -461,7 +551,8 @@ TERNA_FUNCTION(init, 1)
 #define METHOD(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(name)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {METHOD(init), METHOD(bit_linear), METHOD(bit_linear_bf16), METHOD(quant_input), METHOD(linear_packed),
                          METHOD(linear_bf16_packed), METHOD(rmsnorm_quant), METHOD(relu2_mul_rmsnorm_quant), METHOD(quant_from_stats),
-                         METHOD(fused_linear), METHOD(prompt_attention), {nullptr, nullptr, 0, nullptr}};
+                         METHOD(fused_linear), METHOD(prompt_attention), METHOD(decode_attention),
+                         METHOD(attention_merge_rmsnorm_quant), METHOD(step_inputs), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

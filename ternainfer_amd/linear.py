@@ -178,20 +178,7 @@ def attention_merge_rmsnorm_quant(partial, splits, heads, head_dim, norm_weight,
     projection from the partial results of a split attention launch.  Returns (xq int8 [sequences, heads * head_dim],
     s bf16 [sequences], o) -- o the merged attention output with `want_output`, else None -- or None where the library
     does not take the shape (nothing enqueued)."""
-    lib = _lib.load()
-    k = heads * head_dim
-    need = lib.ternaspmm_attention_partial_bytes(sequences, heads, head_dim)
-    if sequences < 1 or need < 0 or partial.numel() * partial.element_size() < need:
-        raise ValueError(f"partial buffer of {partial.numel() * partial.element_size()} bytes does not hold {sequences} sequences")
-    if norm_weight.numel() != k or norm_weight.dtype != torch.bfloat16:
-        raise ValueError("attention_merge_rmsnorm_quant: the norm weight is a bf16 vector of heads * head_dim elements")
-    dev = partial.device
-    xq = torch.empty((sequences, k), dtype=torch.int8, device=dev)
-    s = torch.empty(sequences, dtype=torch.bfloat16, device=dev)
-    o = torch.empty((sequences, k), dtype=torch.bfloat16, device=dev) if want_output else None
-    rc = lib.ternaspmm_attention_merge_rmsnorm_quant(_p(partial), splits, _p(norm_weight), float(eps), _p(o) if o is not None else None, _p(xq), _p(s), sequences, heads,
-                                                     head_dim, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
-    return None if rc != 0 else (xq, s, o)
+    return _lib.native().attention_merge_rmsnorm_quant(partial, splits, heads, head_dim, norm_weight, eps, sequences, want_output)
 
 
 def relu2_mul_rmsnorm_linear_packed(x13, norm_weight, eps, packed, ws, ws_num, out_features):
@@ -249,25 +236,7 @@ def step_inputs(tokens, pos, embedding, rope_table, norm_weight):
     """The inputs of a single-token step in one launch (ternaspmm_step_inputs): tokens int64 [B] (any shape with B
     elements), pos int64 [1] (one position for all) or [B], embedding bf16 [V, K], rope_table fp32 [S, 2, half].
     Returns (x bf16 [B, K], partials fp32 [B, count, 2] under `norm_weight`, cos fp32 [B, half], sin fp32 [B, half])."""
-    b = tokens.numel()
-    v, k = embedding.shape
-    s_len, two, half = rope_table.shape
-    tokens, pos = tokens.reshape(-1).contiguous(), pos.reshape(-1).contiguous()      # (copies only where a caller passed a strided view)
-    if tokens.dtype != torch.int64 or pos.dtype != torch.int64 or pos.numel() not in (1, b) or two != 2 or rope_table.dtype != torch.float32 \
-            or embedding.dtype != torch.bfloat16 or not (embedding.is_contiguous() and rope_table.is_contiguous()):
-        raise ValueError("step_inputs: tokens / pos int64, embedding bf16 [V, K] and rope_table fp32 [S, 2, half] contiguous")
-    _check_rows("step_inputs", embedding, norm_weight=(norm_weight, k))
-    lib = _lib.load()
-    count = lib.ternaspmm_row_stats_count(k)
-    if count < 1:
-        raise ValueError(f"step_inputs: unsupported K={k}")
-    x = torch.empty((b, k), dtype=torch.bfloat16, device=embedding.device)
-    stats = torch.empty((b, count, 2), dtype=torch.float32, device=embedding.device)
-    rope = torch.empty((2, b, half), dtype=torch.float32, device=embedding.device)
-    got = lib.ternaspmm_step_inputs(_p(tokens), _p(pos), int(pos.numel() == b and b > 1), _p(embedding), v, k, _p(rope_table), s_len, half,
-                                    _p(norm_weight), _p(x), _p(stats), _p(rope), b, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
-    if got != count:
-        raise ValueError(f"step_inputs: the library refused the launch (B={b} V={v} K={k} S={s_len} half={half})")
+    x, stats, rope = _lib.native().step_inputs(tokens, pos, embedding, rope_table, norm_weight)
     return x, stats, rope[0], rope[1]
 
 

@@ -9,8 +9,8 @@ per row to int8 in front of every ternary linear.  The residual adds, the four n
 that quantisation run as the library's fused prologue kernels (one launch in front of each
 linear); RoPE + KV-cache write, single-token attention, the multi-token attention of the prompt
 pass, the LM head of a decode step and greedy sampling are library kernels too (the prompt pass projects
-its last rows through the LM head with a PyTorch-ROCm matmul); the prompt pass and one decode step are
-each captured in a HIP graph, as generate.py:204-224 does for the decode step.
+its last rows through the LM head with a PyTorch-ROCm matmul); one decode step is captured in a HIP graph, as
+generate.py:204-224 does.
 """
 from __future__ import annotations
 
@@ -216,6 +216,7 @@ class Block:
         bsz = cache_k.shape[0]
         lib = self.wqkv.lib
         stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        native = _lib.native()
         per_seq = int(pos_idx.dim() == 2)
         cap = self.capture
         pub = cap is not None
@@ -239,15 +240,18 @@ class Block:
             note("wqkv", r)
             qkv = r[0]
         deferred = isinstance(attn_ws, tuple)
+        attend = (qkv, cos, sin, pos_idx, cache_k, cache_v, a.n_heads, a.head_dim, a.head_dim ** -0.5, int(a.rope_adjacent))
         o_kw = dict(epilogue=EPILOGUE_RESIDUAL, residual=x, next_norm_weight=self.ffn_norm, want_raw=pub, publish=pub)
         if deferred:
             partial, splits = attn_ws
             # (weights of the next launches through the caches meanwhile: only next to a short attention -- with caches of
             # 1528 slots the prefetch cost 2 % of the step, at 728 slots it gains 0.5 %)
-            pf = self.prefetch if split and self.prefetch is not None and cache_k.shape[2] <= 1024 else (None, None, None, 0)
-            lib.ternaspmm_rope_decode_attention_partial(
-                _p(qkv), _p(cos), _p(sin), _p(pos_idx), per_seq, _p(cache_k), _p(cache_v), _p(partial), splits, bsz, a.n_heads,
-                a.n_kv_heads, a.head_dim, cache_k.shape[2], a.head_dim ** -0.5, int(a.rope_adjacent), *pf, stream)
+            if split and self.prefetch is not None and cache_k.shape[2] <= 1024:
+                lib.ternaspmm_rope_decode_attention_partial(
+                    _p(qkv), _p(cos), _p(sin), _p(pos_idx), per_seq, _p(cache_k), _p(cache_v), _p(partial), splits, bsz, a.n_heads,
+                    a.n_kv_heads, a.head_dim, cache_k.shape[2], a.head_dim ** -0.5, int(a.rope_adjacent), *self.prefetch, stream)
+            else:
+                native.decode_attention(*attend, None, None, partial, splits)
             r = None
             if split or (bsz > 1 and self.merge_quant):
                 # merge + sub-norm + quantisation once per sequence, then the O projection on the quantised rows
@@ -267,9 +271,9 @@ class Block:
                 lib.ternaspmm_attention_merge(_p(partial), splits, _p(o), bsz, a.n_heads, a.head_dim, stream)
                 r = fused_linear(o, self.attn_sub_norm, a.norm_eps, self.wo.packed, self.wo.ws, self.wo.ws_num, self.wo.n, self.wo.k, **o_kw)
         else:
-            o = torch.empty((bsz, a.n_heads * a.head_dim), dtype=torch.bfloat16, device=x.device)
             o_stats = None
             if self.prefetch is not None:
+                o = torch.empty((bsz, a.n_heads * a.head_dim), dtype=torch.bfloat16, device=x.device)
                 ptrs, sizes, units, count = self.prefetch
                 lib.ternaspmm_rope_decode_attention_prefetch(
                     _p(qkv), _p(cos), _p(sin), _p(pos_idx), per_seq, _p(cache_k), _p(cache_v), _p(o), bsz, a.n_heads, a.n_kv_heads,
@@ -278,15 +282,9 @@ class Block:
             elif (bsz > self.o_norm_rows or (bsz > 1 and self.attention_stats_chain)) and self.attention_stats:
                 # the unsplit launch also leaves the sub-norm's partial statistics per head: the quantised rows of the O
                 # projection then come from the element-wise launch instead of the norm kernel
-                o_stats = torch.empty((bsz, a.n_heads, 2), dtype=torch.float32, device=x.device)
-                if lib.ternaspmm_rope_decode_attention_stats(_p(qkv), _p(cos), _p(sin), _p(pos_idx), per_seq, _p(cache_k), _p(cache_v), _p(o),
-                                                             bsz, a.n_heads, a.n_kv_heads, a.head_dim, cache_k.shape[2], a.head_dim ** -0.5,
-                                                             int(a.rope_adjacent), _p(self.attn_sub_norm), _p(o_stats), stream) != a.n_heads:
-                    raise RuntimeError("ternaspmm_rope_decode_attention_stats refused the launch")
+                o, o_stats = native.decode_attention(*attend, None, self.attn_sub_norm, None, 0)
             else:
-                lib.ternaspmm_rope_decode_attention(_p(qkv), _p(cos), _p(sin), _p(pos_idx), per_seq, _p(cache_k), _p(cache_v), _p(o),
-                                                    bsz, a.n_heads, a.n_kv_heads, a.head_dim, cache_k.shape[2],
-                                                    a.head_dim ** -0.5, int(a.rope_adjacent), _p(attn_ws), stream)
+                o, _ = native.decode_attention(*attend, attn_ws, None, None, 0)
             if pub:
                 cap.append(("attention", None, None, o))
             r = None
@@ -338,40 +336,34 @@ class Block:
         per_seq = int(pos_idx.dim() == 2)
         qkv, x = self._norm_linear(self.wqkv, x, self.attention_norm, residual=pending, name="wqkv")
         rep = a.n_heads // a.n_kv_heads
+        native = _lib.native()
+        attend = (qkv, cos, sin, pos_idx, cache_k, cache_v, a.n_heads, a.head_dim, a.head_dim ** -0.5, int(a.rope_adjacent))
         one_token = mask is None           # the caller's rule: fused, one new token, a head size the kernel has
         deferred = one_token and isinstance(attn_ws, tuple)
         if deferred:
             # the cache prefix of every head split over several workgroups that leave partial results; the O
             # projection's prologue merges them (one sequence; else a merge launch): the launch boundary is the synchronisation
-            lib = self.wqkv.lib
-            stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
             # (no prefetch regions here: this launch is shorter than the prefetch of the following weights would be --
             # measured with them 1005 - 1125 us per step against 960 without and 971 for the unsplit launch that prefetches)
             partial, splits = attn_ws
-            lib.ternaspmm_rope_decode_attention_partial(
-                _p(qkv), _p(cos), _p(sin), _p(pos_idx), per_seq, _p(cache_k), _p(cache_v), _p(partial), splits, bsz, a.n_heads,
-                a.n_kv_heads, a.head_dim, cache_k.shape[2], a.head_dim ** -0.5, int(a.rope_adjacent), None, None, None, 0,
-                stream)
+            native.decode_attention(*attend, None, None, partial, splits)
         elif one_token:                     # RoPE, cache write and attention over the cache prefix: one launch
-            lib = self.wqkv.lib
-            stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-            o = torch.empty((bsz, a.n_heads * a.head_dim), dtype=torch.bfloat16, device=x.device)
             if self.prefetch is not None:
                 # the attention launch occupies one CU per head: extra workgroups of the same launch pull the
                 # weights of the launches that follow through the caches meanwhile
+                lib = self.wqkv.lib
+                stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+                o = torch.empty((bsz, a.n_heads * a.head_dim), dtype=torch.bfloat16, device=x.device)
                 ptrs, sizes, units, count = self.prefetch
                 lib.ternaspmm_rope_decode_attention_prefetch(
                     _p(qkv), _p(cos), _p(sin), _p(pos_idx), per_seq, _p(cache_k), _p(cache_v), _p(o), bsz, a.n_heads, a.n_kv_heads,
                     a.head_dim, cache_k.shape[2], a.head_dim ** -0.5, int(a.rope_adjacent), _p(attn_ws), ptrs, sizes, units,
                     count, stream)
             else:
-                lib.ternaspmm_rope_decode_attention(_p(qkv), _p(cos), _p(sin), _p(pos_idx), per_seq, _p(cache_k), _p(cache_v), _p(o),
-                                                    bsz, a.n_heads, a.n_kv_heads, a.head_dim, cache_k.shape[2],
-                                                    a.head_dim ** -0.5, int(a.rope_adjacent), _p(attn_ws), stream)
+                o, _ = native.decode_attention(*attend, attn_ws, None, None, 0)
         elif self.fused:
             # RoPE + cache write, and on the prompt pass the library's multi-token attention over the cache
-            q = o = _lib.native().prompt_attention(qkv, cos, sin, pos_idx, cache_k, cache_v, a.n_heads, a.head_dim, a.head_dim ** -0.5,
-                                                   int(a.rope_adjacent), mask is KERNEL_ATTENTION)
+            q = o = native.prompt_attention(*attend, mask is KERNEL_ATTENTION)
         else:
             qkv = qkv.view(bsz, t, a.n_heads + 2 * a.n_kv_heads, a.head_dim).transpose(1, 2)
             q, k, v = qkv[:, :a.n_heads], qkv[:, a.n_heads:a.n_heads + a.n_kv_heads], qkv[:, a.n_heads + a.n_kv_heads:]
@@ -613,113 +605,61 @@ class Transformer:
         return F.linear(x, self.tok_embeddings)
 
 
+def _greedy_steps(step, count: int, use_graph: bool) -> float:
+    """`count` calls of `step` (one greedy step on device buffers of its own), and the seconds they take on the device.  With
+    `use_graph` the step is captured once and replayed, so that the host issues one graph launch per token; its first call
+    runs as it is, which is also what loads and initialises everything the capture then finds in place -- a captured step
+    does not run, so nothing has to be put back.  (The prompt pass runs once: capturing it would double its work.)"""
+    ev = [torch.cuda.Event(enable_timing=True) for _ in range(4)]
+    ev[0].record()
+    if count > 0:
+        step()
+    ev[1].record()
+    again = step
+    if use_graph and count > 1:
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            step()
+        again = graph.replay
+    ev[2].record()
+    for _ in range(count - 1):
+        again()
+    ev[3].record()
+    torch.cuda.synchronize()
+    return (ev[0].elapsed_time(ev[1]) + ev[2].elapsed_time(ev[3])) * 1e-3
+
+
 @torch.inference_mode()
 def greedy_decode(model: Transformer, prompt: torch.Tensor, gen_tokens: int, use_graph: bool = True, prompt_lens=None):
     """Prefill `prompt` [B, P], then `gen_tokens` greedy steps.  Returns (tokens [B, gen_tokens],
     prefill seconds, decode seconds).  The decode step (model forward + argmax + position bump) is
-    captured once and replayed, so the host issues one graph launch per token.
+    captured once and replayed (`_greedy_steps`).
     `prompt_lens` (int64 [B], each 1 .. P): the prompts have different lengths and are padded to P with any token
     (generate.py:244-262): sequence b's first generated token comes from its prompt token prompt_lens[b] - 1, and
-    its n-th decode step runs at cache slot prompt_lens[b] + n -- every sequence at its own position."""
+    its n-th decode step runs at cache slot prompt_lens[b] + n -- every sequence at its own position.  A padding token's
+    cache rows are overwritten by the decode steps before any query can see them."""
     bsz, plen = prompt.shape
     cache = model.make_cache(bsz, plen + gen_tokens)
-    ev = [torch.cuda.Event(enable_timing=True) for _ in range(4)]
     slots = torch.arange(plen, device="cuda")
-    if prompt_lens is not None:
-        return _greedy_decode_ragged(model, prompt, prompt_lens.to(device="cuda", dtype=torch.int64), gen_tokens, use_graph,
-                                     cache, slots, ev)
-    if use_graph:
-        # the prompt pass as a graph too (generate.py:100-144): warm up on a side stream, capture, replay
-        side = torch.cuda.Stream()
-        side.wait_stream(torch.cuda.current_stream())
-        with torch.cuda.stream(side):
-            model.forward(prompt, cache, slots)
-        torch.cuda.current_stream().wait_stream(side)
-        prefill = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(prefill):
-            logits = model.forward(prompt, cache, slots)
-        torch.cuda.synchronize()
-        ev[0].record()
-        prefill.replay()
-    else:
-        ev[0].record()
-        logits = model.forward(prompt, cache, slots)
+    ragged = prompt_lens is not None
+    if ragged:
+        prompt_lens = prompt_lens.to(device="cuda", dtype=torch.int64)
+    ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+    ev[0].record()
+    logits = model.forward(prompt, cache, slots, last_idx=prompt_lens - 1 if ragged else None)
     tok = argmax_rows(logits.contiguous())                                    # int64 [B, 1]
     ev[1].record()
-    counters = torch.tensor([plen, 1], dtype=torch.int64, device="cuda")      # cache slot of the next token, tokens stored
-    pos = counters[0:1]
+    # [0] cache slot of the next token (sequences of one length), [1] tokens stored in the history
+    counters = torch.tensor([0 if ragged else plen, 1], dtype=torch.int64, device="cuda")
+    pos = prompt_lens.clone().view(bsz, 1) if ragged else counters[0:1]       # per sequence, or the shared one
     out = torch.empty((bsz, gen_tokens), dtype=torch.int64, device="cuda")
     out[:, 0:1] = tok
     state = greedy_step_state(bsz)
 
     def step():                                                               # the forward has read tok by the time it changes
         greedy_step(model.forward(tok, cache, pos), tok, out, counters, state)
+        if ragged:
+            pos.add_(1)
 
-    graph = None
-    if use_graph:
-        # warm up on a side stream (allocator, lazy inits), then restore the state and capture
-        snap = (tok.clone(), counters.clone())
-        side = torch.cuda.Stream()
-        side.wait_stream(torch.cuda.current_stream())
-        with torch.cuda.stream(side):
-            step()
-        torch.cuda.current_stream().wait_stream(side)
-        tok.copy_(snap[0]); counters.copy_(snap[1])
-        graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph):
-            step()
-        tok.copy_(snap[0]); counters.copy_(snap[1])
-    torch.cuda.synchronize()
-    ev[2].record()
-    for _ in range(gen_tokens):
-        if graph is not None:
-            graph.replay()
-        else:
-            step()
-    ev[3].record()
-    torch.cuda.synchronize()
-    return out, ev[0].elapsed_time(ev[1]) * 1e-3, ev[2].elapsed_time(ev[3]) * 1e-3
-
-
-def _greedy_decode_ragged(model, prompt, prompt_lens, gen_tokens, use_graph, cache, slots, ev):
-    """greedy_decode for prompts of different lengths: the prompt pass runs on the padded prompts (a padding token's
-    cache rows are overwritten by the decode steps before any query can see them), the decode steps carry one cache
-    position per sequence."""
-    bsz = prompt.shape[0]
-    ev[0].record()
-    logits = model.forward(prompt, cache, slots, last_idx=prompt_lens - 1)
-    tok = argmax_rows(logits.contiguous())                                    # int64 [B, 1]
-    ev[1].record()
-    seq_pos = prompt_lens.clone().view(bsz, 1)                                # cache slot of every sequence's next token
-    counters = torch.tensor([0, 1], dtype=torch.int64, device="cuda")         # [1]: tokens stored in the history
-    out = torch.empty((bsz, gen_tokens), dtype=torch.int64, device="cuda")
-    out[:, 0:1] = tok
-    state = greedy_step_state(bsz)
-
-    def step():
-        greedy_step(model.forward(tok, cache, seq_pos), tok, out, counters, state)
-        seq_pos.add_(1)
-
-    graph = None
-    if use_graph:
-        snap = (tok.clone(), counters.clone(), seq_pos.clone())
-        side = torch.cuda.Stream()
-        side.wait_stream(torch.cuda.current_stream())
-        with torch.cuda.stream(side):
-            step()
-        torch.cuda.current_stream().wait_stream(side)
-        tok.copy_(snap[0]); counters.copy_(snap[1]); seq_pos.copy_(snap[2])
-        graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph):
-            step()
-        tok.copy_(snap[0]); counters.copy_(snap[1]); seq_pos.copy_(snap[2])
-    torch.cuda.synchronize()
-    ev[2].record()
-    for _ in range(gen_tokens):
-        if graph is not None:
-            graph.replay()
-        else:
-            step()
-    ev[3].record()
-    torch.cuda.synchronize()
-    return out, ev[0].elapsed_time(ev[1]) * 1e-3, ev[2].elapsed_time(ev[3]) * 1e-3
+    seconds = _greedy_steps(step, gen_tokens, use_graph)
+    return out, ev[0].elapsed_time(ev[1]) * 1e-3, seconds
