@@ -526,8 +526,9 @@ void ternaspmm_repack_cache_stats(long long out[6]);
  * copy.  Returns the kernel: 0 small-M kernel on the reference format, 1 MFMA-tiled kernel decoding the reference
  * format on the fly, 2 per-call transcode into the workspace + MFMA-tiled P2 kernel, 3 small-M kernel on the cached
  * copy, 4 MFMA-tiled kernel on the cached copy; -1 for an unsupported shape.  *workspace_bytes_used (may be NULL):
- * the highest byte offset of `workspace` the call would write, 0 when it stays untouched -- never more than the
- * sizes documented at bitlinear_TernaSpMM. */
+ * the highest byte offset of `workspace` the call may write, 0 when it stays untouched -- never more than the
+ * sizes documented at bitlinear_TernaSpMM.  (Kernels 3 and 4 give way to one that needs no workspace where mid_kernel_takes,
+ * launch_mid.hip, says so.) */
 int ternaspmm_plan_reference_call(int int8_activations, int route, int M, int N, int K, int SPLIT_K,
                                   const void* workspace, int cached, long long* workspace_bytes_used);
 

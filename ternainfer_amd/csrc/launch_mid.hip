@@ -1,0 +1,86 @@
+// Launcher of the kernel for 17 rows .. a few hundred on the P2 layout (mid_kernel.h): which calls it takes, which tile.
+#include "launchers.h"
+#include "host_util.h"
+#include "mid_kernel.h"
+
+namespace terna {
+namespace {
+
+struct MidTile {
+    int rt, fb;                  // 16-row tiles, 16-feature bands of a workgroup
+    long tiles;
+    int waves;
+};
+
+// A CU's load time is what a launch takes beyond its fixed part, so the tile is the one with the least of
+// (workgroups per CU, rounded up) x (bytes of one workgroup per 4 columns of K: 64 rt sz activations + 16 fb weights).
+// One workgroup per CU: as many waves as K has chunks for, evenly; more of them: four waves each, whose small LDS shares
+// let four or five workgroups overlap on a CU (measured at M = 17 .. 512: within 5 % of the best of the tiles and wave counts
+// in all but two of ninety cells).
+MidTile choose_tile(int M, int N, int K, int sz)
+{
+    const int chunks = (K / 64 + 3) / 4;
+    constexpr int kTiles[3][2] = {{1, 2}, {1, 4}, {2, 4}};
+    MidTile best{};
+    long best_cost = 0;
+    for (const auto& t : kTiles) {
+        const long tiles = static_cast<long>((M + 16 * t[0] - 1) / (16 * t[0])) * ((N / 16 + t[1] - 1) / t[1]);
+        const long cost = (tiles + 255) / 256 * (64 * t[0] * sz + 16 * t[1]);
+        if (best.rt == 0 || cost < best_cost) {
+            best = MidTile{t[0], t[1], tiles, 0};
+            best_cost = cost;
+        }
+    }
+    const int fit = 160 * 1024 / (16 * best.rt * 256 * sz);                // LDS of a workgroup
+    const int most = best.tiles > 256 ? 4 : (fit < kMidMaxWaves ? fit : kMidMaxWaves);
+    const int rounds = (chunks + most - 1) / most;
+    best.waves = best.tiles > 256 ? (chunks < most ? chunks : most) : (chunks + rounds - 1) / rounds;
+    return best;
+}
+
+template <typename Act, int RT, int FB>
+void launch_mid_as(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, int waves,
+                   const RepackGuard* guard, hipStream_t st)
+{
+    using S = MidShape<Act, RT, FB>;
+    const int row_tiles = (M + 16 * RT - 1) / (16 * RT), feature_tiles = (N / 16 + FB - 1) / FB;
+    const unsigned grid = static_cast<unsigned>((feature_tiles + 7) / 8 * 8 * row_tiles);
+    const dim3 block(waves * 64);
+    const int lds = waves * S::kWaveBytes;
+    if (guard != nullptr) {
+        auto kernel = terna_mid_kernel<Act, RT, FB, true>;
+        allow_dynamic_lds(kernel, 160 * 1024, "hipFuncSetAttribute(mid)", __LINE__);
+        kernel<<<dim3(grid + 1), block, lds, st>>>(x, packed, out, M, N, K, row_tiles, waves, ep, *guard);
+    } else {
+        auto kernel = terna_mid_kernel<Act, RT, FB, false>;
+        allow_dynamic_lds(kernel, 160 * 1024, "hipFuncSetAttribute(mid)", __LINE__);
+        kernel<<<dim3(grid), block, lds, st>>>(x, packed, out, M, N, K, row_tiles, waves, ep, RepackGuard{});
+    }
+}
+
+}  // namespace
+
+// Up to 16 rows the small-M kernels are faster (3.1 against 3.9 us).  Upwards the MFMA-tiled kernel, whose activations are
+// shared by 128 or 256 features, catches up where the outputs fill the chip several times: measured at M N = 1.9 M
+// (QKV: M = 512, gate+up: M = 140), with bf16 activations and a deep K, whose rows are the most bytes, at 1.05 M.
+bool mid_kernel_takes(const void* x, int M, int N, int K, size_t act_bytes)
+{
+    const long outputs = static_cast<long>(M) * N, most = act_bytes == 2 && K > 4096 ? 1050000 : 1900000;
+    return M > 16 && outputs <= most && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
+           static_cast<uint64_t>(M) * K * act_bytes < (1ull << 31) && static_cast<uint64_t>(N) * K / 4 < (1ull << 31);
+}
+
+template <typename Act>
+void launch_mid(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, hipStream_t st,
+                const RepackGuard* guard)
+{
+    const MidTile t = choose_tile(M, N, K, sizeof(Act));
+    if (t.rt == 2) launch_mid_as<Act, 2, 4>(x, packed, out, ep, M, N, K, t.waves, guard, st);
+    else if (t.fb == 4) launch_mid_as<Act, 1, 4>(x, packed, out, ep, M, N, K, t.waves, guard, st);
+    else launch_mid_as<Act, 1, 2>(x, packed, out, ep, M, N, K, t.waves, guard, st);
+}
+
+template void launch_mid<int8_t>(const int8_t*, const uint32_t*, uint16_t*, const Epilogue&, int, int, int, hipStream_t, const RepackGuard*);
+template void launch_mid<uint16_t>(const uint16_t*, const uint32_t*, uint16_t*, const Epilogue&, int, int, int, hipStream_t, const RepackGuard*);
+
+}  // namespace terna

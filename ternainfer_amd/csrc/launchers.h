@@ -40,6 +40,12 @@ void launch_decode_packed(const Act* x, const uint32_t* packed, uint16_t* out, c
 // next_w; raw_out (optional) the output itself.
 void launch_decode_packed_producer(const int8_t* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K,
                                    const uint16_t* residual, const uint16_t* next_w, float* stats_out, uint16_t* raw_out, hipStream_t st);
+// 17 rows .. a few hundred (launch_mid.hip): whether the kernel between the small-M and the MFMA-tiled one takes a call when the
+// library chooses, and its launch.
+bool mid_kernel_takes(const void* x, int M, int N, int K, size_t act_bytes);
+template <typename Act>
+void launch_mid(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, hipStream_t st,
+                const RepackGuard* guard = nullptr);
 // Fingerprint of the reference-format tensors named by `guard` into *out / the check of it as a launch of its own.
 void launch_repack_fingerprint(const RepackGuard& guard, unsigned long long* out, hipStream_t st);
 void launch_repack_guard(const RepackGuard* guard, hipStream_t st);
@@ -75,6 +81,9 @@ extern template bool launch_prefill_packed<int8_t>(const int8_t*, const uint32_t
                                                    hipStream_t, const RepackGuard*);
 extern template bool launch_prefill_packed<uint16_t>(const uint16_t*, const uint32_t*, uint16_t*, const Epilogue&, int, int, int, void*, size_t,
                                                      hipStream_t, const RepackGuard*);
+
+extern template void launch_mid<int8_t>(const int8_t*, const uint32_t*, uint16_t*, const Epilogue&, int, int, int, hipStream_t, const RepackGuard*);
+extern template void launch_mid<uint16_t>(const uint16_t*, const uint32_t*, uint16_t*, const Epilogue&, int, int, int, hipStream_t, const RepackGuard*);
 
 extern template PrefillPlan plan_prefill_packed<int8_t>(const void*, int, int, int, const void*, size_t);
 extern template PrefillPlan plan_prefill_packed<uint16_t>(const void*, int, int, int, const void*, size_t);

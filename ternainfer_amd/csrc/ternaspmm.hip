@@ -59,6 +59,9 @@ bool packed_small_kernel(int M, int N, int K, bool int8, bool has_scratch)
     return M <= 64;
 }
 
+// (Before this choice: calls that the kernel between the two takes, mid_kernel_takes in launch_mid.hip -- the figures above are
+// of the two kernels alone and draw the line where it does not apply.)
+
 // Scratch for split-K is worth counting on when it holds two planes of partial sums or more.
 bool scratch_for_split(const void* scratch, size_t bytes, int M, int N)
 {
@@ -81,13 +84,14 @@ struct CallPlan {
     size_t p2_bytes;           // bytes of the workspace that receive transcoded weights (CALL_TRANSCODE_LARGE)
     size_t scratch_offset;     // where split-K planes may start
     size_t scratch_bytes;      // ... and how many bytes they may take
+    bool choose;               // the kernel on the P2 copy is the library's choice: mid_kernel_takes is asked first
 };
 CallPlan plan_call(bool int8, Route route, int M, int N, int K, int split_k, const void* workspace, bool cached)
 {
     const bool ref_prefill_path = route == ROUTE_PREFILL || (route == ROUTE_AUTO && M > 64);
     const bool aligned = workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0;
     const size_t avail = aligned ? reference_workspace_bytes(ref_prefill_path, M, N, K, split_k) : 0;
-    CallPlan plan{CALL_REF_SMALL, 0, 0, 0};
+    CallPlan plan{CALL_REF_SMALL, 0, 0, 0, int8 || route == ROUTE_AUTO};
     if (cached) {
         bool small;
         if (int8) small = packed_small_kernel(M, N, K, true, scratch_for_split(workspace, avail, M, N));   // integer sums: any kernel, same bits
@@ -243,12 +247,15 @@ void run_planned(const CallPlan& plan, const Act* x, const Weights& w, const Rep
                  const Epilogue& ep, int M, int N, int K, void* workspace, hipStream_t st)
 {
     char* scratch = plan.scratch_bytes ? static_cast<char*>(workspace) + plan.scratch_offset : nullptr;
+    const bool mid = plan.choose && mid_kernel_takes(x, M, N, K, sizeof(Act));
     switch (plan.kernel) {
     case CALL_P2_SMALL:
-        launch_decode_packed<Act>(x, cached.packed, out, ep, M, N, K, st, &cached.guard);
+        if (mid) launch_mid<Act>(x, cached.packed, out, ep, M, N, K, st, &cached.guard);
+        else launch_decode_packed<Act>(x, cached.packed, out, ep, M, N, K, st, &cached.guard);
         break;
     case CALL_P2_LARGE:
-        if (!launch_prefill_packed<Act>(x, cached.packed, out, ep, M, N, K, scratch, plan.scratch_bytes, st, &cached.guard))
+        if (mid) launch_mid<Act>(x, cached.packed, out, ep, M, N, K, st, &cached.guard);
+        else if (!launch_prefill_packed<Act>(x, cached.packed, out, ep, M, N, K, scratch, plan.scratch_bytes, st, &cached.guard))
             launch_repack_guard(&cached.guard, st);
         break;
     case CALL_REF_SMALL:
@@ -256,7 +263,8 @@ void run_planned(const CallPlan& plan, const Act* x, const Weights& w, const Rep
         break;
     case CALL_TRANSCODE_LARGE:
         launch_repack(w, static_cast<uint32_t*>(workspace), N, K, st);
-        launch_prefill_packed<Act>(x, static_cast<const uint32_t*>(workspace), out, ep, M, N, K, scratch, plan.scratch_bytes, st);
+        if (mid) launch_mid<Act>(x, static_cast<const uint32_t*>(workspace), out, ep, M, N, K, st);
+        else launch_prefill_packed<Act>(x, static_cast<const uint32_t*>(workspace), out, ep, M, N, K, scratch, plan.scratch_bytes, st);
         break;
     case CALL_REF_FUSED_LARGE:
         launch_prefill<Act>(x, w, out, ep, M, N, K, st);
@@ -478,7 +486,8 @@ void bitlinear_TernaSpMM_bf16_packed_ws(const terna_bf16* x, const void* packed,
     const uint32_t* p = static_cast<const uint32_t*>(packed);
     hipStream_t st = static_cast<hipStream_t>(stream);
     const bool small = route == 2 || (route != 1 && packed_small_kernel(M, N, K, false, workspace != nullptr && workspace_bytes > 0));
-    if (small) launch_decode_packed<uint16_t>(x, p, out, ep, M, N, K, st);
+    if (route == 0 && mid_kernel_takes(x, M, N, K, sizeof(uint16_t))) launch_mid<uint16_t>(x, p, out, ep, M, N, K, st);
+    else if (small) launch_decode_packed<uint16_t>(x, p, out, ep, M, N, K, st);
     else launch_prefill_packed<uint16_t>(x, p, out, ep, M, N, K, workspace, workspace_bytes > 0 ? static_cast<size_t>(workspace_bytes) : 0, st);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) die("bitlinear_TernaSpMM_bf16_packed", e, __LINE__);
@@ -501,7 +510,8 @@ void bitlinear_TernaSpMM_packed_ws(const int8_t* x, const void* packed, terna_bf
     const uint32_t* p = static_cast<const uint32_t*>(packed);
     hipStream_t st = static_cast<hipStream_t>(stream);
     const bool small = kernel == 4 || (kernel != 8 && packed_small_kernel(M, N, K, true, workspace != nullptr && workspace_bytes > 0));
-    if (small) launch_decode_packed<int8_t>(x, p, out, ep, M, N, K, st);
+    if (kernel == 0 && mid_kernel_takes(x, M, N, K, sizeof(int8_t))) launch_mid<int8_t>(x, p, out, ep, M, N, K, st);
+    else if (small) launch_decode_packed<int8_t>(x, p, out, ep, M, N, K, st);
     else launch_prefill_packed<int8_t>(x, p, out, ep, M, N, K, workspace, workspace_bytes > 0 ? static_cast<size_t>(workspace_bytes) : 0, st);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) die("bitlinear_TernaSpMM_packed", e, __LINE__);

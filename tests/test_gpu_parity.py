@@ -830,3 +830,39 @@ def test_gpu_sleep_and_error_check(lib):
     torch.cuda.synchronize()
     assert 2.5 <= e0.elapsed_time(e1) <= 30.0
     lib.checkLastCudaError(123)
+
+
+@pytest.mark.parametrize("act", ["int8", "bf16"])
+@pytest.mark.parametrize("m,n,k", [(17, 64, 64), (32, 128, 192), (33, 2560, 320), (37, 192, 6912), (48, 3840, 2560), (100, 2560, 1088),
+                                   (64, 13824, 128), (113, 704, 2560), (300, 2560, 512), (1000, 192, 832)])
+def test_mid_kernel_against_the_forced_kernels(lib, act, m, n, k):
+    """The kernel between the small-M and the MFMA-tiled one (mid_kernel.h), which serves these calls when the library chooses:
+    each tile it has, partial last chunks, row and feature tiles that hang over, one to three scale groups; int8 bit for bit
+    against the small-M kernel and the oracle, bf16 within the family's bar of the float64 golden; an unaligned x leaves it."""
+    from ternainfer_amd import repack_weight
+    fmt = DeviceFormat(make_ternary(n, k, 0.40, 4000 + m + n + k))
+    packed = repack_weight(fmt.vals, fmt.off, fmt.med, fmt.bm, n, k)
+    groups = 3 if n == 3840 else (2 if n % 128 == 0 else 1)
+    scales = np.array([1.25, 0.75, 1.5], np.float32)[:groups]
+    print(f"[case] mid kernel {act} M={m} N={n} K={k} groups={groups}", flush=True)
+    out, forced = [torch.full((m, n), -1, dtype=torch.int16, device="cuda") for _ in range(2)]
+    if act == "int8":
+        xq, s = make_int8_activations(m, k, 4100 + m)
+        ws = O.f32_to_bf16_bits(scales)
+        xd, sd, wd = torch.from_numpy(xq).cuda(), torch.from_numpy(s.view(np.int16)).cuda(), torch.from_numpy(ws.view(np.int16)).cuda()
+        moved = torch.empty(m * k + 1, dtype=torch.int8, device="cuda")[1:].copy_(xd.reshape(-1)).view(m, k)
+        other = torch.full_like(out, -1)
+        for x, route, o in ((xd, 0, out), (xd, 4, forced), (moved, 0, other)):
+            lib.bitlinear_TernaSpMM_packed(vp(x), vp(packed), vp(o), vp(sd), vp(wd), groups, m, n, k, route, None)
+        torch.cuda.synchronize()
+        want = O.spmm_i8(xq, fmt.w, s, ws, groups, 0 if m <= 64 else 1)
+        assert (out.cpu().numpy().view(np.uint16) == want).all()
+        assert (forced.cpu().numpy().view(np.uint16) == want).all()
+        assert moved.data_ptr() % 16 != 0 and torch.equal(out, other)
+    else:
+        xb = make_bf16_activations(m, k, 4200 + m, outlier_frac=0.01)
+        xd, sd = torch.from_numpy(xb.view(np.int16)).cuda(), torch.from_numpy(scales).cuda()
+        lib.bitlinear_TernaSpMM_bf16_packed(vp(xd), vp(packed), vp(out), vp(sd), groups, m, n, k, 0, None)
+        torch.cuda.synchronize()
+        max_err, max_ref, med_ulp, _ = check_against_fp64(out.cpu().numpy().view(np.uint16), O.spmm_bf16_golden(xb, fmt.w, scales, groups))
+        assert max_err <= 1e-2 * max_ref and med_ulp <= 1, (max_err, max_ref, med_ulp)
