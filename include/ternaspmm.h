@@ -202,6 +202,16 @@ void ternaspmm_rmsnorm_quant(const terna_bf16* x, const terna_bf16* residual, te
  * supported and nothing was enqueued.  Only enqueues. */
 int ternaspmm_quant_input(const terna_bf16* x, int8_t* xq_out, terna_bf16* s_out, int M, int K, terna_stream stream);
 
+/* SpBitLinear.forward (model.py:120-133) of a few rows in one launch: quant_input of x bf16 [M][K], then the int8 linear with the
+ * decode epilogue -- the bits of ternaspmm_quant_input followed by bitlinear_TernaSpMM_packed (by bitlinear_TernaSpMM on the
+ * reference format, where it needs the cached P2 copy of the weight: see "Repack cache").  Up to 8 rows, M * K <= 28672,
+ * N <= 8192, 16-byte aligned x.  Returns 1 when the launch was enqueued, 0 when nothing was: the caller then makes the two calls. */
+int bitlinear_TernaSpMM_quant_packed(const terna_bf16* x, const void* packed, terna_bf16* out, const terna_bf16* ws, int ws_num,
+                                     int M, int N, int K, terna_stream stream);
+int bitlinear_TernaSpMM_quant(const terna_bf16* x, const uint64_t* bitmap, const int* tile_offsets_global,
+                              const uint16_t* tile_offsets_median, const uint32_t* sign_words, terna_bf16* out,
+                              const terna_bf16* ws, int ws_num, int M, int N, int K, terna_stream stream);
+
 /* Which of the reference's evaluations of SpBitLinear.quant_input (model.py:120-123) the prologue kernels above and
  * below reproduce -- its two lines leave the intermediate precision to PyTorch, and the ways of running them differ on a
  * few percent of the int8 activations (by one step):

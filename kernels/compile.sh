@@ -41,7 +41,7 @@ torch="$(python3 -c 'import os, torch; print(os.path.dirname(torch.__file__))')"
 python_include="$(python3 -c 'import sysconfig; print(sysconfig.get_paths()["include"])')"
 g++ -std=c++17 -O2 -fPIC -shared -Wall -Wno-unused-function -D__HIP_PLATFORM_AMD__=1 -DUSE_ROCM=1 \
     -isystem "$torch/include" -isystem "$torch/include/torch/csrc/api/include" -isystem "$python_include" -isystem /opt/rocm/include \
-    "$src/py_native.cpp" -L"$torch/lib" -ltorch_python -ltorch_cpu -lc10 -lc10_hip -ldl -o "$here/../ternainfer_amd/_native.so" &
+    "$src/py_native.cpp" -L"$torch/lib" -ltorch_python -ltorch_hip -ltorch_cpu -lc10 -lc10_hip -ldl -o "$here/../ternainfer_amd/_native.so" &
 pids+=($!)
 for p in "${pids[@]}"; do wait "$p"; done
 

@@ -339,6 +339,33 @@ bool launch_norm_linear_chunk(const uint16_t* x, const uint16_t* norm_w, const u
     return launch_norm_chunk_by_rows<CEPI_STORE>(a, (K / 64 + 3) / 4);
 }
 
+bool launch_quant_linear(const uint16_t* x, const uint32_t* packed, uint16_t* out, const uint16_t* ws, int ws_num, int M, int N, int K,
+                         hipStream_t st, const RepackGuard* guard)
+{
+    const int chunks = (K / 64 + 3) / 4, qm = quant_mode();
+    if (M > 8 || static_cast<long>(M) * K > kQuantLinearElements || chunks > 2 * kChunkWaves || N / 16 > 512 || static_cast<long long>(N) * K / 4 >= (1ll << 31) ||
+        (reinterpret_cast<uintptr_t>(x) & 15) != 0 || (reinterpret_cast<uintptr_t>(out) & 3) != 0)
+        return false;
+    const dim3 grid(N / 16 + (guard != nullptr ? 1 : 0)), block(kChunkWaves * 64);
+#define TERNA_QUANT_LINEAR(CT, MR)                                                                                                     \
+    do {                                                                                                                              \
+        if (guard != nullptr) terna_quant_linear_kernel<CT, MR, true><<<grid, block, 0, st>>>(x, packed, out, ws, M, N, K, ws_num, qm, *guard); \
+        else terna_quant_linear_kernel<CT, MR, false><<<grid, block, 0, st>>>(x, packed, out, ws, M, N, K, ws_num, qm, RepackGuard{});         \
+    } while (0)
+#define TERNA_QUANT_LINEAR_CT(MR)                                                                                                      \
+    do {                                                                                                                              \
+        if (chunks <= kChunkWaves) TERNA_QUANT_LINEAR(1, MR);                                                                           \
+        else TERNA_QUANT_LINEAR(2, MR);                                                                                                 \
+    } while (0)
+    if (M == 1) TERNA_QUANT_LINEAR_CT(1);
+    else if (M == 2) TERNA_QUANT_LINEAR_CT(2);
+    else if (M <= 4) TERNA_QUANT_LINEAR_CT(4);
+    else TERNA_QUANT_LINEAR_CT(8);
+#undef TERNA_QUANT_LINEAR_CT
+#undef TERNA_QUANT_LINEAR
+    return true;
+}
+
 }  // namespace terna
 
 extern "C" {

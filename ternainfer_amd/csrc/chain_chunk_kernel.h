@@ -72,34 +72,30 @@ __device__ __forceinline__ void chain_reduce_partials(const float2 (&part)[kStat
     }
 }
 
-// NE (4 or 8) columns of one row: norm + quantisation, packed int8 (NE / 4 dwords).
-template <int NE>
+// NE (4 or 8) columns of one row: norm (NORM) + quantisation, packed int8 (NE / 4 dwords).
+template <int NE, bool NORM = true>
 __device__ __forceinline__ void chain_quantise(const uint32_t (&hraw)[NE / 2], const uint32_t (&wraw)[NE / 2], float rstd, float s_mul, int quant_mode,
                                                uint32_t (&d)[NE / 4])
 {
-    float f[NE], w[NE];
+    float f[NE];
 #pragma unroll
     for (int j = 0; j < NE / 2; ++j) {
         f[2 * j] = __uint_as_float(hraw[j] << 16);
         f[2 * j + 1] = __uint_as_float(hraw[j] & 0xffff0000u);
-        w[2 * j] = __uint_as_float(wraw[j] << 16);
-        w[2 * j + 1] = __uint_as_float(wraw[j] & 0xffff0000u);
+        if constexpr (NORM) {
+            f[2 * j] = round_bf16(__fmul_rn(__fmul_rn(f[2 * j], __uint_as_float(wraw[j] << 16)), rstd));
+            f[2 * j + 1] = round_bf16(__fmul_rn(__fmul_rn(f[2 * j + 1], __uint_as_float(wraw[j] & 0xffff0000u)), rstd));
+        }
     }
 #pragma unroll
     for (int j = 0; j < NE / 4; ++j) d[j] = 0u;
     const bool eager = quant_mode == QUANT_EAGER;            // uniform: one branch, not one per element
     if (eager) {
 #pragma unroll
-        for (int e = 0; e < NE; ++e) {
-            const float y = round_bf16(__fmul_rn(__fmul_rn(f[e], w[e]), rstd));
-            d[e >> 2] = __builtin_amdgcn_cvt_pk_u8_f32(quant_value(y, s_mul, QUANT_EAGER) + 128.0f, e & 3, d[e >> 2]);
-        }
+        for (int e = 0; e < NE; ++e) d[e >> 2] = __builtin_amdgcn_cvt_pk_u8_f32(quant_value(f[e], s_mul, QUANT_EAGER) + 128.0f, e & 3, d[e >> 2]);
     } else {
 #pragma unroll
-        for (int e = 0; e < NE; ++e) {
-            const float y = round_bf16(__fmul_rn(__fmul_rn(f[e], w[e]), rstd));
-            d[e >> 2] = __builtin_amdgcn_cvt_pk_u8_f32(quant_value(y, s_mul, QUANT_ROUNDED) + 128.0f, e & 3, d[e >> 2]);
-        }
+        for (int e = 0; e < NE; ++e) d[e >> 2] = __builtin_amdgcn_cvt_pk_u8_f32(quant_value(f[e], s_mul, QUANT_ROUNDED) + 128.0f, e & 3, d[e >> 2]);
     }
 #pragma unroll
     for (int j = 0; j < NE / 4; ++j) d[j] ^= 0x80808080u;
@@ -405,19 +401,22 @@ __global__ __launch_bounds__(kChunkWaves * 64) void terna_chain_chunk_kernel(
 //   CPRO_ATTN  one row: x is the fp32 buffer a deferred-merge attention launch left (attention_kernel.h) -- per head the
 //              score maxima and sums of its ASP splits, then the splits' unnormalised results; a lane merges its four
 //              columns with attention_merge's arithmetic, so the row has the bits the merge kernel would give
+//   CPRO_PLAIN x is bf16 [M][K] and no norm stands in front of the linear (SpBitLinear on its own): only the row maximum is
+//              taken inside, the values are quantised as they are; norm_w and eps are not used
 // One band per workgroup, every wave works (unit = chunk, wave w takes chunks w, w + 16, ...).  The prologue is a chain
 // of its own here -- values, partial statistics per wave, barrier, totals, norm, quantisation -- so everything it reads
 // (cache resident) is requested by ALL waves first, then a barrier, then the weights: the vector cache returns data in
 // the order of the requests of the whole CU, and what is requested behind a weight load arrives with the weights.  The
 // chain then runs under the weights' round trip.  Sums of squares: per lane in column order, the lanes of a row pairwise
 // (group_reduce), the waves pairwise -- the same in every workgroup.
-enum ChainPrologue { CPRO_NORM, CPRO_ATTN };
+enum ChainPrologue { CPRO_NORM, CPRO_ATTN, CPRO_PLAIN };
 
-template <int PRO, int CT, int MR, int EPI, int ASP = 1, int AHD = 128>
-__global__ __launch_bounds__(kChunkWaves * 64) void terna_chain_norm_kernel(
-    const void* __restrict__ xin, const uint16_t* __restrict__ norm_w, const uint32_t* __restrict__ packed,
-    int M, int N, int K, float eps, int ws_num, int quant_mode, ChainIo io)
+template <int PRO, int CT, int MR, int EPI, int ASP, int AHD>
+__device__ __forceinline__ void chain_norm_linear(
+    const int band, const void* __restrict__ xin, const uint16_t* __restrict__ norm_w, const uint32_t* __restrict__ packed,
+    int M, int N, int K, float eps, int ws_num, int quant_mode, const ChainIo& io)
 {
+    constexpr bool NORM = PRO != CPRO_PLAIN;
     static_assert(EPI == CEPI_STORE || EPI == CEPI_RESIDUAL, "one band per workgroup");
     static_assert(MR == 1 || MR == 2 || MR == 4 || MR == 8, "rows of the slab");
     static_assert(PRO != CPRO_ATTN || MR == 1, "the attention merge feeds a single row");
@@ -438,11 +437,10 @@ __global__ __launch_bounds__(kChunkWaves * 64) void terna_chain_norm_kernel(
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int band = blockIdx.x;
     const int ktiles = K >> 6;
     const int chunks = (ktiles + 3) >> 2;
     const int i = lane & 15, g = lane >> 4;
-    const bool writer = blockIdx.x == 0;
+    const bool writer = band == 0;
     int uchunk[CT];
     bool uok[CT];
 #pragma unroll
@@ -498,7 +496,8 @@ __global__ __launch_bounds__(kChunkWaves * 64) void terna_chain_norm_kernel(
                 }
             }
             const int woff = col_ok ? xcol * 2 : kBufferOutOfRange;
-            if constexpr (NE == 8) {
+            if constexpr (!NORM) {
+            } else if constexpr (NE == 8) {
                 const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rn, woff, col0 * 2, 0));
                 nw[t][0] = v.x; nw[t][1] = v.y; nw[t][2] = v.z; nw[t][3] = v.w;
             } else {
@@ -566,6 +565,10 @@ __global__ __launch_bounds__(kChunkWaves * 64) void terna_chain_norm_kernel(
 #pragma unroll
                 for (int j = 0; j < NE / 2; ++j) {
                     const float f0 = __uint_as_float(xr[t][q][j] << 16), f1 = __uint_as_float(xr[t][q][j] & 0xffff0000u);
+                    if constexpr (!NORM) {
+                        pmx[q] = fmaxf(pmx[q], fmaxf(fabsf(f0), fabsf(f1)));
+                        continue;
+                    }
                     const float w0 = __uint_as_float(nw[t][j] << 16), w1 = __uint_as_float(nw[t][j] & 0xffff0000u);
                     pss[q] = fmaf(f0, f0, pss[q]);
                     pss[q] = fmaf(f1, f1, pss[q]);
@@ -576,7 +579,7 @@ __global__ __launch_bounds__(kChunkWaves * 64) void terna_chain_norm_kernel(
     }
 #pragma unroll
     for (int q = 0; q < XL; ++q) {
-        const float a = group_reduce<LPR, false>(pss[q]);
+        const float a = NORM ? group_reduce<LPR, false>(pss[q]) : 0.0f;
         const float b = group_reduce<LPR, true>(pmx[q]);
         if ((lane % LPR) == 0) part_s[xrow0 + RPL * q][wave] = float2{a, b};
     }
@@ -591,7 +594,7 @@ __global__ __launch_bounds__(kChunkWaves * 64) void terna_chain_norm_kernel(
         const float total = group_reduce<16, false>(v.x);
         const float pmax = group_reduce<16, true>(v.y);
         const float r = rsqrtf(total / static_cast<float>(K) + eps);
-        const float amax_y = fabsf(round_bf16(__fmul_rn(pmax, r)));          // = max |y| of the row, exactly
+        const float amax_y = NORM ? fabsf(round_bf16(__fmul_rn(pmax, r))) : pmax;          // = max |y| of the row, exactly
         uint16_t sb;
         const float s_mul = quant_scale(amax_y, quant_mode, &sb);
         if ((lane & 15) == 0 && row < MR) {
@@ -613,7 +616,7 @@ __global__ __launch_bounds__(kChunkWaves * 64) void terna_chain_norm_kernel(
             for (int q = 0; q < XL; ++q) {
                 const int row = xrow0 + RPL * q;
                 uint32_t d[NE / 4];
-                chain_quantise<NE>(xr[t][q], nw[t], stat_w[wave][row][0], stat_w[wave][row][1], quant_mode, d);
+                chain_quantise<NE, NORM>(xr[t][q], nw[t], stat_w[wave][row][0], stat_w[wave][row][1], quant_mode, d);
                 const bool pub = writer && io.xq_out != nullptr && row < M && uok[t] && col0 + xcol < K;
                 if constexpr (NE == 8) {
                     *reinterpret_cast<u32x2*>(slab + row * kChainSlabPitch + xcol) = u32x2{d[0], d[1]};
@@ -673,6 +676,33 @@ __global__ __launch_bounds__(kChunkWaves * 64) void terna_chain_norm_kernel(
             }
         }
     }
+}
+
+template <int PRO, int CT, int MR, int EPI, int ASP = 1, int AHD = 128>
+__global__ __launch_bounds__(kChunkWaves * 64) void terna_chain_norm_kernel(
+    const void* __restrict__ xin, const uint16_t* __restrict__ norm_w, const uint32_t* __restrict__ packed,
+    int M, int N, int K, float eps, int ws_num, int quant_mode, ChainIo io)
+{
+    chain_norm_linear<PRO, CT, MR, EPI, ASP, AHD>(blockIdx.x, xin, norm_w, packed, M, N, K, eps, ws_num, quant_mode, io);
+}
+
+// quant_input + int8 linear of a module call in one launch (CPRO_PLAIN), up to 8 rows.  Bound: the host -- a launch costs it
+// 3.1 us, the quantise launch and the linear behind it 2 + 3 us of the device.  GUARD: the first workgroup checks the
+// cached copy of a reference-format weight (decode_chunk_kernel.h).
+template <int CT, int MR, bool GUARD>
+__global__ __launch_bounds__(kChunkWaves * 64) void terna_quant_linear_kernel(
+    const uint16_t* __restrict__ x, const uint32_t* __restrict__ packed, uint16_t* __restrict__ out, const uint16_t* __restrict__ ws,
+    int M, int N, int K, int ws_num, int quant_mode, RepackGuard guard)
+{
+    if constexpr (GUARD) {
+        if (blockIdx.x == 0) {
+            if (threadIdx.x < 64) repack_guard_role(guard, threadIdx.x);
+            return;
+        }
+    }
+    const ChainIo io{out, ws, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+    chain_norm_linear<CPRO_PLAIN, CT, MR, CEPI_STORE, 1, 128>(static_cast<int>(blockIdx.x) - (GUARD ? 1 : 0), x, nullptr, packed, M, N, K, 0.0f, ws_num,
+                                                              quant_mode, io);
 }
 
 }  // namespace terna

@@ -94,6 +94,14 @@ bool launch_norm_linear_chunk(const uint16_t* x, const uint16_t* norm_w, const u
                               int ws_num, int8_t* xq_out, uint16_t* s_out, int M, int N, int K, float eps, int quant_mode,
                               hipStream_t st);
 
+// quant_input + int8 linear on a P2 weight in one launch (terna_quant_linear_kernel, abi_chain.hip): up to 8 rows of together
+// kQuantLinearElements elements and two workgroups per CU -- every workgroup quantises all of them (host-bound calls in a
+// row, us, two launches -> one: 2560x2560 one row 6.4 -> 3.6, 8 rows 6.4 -> 5.0; K = 6912 one row 6.4 -> 3.8, 3 rows -> 5.2;
+// gate+up with its 864 bands gains nothing).  False: not covered, nothing enqueued.
+constexpr long kQuantLinearElements = 28 * 1024;
+bool launch_quant_linear(const uint16_t* x, const uint32_t* packed, uint16_t* out, const uint16_t* ws, int ws_num, int M, int N, int K,
+                         hipStream_t st, const RepackGuard* guard = nullptr);
+
 // Tuning override shared by the two small-M launchers: TERNASPMM_DECODE_WAVES=4|8|16 forces one variant.
 int decode_waves_override();
 

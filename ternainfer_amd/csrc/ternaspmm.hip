@@ -517,6 +517,30 @@ void bitlinear_TernaSpMM_packed_ws(const int8_t* x, const void* packed, terna_bf
     if (e != hipSuccess) die("bitlinear_TernaSpMM_packed", e, __LINE__);
 }
 
+int bitlinear_TernaSpMM_quant_packed(const terna_bf16* x, const void* packed, terna_bf16* out, const terna_bf16* ws, int ws_num,
+                                     int M, int N, int K, terna_stream stream)
+{
+    if (!shape_ok(M, N, K) || !groups_ok(ws_num)) return 0;
+    if (!launch_quant_linear(x, static_cast<const uint32_t*>(packed), out, ws, ws_num, M, N, K, static_cast<hipStream_t>(stream))) return 0;
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) die("bitlinear_TernaSpMM_quant_packed", e, __LINE__);
+    return 1;
+}
+
+int bitlinear_TernaSpMM_quant(const terna_bf16* x, const uint64_t* bitmap, const int* tile_off, const uint16_t* median_off,
+                              const uint32_t* sign_words, terna_bf16* out, const terna_bf16* ws, int ws_num, int M, int N, int K,
+                              terna_stream stream)
+{
+    if (M > 8 || static_cast<long>(M) * K > kQuantLinearElements || !shape_ok(M, N, K) || !groups_ok(ws_num)) return 0;
+    const Weights w{bitmap, tile_off, median_off, sign_words};
+    RepackLaunch cached{};
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (!cached_packed(w, N, K, st, &cached, __LINE__) || !launch_quant_linear(x, cached.packed, out, ws, ws_num, M, N, K, st, &cached.guard)) return 0;
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) die("bitlinear_TernaSpMM_quant", e, __LINE__);
+    return 1;
+}
+
 void bitlinear_TernaSpMM_packed(const int8_t* x, const void* packed, terna_bf16* out, const terna_bf16* s,
                                 const terna_bf16* ws, int ws_num, int M, int N, int K, int route, terna_stream stream)
 {

@@ -92,3 +92,32 @@ def test_spbitlinear_bf16_module_and_call_site(shape, n, k, scales):
         torch.cuda.synchronize()
         assert tuple(out.shape) == tuple(shape[:-1]) + (n,)
         _check(bits(out).reshape(m, n), ref)
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 64, 64), (1, 2560, 2560), (2, 192, 8192), (3, 2560, 6912), (4, 320, 4160), (5, 3840, 320), (8, 13824, 2560),
+                                   (8, 256, 3584), (8, 256, 3648), (9, 256, 512)])
+def test_spbitlinear_few_rows_in_one_launch(m, n, k):
+    """Quantisation and linear of a few rows in one launch (terna_quant_linear_kernel; the last two cases and the widest matrix are beyond it):
+    the integer oracle's bits with a repacked weight and, through the library's cached copy, on the reference format."""
+    import ternainfer_amd as T
+    from ternainfer_amd import _lib
+    lib = _lib.load()
+    w = make_ternary(n, k, 0.40, 800 + m + n + k)
+    scales = [0.75, 1.5, 1.125] if n == 3840 else [1.375]
+    dic, ws = checkpoint_entry(w, scales)
+    x_bits = make_bf16_activations(m, k, 810 + m + k, outlier_frac=0.01)
+    x_bits[m // 2, : k // 2] = 0
+    x = torch.from_numpy(x_bits.view(np.int16)).view(torch.bfloat16).cuda()
+    print(f"[case] quantise + linear in one launch M={m} N={n} K={k}", flush=True)
+    q, s = O.quant_input(x_bits)
+    want = O.spmm_i8(q, w, s, bits(ws), len(scales), 0)
+    assert (bits(T.SpBitLinear(k, n, dic, "l", repack=True)(x)) == want).all()
+    was = lib.ternaspmm_repack_cache_enable(1)
+    try:
+        lib.ternaspmm_repack_cache_clear()
+        module = T.SpBitLinear(k, n, dic, "l")
+        for _ in range(2):                        # first sight makes the copy, both calls run on it
+            assert (bits(module(x)) == want).all()
+    finally:
+        lib.ternaspmm_repack_cache_clear()
+        lib.ternaspmm_repack_cache_enable(was)
