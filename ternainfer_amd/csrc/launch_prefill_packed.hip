@@ -2,7 +2,7 @@
 // type (-DTERNA_PREFILL_ACT=int8_t | uint16_t): the two sets of instantiations build in parallel.
 #include "launchers.h"
 #include "host_util.h"
-#include "prefill_packed_kernel.h"
+#include "prefill_deep_kernel.h"
 
 #ifndef TERNA_PREFILL_ACT
 #error "define TERNA_PREFILL_ACT (int8_t or uint16_t)"
@@ -56,9 +56,19 @@ template <typename Act, int MB, int NA>
 void launch_prefill_packed_dma_as(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M,
                                   int N, int K, const PrefillPlan& plan, void* scratch, hipStream_t st, const RepackGuard* guard)
 {
-    using S = PackedPrefillDmaSmem<MB>;
+    // Up to two workgroups of the 64 x 128 tile per CU: the kernel whose waves do not count on others (prefill_deep_kernel.h); with
+    // split-K it was level for bf16 and slower for int8 (down projection M = 512, three splits: 19.2 -> 21.9 us)
+    constexpr bool kDeep = MB == 2 && NA == 1;
+    const bool deep = kDeep && plan.splits == 1 && static_cast<long>(plan.grid_x) * plan.grid_y <= 512;
     auto kernel = terna_prefill_packed_dma_kernel<Act, MB, NA>;
-    allow_dynamic_lds(kernel, S::kBytes, "hipFuncSetAttribute(prefill packed dma)", __LINE__);
+    int lds = PackedPrefillDmaSmem<MB>::kBytes;
+    if constexpr (kDeep) {
+        if (deep) {
+            kernel = terna_prefill_deep_kernel<Act, MB, NA>;
+            lds = DeepShape<Act, MB, NA>::kBytes;
+        }
+    }
+    allow_dynamic_lds(kernel, lds, "hipFuncSetAttribute(prefill packed dma)", __LINE__);
     const int splits = plan.splits;
     // The check of a cached copy rides in the launch: as one more row of workgroups in y, or -- with split-K planes, whose
     // workgroup -> XCD pattern an extra row per plane would shift -- as the first workgroup of the reduce launch.
@@ -73,7 +83,7 @@ void launch_prefill_packed_dma_as(const Act* x, const uint32_t* packed, uint16_t
     // TERNASPMM_PREFILL_XCD_MAP=0|1 forces it off / on (tuning aid).
     const bool big_x = static_cast<size_t>(M) * K * sizeof(Act) > (4u << 20);
     const int xcd_map = (plan.grid_y % 8 == 0) && (xcd_forced < 0 ? big_x : xcd_forced != 0);
-    kernel<<<grid, dim3(256), S::kBytes, st>>>(x, packed, out, ep, M, N, K, xcd_map, splits, splits > 1 ? scratch : nullptr,
+    kernel<<<grid, dim3(256), lds, st>>>(x, packed, out, ep, M, N, K, xcd_map, splits, splits > 1 ? scratch : nullptr,
                                                guard_row ? 1 : 0, guard_row ? *guard : RepackGuard{});
     if (splits > 1) {
         using AccT = typename std::conditional<sizeof(Act) == 1, int, float>::type;

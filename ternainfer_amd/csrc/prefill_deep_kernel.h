@@ -1,0 +1,192 @@
+// The MFMA-tiled kernel for grids that leave a CU with few workgroups (prefill_packed_kernel.h has the one for full chips).
+//
+// What bounds such a launch: what one wave does in a row.  A step's matrix instructions take 256 - 512 clocks of a wave; in the
+// kernel for full chips, which counts on three more waves on the SIMD, the step of a lone wave takes 800 - 1000 clocks, because an
+// operand read waits an LDS trip for every group of matrix instructions (64 clocks of work).  Here
+//   * a step's operands are read from LDS while the step before multiplies;
+//   * a stage is 128 columns of the tile's activations (direct loads, 16-byte pieces XOR-swizzled) AND of its weights (2-bit words,
+//     1 KB per 32 features, wave-private, one direct load; one LDS read per step and operand): half as many steps and barriers
+//     for bf16, and no register ring;
+//   * one wait + barrier per step; D - 1 stages in flight (more than three bought nothing); behind the last step the last one is
+//     loaded again, so that the number of younger loads is always (D - 3) stages'.
+// Measured, us, kernel for full chips / this one, 64 x 128 tiles: QKV M = 512 bf16 17.9 / 13.1, int8 11.2 / 9.5; gate+up M = 256
+// bf16 20.2 / 19.4, int8 12.9 / 12.2; O M = 1024 bf16 19.5 / 18.1, int8 12.6 / 11.7; at 640 tiles (O M = 2048) 26.6 / 29.9.
+// Tried: matrix, LDS and vector instructions interleaved by hand (2 - 8 % slower), four more waves that only issue the loads
+// (level), 32-, 128-row and 256-feature tiles (slower in all but a few cells).
+#pragma once
+
+#include "prefill_packed_kernel.h"
+
+namespace terna {
+
+constexpr int kDeepStages = 4;
+
+template <typename Act, int MB, int NA, int D = kDeepStages>
+struct DeepShape {
+    static constexpr int kRow = 128 * static_cast<int>(sizeof(Act));     // a stage's piece of an activation row
+    static constexpr int kX = 32 * MB * kRow;
+    static constexpr int kStage = kX + 4 * NA * 1024;
+    static constexpr int kBytes = D * kStage;
+};
+
+template <typename Act, int MB, int NA, int D = kDeepStages>
+__global__ __launch_bounds__(256) void terna_prefill_deep_kernel(
+    const Act* __restrict__ x, const uint32_t* __restrict__ packed, uint16_t* __restrict__ out,
+    Epilogue ep, int M, int N, int K, int xcd_map, int splits, void* __restrict__ partial, int guard_on, RepackGuard guard)
+{
+    const int tile_rows = static_cast<int>(gridDim.y) - (guard_on ? 1 : 0);
+    if (guard_on && static_cast<int>(blockIdx.y) == tile_rows) {         // the check of a cached copy (see the other kernel)
+        if (blockIdx.x == 0 && blockIdx.z == 0 && threadIdx.x < 64) repack_guard_role(guard, threadIdx.x);
+        return;
+    }
+    using S = DeepShape<Act, MB, NA, D>;
+    constexpr bool I8 = sizeof(Act) == 1;
+    constexpr int SZ = static_cast<int>(sizeof(Act));
+    using AccV = typename std::conditional<I8, i32x16, f32x16>::type;
+    constexpr int BN = 128 * NA, BM = 32 * MB;
+    constexpr int PIECES = 8 * SZ, ROWS = 64 / PIECES;                   // 16-byte pieces of a stage row, rows per direct load
+    constexpr int XI = BM / ROWS / 4;                                     // direct loads of activations per wave and stage
+    constexpr int PER = XI + NA;
+    constexpr int GROUPS = 4 * SZ;                                        // matrix instructions per accumulator and stage
+    constexpr int TW = I8 ? 1 : 2;                                        // weight reads per 32 features and stage
+    static_assert(D >= 3 && (D - 3) * PER < 64, "vmcnt is a six-bit count");
+
+    extern __shared__ __align__(16) uint8_t smem[];
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int n_tile = blockIdx.x, m_tile = blockIdx.y;
+    if (xcd_map) {                                                        // as in the other kernel
+        const int linear = blockIdx.y * gridDim.x + blockIdx.x;
+        const int per_xcd = tile_rows >> 3;
+        const int xcd = linear & 7, idx = linear >> 3;
+        m_tile = xcd * per_xcd + idx % per_xcd;
+        n_tile = idx / per_xcd;
+    }
+    const int n0 = n_tile * BN, m0 = m_tile * BM;
+    const int ktiles = K >> 6, steps = (ktiles + 1) >> 1;
+    const bool half_tail = ktiles & 1;                                    // the last stage has one 64-column tile only
+    const int k_begin = splits > 1 ? static_cast<int>(static_cast<long>(steps) * blockIdx.z / splits) : 0;
+    const int k_end = splits > 1 ? static_cast<int>(static_cast<long>(steps) * (blockIdx.z + 1) / splits) : steps;
+    const int last_band = (N >> 4) - 1;
+    const int kb = lane >> 5, l32 = lane & 31;
+
+    // ---- this lane's place in the direct loads
+    auto swizzle = [](int row) { return I8 ? (row >> 1) & 7 : row & 15; };
+    uint32_t x_off[XI], x_back[XI], w_off[NA];
+#pragma unroll
+    for (int j = 0; j < XI; ++j) {
+        const int row = ROWS * (wave + 4 * j) + lane / PIECES;
+        const int piece = (lane % PIECES) ^ swizzle(row);
+        const int m = m0 + row < M ? m0 + row : M - 1;
+        x_off[j] = static_cast<uint32_t>(m) * static_cast<uint32_t>(K * SZ) + piece * 16;
+        x_back[j] = piece >= 4 * SZ ? 64 * SZ : 0;                        // a tile that does not exist: the one before it
+    }
+#pragma unroll
+    for (int a = 0; a < NA; ++a) {
+        int band = (n0 >> 4) + 2 * NA * wave + 2 * a + (lane >> 5);
+        band = band < last_band ? band : last_band;
+        w_off[a] = static_cast<uint32_t>(band) * static_cast<uint32_t>(ktiles) * 256u + (lane & 31) * 16;
+    }
+    const uint32_t w_back = (lane & 31) >= 16 ? 256 : 0;
+    const uint8_t* x_base = reinterpret_cast<const uint8_t*>(x);
+    const uint8_t* w_base = reinterpret_cast<const uint8_t*>(packed);
+    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem));
+    auto issue = [&](int kk, int st) __attribute__((always_inline)) {
+        const int k = kk < k_end - 1 ? kk : k_end - 1;
+        const bool back = half_tail && k == steps - 1;
+        const uint8_t* xs = x_base + static_cast<size_t>(k) * S::kRow;
+        const uint8_t* ws = w_base + static_cast<size_t>(k) * 512;
+#pragma unroll
+        for (int j = 0; j < XI; ++j) lds_dma_b128(xs, back ? x_off[j] - x_back[j] : x_off[j], lds0 + st + (wave + 4 * j) * 1024);
+#pragma unroll
+        for (int a = 0; a < NA; ++a) lds_dma_b128(ws, back ? w_off[a] - w_back : w_off[a], lds0 + st + S::kX + (wave * NA + a) * 1024);
+    };
+
+    AccV acc[NA][MB];
+#pragma unroll
+    for (int a = 0; a < NA; ++a)
+#pragma unroll
+        for (int b = 0; b < MB; ++b)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[a][b][v] = 0;
+
+    // B operand of group q, row tile b: int8 columns 64 kb + 16 q .. +15, bf16 columns 16 q + 8 kb .. +7
+    // ... and the weight words of the wave's features: everything one step multiplies, in registers
+    struct Ops { u32x4 b[GROUPS][MB], w[NA][TW]; };
+    const int b_row = l32 * S::kRow;
+    const int w_lane = S::kX + wave * NA * 1024 + (l32 >> 4) * 512 + (I8 ? kb * 256 : 0) + (l32 & 15) * 16;
+    auto load = [&](int st, auto qc, Ops& r) __attribute__((always_inline)) {
+        constexpr int q = decltype(qc)::value;
+        const int piece = (I8 ? 4 * kb + q : 2 * q + kb) ^ swizzle(l32);
+#pragma unroll
+        for (int b = 0; b < MB; ++b) r.b[q][b] = *reinterpret_cast<const u32x4*>(smem + st + b_row + b * 32 * S::kRow + piece * 16);
+        if constexpr (q % 4 == 0 && q / 4 < TW) {
+#pragma unroll
+            for (int a = 0; a < NA; ++a) r.w[a][q / 4] = *reinterpret_cast<const u32x4*>(smem + st + w_lane + a * 1024 + q / 4 * 256);
+        }
+    };
+    const int wshift = 4 - 4 * kb;
+    uint32_t wmask = kTopFieldMask;                                       // 0: the lane's (int8) or the upper groups' (bf16) tile does not exist
+    auto mma = [&](const Ops& v, auto qc) __attribute__((always_inline)) {
+        constexpr int q = decltype(qc)::value;
+#pragma unroll
+        for (int a = 0; a < NA; ++a) {
+            if constexpr (I8) {
+                const i32x4 af = expand_word_i8(v.w[a][0][q], wmask);
+#pragma unroll
+                for (int b = 0; b < MB; ++b) acc[a][b] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, __builtin_bit_cast(i32x4, v.b[q][b]), acc[a][b], 0, 0, 0);
+            } else {
+                const uint32_t word = v.w[a][q >> 2][q & 3] & (q >= 4 ? wmask : ~0u);
+                const bf16x8 af = __builtin_bit_cast(bf16x8, expand_chunk_bf16(word << wshift));
+#pragma unroll
+                for (int b = 0; b < MB; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, __builtin_bit_cast(bf16x8, v.b[q][b]), acc[a][b], 0, 0, 0);
+            }
+        }
+    };
+
+    auto next = [](int st) { return st == (D - 1) * S::kStage ? 0 : st + S::kStage; };
+#pragma unroll
+    for (int d = 0; d < D - 1; ++d) issue(k_begin + d, d * S::kStage);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((D - 2) * PER) : "memory");
+    int st_next = S::kStage, st_dma = (D - 1) * S::kStage;
+    Ops even, odd;
+    static_for<0, GROUPS>([&](auto qc) { load(0, qc, even); });
+    auto step = [&](int k, const Ops& cur, Ops& nxt) __attribute__((always_inline)) {
+        if constexpr (I8) wmask = (half_tail && k == steps - 1 && kb) ? 0u : kTopFieldMask;
+        else wmask = (half_tail && k == steps - 1) ? 0u : ~0u;
+        // own part of stage k + 1 landed; everybody's, and everybody is past the operand reads of stage k - 1
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((D - 3) * PER) : "memory");
+        issue(k + D - 1, st_dma);                                         // into the stage of step k - 1
+        static_for<0, GROUPS>([&](auto qc) {
+            __builtin_amdgcn_sched_barrier(0);                            // keeps the reads between the groups
+            load(st_next, qc, nxt);
+            mma(cur, qc);
+        });
+        __builtin_amdgcn_sched_barrier(0);
+        st_next = next(st_next);
+        st_dma = next(st_dma);
+    };
+    int k = k_begin;
+    for (; k + 1 < k_end; k += 2) {
+        step(k, even, odd);
+        step(k + 1, odd, even);
+    }
+    if (k < k_end) step(k, even, odd);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+
+    // ---- results as whole rows through LDS, in place of the stages (prefill_packed_kernel.h)
+    static_assert(4 * OutTile<NA>::kBytes <= S::kBytes && 4 * kPartialTileBytes <= S::kBytes, "output tiles fit in the stages");
+    __syncthreads();
+    if (partial != nullptr) {
+        using AccT = typename std::conditional<I8, int, float>::type;
+        packed_prefill_store_partial<MB, NA>(acc, static_cast<AccT*>(partial) + static_cast<size_t>(blockIdx.z) * M * N, M, N,
+                                             n0 + 32 * NA * wave, m0, lane, smem + wave * kPartialTileBytes);
+        return;
+    }
+    const bool rows_ok = ((reinterpret_cast<uintptr_t>(out) | (static_cast<uintptr_t>(N) * 2)) & 15) == 0;
+    packed_prefill_epilogue<MB, NA, AccV, MB * NA <= 2>(acc, out, ep, M, N, n0 + 32 * NA * wave, m0, lane,
+                                                        rows_ok ? smem + wave * OutTile<NA>::kBytes : nullptr);
+}
+
+}  // namespace terna

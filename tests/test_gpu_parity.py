@@ -866,3 +866,32 @@ def test_mid_kernel_against_the_forced_kernels(lib, act, m, n, k):
         torch.cuda.synchronize()
         max_err, max_ref, med_ulp, _ = check_against_fp64(out.cpu().numpy().view(np.uint16), O.spmm_bf16_golden(xb, fmt.w, scales, groups))
         assert max_err <= 1e-2 * max_ref and med_ulp <= 1, (max_err, max_ref, med_ulp)
+
+
+@pytest.mark.parametrize("act", ["int8", "bf16"])
+@pytest.mark.parametrize("m,n,k", [(641, 2112, 64), (1100, 1280, 128), (520, 2560, 448), (97, 13824, 192), (750, 1792, 960), (1340, 1088, 832)])
+def test_deep_tile_kernel(lib, act, m, n, k):
+    """The MFMA-tiled kernel of grids with up to two workgroups per CU (prefill_deep_kernel.h): one stage of 64 columns, one
+    whole, few and many stages, a last one of half width, row and feature tiles that hang over: int8 bit for bit against the
+    oracle, bf16 within the family's bar of the float64 golden."""
+    from ternainfer_amd import repack_weight
+    fmt = DeviceFormat(make_ternary(n, k, 0.40, 5000 + m + n + k))
+    packed = repack_weight(fmt.vals, fmt.off, fmt.med, fmt.bm, n, k)
+    groups = 2 if n % 128 == 0 else 1
+    scales = np.array([1.25, 0.75], np.float32)[:groups]
+    print(f"[case] deep tile kernel {act} M={m} N={n} K={k} groups={groups}", flush=True)
+    out = torch.full((m, n), -1, dtype=torch.int16, device="cuda")
+    if act == "int8":
+        xq, s = make_int8_activations(m, k, 5100 + m)
+        ws = O.f32_to_bf16_bits(scales)
+        xd, sd, wd = torch.from_numpy(xq).cuda(), torch.from_numpy(s.view(np.int16)).cuda(), torch.from_numpy(ws.view(np.int16)).cuda()
+        lib.bitlinear_TernaSpMM_packed(vp(xd), vp(packed), vp(out), vp(sd), vp(wd), groups, m, n, k, 0, None)
+        torch.cuda.synchronize()
+        assert (out.cpu().numpy().view(np.uint16) == O.spmm_i8(xq, fmt.w, s, ws, groups, 1)).all()
+    else:
+        xb = make_bf16_activations(m, k, 5200 + m, outlier_frac=0.01)
+        xd, sd = torch.from_numpy(xb.view(np.int16)).cuda(), torch.from_numpy(scales).cuda()
+        lib.bitlinear_TernaSpMM_bf16_packed(vp(xd), vp(packed), vp(out), vp(sd), groups, m, n, k, 0, None)
+        torch.cuda.synchronize()
+        max_err, max_ref, med_ulp, _ = check_against_fp64(out.cpu().numpy().view(np.uint16), O.spmm_bf16_golden(xb, fmt.w, scales, groups))
+        assert max_err <= 1e-2 * max_ref and med_ulp <= 1, (max_err, max_ref, med_ulp)
