@@ -331,6 +331,33 @@ def test_prefill_attention_kernels_give_the_same_bits(lib):
     assert theirs == mine, (theirs, mine)
 
 
+@pytest.mark.parametrize("b,h,kv,s_max,first,t", [(1, 4, 1, 33, 0, 33), (5, 8, 2, 64, 31, 2), (1, 20, 5, 257, 0, 257), (2, 4, 1, 700, 37, 300), (1, 8, 2, 400, 63, 161),
+                                                  (3, 12, 3, 150, 0, 145), (1, 20, 5, 1100, 0, 1090)])
+def test_wide_prefill_attention(lib, b, h, kv, s_max, first, t):
+    """Four query heads of 128 dimensions per kv head (prefill_attention_wide_kernel.h): one step, two, one more than the unrolled
+    ones; ragged query blocks and last steps; prefixes; query-block counts that are no multiple of eight, more and fewer
+    (sequence, kv head) pairs than eight."""
+    prefill_attention_case(lib, b, h, kv, 128, s_max, first, t)
+
+
+def test_wide_prefill_attention_positions_per_sequence(lib):
+    """Positions of its own for every sequence, some before the first slot, some past the last: clamped as in the other kernels."""
+    b, h, kv, d, s_max, t = 2, 8, 2, 128, 320, 270
+    q = make_bf16_activations(b * h * t, d, 731).reshape(b, h, t, d)
+    k = make_bf16_activations(b * kv * s_max, d, 732).reshape(b, kv, s_max, d)
+    v = make_bf16_activations(b * kv * s_max, d, 733).reshape(b, kv, s_max, d)
+    pos = np.stack([np.arange(t) - 5, np.arange(t) + 60]).astype(np.int64)
+    od = torch.full((b * t, h * d), 0x7FC0, dtype=torch.int16, device="cuda")
+    qd, kd, vd, pd = _dev(q), _dev(k), _dev(v), _dev(pos)
+    lib.ternaspmm_prefill_attention(_vp(qd), _vp(kd), _vp(vd), _vp(pd), 1, _vp(od), b, t, h, kv, d, s_max, float(d) ** -0.5, None)
+    torch.cuda.synchronize()
+    got = O.bf16_bits_to_f32(od.cpu().numpy().view(np.uint16)).reshape(b, t, h, d).astype(np.float64)
+    for i in range(b):
+        want = O.attention_new_tokens(q[i:i + 1], k[i:i + 1], v[i:i + 1], np.clip(pos[i], 0, s_max - 1), float(d) ** -0.5)
+        tol = 2.0 ** -7 * np.abs(want).max(axis=-1, keepdims=True) + 1e-6
+        assert (np.abs(got[i:i + 1] - want) <= tol).all()
+
+
 def _attn_workspace(lib, b, h, d):
     nbytes = lib.ternaspmm_attention_workspace_bytes(b, h, d)
     assert nbytes > 0
