@@ -61,12 +61,11 @@ void launch_mid_as(const Act* x, const uint32_t* packed, uint16_t* out, const Ep
 }  // namespace
 
 // Up to 16 rows the small-M kernels are faster (3.1 against 3.9 us).  Upwards the MFMA-tiled kernel, whose activations are
-// shared by 128 or 256 features, catches up where the outputs fill the chip several times: measured at M N = 1.3 M (QKV:
-// M = 330, O: M = 500, gate+up: M = 95); with a deep K, where it has 54 or 108 steps to do one after the other, at 1.9 M, and with
-// bf16 activations, whose rows are the most bytes here, at 1.05 M.
+// shared by 128 or 256 features, catches up where the outputs fill the chip several times: measured at M N = 1.0 - 1.25 M for both
+// types and every matrix (gate+up: M = 80, QKV: M = 300, O and down projection: M = 420 - 450).
 bool mid_kernel_takes(const void* x, int M, int N, int K, size_t act_bytes)
 {
-    const long outputs = static_cast<long>(M) * N, most = K <= 4096 ? 1300000 : (act_bytes == 2 ? 1050000 : 1900000);
+    const long outputs = static_cast<long>(M) * N, most = 1100000;
     return M > 16 && outputs <= most && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
            static_cast<uint64_t>(M) * K * act_bytes < (1ull << 31) && static_cast<uint64_t>(N) * K / 4 < (1ull << 31);
 }

@@ -29,8 +29,8 @@ void launch_prefill_packed_as(const Act* x, const uint32_t* packed, uint16_t* ou
 // family stays bit-exact: integer sums; the bf16 family sums in another order, within its tolerance).
 // Rule, from timings of the four BitNet-2B matrices at M = 128 .. 512 with 1 .. 8 splits (a step is 64 columns of bf16
 // or 128 of int8 activations): a split must keep 13 steps or more; up to 96 tiles three splits (six up to 48 tiles);
-// up to 192 tiles three splits if K gives 48 steps or more, else none (the second launch and the partial planes then
-// cost more than the shorter chains save); above that none.  Measured: down projection at M = 256 / 512, bf16
+// above that none (the second launch and the partial planes then cost more than the shorter chains save; up to 256 tiles a
+// workgroup holds two halves of K itself: down projection at M = 512, int8, 19.2 us with three splits, 15.6 so).  Measured: down projection at M = 256 / 512, bf16
 // 44.5 -> 22.5 us / 44.8 -> 29.3 us, int8 25.1 -> 17.5 / 25.9 -> 21.8; O projection at M = 256, bf16 18.6 -> 14.8.
 // TERNASPMM_PREFILL_SPLITS=1..8 forces a count (tuning aid).
 int prefill_splits(long tiles, int steps, int M, int N, size_t scratch_bytes)
@@ -45,7 +45,6 @@ int prefill_splits(long tiles, int steps, int M, int N, size_t scratch_bytes)
     if (forced) sp = forced;
     else if (tiles <= 48) sp = 6;
     else if (tiles <= 96) sp = 3;
-    else if (tiles <= 192 && steps >= 48) sp = 3;
     if (!forced && sp > steps / 13) sp = steps / 13;
     if (sp > steps) sp = steps;
     if (sp > fit) sp = fit;
@@ -61,11 +60,18 @@ void launch_prefill_packed_dma_as(const Act* x, const uint32_t* packed, uint16_t
     constexpr bool kDeep = MB == 2 && NA == 1;
     const bool deep = kDeep && plan.splits == 1 && static_cast<long>(plan.grid_x) * plan.grid_y <= 512;
     auto kernel = terna_prefill_packed_dma_kernel<Act, MB, NA>;
-    int lds = PackedPrefillDmaSmem<MB>::kBytes;
+    int lds = PackedPrefillDmaSmem<MB>::kBytes, threads = 256;
     if constexpr (kDeep) {
         if (deep) {
-            kernel = terna_prefill_deep_kernel<Act, MB, NA>;
-            lds = DeepShape<Act, MB, NA>::kBytes;
+            // up to one workgroup per CU: two halves of K in it (at two, they cost 3 - 7 us)
+            if (static_cast<long>(plan.grid_x) * plan.grid_y <= 256) {
+                kernel = terna_prefill_deep_kernel<Act, MB, NA, 2>;
+                lds = 2 * DeepShape<Act, MB, NA>::kBytes;
+                threads = 512;
+            } else {
+                kernel = terna_prefill_deep_kernel<Act, MB, NA>;
+                lds = DeepShape<Act, MB, NA>::kBytes;
+            }
         }
     }
     allow_dynamic_lds(kernel, lds, "hipFuncSetAttribute(prefill packed dma)", __LINE__);
@@ -83,7 +89,7 @@ void launch_prefill_packed_dma_as(const Act* x, const uint32_t* packed, uint16_t
     // TERNASPMM_PREFILL_XCD_MAP=0|1 forces it off / on (tuning aid).
     const bool big_x = static_cast<size_t>(M) * K * sizeof(Act) > (4u << 20);
     const int xcd_map = (plan.grid_y % 8 == 0) && (xcd_forced < 0 ? big_x : xcd_forced != 0);
-    kernel<<<grid, dim3(256), lds, st>>>(x, packed, out, ep, M, N, K, xcd_map, splits, splits > 1 ? scratch : nullptr,
+    kernel<<<grid, dim3(threads), lds, st>>>(x, packed, out, ep, M, N, K, xcd_map, splits, splits > 1 ? scratch : nullptr,
                                                guard_row ? 1 : 0, guard_row ? *guard : RepackGuard{});
     if (splits > 1) {
         using AccT = typename std::conditional<sizeof(Act) == 1, int, float>::type;

@@ -7,10 +7,14 @@
 //   * a stage is 128 columns of the tile's activations (direct loads, 16-byte pieces XOR-swizzled) AND of its weights (2-bit words,
 //     1 KB per 32 features, wave-private, one direct load; one LDS read per step and operand): half as many steps and barriers
 //     for bf16, and no register ring;
+//   * with at most one workgroup per CU it has two sets of four waves (KS = 2): each takes half of K with stages of its own, and in
+//     the end each finishes one of the two row tiles -- two waves per SIMD and half the steps in a row;
 //   * one wait + barrier per step; D - 1 stages in flight (more than three bought nothing); behind the last step the last one is
 //     loaded again, so that the number of younger loads is always (D - 3) stages'.
 // Measured, us, kernel for full chips / this one, 64 x 128 tiles: QKV M = 512 bf16 17.9 / 13.1, int8 11.2 / 9.5; gate+up M = 256
 // bf16 20.2 / 19.4, int8 12.9 / 12.2; O M = 1024 bf16 19.5 / 18.1, int8 12.6 / 11.7; at 640 tiles (O M = 2048) 26.6 / 29.9.
+// Halves of K: gate+up M = 100 int8 9.8 -> 9.0, QKV M = 400 int8 9.5 -> 8.7, bf16 12.6 -> 12.0, O M = 600 int8 9.5 -> 8.4 (at 257 - 512
+// tiles they lose 3 - 5 us).
 // Tried: matrix, LDS and vector instructions interleaved by hand (2 - 8 % slower), four more waves that only issue the loads
 // (level), 32-, 128-row and 256-feature tiles (slower in all but a few cells).
 #pragma once
@@ -29,14 +33,14 @@ struct DeepShape {
     static constexpr int kBytes = D * kStage;
 };
 
-template <typename Act, int MB, int NA, int D = kDeepStages>
-__global__ __launch_bounds__(256) void terna_prefill_deep_kernel(
+template <typename Act, int MB, int NA, int KS = 1, int D = kDeepStages>
+__global__ __launch_bounds__(256 * KS) void terna_prefill_deep_kernel(
     const Act* __restrict__ x, const uint32_t* __restrict__ packed, uint16_t* __restrict__ out,
-    Epilogue ep, int M, int N, int K, int xcd_map, int splits, void* __restrict__ partial, int guard_on, RepackGuard guard)
+    Epilogue ep, int M, int N, int K, int xcd_map, int /*splits: 1*/, void* /*partial*/, int guard_on, RepackGuard guard)
 {
     const int tile_rows = static_cast<int>(gridDim.y) - (guard_on ? 1 : 0);
     if (guard_on && static_cast<int>(blockIdx.y) == tile_rows) {         // the check of a cached copy (see the other kernel)
-        if (blockIdx.x == 0 && blockIdx.z == 0 && threadIdx.x < 64) repack_guard_role(guard, threadIdx.x);
+        if (blockIdx.x == 0 && threadIdx.x < 64) repack_guard_role(guard, threadIdx.x);
         return;
     }
     using S = DeepShape<Act, MB, NA, D>;
@@ -54,7 +58,8 @@ __global__ __launch_bounds__(256) void terna_prefill_deep_kernel(
     extern __shared__ __align__(16) uint8_t smem[];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int part = __builtin_amdgcn_readfirstlane(tid >> 8);            // of K
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3;
     int n_tile = blockIdx.x, m_tile = blockIdx.y;
     if (xcd_map) {                                                        // as in the other kernel
         const int linear = blockIdx.y * gridDim.x + blockIdx.x;
@@ -66,8 +71,9 @@ __global__ __launch_bounds__(256) void terna_prefill_deep_kernel(
     const int n0 = n_tile * BN, m0 = m_tile * BM;
     const int ktiles = K >> 6, steps = (ktiles + 1) >> 1;
     const bool half_tail = ktiles & 1;                                    // the last stage has one 64-column tile only
-    const int k_begin = splits > 1 ? static_cast<int>(static_cast<long>(steps) * blockIdx.z / splits) : 0;
-    const int k_end = splits > 1 ? static_cast<int>(static_cast<long>(steps) * (blockIdx.z + 1) / splits) : steps;
+    const int turns = (steps + KS - 1) / KS;                              // steps of a part (the last one's last may not exist)
+    const int k_begin = part * turns;
+    const int k_end = k_begin + turns < steps ? k_begin + turns : steps;
     const int last_band = (N >> 4) - 1;
     const int kb = lane >> 5, l32 = lane & 31;
 
@@ -91,7 +97,8 @@ __global__ __launch_bounds__(256) void terna_prefill_deep_kernel(
     const uint32_t w_back = (lane & 31) >= 16 ? 256 : 0;
     const uint8_t* x_base = reinterpret_cast<const uint8_t*>(x);
     const uint8_t* w_base = reinterpret_cast<const uint8_t*>(packed);
-    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem));
+    uint8_t* const stages = smem + part * S::kBytes;
+    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(stages));
     auto issue = [&](int kk, int st) __attribute__((always_inline)) {
         const int k = kk < k_end - 1 ? kk : k_end - 1;
         const bool back = half_tail && k == steps - 1;
@@ -120,10 +127,10 @@ __global__ __launch_bounds__(256) void terna_prefill_deep_kernel(
         constexpr int q = decltype(qc)::value;
         const int piece = (I8 ? 4 * kb + q : 2 * q + kb) ^ swizzle(l32);
 #pragma unroll
-        for (int b = 0; b < MB; ++b) r.b[q][b] = *reinterpret_cast<const u32x4*>(smem + st + b_row + b * 32 * S::kRow + piece * 16);
+        for (int b = 0; b < MB; ++b) r.b[q][b] = *reinterpret_cast<const u32x4*>(stages + st + b_row + b * 32 * S::kRow + piece * 16);
         if constexpr (q % 4 == 0 && q / 4 < TW) {
 #pragma unroll
-            for (int a = 0; a < NA; ++a) r.w[a][q / 4] = *reinterpret_cast<const u32x4*>(smem + st + w_lane + a * 1024 + q / 4 * 256);
+            for (int a = 0; a < NA; ++a) r.w[a][q / 4] = *reinterpret_cast<const u32x4*>(stages + st + w_lane + a * 1024 + q / 4 * 256);
         }
     };
     const int wshift = 4 - 4 * kb;
@@ -152,9 +159,12 @@ __global__ __launch_bounds__(256) void terna_prefill_deep_kernel(
     int st_next = S::kStage, st_dma = (D - 1) * S::kStage;
     Ops even, odd;
     static_for<0, GROUPS>([&](auto qc) { load(0, qc, even); });
-    auto step = [&](int k, const Ops& cur, Ops& nxt) __attribute__((always_inline)) {
+    auto set_mask = [&](int k) __attribute__((always_inline)) {
         if constexpr (I8) wmask = (half_tail && k == steps - 1 && kb) ? 0u : kTopFieldMask;
         else wmask = (half_tail && k == steps - 1) ? 0u : ~0u;
+    };
+    auto step = [&](int k, const Ops& cur, Ops& nxt) __attribute__((always_inline)) {
+        set_mask(k);
         // own part of stage k + 1 landed; everybody's, and everybody is past the operand reads of stage k - 1
         asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((D - 3) * PER) : "memory");
         issue(k + D - 1, st_dma);                                         // into the stage of step k - 1
@@ -167,24 +177,53 @@ __global__ __launch_bounds__(256) void terna_prefill_deep_kernel(
         st_next = next(st_next);
         st_dma = next(st_dma);
     };
-    int k = k_begin;
-    for (; k + 1 < k_end; k += 2) {
-        step(k, even, odd);
-        step(k + 1, odd, even);
+    // the last turn multiplies what is in registers
+    auto last_step = [&](int k, const Ops& cur) __attribute__((always_inline)) {
+        if (k >= k_end) return;                                           // uniform over the part
+        set_mask(k);
+        static_for<0, GROUPS>([&](auto qc) { mma(cur, qc); });
+    };
+    int t = 0;
+    for (; t + 2 < turns; t += 2) {
+        step(k_begin + t, even, odd);
+        step(k_begin + t + 1, odd, even);
     }
-    if (k < k_end) step(k, even, odd);
+    if (t + 1 < turns) {
+        step(k_begin + t, even, odd);
+        last_step(k_begin + t + 1, odd);
+    } else {
+        last_step(k_begin + t, even);
+    }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
     // ---- results as whole rows through LDS, in place of the stages (prefill_packed_kernel.h)
-    static_assert(4 * OutTile<NA>::kBytes <= S::kBytes && 4 * kPartialTileBytes <= S::kBytes, "output tiles fit in the stages");
+    static_assert(4 * OutTile<NA>::kBytes <= S::kBytes, "output tiles fit in the stages");
     __syncthreads();
-    if (partial != nullptr) {
-        using AccT = typename std::conditional<I8, int, float>::type;
-        packed_prefill_store_partial<MB, NA>(acc, static_cast<AccT*>(partial) + static_cast<size_t>(blockIdx.z) * M * N, M, N,
-                                             n0 + 32 * NA * wave, m0, lane, smem + wave * kPartialTileBytes);
+    const bool rows_ok = ((reinterpret_cast<uintptr_t>(out) | (static_cast<uintptr_t>(N) * 2)) & 15) == 0;
+    if constexpr (KS == 2) {
+        // each part leaves the row tile that the other one finishes
+        static_assert(KS == 1 || (MB == 2 && 4 * NA * 4096 <= S::kBytes), "two row tiles, one per part");
+        float* mine = reinterpret_cast<float*>(stages) + wave * NA * 1024 + lane;
+        const float* other = reinterpret_cast<const float*>(smem + (part ^ 1) * S::kBytes) + wave * NA * 1024 + lane;
+        AccV sum[NA][1];
+#pragma unroll
+        for (int a = 0; a < NA; ++a)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const auto give = part == 0 ? acc[a][1][v] : acc[a][0][v];
+                mine[(16 * a + v) * 64] = __builtin_bit_cast(float, give);
+                sum[a][0][v] = part == 0 ? acc[a][0][v] : acc[a][1][v];
+            }
+        __syncthreads();
+#pragma unroll
+        for (int a = 0; a < NA; ++a)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) sum[a][0][v] += __builtin_bit_cast(typename std::conditional<I8, int, float>::type, other[(16 * a + v) * 64]);
+        __syncthreads();
+        packed_prefill_epilogue<1, NA, AccV, true>(sum, out, ep, M, N, n0 + 32 * NA * wave, m0 + 32 * part, lane,
+                                                   rows_ok ? stages + wave * OutTile<NA>::kBytes : nullptr);
         return;
     }
-    const bool rows_ok = ((reinterpret_cast<uintptr_t>(out) | (static_cast<uintptr_t>(N) * 2)) & 15) == 0;
     packed_prefill_epilogue<MB, NA, AccV, MB * NA <= 2>(acc, out, ep, M, N, n0 + 32 * NA * wave, m0, lane,
                                                         rows_ok ? smem + wave * OutTile<NA>::kBytes : nullptr);
 }

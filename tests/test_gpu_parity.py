@@ -869,10 +869,12 @@ def test_mid_kernel_against_the_forced_kernels(lib, act, m, n, k):
 
 
 @pytest.mark.parametrize("act", ["int8", "bf16"])
-@pytest.mark.parametrize("m,n,k", [(641, 2112, 64), (1100, 1280, 128), (520, 2560, 448), (97, 13824, 192), (750, 1792, 960), (1340, 1088, 832)])
+@pytest.mark.parametrize("m,n,k", [(641, 2112, 64), (1100, 1280, 128), (520, 2560, 448), (97, 13824, 192), (750, 1792, 960), (1340, 1088, 832),
+                                   (900, 3328, 192), (1300, 2560, 448)])
 def test_deep_tile_kernel(lib, act, m, n, k):
-    """The MFMA-tiled kernel of grids with up to two workgroups per CU (prefill_deep_kernel.h): one stage of 64 columns, one
-    whole, few and many stages, a last one of half width, row and feature tiles that hang over: int8 bit for bit against the
+    """The MFMA-tiled kernel of grids with up to two workgroups per CU (prefill_deep_kernel.h), one with two halves of K (an odd
+    number of stages, none for the second half) and two: one stage of 64 columns, one whole, few and many stages, a last one of half
+    width, row and feature tiles that hang over: int8 bit for bit against the
     oracle, bf16 within the family's bar of the float64 golden."""
     from ternainfer_amd import repack_weight
     fmt = DeviceFormat(make_ternary(n, k, 0.40, 5000 + m + n + k))
