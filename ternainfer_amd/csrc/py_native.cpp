@@ -421,24 +421,23 @@ TERNA_FUNCTION(fused_linear, 17)
     return pack(std::move(out), std::move(stats_out), std::move(raw), std::move(xq), std::move(s));
 }
 
-// What the attention entry points read of a block's new tokens, checked against each other.
+// What the attention entry points read beside a block's new rows, checked against these and each other.
 struct AttentionArgs {
-    const at::Tensor &qkv, &cos, &sin, &pos, &ck, &cv;
+    const at::Tensor &cos, &sin, &pos, &ck, &cv;
     int64_t heads, head_dim, batch, kv, slots, t;
     float scale;
     int adjacent;
     bool each;                     // every sequence has its own positions
 
-    // a: qkv bf16 [B * T, (H + 2 KV) D], cos, sin, pos, cache_k, cache_v, heads, head_dim, scale, adjacent
-    AttentionArgs(const char* who, PyObject* const* a)
-        : qkv(*tensor(a[0])), cos(*tensor(a[1])), sin(*tensor(a[2])), pos(*tensor(a[3])), ck(*tensor(a[4])), cv(*tensor(a[5])),
-          heads(integer32(a[6])), head_dim(integer32(a[7])), scale(real(a[8])), adjacent(integer32(a[9]))
+    // a: cos, sin, pos, cache_k, cache_v, heads, head_dim, scale, adjacent; qkv is [new_rows = B * T, columns = (H + 2 KV) D]
+    AttentionArgs(const char* who, PyObject* const* a, int64_t new_rows, int64_t columns)
+        : cos(*tensor(a[0])), sin(*tensor(a[1])), pos(*tensor(a[2])), ck(*tensor(a[3])), cv(*tensor(a[4])), heads(integer32(a[5])),
+          head_dim(integer32(a[6])), scale(real(a[7])), adjacent(integer32(a[8]))
     {
-        check_matrix(who, qkv);
         if (ck.dim() != 4 || ck.sizes() != cv.sizes() || ck.size(0) < 1 || ck.size(3) != head_dim || !ck.is_contiguous() || !cv.is_contiguous())
             refuse("%s: the caches are contiguous [B, KV, S, D] tensors of one shape", who);
-        batch = ck.size(0), kv = ck.size(1), slots = ck.size(2), t = qkv.size(0) / batch;
-        if (qkv.size(0) != batch * t || qkv.size(1) != (heads + 2 * kv) * head_dim || !qkv.is_contiguous())
+        batch = ck.size(0), kv = ck.size(1), slots = ck.size(2), t = new_rows / batch;
+        if (t < 1 || new_rows != batch * t || columns != (heads + 2 * kv) * head_dim)
             refuse("%s: qkv does not have the shape of its caches", who);
         each = pos.dim() == 2;
         const int64_t rows = each ? batch * t : t;
@@ -449,32 +448,45 @@ struct AttentionArgs {
             refuse("%s: cos / sin are contiguous fp32 rows of D / 2, one per position", who);
     }
 };
-#define TERNA_ATTENTION_INPUTS(g)                                                                                      \
-    data<terna_bf16>(&(g).qkv), data<float>(&(g).cos), data<float>(&(g).sin), data<long long>(&(g).pos), (g).each
+// the leading arguments of those entry points
+#define TERNA_ATTENTION_INPUTS(qkv, g)                                                                                 \
+    qkv, data<float>(&(g).cos), data<float>(&(g).sin), data<long long>(&(g).pos), (g).each
 
-// (the ten of AttentionArgs, attention): RoPE and cache write of T new tokens per sequence, and with `attention` the multi-token
+// the new rows of an attention call
+const at::Tensor& new_rows(const char* who, PyObject* o)
+{
+    const at::Tensor& qkv = *tensor(o);
+    check_matrix(who, qkv);
+    if (!qkv.is_contiguous()) refuse("%s: qkv is a contiguous tensor", who);
+    return qkv;
+}
+
+// (qkv, the nine of AttentionArgs, attention): RoPE and cache write of T new tokens per sequence, and with `attention` the multi-token
 // attention -> bf16 [B * T, H D]; without it the rotated q [B, H, T, D]
 TERNA_FUNCTION(prompt_attention, 11)
 {
-    const AttentionArgs g("prompt_attention", a);
-    at::Tensor q = make({g.batch, g.heads, g.t, g.head_dim}, at::kBFloat16, g.qkv);
+    const char* who = "prompt_attention";
+    const at::Tensor& qkv = new_rows(who, a[0]);
+    const AttentionArgs g(who, a + 1, qkv.size(0), qkv.size(1));
+    at::Tensor q = make({g.batch, g.heads, g.t, g.head_dim}, at::kBFloat16, qkv);
     const terna_stream st = stream();
-    lib.ternaspmm_rope_kv_store(TERNA_ATTENTION_INPUTS(g), data<terna_bf16>(&q), data<terna_bf16>(&g.ck), data<terna_bf16>(&g.cv), g.batch, g.t, g.heads,
+    lib.ternaspmm_rope_kv_store(TERNA_ATTENTION_INPUTS(data<terna_bf16>(&qkv), g), data<terna_bf16>(&q), data<terna_bf16>(&g.ck), data<terna_bf16>(&g.cv), g.batch, g.t, g.heads,
                                 g.kv, g.head_dim, g.slots, g.adjacent, st);
     if (!PyObject_IsTrue(a[10])) return wrap(std::move(q));
-    at::Tensor o = make({g.batch * g.t, g.heads * g.head_dim}, at::kBFloat16, g.qkv);
+    at::Tensor o = make({g.batch * g.t, g.heads * g.head_dim}, at::kBFloat16, qkv);
     lib.ternaspmm_prefill_attention(data<terna_bf16>(&q), data<terna_bf16>(&g.ck), data<terna_bf16>(&g.cv), data<long long>(&g.pos), g.each,
                                     data<terna_bf16>(&o), g.batch, g.t, g.heads, g.kv, g.head_dim, g.slots, g.scale, st);
     return wrap(std::move(o));
 }
 
-// (the ten of AttentionArgs, workspace | None, norm_weight | None, partial | None, splits): RoPE, cache write and attention of one new
+// (qkv, the nine of AttentionArgs, workspace | None, norm_weight | None, partial | None, splits): RoPE, cache write and attention of one new
 // token per sequence -> (out bf16 [B, H D], None); with the norm's weights (out, its partial statistics [B, H, 2]); with a
 // buffer for partial results these are all that is written -> None
 TERNA_FUNCTION(decode_attention, 14)
 {
     const char* who = "decode_attention";
-    const AttentionArgs g(who, a);
+    const at::Tensor& qkv = new_rows(who, a[0]);
+    const AttentionArgs g(who, a + 1, qkv.size(0), qkv.size(1));
     const at::Tensor *workspace = tensor(a[10]), *weight = tensor(a[11]), *partial = tensor(a[12]);
     if (g.t != 1) refuse("%s: one new token per sequence", who);
     const terna_stream st = stream();
@@ -482,25 +494,106 @@ TERNA_FUNCTION(decode_attention, 14)
     if (partial != nullptr) {
         const long long need = lib.ternaspmm_attention_partial_bytes(g.batch, g.heads, g.head_dim);
         if (need < 0 || static_cast<long long>(partial->numel() * partial->element_size()) < need) refuse("%s: the partial buffer is too small", who);
-        lib.ternaspmm_rope_decode_attention_partial(TERNA_ATTENTION_INPUTS(g), ck, cv, data<float>(partial), integer32(a[13]), g.batch, g.heads, g.kv,
+        lib.ternaspmm_rope_decode_attention_partial(TERNA_ATTENTION_INPUTS(data<terna_bf16>(&qkv), g), ck, cv, data<float>(partial), integer32(a[13]), g.batch, g.heads, g.kv,
                                                     g.head_dim, g.slots, g.scale, g.adjacent, nullptr, nullptr, nullptr, 0, st);
         Py_RETURN_NONE;
     }
-    at::Tensor o = make({g.batch, g.heads * g.head_dim}, at::kBFloat16, g.qkv), stats;
+    at::Tensor o = make({g.batch, g.heads * g.head_dim}, at::kBFloat16, qkv), stats;
     if (weight != nullptr) {
         check_numel(who, "norm_weight", weight, g.heads * g.head_dim);
-        stats = make({g.batch, g.heads, 2}, at::kFloat, g.qkv);
-        if (lib.ternaspmm_rope_decode_attention_stats(TERNA_ATTENTION_INPUTS(g), ck, cv, data<terna_bf16>(&o), g.batch, g.heads, g.kv, g.head_dim, g.slots,
+        stats = make({g.batch, g.heads, 2}, at::kFloat, qkv);
+        if (lib.ternaspmm_rope_decode_attention_stats(TERNA_ATTENTION_INPUTS(data<terna_bf16>(&qkv), g), ck, cv, data<terna_bf16>(&o), g.batch, g.heads, g.kv, g.head_dim, g.slots,
                                                       g.scale, g.adjacent, data<terna_bf16>(weight), data<float>(&stats), st) != g.heads)
             refuse("%s: ternaspmm_rope_decode_attention_stats refused the launch", who);
     } else {
         if (workspace != nullptr && static_cast<long long>(workspace->numel() * workspace->element_size()) <
                                         lib.ternaspmm_attention_workspace_bytes(g.batch, g.heads, g.head_dim))
             refuse("%s: the workspace is too small", who);
-        lib.ternaspmm_rope_decode_attention(TERNA_ATTENTION_INPUTS(g), ck, cv, data<terna_bf16>(&o), g.batch, g.heads, g.kv, g.head_dim, g.slots, g.scale,
+        lib.ternaspmm_rope_decode_attention(TERNA_ATTENTION_INPUTS(data<terna_bf16>(&qkv), g), ck, cv, data<terna_bf16>(&o), g.batch, g.heads, g.kv, g.head_dim, g.slots, g.scale,
                                             g.adjacent, data(workspace), st);
     }
     return pack(std::move(o), std::move(stats));
+}
+
+// A ternary matrix of a block as four arguments: packed, ws, ws_num, out_features.
+struct BlockLinear {
+    const at::Tensor &packed, &ws;
+    int ws_num;
+    int64_t n;
+    BlockLinear(const char* who, PyObject* const* a, int64_t k) : packed(*tensor(a[0])), ws(*tensor(a[1])), ws_num(integer32(a[2])), n(integer32(a[3]))
+    {
+        check_weight(who, packed, ws, ws_num, n, k);
+    }
+};
+
+// (x, pending | None, cos, sin, pos, cache_k, cache_v, heads, head_dim, scale, adjacent, eps, attention workspace | None, linear workspace | None,
+//  attention_norm, attn_sub_norm, ffn_norm, ffn_sub_norm, wqkv [4], wo [4], w13 [4], w2 [4]) -> (stream, pending): a whole block on int8
+// activations with its norms as launches of their own (prompt pass, decode steps of many sequences): the nine launches and nothing
+// else.  Called one by one from Python they cost 53 us of host time, more than they take on the device up to a hundred tokens.
+TERNA_FUNCTION(block, 34)
+{
+    const char* who = "block";
+    const at::Tensor& x = *tensor(a[0]);
+    const at::Tensor *pending = tensor(a[1]), *attn_work = tensor(a[12]), *work = tensor(a[13]);
+    const at::Tensor *norm[4] = {tensor(a[14]), tensor(a[15]), tensor(a[16]), tensor(a[17])};
+    const int64_t heads = integer32(a[7]), head_dim = integer32(a[8]);
+    const float eps = real(a[11]);
+    check_matrix(who, x);
+    const int64_t m = x.size(0), dim = x.size(1), wide = heads * head_dim;
+    const BlockLinear qkv_w(who, a + 18, dim), o_w(who, a + 22, wide), gate_w(who, a + 26, dim), down_w(who, a + 30, gate_w.n / 2);
+    const int64_t ffn = gate_w.n / 2;
+    check_numel(who, "pending", pending, m * dim);
+    check_numel(who, "attention_norm", norm[0], dim);
+    check_numel(who, "attn_sub_norm", norm[1], wide);
+    check_numel(who, "ffn_norm", norm[2], dim);
+    check_numel(who, "ffn_sub_norm", norm[3], ffn);
+    if (!x.is_contiguous() || (pending != nullptr && !pending->is_contiguous()) || x.scalar_type() != at::kBFloat16 || o_w.n != dim || down_w.n != dim)
+        refuse("%s: the stream is a contiguous bf16 [M, dim] tensor, and the O and down projections return to it", who);
+
+    const AttentionArgs g(who, a + 2, m, qkv_w.n);
+    if (g.t == 1 && attn_work != nullptr && static_cast<long long>(attn_work->numel() * attn_work->element_size()) <
+                                                lib.ternaspmm_attention_workspace_bytes(g.batch, heads, head_dim))
+        refuse("%s: the attention workspace is too small", who);
+
+    // scratch of this call, in one piece: int8 rows and scales; then qkv, rotated queries, attention output and its projection,
+    // in whose place the gate and up outputs go
+    auto up = [](int64_t bytes) { return (bytes + 255) & ~int64_t{255}; };
+    const int64_t q_bytes = up(m * std::max(std::max(dim, wide), ffn)), s_bytes = up(2 * m), qkv_bytes = up(2 * m * qkv_w.n), wide_bytes = up(2 * m * wide);
+    const int64_t attn_bytes = qkv_bytes + 2 * wide_bytes + up(2 * m * dim);
+    const c10::DataPtr held = device_allocator()->allocate(q_bytes + s_bytes + std::max(attn_bytes, up(2 * m * gate_w.n)));
+    char* at_byte = static_cast<char*>(held.get());
+    int8_t* xq = reinterpret_cast<int8_t*>(at_byte);
+    terna_bf16* s = reinterpret_cast<terna_bf16*>(at_byte + q_bytes);
+    auto rows = [&](int64_t offset) { return reinterpret_cast<terna_bf16*>(at_byte + q_bytes + s_bytes + offset); };
+    terna_bf16 *qkv = rows(0), *q = rows(qkv_bytes), *o = rows(qkv_bytes + wide_bytes), *attn = rows(qkv_bytes + 2 * wide_bytes), *x13 = rows(0);
+
+    at::Tensor mid = make({m, dim}, at::kBFloat16, x), out = make({m, dim}, at::kBFloat16, x), first;
+    if (pending != nullptr) first = make({m, dim}, at::kBFloat16, x);
+    const terna_bf16* in = data<terna_bf16>(&x);
+    const terna_stream st = stream();
+    terna_bf16 *ck = data<terna_bf16>(&g.ck), *cv = data<terna_bf16>(&g.cv);
+    auto linear = [&](const BlockLinear& w, int64_t k, terna_bf16* to) {
+        lib.bitlinear_TernaSpMM_packed_ws(xq, data(&w.packed), to, s, data<terna_bf16>(&w.ws), w.ws_num, m, w.n, k, 0, data(work),
+                                          work != nullptr ? work->numel() : 0, st);
+    };
+    lib.ternaspmm_rmsnorm_quant(in, data<terna_bf16>(pending), pending != nullptr ? data<terna_bf16>(&first) : nullptr, data<terna_bf16>(norm[0]), eps, nullptr,
+                                xq, s, m, dim, st);
+    if (pending != nullptr) in = data<terna_bf16>(&first);
+    linear(qkv_w, dim, qkv);
+    if (g.t > 1) {
+        lib.ternaspmm_rope_kv_store(TERNA_ATTENTION_INPUTS(qkv, g), q, ck, cv, g.batch, g.t, heads, g.kv, head_dim, g.slots, g.adjacent, st);
+        lib.ternaspmm_prefill_attention(q, ck, cv, data<long long>(&g.pos), g.each, o, g.batch, g.t, heads, g.kv, head_dim, g.slots, g.scale, st);
+    } else {
+        lib.ternaspmm_rope_decode_attention(TERNA_ATTENTION_INPUTS(qkv, g), ck, cv, o, g.batch, heads, g.kv, head_dim, g.slots, g.scale, g.adjacent,
+                                            data(attn_work), st);
+    }
+    lib.ternaspmm_rmsnorm_quant(o, nullptr, nullptr, data<terna_bf16>(norm[1]), eps, nullptr, xq, s, m, wide, st);
+    linear(o_w, wide, attn);
+    lib.ternaspmm_rmsnorm_quant(in, attn, data<terna_bf16>(&mid), data<terna_bf16>(norm[2]), eps, nullptr, xq, s, m, dim, st);
+    linear(gate_w, dim, x13);
+    lib.ternaspmm_relu2_mul_rmsnorm_quant(x13, data<terna_bf16>(norm[3]), eps, nullptr, xq, s, m, ffn, st);
+    linear(down_w, ffn, data<terna_bf16>(&out));
+    return pack(std::move(mid), std::move(out));
 }
 
 // (partial, splits, heads, head_dim, norm_weight, eps, sequences, want_output) -> (xq, s, o | None), or None
@@ -569,7 +662,7 @@ TERNA_FUNCTION(init, 1)
 #define METHOD(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(name)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {METHOD(init), METHOD(bit_linear), METHOD(bit_linear_bf16), METHOD(quant_input), METHOD(linear_packed),
                          METHOD(linear_bf16_packed), METHOD(rmsnorm_quant), METHOD(relu2_mul_rmsnorm_quant), METHOD(quant_from_stats),
-                         METHOD(fused_linear), METHOD(prompt_attention), METHOD(decode_attention),
+                         METHOD(fused_linear), METHOD(prompt_attention), METHOD(decode_attention), METHOD(block),
                          METHOD(attention_merge_rmsnorm_quant), METHOD(step_inputs), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -334,11 +334,20 @@ class Block:
         bsz = cache_k.shape[0]
         t = x.shape[0] // bsz
         per_seq = int(pos_idx.dim() == 2)
+        one_token = mask is None           # the caller's rule: fused, one new token, a head size the kernel has
+        # more rows than _norm_linear's one-launch forms take: the launches of the block as one native call
+        if x.shape[0] > 8 and self.fused and self.act == "int8" and self.capture is None and \
+                (mask is KERNEL_ATTENTION or (one_token and self.prefetch is None and not isinstance(attn_ws, tuple))):
+            wqkv, wo, w13, w2 = self.wqkv, self.wo, self.w13, self.w2
+            return _lib.native().block(
+                x, pending, cos, sin, pos_idx, cache_k, cache_v, a.n_heads, a.head_dim, a.head_dim ** -0.5, int(a.rope_adjacent), a.norm_eps,
+                attn_ws, get_global_workspace(x.device) if x.shape[0] > 64 else None, self.attention_norm, self.attn_sub_norm, self.ffn_norm,
+                self.ffn_sub_norm, wqkv.packed, wqkv.ws, wqkv.ws_num, wqkv.n, wo.packed, wo.ws, wo.ws_num, wo.n, w13.packed, w13.ws, w13.ws_num, w13.n,
+                w2.packed, w2.ws, w2.ws_num, w2.n)
         qkv, x = self._norm_linear(self.wqkv, x, self.attention_norm, residual=pending, name="wqkv")
         rep = a.n_heads // a.n_kv_heads
         native = _lib.native()
         attend = (qkv, cos, sin, pos_idx, cache_k, cache_v, a.n_heads, a.head_dim, a.head_dim ** -0.5, int(a.rope_adjacent))
-        one_token = mask is None           # the caller's rule: fused, one new token, a head size the kernel has
         deferred = one_token and isinstance(attn_ws, tuple)
         if deferred:
             # the cache prefix of every head split over several workgroups that leave partial results; the O
@@ -556,9 +565,11 @@ class Transformer:
         # one new token for a few sequences: the linears chained through producer-side norm statistics (forward_chain)
         chain = one_launch_attention and self.layers[0].act == "int8" and bsz <= max(self.chain_rows, self.split_rows) and getattr(self, "chain", True) and self.chain_supported()
         stats = None
-        if chain and getattr(self, "step_inputs", True):
-            # embedding rows, their partials under the first block's norm and the RoPE rows of the positions: one launch
-            x, stats, cos, sin = step_inputs(tokens, pos_idx.reshape(-1), self.tok_embeddings, self.rope_tables(max_seq, dev), self.layers[0].attention_norm)
+        if kernels_fit and bsz * t <= 65535 and getattr(self, "step_inputs", True) and self.chain_supported():
+            # embedding rows, their partials under the first block's norm (which only the chain reads) and the RoPE rows of the
+            # positions: one launch; positions that sequences share are repeated, their first T rows are what the kernels read
+            rows = pos_idx.repeat(bsz) if bsz > 1 and t > 1 and pos_idx.dim() == 1 else pos_idx.reshape(-1)
+            x, stats, cos, sin = step_inputs(tokens, rows, self.tok_embeddings, self.rope_tables(max_seq, dev), self.layers[0].attention_norm)
         else:
             rows = self.rope_tables(max_seq, dev).index_select(0, pos_idx.reshape(-1))   # fp32 [T | B*T, 2, head_dim / 2]
             cos, sin = rows[:, 0].contiguous(), rows[:, 1].contiguous()       # views when one row

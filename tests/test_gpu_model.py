@@ -300,3 +300,28 @@ def test_converted_checkpoint_loads_and_matches_cpu_golden(tmp_path):
     err, ref = (got - want).abs().max().item(), want.abs().max().item()
     assert err <= 3e-2 * ref, (err, ref)
     assert torch.nn.functional.cosine_similarity(got.flatten(), want.flatten(), dim=0).item() > 0.999
+
+
+@pytest.mark.parametrize("batch,tokens,per_seq", [(1, 9, False), (3, 5, False), (2, 70, True), (1, 130, False), (17, 1, False), (20, 1, True)])
+def test_native_block_is_the_launches_one_by_one(batch, tokens, per_seq):
+    """Rows above the one-launch forms: a block's launches as one native call, and the step's inputs as one launch, against
+    the same launches made from Python (which recording asks for) and torch's gathers: logits and caches bit for bit."""
+    from ternainfer_amd.model import ModelArgs, Transformer
+    args = ModelArgs(dim=256, n_layers=2, n_heads=4, n_kv_heads=2, vocab_size=512, ffn_dim=384)
+    model = Transformer(args, seed=31)
+    ids = torch.randint(0, args.vocab_size, (batch, tokens), generator=torch.Generator().manual_seed(3)).cuda()
+    pos = torch.arange(tokens, device="cuda") + 4
+    if per_seq:
+        pos = pos + torch.arange(batch, device="cuda")[:, None]
+    print(f"[case] native block batch={batch} tokens={tokens} per_seq={per_seq}", flush=True)
+    results = []
+    for one_by_one in (False, True):
+        model.step_inputs = not one_by_one
+        for layer in model.layers:
+            layer.capture = [] if one_by_one else None
+        cache = model.make_cache(batch, tokens + 40)
+        with torch.inference_mode():
+            logits = model.forward(ids, cache, pos)
+        results.append([logits] + [t for pair in cache for t in pair])
+    for mine, theirs in zip(*results):
+        assert torch.equal(mine, theirs)
