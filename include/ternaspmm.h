@@ -354,6 +354,14 @@ int ternaspmm_step_inputs(const long long* tokens, const long long* pos, int per
  * rows 16j .. 16j+15 of w1, band 2j+1 <- the same rows of w3.  packed_out: N*K/4 bytes, not `packed`.  Returns 0 / -1. */
 int ternaspmm_interleave_gate_up(const void* packed, void* packed_out, int N, int K, terna_stream stream);
 
+/* The gate+up projection with its gate for more than 16 rows of int8 activations (quant_input's xq and s): out bf16 [M][N / 2] =
+ * bf16(bf16(relu(x1)^2) * x3) of the outputs x1 | x3 that bitlinear_TernaSpMM_packed gives on the matrix before it was interleaved
+ * -- the bits ternaspmm_relu2_mul_rmsnorm_quant forms from them, so that ternaspmm_rmsnorm_quant on `out` replaces it.
+ * packed: ternaspmm_interleave_gate_up's; ws = one scale, or [scale of w1, scale of w3] where N % 256 == 0; x and out 16-byte
+ * aligned.  Returns 1 when the launch was enqueued, 0 when nothing was. */
+int ternaspmm_gate_linear(const int8_t* x, const void* packed_interleaved, terna_bf16* out, const terna_bf16* s, const terna_bf16* ws,
+                          int ws_num, int M, int N, int K, terna_stream stream);
+
 /* ---- Attention-side kernels of a decode step (no counterpart in the reference's library) -----------
  * They stand where the reference calls xformers' rope_padded (model.py:218-229) and
  * fmha.memory_efficient_attention_forward (model.py:231-233).

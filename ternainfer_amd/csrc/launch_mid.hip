@@ -38,7 +38,7 @@ MidTile choose_tile(int M, int N, int K, int sz)
     return best;
 }
 
-template <typename Act, int RT, int FB>
+template <typename Act, int RT, int FB, bool GATE = false>
 void launch_mid_as(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, int waves,
                    const RepackGuard* guard, hipStream_t st)
 {
@@ -52,7 +52,7 @@ void launch_mid_as(const Act* x, const uint32_t* packed, uint16_t* out, const Ep
         allow_dynamic_lds(kernel, 160 * 1024, "hipFuncSetAttribute(mid)", __LINE__);
         kernel<<<dim3(grid + 1), block, lds, st>>>(x, packed, out, M, N, K, row_tiles, waves, ep, *guard);
     } else {
-        auto kernel = terna_mid_kernel<Act, RT, FB, false>;
+        auto kernel = terna_mid_kernel<Act, RT, FB, false, GATE>;
         allow_dynamic_lds(kernel, 160 * 1024, "hipFuncSetAttribute(mid)", __LINE__);
         kernel<<<dim3(grid), block, lds, st>>>(x, packed, out, M, N, K, row_tiles, waves, ep, RepackGuard{});
     }
@@ -78,6 +78,14 @@ void launch_mid(const Act* x, const uint32_t* packed, uint16_t* out, const Epilo
     if (t.rt == 2) launch_mid_as<Act, 2, 4>(x, packed, out, ep, M, N, K, t.waves, guard, st);
     else if (t.fb == 4) launch_mid_as<Act, 1, 4>(x, packed, out, ep, M, N, K, t.waves, guard, st);
     else launch_mid_as<Act, 1, 2>(x, packed, out, ep, M, N, K, t.waves, guard, st);
+}
+
+void launch_mid_gate(const int8_t* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, hipStream_t st)
+{
+    const MidTile t = choose_tile(M, N, K, 1);
+    if (t.rt == 2) launch_mid_as<int8_t, 2, 4, true>(x, packed, out, ep, M, N, K, t.waves, nullptr, st);
+    else if (t.fb == 4) launch_mid_as<int8_t, 1, 4, true>(x, packed, out, ep, M, N, K, t.waves, nullptr, st);
+    else launch_mid_as<int8_t, 1, 2, true>(x, packed, out, ep, M, N, K, t.waves, nullptr, st);
 }
 
 template void launch_mid<int8_t>(const int8_t*, const uint32_t*, uint16_t*, const Epilogue&, int, int, int, hipStream_t, const RepackGuard*);

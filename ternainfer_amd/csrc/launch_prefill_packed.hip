@@ -51,7 +51,7 @@ int prefill_splits(long tiles, int steps, int M, int N, size_t scratch_bytes)
     return sp < 1 ? 1 : static_cast<int>(sp);
 }
 
-template <typename Act, int MB, int NA>
+template <typename Act, int MB, int NA, bool GATE = false>
 void launch_prefill_packed_dma_as(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M,
                                   int N, int K, const PrefillPlan& plan, void* scratch, hipStream_t st, const RepackGuard* guard)
 {
@@ -59,17 +59,17 @@ void launch_prefill_packed_dma_as(const Act* x, const uint32_t* packed, uint16_t
     // split-K it was level for bf16 and slower for int8 (down projection M = 512, three splits: 19.2 -> 21.9 us)
     constexpr bool kDeep = MB == 2 && NA == 1;
     const bool deep = kDeep && plan.splits == 1 && static_cast<long>(plan.grid_x) * plan.grid_y <= 512;
-    auto kernel = terna_prefill_packed_dma_kernel<Act, MB, NA>;
+    auto kernel = terna_prefill_packed_dma_kernel<Act, MB, NA, GATE>;
     int lds = PackedPrefillDmaSmem<MB>::kBytes, threads = 256;
     if constexpr (kDeep) {
         if (deep) {
             // up to one workgroup per CU: two halves of K in it (at two, they cost 3 - 7 us)
             if (static_cast<long>(plan.grid_x) * plan.grid_y <= 256) {
-                kernel = terna_prefill_deep_kernel<Act, MB, NA, 2>;
+                kernel = terna_prefill_deep_kernel<Act, MB, NA, 2, GATE>;
                 lds = 2 * DeepShape<Act, MB, NA>::kBytes;
                 threads = 512;
             } else {
-                kernel = terna_prefill_deep_kernel<Act, MB, NA>;
+                kernel = terna_prefill_deep_kernel<Act, MB, NA, 1, GATE>;
                 lds = DeepShape<Act, MB, NA>::kBytes;
             }
         }
@@ -183,6 +183,21 @@ bool launch_prefill_packed(const Act* x, const uint32_t* packed, uint16_t* out, 
     else launch_prefill_packed_as<Act, 2>(x, packed, out, ep, M, N, K, st);
     return false;
 }
+
+template <typename Act>
+bool launch_prefill_gate(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, hipStream_t st)
+{
+    if constexpr (sizeof(Act) == 1) {
+        const PrefillPlan plan = plan_prefill_packed<Act>(x, M, N, K, nullptr, 0);
+        if (!plan.direct_lds || plan.bm != 64) return false;
+        if (plan.bn == 128) launch_prefill_packed_dma_as<Act, 2, 1, true>(x, packed, out, ep, M, N, K, plan, nullptr, st, nullptr);
+        else launch_prefill_packed_dma_as<Act, 2, 2, true>(x, packed, out, ep, M, N, K, plan, nullptr, st, nullptr);
+        return true;
+    }
+    return false;
+}
+
+template bool launch_prefill_gate<TERNA_PREFILL_ACT>(const TERNA_PREFILL_ACT*, const uint32_t*, uint16_t*, const Epilogue&, int, int, int, hipStream_t);
 
 template bool launch_prefill_packed<TERNA_PREFILL_ACT>(const TERNA_PREFILL_ACT*, const uint32_t*, uint16_t*, const Epilogue&, int, int, int,
                                                        void*, size_t, hipStream_t, const RepackGuard*);

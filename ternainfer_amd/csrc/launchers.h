@@ -46,6 +46,10 @@ bool mid_kernel_takes(const void* x, int M, int N, int K, size_t act_bytes);
 template <typename Act>
 void launch_mid(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, hipStream_t st,
                 const RepackGuard* guard = nullptr);
+// The gate+up matrix with its gate (bands of w1 and w3 interleaved, int8 activations, out [M][N / 2]): the kernels of more than 16 rows.
+void launch_mid_gate(const int8_t* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, hipStream_t st);
+template <typename Act>
+bool launch_prefill_gate(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, hipStream_t st);
 // Fingerprint of the reference-format tensors named by `guard` into *out / the check of it as a launch of its own.
 void launch_repack_fingerprint(const RepackGuard& guard, unsigned long long* out, hipStream_t st);
 void launch_repack_guard(const RepackGuard* guard, hipStream_t st);

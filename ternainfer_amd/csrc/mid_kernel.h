@@ -39,7 +39,8 @@ struct MidShape {
     static_assert(RT * FB * 1024 <= kWaveBytes, "partial sums (1 KB per 16 x 16 tile) take the place of the activations");
 };
 
-template <typename Act, int RT, int FB, bool GUARD>
+// GATE: the feed-forward gate on interleaved bands, out [M][N / 2] (packed_prefill_gate_epilogue in prefill_packed_kernel.h)
+template <typename Act, int RT, int FB, bool GUARD, bool GATE = false>
 __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
     const Act* __restrict__ x, const uint32_t* __restrict__ packed, uint16_t* __restrict__ out,
     int M, int N, int K, int row_tiles, int waves, Epilogue ep, RepackGuard guard)
@@ -180,6 +181,33 @@ __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
             *reinterpret_cast<Acc*>(mine + ((16 * r + i) * UNITS + ((4 * b + g) ^ ((i >> SWZ) & (UNITS - 1)))) * 16) = acc[r][b];
     asm volatile("" : "+v"(raw.s), "+v"(raw.w[0]), "+v"(raw.w[1]), "+v"(raw.w[2]), "+v"(raw.w[3]));
     __syncthreads();
+    if constexpr (GATE) {
+        for (int idx = tid; idx < RESULTS / 2; idx += waves * 64) {
+            const int row = idx / (UNITS / 2), u = idx % (UNITS / 2), m = m0 + row, q = 8 * (u >> 2) + (u & 3);
+            if (m >= M) break;
+            const int swz = ((row & 15) >> SWZ) & (UNITS - 1);
+            const uint8_t *from1 = smem + (row * UNITS + (q ^ swz)) * 16, *from3 = smem + (row * UNITS + ((q + 4) ^ swz)) * 16;
+            Acc x1 = *reinterpret_cast<const Acc*>(from1), x3 = *reinterpret_cast<const Acc*>(from3);
+            for (int v = 1; v < waves; ++v) {
+                x1 += *reinterpret_cast<const Acc*>(from1 + v * S::kWaveBytes);
+                x3 += *reinterpret_cast<const Acc*>(from3 + v * S::kWaveBytes);
+            }
+            EpilogueRegs e1, e3;
+            e1.s = e3.s = bf16_bits_to_float(ep.s[m]);
+            uint16_t o[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                e1.w[v] = bf16_bits_to_float(ep.ws[0]);
+                e3.w[v] = bf16_bits_to_float(ep.ws[ep.ws_num - 1]);
+                const float r = fmaxf(bf16_bits_to_float(apply_epilogue<int>(ep.kind, e1, v, x1[v] >> kI8WeightShift)), 0.0f);
+                o[v] = float_to_bf16_bits(bf16_bits_to_float(float_to_bf16_bits(r * r)) *
+                                          bf16_bits_to_float(apply_epilogue<int>(ep.kind, e3, v, x3[v] >> kI8WeightShift)));
+            }
+            *reinterpret_cast<u32x2*>(out + static_cast<size_t>(m) * (N >> 1) + band0 * 8 + 4 * u) =
+                u32x2{o[0] | (static_cast<uint32_t>(o[1]) << 16), o[2] | (static_cast<uint32_t>(o[3]) << 16)};
+        }
+        return;
+    }
     for (int idx = tid; idx < RESULTS; idx += waves * 64) {
         const int row = idx / UNITS, q = idx % UNITS, m = m0 + row, n0 = band0 * 16 + 4 * q;
         if (m >= M) break;

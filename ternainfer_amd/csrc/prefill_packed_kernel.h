@@ -69,6 +69,54 @@ __host__ __device__ inline bool epilogue_scales_per_tile(const Epilogue& ep, int
     return ep.kind == EP_I8_PREFILL || ep.ws_num == 1 || (N == 3840 && ep.ws_num == 3) || (N / ep.ws_num) % 32 == 0;
 }
 
+// The gate of a feed-forward layer on the matrix whose w1 and w3 bands are interleaved (ternaspmm_interleave_gate_up): rows 0 .. 15 of a
+// 32-feature tile are x1, rows 16 .. 31 the x3 of the same features, and a lane holds both (its values v and v + 8).  Every product is
+// rounded to bf16 where the separate launches store it.  out [M][N / 2]: half the bytes here, a quarter in the norm that
+// follows (it read both halves).  int8 family, one scale per half: see gate_linear_takes.
+template <int MB, int NA, typename AccV>
+__device__ __forceinline__ void packed_prefill_gate_epilogue(AccV (&acc)[NA][MB], uint16_t* __restrict__ out, const Epilogue& ep, int M, int N,
+                                                             int n_wave, int m0, int lane, uint8_t* tile)
+{
+    constexpr int PIECES = 2 * NA, ROW = 16 * PIECES, PER_READ = 64 / PIECES;           // a wave's 16 NA features as rows in LDS
+    const int kb = lane >> 5, l32 = lane & 31, F = N >> 1;
+    const float w1 = bf16_bits_to_float(ep.ws[0]), w3 = bf16_bits_to_float(ep.ws[ep.ws_num - 1]);
+    auto swizzle = [](int row) { return NA == 2 ? (row >> 2) & 3 : 0; };
+    auto rows = [&](auto&& element) {
+        static_for<0, MB>([&](auto bc) {
+            constexpr int b = decltype(bc)::value;
+            const int row_m = m0 + 32 * b + l32;
+            const float s = bf16_bits_to_float(ep.s[row_m < M ? row_m : M - 1]);
+            const float c1 = s != 0.0f ? __fdiv_rn(w1, s) : 0.0f, c3 = s != 0.0f ? __fdiv_rn(w3, s) : 0.0f;
+            static_for<0, 2 * NA>([&](auto tc) {
+                constexpr int a = decltype(tc)::value >> 1, vq = decltype(tc)::value & 1;
+                float h[4];
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const float x1 = element(static_cast<float>(acc[a][b][4 * vq + v] >> kI8WeightShift), s, w1, c1);
+                    const float x3 = element(static_cast<float>(acc[a][b][8 + 4 * vq + v] >> kI8WeightShift), s, w3, c3);
+                    const float r = fmaxf(bf16_bits_to_float(float_to_bf16_bits(x1)), 0.0f);
+                    h[v] = bf16_bits_to_float(float_to_bf16_bits(r * r)) * bf16_bits_to_float(float_to_bf16_bits(x3));
+                }
+                *reinterpret_cast<u32x2*>(tile + l32 * ROW + (((2 * a + vq) ^ swizzle(l32)) << 4) + 8 * kb) =
+                    u32x2{pack_bf16x2(h[0], h[1]), pack_bf16x2(h[2], h[3])};
+            });
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            const int piece = lane & (PIECES - 1), n = n_wave / 2 + 8 * piece;
+#pragma unroll
+            for (int i = 0; i < 32 / PER_READ; ++i) {
+                const int row = i * PER_READ + lane / PIECES, m = m0 + 32 * b + row;
+                const u32x4 v = *reinterpret_cast<const u32x4*>(tile + row * ROW + ((piece ^ swizzle(row)) << 4));
+                if (m < M && n < F) *reinterpret_cast<u32x4*>(out + static_cast<size_t>(m) * F + n) = v;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        });
+    };
+    if (ep.kind == EP_I8_DECODE) rows([](float x, float s, float w, float) { return __fmul_rn(__fdiv_rn(x, s), w); });
+    else rows([](float x, float, float, float c) { return __fmul_rn(x, c); });
+}
+
 // COLS = false leaves out the per-column path (scales that change inside a 32-feature tile): unrolled next to 64 - 128 live
 // accumulators it spilled up to 88 registers, so every launch of the larger tiles carried scratch memory for a path that
 // almost no call takes.  The launcher sends such calls to the 128 x 64 instantiation, which keeps the path.
@@ -442,7 +490,7 @@ struct PackedPrefillDmaSmem {
     static constexpr int kBytes = kStages * kStage;
 };
 
-template <typename Act, int MB, int NA>
+template <typename Act, int MB, int NA, bool GATE = false>
 __global__ __launch_bounds__(256, MB * NA <= 4 ? 4 : (MB * NA <= 8 ? 2 : 1)) void terna_prefill_packed_dma_kernel(
     const Act* __restrict__ x, const uint32_t* __restrict__ packed, uint16_t* __restrict__ out,
     Epilogue ep, int M, int N, int K, int xcd_map, int splits, void* __restrict__ partial, int guard_on, RepackGuard guard)
@@ -655,6 +703,10 @@ __global__ __launch_bounds__(256, MB * NA <= 4 ? 4 : (MB * NA <= 8 ? 2 : 1)) voi
         return;
     }
     // ... for the final results whenever 16-byte stores can address the output
+    if constexpr (GATE) {
+        packed_prefill_gate_epilogue<MB, NA>(acc, out, ep, M, N, n0 + 32 * NA * wave, m0, lane, smem + wave * OutTile<NA>::kBytes);
+        return;
+    }
     const bool rows_ok = ((reinterpret_cast<uintptr_t>(out) | (static_cast<uintptr_t>(N) * 2)) & 15) == 0;
     packed_prefill_epilogue<MB, NA, AccV, MB == 2 && NA == 1>(acc, out, ep, M, N, n0 + 32 * NA * wave, m0, lane,
                                                                 rows_ok ? smem + wave * OutTile<NA>::kBytes : nullptr);

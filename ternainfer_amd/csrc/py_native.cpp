@@ -30,6 +30,7 @@ namespace {
     X(bitlinear_TernaSpMM_bf16_packed_ws)                                                                              \
     X(bitlinear_TernaSpMM_quant)                                                                                       \
     X(bitlinear_TernaSpMM_quant_packed)                                                                                \
+    X(ternaspmm_gate_linear)                                                                                           \
     X(ternaspmm_quant_input)                                                                                           \
     X(ternaspmm_rmsnorm_quant)                                                                                         \
     X(ternaspmm_relu2_mul_rmsnorm_quant)                                                                               \
@@ -527,14 +528,14 @@ struct BlockLinear {
 };
 
 // (x, pending | None, cos, sin, pos, cache_k, cache_v, heads, head_dim, scale, adjacent, eps, attention workspace | None, linear workspace | None,
-//  attention_norm, attn_sub_norm, ffn_norm, ffn_sub_norm, wqkv [4], wo [4], w13 [4], w2 [4]) -> (stream, pending): a whole block on int8
+//  attention_norm, attn_sub_norm, ffn_norm, ffn_sub_norm, wqkv [4], wo [4], w13 [4], w2 [4], interleaved w13 | None) -> (stream, pending): a whole block on int8
 // activations with its norms as launches of their own (prompt pass, decode steps of many sequences): the nine launches and nothing
 // else.  Called one by one from Python they cost 53 us of host time, more than they take on the device up to a hundred tokens.
-TERNA_FUNCTION(block, 34)
+TERNA_FUNCTION(block, 35)
 {
     const char* who = "block";
     const at::Tensor& x = *tensor(a[0]);
-    const at::Tensor *pending = tensor(a[1]), *attn_work = tensor(a[12]), *work = tensor(a[13]);
+    const at::Tensor *pending = tensor(a[1]), *attn_work = tensor(a[12]), *work = tensor(a[13]), *interleaved = tensor(a[34]);
     const at::Tensor *norm[4] = {tensor(a[14]), tensor(a[15]), tensor(a[16]), tensor(a[17])};
     const int64_t heads = integer32(a[7]), head_dim = integer32(a[8]);
     const float eps = real(a[11]);
@@ -542,6 +543,7 @@ TERNA_FUNCTION(block, 34)
     const int64_t m = x.size(0), dim = x.size(1), wide = heads * head_dim;
     const BlockLinear qkv_w(who, a + 18, dim), o_w(who, a + 22, wide), gate_w(who, a + 26, dim), down_w(who, a + 30, gate_w.n / 2);
     const int64_t ffn = gate_w.n / 2;
+    if (interleaved != nullptr) check_weight(who, *interleaved, gate_w.ws, gate_w.ws_num, gate_w.n, dim);
     check_numel(who, "pending", pending, m * dim);
     check_numel(who, "attention_norm", norm[0], dim);
     check_numel(who, "attn_sub_norm", norm[1], wide);
@@ -590,8 +592,12 @@ TERNA_FUNCTION(block, 34)
     lib.ternaspmm_rmsnorm_quant(o, nullptr, nullptr, data<terna_bf16>(norm[1]), eps, nullptr, xq, s, m, wide, st);
     linear(o_w, wide, attn);
     lib.ternaspmm_rmsnorm_quant(in, attn, data<terna_bf16>(&mid), data<terna_bf16>(norm[2]), eps, nullptr, xq, s, m, dim, st);
-    linear(gate_w, dim, x13);
-    lib.ternaspmm_relu2_mul_rmsnorm_quant(x13, data<terna_bf16>(norm[3]), eps, nullptr, xq, s, m, ffn, st);
+    if (interleaved != nullptr && lib.ternaspmm_gate_linear(xq, data(interleaved), x13, s, data<terna_bf16>(&gate_w.ws), gate_w.ws_num, m, gate_w.n, dim, st)) {
+        lib.ternaspmm_rmsnorm_quant(x13, nullptr, nullptr, data<terna_bf16>(norm[3]), eps, nullptr, xq, s, m, ffn, st);
+    } else {
+        linear(gate_w, dim, x13);
+        lib.ternaspmm_relu2_mul_rmsnorm_quant(x13, data<terna_bf16>(norm[3]), eps, nullptr, xq, s, m, ffn, st);
+    }
     linear(down_w, ffn, data<terna_bf16>(&out));
     return pack(std::move(mid), std::move(out));
 }

@@ -517,6 +517,24 @@ void bitlinear_TernaSpMM_packed_ws(const int8_t* x, const void* packed, terna_bf
     if (e != hipSuccess) die("bitlinear_TernaSpMM_packed", e, __LINE__);
 }
 
+int ternaspmm_gate_linear(const int8_t* x, const void* packed, terna_bf16* out, const terna_bf16* s, const terna_bf16* ws, int ws_num,
+                          int M, int N, int K, terna_stream stream)
+{
+    // one scale per half under both epilogue rules (their groups end at N / 2, a whole number of 128 columns); up to 16 rows the
+    // fused linear's gate is the faster one
+    const bool scales_ok = N != 3840 && (ws_num == 1 || (ws_num == 2 && N % 256 == 0));
+    if (M <= 16 || N < 64 || K < 64 || (N % 64) || (K % 64) || !scales_ok || ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out)) & 15)) return 0;
+    if (!shape_ok(M, N, K) || !i8_depth_ok(K)) return 0;
+    const Epilogue ep{s, ws, nullptr, ws_num, M <= 64 ? EP_I8_DECODE : EP_I8_PREFILL};
+    const uint32_t* p = static_cast<const uint32_t*>(packed);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (mid_kernel_takes(x, M, N, K, sizeof(int8_t))) launch_mid_gate(x, p, out, ep, M, N, K, st);
+    else if (!launch_prefill_gate<int8_t>(x, p, out, ep, M, N, K, st)) return 0;
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) die("ternaspmm_gate_linear", e, __LINE__);
+    return 1;
+}
+
 int bitlinear_TernaSpMM_quant_packed(const terna_bf16* x, const void* packed, terna_bf16* out, const terna_bf16* ws, int ws_num,
                                      int M, int N, int K, terna_stream stream)
 {

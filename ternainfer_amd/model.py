@@ -343,7 +343,8 @@ class Block:
                 x, pending, cos, sin, pos_idx, cache_k, cache_v, a.n_heads, a.head_dim, a.head_dim ** -0.5, int(a.rope_adjacent), a.norm_eps,
                 attn_ws, get_global_workspace(x.device) if x.shape[0] > 64 else None, self.attention_norm, self.attn_sub_norm, self.ffn_norm,
                 self.ffn_sub_norm, wqkv.packed, wqkv.ws, wqkv.ws_num, wqkv.n, wo.packed, wo.ws, wo.ws_num, wo.n, w13.packed, w13.ws, w13.ws_num, w13.n,
-                w2.packed, w2.ws, w2.ws_num, w2.n)
+                w2.packed, w2.ws, w2.ws_num, w2.n,
+                self.gate_up_interleaved())
         qkv, x = self._norm_linear(self.wqkv, x, self.attention_norm, residual=pending, name="wqkv")
         rep = a.n_heads // a.n_kv_heads
         native = _lib.native()

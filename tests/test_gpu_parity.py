@@ -897,3 +897,34 @@ def test_deep_tile_kernel(lib, act, m, n, k):
         torch.cuda.synchronize()
         max_err, max_ref, med_ulp, _ = check_against_fp64(out.cpu().numpy().view(np.uint16), O.spmm_bf16_golden(xb, fmt.w, scales, groups))
         assert max_err <= 1e-2 * max_ref and med_ulp <= 1, (max_err, max_ref, med_ulp)
+
+
+@pytest.mark.parametrize("m,f,k,groups", [(17, 32, 64, 1), (33, 6912, 128, 2), (64, 384, 2560, 2), (65, 384, 320, 1), (130, 1152, 192, 2), (97, 6912, 192, 2),
+                                          (700, 1664, 448, 2), (2100, 5504, 64, 2), (1500, 6912, 192, 2)])
+def test_gate_linear(lib, m, f, k, groups):
+    """The gate+up projection with its gate in the epilogue, in every kernel of more than 16 rows and at their tiles' edges:
+    the bits of squared_relu(x1) * x3 in bf16 on the oracle's outputs, scale rules of both row counts, one scale and two."""
+    from ternainfer_amd import repack_weight
+    from ternainfer_amd.linear import interleave_gate_up
+    n = 2 * f
+    fmt = DeviceFormat(make_ternary(n, k, 0.40, 6000 + m + n + k))
+    packed = interleave_gate_up(repack_weight(fmt.vals, fmt.off, fmt.med, fmt.bm, n, k), n, k)
+    xq, s = make_int8_activations(m, k, 6100 + m)
+    ws = O.f32_to_bf16_bits(np.array([1.25, 0.75], np.float32)[:groups])
+    xd, sd, wd = torch.from_numpy(xq).cuda(), torch.from_numpy(s.view(np.int16)).cuda(), torch.from_numpy(ws.view(np.int16)).cuda()
+    out = torch.zeros((m, f), dtype=torch.bfloat16, device="cuda")
+    print(f"[case] gate linear M={m} F={f} K={k} groups={groups}", flush=True)
+    assert lib.ternaspmm_gate_linear(vp(xd), vp(packed), vp(out), vp(sd), vp(wd), groups, m, n, k, None) == 1
+    torch.cuda.synchronize()
+    x13 = torch.from_numpy(O.spmm_i8(xq, fmt.w, s, ws, groups, 0 if m <= 64 else 1).view(np.int16)).view(torch.bfloat16)
+    want = torch.relu(x13[:, :f]).square() * x13[:, f:]
+    assert torch.equal(out.cpu().view(torch.int16), want.view(torch.int16)) or torch.equal(out.cpu(), want)
+
+
+def test_gate_linear_refuses(lib):
+    """Few rows, a half that is no whole number of 128 columns with two scales, an unaligned x: nothing is enqueued."""
+    x = torch.zeros(64 * 64 + 1, dtype=torch.int8, device="cuda")
+    p, out, s = torch.zeros(64 * 320, dtype=torch.int8, device="cuda"), torch.zeros(64 * 160, dtype=torch.bfloat16, device="cuda"), torch.ones(64, dtype=torch.bfloat16, device="cuda")
+    assert lib.ternaspmm_gate_linear(vp(x), vp(p), vp(out), vp(s), vp(s), 1, 16, 256, 64, None) == 0
+    assert lib.ternaspmm_gate_linear(vp(x), vp(p), vp(out), vp(s), vp(s), 2, 32, 320, 64, None) == 0
+    assert lib.ternaspmm_gate_linear(vp(x[1:]), vp(p), vp(out), vp(s), vp(s), 1, 32, 256, 64, None) == 0
