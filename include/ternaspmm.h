@@ -354,6 +354,16 @@ int ternaspmm_step_inputs(const long long* tokens, const long long* pos, int per
  * rows 16j .. 16j+15 of w1, band 2j+1 <- the same rows of w3.  packed_out: N*K/4 bytes, not `packed`.  Returns 0 / -1. */
 int ternaspmm_interleave_gate_up(const void* packed, void* packed_out, int N, int K, terna_stream stream);
 
+/* The QKV projection of a prompt pass (more than 16 rows of int8 activations) with ternaspmm_rope_kv_store in its epilogue, adjacent
+ * pairs: out bf16 [M][N], N = (H + 2 KV) D, row b * T + t, of which the H * D columns of the queries are written, rotated; rotated
+ * keys and values go into the caches (bf16 [B][KV][S][D], B = M / T) at the tokens' slots; the other columns of out stay as they
+ * are.  The bits of bitlinear_TernaSpMM_packed followed by ternaspmm_rope_kv_store (arguments as there); ternaspmm_prefill_attention_rows
+ * reads such an output.  x, out and the caches 16-byte aligned; scale groups of whole 32 columns.  Returns 1 when the launch
+ * was enqueued, 0 when nothing was. */
+int ternaspmm_qkv_rope_linear(const int8_t* x, const void* packed, terna_bf16* out, const terna_bf16* s, const terna_bf16* ws, int ws_num,
+                              int M, int N, int K, const float* cos, const float* sin, const long long* pos, int per_sequence,
+                              terna_bf16* cache_k, terna_bf16* cache_v, int T, int H, int KV, int D, int S, terna_stream stream);
+
 /* The gate+up projection with its gate for more than 16 rows of int8 activations (quant_input's xq and s): out bf16 [M][N / 2] =
  * bf16(bf16(relu(x1)^2) * x3) of the outputs x1 | x3 that bitlinear_TernaSpMM_packed gives on the matrix before it was interleaved
  * -- the bits ternaspmm_relu2_mul_rmsnorm_quant forms from them, so that ternaspmm_rmsnorm_quant on `out` replaces it.
@@ -405,6 +415,12 @@ void ternaspmm_decode_attention(const terna_bf16* q, const terna_bf16* cache_k, 
 void ternaspmm_prefill_attention(const terna_bf16* q, const terna_bf16* cache_k, const terna_bf16* cache_v,
                                  const long long* pos, int per_sequence, terna_bf16* out, int B, int T, int H, int KV, int D, int S,
                                  float scale, terna_stream stream);
+/* The same with the queries as the leading H * D columns of rows of `row` elements (bf16 [B * T][row]; ternaspmm_qkv_rope_linear's
+ * output).  Four query heads per kv head and D = 128 only, row a multiple of 8: returns 1 when the launch was enqueued, 0 when
+ * nothing was. */
+int ternaspmm_prefill_attention_rows(const terna_bf16* q_rows, int row, const terna_bf16* cache_k, const terna_bf16* cache_v,
+                                     const long long* pos, int per_sequence, terna_bf16* out, int B, int T, int H, int KV, int D,
+                                     int S, float scale, terna_stream stream);
 
 /* ternaspmm_decode_attention for callers that cannot allocate or bring a workspace (code under HIP graph capture
  * that owns no buffers, tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.

@@ -78,6 +78,8 @@ PROTOTYPES = {
     "ternaspmm_repack_cache_limit": ([ctypes.c_longlong], ctypes.c_longlong),
     "ternaspmm_repack_cache_stats": ([_vp], None),
     "ternaspmm_plan_reference_call": ([_ci] * 6 + [_vp, _ci, _vp], _ci),
+    "ternaspmm_qkv_rope_linear": ([_vp] * 5 + [_ci] * 4 + [_vp] * 3 + [_ci] + [_vp] * 2 + [_ci] * 5 + [_vp], _ci),
+    "ternaspmm_prefill_attention_rows": ([_vp, _ci] + [_vp] * 3 + [_ci, _vp] + [_ci] * 6 + [ctypes.c_float, _vp], _ci),
     "ternaspmm_gate_linear": ([_vp] * 5 + [_ci] * 4 + [_vp], _ci),
     "bitlinear_TernaSpMM_quant_packed": ([_vp, _vp, _vp, _vp, _ci, _ci, _ci, _ci, _vp], _ci),
     "bitlinear_TernaSpMM_quant": ([_vp] * 7 + [_ci] * 4 + [_vp], _ci),

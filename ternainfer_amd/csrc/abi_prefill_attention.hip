@@ -37,7 +37,7 @@ void ternaspmm_prefill_attention(const terna_bf16* q, const terna_bf16* cache_k,
     if (!group_off && D == 128 && G == 4)
         // measured faster at every length and batch, from 1 x 2 tokens (2.9 against 3.7 us) to 2 x 2048
         terna_prefill_attention_wide_kernel<<<dim3(8u * B * KV * ((T + 127) / 128)), dim3(256), 0, st>>>(q, cache_k, cache_v, pos, out, B, T, H, KV, S,
-                                                                                                         scale, ps);
+                                                                                                         scale, ps, 0);
 #define TERNA_GROUP_ATTN(DD, GG) \
     terna_prefill_attention_group_kernel<DD, GG><<<ggrid, dim3(64 * GG), 0, st>>>(q, cache_k, cache_v, pos, out, T, H, KV, S, scale, ps)
     else if (!group_off && D == 128 && G == 8) TERNA_GROUP_ATTN(128, 8);
@@ -55,6 +55,18 @@ void ternaspmm_prefill_attention(const terna_bf16* q, const terna_bf16* cache_k,
     }
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) die("ternaspmm_prefill_attention", e, __LINE__);
+}
+
+int ternaspmm_prefill_attention_rows(const terna_bf16* q_rows, int row, const terna_bf16* cache_k, const terna_bf16* cache_v,
+                                     const long long* pos, int per_sequence, terna_bf16* out, int B, int T, int H, int KV, int D, int S,
+                                     float scale, terna_stream stream)
+{
+    if (B < 1 || T < 1 || H < 1 || KV < 1 || H != 4 * KV || D != 128 || S < 1 || S > 8192 || B > 65535 || row < H * D || (row & 7)) return 0;
+    terna_prefill_attention_wide_kernel<<<dim3(8u * B * KV * ((T + 127) / 128)), dim3(256), 0, static_cast<hipStream_t>(stream)>>>(
+        q_rows, cache_k, cache_v, pos, out, B, T, H, KV, S, scale, per_sequence != 0, row);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) die("ternaspmm_prefill_attention_rows", e, __LINE__);
+    return 1;
 }
 
 }  // extern "C"

@@ -38,24 +38,36 @@ MidTile choose_tile(int M, int N, int K, int sz)
     return best;
 }
 
-template <typename Act, int RT, int FB, bool GATE = false>
+template <typename Act, int RT, int FB, int EPI = PACKED_STORE>
 void launch_mid_as(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, int waves,
-                   const RepackGuard* guard, hipStream_t st)
+                   const PackedExtra<EPI>* extra, hipStream_t st)
 {
     using S = MidShape<Act, RT, FB>;
     const int row_tiles = (M + 16 * RT - 1) / (16 * RT), feature_tiles = (N / 16 + FB - 1) / FB;
     const unsigned grid = static_cast<unsigned>((feature_tiles + 7) / 8 * 8 * row_tiles);
     const dim3 block(waves * 64);
     const int lds = waves * S::kWaveBytes;
-    if (guard != nullptr) {
-        auto kernel = terna_mid_kernel<Act, RT, FB, true>;
-        allow_dynamic_lds(kernel, 160 * 1024, "hipFuncSetAttribute(mid)", __LINE__);
-        kernel<<<dim3(grid + 1), block, lds, st>>>(x, packed, out, M, N, K, row_tiles, waves, ep, *guard);
-    } else {
-        auto kernel = terna_mid_kernel<Act, RT, FB, false, GATE>;
-        allow_dynamic_lds(kernel, 160 * 1024, "hipFuncSetAttribute(mid)", __LINE__);
-        kernel<<<dim3(grid), block, lds, st>>>(x, packed, out, M, N, K, row_tiles, waves, ep, RepackGuard{});
+    if constexpr (EPI == PACKED_STORE) {
+        if (extra != nullptr) {
+            auto kernel = terna_mid_kernel<Act, RT, FB, true>;
+            allow_dynamic_lds(kernel, 160 * 1024, "hipFuncSetAttribute(mid)", __LINE__);
+            kernel<<<dim3(grid + 1), block, lds, st>>>(x, packed, out, M, N, K, row_tiles, waves, ep, *extra);
+            return;
+        }
     }
+    auto kernel = terna_mid_kernel<Act, RT, FB, false, EPI>;
+    allow_dynamic_lds(kernel, 160 * 1024, "hipFuncSetAttribute(mid)", __LINE__);
+    kernel<<<dim3(grid), block, lds, st>>>(x, packed, out, M, N, K, row_tiles, waves, ep, extra != nullptr ? *extra : PackedExtra<EPI>{});
+}
+
+template <typename Act, int EPI>
+void launch_mid_tile(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, hipStream_t st,
+                     const PackedExtra<EPI>* extra)
+{
+    const MidTile t = choose_tile(M, N, K, sizeof(Act));
+    if (t.rt == 2) launch_mid_as<Act, 2, 4, EPI>(x, packed, out, ep, M, N, K, t.waves, extra, st);
+    else if (t.fb == 4) launch_mid_as<Act, 1, 4, EPI>(x, packed, out, ep, M, N, K, t.waves, extra, st);
+    else launch_mid_as<Act, 1, 2, EPI>(x, packed, out, ep, M, N, K, t.waves, extra, st);
 }
 
 }  // namespace
@@ -74,18 +86,16 @@ template <typename Act>
 void launch_mid(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, hipStream_t st,
                 const RepackGuard* guard)
 {
-    const MidTile t = choose_tile(M, N, K, sizeof(Act));
-    if (t.rt == 2) launch_mid_as<Act, 2, 4>(x, packed, out, ep, M, N, K, t.waves, guard, st);
-    else if (t.fb == 4) launch_mid_as<Act, 1, 4>(x, packed, out, ep, M, N, K, t.waves, guard, st);
-    else launch_mid_as<Act, 1, 2>(x, packed, out, ep, M, N, K, t.waves, guard, st);
+    launch_mid_tile<Act, PACKED_STORE>(x, packed, out, ep, M, N, K, st, guard);
 }
 
 void launch_mid_gate(const int8_t* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, hipStream_t st)
 {
-    const MidTile t = choose_tile(M, N, K, 1);
-    if (t.rt == 2) launch_mid_as<int8_t, 2, 4, true>(x, packed, out, ep, M, N, K, t.waves, nullptr, st);
-    else if (t.fb == 4) launch_mid_as<int8_t, 1, 4, true>(x, packed, out, ep, M, N, K, t.waves, nullptr, st);
-    else launch_mid_as<int8_t, 1, 2, true>(x, packed, out, ep, M, N, K, t.waves, nullptr, st);
+    launch_mid_tile<int8_t, PACKED_GATE>(x, packed, out, ep, M, N, K, st, nullptr);
+}
+void launch_mid_rope(const int8_t* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, const RopeStore& rope, hipStream_t st)
+{
+    launch_mid_tile<int8_t, PACKED_ROPE>(x, packed, out, ep, M, N, K, st, &rope);
 }
 
 template void launch_mid<int8_t>(const int8_t*, const uint32_t*, uint16_t*, const Epilogue&, int, int, int, hipStream_t, const RepackGuard*);

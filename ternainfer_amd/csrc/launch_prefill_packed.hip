@@ -51,25 +51,25 @@ int prefill_splits(long tiles, int steps, int M, int N, size_t scratch_bytes)
     return sp < 1 ? 1 : static_cast<int>(sp);
 }
 
-template <typename Act, int MB, int NA, bool GATE = false>
+template <typename Act, int MB, int NA, int EPI = PACKED_STORE>
 void launch_prefill_packed_dma_as(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M,
-                                  int N, int K, const PrefillPlan& plan, void* scratch, hipStream_t st, const RepackGuard* guard)
+                                  int N, int K, const PrefillPlan& plan, void* scratch, hipStream_t st, const PackedExtra<EPI>* guard)
 {
     // Up to two workgroups of the 64 x 128 tile per CU: the kernel whose waves do not count on others (prefill_deep_kernel.h); with
     // split-K it was level for bf16 and slower for int8 (down projection M = 512, three splits: 19.2 -> 21.9 us)
     constexpr bool kDeep = MB == 2 && NA == 1;
     const bool deep = kDeep && plan.splits == 1 && static_cast<long>(plan.grid_x) * plan.grid_y <= 512;
-    auto kernel = terna_prefill_packed_dma_kernel<Act, MB, NA, GATE>;
+    auto kernel = terna_prefill_packed_dma_kernel<Act, MB, NA, EPI>;
     int lds = PackedPrefillDmaSmem<MB>::kBytes, threads = 256;
     if constexpr (kDeep) {
         if (deep) {
             // up to one workgroup per CU: two halves of K in it (at two, they cost 3 - 7 us)
             if (static_cast<long>(plan.grid_x) * plan.grid_y <= 256) {
-                kernel = terna_prefill_deep_kernel<Act, MB, NA, 2, GATE>;
+                kernel = terna_prefill_deep_kernel<Act, MB, NA, 2, EPI>;
                 lds = 2 * DeepShape<Act, MB, NA>::kBytes;
                 threads = 512;
             } else {
-                kernel = terna_prefill_deep_kernel<Act, MB, NA, 1, GATE>;
+                kernel = terna_prefill_deep_kernel<Act, MB, NA, 1, EPI>;
                 lds = DeepShape<Act, MB, NA>::kBytes;
             }
         }
@@ -78,7 +78,7 @@ void launch_prefill_packed_dma_as(const Act* x, const uint32_t* packed, uint16_t
     const int splits = plan.splits;
     // The check of a cached copy rides in the launch: as one more row of workgroups in y, or -- with split-K planes, whose
     // workgroup -> XCD pattern an extra row per plane would shift -- as the first workgroup of the reduce launch.
-    const bool guard_row = guard != nullptr && splits == 1;
+    const bool guard_row = EPI == PACKED_STORE && guard != nullptr && splits == 1;
     const dim3 grid(plan.grid_x, plan.grid_y + (guard_row ? 1 : 0), plan.splits);
     static const int xcd_forced = [] {
         const char* v = tuning_env("TERNASPMM_PREFILL_XCD_MAP");
@@ -90,8 +90,8 @@ void launch_prefill_packed_dma_as(const Act* x, const uint32_t* packed, uint16_t
     const bool big_x = static_cast<size_t>(M) * K * sizeof(Act) > (4u << 20);
     const int xcd_map = (plan.grid_y % 8 == 0) && (xcd_forced < 0 ? big_x : xcd_forced != 0);
     kernel<<<grid, dim3(threads), lds, st>>>(x, packed, out, ep, M, N, K, xcd_map, splits, splits > 1 ? scratch : nullptr,
-                                               guard_row ? 1 : 0, guard_row ? *guard : RepackGuard{});
-    if (splits > 1) {
+                                               guard_row ? 1 : 0, guard_row || (EPI == PACKED_ROPE && guard != nullptr) ? *guard : PackedExtra<EPI>{});
+    if constexpr (EPI == PACKED_STORE) if (splits > 1) {
         using AccT = typename std::conditional<sizeof(Act) == 1, int, float>::type;
         const long quads = static_cast<long>(M) * (N >> 2);
         const bool guard_first = guard != nullptr;
@@ -184,20 +184,33 @@ bool launch_prefill_packed(const Act* x, const uint32_t* packed, uint16_t* out, 
     return false;
 }
 
-template <typename Act>
-bool launch_prefill_gate(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, hipStream_t st)
+template <int EPI, typename Act>
+bool launch_prefill_producer(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, const PackedExtra<EPI>* extra,
+                             hipStream_t st)
 {
     if constexpr (sizeof(Act) == 1) {
         const PrefillPlan plan = plan_prefill_packed<Act>(x, M, N, K, nullptr, 0);
         if (!plan.direct_lds || plan.bm != 64) return false;
-        if (plan.bn == 128) launch_prefill_packed_dma_as<Act, 2, 1, true>(x, packed, out, ep, M, N, K, plan, nullptr, st, nullptr);
-        else launch_prefill_packed_dma_as<Act, 2, 2, true>(x, packed, out, ep, M, N, K, plan, nullptr, st, nullptr);
+        if (plan.bn == 128) launch_prefill_packed_dma_as<Act, 2, 1, EPI>(x, packed, out, ep, M, N, K, plan, nullptr, st, extra);
+        else launch_prefill_packed_dma_as<Act, 2, 2, EPI>(x, packed, out, ep, M, N, K, plan, nullptr, st, extra);
         return true;
     }
     return false;
 }
+template <typename Act>
+bool launch_prefill_gate(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, hipStream_t st)
+{
+    return launch_prefill_producer<PACKED_GATE>(x, packed, out, ep, M, N, K, nullptr, st);
+}
+template <typename Act>
+bool launch_prefill_rope(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, const RopeStore& rope, hipStream_t st)
+{
+    return launch_prefill_producer<PACKED_ROPE>(x, packed, out, ep, M, N, K, &rope, st);
+}
 
 template bool launch_prefill_gate<TERNA_PREFILL_ACT>(const TERNA_PREFILL_ACT*, const uint32_t*, uint16_t*, const Epilogue&, int, int, int, hipStream_t);
+template bool launch_prefill_rope<TERNA_PREFILL_ACT>(const TERNA_PREFILL_ACT*, const uint32_t*, uint16_t*, const Epilogue&, int, int, int, const RopeStore&,
+                                                     hipStream_t);
 
 template bool launch_prefill_packed<TERNA_PREFILL_ACT>(const TERNA_PREFILL_ACT*, const uint32_t*, uint16_t*, const Epilogue&, int, int, int,
                                                        void*, size_t, hipStream_t, const RepackGuard*);

@@ -50,6 +50,10 @@ void launch_mid(const Act* x, const uint32_t* packed, uint16_t* out, const Epilo
 void launch_mid_gate(const int8_t* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, hipStream_t st);
 template <typename Act>
 bool launch_prefill_gate(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, hipStream_t st);
+// The QKV projection of a prompt pass with RoPE and the cache write: the same kernels.
+void launch_mid_rope(const int8_t* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, const RopeStore& rope, hipStream_t st);
+template <typename Act>
+bool launch_prefill_rope(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, const RopeStore& rope, hipStream_t st);
 // Fingerprint of the reference-format tensors named by `guard` into *out / the check of it as a launch of its own.
 void launch_repack_fingerprint(const RepackGuard& guard, unsigned long long* out, hipStream_t st);
 void launch_repack_guard(const RepackGuard* guard, hipStream_t st);

@@ -39,11 +39,11 @@ struct MidShape {
     static_assert(RT * FB * 1024 <= kWaveBytes, "partial sums (1 KB per 16 x 16 tile) take the place of the activations");
 };
 
-// GATE: the feed-forward gate on interleaved bands, out [M][N / 2] (packed_prefill_gate_epilogue in prefill_packed_kernel.h)
-template <typename Act, int RT, int FB, bool GUARD, bool GATE = false>
+// EPI: plain outputs, the feed-forward gate or the rotary embedding and cache write (see the epilogues of prefill_packed_kernel.h)
+template <typename Act, int RT, int FB, bool GUARD, int EPI = PACKED_STORE>
 __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
     const Act* __restrict__ x, const uint32_t* __restrict__ packed, uint16_t* __restrict__ out,
-    int M, int N, int K, int row_tiles, int waves, Epilogue ep, RepackGuard guard)
+    int M, int N, int K, int row_tiles, int waves, Epilogue ep, PackedExtra<EPI> guard)
 {
     if constexpr (GUARD) {
         if (blockIdx.x == 0) {
@@ -162,6 +162,17 @@ __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
     const int fin_m = m0 + tid / UNITS;
     const bool fin = tid < RESULTS && fin_m < M;
     EpilogueRaw raw = load_epilogue_raw_flat<BF16>(ep, fin ? fin_m : 0, band0 * 16 + 4 * (tid % UNITS), N);
+    float2 turn_c = {1.0f, 1.0f}, turn_s = {0.0f, 0.0f};
+    uint16_t* turn_to = nullptr;
+    auto load_turn = [&](int m, int n0) __attribute__((always_inline)) {
+        if constexpr (EPI == PACKED_ROPE) {
+            const int table_row = guard.table_row(m);
+            turn_c = guard.angles2(guard.cos, table_row, n0);
+            turn_s = guard.angles2(guard.sin, table_row, n0);
+            turn_to = guard.place(out, m, n0, N);
+        }
+    };
+    if (fin) load_turn(fin_m, band0 * 16 + 4 * (tid % UNITS));
     for (int chunk = wave;;) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
@@ -181,7 +192,7 @@ __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
             *reinterpret_cast<Acc*>(mine + ((16 * r + i) * UNITS + ((4 * b + g) ^ ((i >> SWZ) & (UNITS - 1)))) * 16) = acc[r][b];
     asm volatile("" : "+v"(raw.s), "+v"(raw.w[0]), "+v"(raw.w[1]), "+v"(raw.w[2]), "+v"(raw.w[3]));
     __syncthreads();
-    if constexpr (GATE) {
+    if constexpr (EPI == PACKED_GATE) {
         for (int idx = tid; idx < RESULTS / 2; idx += waves * 64) {
             const int row = idx / (UNITS / 2), u = idx % (UNITS / 2), m = m0 + row, q = 8 * (u >> 2) + (u & 3);
             if (m >= M) break;
@@ -221,6 +232,13 @@ __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
         for (int v = 0; v < 4; ++v) {
             if constexpr (BF16) o[v] = apply_epilogue<float>(EP_BF16, e, v, static_cast<AccScalar>(sum[v] * kBf16WeightUndo));
             else o[v] = apply_epilogue<int>(ep.kind, e, v, sum[v] >> kI8WeightShift);
+        }
+        if constexpr (EPI == PACKED_ROPE) {
+            if (idx != tid) load_turn(m, n0);
+            u32x2 turned = {o[0] | (static_cast<uint32_t>(o[1]) << 16), o[2] | (static_cast<uint32_t>(o[3]) << 16)};
+            if (guard.part(n0) < 2) turned = u32x2{RopeStore::rotate(turned.x, turn_c.x, turn_s.x), RopeStore::rotate(turned.y, turn_c.y, turn_s.y)};
+            if (turn_to != nullptr) *reinterpret_cast<u32x2*>(turn_to) = turned;
+            continue;
         }
         *reinterpret_cast<u32x2*>(out + static_cast<size_t>(m) * N + n0) =
             u32x2{o[0] | (static_cast<uint32_t>(o[1]) << 16), o[2] | (static_cast<uint32_t>(o[3]) << 16)};

@@ -48,7 +48,7 @@ __device__ __forceinline__ float wide_groups_reduce(float v)
 
 __global__ __launch_bounds__(256, 2) void terna_prefill_attention_wide_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ cache_k, const uint16_t* __restrict__ cache_v,
-    const long long* __restrict__ pos, uint16_t* __restrict__ out, int B, int T, int H, int KV, int S, float scale, int per_seq)
+    const long long* __restrict__ pos, uint16_t* __restrict__ out, int B, int T, int H, int KV, int S, float scale, int per_seq, int q_row)
 {
 // as in the other kernels: the bits have to be theirs
 #pragma clang fp contract(off)
@@ -84,10 +84,13 @@ __global__ __launch_bounds__(256, 2) void terna_prefill_attention_wide_kernel(
     n_full = __builtin_amdgcn_readfirstlane(n_full);
     const int steps = (n_keys + KB - 1) / KB;
 
+    // q [B][H][T][D], or rows of q_row elements (q_row != 0)
+    const uint16_t* qrow = q + (q_row ? (static_cast<size_t>(b) * T + t) * q_row + static_cast<size_t>(h) * D
+                                      : ((static_cast<size_t>(b) * H + h) * T + t) * D);
     bf16x8 bq[DS];
 #pragma unroll
     for (int ds = 0; ds < DS; ++ds)
-        bq[ds] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(q + ((static_cast<size_t>(b) * H + h) * T + t) * D + 32 * ds + 8 * g));
+        bq[ds] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(qrow + 32 * ds + 8 * g));
 #pragma unroll
     for (int ds = 0; ds < DS; ++ds) asm volatile("" : "+v"(bq[ds]));   // landed before the first hand-issued request
 

@@ -33,15 +33,17 @@ struct DeepShape {
     static constexpr int kBytes = D * kStage;
 };
 
-template <typename Act, int MB, int NA, int KS = 1, bool GATE = false, int D = kDeepStages>
+template <typename Act, int MB, int NA, int KS = 1, int EPI = PACKED_STORE, int D = kDeepStages>
 __global__ __launch_bounds__(256 * KS) void terna_prefill_deep_kernel(
     const Act* __restrict__ x, const uint32_t* __restrict__ packed, uint16_t* __restrict__ out,
-    Epilogue ep, int M, int N, int K, int xcd_map, int /*splits: 1*/, void* /*partial*/, int guard_on, RepackGuard guard)
+    Epilogue ep, int M, int N, int K, int xcd_map, int /*splits: 1*/, void* /*partial*/, int guard_on, PackedExtra<EPI> guard)
 {
     const int tile_rows = static_cast<int>(gridDim.y) - (guard_on ? 1 : 0);
-    if (guard_on && static_cast<int>(blockIdx.y) == tile_rows) {         // the check of a cached copy (see the other kernel)
-        if (blockIdx.x == 0 && threadIdx.x < 64) repack_guard_role(guard, threadIdx.x);
-        return;
+    if constexpr (EPI == PACKED_STORE) {
+        if (guard_on && static_cast<int>(blockIdx.y) == tile_rows) {     // the check of a cached copy (see the other kernel)
+            if (blockIdx.x == 0 && threadIdx.x < 64) repack_guard_role(guard, threadIdx.x);
+            return;
+        }
     }
     using S = DeepShape<Act, MB, NA, D>;
     constexpr bool I8 = sizeof(Act) == 1;
@@ -220,16 +222,24 @@ __global__ __launch_bounds__(256 * KS) void terna_prefill_deep_kernel(
 #pragma unroll
             for (int v = 0; v < 16; ++v) sum[a][0][v] += __builtin_bit_cast(typename std::conditional<I8, int, float>::type, other[(16 * a + v) * 64]);
         __syncthreads();
-        if constexpr (GATE) {
+        if constexpr (EPI == PACKED_GATE) {
             packed_prefill_gate_epilogue<1, NA>(sum, out, ep, M, N, n0 + 32 * NA * wave, m0 + 32 * part, lane, stages + wave * OutTile<NA>::kBytes);
+            return;
+        }
+        if constexpr (EPI == PACKED_ROPE) {
+            packed_prefill_rope_epilogue<1, NA>(sum, out, ep, guard, M, N, n0 + 32 * NA * wave, m0 + 32 * part, lane, stages + wave * OutTile<NA>::kBytes);
             return;
         }
         packed_prefill_epilogue<1, NA, AccV, true>(sum, out, ep, M, N, n0 + 32 * NA * wave, m0 + 32 * part, lane,
                                                    rows_ok ? stages + wave * OutTile<NA>::kBytes : nullptr);
         return;
     }
-    if constexpr (GATE) {
+    if constexpr (EPI == PACKED_GATE) {
         packed_prefill_gate_epilogue<MB, NA>(acc, out, ep, M, N, n0 + 32 * NA * wave, m0, lane, smem + wave * OutTile<NA>::kBytes);
+        return;
+    }
+    if constexpr (EPI == PACKED_ROPE) {
+        packed_prefill_rope_epilogue<MB, NA>(acc, out, ep, guard, M, N, n0 + 32 * NA * wave, m0, lane, smem + wave * OutTile<NA>::kBytes);
         return;
     }
     packed_prefill_epilogue<MB, NA, AccV, MB * NA <= 2>(acc, out, ep, M, N, n0 + 32 * NA * wave, m0, lane,

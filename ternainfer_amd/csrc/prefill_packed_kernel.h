@@ -117,6 +117,75 @@ __device__ __forceinline__ void packed_prefill_gate_epilogue(AccV (&acc)[NA][MB]
     else rows([](float x, float, float, float c) { return __fmul_rn(x, c); });
 }
 
+template <int MB, int NA, typename AccV>
+__device__ __forceinline__ void packed_prefill_rope_epilogue(AccV (&acc)[NA][MB], uint16_t* __restrict__ out, const Epilogue& ep, const RopeStore& rope,
+                                                             int M, int N, int n_wave, int m0, int lane, uint8_t* tile)
+{
+    using OT = OutTile<NA>;
+    const int kb = lane >> 5, l32 = lane & 31;
+    if (n_wave >= N) return;
+    const bool turn = rope.part(n_wave) < 2;     // a wave's 32 NA features belong to one head
+    float w_of[NA];
+    static_for<0, NA>([&](auto ac) {
+        constexpr int a = decltype(ac)::value;
+        const int g = ep.ws_num == 1 ? 0 : (ep.kind == EP_I8_PREFILL ? ws_group_prefill(n_wave + 32 * a, N, ep.ws_num) : ws_group_decode(n_wave + 32 * a, N, ep.ws_num));
+        w_of[a] = bf16_bits_to_float(ep.ws[g]);
+    });
+    const int piece = lane & (OT::kPieces - 1), n = n_wave + 8 * piece;
+    static_for<0, MB>([&](auto bc) {
+        constexpr int b = decltype(bc)::value;
+        // requested first: the angles of the pairs that this lane turns and stores, whole rows of them (by accumulator, a lane's
+        // pairs are gathered from 32 rows four times as often: 5 us of a launch of 25)
+        f32x4 c[OT::kReads], sn[OT::kReads];
+        uint16_t* to[OT::kReads];
+#pragma unroll
+        for (int i = 0; i < OT::kReads; ++i) {
+            const int m = m0 + 32 * b + i * OT::kRowsPerRead + lane / OT::kPieces;
+            const int row = rope.table_row(m < M ? m : M - 1);
+            c[i] = rope.angles4(rope.cos, row, n);
+            sn[i] = rope.angles4(rope.sin, row, n);
+            to[i] = m < M ? rope.place(out, m, n, N) : nullptr;
+        }
+        const int m = m0 + 32 * b + l32 < M ? m0 + 32 * b + l32 : M - 1;
+        const float s = bf16_bits_to_float(ep.s[m]);
+        static_for<0, NA>([&](auto ac) {
+            constexpr int a = decltype(ac)::value;
+            const float coeff = s != 0.0f ? __fdiv_rn(w_of[a], s) : 0.0f;
+            static_for<0, 4>([&](auto vc) {
+                constexpr int vq = decltype(vc)::value;
+                float x[4];
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const float sum = static_cast<float>(acc[a][b][4 * vq + v] >> kI8WeightShift);
+                    x[v] = ep.kind == EP_I8_DECODE ? __fmul_rn(__fdiv_rn(sum, s), w_of[a]) : __fmul_rn(sum, coeff);
+                }
+                *reinterpret_cast<u32x2*>(tile + l32 * OT::kRowBytes + 8 * kb + (((4 * a + vq) ^ OT::swizzle(l32)) << 4)) =
+                    u32x2{pack_bf16x2(x[0], x[1]), pack_bf16x2(x[2], x[3])};
+            });
+        });
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int i = 0; i < OT::kReads; ++i) {
+            const int row_in = i * OT::kRowsPerRead + lane / OT::kPieces;
+            u32x4 v = *reinterpret_cast<const u32x4*>(tile + row_in * OT::kRowBytes + ((piece ^ OT::swizzle(row_in)) << 4));
+            if (turn) {
+#pragma unroll
+                for (int p = 0; p < 4; ++p) v[p] = RopeStore::rotate(v[p], c[i][p], sn[i][p]);
+            }
+            if (to[i] != nullptr) *reinterpret_cast<u32x4*>(to[i]) = v;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    });
+}
+
+// What a kernel does with its sums, and what it is handed for it in the place of the check of a cached copy (which rides along
+// with plain outputs only).
+enum PackedEpilogue { PACKED_STORE, PACKED_GATE, PACKED_ROPE };
+template <int EPI>
+using PackedExtra = typename std::conditional<EPI == PACKED_ROPE, RopeStore, RepackGuard>::type;
+
 // COLS = false leaves out the per-column path (scales that change inside a 32-feature tile): unrolled next to 64 - 128 live
 // accumulators it spilled up to 88 registers, so every launch of the larger tiles carried scratch memory for a path that
 // almost no call takes.  The launcher sends such calls to the 128 x 64 instantiation, which keeps the path.
@@ -490,18 +559,20 @@ struct PackedPrefillDmaSmem {
     static constexpr int kBytes = kStages * kStage;
 };
 
-template <typename Act, int MB, int NA, bool GATE = false>
+template <typename Act, int MB, int NA, int EPI = PACKED_STORE>
 __global__ __launch_bounds__(256, MB * NA <= 4 ? 4 : (MB * NA <= 8 ? 2 : 1)) void terna_prefill_packed_dma_kernel(
     const Act* __restrict__ x, const uint32_t* __restrict__ packed, uint16_t* __restrict__ out,
-    Epilogue ep, int M, int N, int K, int xcd_map, int splits, void* __restrict__ partial, int guard_on, RepackGuard guard)
+    Epilogue ep, int M, int N, int K, int xcd_map, int splits, void* __restrict__ partial, int guard_on, PackedExtra<EPI> guard)
 {
     // guard_on: the launch runs on a cached copy of a caller's weight and carries one extra row of workgroups in y, the
     // first of which checks the copy's fingerprint next to the others (a launch of its own cost 1.5 - 2 us per call: 11 %
     // of a step at M = 256); the rest of that row leaves at once.
     const int tile_rows = static_cast<int>(gridDim.y) - (guard_on ? 1 : 0);
-    if (guard_on && static_cast<int>(blockIdx.y) == tile_rows) {
-        if (blockIdx.x == 0 && blockIdx.z == 0 && threadIdx.x < 64) repack_guard_role(guard, threadIdx.x);
-        return;
+    if constexpr (EPI == PACKED_STORE) {
+        if (guard_on && static_cast<int>(blockIdx.y) == tile_rows) {
+            if (blockIdx.x == 0 && blockIdx.z == 0 && threadIdx.x < 64) repack_guard_role(guard, threadIdx.x);
+            return;
+        }
     }
     using S = PackedPrefillDmaSmem<MB>;
     constexpr int BN = 128 * NA, BM = S::BM;
@@ -703,8 +774,12 @@ __global__ __launch_bounds__(256, MB * NA <= 4 ? 4 : (MB * NA <= 8 ? 2 : 1)) voi
         return;
     }
     // ... for the final results whenever 16-byte stores can address the output
-    if constexpr (GATE) {
+    if constexpr (EPI == PACKED_GATE) {
         packed_prefill_gate_epilogue<MB, NA>(acc, out, ep, M, N, n0 + 32 * NA * wave, m0, lane, smem + wave * OutTile<NA>::kBytes);
+        return;
+    }
+    if constexpr (EPI == PACKED_ROPE) {
+        packed_prefill_rope_epilogue<MB, NA>(acc, out, ep, guard, M, N, n0 + 32 * NA * wave, m0, lane, smem + wave * OutTile<NA>::kBytes);
         return;
     }
     const bool rows_ok = ((reinterpret_cast<uintptr_t>(out) | (static_cast<uintptr_t>(N) * 2)) & 15) == 0;

@@ -30,6 +30,8 @@ namespace {
     X(bitlinear_TernaSpMM_bf16_packed_ws)                                                                              \
     X(bitlinear_TernaSpMM_quant)                                                                                       \
     X(bitlinear_TernaSpMM_quant_packed)                                                                                \
+    X(ternaspmm_qkv_rope_linear)                                                                                       \
+    X(ternaspmm_prefill_attention_rows)                                                                                \
     X(ternaspmm_gate_linear)                                                                                           \
     X(ternaspmm_quant_input)                                                                                           \
     X(ternaspmm_rmsnorm_quant)                                                                                         \
@@ -581,8 +583,17 @@ TERNA_FUNCTION(block, 35)
     lib.ternaspmm_rmsnorm_quant(in, data<terna_bf16>(pending), pending != nullptr ? data<terna_bf16>(&first) : nullptr, data<terna_bf16>(norm[0]), eps, nullptr,
                                 xq, s, m, dim, st);
     if (pending != nullptr) in = data<terna_bf16>(&first);
-    linear(qkv_w, dim, qkv);
-    if (g.t > 1) {
+    // RoPE and the cache write in the projection's epilogue, for the attention that reads its rows
+    const bool rows_in_place =
+        g.t > 1 && g.adjacent && head_dim == 128 && heads == 4 * g.kv &&
+        lib.ternaspmm_qkv_rope_linear(xq, data(&qkv_w.packed), qkv, s, data<terna_bf16>(&qkv_w.ws), qkv_w.ws_num, m, qkv_w.n, dim, data<float>(&g.cos),
+                                      data<float>(&g.sin), data<long long>(&g.pos), g.each, ck, cv, g.t, heads, g.kv, head_dim, g.slots, st);
+    if (!rows_in_place) linear(qkv_w, dim, qkv);
+    if (rows_in_place) {
+        if (!lib.ternaspmm_prefill_attention_rows(qkv, qkv_w.n, ck, cv, data<long long>(&g.pos), g.each, o, g.batch, g.t, heads, g.kv, head_dim, g.slots,
+                                                  g.scale, st))
+            refuse("%s: the attention over the projection's rows refused the launch", who);
+    } else if (g.t > 1) {
         lib.ternaspmm_rope_kv_store(TERNA_ATTENTION_INPUTS(qkv, g), q, ck, cv, g.batch, g.t, heads, g.kv, head_dim, g.slots, g.adjacent, st);
         lib.ternaspmm_prefill_attention(q, ck, cv, data<long long>(&g.pos), g.each, o, g.batch, g.t, heads, g.kv, head_dim, g.slots, g.scale, st);
     } else {

@@ -369,4 +369,39 @@ __device__ __forceinline__ uint32_t make_lut_i8(int e)
     return r;
 }
 
+// What the QKV projection of a prompt pass does with its outputs besides: rotary embedding of queries and keys (adjacent pairs), keys
+// and values straight into the cache.  A lane holds four features of one row, whole pairs; the outputs are rounded to bf16
+// first, where the separate launches store them.
+struct RopeStore {
+    const float *cos, *sin;      // [T | B T][D / 2]
+    const long long* pos;        // [T] cache slots, or [B T]
+    uint16_t *cache_k, *cache_v; // [B][KV][S][D]
+    int per_seq, T, H, KV, D, S;
+
+    // row m of the tables
+    __device__ int table_row(int m) const { return per_seq ? m : m % T; }
+    __device__ int part(int n) const { return n < H * D ? 0 : (n < (H + KV) * D ? 1 : 2); }                // queries, keys, values
+    // features n .. n + 7 (n .. n + 3): their four (two) pairs' cosines or sines
+    __device__ f32x4 angles4(const float* table, int row, int n) const { return *reinterpret_cast<const f32x4*>(table + row * (D >> 1) + ((n % D) >> 1)); }
+    __device__ float2 angles2(const float* table, int row, int n) const { return *reinterpret_cast<const float2*>(table + row * (D >> 1) + ((n % D) >> 1)); }
+    // a pair, two bf16 in a word
+    __device__ static uint32_t rotate(uint32_t pair, float c, float s)
+    {
+#pragma clang fp contract(off)                   // as terna_rope_kv_store_kernel: every product and sum rounded once
+        const float x = __uint_as_float(pair << 16), y = __uint_as_float(pair & 0xffff0000u);
+        const float a = x * c - y * s, b = y * c + x * s;
+        return pack_bf16x2(a, b);
+    }
+    // where feature n of row m goes: the output row for queries, else the cache (nullptr: a position outside it)
+    __device__ uint16_t* place(uint16_t* out, int m, int n, int N) const
+    {
+        const int which = part(n);
+        if (which == 0) return out + static_cast<size_t>(m) * N + n;
+        const int b = m / T, in = n - (H + (which == 2 ? KV : 0)) * D;
+        const long long slot = pos[table_row(m)];
+        if (slot < 0 || slot >= S) return nullptr;
+        return (which == 1 ? cache_k : cache_v) + ((static_cast<size_t>(b) * KV + in / D) * S + slot) * D + in % D;
+    }
+};
+
 }  // namespace terna

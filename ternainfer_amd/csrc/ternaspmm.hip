@@ -535,6 +535,27 @@ int ternaspmm_gate_linear(const int8_t* x, const void* packed, terna_bf16* out, 
     return 1;
 }
 
+int ternaspmm_qkv_rope_linear(const int8_t* x, const void* packed, terna_bf16* out, const terna_bf16* s, const terna_bf16* ws, int ws_num,
+                              int M, int N, int K, const float* cos, const float* sin, const long long* pos, int per_sequence, terna_bf16* cache_k,
+                              terna_bf16* cache_v, int T, int H, int KV, int D, int S, terna_stream stream)
+{
+    if (M <= 16 || N < 64 || K < 64 || (N % 64) || (K % 64) || T < 1 || M % T || H < 1 || KV < 1 || (D != 64 && D != 128) || S < 1 || N != (H + 2 * KV) * D ||
+        ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(cache_k) | reinterpret_cast<uintptr_t>(cache_v)) & 15) ||
+        ((reinterpret_cast<uintptr_t>(cos) | reinterpret_cast<uintptr_t>(sin)) & 15))
+        return 0;
+    if (!shape_ok(M, N, K) || !groups_ok(ws_num) || !i8_depth_ok(K)) return 0;
+    const Epilogue ep{s, ws, nullptr, ws_num, M <= 64 ? EP_I8_DECODE : EP_I8_PREFILL};
+    if (!(ep.kind == EP_I8_PREFILL || ws_num == 1 || (N == 3840 && ws_num == 3) || (N / ws_num) % 32 == 0)) return 0;      // one scale per 32 features
+    const RopeStore rope{cos, sin, pos, cache_k, cache_v, per_sequence != 0, T, H, KV, D, S};
+    const uint32_t* p = static_cast<const uint32_t*>(packed);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (mid_kernel_takes(x, M, N, K, sizeof(int8_t))) launch_mid_rope(x, p, out, ep, M, N, K, rope, st);
+    else if (!launch_prefill_rope<int8_t>(x, p, out, ep, M, N, K, rope, st)) return 0;
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) die("ternaspmm_qkv_rope_linear", e, __LINE__);
+    return 1;
+}
+
 int bitlinear_TernaSpMM_quant_packed(const terna_bf16* x, const void* packed, terna_bf16* out, const terna_bf16* ws, int ws_num,
                                      int M, int N, int K, terna_stream stream)
 {

@@ -928,3 +928,45 @@ def test_gate_linear_refuses(lib):
     assert lib.ternaspmm_gate_linear(vp(x), vp(p), vp(out), vp(s), vp(s), 1, 16, 256, 64, None) == 0
     assert lib.ternaspmm_gate_linear(vp(x), vp(p), vp(out), vp(s), vp(s), 2, 32, 320, 64, None) == 0
     assert lib.ternaspmm_gate_linear(vp(x[1:]), vp(p), vp(out), vp(s), vp(s), 1, 32, 256, 64, None) == 0
+
+
+@pytest.mark.parametrize("b,t,h,kv,d,k,groups,per_seq", [(1, 17, 4, 1, 128, 64, 1, False), (3, 33, 20, 5, 128, 320, 3, True), (2, 200, 20, 5, 128, 192, 3, False),
+                                                         (1, 1000, 20, 5, 128, 64, 3, False), (1, 70, 3, 1, 64, 128, 1, False), (4, 600, 20, 5, 128, 128, 3, True),
+                                                         (1, 2900, 20, 5, 128, 64, 3, False)])
+def test_qkv_rope_linear(lib, b, t, h, kv, d, k, groups, per_seq):
+    """The QKV projection with RoPE and the cache write in its epilogue, in every kernel of more than 16 rows: rotated queries and
+    both caches with the bits of the linear and ternaspmm_rope_kv_store, a position outside the cache among them; then the
+    attention that reads the projection's rows against the one that reads them per head."""
+    from ternainfer_amd import repack_weight
+    m, n, slots = b * t, (h + 2 * kv) * d, t + 9
+    fmt = DeviceFormat(make_ternary(n, k, 0.40, 7000 + m + n + k))
+    packed = repack_weight(fmt.vals, fmt.off, fmt.med, fmt.bm, n, k)
+    gen = torch.Generator(device="cuda").manual_seed(m)
+    x = torch.randint(-127, 128, (m, k), generator=gen, device="cuda", dtype=torch.int8)
+    s = (torch.rand(m, generator=gen, device="cuda") + 20).to(torch.bfloat16)
+    ws = torch.tensor([1.25, 0.75, 1.5][:groups], dtype=torch.bfloat16, device="cuda")
+    pos = torch.arange(t, device="cuda") + 4
+    if per_seq:
+        pos = pos + torch.arange(b, device="cuda")[:, None]
+    pos.view(-1)[t // 2] = slots + 3
+    angle = torch.rand((pos.numel(), d // 2), generator=gen, device="cuda") * 6
+    cos, sin = angle.cos().contiguous(), angle.sin().contiguous()
+    print(f"[case] qkv rope linear B={b} T={t} H={h} KV={kv} D={d} K={k} per_seq={per_seq}", flush=True)
+    caches = torch.zeros((4, b, kv, slots, d), dtype=torch.bfloat16, device="cuda")
+    rows, qkv = torch.zeros((2, m, n), dtype=torch.bfloat16, device="cuda")
+    q = torch.zeros((b, h, t, d), dtype=torch.bfloat16, device="cuda")
+    assert lib.ternaspmm_qkv_rope_linear(vp(x), vp(packed), vp(rows), vp(s), vp(ws), groups, m, n, k, vp(cos), vp(sin), vp(pos), int(per_seq), vp(caches[0]),
+                                         vp(caches[1]), t, h, kv, d, slots, None) == 1
+    lib.bitlinear_TernaSpMM_packed(vp(x), vp(packed), vp(qkv), vp(s), vp(ws), groups, m, n, k, 0, None)
+    lib.ternaspmm_rope_kv_store(vp(qkv), vp(cos), vp(sin), vp(pos), int(per_seq), vp(q), vp(caches[2]), vp(caches[3]), b, t, h, kv, d, slots, 1, None)
+    torch.cuda.synchronize()
+    bits = lambda a: a.contiguous().view(torch.int16)
+    assert torch.equal(bits(rows[:, :h * d]), bits(q.transpose(1, 2).reshape(m, h * d)))
+    assert torch.equal(bits(caches[0]), bits(caches[2])) and torch.equal(bits(caches[1]), bits(caches[3]))
+    if d == 128:
+        outs = torch.zeros((2, m, h * d), dtype=torch.bfloat16, device="cuda")
+        assert lib.ternaspmm_prefill_attention_rows(vp(rows), n, vp(caches[0]), vp(caches[1]), vp(pos), int(per_seq), vp(outs[0]), b, t, h, kv, d, slots,
+                                                    ctypes.c_float(d ** -0.5), None) == 1
+        lib.ternaspmm_prefill_attention(vp(q), vp(caches[0]), vp(caches[1]), vp(pos), int(per_seq), vp(outs[1]), b, t, h, kv, d, slots, ctypes.c_float(d ** -0.5), None)
+        torch.cuda.synchronize()
+        assert torch.equal(bits(outs[0]), bits(outs[1]))
