@@ -88,7 +88,7 @@ int attention_splits(int B, int H, int S, const AttentionScratch& scratch)
     return sp;
 }
 
-template <int D, bool ROPE, bool ADJ, int NW, bool SPLIT, int KT = 4>
+template <int D, bool ROPE, bool ADJ, int NW, bool SPLIT, int KT = 4, bool ROUNDS = false>
 void launch_attention_as(const uint16_t* q, uint16_t* ck, uint16_t* cv, const float* cos, const float* sin,
                          const long long* pos, int per_seq, uint16_t* out, int B, int H, int KV, int S, float scale, int splits,
                          const AttentionScratch& scratch, const AttentionPrefetch& pf_in, hipStream_t st, AttentionStats stats)
@@ -96,7 +96,7 @@ void launch_attention_as(const uint16_t* q, uint16_t* ck, uint16_t* cv, const fl
     if (stats.norm_w == nullptr || stats.out == nullptr) stats = AttentionStats{q, nullptr};   // (the kernel loads norm_w unconditionally)
     AttentionPrefetch pf = pf_in;
     if (splits > 1) pf.workgroups = 0;                       // the split grid is two-dimensional: no extra workgroups
-    auto kernel = terna_decode_attention_kernel<D, ROPE, ADJ, NW, SPLIT, false, KT>;
+    auto kernel = terna_decode_attention_kernel<D, ROPE, ADJ, NW, SPLIT, false, KT, ROUNDS>;
     const size_t lds = decode_attention_lds_bytes(D, NW, S);
     if (lds > 64 * 1024) allow_dynamic_lds(kernel, 159 * 1024, "hipFuncSetAttribute(decode attention)", __LINE__);
     const int slots = attention_slots(B, H, KV);
@@ -186,15 +186,23 @@ void launch_attention(const uint16_t* q, uint16_t* ck, uint16_t* cv, const float
         else if (S <= 384) launch_attention_as<DIM, ROPE, ADJ, 8, false, 3>(q, ck, cv, cos, sin, pos, per_seq, out, B, H, KV, S, scale, splits, scratch, pf, st, stats); \
         else TERNA_ATTN(DIM, 8, false);                                                                                              \
     } while (0)
+    // The narrow unsplit workgroup of many sequences walks a long cache in pipelined rounds; up to about 900 slots their code costs
+    // more than the trips they save (see key_rounds).
+#define TERNA_ATTN_NARROW(DIM)                                                                                                       \
+    do {                                                                                                                             \
+        if (S >= 1024) launch_attention_as<DIM, ROPE, ADJ, 4, false, 4, true>(q, ck, cv, cos, sin, pos, per_seq, out, B, H, KV, S, scale, splits, scratch, pf, st, stats); \
+        else TERNA_ATTN(DIM, 4, false);                                                                                              \
+    } while (0)
     if (D == 128) {
         if (splits > 1) TERNA_ATTN(128, 4, true);
         else if (nw == 8) TERNA_ATTN_WIDE(128);
-        else TERNA_ATTN(128, 4, false);
+        else TERNA_ATTN_NARROW(128);
     } else {
         if (splits > 1) TERNA_ATTN(64, 4, true);
         else if (nw == 8) TERNA_ATTN_WIDE(64);
-        else TERNA_ATTN(64, 4, false);
+        else TERNA_ATTN_NARROW(64);
     }
+#undef TERNA_ATTN_NARROW
 #undef TERNA_ATTN_WIDE
 #undef TERNA_ATTN
 }

@@ -339,7 +339,47 @@ constexpr size_t decode_attention_lds_bytes(int D, int NW, int S)
     return (static_cast<size_t>(S) + (64 * NW / (D / 8)) * D + 64 * NW) * sizeof(float);
 }
 
-template <int D, bool ROPE, bool ADJACENT = false, int NW = 4, bool SPLIT = false, bool DEFER = false, int KT = 4>
+// Pass 1 of a decode attention over a wave's key tiles, and pass 3 over a thread's value rows, for prefixes well beyond what the
+// launch requests before it knows their length (ROUNDS).  The plain loops take one dependent round trip per tile and per VU rows: at
+// 614 slots the four waves of the narrow workgroup make ten, one after the other.  Here a tile's registers are requested again as soon
+// as its scores are out, and the second round of value rows right after the last scores, in the registers that held keys; no byte
+// more is read (the requests are bounded by the prefix).  The branch stands in front of the whole pass: within it the number of requests in
+// flight is known at every wait.  The price is twice the code, which every launch fetches anew: 1.2 us at prefixes of one or two rounds.
+// Measured, us per decode step of the 2B shape, caches filled to 60 %, plain -> rounds: 32 sequences x 512 slots 1630 -> 1680, x 768
+// 1730 -> 1777, x 1024 1847 -> 1829, x 2048 2401 -> 2184; 48 x 1024 2254 -> 2100; 64 x 1024 2434 -> 2327.
+template <int KT, int STEP, typename Load, typename Score, typename Tile>
+__device__ __forceinline__ void key_rounds(int first, int tiles, Tile (&k)[KT], Load load, Score score)
+{
+    int at = first;
+    if (tiles > STEP * KT) {                     // uniform
+        int left = tiles;
+        for (; left > STEP * KT; left -= STEP * KT) {
+#pragma unroll
+            for (int t = 0; t < KT; ++t) {
+                score(at + STEP * t, k[t]);      // all tiles of the round exist
+                load(at + STEP * (t + KT), k[t]);
+            }
+            at += STEP * KT;
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < KT; ++t)
+        if (at + STEP * t < tiles) score(at + STEP * t, k[t]);
+}
+// a: round 0 (requested), b: round 1 (requested if there is one); a round is ROUND slots
+template <int ROUND, typename Rows, typename Load, typename Use>
+__device__ __forceinline__ void value_rounds(int slots, Rows& a, Rows& b, Load load, Use use)
+{
+    for (int l0 = 0; l0 < slots; l0 += 2 * ROUND) {
+        use(l0, a);
+        if (l0 + ROUND >= slots) break;
+        load(l0 + 2 * ROUND, a);
+        use(l0 + ROUND, b);
+        load(l0 + 3 * ROUND, b);
+    }
+}
+
+template <int D, bool ROPE, bool ADJACENT = false, int NW = 4, bool SPLIT = false, bool DEFER = false, int KT = 4, bool ROUNDS = false>
 __global__ __launch_bounds__(64 * NW) void terna_decode_attention_kernel(
     // what the first loads depend on comes first: the leading sixteen dwords of the arguments arrive in scalar registers
     const uint16_t* __restrict__ q, uint16_t* __restrict__ cache_k, uint16_t* __restrict__ cache_v,
@@ -423,8 +463,7 @@ __global__ __launch_bounds__(64 * NW) void terna_decode_attention_kernel(
     // partial score of row i and a slot's score is the sum over its R rows: the accumulator puts
     // them in R neighbouring lanes (columns 0 .. R-1), one quad permutation or two add them up.
     constexpr int NJ = D / 32;                   // MFMAs (32 dimensions each) per tile
-    // KT key tiles in flight per wave (slots 0 .. 64 NW KT - 1 of the split; tiles beyond go through the loop below, one
-    // dependent round trip each).  The launcher picks KT so that the requests just cover the cache: every request costs the
+    // KT key tiles in flight per wave (slots 0 .. 16 NW KT - 1 of the split; tiles beyond: key_rounds).  The launcher picks KT so that the requests just cover the cache: every request costs the
     // CU's address unit a slot whatever it returns, and a test in the kernel -- even a wave-uniform one on a kernel argument
     // -- made the waits around the requests conservative (8 sequences, caches of 384 slots: four tiles 6951 tokens/s,
     // three 7001, four with the fourth behind such a test 6919).
@@ -440,11 +479,18 @@ __global__ __launch_bounds__(64 * NW) void terna_decode_attention_kernel(
     // but neither a memory access nor a returned kilobyte (a clamped address did both).
     const __amdgpu_buffer_rsrc_t rk = make_raw_buffer(kbase, static_cast<uint32_t>(S) * D * 2u);
     const __amdgpu_buffer_rsrc_t rv = make_raw_buffer(vbase, static_cast<uint32_t>(S) * D * 2u);
-    auto load_keys = [&](int ltile, u32x4 (&dst)[NJ]) {
+    auto load_keys = [&](__amdgpu_buffer_rsrc_t rows, int ltile, u32x4 (&dst)[NJ]) {
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
             const int sk = 16 * (ltile * SP + sp) + SPM * j + sl;
-            dst[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, (sk * D + 8 * piece) * 2, 0, 0));
+            dst[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rows, (sk * D + 8 * piece) * 2, 0, 0));
+        }
+    };
+    auto load_values = [&](__amdgpu_buffer_rsrc_t rows, int l0, u32x4 (&dst)[VU]) {
+#pragma unroll
+        for (int u = 0; u < VU; ++u) {
+            const int sv = cache_slot(l0 + slice + u * SLICES);
+            dst[u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rows, (sv * D + chunk * 8) * 2, 0, 0));
         }
     };
     // Order of the requests: the new token's own row pieces and angles first (ROPE) -- loads return in order, so
@@ -478,12 +524,8 @@ __global__ __launch_bounds__(64 * NW) void terna_decode_attention_kernel(
     if constexpr (!SPLIT && !DEFER) nw_raw = stats.norm_w[h * D + (tid & (D - 1))];
     __builtin_amdgcn_sched_barrier(0);           // the requests above stay above the ones below
 #pragma unroll
-    for (int t = 0; t < KT; ++t) load_keys(wave + NW * t, kr[t]);
-#pragma unroll
-    for (int u = 0; u < VU; ++u) {
-        const int sv = cache_slot(slice + u * SLICES);
-        vr[u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rv, (sv * D + chunk * 8) * 2, 0, 0));
-    }
+    for (int t = 0; t < KT; ++t) load_keys(rk, wave + NW * t, kr[t]);
+    load_values(rv, 0, vr);
     __builtin_amdgcn_sched_barrier(0);           // everything is requested; only now the position is looked at
     // Prefix length: slots 0 .. pos.  It comes from device memory the host cannot check, so it is clamped to the
     // cache -- the LDS score buffer and every cache address are sized by S -- and a position outside [0, S) writes no
@@ -574,13 +616,22 @@ __global__ __launch_bounds__(64 * NW) void terna_decode_attention_kernel(
     const int tiles = (n + 15) >> 4;                                  // tiles with a valid slot, all splits
     const int ltiles = tiles > sp ? (tiles - sp + SP - 1) / SP : 0;  // ... of this split
     const int nl = 16 * ltiles;                                       // local slots (the last tile may be partly valid)
+    // from here on requests are bounded by the prefix
+    const uint32_t seen = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(n)) * D * 2u;
+    const __amdgpu_buffer_rsrc_t rk_seen = make_raw_buffer(kbase, seen), rv_seen = make_raw_buffer(vbase, seen);
+    u32x4 vn[VU];                                // ROUNDS: the second round of value rows
+    if constexpr (ROUNDS) {
+        key_rounds<KT, NW>(wave, ltiles, kr, [&](int tile, u32x4 (&dst)[NJ]) { load_keys(rk_seen, tile, dst); }, score_tile);
+        if (nl > VU * SLICES) load_values(rv_seen, VU * SLICES, vn);
+    } else {
 #pragma unroll
-    for (int t = 0; t < KT; ++t)
-        if (wave + NW * t < ltiles) score_tile(wave + NW * t, kr[t]);
-    for (int tile = wave + NW * KT; tile < ltiles; tile += NW) {      // beyond the tiles requested up front: plain loop
-        u32x4 k[NJ];
-        load_keys(tile, k);
-        score_tile(tile, k);
+        for (int t = 0; t < KT; ++t)
+            if (wave + NW * t < ltiles) score_tile(wave + NW * t, kr[t]);
+        for (int tile = wave + NW * KT; tile < ltiles; tile += NW) {      // beyond the tiles requested up front: plain loop
+            u32x4 k[NJ];
+            load_keys(rk, tile, k);
+            score_tile(tile, k);
+        }
     }
     mx = wave_max(mx);
     if (lane == 0) red[wave] = mx;
@@ -605,29 +656,36 @@ __global__ __launch_bounds__(64 * NW) void terna_decode_attention_kernel(
 
     // ---- pass 3: weighted sum of the value rows, VU rows per round (the first round is already here)
     float acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-    for (int l0 = slice; l0 < nl; l0 += VU * SLICES) {
-        if (l0 != slice) {                       // all VU rows of the round requested before any is used
-#pragma unroll
-            for (int u = 0; u < VU; ++u) {
-                const int l = l0 + u * SLICES;
-                const int s = cache_slot(l);
-                const bool ok = l < nl && s < n; // past the end: re-read slot 0, it gets weight 0 below
-                vr[u] = *reinterpret_cast<const u32x4*>(vbase + static_cast<size_t>(ok ? s : 0) * D + chunk * 8);
-            }
-        }
+    auto weigh = [&](int l0, const u32x4 (&rows)[VU]) {
 #pragma unroll
         for (int u = 0; u < VU; ++u) {
-            const int l = l0 + u * SLICES;
+            const int l = l0 + slice + u * SLICES;
             const int s = cache_slot(l);
             const bool ok = l < nl && s < n;
             const float p = ok ? score[ok ? l : 0] : 0.0f;
-            u32x4 row = vr[u];
+            u32x4 row = rows[u];
             if constexpr (ROPE) row = (s == n - 1) ? vnew : row;
             row = ok ? row : u32x4{0u, 0u, 0u, 0u};          // never multiply stale cache contents (could be NaN)
             float vf[8];
             unpack_bf16x8(row, vf);
 #pragma unroll
             for (int e = 0; e < 8; ++e) acc[e] = fmaf(p, vf[e], acc[e]);
+        }
+    };
+    if constexpr (ROUNDS) {
+        value_rounds<VU * SLICES>(nl, vr, vn, [&](int l0, u32x4 (&dst)[VU]) { load_values(rv_seen, l0, dst); }, weigh);
+    } else {
+        for (int l0 = 0; l0 + slice < nl; l0 += VU * SLICES) {
+            if (l0 != 0) {                       // all VU rows of the round requested before any is used
+#pragma unroll
+                for (int u = 0; u < VU; ++u) {
+                    const int l = l0 + slice + u * SLICES;
+                    const int s = cache_slot(l);
+                    const bool ok = l < nl && s < n; // past the end: re-read slot 0, it gets weight 0 in weigh
+                    vr[u] = *reinterpret_cast<const u32x4*>(vbase + static_cast<size_t>(ok ? s : 0) * D + chunk * 8);
+                }
+            }
+            weigh(l0, vr);
         }
     }
 #pragma unroll

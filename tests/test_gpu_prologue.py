@@ -724,6 +724,29 @@ def test_decode_attention_random_shapes(lib, b, h, kv, d, s_max, lens, split):
     _decode_attention_per_sequence_case(lib, b, h, kv, d, s_max, lens, split)
 
 
+@pytest.mark.parametrize("h,kv,d,s_max", [(20, 5, 128, 1024), (20, 5, 128, 1031), (32, 8, 64, 2000)])
+def test_decode_attention_rounds(lib, h, kv, d, s_max):
+    """More than 512 heads over a long cache (the pipelined rounds of attention_kernel.h): prefixes around a round of value rows (128
+    slots, 256 with 64 dimensions) and of key tiles (256), one token, the whole cache."""
+    lens = (1, 16, 17, 127, 128, 129, 255, 256, 257, 272, 383, 384, 385, 511, 512, 513, 527, 528, 640, 768, 769, 1000, s_max - 8, s_max - 1, s_max, 300)
+    _decode_attention_per_sequence_case(lib, len(lens), h, kv, d, s_max, lens, False)
+    b, scale = len(lens), float(d) ** -0.5
+    pos = np.array(lens, np.int64) - 1
+    cos, sin = _angles(pos, d)
+    xd, cd, sd, pd = _dev(make_bf16_activations(b, (h + 2 * kv) * d, 1741)), _dev(cos), _dev(sin), _dev(pos)
+    k0, v0 = (make_bf16_activations(b * kv * s_max, d, seed).reshape(b, kv, s_max, d) for seed in (1742, 1743))
+    for adjacent in (0, 1):
+        ck1, cv1, ck2, cv2 = _dev(k0), _dev(v0), _dev(k0), _dev(v0)
+        q1 = torch.zeros((b, h, 1, d), dtype=torch.int16, device="cuda")
+        o1 = torch.zeros((b, h * d), dtype=torch.int16, device="cuda")
+        o2 = torch.zeros_like(o1)
+        lib.ternaspmm_rope_kv_store(_vp(xd), _vp(cd), _vp(sd), _vp(pd), 1, _vp(q1), _vp(ck1), _vp(cv1), b, 1, h, kv, d, s_max, adjacent, None)
+        lib.ternaspmm_decode_attention(_vp(q1), _vp(ck1), _vp(cv1), _vp(pd), 1, _vp(o1), b, h, kv, d, s_max, scale, None, None)
+        lib.ternaspmm_rope_decode_attention(_vp(xd), _vp(cd), _vp(sd), _vp(pd), 1, _vp(ck2), _vp(cv2), _vp(o2), b, h, kv, d, s_max, scale, adjacent, None, None)
+        torch.cuda.synchronize()
+        assert torch.equal(ck1, ck2) and torch.equal(cv1, cv2) and torch.equal(o1, o2), adjacent
+
+
 def _decode_attention_per_sequence_case(lib, b, h, kv, d, s_max, lens, split):
     q = make_bf16_activations(b * h, d, 1710 + b).reshape(b, h, d)
     k = make_bf16_activations(b * kv * s_max, d, 1711 + b).reshape(b, kv, s_max, d)
