@@ -372,6 +372,13 @@ int ternaspmm_qkv_rope_linear(const int8_t* x, const void* packed, terna_bf16* o
 int ternaspmm_gate_linear(const int8_t* x, const void* packed_interleaved, terna_bf16* out, const terna_bf16* s, const terna_bf16* ws,
                           int ws_num, int M, int N, int K, terna_stream stream);
 
+/* A linear whose output returns to the residual stream (O and down projection), for more than 16 rows of int8 activations:
+ * out bf16 [M][N] = bf16(residual + output of bitlinear_TernaSpMM_packed_ws), the sum ternaspmm_rmsnorm_quant forms from the two.
+ * x, out and residual 16-byte aligned; scale groups of whole 32 columns.  workspace: split-K scratch as for
+ * bitlinear_TernaSpMM_packed_ws, or NULL.  Returns 1 when the launch was enqueued, 0 when nothing was. */
+int ternaspmm_residual_linear(const int8_t* x, const void* packed, terna_bf16* out, const terna_bf16* s, const terna_bf16* ws, int ws_num,
+                              const terna_bf16* residual, int M, int N, int K, void* workspace, long long workspace_bytes, terna_stream stream);
+
 /* ---- Attention-side kernels of a decode step (no counterpart in the reference's library) -----------
  * They stand where the reference calls xformers' rope_padded (model.py:218-229) and
  * fmha.memory_efficient_attention_forward (model.py:231-233).

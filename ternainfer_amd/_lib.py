@@ -80,6 +80,7 @@ PROTOTYPES = {
     "ternaspmm_plan_reference_call": ([_ci] * 6 + [_vp, _ci, _vp], _ci),
     "ternaspmm_qkv_rope_linear": ([_vp] * 5 + [_ci] * 4 + [_vp] * 3 + [_ci] + [_vp] * 2 + [_ci] * 5 + [_vp], _ci),
     "ternaspmm_prefill_attention_rows": ([_vp, _ci] + [_vp] * 3 + [_ci, _vp] + [_ci] * 6 + [ctypes.c_float, _vp], _ci),
+    "ternaspmm_residual_linear": ([_vp] * 5 + [_ci, _vp] + [_ci] * 3 + [_vp, ctypes.c_longlong, _vp], _ci),
     "ternaspmm_gate_linear": ([_vp] * 5 + [_ci] * 4 + [_vp], _ci),
     "bitlinear_TernaSpMM_quant_packed": ([_vp, _vp, _vp, _vp, _ci, _ci, _ci, _ci, _vp], _ci),
     "bitlinear_TernaSpMM_quant": ([_vp] * 7 + [_ci] * 4 + [_vp], _ci),

@@ -97,6 +97,11 @@ void launch_mid_rope(const int8_t* x, const uint32_t* packed, uint16_t* out, con
 {
     launch_mid_tile<int8_t, PACKED_ROPE>(x, packed, out, ep, M, N, K, st, &rope);
 }
+void launch_mid_residual(const int8_t* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, const ResidualRows& stream,
+                         hipStream_t st)
+{
+    launch_mid_tile<int8_t, PACKED_RESIDUAL>(x, packed, out, ep, M, N, K, st, &stream);
+}
 
 template void launch_mid<int8_t>(const int8_t*, const uint32_t*, uint16_t*, const Epilogue&, int, int, int, hipStream_t, const RepackGuard*);
 template void launch_mid<uint16_t>(const uint16_t*, const uint32_t*, uint16_t*, const Epilogue&, int, int, int, hipStream_t, const RepackGuard*);

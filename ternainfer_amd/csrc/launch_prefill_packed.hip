@@ -90,13 +90,17 @@ void launch_prefill_packed_dma_as(const Act* x, const uint32_t* packed, uint16_t
     const bool big_x = static_cast<size_t>(M) * K * sizeof(Act) > (4u << 20);
     const int xcd_map = (plan.grid_y % 8 == 0) && (xcd_forced < 0 ? big_x : xcd_forced != 0);
     kernel<<<grid, dim3(threads), lds, st>>>(x, packed, out, ep, M, N, K, xcd_map, splits, splits > 1 ? scratch : nullptr,
-                                               guard_row ? 1 : 0, guard_row || (EPI == PACKED_ROPE && guard != nullptr) ? *guard : PackedExtra<EPI>{});
-    if constexpr (EPI == PACKED_STORE) if (splits > 1) {
+                                               guard_row ? 1 : 0, guard_row || (EPI != PACKED_STORE && guard != nullptr) ? *guard : PackedExtra<EPI>{});
+    if constexpr (EPI == PACKED_STORE || EPI == PACKED_RESIDUAL) if (splits > 1) {
         using AccT = typename std::conditional<sizeof(Act) == 1, int, float>::type;
         const long quads = static_cast<long>(M) * (N >> 2);
-        const bool guard_first = guard != nullptr;
+        ResidualRows stream{nullptr};
+        RepackGuard check{};
+        if constexpr (EPI == PACKED_RESIDUAL) stream = *guard;
+        else if (guard != nullptr) check = *guard;
+        const bool guard_first = EPI == PACKED_STORE && guard != nullptr;
         terna_splitk_reduce_kernel<AccT><<<dim3(static_cast<unsigned>((quads + 255) / 256) + (guard_first ? 1 : 0)), dim3(256), 0, st>>>(
-            static_cast<const AccT*>(scratch), out, ep, M, N, splits, guard_first ? 1 : 0, guard_first ? *guard : RepackGuard{});
+            static_cast<const AccT*>(scratch), out, ep, M, N, splits, guard_first ? 1 : 0, check, stream);
     }
 }
 
@@ -186,13 +190,13 @@ bool launch_prefill_packed(const Act* x, const uint32_t* packed, uint16_t* out, 
 
 template <int EPI, typename Act>
 bool launch_prefill_producer(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, const PackedExtra<EPI>* extra,
-                             hipStream_t st)
+                             hipStream_t st, void* scratch = nullptr, size_t scratch_bytes = 0)
 {
     if constexpr (sizeof(Act) == 1) {
-        const PrefillPlan plan = plan_prefill_packed<Act>(x, M, N, K, nullptr, 0);
+        const PrefillPlan plan = plan_prefill_packed<Act>(x, M, N, K, scratch, scratch_bytes);
         if (!plan.direct_lds || plan.bm != 64) return false;
-        if (plan.bn == 128) launch_prefill_packed_dma_as<Act, 2, 1, EPI>(x, packed, out, ep, M, N, K, plan, nullptr, st, extra);
-        else launch_prefill_packed_dma_as<Act, 2, 2, EPI>(x, packed, out, ep, M, N, K, plan, nullptr, st, extra);
+        if (plan.bn == 128) launch_prefill_packed_dma_as<Act, 2, 1, EPI>(x, packed, out, ep, M, N, K, plan, scratch, st, extra);
+        else launch_prefill_packed_dma_as<Act, 2, 2, EPI>(x, packed, out, ep, M, N, K, plan, scratch, st, extra);
         return true;
     }
     return false;
@@ -207,7 +211,15 @@ bool launch_prefill_rope(const Act* x, const uint32_t* packed, uint16_t* out, co
 {
     return launch_prefill_producer<PACKED_ROPE>(x, packed, out, ep, M, N, K, &rope, st);
 }
+template <typename Act>
+bool launch_prefill_residual(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, const ResidualRows& stream,
+                             void* scratch, size_t scratch_bytes, hipStream_t st)
+{
+    return launch_prefill_producer<PACKED_RESIDUAL>(x, packed, out, ep, M, N, K, &stream, st, scratch, scratch_bytes);
+}
 
+template bool launch_prefill_residual<TERNA_PREFILL_ACT>(const TERNA_PREFILL_ACT*, const uint32_t*, uint16_t*, const Epilogue&, int, int, int,
+                                                         const ResidualRows&, void*, size_t, hipStream_t);
 template bool launch_prefill_gate<TERNA_PREFILL_ACT>(const TERNA_PREFILL_ACT*, const uint32_t*, uint16_t*, const Epilogue&, int, int, int, hipStream_t);
 template bool launch_prefill_rope<TERNA_PREFILL_ACT>(const TERNA_PREFILL_ACT*, const uint32_t*, uint16_t*, const Epilogue&, int, int, int, const RopeStore&,
                                                      hipStream_t);

@@ -39,7 +39,7 @@ struct MidShape {
     static_assert(RT * FB * 1024 <= kWaveBytes, "partial sums (1 KB per 16 x 16 tile) take the place of the activations");
 };
 
-// EPI: plain outputs, the feed-forward gate or the rotary embedding and cache write (see the epilogues of prefill_packed_kernel.h)
+// EPI: plain outputs, the sum with the stream, the feed-forward gate or the rotary embedding and cache write (see the epilogues of prefill_packed_kernel.h)
 template <typename Act, int RT, int FB, bool GUARD, int EPI = PACKED_STORE>
 __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
     const Act* __restrict__ x, const uint32_t* __restrict__ packed, uint16_t* __restrict__ out,
@@ -173,6 +173,11 @@ __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
         }
     };
     if (fin) load_turn(fin_m, band0 * 16 + 4 * (tid % UNITS));
+    u32x2 stream = {0u, 0u};
+    if constexpr (EPI == PACKED_RESIDUAL) {
+        const int n0 = band0 * 16 + 4 * (tid % UNITS);
+        stream = *reinterpret_cast<const u32x2*>(guard.rows + static_cast<size_t>(fin ? fin_m : 0) * N + (n0 < N ? n0 : 0));
+    }
     for (int chunk = wave;;) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
@@ -240,8 +245,12 @@ __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
             if (turn_to != nullptr) *reinterpret_cast<u32x2*>(turn_to) = turned;
             continue;
         }
-        *reinterpret_cast<u32x2*>(out + static_cast<size_t>(m) * N + n0) =
-            u32x2{o[0] | (static_cast<uint32_t>(o[1]) << 16), o[2] | (static_cast<uint32_t>(o[3]) << 16)};
+        u32x2 v = {o[0] | (static_cast<uint32_t>(o[1]) << 16), o[2] | (static_cast<uint32_t>(o[3]) << 16)};
+        if constexpr (EPI == PACKED_RESIDUAL) {
+            if (idx != tid) stream = *reinterpret_cast<const u32x2*>(guard.rows + static_cast<size_t>(m) * N + n0);
+            v = ResidualRows::add(v, stream);
+        }
+        *reinterpret_cast<u32x2*>(out + static_cast<size_t>(m) * N + n0) = v;
     }
 }
 

@@ -230,6 +230,11 @@ __global__ __launch_bounds__(256 * KS) void terna_prefill_deep_kernel(
             packed_prefill_rope_epilogue<1, NA>(sum, out, ep, guard, M, N, n0 + 32 * NA * wave, m0 + 32 * part, lane, stages + wave * OutTile<NA>::kBytes);
             return;
         }
+        if constexpr (EPI == PACKED_RESIDUAL) {
+            packed_prefill_epilogue<1, NA, AccV, false, true>(sum, out, ep, M, N, n0 + 32 * NA * wave, m0 + 32 * part, lane,
+                                                              stages + wave * OutTile<NA>::kBytes, guard);
+            return;
+        }
         packed_prefill_epilogue<1, NA, AccV, true>(sum, out, ep, M, N, n0 + 32 * NA * wave, m0 + 32 * part, lane,
                                                    rows_ok ? stages + wave * OutTile<NA>::kBytes : nullptr);
         return;
@@ -240,6 +245,10 @@ __global__ __launch_bounds__(256 * KS) void terna_prefill_deep_kernel(
     }
     if constexpr (EPI == PACKED_ROPE) {
         packed_prefill_rope_epilogue<MB, NA>(acc, out, ep, guard, M, N, n0 + 32 * NA * wave, m0, lane, smem + wave * OutTile<NA>::kBytes);
+        return;
+    }
+    if constexpr (EPI == PACKED_RESIDUAL) {
+        packed_prefill_epilogue<MB, NA, AccV, false, true>(acc, out, ep, M, N, n0 + 32 * NA * wave, m0, lane, smem + wave * OutTile<NA>::kBytes, guard);
         return;
     }
     packed_prefill_epilogue<MB, NA, AccV, MB * NA <= 2>(acc, out, ep, M, N, n0 + 32 * NA * wave, m0, lane,

@@ -182,17 +182,18 @@ __device__ __forceinline__ void packed_prefill_rope_epilogue(AccV (&acc)[NA][MB]
 
 // What a kernel does with its sums, and what it is handed for it in the place of the check of a cached copy (which rides along
 // with plain outputs only).
-enum PackedEpilogue { PACKED_STORE, PACKED_GATE, PACKED_ROPE };
+enum PackedEpilogue { PACKED_STORE, PACKED_GATE, PACKED_ROPE, PACKED_RESIDUAL };
 template <int EPI>
-using PackedExtra = typename std::conditional<EPI == PACKED_ROPE, RopeStore, RepackGuard>::type;
+using PackedExtra = typename std::conditional<EPI == PACKED_ROPE, RopeStore, typename std::conditional<EPI == PACKED_RESIDUAL, ResidualRows, RepackGuard>::type>::type;
 
 // COLS = false leaves out the per-column path (scales that change inside a 32-feature tile): unrolled next to 64 - 128 live
 // accumulators it spilled up to 88 registers, so every launch of the larger tiles carried scratch memory for a path that
 // almost no call takes.  The launcher sends such calls to the 128 x 64 instantiation, which keeps the path.
-template <int MB, int NA, typename AccV, bool COLS = true>
+// ADD: the outputs are added to the rows of `stream` (needs the tile); a block's pieces of it are requested before its sums are scaled.
+template <int MB, int NA, typename AccV, bool COLS = true, bool ADD = false>
 __device__ __forceinline__ void packed_prefill_epilogue(AccV (&acc)[NA][MB], uint16_t* __restrict__ out,
                                                         const Epilogue& ep, int M, int N, int n_wave, int m0, int lane,
-                                                        uint8_t* tile = nullptr)
+                                                        uint8_t* tile = nullptr, const ResidualRows& stream = ResidualRows{nullptr})
 {
     using OT = OutTile<NA>;
     const int kb = lane >> 5, l32 = lane & 31;
@@ -213,16 +214,27 @@ __device__ __forceinline__ void packed_prefill_epilogue(AccV (&acc)[NA][MB], uin
     const int tile_put = l32 * OT::kRowBytes + 8 * kb, tile_swz = OT::swizzle(l32);
     auto store4 = [&](int a, int b, int vq, float r0, float r1, float r2, float r3) {
         const u32x2 v = {pack_bf16x2(r0, r1), pack_bf16x2(r2, r3)};
-        if (tile != nullptr) {
+        if (ADD || tile != nullptr) {
             *reinterpret_cast<u32x2*>(tile + tile_put + (((4 * a + vq) ^ tile_swz) << 4)) = v;
         } else {
             const int n = n_wave + 32 * a + 8 * vq + 4 * kb;
             if (m_of[b] < M && n < N) *reinterpret_cast<u32x2*>(out + static_cast<size_t>(m_of[b]) * N + n) = v;
         }
     };
+    u32x4 added[OT::kReads];
+    auto request = [&](int b) {
+        if constexpr (ADD) {
+            const int n = n_wave + 8 * (lane & (OT::kPieces - 1));
+#pragma unroll
+            for (int i = 0; i < OT::kReads; ++i) {
+                const int m = m0 + 32 * b + i * OT::kRowsPerRead + lane / OT::kPieces;
+                added[i] = *reinterpret_cast<const u32x4*>(stream.rows + static_cast<size_t>(m < M ? m : M - 1) * N + (n < N ? n : 0));
+            }
+        }
+    };
     // after the last store4 of batch block b: its 32 rows leave the tile as rows
     auto flush = [&](int b) {
-        if (tile == nullptr) return;
+        if (!ADD && tile == nullptr) return;
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         const int piece = lane & (OT::kPieces - 1);
@@ -230,7 +242,8 @@ __device__ __forceinline__ void packed_prefill_epilogue(AccV (&acc)[NA][MB], uin
 #pragma unroll
         for (int i = 0; i < OT::kReads; ++i) {
             const int row = i * OT::kRowsPerRead + lane / OT::kPieces;
-            const u32x4 v = *reinterpret_cast<const u32x4*>(tile + row * OT::kRowBytes + ((piece ^ OT::swizzle(row)) << 4));
+            u32x4 v = *reinterpret_cast<const u32x4*>(tile + row * OT::kRowBytes + ((piece ^ OT::swizzle(row)) << 4));
+            if constexpr (ADD) v = ResidualRows::add(v, added[i]);
             const int m = m0 + 32 * b + row;
             // written once and read by a later launch: a streaming store keeps it from displacing the operands in L2
             if (m < M && n < N) __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(out + static_cast<size_t>(m) * N + n));
@@ -259,6 +272,7 @@ __device__ __forceinline__ void packed_prefill_epilogue(AccV (&acc)[NA][MB], uin
         auto tiles = [&](auto&& element) {
             static_for<0, MB>([&](auto bc) {
                 constexpr int b = decltype(bc)::value;
+                request(b);
                 static_for<0, NA>([&](auto ac) {
                     constexpr int a = decltype(ac)::value;
                     static_for<0, 4>([&](auto vc) {
@@ -782,6 +796,10 @@ __global__ __launch_bounds__(256, MB * NA <= 4 ? 4 : (MB * NA <= 8 ? 2 : 1)) voi
         packed_prefill_rope_epilogue<MB, NA>(acc, out, ep, guard, M, N, n0 + 32 * NA * wave, m0, lane, smem + wave * OutTile<NA>::kBytes);
         return;
     }
+    if constexpr (EPI == PACKED_RESIDUAL) {
+        packed_prefill_epilogue<MB, NA, AccV, false, true>(acc, out, ep, M, N, n0 + 32 * NA * wave, m0, lane, smem + wave * OutTile<NA>::kBytes, guard);
+        return;
+    }
     const bool rows_ok = ((reinterpret_cast<uintptr_t>(out) | (static_cast<uintptr_t>(N) * 2)) & 15) == 0;
     packed_prefill_epilogue<MB, NA, AccV, MB == 2 && NA == 1>(acc, out, ep, M, N, n0 + 32 * NA * wave, m0, lane,
                                                                 rows_ok ? smem + wave * OutTile<NA>::kBytes : nullptr);
@@ -792,7 +810,7 @@ __global__ __launch_bounds__(256, MB * NA <= 4 ? 4 : (MB * NA <= 8 ? 2 : 1)) voi
 // family: weights were +-2, the sum is halved first, as in the unsplit epilogue).  One thread per four columns.
 template <typename AccT>
 __global__ __launch_bounds__(256) void terna_splitk_reduce_kernel(const AccT* __restrict__ partial, uint16_t* __restrict__ out,
-                                                                  Epilogue ep, int M, int N, int splits, int guard_on, RepackGuard guard)
+                                                                  Epilogue ep, int M, int N, int splits, int guard_on, RepackGuard guard, ResidualRows stream)
 {
     // guard_on: the first workgroup of the grid checks the cached copy the planes were computed from (see the main kernel)
     if (guard_on && blockIdx.x == 0) {
@@ -814,7 +832,9 @@ __global__ __launch_bounds__(256) void terna_splitk_reduce_kernel(const AccT* __
         if constexpr (std::is_same<AccT, float>::value) o[v] = apply_epilogue<float>(ep.kind, e, v, sum[v] * kBf16WeightUndo);
         else o[v] = apply_epilogue<int>(ep.kind, e, v, sum[v] >> kI8WeightShift);   // planes hold the sums << 6, like the accumulators
     }
-    *reinterpret_cast<u32x2*>(out + at) = u32x2{o[0] | (static_cast<uint32_t>(o[1]) << 16), o[2] | (static_cast<uint32_t>(o[3]) << 16)};
+    u32x2 v = {o[0] | (static_cast<uint32_t>(o[1]) << 16), o[2] | (static_cast<uint32_t>(o[3]) << 16)};
+    if (stream.rows != nullptr) v = ResidualRows::add(v, *reinterpret_cast<const u32x2*>(stream.rows + at));
+    *reinterpret_cast<u32x2*>(out + at) = v;
 }
 
 }  // namespace terna

@@ -33,6 +33,7 @@ namespace {
     X(ternaspmm_qkv_rope_linear)                                                                                       \
     X(ternaspmm_prefill_attention_rows)                                                                                \
     X(ternaspmm_gate_linear)                                                                                           \
+    X(ternaspmm_residual_linear)                                                                                       \
     X(ternaspmm_quant_input)                                                                                           \
     X(ternaspmm_rmsnorm_quant)                                                                                         \
     X(ternaspmm_relu2_mul_rmsnorm_quant)                                                                               \
@@ -530,7 +531,7 @@ struct BlockLinear {
 };
 
 // (x, pending | None, cos, sin, pos, cache_k, cache_v, heads, head_dim, scale, adjacent, eps, attention workspace | None, linear workspace | None,
-//  attention_norm, attn_sub_norm, ffn_norm, ffn_sub_norm, wqkv [4], wo [4], w13 [4], w2 [4], interleaved w13 | None) -> (stream, pending): a whole block on int8
+//  attention_norm, attn_sub_norm, ffn_norm, ffn_sub_norm, wqkv [4], wo [4], w13 [4], w2 [4], interleaved w13 | None) -> (stream, pending; None where the stream has it): a whole block on int8
 // activations with its norms as launches of their own (prompt pass, decode steps of many sequences): the nine launches and nothing
 // else.  Called one by one from Python they cost 53 us of host time, more than they take on the device up to a hundred tokens.
 TERNA_FUNCTION(block, 35)
@@ -600,15 +601,25 @@ TERNA_FUNCTION(block, 35)
         lib.ternaspmm_rope_decode_attention(TERNA_ATTENTION_INPUTS(qkv, g), ck, cv, o, g.batch, heads, g.kv, head_dim, g.slots, g.scale, g.adjacent,
                                             data(attn_work), st);
     }
+    // the stream's sums in the epilogues of the projections that return to it, where these have one (elsewhere in the norm that follows)
+    auto add_linear = [&](const BlockLinear& w, int64_t k, const terna_bf16* stream_in, terna_bf16* to) {
+        return lib.ternaspmm_residual_linear(xq, data(&w.packed), to, s, data<terna_bf16>(&w.ws), w.ws_num, stream_in, m, w.n, k, data(work),
+                                             work != nullptr ? work->numel() : 0, st) == 1;
+    };
     lib.ternaspmm_rmsnorm_quant(o, nullptr, nullptr, data<terna_bf16>(norm[1]), eps, nullptr, xq, s, m, wide, st);
-    linear(o_w, wide, attn);
-    lib.ternaspmm_rmsnorm_quant(in, attn, data<terna_bf16>(&mid), data<terna_bf16>(norm[2]), eps, nullptr, xq, s, m, dim, st);
+    if (add_linear(o_w, wide, in, data<terna_bf16>(&mid))) {
+        lib.ternaspmm_rmsnorm_quant(data<terna_bf16>(&mid), nullptr, nullptr, data<terna_bf16>(norm[2]), eps, nullptr, xq, s, m, dim, st);
+    } else {
+        linear(o_w, wide, attn);
+        lib.ternaspmm_rmsnorm_quant(in, attn, data<terna_bf16>(&mid), data<terna_bf16>(norm[2]), eps, nullptr, xq, s, m, dim, st);
+    }
     if (interleaved != nullptr && lib.ternaspmm_gate_linear(xq, data(interleaved), x13, s, data<terna_bf16>(&gate_w.ws), gate_w.ws_num, m, gate_w.n, dim, st)) {
         lib.ternaspmm_rmsnorm_quant(x13, nullptr, nullptr, data<terna_bf16>(norm[3]), eps, nullptr, xq, s, m, ffn, st);
     } else {
         linear(gate_w, dim, x13);
         lib.ternaspmm_relu2_mul_rmsnorm_quant(x13, data<terna_bf16>(norm[3]), eps, nullptr, xq, s, m, ffn, st);
     }
+    if (add_linear(down_w, ffn, data<terna_bf16>(&mid), data<terna_bf16>(&out))) return pack(std::move(out), at::Tensor());
     linear(down_w, ffn, data<terna_bf16>(&out));
     return pack(std::move(mid), std::move(out));
 }

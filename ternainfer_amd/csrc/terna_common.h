@@ -369,6 +369,20 @@ __device__ __forceinline__ uint32_t make_lut_i8(int e)
     return r;
 }
 
+// What the O and the down projection do with their outputs on more than 16 rows: add them to the stream.  The outputs are rounded to bf16
+// first, where the norm kernel that used to add them reads them.
+struct ResidualRows {
+    const uint16_t* rows;        // bf16 [M][N], or nullptr
+
+    // eight (four) features of both
+    __device__ static u32x4 add(const u32x4& a, const u32x4& b) { return u32x4{pair(a.x, b.x), pair(a.y, b.y), pair(a.z, b.z), pair(a.w, b.w)}; }
+    __device__ static u32x2 add(const u32x2& a, const u32x2& b) { return u32x2{pair(a.x, b.x), pair(a.y, b.y)}; }
+    __device__ static uint32_t pair(uint32_t a, uint32_t b)
+    {
+        return pack_bf16x2(__uint_as_float(a << 16) + __uint_as_float(b << 16), __uint_as_float(a & 0xffff0000u) + __uint_as_float(b & 0xffff0000u));
+    }
+};
+
 // What the QKV projection of a prompt pass does with its outputs besides: rotary embedding of queries and keys (adjacent pairs), keys
 // and values straight into the cache.  A lane holds four features of one row, whole pairs; the outputs are rounded to bf16
 // first, where the separate launches store them.

@@ -329,7 +329,7 @@ class Block:
         has not been added to the stream yet (None for the first block): the add is part of this
         block's first fused kernel.  cache_* [B, n_kv, S, hd]; pos_idx int64 [T] cache slots shared by the
         sequences, or [B, T] with cos / sin [B*T, hd/2]: every sequence at its own positions (generate.py:253-262).
-        Returns (stream, pending) for the next block."""
+        Returns (stream, pending) for the next block; pending None where the down projection has added its output to the stream."""
         a = self.args
         bsz = cache_k.shape[0]
         t = x.shape[0] // bsz
@@ -605,11 +605,11 @@ class Transformer:
                 trace(index, x_in, pending_in, x, pending)
         if last_idx is not None:                                              # padded prompts: each sequence's own last token
             pick = torch.arange(bsz, device=dev) * t + last_idx
-            x, pending = x.index_select(0, pick), pending.index_select(0, pick)
+            x, pending = x.index_select(0, pick), None if pending is None else pending.index_select(0, pick)
         elif t > 1:                                                           # only the last new token feeds the head
-            x, pending = x.view(bsz, t, a.dim)[:, -1].contiguous(), pending.view(bsz, t, a.dim)[:, -1].contiguous()
+            x, pending = x.view(bsz, t, a.dim)[:, -1].contiguous(), None if pending is None else pending.view(bsz, t, a.dim)[:, -1].contiguous()
         if self.layers[0].fused and x.is_cuda:                                # last residual add + final norm: one launch
-            x, _ = rmsnorm_quant(x, self.norm, a.norm_eps, residual=pending, quant=False)     # (chain: pending is None, the stream has it)
+            x, _ = rmsnorm_quant(x, self.norm, a.norm_eps, residual=pending, quant=False)     # (pending None: the stream has it)
         else:
             x = rms_norm(x + pending, self.norm, a.norm_eps)
         if x.is_cuda and bsz <= 16 and a.dim % 32 == 0 and bsz * (2 * a.dim + 16) <= 160 * 1024:

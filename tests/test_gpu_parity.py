@@ -899,6 +899,30 @@ def test_deep_tile_kernel(lib, act, m, n, k):
         assert max_err <= 1e-2 * max_ref and med_ulp <= 1, (max_err, max_ref, med_ulp)
 
 
+@pytest.mark.parametrize("m,n,k,groups", [(17, 64, 64, 1), (33, 2560, 320, 1), (64, 192, 2560, 2), (65, 320, 448, 1), (100, 2560, 192, 1), (256, 2560, 6912, 1),
+                                          (300, 2560, 3392, 1), (431, 2560, 128, 1), (1000, 2560, 192, 1), (1930, 2624, 64, 1), (2000, 6912, 192, 1)])
+def test_residual_linear(lib, m, n, k, groups):
+    """Linears that return to the stream, in every kernel of more than 16 rows (split-K among them) and at their tiles' edges: the bits of
+    stream + output in bf16 on the oracle's outputs."""
+    from ternainfer_amd import repack_weight
+    fmt = DeviceFormat(make_ternary(n, k, 0.40, 7000 + m + n + k))
+    packed = repack_weight(fmt.vals, fmt.off, fmt.med, fmt.bm, n, k)
+    xq, s = make_int8_activations(m, k, 7100 + m)
+    ws = O.f32_to_bf16_bits(np.array([1.25, 0.75], np.float32)[:groups])
+    xd, sd, wd = torch.from_numpy(xq).cuda(), torch.from_numpy(s.view(np.int16)).cuda(), torch.from_numpy(ws.view(np.int16)).cuda()
+    linear = torch.from_numpy(O.spmm_i8(xq, fmt.w, s, ws, groups, 0 if m <= 64 else 1).view(np.int16)).view(torch.bfloat16)
+    stream = (torch.randn(m, n) * linear.float().std()).to(torch.bfloat16)
+    work = torch.zeros(1 << 26, dtype=torch.int8, device="cuda")
+    out, added = torch.zeros((m, n), dtype=torch.bfloat16, device="cuda"), stream.cuda()
+    for scratch in (None, work):
+        print(f"[case] residual linear M={m} N={n} K={k} groups={groups} scratch={scratch is not None}", flush=True)
+        out.zero_()
+        assert lib.ternaspmm_residual_linear(vp(xd), vp(packed), vp(out), vp(sd), vp(wd), groups, vp(added), m, n, k, None if scratch is None else vp(scratch),
+                                             0 if scratch is None else scratch.numel(), None) == 1
+        torch.cuda.synchronize()
+        assert torch.equal(out.cpu(), stream + linear)
+
+
 @pytest.mark.parametrize("m,f,k,groups", [(17, 32, 64, 1), (33, 6912, 128, 2), (64, 384, 2560, 2), (65, 384, 320, 1), (130, 1152, 192, 2), (97, 6912, 192, 2),
                                           (700, 1664, 448, 2), (2100, 5504, 64, 2), (1500, 6912, 192, 2)])
 def test_gate_linear(lib, m, f, k, groups):
