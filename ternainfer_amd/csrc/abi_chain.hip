@@ -34,11 +34,11 @@ __global__ __launch_bounds__(256) void terna_row_stats_kernel(const uint16_t* __
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 ssq = fmaf(f[e], f[e], ssq);
-                pmax = fmaxf(pmax, fabsf(__fmul_rn(f[e], w[e])));
+                pmax = max_keep_nan(pmax, fabsf(__fmul_rn(f[e], w[e])));
             }
         }
         ssq = wave_sum(ssq);
-        pmax = wave_max(pmax);
+        pmax = wave_amax(pmax);
         if (lane == 0) stats_out[row * count + p] = float2{ssq, pmax};
     }
 }
@@ -76,11 +76,11 @@ __global__ __launch_bounds__(256) void terna_step_inputs_kernel(const long long*
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 ssq = fmaf(f[e], f[e], ssq);
-                pmax = fmaxf(pmax, fabsf(__fmul_rn(f[e], w[e])));
+                pmax = max_keep_nan(pmax, fabsf(__fmul_rn(f[e], w[e])));
             }
         }
         ssq = wave_sum(ssq);
-        pmax = wave_max(pmax);
+        pmax = wave_amax(pmax);
         if (lane == 0) stats_out[static_cast<size_t>(b) * count + part] = float2{ssq, pmax};
     }
 }
@@ -125,11 +125,11 @@ __global__ __launch_bounds__(256) void terna_quant_stats_kernel(const uint16_t* 
     for (int t = 0; t < PT; ++t) {
         if (lane + 64 * t < count) {
             sum += part[t].x;
-            pmax = fmaxf(pmax, part[t].y);
+            pmax = max_keep_nan(pmax, part[t].y);
         }
     }
     sum = wave_sum(sum);
-    pmax = wave_max(pmax);
+    pmax = wave_amax(pmax);
     const float rstd = rsqrtf(sum / static_cast<float>(K) + eps);
     uint16_t sb;
     const float s = quant_scale(fabsf(round_bf16(__fmul_rn(pmax, rstd))), quant_mode, &sb);

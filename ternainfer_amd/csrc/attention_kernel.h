@@ -717,7 +717,7 @@ __global__ __launch_bounds__(64 * NW) void terna_decode_attention_kernel(
                 float ssq = v * v;
                 float pm = tid < D ? fabsf(__fmul_rn(v, __uint_as_float(nw_raw << 16))) : 0.0f;
                 ssq = wave_sum(ssq);
-                pm = wave_max(pm);
+                pm = wave_amax(pm);
                 if (lane == 0 && wave < D / 64) {
                     red[wave] = ssq;
                     red[NW + wave] = pm;
@@ -725,7 +725,7 @@ __global__ __launch_bounds__(64 * NW) void terna_decode_attention_kernel(
                 __syncthreads();
                 if (tid == 0) {
                     float2 r{red[0], red[NW]};
-                    if constexpr (D == 128) r = float2{red[0] + red[1], fmaxf(red[NW], red[NW + 1])};
+                    if constexpr (D == 128) r = float2{red[0] + red[1], max_keep_nan(red[NW], red[NW + 1])};
                     stats.out[bh] = r;
                 }
             }

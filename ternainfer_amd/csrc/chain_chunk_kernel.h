@@ -56,10 +56,10 @@ __device__ __forceinline__ void chain_reduce_partials(const float2 (&part)[kStat
 #pragma unroll
     for (int t = 0; t < kStatsMaxPartials / 64; ++t) {      // entries past the count were out of range: zeros
         sum += part[t].x;
-        pmax = fmaxf(pmax, part[t].y);
+        pmax = max_keep_nan(pmax, part[t].y);
     }
     sum = wave_sum(sum);
-    pmax = wave_max(pmax);
+    pmax = wave_amax(pmax);
     if (lane == 0) {
         const float r = rsqrtf(sum / static_cast<float>(K) + eps);
         const float amax_y = fabsf(round_bf16(__fmul_rn(pmax, r)));      // = max |y| of the row, exactly
@@ -353,12 +353,12 @@ __global__ __launch_bounds__(kChunkWaves * 64) void terna_chain_chunk_kernel(
             const float x1 = bf16_bits_to_float(apply_epilogue<int>(EP_I8_DECODE, e, 0, sum1 >> kI8WeightShift));
             e.w[0] = __uint_as_float(ew3 << 16);
             const float x3 = bf16_bits_to_float(apply_epilogue<int>(EP_I8_DECODE, e, 0, sum3 >> kI8WeightShift));
-            const float p = fmaxf(x1, 0.0f);
+            const float p = max_keep_nan(x1, 0.0f);
             const float hv = row_ok ? round_bf16(round_bf16(p * p) * x3) : 0.0f;
             float ssq = hv * hv;
             float pmax = fabsf(__fmul_rn(hv, __uint_as_float(enw << 16)));
             ssq = group_reduce<16, false>(ssq);
-            pmax = group_reduce<16, true>(pmax);
+            pmax = group_amax<16>(pmax);
             const uint32_t h32 = float_to_bf16_bits(hv);
             const uint32_t hp = h32 | (dpp_permute_u32<kDppSwapPairs>(h32) << 16);
             if (row_ok) {
@@ -381,7 +381,7 @@ __global__ __launch_bounds__(kChunkWaves * 64) void terna_chain_chunk_kernel(
                 float ssq = hv * hv;
                 float pmax = fabsf(__fmul_rn(hv, __uint_as_float(enw << 16)));
                 ssq = group_reduce<16, false>(ssq);
-                pmax = group_reduce<16, true>(pmax);
+                pmax = group_amax<16>(pmax);
                 const uint32_t h32 = float_to_bf16_bits(hv);
                 const uint32_t hp = h32 | (dpp_permute_u32<kDppSwapPairs>(h32) << 16);
                 if (row_ok) {
@@ -566,13 +566,13 @@ __device__ __forceinline__ void chain_norm_linear(
                 for (int j = 0; j < NE / 2; ++j) {
                     const float f0 = __uint_as_float(xr[t][q][j] << 16), f1 = __uint_as_float(xr[t][q][j] & 0xffff0000u);
                     if constexpr (!NORM) {
-                        pmx[q] = fmaxf(pmx[q], fmaxf(fabsf(f0), fabsf(f1)));
+                        pmx[q] = max_keep_nan(max_keep_nan(pmx[q], fabsf(f0)), fabsf(f1));
                         continue;
                     }
                     const float w0 = __uint_as_float(nw[t][j] << 16), w1 = __uint_as_float(nw[t][j] & 0xffff0000u);
                     pss[q] = fmaf(f0, f0, pss[q]);
                     pss[q] = fmaf(f1, f1, pss[q]);
-                    pmx[q] = fmaxf(pmx[q], fmaxf(fabsf(__fmul_rn(f0, w0)), fabsf(__fmul_rn(f1, w1))));
+                    pmx[q] = max_keep_nan(max_keep_nan(pmx[q], fabsf(__fmul_rn(f0, w0))), fabsf(__fmul_rn(f1, w1)));
                 }
             }
         }
@@ -580,7 +580,7 @@ __device__ __forceinline__ void chain_norm_linear(
 #pragma unroll
     for (int q = 0; q < XL; ++q) {
         const float a = NORM ? group_reduce<LPR, false>(pss[q]) : 0.0f;
-        const float b = group_reduce<LPR, true>(pmx[q]);
+        const float b = group_amax<LPR>(pmx[q]);
         if ((lane % LPR) == 0) part_s[xrow0 + RPL * q][wave] = float2{a, b};
     }
     __syncthreads();                             // barrier 1: every wave's partials
@@ -592,7 +592,7 @@ __device__ __forceinline__ void chain_norm_linear(
         const int row = 4 * ps + (lane >> 4);
         const float2 v = part_s[row < MR ? row : 0][lane & 15];
         const float total = group_reduce<16, false>(v.x);
-        const float pmax = group_reduce<16, true>(v.y);
+        const float pmax = group_amax<16>(v.y);
         const float r = rsqrtf(total / static_cast<float>(K) + eps);
         const float amax_y = NORM ? fabsf(round_bf16(__fmul_rn(pmax, r))) : pmax;          // = max |y| of the row, exactly
         uint16_t sb;
@@ -664,7 +664,7 @@ __device__ __forceinline__ void chain_norm_linear(
             float ssq = hv * hv;
             float pmax = fabsf(__fmul_rn(hv, __uint_as_float(enw << 16)));
             ssq = group_reduce<16, false>(ssq);
-            pmax = group_reduce<16, true>(pmax);
+            pmax = group_amax<16>(pmax);
             const uint32_t h32 = float_to_bf16_bits(hv);
             const uint32_t hp = h32 | (dpp_permute_u32<kDppSwapPairs>(h32) << 16);
             if (row_ok) {

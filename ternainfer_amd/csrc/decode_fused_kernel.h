@@ -294,7 +294,7 @@ __global__ __launch_bounds__(WAVES * 64) void terna_decode_fused_kernel(
             rr[t].unpack(r);
 #pragma unroll
             for (int e = 0; e < MP; ++e) {
-                const float p = fmaxf(f[e], 0.0f);
+                const float p = max_keep_nan(f[e], 0.0f);
                 f[e] = round_bf16(round_bf16(p * p) * r[e]);
             }
             xr[t].pack(f);
@@ -305,7 +305,7 @@ __global__ __launch_bounds__(WAVES * 64) void terna_decode_fused_kernel(
 
     // ---- phase B: sum of squares per row (LPR lanes share a row, then the waves)
     auto row_reduce = [&](float v, int which, bool is_max) {
-        v = is_max ? group_reduce<LPR, true>(v) : group_reduce<LPR, false>(v);
+        v = is_max ? group_amax<LPR>(v) : group_reduce<LPR, false>(v);
         if ((lane % LPR) == 0) stat[which][row][wave] = v;
         __syncthreads();
         const f32x4* p = reinterpret_cast<const f32x4*>(stat[which][row]);
@@ -313,7 +313,7 @@ __global__ __launch_bounds__(WAVES * 64) void terna_decode_fused_kernel(
 #pragma unroll
         for (int q4 = 0; q4 < WAVES / 4; ++q4) {
             const f32x4 c = p[q4];
-            if (is_max) r = fmaxf(fmaxf(r, fmaxf(c.x, c.y)), fmaxf(c.z, c.w));
+            if (is_max) r = max_keep_nan(max_keep_nan(max_keep_nan(max_keep_nan(r, c.x), c.y), c.z), c.w);
             else r += (c.x + c.y) + (c.z + c.w);
         }
         return r;
@@ -328,11 +328,11 @@ __global__ __launch_bounds__(WAVES * 64) void terna_decode_fused_kernel(
             for (int t = 0; t < PT; ++t) {
                 if (lane + 64 * t < ex.stats_count) {
                     sum += part[t].x;
-                    pmax = fmaxf(pmax, part[t].y);
+                    pmax = max_keep_nan(pmax, part[t].y);
                 }
             }
             sum = wave_sum(sum);
-            pmax = wave_max(pmax);
+            pmax = wave_amax(pmax);
             if (lane == 0) {
                 const float r = rsqrtf(sum / static_cast<float>(K) + eps);
                 const float amax_y = fabsf(round_bf16(__fmul_rn(pmax, r)));      // = max |y| of the row, exactly
@@ -362,7 +362,7 @@ __global__ __launch_bounds__(WAVES * 64) void terna_decode_fused_kernel(
 #pragma unroll
         for (int e = 0; e < MP; ++e) {
             f[e] = round_bf16(__fmul_rn(__fmul_rn(f[e], w[e]), rstd));
-            if (valid) amax = fmaxf(amax, fabsf(f[e]));
+            if (valid) amax = max_keep_nan(amax, fabsf(f[e]));
         }
         xr[t].pack(f);
     }
@@ -479,14 +479,14 @@ __global__ __launch_bounds__(WAVES * 64) void terna_decode_fused_kernel(
                 const float x1 = bf16_bits_to_float(apply_epilogue<int>(EP_I8_DECODE, e, v, sum1[v] >> kI8WeightShift));
                 e.w[v] = w3;
                 const float x3 = bf16_bits_to_float(apply_epilogue<int>(EP_I8_DECODE, e, v, sum3[v] >> kI8WeightShift));
-                const float p = fmaxf(x1, 0.0f);
+                const float p = max_keep_nan(x1, 0.0f);
                 hv[v] = i < M ? round_bf16(round_bf16(p * p) * x3) : 0.0f;
                 ssq_o = fmaf(hv[v], hv[v], ssq_o);
-                pmax_o = fmaxf(pmax_o, fabsf(__fmul_rn(hv[v], nwv[v])));
+                pmax_o = max_keep_nan(pmax_o, fabsf(__fmul_rn(hv[v], nwv[v])));
             }
             // the four lanes (g = 0 .. 3) of a batch row hold the band's sixteen features between them
             ssq_o = cross_row_reduce<false>(ssq_o);
-            pmax_o = cross_row_reduce<true>(pmax_o);
+            pmax_o = cross_row_amax(pmax_o);
             if (i < M) {
                 *reinterpret_cast<u32x2*>(out + static_cast<size_t>(i) * out_cols + epi_col) =
                     u32x2{pack_bf16x2(hv[0], hv[1]), pack_bf16x2(hv[2], hv[3])};
@@ -513,10 +513,10 @@ __global__ __launch_bounds__(WAVES * 64) void terna_decode_fused_kernel(
                 for (int v = 0; v < 4; ++v) {
                     hv[v] = i < M ? round_bf16(rv[v] + bf16_bits_to_float(o[v])) : 0.0f;
                     ssq_o = fmaf(hv[v], hv[v], ssq_o);
-                    pmax_o = fmaxf(pmax_o, fabsf(__fmul_rn(hv[v], nwv[v])));
+                    pmax_o = max_keep_nan(pmax_o, fabsf(__fmul_rn(hv[v], nwv[v])));
                 }
                 ssq_o = cross_row_reduce<false>(ssq_o);
-                pmax_o = cross_row_reduce<true>(pmax_o);
+                pmax_o = cross_row_amax(pmax_o);
                 if (i < M) {
                     *reinterpret_cast<u32x2*>(out + static_cast<size_t>(i) * N + epi_col) =
                         u32x2{pack_bf16x2(hv[0], hv[1]), pack_bf16x2(hv[2], hv[3])};

@@ -237,10 +237,10 @@ __global__ __launch_bounds__(WAVES * 64) void terna_decode_packed_kernel(
                 const float wv = (v & 1) ? __uint_as_float(wbits[v >> 1] & 0xffff0000u) : __uint_as_float(wbits[v >> 1] << 16);
                 hv[v] = m < M ? bf16_bits_to_float(float_to_bf16_bits(rv + bf16_bits_to_float(o[v]))) : 0.0f;
                 ssq_o = fmaf(hv[v], hv[v], ssq_o);
-                pmax_o = fmaxf(pmax_o, fabsf(__fmul_rn(hv[v], wv)));
+                pmax_o = max_keep_nan(pmax_o, fabsf(__fmul_rn(hv[v], wv)));
             }
             ssq_o = cross_row_reduce<false>(ssq_o);              // the four lanes (g = 0 .. 3) of a batch row: the band's sixteen features
-            pmax_o = cross_row_reduce<true>(pmax_o);
+            pmax_o = cross_row_amax(pmax_o);
             if (m < M) {
                 *reinterpret_cast<u32x2*>(out + static_cast<size_t>(m) * N + n0) = u32x2{pack_bf16x2(hv[0], hv[1]), pack_bf16x2(hv[2], hv[3])};
                 if (prod.raw_out != nullptr)

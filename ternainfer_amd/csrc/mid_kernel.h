@@ -215,7 +215,7 @@ __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
             for (int v = 0; v < 4; ++v) {
                 e1.w[v] = bf16_bits_to_float(ep.ws[0]);
                 e3.w[v] = bf16_bits_to_float(ep.ws[ep.ws_num - 1]);
-                const float r = fmaxf(bf16_bits_to_float(apply_epilogue<int>(ep.kind, e1, v, x1[v] >> kI8WeightShift)), 0.0f);
+                const float r = max_keep_nan(bf16_bits_to_float(apply_epilogue<int>(ep.kind, e1, v, x1[v] >> kI8WeightShift)), 0.0f);
                 o[v] = float_to_bf16_bits(bf16_bits_to_float(float_to_bf16_bits(r * r)) *
                                           bf16_bits_to_float(apply_epilogue<int>(ep.kind, e3, v, x3[v] >> kI8WeightShift)));
             }

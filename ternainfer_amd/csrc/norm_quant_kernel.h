@@ -47,35 +47,42 @@ constexpr int kDppSwapHalfQuads = 0x4E;   // quad_perm [2, 3, 0, 1]: lane ^ 2
 constexpr int kDppHalfRowMirror = 0x141;  // lane i <-> 7 - i within 8 lanes
 constexpr int kDppRowMirror = 0x140;      // lane i <-> 15 - i within 16 lanes
 
+template <int LANES, typename Op>
+__device__ __forceinline__ uint32_t group_fold(uint32_t v, Op op)
+{
+    static_assert(LANES >= 1 && LANES <= 64 && (LANES & (LANES - 1)) == 0, "group size");
+    if constexpr (LANES >= 2) v = op(v, dpp_permute_u32<kDppSwapPairs>(v));
+    if constexpr (LANES >= 4) v = op(v, dpp_permute_u32<kDppSwapHalfQuads>(v));
+    if constexpr (LANES >= 8) v = op(v, dpp_permute_u32<kDppHalfRowMirror>(v));     // quads are uniform by now
+    if constexpr (LANES >= 16) v = op(v, dpp_permute_u32<kDppRowMirror>(v));        // ... and so are the halves of a row
+    if constexpr (LANES >= 32) {
+        const uint32_t r0 = __builtin_amdgcn_readlane(v, 0), r1 = __builtin_amdgcn_readlane(v, 16);
+        const uint32_t r2 = __builtin_amdgcn_readlane(v, 32), r3 = __builtin_amdgcn_readlane(v, 48);
+        // 32 lanes: rows 0|1 and 2|3, lane ^ 16 through the row's uniform value of the neighbouring row
+        if constexpr (LANES == 32) v = (threadIdx.x & 32) ? op(r2, r3) : op(r0, r1);
+        else v = op(op(r0, r1), op(r2, r3));
+    }
+    return v;
+}
 template <int LANES, bool IS_MAX>
 __device__ __forceinline__ float group_reduce(float v)
 {
-    static_assert(LANES >= 1 && LANES <= 64 && (LANES & (LANES - 1)) == 0, "group size");
-    auto op = [](float a, float b) { return IS_MAX ? fmaxf(a, b) : a + b; };
-    if constexpr (LANES >= 2) v = op(v, dpp_permute<kDppSwapPairs>(v));
-    if constexpr (LANES >= 4) v = op(v, dpp_permute<kDppSwapHalfQuads>(v));
-    if constexpr (LANES >= 8) v = op(v, dpp_permute<kDppHalfRowMirror>(v));     // quads are uniform by now
-    if constexpr (LANES >= 16) v = op(v, dpp_permute<kDppRowMirror>(v));        // ... and so are the halves of a row
-    if constexpr (LANES == 32) {
-        // rows 0|1 and 2|3: lane ^ 16 through the row's uniform value of the neighbouring row
-        const float r0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 0));
-        const float r1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 16));
-        const float r2 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 32));
-        const float r3 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 48));
-        v = (threadIdx.x & 32) ? op(r2, r3) : op(r0, r1);
-    }
-    if constexpr (LANES == 64) {
-        const float r0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 0));
-        const float r1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 16));
-        const float r2 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 32));
-        const float r3 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 48));
-        v = op(op(r0, r1), op(r2, r3));
-    }
-    return v;
+    return __uint_as_float(group_fold<LANES>(__float_as_uint(v), [](uint32_t a, uint32_t b) {
+        const float x = __uint_as_float(a), y = __uint_as_float(b);
+        return __float_as_uint(IS_MAX ? fmaxf(x, y) : x + y);
+    }));
+}
+// Maximum of magnitudes that keeps a NaN (max_keep_nan): as bits, without their sign, numbers, infinity and NaN are in order,
+// and an integer maximum takes its operand through the permutation where a float one needs three instructions.
+template <int LANES>
+__device__ __forceinline__ float group_amax(float v)
+{
+    return __uint_as_float(group_fold<LANES>(__float_as_uint(v) & 0x7fffffffu, [](uint32_t a, uint32_t b) { return a > b ? a : b; }));
 }
 
 __device__ __forceinline__ float wave_sum(float v) { return group_reduce<64, false>(v); }
 __device__ __forceinline__ float wave_max(float v) { return group_reduce<64, true>(v); }
+__device__ __forceinline__ float wave_amax(float v) { return group_amax<64>(v); }
 
 __device__ __forceinline__ void unpack_bf16x8(const u32x4& v, float f[8])
 {
@@ -103,10 +110,10 @@ __device__ __forceinline__ void quant_pass(const float (&h)[NV][8], float amax, 
     __shared__ float red[kNormThreads / 64];
     const int tid = threadIdx.x;
     const int nvec = K >> 3;
-    amax = wave_max(amax);
+    amax = wave_amax(amax);
     if ((tid & 63) == 0) red[tid >> 6] = amax;
     __syncthreads();
-    amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    amax = max_keep_nan(max_keep_nan(red[0], red[1]), max_keep_nan(red[2], red[3]));
     uint16_t s_bits;
     const float s = quant_scale(amax, quant_mode, &s_bits);
     if (tid == 0) s_out[row] = s_bits;
@@ -162,7 +169,7 @@ __device__ __forceinline__ void norm_quant_passes(float (&h)[NV][8], const u32x4
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 h[i][j] = round_bf16(h[i][j] * rstd * w[j]);
-                amax = fmaxf(amax, fabsf(h[i][j]));
+                amax = max_keep_nan(amax, fabsf(h[i][j]));
             }
             if (y_out != nullptr) *reinterpret_cast<u32x4*>(y_out + row * K + 8 * v) = pack_bf16x8(h[i]);
         }
@@ -221,7 +228,7 @@ __global__ __launch_bounds__(kNormThreads) void terna_norm_quant_kernel(
                 unpack_bf16x8(raw_b[i], g);
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
-                    const float r = fmaxf(h[i][j], 0.0f);
+                    const float r = max_keep_nan(h[i][j], 0.0f);
                     h[i][j] = round_bf16(round_bf16(r * r) * g[j]);
                 }
             } else if constexpr (SECOND) {
@@ -257,7 +264,7 @@ __global__ __launch_bounds__(kNormThreads) void terna_quant_input_kernel(const u
     for (int i = 0; i < NV; ++i) {              // (a clamped vector is one of the row's: the maximum may see it twice)
         unpack_bf16x8(raw[i], h[i]);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(h[i][j]));
+        for (int j = 0; j < 8; ++j) amax = max_keep_nan(amax, fabsf(h[i][j]));
     }
     quant_pass<NV>(h, amax, K, row, xq_out, s_out, quant_mode);
 }

@@ -94,7 +94,7 @@ __device__ __forceinline__ void packed_prefill_gate_epilogue(AccV (&acc)[NA][MB]
                 for (int v = 0; v < 4; ++v) {
                     const float x1 = element(static_cast<float>(acc[a][b][4 * vq + v] >> kI8WeightShift), s, w1, c1);
                     const float x3 = element(static_cast<float>(acc[a][b][8 + 4 * vq + v] >> kI8WeightShift), s, w3, c3);
-                    const float r = fmaxf(bf16_bits_to_float(float_to_bf16_bits(x1)), 0.0f);
+                    const float r = max_keep_nan(bf16_bits_to_float(float_to_bf16_bits(x1)), 0.0f);
                     h[v] = bf16_bits_to_float(float_to_bf16_bits(r * r)) * bf16_bits_to_float(float_to_bf16_bits(x3));
                 }
                 *reinterpret_cast<u32x2*>(tile + l32 * ROW + (((2 * a + vq) ^ swizzle(l32)) << 4) + 8 * kb) =

@@ -81,12 +81,16 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi)
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{lo, hi}, bf16x2_t));
 }
 
+// Maximum that keeps a NaN, as torch's abs().amax() and relu() do (fmaxf drops it, and a broken row would come out as finite,
+// plausible numbers): one instruction, three operands and their magnitudes included.
+__device__ __forceinline__ float max_keep_nan(float a, float b) { return __builtin_elementwise_maximum(a, b); }
+
 // The per-row scale of quant_input from the row's max |x|: `s_bits` is what is published, the return value what
-// multiplies the activations.
+// multiplies the activations.  A NaN in the row makes the scale NaN, an infinity makes it 0.
 __device__ __forceinline__ float quant_scale(float amax, int mode, uint16_t* s_bits)
 {
     const float floor_v = mode == QUANT_EAGER ? 1.0013580322265625e-05f /* bf16(1e-5) */ : 1e-5f;
-    const float a = fmaxf(amax, floor_v);
+    const float a = max_keep_nan(amax, floor_v);
     float t;
     if (mode == QUANT_ROUNDED) {
         t = __fdiv_rn(127.0f, a);
@@ -99,12 +103,13 @@ __device__ __forceinline__ float quant_scale(float amax, int mode, uint16_t* s_b
     return mode == QUANT_COMPILED ? t : bf16_bits_to_float(*s_bits);
 }
 // One activation: clamp(rint(x * s_mul)), the product rounded to bf16 first in QUANT_EAGER.  Returned as a float in
-// [-128, 127].
+// [-128, 127].  Products are NaN only where the scale is NaN or 0 (see quant_scale), and there every integer is 0, which is what
+// the conversion of a NaN to int8 gives in torch: the median of a NaN and two bounds is the lower bound.
 __device__ __forceinline__ float quant_value(float x, float s_mul, int mode)
 {
     float p = __fmul_rn(x, s_mul);
     if (mode == QUANT_EAGER) p = bf16_bits_to_float(float_to_bf16_bits(p));
-    return __builtin_amdgcn_fmed3f(rintf(p), -128.0f, 127.0f);
+    return __builtin_amdgcn_fmed3f(rintf(p), s_mul > 0.0f ? -128.0f : 0.0f, 127.0f);      // (the bound: once per row)
 }
 
 // Weight-scale group of output column n on the decode path (Reduction_Kernel.cuh:46-54).
@@ -185,6 +190,16 @@ __device__ __forceinline__ float cross_row_reduce(float v)
     b = v;
     asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
     return op(a, b);
+}
+
+// The same for a maximum of magnitudes that keeps a NaN: as bits, without their sign, numbers, infinity and NaN are in order.
+__device__ __forceinline__ float cross_row_amax(float v)
+{
+    uint32_t a = __float_as_uint(v) & 0x7fffffffu, b = a;
+    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+    a = b = a > b ? a : b;
+    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+    return __uint_as_float(a > b ? a : b);
 }
 
 // Compile-time loop: the body receives the index as a constant, so register arrays indexed by it

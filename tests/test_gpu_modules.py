@@ -121,3 +121,103 @@ def test_spbitlinear_few_rows_in_one_launch(m, n, k):
     finally:
         lib.ternaspmm_repack_cache_clear()
         lib.ternaspmm_repack_cache_enable(was)
+
+
+def _with_broken_rows(x_bits, kind):
+    """NaN, infinities or both in some rows: -> (bits, rows with a NaN, rows with infinities only)."""
+    m, k = x_bits.shape
+    x = x_bits.copy()
+    nan, inf, neg = 0x7FC0, 0x7F80, 0xFF80
+    if m < 4:
+        x[m - 1, k - 1] = {"nan": nan, "inf": inf, "-inf": neg}[kind]
+        return (x, [m - 1], []) if kind == "nan" else (x, [], [m - 1])
+    x[0, k - 1], x[1, 3], x[m - 1, k // 2], x[m - 1, 1] = nan, inf, neg, 0xFFC0
+    x[2, k - 8:] = neg
+    return x, [0, m - 1], [1, 2]
+
+
+@pytest.mark.parametrize("m,kind", [(1, "nan"), (1, "inf"), (1, "-inf"), (2, "nan"), (3, "inf"), (4, ""), (8, ""), (9, ""), (64, ""), (65, ""), (300, "")])
+@pytest.mark.parametrize("k", [192, 2560])
+def test_spbitlinear_broken_activations_show_in_the_output(m, kind, k):
+    """A NaN in a row makes the row's scale and with it all of its outputs NaN; an infinity makes the scale 0 and the integers 0,
+    hence outputs 0 / 0 under the rule of up to 64 rows and 0 above (s == 0, epilogue_visitor_scale_ws.h:180-191): on every
+    route, in every quantisation mode, and the other rows keep their bits."""
+    import ternainfer_amd as T
+    from ternainfer_amd import _lib, linear as L
+    lib = _lib.load()
+    n = 256
+    w = make_ternary(n, k, 0.40, 900 + m + k)
+    dic, ws = checkpoint_entry(w, [1.375])
+    x_bits, nan_rows, inf_rows = _with_broken_rows(make_bf16_activations(m, k, 910 + m + k), kind)
+    good = [r for r in range(m) if r not in nan_rows + inf_rows]
+    x = torch.from_numpy(x_bits.view(np.int16)).view(torch.bfloat16).cuda()
+    print(f"[case] broken activations M={m} K={k} {kind}", flush=True)
+    q, s = L.quant_input(x)
+    assert torch.isnan(s[nan_rows]).all() and (s[inf_rows] == 0).all() and (q[nan_rows + inf_rows] == 0).all()
+    was = lib.ternaspmm_quant_mode(-1)
+    try:
+        for mode in (L.QUANT_ROUNDED, L.QUANT_COMPILED, L.QUANT_EAGER):
+            lib.ternaspmm_quant_mode(mode)
+            qm, sm = L.quant_input(x)
+            want_q, want_s = L.quant_input(x.float(), mode)      # (another activation type: the torch lines)
+            assert torch.equal(qm, want_q) and torch.equal(sm.nan_to_num(nan=-1.0), want_s.to(torch.bfloat16).nan_to_num(nan=-1.0)), mode
+    finally:
+        lib.ternaspmm_quant_mode(was)
+    q_good, s_good = O.quant_input(x_bits[good]) if good else (None, None)
+    for repack in (False, True):
+        out = T.SpBitLinear(k, n, dic, "l", repack=repack)(x)
+        torch.cuda.synchronize()
+        assert torch.isnan(out[nan_rows]).all()
+        assert torch.isnan(out[inf_rows]).all() if m <= 64 else (out[inf_rows] == 0).all()
+        if good:
+            assert (bits(out[good]) == O.spmm_i8(q_good, w, s_good, bits(ws), 1, 0 if m <= 64 else 1)).all()
+
+
+@pytest.mark.parametrize("m", [4, 8, 12, 70])
+def test_broken_rows_behind_a_norm_are_nan_on_every_route(m):
+    """NaN and infinities in a row in front of a norm: all of the row's outputs are NaN, whether the norm takes its statistics
+    itself or from partials (also where the norm's weight of an infinite element is 0), and the other rows keep their bits."""
+    import ternainfer_amd as T
+    from ternainfer_amd import linear as L
+    n, k = 256, 512
+    w = make_ternary(n, k, 0.40, 930 + m)
+    dic, ws = checkpoint_entry(w, [1.375])
+    dev = lambda b: torch.from_numpy(b.view(np.int16)).view(torch.bfloat16).cuda()
+    packed = L.repack_weight(*(dic["l.weight" + p].cuda() for p in ("_compressed_val", "_TileOffsets_global", "_TileOffsets_median", "_bitmap")), n, k)
+    clean = make_bf16_activations(m, k, 940 + m)
+    broken, nan_rows, inf_rows = _with_broken_rows(clean, "")
+    bad = nan_rows + inf_rows
+    good = [r for r in range(m) if r not in bad]
+    g = torch.rand(k, device="cuda").to(torch.bfloat16) + 0.5
+    g[3] = 0                                      # (the infinity of row 1)
+    scale = ws.cuda()
+    zeros = torch.zeros((m, n), dtype=torch.bfloat16, device="cuda")
+    ones = torch.ones(n, dtype=torch.bfloat16, device="cuda")
+
+    def with_stats(x):
+        st = L.row_stats(x, g)
+        q, s = L.quant_from_stats(x, st, g, 1e-5)
+        outs = [L.TernaInfer_linear_packed(q, packed, s, scale, 1, n)]
+        if m <= 8:
+            outs.append(L.fused_linear(x, g, 1e-5, packed, scale, 1, n, k, stats=st)[0])
+        if m <= 16:
+            r = L.fused_linear(q, None, 1e-5, packed, scale, 1, n, k, quantised=s, epilogue=L.EPILOGUE_RESIDUAL, residual=zeros, next_norm_weight=ones)
+            outs += [r[0], r[1].reshape(m, -1)]       # the stream and its partials
+        return outs
+
+    def with_norm(x):
+        q, s, _ = L.rmsnorm_quant(x, g, 1e-5)
+        return [L.TernaInfer_linear_packed(q, packed, s, scale, 1, n), L.rmsnorm_linear_packed(x, g, 1e-5, packed, scale, 1, n)[0]]
+
+    def gated(x):
+        x13 = torch.cat([x, torch.ones_like(x)], dim=1)
+        q, s = L.relu2_mul_rmsnorm_quant(x13, g, 1e-5)
+        return [L.TernaInfer_linear_packed(q, packed, s, scale, 1, n), L.relu2_mul_rmsnorm_linear_packed(x13, g, 1e-5, packed, scale, 1, n)]
+
+    print(f"[case] broken rows behind a norm M={m}", flush=True)
+    for route in (with_stats, with_norm, gated):
+        rows = [r for r in bad if not (route is gated and r == 2)]     # (relu of -infinity is 0: that row is whole)
+        for i, (got, want) in enumerate(zip(route(dev(broken)), route(dev(clean)))):
+            torch.cuda.synchronize()
+            assert torch.isnan(got[rows]).all(), (route.__name__, i)
+            assert torch.equal(got[good], want[good]), (route.__name__, i)
