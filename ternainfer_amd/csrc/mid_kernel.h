@@ -95,7 +95,7 @@ __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
     RawW rw;
     auto issue = [&](int at_chunk) __attribute__((always_inline)) {
         const int chunk = __builtin_amdgcn_readfirstlane(at_chunk);
-        // columns past K (a partial last chunk): loads pulled back into the row, the weights zeroed when they are used
+        // columns past K (a partial last chunk): loads pulled back into the row, one of the operands zeroed when they are used
         const int tile0 = chunk * 4;
         const int left = ktiles - 1 - tile0;
         const uint32_t woff = static_cast<uint32_t>(tile0 * 256 + (g < left ? g : left) * 256 + i * 16);
@@ -118,12 +118,24 @@ __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
     auto multiply = [&](int chunk) __attribute__((always_inline)) {
 #pragma unroll
         for (int b = 0; b < FB; ++b) landed(rw.w[b]);
+        uint8_t* src = mine + i * S::kRowBytes;
         if (chunk * 4 + 4 > ktiles) {                    // uniform
-            const uint32_t keep = chunk * 4 + g < ktiles ? ~0u : 0u;
+            const bool exists = chunk * 4 + g < ktiles;  // this lane's tile
+            if constexpr (BF16) {
+                // the activations in the place of a tile that does not exist are others of the row, which may be infinite: they are
+                // overwritten (each lane what it will read), zero weights would make NaN of them
+                if (!exists) {
 #pragma unroll
-            for (int b = 0; b < FB; ++b) rw.w[b] = u32x4{rw.w[b].x & keep, rw.w[b].y & keep, rw.w[b].z & keep, rw.w[b].w & keep};
+                    for (int r = 0; r < RT; ++r)
+#pragma unroll
+                        for (int p = 0; p < 8; ++p) *reinterpret_cast<u32x4*>(src + 16 * r * S::kRowBytes + (((8 * g + p) ^ i) * 16)) = u32x4{0u, 0u, 0u, 0u};
+                }
+            } else {
+                const uint32_t keep = exists ? ~0u : 0u;
+#pragma unroll
+                for (int b = 0; b < FB; ++b) rw.w[b] = u32x4{rw.w[b].x & keep, rw.w[b].y & keep, rw.w[b].z & keep, rw.w[b].w & keep};
+            }
         }
-        const uint8_t* src = mine + i * S::kRowBytes;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             if constexpr (BF16) {

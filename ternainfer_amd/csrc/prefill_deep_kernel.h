@@ -136,7 +136,10 @@ __global__ __launch_bounds__(256 * KS) void terna_prefill_deep_kernel(
         }
     };
     const int wshift = 4 - 4 * kb;
-    uint32_t wmask = kTopFieldMask;                                       // 0: the lane's (int8) or the upper groups' (bf16) tile does not exist
+    // Of a last stage with one tile: int8 multiplies both by weights that are 0 where the lane's tile does not exist; bf16 leaves the
+    // groups of the other one out (its activations are the first tile's, which may be infinite: 0 times that is NaN).
+    uint32_t wmask = kTopFieldMask;
+    bool upper = true;
     auto mma = [&](const Ops& v, auto qc) __attribute__((always_inline)) {
         constexpr int q = decltype(qc)::value;
 #pragma unroll
@@ -146,8 +149,7 @@ __global__ __launch_bounds__(256 * KS) void terna_prefill_deep_kernel(
 #pragma unroll
                 for (int b = 0; b < MB; ++b) acc[a][b] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, __builtin_bit_cast(i32x4, v.b[q][b]), acc[a][b], 0, 0, 0);
             } else {
-                const uint32_t word = v.w[a][q >> 2][q & 3] & (q >= 4 ? wmask : ~0u);
-                const bf16x8 af = __builtin_bit_cast(bf16x8, expand_chunk_bf16(word << wshift));
+                const bf16x8 af = __builtin_bit_cast(bf16x8, expand_chunk_bf16(v.w[a][q >> 2][q & 3] << wshift));
 #pragma unroll
                 for (int b = 0; b < MB; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, __builtin_bit_cast(bf16x8, v.b[q][b]), acc[a][b], 0, 0, 0);
             }
@@ -163,18 +165,22 @@ __global__ __launch_bounds__(256 * KS) void terna_prefill_deep_kernel(
     static_for<0, GROUPS>([&](auto qc) { load(0, qc, even); });
     auto set_mask = [&](int k) __attribute__((always_inline)) {
         if constexpr (I8) wmask = (half_tail && k == steps - 1 && kb) ? 0u : kTopFieldMask;
-        else wmask = (half_tail && k == steps - 1) ? 0u : ~0u;
+        else upper = !(half_tail && k == steps - 1);
     };
+    constexpr int LOWER = I8 ? GROUPS : GROUPS / 2;                       // groups of the first tile (int8: of both)
     auto step = [&](int k, const Ops& cur, Ops& nxt) __attribute__((always_inline)) {
         set_mask(k);
         // own part of stage k + 1 landed; everybody's, and everybody is past the operand reads of stage k - 1
         asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((D - 3) * PER) : "memory");
         issue(k + D - 1, st_dma);                                         // into the stage of step k - 1
-        static_for<0, GROUPS>([&](auto qc) {
+        auto group = [&](auto qc) __attribute__((always_inline)) {
             __builtin_amdgcn_sched_barrier(0);                            // keeps the reads between the groups
             load(st_next, qc, nxt);
             mma(cur, qc);
-        });
+        };
+        static_for<0, LOWER>(group);
+        if (I8 || upper) static_for<LOWER, GROUPS>(group);                // uniform
+        else static_for<LOWER, GROUPS>([&](auto qc) { load(st_next, qc, nxt); });
         __builtin_amdgcn_sched_barrier(0);
         st_next = next(st_next);
         st_dma = next(st_dma);
@@ -183,7 +189,8 @@ __global__ __launch_bounds__(256 * KS) void terna_prefill_deep_kernel(
     auto last_step = [&](int k, const Ops& cur) __attribute__((always_inline)) {
         if (k >= k_end) return;                                           // uniform over the part
         set_mask(k);
-        static_for<0, GROUPS>([&](auto qc) { mma(cur, qc); });
+        static_for<0, LOWER>([&](auto qc) { mma(cur, qc); });
+        if (I8 || upper) static_for<LOWER, GROUPS>([&](auto qc) { mma(cur, qc); });
     };
     int t = 0;
     for (; t + 2 < turns; t += 2) {

@@ -221,3 +221,34 @@ def test_broken_rows_behind_a_norm_are_nan_on_every_route(m):
             torch.cuda.synchronize()
             assert torch.isnan(got[rows]).all(), (route.__name__, i)
             assert torch.equal(got[good], want[good]), (route.__name__, i)
+
+
+# decode kernels; the kernel for 17 rows .. a few hundred (K in chunks of 256 columns); the MFMA-tiled ones (in stages of 128)
+@pytest.mark.parametrize("m,n,k", [(1, 256, 320), (16, 256, 320), (17, 256, 320), (37, 256, 64), (37, 2560, 2624), (100, 3840, 448), (100, 512, 192), (300, 2560, 2560),
+                                   (500, 2560, 192), (500, 2560, 320), (500, 2560, 256), (1000, 2560, 64), (1000, 2560, 448), (2048, 2560, 320)])
+def test_infinite_bf16_activations_at_the_end_of_a_row(m, n, k):
+    """bf16 linears: an infinity in the last columns gives +-infinity where its weight is not 0 (0 times it is NaN) and nowhere
+    else, whatever part of a kernel's last piece of K the row leaves empty."""
+    import ternainfer_amd as T
+    from ternainfer_amd import _lib, linear as L
+    w = make_ternary(n, k, 0.40, 950 + m + k)
+    dic, ws = checkpoint_entry(w, [1.25])
+    packed = L.repack_weight(*(dic["l.weight" + p].cuda() for p in ("_compressed_val", "_TileOffsets_global", "_TileOffsets_median", "_bitmap")), n, k)
+    x_bits = make_bf16_activations(m, k, 960 + m + k)
+    x_bits[0, k - 1] = 0x7F80
+    x_bits[m // 2, k - 8] = 0xFF80
+    x_bits[m - 1, k - 20] = 0x7F80
+    x = torch.from_numpy(x_bits.view(np.int16)).view(torch.bfloat16)
+    print(f"[case] infinite bf16 activations M={m} N={n} K={k}", flush=True)
+    got = _lib.native().linear_bf16_packed(x.cuda(), packed, torch.tensor([1.25], device="cuda"), 1, n, None)
+    torch.cuda.synchronize()
+    got = got.cpu().double()
+    broken = sorted({0, m // 2, m - 1})
+    xw = x.double()
+    want = (xw @ torch.from_numpy(w).double().t()) * 1.25
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(torch.isinf(got), torch.isinf(want)) and torch.equal(got[torch.isinf(got)], want[torch.isinf(want)])
+    assert torch.isinf(want[broken]).any(dim=1).all() and torch.isfinite(want).any(dim=1).sum() == m - len(broken)
+    whole = torch.isfinite(want)
+    if whole.any():
+        assert (got[whole] - want[whole]).abs().max() <= 1e-2 * want[whole].abs().max()
