@@ -4,7 +4,8 @@
 // and streams.  The library is the one _lib.py loads; init() binds its entry points by name.
 //
 // Every function checks shapes and element counts before anything is enqueued (the C ABI takes pointers on trust) and
-// raises ValueError; the tensors' types and devices are the caller's business where linear.py does not state otherwise.
+// raises ValueError, or TypeError where an argument is no tensor; the tensors' types and devices are the caller's business
+// where linear.py does not state otherwise.
 #include <dlfcn.h>
 
 #include <torch/csrc/Exceptions.h>
@@ -55,9 +56,20 @@ struct Library {
 #undef X
 } lib;
 
-const at::Tensor* tensor(PyObject* o) { return o == Py_None ? nullptr : &THPVariable_Unpack(o); }
-
 struct Refused : std::exception {};            // a Python error is set
+
+// an argument that is a tensor
+const at::Tensor& tensor(PyObject* o)
+{
+    if (!THPVariable_CheckExact(o) && !THPVariable_Check(o)) {
+        PyErr_Format(PyExc_TypeError, "expected a torch.Tensor, got %s", Py_TYPE(o)->tp_name);
+        throw Refused();
+    }
+    return THPVariable_Unpack(o);
+}
+// ... or None
+const at::Tensor* optional(PyObject* o) { return o == Py_None ? nullptr : &tensor(o); }
+
 [[noreturn]] void refuse(const char* format, ...)
 {
     va_list args;
@@ -187,8 +199,8 @@ void check_format(const char* who, const at::Tensor& bitmap, int64_t n, int64_t 
 // the rows, then the int8 linear on the repacked weight or on the reference format.  None: x is not for this path.
 TERNA_FUNCTION(bit_linear, 10)
 {
-    const at::Tensor &x = *tensor(a[0]), &bitmap = *tensor(a[2]), &ws = *tensor(a[6]);
-    const at::Tensor *packed = tensor(a[1]), *workspace = tensor(a[9]);
+    const at::Tensor &x = tensor(a[0]), &bitmap = tensor(a[2]), &offsets = tensor(a[3]), &median = tensor(a[4]), &signs = tensor(a[5]), &ws = tensor(a[6]);
+    const at::Tensor *packed = optional(a[1]), *workspace = optional(a[9]);
     const int ws_num = integer32(a[7]);
     const int64_t n = integer32(a[8]);
     at::Tensor rows;
@@ -201,8 +213,8 @@ TERNA_FUNCTION(bit_linear, 10)
     if (m <= 8) {                       // a few rows: both steps in one launch
         const int done = packed != nullptr ? lib.bitlinear_TernaSpMM_quant_packed(data<terna_bf16>(&rows), data(packed), data<terna_bf16>(&out),
                                                                                   data<terna_bf16>(&ws), ws_num, m, n, k, st)
-                                           : lib.bitlinear_TernaSpMM_quant(data<terna_bf16>(&rows), data<uint64_t>(&bitmap), data<int>(tensor(a[3])),
-                                                                           data<uint16_t>(tensor(a[4])), data<uint32_t>(tensor(a[5])), data<terna_bf16>(&out),
+                                           : lib.bitlinear_TernaSpMM_quant(data<terna_bf16>(&rows), data<uint64_t>(&bitmap), data<int>(&offsets),
+                                                                           data<uint16_t>(&median), data<uint32_t>(&signs), data<terna_bf16>(&out),
                                                                            data<terna_bf16>(&ws), ws_num, m, n, k, st);
         if (done) return wrap(std::move(out));
     }
@@ -212,7 +224,7 @@ TERNA_FUNCTION(bit_linear, 10)
         lib.bitlinear_TernaSpMM_packed_ws(q.q, data(packed), data<terna_bf16>(&out), q.s, data<terna_bf16>(&ws), ws_num, m, n, k, 0,
                                           data(workspace), workspace != nullptr ? workspace->numel() : 0, st);
     else
-        lib.bitlinear_TernaSpMM(q.q, data<uint64_t>(&bitmap), data<int>(tensor(a[3])), data<uint16_t>(tensor(a[4])), data<uint32_t>(tensor(a[5])),
+        lib.bitlinear_TernaSpMM(q.q, data<uint64_t>(&bitmap), data<int>(&offsets), data<uint16_t>(&median), data<uint32_t>(&signs),
                                 data<terna_bf16>(&out), q.s, data<terna_bf16>(&ws), ws_num, m, n, k, 7, data<int32_t>(workspace), st);
     return wrap(std::move(out));
 }
@@ -220,7 +232,7 @@ TERNA_FUNCTION(bit_linear, 10)
 // (x, bitmap, tile offsets, median offsets, signs, scale, ws_num, out_features, route 0 auto / 1 decode / 2 prefill)
 TERNA_FUNCTION(bit_linear_bf16, 9)
 {
-    const at::Tensor &x = *tensor(a[0]), &bitmap = *tensor(a[1]);
+    const at::Tensor &x = tensor(a[0]), &bitmap = tensor(a[1]), &offsets = tensor(a[2]), &median = tensor(a[3]), &signs = tensor(a[4]), &scale = tensor(a[5]);
     const int ws_num = integer32(a[6]), route = integer32(a[8]);
     const int64_t n = integer32(a[7]);
     at::Tensor rows;
@@ -229,15 +241,15 @@ TERNA_FUNCTION(bit_linear_bf16, 9)
     check_format("TernaInfer_linear_bf16", bitmap, n, k);
     at::Tensor out = make_output(x, n);
     const auto fn = route == 1 ? lib.bitlinear_TernaSpMM_bf16_decode : route == 2 ? lib.bitlinear_TernaSpMM_bf16_prefill : lib.bitlinear_TernaSpMM_bf16;
-    fn(data<terna_bf16>(&rows), data<uint64_t>(&bitmap), data<int>(tensor(a[2])), data<uint16_t>(tensor(a[3])), data<uint32_t>(tensor(a[4])),
-       data<terna_bf16>(&out), data<float>(tensor(a[5])), ws_num, m, n, k, 1, nullptr, stream());
+    fn(data<terna_bf16>(&rows), data<uint64_t>(&bitmap), data<int>(&offsets), data<uint16_t>(&median), data<uint32_t>(&signs),
+       data<terna_bf16>(&out), data<float>(&scale), ws_num, m, n, k, 1, nullptr, stream());
     return wrap(std::move(out));
 }
 
 // (x bf16 [..., K]) -> (int8 [..., K], bf16 [..., 1]), or None
 TERNA_FUNCTION(quant_input, 1)
 {
-    const at::Tensor& x = *tensor(a[0]);
+    const at::Tensor& x = tensor(a[0]);
     at::Tensor rows;
     int64_t m, k;
     if (!bf16_rows(x, &rows, &m, &k)) Py_RETURN_NONE;
@@ -253,8 +265,8 @@ TERNA_FUNCTION(quant_input, 1)
 TERNA_FUNCTION(linear_packed, 7)
 {
     const char* who = "TernaInfer_linear_packed";
-    const at::Tensor &x = *tensor(a[0]), &s = *tensor(a[1]), &packed = *tensor(a[2]), &ws = *tensor(a[3]);
-    const at::Tensor* workspace = tensor(a[6]);
+    const at::Tensor &x = tensor(a[0]), &s = tensor(a[1]), &packed = tensor(a[2]), &ws = tensor(a[3]);
+    const at::Tensor* workspace = optional(a[6]);
     const int ws_num = integer32(a[4]);
     const int64_t n = integer32(a[5]);
     check_matrix(who, x);
@@ -272,8 +284,8 @@ TERNA_FUNCTION(linear_packed, 7)
 TERNA_FUNCTION(linear_bf16_packed, 6)
 {
     const char* who = "bf16 linear on a packed weight";
-    const at::Tensor &x = *tensor(a[0]), &packed = *tensor(a[1]), &scale = *tensor(a[2]);
-    const at::Tensor* workspace = tensor(a[5]);
+    const at::Tensor &x = tensor(a[0]), &packed = tensor(a[1]), &scale = tensor(a[2]);
+    const at::Tensor* workspace = optional(a[5]);
     const int ws_num = integer32(a[3]);
     const int64_t n = integer32(a[4]);
     check_matrix(who, x);
@@ -290,8 +302,8 @@ TERNA_FUNCTION(linear_bf16_packed, 6)
 TERNA_FUNCTION(rmsnorm_quant, 5)
 {
     const char* who = "rmsnorm_quant";
-    const at::Tensor &x = *tensor(a[0]), &weight = *tensor(a[1]);
-    const at::Tensor* residual = tensor(a[3]);
+    const at::Tensor &x = tensor(a[0]), &weight = tensor(a[1]);
+    const at::Tensor* residual = optional(a[3]);
     const float eps = real(a[2]);
     check_matrix(who, x);
     const int64_t m = x.size(0), k = x.size(1);
@@ -317,7 +329,7 @@ TERNA_FUNCTION(rmsnorm_quant, 5)
 TERNA_FUNCTION(relu2_mul_rmsnorm_quant, 4)
 {
     const char* who = "relu2_mul_rmsnorm_quant";
-    const at::Tensor &x = *tensor(a[0]), &weight = *tensor(a[1]);
+    const at::Tensor &x = tensor(a[0]), &weight = tensor(a[1]);
     const float eps = real(a[2]);
     check_matrix(who, x);
     const int64_t m = x.size(0), f = x.size(1) / 2;
@@ -341,7 +353,7 @@ void check_stats(const char* who, const at::Tensor& stats, int64_t m)
 TERNA_FUNCTION(quant_from_stats, 4)
 {
     const char* who = "quant_from_stats";
-    const at::Tensor &h = *tensor(a[0]), &stats = *tensor(a[1]), &weight = *tensor(a[2]);
+    const at::Tensor &h = tensor(a[0]), &stats = tensor(a[1]), &weight = tensor(a[2]);
     const float eps = real(a[3]);
     check_matrix(who, h);
     const int64_t m = h.size(0), k = h.size(1);
@@ -361,8 +373,8 @@ TERNA_FUNCTION(quant_from_stats, 4)
 TERNA_FUNCTION(fused_linear, 17)
 {
     const char* who = "fused_linear";
-    const at::Tensor &x = *tensor(a[0]), &packed = *tensor(a[3]), &ws = *tensor(a[4]);
-    const at::Tensor *weight = tensor(a[1]), *stats = tensor(a[8]), *quantised = tensor(a[11]), *residual = tensor(a[13]), *next_weight = tensor(a[14]);
+    const at::Tensor &x = tensor(a[0]), &packed = tensor(a[3]), &ws = tensor(a[4]);
+    const at::Tensor *weight = optional(a[1]), *stats = optional(a[8]), *quantised = optional(a[11]), *residual = optional(a[13]), *next_weight = optional(a[14]);
     const int64_t n = integer32(a[6]), k = integer32(a[7]);
     ternaspmm_fused_linear_desc d{};
     d.eps = real(a[2]);
@@ -435,7 +447,7 @@ struct AttentionArgs {
 
     // a: cos, sin, pos, cache_k, cache_v, heads, head_dim, scale, adjacent; qkv is [new_rows = B * T, columns = (H + 2 KV) D]
     AttentionArgs(const char* who, PyObject* const* a, int64_t new_rows, int64_t columns)
-        : cos(*tensor(a[0])), sin(*tensor(a[1])), pos(*tensor(a[2])), ck(*tensor(a[3])), cv(*tensor(a[4])), heads(integer32(a[5])),
+        : cos(tensor(a[0])), sin(tensor(a[1])), pos(tensor(a[2])), ck(tensor(a[3])), cv(tensor(a[4])), heads(integer32(a[5])),
           head_dim(integer32(a[6])), scale(real(a[7])), adjacent(integer32(a[8]))
     {
         if (ck.dim() != 4 || ck.sizes() != cv.sizes() || ck.size(0) < 1 || ck.size(3) != head_dim || !ck.is_contiguous() || !cv.is_contiguous())
@@ -459,7 +471,7 @@ struct AttentionArgs {
 // the new rows of an attention call
 const at::Tensor& new_rows(const char* who, PyObject* o)
 {
-    const at::Tensor& qkv = *tensor(o);
+    const at::Tensor& qkv = tensor(o);
     check_matrix(who, qkv);
     if (!qkv.is_contiguous()) refuse("%s: qkv is a contiguous tensor", who);
     return qkv;
@@ -491,7 +503,7 @@ TERNA_FUNCTION(decode_attention, 14)
     const char* who = "decode_attention";
     const at::Tensor& qkv = new_rows(who, a[0]);
     const AttentionArgs g(who, a + 1, qkv.size(0), qkv.size(1));
-    const at::Tensor *workspace = tensor(a[10]), *weight = tensor(a[11]), *partial = tensor(a[12]);
+    const at::Tensor *workspace = optional(a[10]), *weight = optional(a[11]), *partial = optional(a[12]);
     if (g.t != 1) refuse("%s: one new token per sequence", who);
     const terna_stream st = stream();
     terna_bf16 *ck = data<terna_bf16>(&g.ck), *cv = data<terna_bf16>(&g.cv);
@@ -524,7 +536,7 @@ struct BlockLinear {
     const at::Tensor &packed, &ws;
     int ws_num;
     int64_t n;
-    BlockLinear(const char* who, PyObject* const* a, int64_t k) : packed(*tensor(a[0])), ws(*tensor(a[1])), ws_num(integer32(a[2])), n(integer32(a[3]))
+    BlockLinear(const char* who, PyObject* const* a, int64_t k) : packed(tensor(a[0])), ws(tensor(a[1])), ws_num(integer32(a[2])), n(integer32(a[3]))
     {
         check_weight(who, packed, ws, ws_num, n, k);
     }
@@ -537,9 +549,9 @@ struct BlockLinear {
 TERNA_FUNCTION(block, 35)
 {
     const char* who = "block";
-    const at::Tensor& x = *tensor(a[0]);
-    const at::Tensor *pending = tensor(a[1]), *attn_work = tensor(a[12]), *work = tensor(a[13]), *interleaved = tensor(a[34]);
-    const at::Tensor *norm[4] = {tensor(a[14]), tensor(a[15]), tensor(a[16]), tensor(a[17])};
+    const at::Tensor& x = tensor(a[0]);
+    const at::Tensor *pending = optional(a[1]), *attn_work = optional(a[12]), *work = optional(a[13]), *interleaved = optional(a[34]);
+    const at::Tensor *norm[4] = {&tensor(a[14]), &tensor(a[15]), &tensor(a[16]), &tensor(a[17])};
     const int64_t heads = integer32(a[7]), head_dim = integer32(a[8]);
     const float eps = real(a[11]);
     check_matrix(who, x);
@@ -628,7 +640,7 @@ TERNA_FUNCTION(block, 35)
 TERNA_FUNCTION(attention_merge_rmsnorm_quant, 8)
 {
     const char* who = "attention_merge_rmsnorm_quant";
-    const at::Tensor &partial = *tensor(a[0]), &weight = *tensor(a[4]);
+    const at::Tensor &partial = tensor(a[0]), &weight = tensor(a[4]);
     const int splits = integer32(a[1]), heads = integer32(a[2]), head_dim = integer32(a[3]), sequences = integer32(a[6]);
     const float eps = real(a[5]);
     const int64_t k = static_cast<int64_t>(heads) * head_dim;
@@ -647,7 +659,7 @@ TERNA_FUNCTION(attention_merge_rmsnorm_quant, 8)
 TERNA_FUNCTION(step_inputs, 5)
 {
     const char* who = "step_inputs";
-    const at::Tensor &tokens = *tensor(a[0]), &pos = *tensor(a[1]), &embedding = *tensor(a[2]), &table = *tensor(a[3]), &weight = *tensor(a[4]);
+    const at::Tensor &tokens = tensor(a[0]), &pos = tensor(a[1]), &embedding = tensor(a[2]), &table = tensor(a[3]), &weight = tensor(a[4]);
     check_matrix(who, embedding);
     const int64_t b = tokens.numel(), v = embedding.size(0), k = embedding.size(1);
     if (table.dim() != 3 || table.size(1) != 2 || tokens.scalar_type() != at::kLong || pos.scalar_type() != at::kLong || (pos.numel() != 1 && pos.numel() != b) ||
