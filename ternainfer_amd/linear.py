@@ -396,19 +396,24 @@ class SpBitLinear(_CompressedWeight):
     def forward(self, input):
         p = self._parameters
         packed = p.get("weight_packed")
-        work = get_global_workspace() if packed is None or input.numel() > 64 * self.in_features else None
-        out = _lib.native().bit_linear(input, packed, p["weight_bitmap"], p["weight_TileOffsets_global"],
-                                       p["weight_TileOffsets_median"], p["weight_compressed_val"], p["weight_scale"], self.ws_num,
-                                       self.out_features, work)
-        if out is not None:
-            return out
-        input, s = self.quant_input(input)        # other activation types and row lengths
+        if getattr(self.quant_input, "__func__", None) is _SPBITLINEAR_QUANT_INPUT:      # else: another quantiser than the library's
+            work = get_global_workspace() if packed is None or input.numel() > 64 * self.in_features else None
+            out = _lib.native().bit_linear(input, packed, p["weight_bitmap"], p["weight_TileOffsets_global"],
+                                           p["weight_TileOffsets_median"], p["weight_compressed_val"], p["weight_scale"], self.ws_num,
+                                           self.out_features, work)
+            if out is not None:
+                return out
+        input, s = self.quant_input(input)        # also other activation types and row lengths
         if self.weight_packed is not None:
             return TernaInfer_linear_packed(input, self.weight_packed, s, self.weight_scale,
                                             self.ws_num, self.out_features)
         return TernaInfer_linear(
             input, self.weight_compressed_val, self.weight_TileOffsets_global, self.weight_TileOffsets_median,
             self.weight_bitmap, get_global_workspace(), s, self.weight_scale, self.ws_num, self.out_features)
+
+
+#: the method `forward` may leave out: quantisation and linear in one native call
+_SPBITLINEAR_QUANT_INPUT = SpBitLinear.quant_input
 
 
 class SpBitLinearBF16(_CompressedWeight):

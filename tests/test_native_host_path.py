@@ -1,9 +1,10 @@
-"""The native host path (csrc/py_native.cpp) where it can be tested without a GPU: what it refuses before it looks at a tensor."""
+"""The native host path (csrc/py_native.cpp) and its callers where they can be tested without a GPU: what is refused before a
+tensor is looked at, and which calls take that path."""
 import numpy as np
 import pytest
 import torch
 
-from ternainfer_amd import _lib
+from ternainfer_amd import _lib, linear
 
 #: arguments of every function: T a tensor, o a tensor or None, i an integer, f a number, b a truth value
 ATTENTION = "TTTTTiifi"
@@ -53,3 +54,44 @@ def test_wrong_argument_count_raises_type_error():
     for name, kinds in SIGNATURES.items():
         with pytest.raises(TypeError, match="arguments expected"):
             getattr(_lib.native(), name)(*[None] * (len(kinds) + 1))
+
+
+class _Quantised(Exception):
+    pass
+
+
+def _own_quantiser(*_):
+    raise _Quantised
+
+
+def _module(cls=linear.SpBitLinear):
+    """An `SpBitLinear` of 64 x 64 without its weights on a GPU."""
+    m = cls.__new__(cls)
+    torch.nn.Module.__init__(m)
+    m.in_features = m.out_features = 64
+    m.ws_num = 1
+    for name in ("packed", "bitmap", "TileOffsets_global", "TileOffsets_median", "compressed_val", "scale"):
+        m.register_parameter("weight_" + name, torch.nn.Parameter(torch.zeros(1), requires_grad=False))
+    return m
+
+
+@pytest.mark.parametrize("how", ["subclass", "instance", "class"])
+def test_spbitlinear_calls_a_quant_input_of_its_own(how, monkeypatch):
+    """A `quant_input` that a subclass, an instance or a patch of the class brings is the one that `forward` quantises with; only
+    the module's own is left to the native call."""
+    taken = []
+    monkeypatch.setattr(_lib, "native", lambda: type("Native", (), {"bit_linear": staticmethod(lambda x, *_: taken.append(x) or x)}))
+    monkeypatch.setattr(linear, "get_global_workspace", lambda *_: None)
+    x = torch.zeros((2, 64), dtype=torch.bfloat16)
+    assert _module()(x) is x and len(taken) == 1
+    if how == "subclass":
+        module = _module(type("Own", (linear.SpBitLinear,), {"quant_input": _own_quantiser}))
+    else:
+        module = _module()
+        if how == "instance":
+            module.quant_input = _own_quantiser
+        else:
+            monkeypatch.setattr(linear.SpBitLinear, "quant_input", _own_quantiser)
+    with pytest.raises(_Quantised):
+        module(x)
+    assert len(taken) == 1
