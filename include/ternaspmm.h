@@ -350,6 +350,14 @@ int ternaspmm_step_inputs(const long long* tokens, const long long* pos, int per
                           const float* rope_table, int S, int rope_half, const terna_bf16* norm_weight, terna_bf16* x_out,
                           float* stats_out, float* rope_out, int B, terna_stream stream);
 
+/* The inputs of a pass over several new tokens (M = sequences x tokens of each), as indexing gives them: x_out bf16 [M][K] =
+ * embedding[tokens[r]] (negative tokens count from the end) and rope_out fp32 [2][pos_rows][rope_half] = the cos rows, then the
+ * sin rows, at pos[0 .. pos_rows - 1] (pos_rows = the tokens of one sequence where the sequences share their positions, else M).
+ * tokens, pos: int64 in device memory the host cannot check; one outside its table leaves a row of NaN.  Shapes and alignment as
+ * ternaspmm_step_inputs.  Returns 0 / -1.  Only enqueues. */
+int ternaspmm_prompt_inputs(const long long* tokens, const long long* pos, int pos_rows, const terna_bf16* embedding, int V, int K,
+                            const float* rope_table, int S, int rope_half, terna_bf16* x_out, float* rope_out, int M, terna_stream stream);
+
 /* Load time: band permutation of a P2 gate+up matrix [w1; w3] ([N][K], N = 2F) for TERNASPMM_EPILOGUE_GATE -- band 2j <-
  * rows 16j .. 16j+15 of w1, band 2j+1 <- the same rows of w3.  packed_out: N*K/4 bytes, not `packed`.  Returns 0 / -1. */
 int ternaspmm_interleave_gate_up(const void* packed, void* packed_out, int N, int K, terna_stream stream);

@@ -85,6 +85,33 @@ __global__ __launch_bounds__(256) void terna_step_inputs_kernel(const long long*
     }
 }
 
+// The inputs of a pass over T new tokens per sequence, as indexing gives them: x_out[r] = embedding[tokens[r]], negative tokens
+// counted from the end, and the RoPE rows of the positions (rope_out [2][gridDim.x or T][half]).  There is no host to raise an
+// error on: a token or position outside its table leaves a row of NaN, which every output that sees it shows.  One workgroup of
+// 256 threads per token; the copies of one row are all there is to do.
+__global__ __launch_bounds__(256) void terna_prompt_inputs_kernel(const long long* __restrict__ tokens, const long long* __restrict__ pos,
+                                                                   int pos_rows, const uint16_t* __restrict__ embedding, int V, int K,
+                                                                   const float* __restrict__ rope_table, int S, int half,
+                                                                   uint16_t* __restrict__ x_out, float* __restrict__ rope_out)
+{
+    const int tid = threadIdx.x;
+    const size_t r = blockIdx.x;
+    long long t = tokens[r];
+    if (t < 0) t += V;
+    const bool known = t >= 0 && t < V;
+    const u32x4* row = reinterpret_cast<const u32x4*>(embedding + static_cast<size_t>(known ? t : 0) * K);
+    u32x4* to = reinterpret_cast<u32x4*>(x_out + r * K);
+    for (int c = tid; c < K / 8; c += 256) to[c] = known ? row[c] : u32x4{0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u};
+    if (static_cast<int>(r) < pos_rows && tid < half / 2) {            // half is a multiple of 4: 16-byte pieces, cos row then sin row
+        const long long p = pos[r];
+        const bool inside = p >= 0 && p < S;
+        const int which = tid / (half / 4), piece = tid - which * (half / 4);
+        const f32x4 v = *reinterpret_cast<const f32x4*>(rope_table + (static_cast<size_t>(inside ? p : 0) * 2 + which) * half + 4 * piece);
+        *reinterpret_cast<f32x4*>(rope_out + (static_cast<size_t>(which) * pos_rows + r) * half + 4 * piece) =
+            inside ? v : f32x4{__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""), __builtin_nanf("")};
+    }
+}
+
 // Band permutation of a P2 gate+up matrix ([w1; w3], N = 2F rows) for the FEPI_GLU epilogue: band 2j <- band j (rows
 // 16j .. of w1), band 2j + 1 <- band F/16 + j (the same rows of w3).  One workgroup per destination band.
 __global__ __launch_bounds__(256) void terna_interleave_gate_up_kernel(const uint32_t* __restrict__ src, uint32_t* __restrict__ dst,
@@ -404,6 +431,23 @@ int ternaspmm_step_inputs(const long long* tokens, const long long* pos, int per
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) die("ternaspmm_step_inputs", e, __LINE__);
     return count;
+}
+
+int ternaspmm_prompt_inputs(const long long* tokens, const long long* pos, int pos_rows, const terna_bf16* embedding, int V, int K,
+                            const float* rope_table, int S, int rope_half, terna_bf16* x_out, float* rope_out, int M, terna_stream stream)
+{
+    if (M < 1 || pos_rows < 1 || pos_rows > M || V < 1 || S < 1 || K < 8 || (K & 7) || rope_half < 4 || (rope_half & 3) || rope_half > 512 ||
+        tokens == nullptr || pos == nullptr || embedding == nullptr || rope_table == nullptr || x_out == nullptr || rope_out == nullptr ||
+        ((reinterpret_cast<uintptr_t>(embedding) | reinterpret_cast<uintptr_t>(x_out) | reinterpret_cast<uintptr_t>(rope_table) |
+          reinterpret_cast<uintptr_t>(rope_out)) & 15)) {
+        std::fprintf(stderr, "ternaspmm_prompt_inputs: unsupported arguments (M=%d positions=%d V=%d K=%d S=%d rope_half=%d)\n", M, pos_rows, V, K, S, rope_half);
+        return -1;
+    }
+    terna_prompt_inputs_kernel<<<dim3(M), dim3(256), 0, static_cast<hipStream_t>(stream)>>>(tokens, pos, pos_rows, embedding, V, K, rope_table, S, rope_half,
+                                                                                            x_out, rope_out);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) die("ternaspmm_prompt_inputs", e, __LINE__);
+    return 0;
 }
 
 int ternaspmm_interleave_gate_up(const void* packed, void* packed_out, int N, int K, terna_stream stream)

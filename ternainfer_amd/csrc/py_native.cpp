@@ -49,7 +49,8 @@ namespace {
     X(ternaspmm_attention_workspace_bytes)                                                                             \
     X(ternaspmm_attention_merge_rmsnorm_quant)                                                                         \
     X(ternaspmm_row_stats_count)                                                                                       \
-    X(ternaspmm_step_inputs)
+    X(ternaspmm_step_inputs)                                                                                           \
+    X(ternaspmm_prompt_inputs)
 struct Library {
 #define X(name) decltype(&::name) name = nullptr;
     TERNA_ENTRY_POINTS(X)
@@ -679,6 +680,28 @@ TERNA_FUNCTION(step_inputs, 5)
     return pack(std::move(x), std::move(stats), std::move(rope));
 }
 
+// (tokens, pos, embedding, rope_table) -> (x, rope [2, positions, half]): int64 tokens [B, T] and positions of T or B T elements
+TERNA_FUNCTION(prompt_inputs, 4)
+{
+    const char* who = "prompt_inputs";
+    const at::Tensor &tokens = tensor(a[0]), &pos = tensor(a[1]), &embedding = tensor(a[2]), &table = tensor(a[3]);
+    check_matrix(who, embedding);
+    const int64_t m = tokens.numel(), v = embedding.size(0), k = embedding.size(1), rows = pos.numel();
+    if (tokens.dim() != 2 || m < 1 || m > INT32_MAX || (rows != m && rows != tokens.size(1)))
+        refuse("%s: tokens [B, T] and positions of T or B * T elements", who);
+    if (table.dim() != 3 || table.size(1) != 2 || tokens.scalar_type() != at::kLong || pos.scalar_type() != at::kLong || table.scalar_type() != at::kFloat ||
+        embedding.scalar_type() != at::kBFloat16 || !embedding.is_contiguous() || !table.is_contiguous())
+        refuse("%s: tokens / pos int64, embedding bf16 [V, K] and rope_table fp32 [S, 2, half] contiguous", who);
+    const at::Tensor ids = tokens.contiguous(), at_slot = pos.contiguous();
+    const int64_t slots = table.size(0), half = table.size(2);
+    at::Tensor x = make({m, k}, at::kBFloat16, embedding), rope = make({2, rows, half}, at::kFloat, embedding);
+    if (lib.ternaspmm_prompt_inputs(data<long long>(&ids), data<long long>(&at_slot), rows, data<terna_bf16>(&embedding), v, k, data<float>(&table), slots, half,
+                                    data<terna_bf16>(&x), data<float>(&rope), m, stream()) != 0)
+        refuse("%s: the library refused the launch (M=%d V=%d K=%d S=%d half=%d)", who, static_cast<int>(m), static_cast<int>(v), static_cast<int>(k),
+               static_cast<int>(slots), static_cast<int>(half));
+    return pack(std::move(x), std::move(rope));
+}
+
 // (path of libternaspmm.so)
 TERNA_FUNCTION(init, 1)
 {
@@ -703,7 +726,7 @@ TERNA_FUNCTION(init, 1)
 PyMethodDef methods[] = {METHOD(init), METHOD(bit_linear), METHOD(bit_linear_bf16), METHOD(quant_input), METHOD(linear_packed),
                          METHOD(linear_bf16_packed), METHOD(rmsnorm_quant), METHOD(relu2_mul_rmsnorm_quant), METHOD(quant_from_stats),
                          METHOD(fused_linear), METHOD(prompt_attention), METHOD(decode_attention), METHOD(block),
-                         METHOD(attention_merge_rmsnorm_quant), METHOD(step_inputs), {nullptr, nullptr, 0, nullptr}};
+                         METHOD(attention_merge_rmsnorm_quant), METHOD(step_inputs), METHOD(prompt_inputs), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

@@ -240,6 +240,14 @@ def step_inputs(tokens, pos, embedding, rope_table, norm_weight):
     return x, stats, rope[0], rope[1]
 
 
+def prompt_inputs(tokens, pos, embedding, rope_table):
+    """The inputs of a pass over T new tokens of B sequences in one launch (ternaspmm_prompt_inputs): tokens int [B, T], pos int64
+    [T] or [B, T], embedding and rope_table as for `step_inputs`.  Returns (x bf16 [B * T, K] = embedding[tokens], cos fp32
+    [T or B * T, half], sin) -- a row of NaN for a token or position outside its table."""
+    x, rope = _lib.native().prompt_inputs(tokens.long() if tokens.dtype == torch.int32 else tokens, pos, embedding, rope_table)
+    return x, rope[0], rope[1]
+
+
 def quant_from_stats(h, stats, norm_weight, eps):
     """Norm + quant_input of h bf16 [M, K] from the partials its producer left (ternaspmm_quant_from_stats):
     (xq int8 [M, K], s bf16 [M])."""

@@ -23,7 +23,7 @@ from torch.nn import functional as F
 
 from . import _lib
 from .linear import (EPILOGUE_GATE, EPILOGUE_RESIDUAL, argmax_rows, attention_merge_rmsnorm_linear_packed, attention_merge_rmsnorm_quant, fused_linear, get_global_workspace, greedy_step,
-                     greedy_step_state, interleave_gate_up, lm_head, quant_from_stats, quant_input, row_stats, relu2_mul_rmsnorm_linear_packed, relu2_mul_rmsnorm_quant, step_inputs,
+                     greedy_step_state, interleave_gate_up, lm_head, prompt_inputs, quant_from_stats, quant_input, row_stats, relu2_mul_rmsnorm_linear_packed, relu2_mul_rmsnorm_quant, step_inputs,
                      repack_weight, rmsnorm_linear_packed, rmsnorm_quant)
 
 
@@ -566,11 +566,11 @@ class Transformer:
         # one new token for a few sequences: the linears chained through producer-side norm statistics (forward_chain)
         chain = one_launch_attention and self.layers[0].act == "int8" and bsz <= max(self.chain_rows, self.split_rows) and getattr(self, "chain", True) and self.chain_supported()
         stats = None
-        if kernels_fit and bsz * t <= 65535 and getattr(self, "step_inputs", True) and self.chain_supported():
-            # embedding rows, their partials under the first block's norm (which only the chain reads) and the RoPE rows of the
-            # positions: one launch; positions that sequences share are repeated, their first T rows are what the kernels read
-            rows = pos_idx.repeat(bsz) if bsz > 1 and t > 1 and pos_idx.dim() == 1 else pos_idx.reshape(-1)
-            x, stats, cos, sin = step_inputs(tokens, rows, self.tok_embeddings, self.rope_tables(max_seq, dev), self.layers[0].attention_norm)
+        if chain and getattr(self, "step_inputs", True):
+            # embedding rows, their partials under the first block's norm and the RoPE rows of the positions: one launch
+            x, stats, cos, sin = step_inputs(tokens, pos_idx.reshape(-1), self.tok_embeddings, self.rope_tables(max_seq, dev), self.layers[0].attention_norm)
+        elif kernels_fit and getattr(self, "step_inputs", True) and a.dim % 8 == 0:
+            x, cos, sin = prompt_inputs(tokens, pos_idx, self.tok_embeddings, self.rope_tables(max_seq, dev))
         else:
             rows = self.rope_tables(max_seq, dev).index_select(0, pos_idx.reshape(-1))   # fp32 [T | B*T, 2, head_dim / 2]
             cos, sin = rows[:, 0].contiguous(), rows[:, 1].contiguous()       # views when one row

@@ -129,6 +129,35 @@ def test_step_inputs_clamps_and_refuses():
     torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("b,t,v,k,s_len,half,per_seq", [(1, 1, 50, 8, 7, 4, False), (1, 300, 128256, 2560, 384, 64, False), (5, 7, 1000, 520, 40, 32, True),
+                                                          (3, 2, 300, 6912, 2048, 512, False), (17, 1, 64, 4104, 9, 32, True)])
+def test_prompt_inputs(b, t, v, k, s_len, half, per_seq):
+    """ternaspmm_prompt_inputs against indexing: both index types, negative tokens from the end, strided views; rows of NaN for what
+    lies outside the tables, and nothing beside them."""
+    gen = torch.Generator().manual_seed(1350 + b + k)
+    emb = (torch.randn((v, k), generator=gen) * 0.02).to(torch.bfloat16).cuda()
+    table = torch.randn((s_len, 2, half), generator=gen).cuda()
+    tokens = torch.randint(-v, v, (b, t), generator=gen).cuda()
+    tokens[-1, -1], tokens[0, 0] = v - 1, -v
+    pos = torch.randint(0, s_len, (b, t) if per_seq else (t,), generator=gen).cuda()
+    pos.view(-1)[-1] = s_len - 1
+    print(f"[case] prompt inputs b={b} t={t} v={v} k={k} S={s_len} half={half} per_seq={per_seq}", flush=True)
+    want, rows = emb[tokens.reshape(-1)], table.index_select(0, pos.reshape(-1))
+    for ids in (tokens, tokens.to(torch.int32), tokens.t().contiguous().t()):
+        x, cos, sin = L.prompt_inputs(ids, pos, emb, table)
+        torch.cuda.synchronize()
+        assert torch.equal(x, want) and torch.equal(cos, rows[:, 0]) and torch.equal(sin, rows[:, 1])
+        assert cos.is_contiguous() and sin.is_contiguous()
+    for token, slot in ((v, s_len), (-v - 1, -1), (2 ** 40, -2 ** 40)):
+        wrong, at = tokens.clone(), pos.clone()
+        wrong[b // 2, t // 2], at.view(-1)[0] = token, slot
+        x, cos, sin = L.prompt_inputs(wrong, at, emb, table)
+        r = (b // 2) * t + t // 2
+        assert torch.isnan(x[r]).all() and torch.isnan(cos[0]).all() and torch.isnan(sin[0]).all()
+        keep = torch.arange(b * t, device="cuda") != r
+        assert torch.equal(x[keep], want[keep]) and torch.equal(cos[1:], rows[1:, 0]) and torch.equal(sin[1:], rows[1:, 1])
+
+
 @pytest.mark.parametrize("m", [1, 2, 3, 4, 8])
 @pytest.mark.parametrize("n,k,ws_num", [(3840, 2560, 3), (2560, 2560, 1), (2560, 6912, 1), (256, 192, 2)])
 def test_stats_prologue_with_store_and_residual_epilogues(m, n, k, ws_num):

@@ -325,3 +325,31 @@ def test_native_block_is_the_launches_one_by_one(batch, tokens, per_seq):
         results.append([logits] + [t for pair in cache for t in pair])
     for mine, theirs in zip(*results):
         assert torch.equal(mine, theirs)
+
+
+@pytest.mark.parametrize("batch,tokens", [(1, 9), (3, 5), (17, 1)])
+def test_token_ids_are_indices(batch, tokens):
+    """The token ids of a prompt pass, and of a step of many sequences, are indices of the embedding: int32 ids and ids from the end
+    give the same bits, an id outside the table gives NaN logits in its sequence and changes no other."""
+    from ternainfer_amd.model import ModelArgs, Transformer
+    args = ModelArgs(dim=256, n_layers=2, n_heads=4, n_kv_heads=2, vocab_size=512, ffn_dim=384)
+    model = Transformer(args, seed=32)
+    ids = torch.randint(0, args.vocab_size, (batch, tokens), generator=torch.Generator().manual_seed(4)).cuda()
+    ids[0, 0] = args.vocab_size - 1
+    pos = torch.arange(tokens, device="cuda") + 2
+    print(f"[case] token ids as indices batch={batch} tokens={tokens}", flush=True)
+
+    def logits(t):
+        with torch.inference_mode():
+            return model.forward(t, model.make_cache(batch, tokens + 8), pos)
+
+    want = logits(ids)
+    assert torch.isfinite(want).all()
+    from_end = ids.clone()
+    from_end[0, 0] = -1
+    assert torch.equal(logits(ids.to(torch.int32)), want) and torch.equal(logits(from_end), want)
+    for outside in (args.vocab_size, -args.vocab_size - 1):
+        wrong = ids.clone()
+        wrong[0, 0] = outside
+        got = logits(wrong)
+        assert torch.isnan(got[0]).all() and torch.equal(got[1:], want[1:])

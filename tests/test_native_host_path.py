@@ -13,6 +13,7 @@ SIGNATURES = {
     "rmsnorm_quant": "TTfob", "relu2_mul_rmsnorm_quant": "TTfb", "quant_from_stats": "TTTf", "fused_linear": "TofTTiiioiioioobb",
     "prompt_attention": "T" + ATTENTION + "b", "decode_attention": "T" + ATTENTION + "oooi",
     "block": "To" + ATTENTION + "foo" + "TTTT" + "TTii" * 4 + "o", "attention_merge_rmsnorm_quant": "TiiiTfib", "step_inputs": "TTTTT",
+    "prompt_inputs": "TTTT",
 }
 VALUES = {"T": torch.zeros((1, 64)), "o": None, "i": 1, "f": 1.0, "b": False}
 
