@@ -1,5 +1,5 @@
 #!/usr/bin/env bash
-# Builds kernels/libternaspmm.so for MI355X (gfx950) and the tests/test_kernel harness.
+# Builds kernels/libternaspmm.so for MI355X (gfx950), the Python package's native host path and the tests/test_kernel harness.
 # Run from anywhere:  bash kernels/compile.sh
 # One hipcc compile per translation unit, all at once (each kernel family is instantiated in a
 # file of its own), then one link.  -amdgpu-kernarg-preload-count: the first 16 dwords of a kernel's
@@ -36,14 +36,24 @@ compile abi_prefill_attention.hip abi_prefill_attention.o -mllvm -amdgpu-mfma-vg
 compile abi_head.hip abi_head.o
 compile abi_probe.hip abi_probe.o
 compile format_host.cpp format_host.o
-# the host path of the Python package: a CPython module on torch's C++ headers, bound to the library at run time
-torch="$(python3 -c 'import os, torch; print(os.path.dirname(torch.__file__))')"
-python_include="$(python3 -c 'import sysconfig; print(sysconfig.get_paths()["include"])')"
-g++ -std=c++17 -O2 -fPIC -shared -Wall -Wno-unused-function -D__HIP_PLATFORM_AMD__=1 -DUSE_ROCM=1 \
-    -isystem "$torch/include" -isystem "$torch/include/torch/csrc/api/include" -isystem "$python_include" -isystem /opt/rocm/include \
-    "$src/py_native.cpp" -L"$torch/lib" -ltorch_python -ltorch_hip -ltorch_cpu -lc10 -lc10_hip -ldl -o "$here/../ternainfer_amd/_native.so" &
-pids+=($!)
-for p in "${pids[@]}"; do wait "$p"; done
+# The host path of the Python package: a CPython module on torch's C++ headers, bound to the library at run time.  The library
+# itself needs neither; where they are missing it is all that is built, and the package says so when it is used.
+native=
+if torch="$(python3 -c 'import os, torch; print(os.path.dirname(torch.__file__))' 2> /dev/null)"; then
+    python_include="$(python3 -c 'import sysconfig; print(sysconfig.get_paths()["include"])')"
+    g++ -std=c++17 -O2 -fPIC -shared -Wall -Wno-unused-function -D__HIP_PLATFORM_AMD__=1 -DUSE_ROCM=1 \
+        -isystem "$torch/include" -isystem "$torch/include/torch/csrc/api/include" -isystem "$python_include" -isystem /opt/rocm/include \
+        "$src/py_native.cpp" -L"$torch/lib" -ltorch_python -ltorch_hip -ltorch_cpu -lc10 -lc10_hip -ldl -o "$here/../ternainfer_amd/_native.so" &
+    native=$!
+else
+    echo "compile.sh: python3 has no PyTorch: the Python package's ternainfer_amd/_native.so is not built" >&2
+fi
+# every compile is waited for, also behind one that failed: none is left running
+failed=0
+for p in "${pids[@]}"; do wait "$p" || failed=1; done
+native_failed=0
+if [ -n "$native" ]; then wait "$native" || native_failed=1; fi
+[ "$failed" = 0 ]
 
 hipcc -shared -fPIC --offload-arch=gfx950 "$obj"/*.o -o "$here/libternaspmm.so"
 
@@ -54,3 +64,4 @@ if [ -f "$here/../tests/test_kernel.hip" ]; then
         -Wl,-rpath,'$ORIGIN/../kernels' \
         -o "$here/../tests/test_kernel"
 fi
+[ "$native_failed" = 0 ]
