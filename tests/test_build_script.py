@@ -34,23 +34,25 @@ def _build(tmp_path, python, **env):
         (tools / name).symlink_to(shutil.which(name))
     log = tmp_path / "log"
     log.write_text("")
-    r = subprocess.run(["bash", str(tree / "kernels" / "compile.sh")], env={"PATH": str(tools), "LOG": str(log), **env}, capture_output=True, text=True, timeout=60)
-    return r, tree, log.read_text().split()
+    said = tmp_path / "said"                      # (a file: a pipe would wait for whatever the script leaves running)
+    with open(said, "w") as f:
+        code = subprocess.run(["bash", str(tree / "kernels" / "compile.sh")], env={"PATH": str(tools), "LOG": str(log), **env}, stdout=f, stderr=f, timeout=60).returncode
+    return code, said.read_text(), tree, log.read_text().split()
 
 
 @pytest.mark.parametrize("python", sorted(PYTHON))
 def test_library_is_built_without_pytorch(tmp_path, python):
-    r, tree, log = _build(tmp_path, python)
-    assert r.returncode == 0, r.stderr
+    code, said, tree, log = _build(tmp_path, python)
+    assert code == 0, said
     assert (tree / "kernels" / "libternaspmm.so").exists()
     assert (tree / "ternainfer_amd" / "_native.so").exists() == (python == "torch")
-    assert ("no PyTorch" in r.stderr) == (python != "torch")
+    assert ("no PyTorch" in said) == (python != "torch")
     assert log.count("start") == log.count("end")
 
 
 @pytest.mark.parametrize("source,library", [("ternaspmm.hip", False), ("py_native.cpp", True)])
 def test_a_failed_compile_fails_the_build_and_leaves_none_running(tmp_path, source, library):
-    r, tree, log = _build(tmp_path, "torch", FAIL=source, DELAY="0.3")
-    assert r.returncode != 0
+    code, _, tree, log = _build(tmp_path, "torch", FAIL=source, DELAY="0.3")
+    assert code != 0
     assert log.count("failed") == 1 and log.count("start") == log.count("end") + 1
     assert (tree / "kernels" / "libternaspmm.so").exists() == library
