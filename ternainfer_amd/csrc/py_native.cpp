@@ -5,7 +5,8 @@
 //
 // Every function checks shapes and element counts before anything is enqueued (the C ABI takes pointers on trust) and
 // raises ValueError, or TypeError where an argument is no tensor; the tensors' types and devices are the caller's business
-// where linear.py does not state otherwise.
+// where linear.py does not state otherwise.  What follows the checks -- allocations, copies, launches, which may wait for the
+// device -- runs without the interpreter's lock, as the same calls do from Python.
 #include <dlfcn.h>
 
 #include <torch/csrc/Exceptions.h>
@@ -58,6 +59,21 @@ struct Library {
 } lib;
 
 struct Refused : std::exception {};            // a Python error is set
+
+// From its construction to end() other Python threads run: no Python object is touched and nothing refused in between.
+class Unlocked {
+    PyThreadState* state = PyEval_SaveThread();
+
+public:
+    Unlocked() = default;
+    Unlocked(const Unlocked&) = delete;
+    ~Unlocked() { end(); }
+    void end()
+    {
+        if (state != nullptr) PyEval_RestoreThread(state);
+        state = nullptr;
+    }
+};
 
 // an argument that is a tensor
 const at::Tensor& tensor(PyObject* o)
@@ -144,26 +160,36 @@ QuantRows make_quant_rows(int64_t m, int64_t k)
     return r;
 }
 
-PyObject* wrap(at::Tensor t) { return THPVariable_Wrap(std::move(t)); }
-PyObject* wrap_or_none(at::Tensor t) { return t.defined() ? wrap(std::move(t)) : Py_NewRef(Py_None); }
-template <typename... Ts>
-PyObject* pack(Ts&&... items)
+// Results: the end of an unlocked stretch.
+PyObject* none(Unlocked& unlocked)
 {
+    unlocked.end();
+    Py_RETURN_NONE;
+}
+PyObject* wrap(at::Tensor t, Unlocked& unlocked)
+{
+    unlocked.end();
+    return THPVariable_Wrap(std::move(t));
+}
+PyObject* wrap_or_none(at::Tensor t) { return t.defined() ? THPVariable_Wrap(std::move(t)) : Py_NewRef(Py_None); }
+template <typename... Ts>
+PyObject* pack(Unlocked& unlocked, Ts&&... items)
+{
+    unlocked.end();
     PyObject* tuple = PyTuple_New(sizeof...(items));
     Py_ssize_t i = 0;
     (PyTuple_SET_ITEM(tuple, i++, wrap_or_none(std::forward<Ts>(items))), ...);
     return tuple;
 }
 
-// A module's activations as the kernels read them: bf16 rows on the current device, in one piece.  False: something the
-// native path does not take (another type, an empty batch ...), linear.py goes on.
-bool bf16_rows(const at::Tensor& x, at::Tensor* rows, int64_t* m, int64_t* k)
+// A module's activations: bf16 rows on the current device.  False: something the native path does not take (another type, an
+// empty batch ...), linear.py goes on.
+bool bf16_rows(const at::Tensor& x, int64_t* m, int64_t* k)
 {
     if (!x.is_cuda() || x.scalar_type() != at::kBFloat16 || x.dim() < 1) return false;
     *k = x.size(-1);
     if (*k < 64 || x.numel() == 0 || x.device().index() != c10::hip::current_device()) return false;
     *m = x.numel() / *k;
-    *rows = x.is_contiguous() ? x : x.contiguous();
     return *m <= INT32_MAX && *k <= INT32_MAX;
 }
 at::Tensor make_output(const at::Tensor& x, int64_t n)
@@ -204,11 +230,12 @@ TERNA_FUNCTION(bit_linear, 10)
     const at::Tensor *packed = optional(a[1]), *workspace = optional(a[9]);
     const int ws_num = integer32(a[7]);
     const int64_t n = integer32(a[8]);
-    at::Tensor rows;
     int64_t m, k;
-    if (!bf16_rows(x, &rows, &m, &k) || k > 8192) Py_RETURN_NONE;
+    if (!bf16_rows(x, &m, &k) || k > 8192) Py_RETURN_NONE;
     if (packed != nullptr) check_weight("SpBitLinear", *packed, ws, ws_num, n, k);
     else check_format("SpBitLinear", bitmap, n, k);
+    Unlocked unlocked;
+    const at::Tensor rows = x.contiguous();
     at::Tensor out = make_output(x, n);
     const terna_stream st = stream();
     if (m <= 8) {                       // a few rows: both steps in one launch
@@ -217,17 +244,17 @@ TERNA_FUNCTION(bit_linear, 10)
                                            : lib.bitlinear_TernaSpMM_quant(data<terna_bf16>(&rows), data<uint64_t>(&bitmap), data<int>(&offsets),
                                                                            data<uint16_t>(&median), data<uint32_t>(&signs), data<terna_bf16>(&out),
                                                                            data<terna_bf16>(&ws), ws_num, m, n, k, st);
-        if (done) return wrap(std::move(out));
+        if (done) return wrap(std::move(out), unlocked);
     }
     QuantRows q = make_quant_rows(m, k);
-    if (lib.ternaspmm_quant_input(data<terna_bf16>(&rows), q.q, q.s, m, k, st) != 0) Py_RETURN_NONE;
+    if (lib.ternaspmm_quant_input(data<terna_bf16>(&rows), q.q, q.s, m, k, st) != 0) return none(unlocked);
     if (packed != nullptr)
         lib.bitlinear_TernaSpMM_packed_ws(q.q, data(packed), data<terna_bf16>(&out), q.s, data<terna_bf16>(&ws), ws_num, m, n, k, 0,
                                           data(workspace), workspace != nullptr ? workspace->numel() : 0, st);
     else
         lib.bitlinear_TernaSpMM(q.q, data<uint64_t>(&bitmap), data<int>(&offsets), data<uint16_t>(&median), data<uint32_t>(&signs),
                                 data<terna_bf16>(&out), q.s, data<terna_bf16>(&ws), ws_num, m, n, k, 7, data<int32_t>(workspace), st);
-    return wrap(std::move(out));
+    return wrap(std::move(out), unlocked);
 }
 
 // (x, bitmap, tile offsets, median offsets, signs, scale, ws_num, out_features, route 0 auto / 1 decode / 2 prefill)
@@ -236,30 +263,32 @@ TERNA_FUNCTION(bit_linear_bf16, 9)
     const at::Tensor &x = tensor(a[0]), &bitmap = tensor(a[1]), &offsets = tensor(a[2]), &median = tensor(a[3]), &signs = tensor(a[4]), &scale = tensor(a[5]);
     const int ws_num = integer32(a[6]), route = integer32(a[8]);
     const int64_t n = integer32(a[7]);
-    at::Tensor rows;
     int64_t m, k;
-    if (!bf16_rows(x, &rows, &m, &k)) Py_RETURN_NONE;
+    if (!bf16_rows(x, &m, &k)) Py_RETURN_NONE;
     check_format("TernaInfer_linear_bf16", bitmap, n, k);
+    Unlocked unlocked;
+    const at::Tensor rows = x.contiguous();
     at::Tensor out = make_output(x, n);
     const auto fn = route == 1 ? lib.bitlinear_TernaSpMM_bf16_decode : route == 2 ? lib.bitlinear_TernaSpMM_bf16_prefill : lib.bitlinear_TernaSpMM_bf16;
     fn(data<terna_bf16>(&rows), data<uint64_t>(&bitmap), data<int>(&offsets), data<uint16_t>(&median), data<uint32_t>(&signs),
        data<terna_bf16>(&out), data<float>(&scale), ws_num, m, n, k, 1, nullptr, stream());
-    return wrap(std::move(out));
+    return wrap(std::move(out), unlocked);
 }
 
 // (x bf16 [..., K]) -> (int8 [..., K], bf16 [..., 1]), or None
 TERNA_FUNCTION(quant_input, 1)
 {
     const at::Tensor& x = tensor(a[0]);
-    at::Tensor rows;
     int64_t m, k;
-    if (!bf16_rows(x, &rows, &m, &k)) Py_RETURN_NONE;
+    if (!bf16_rows(x, &m, &k)) Py_RETURN_NONE;
+    Unlocked unlocked;
+    const at::Tensor rows = x.contiguous();
     at::DimVector shape(x.sizes());
     at::Tensor q = make(shape, at::kChar, x);
     shape.back() = 1;
     at::Tensor s = make(shape, at::kBFloat16, x);
-    if (lib.ternaspmm_quant_input(data<terna_bf16>(&rows), data<int8_t>(&q), data<terna_bf16>(&s), m, k, stream()) != 0) Py_RETURN_NONE;
-    return pack(std::move(q), std::move(s));
+    if (lib.ternaspmm_quant_input(data<terna_bf16>(&rows), data<int8_t>(&q), data<terna_bf16>(&s), m, k, stream()) != 0) return none(unlocked);
+    return pack(unlocked, std::move(q), std::move(s));
 }
 
 // (x int8 [M, K], s, packed, ws, ws_num, out_features, workspace | None)
@@ -274,11 +303,12 @@ TERNA_FUNCTION(linear_packed, 7)
     const int64_t m = x.size(0), k = x.size(1);
     check_numel(who, "s", &s, m);
     check_weight(who, packed, ws, ws_num, n, k);
+    Unlocked unlocked;
     const at::Tensor rows = x.contiguous(), scales = s.contiguous();
     at::Tensor out = make({m, n}, at::kBFloat16, x);
     lib.bitlinear_TernaSpMM_packed_ws(data<int8_t>(&rows), data(&packed), data<terna_bf16>(&out), data<terna_bf16>(&scales), data<terna_bf16>(&ws),
                                       ws_num, m, n, k, 0, data(workspace), workspace != nullptr ? workspace->numel() : 0, stream());
-    return wrap(std::move(out));
+    return wrap(std::move(out), unlocked);
 }
 
 // (x bf16 [M, K], packed, scale fp32, ws_num, out_features, workspace | None)
@@ -292,11 +322,12 @@ TERNA_FUNCTION(linear_bf16_packed, 6)
     check_matrix(who, x);
     const int64_t m = x.size(0), k = x.size(1);
     check_weight(who, packed, scale, ws_num, n, k);
+    Unlocked unlocked;
     const at::Tensor rows = x.contiguous();
     at::Tensor out = make({m, n}, at::kBFloat16, x);
     lib.bitlinear_TernaSpMM_bf16_packed_ws(data<terna_bf16>(&rows), data(&packed), data<terna_bf16>(&out), data<float>(&scale), ws_num, m, n, k, 0,
                                            data(workspace), workspace != nullptr ? workspace->numel() : 0, stream());
-    return wrap(std::move(out));
+    return wrap(std::move(out), unlocked);
 }
 
 // (x, weight, eps, residual | None, quant) -> (xq, s, h) or (y, None, h)
@@ -310,20 +341,21 @@ TERNA_FUNCTION(rmsnorm_quant, 5)
     const int64_t m = x.size(0), k = x.size(1);
     check_numel(who, "residual", residual, m * k);
     check_numel(who, "weight", &weight, k);
+    const bool quant = PyObject_IsTrue(a[4]);
+    Unlocked unlocked;
     const at::Tensor rows = x.contiguous();
     at::Tensor added, h = rows, q, s;
     if (residual != nullptr) {
         added = residual->contiguous();
         h = make({m, k}, at::kBFloat16, x);
     }
-    const bool quant = PyObject_IsTrue(a[4]);
     q = make({m, k}, quant ? at::kChar : at::kBFloat16, x);
     if (quant) s = make({m}, at::kBFloat16, x);
     lib.ternaspmm_rmsnorm_quant(data<terna_bf16>(&rows), residual != nullptr ? data<terna_bf16>(&added) : nullptr,
                                 residual != nullptr ? data<terna_bf16>(&h) : nullptr, data<terna_bf16>(&weight), eps,
                                 quant ? nullptr : data<terna_bf16>(&q), quant ? data<int8_t>(&q) : nullptr, quant ? data<terna_bf16>(&s) : nullptr, m, k,
                                 stream());
-    return pack(std::move(q), std::move(s), residual != nullptr ? std::move(h) : x.is_contiguous() ? x : rows);
+    return pack(unlocked, std::move(q), std::move(s), std::move(h));             // (x itself where it is neither added to nor copied)
 }
 
 // (x13, weight, eps, quant) -> (xq, s) or (y, None)
@@ -335,13 +367,14 @@ TERNA_FUNCTION(relu2_mul_rmsnorm_quant, 4)
     check_matrix(who, x);
     const int64_t m = x.size(0), f = x.size(1) / 2;
     check_numel(who, "weight", &weight, f);
-    const at::Tensor rows = x.contiguous();
     const bool quant = PyObject_IsTrue(a[3]);
+    Unlocked unlocked;
+    const at::Tensor rows = x.contiguous();
     at::Tensor q = make({m, f}, quant ? at::kChar : at::kBFloat16, x), s;
     if (quant) s = make({m}, at::kBFloat16, x);
     lib.ternaspmm_relu2_mul_rmsnorm_quant(data<terna_bf16>(&rows), data<terna_bf16>(&weight), eps, quant ? nullptr : data<terna_bf16>(&q),
                                           quant ? data<int8_t>(&q) : nullptr, quant ? data<terna_bf16>(&s) : nullptr, m, f, stream());
-    return pack(std::move(q), std::move(s));
+    return pack(unlocked, std::move(q), std::move(s));
 }
 
 void check_stats(const char* who, const at::Tensor& stats, int64_t m)
@@ -360,12 +393,14 @@ TERNA_FUNCTION(quant_from_stats, 4)
     const int64_t m = h.size(0), k = h.size(1);
     check_numel(who, "norm_weight", &weight, k);
     check_stats(who, stats, m);
+    Unlocked unlocked;
     const at::Tensor rows = h.contiguous();
     at::Tensor q = make({m, k}, at::kChar, h), s = make({m}, at::kBFloat16, h);
-    if (lib.ternaspmm_quant_from_stats(data<terna_bf16>(&rows), data<float>(&stats), stats.size(1), data<terna_bf16>(&weight), eps, data<int8_t>(&q),
-                                       data<terna_bf16>(&s), m, k, stream()) != 0)
-        refuse("%s: unsupported shape M=%d K=%d", who, static_cast<int>(m), static_cast<int>(k));
-    return pack(std::move(q), std::move(s));
+    const int rc = lib.ternaspmm_quant_from_stats(data<terna_bf16>(&rows), data<float>(&stats), stats.size(1), data<terna_bf16>(&weight), eps,
+                                                  data<int8_t>(&q), data<terna_bf16>(&s), m, k, stream());
+    unlocked.end();
+    if (rc != 0) refuse("%s: unsupported shape M=%d K=%d", who, static_cast<int>(m), static_cast<int>(k));
+    return pack(unlocked, std::move(q), std::move(s));
 }
 
 // (x, norm_weight | None, eps, packed, ws, ws_num, out_features, in_features, stats | None, attention splits (0: none), head_dim,
@@ -391,14 +426,11 @@ TERNA_FUNCTION(fused_linear, 17)
         check_matrix(who, x);
         m = x.size(0);
         if (x.size(1) != k) refuse("%s: expected a [M, %lld] tensor", who, static_cast<long long>(k));
-        rows = x.contiguous();
         if (quantised != nullptr) {
             d.prologue = TERNASPMM_PROLOGUE_QUANTISED;
             check_numel(who, "s", quantised, m);
             if (x.scalar_type() != at::kChar || quantised->scalar_type() != at::kBFloat16)
                 refuse("%s: quantised activations are int8 with bf16 scales", who);
-            scales = quantised->contiguous();
-            d.s_in = data<terna_bf16>(&scales);
         } else {
             d.prologue = stats != nullptr ? TERNASPMM_PROLOGUE_STATS : TERNASPMM_PROLOGUE_NORM;
             check_numel(who, "norm_weight", weight, k);
@@ -406,7 +438,7 @@ TERNA_FUNCTION(fused_linear, 17)
     }
     check_weight(who, packed, ws, d.ws_num, n, k);
     d.M = m, d.N = n, d.K = k;
-    d.x = data(&rows), d.packed = data(&packed), d.ws = data<terna_bf16>(&ws), d.norm_weight = data<terna_bf16>(weight);
+    d.packed = data(&packed), d.ws = data<terna_bf16>(&ws), d.norm_weight = data<terna_bf16>(weight);
     if (stats != nullptr) {
         check_stats(who, *stats, m);
         d.stats_in = data<float>(stats), d.stats_count = stats->size(1);
@@ -417,12 +449,23 @@ TERNA_FUNCTION(fused_linear, 17)
     if (d.epilogue == TERNASPMM_EPILOGUE_RESIDUAL) {
         if (residual == nullptr || residual->numel() != m * n || residual->scalar_type() != at::kBFloat16)
             refuse("%s: the residual epilogue needs a bf16 [M, N] stream", who);
+    }
+    const bool want_raw = d.epilogue == TERNASPMM_EPILOGUE_RESIDUAL && PyObject_IsTrue(a[15]), publish = PyObject_IsTrue(a[16]);
+
+    Unlocked unlocked;
+    if (d.attention_splits <= 0) rows = x.contiguous();
+    d.x = data(&rows);
+    if (d.prologue == TERNASPMM_PROLOGUE_QUANTISED) {
+        scales = quantised->contiguous();
+        d.s_in = data<terna_bf16>(&scales);
+    }
+    if (d.epilogue == TERNASPMM_EPILOGUE_RESIDUAL) {
         stream_in = residual->contiguous();
         d.residual = data<terna_bf16>(&stream_in);
-        if (PyObject_IsTrue(a[15])) {
-            raw = make({m, n}, at::kBFloat16, packed);
-            d.raw_out = data<terna_bf16>(&raw);
-        }
+    }
+    if (want_raw) {
+        raw = make({m, n}, at::kBFloat16, packed);
+        d.raw_out = data<terna_bf16>(&raw);
     }
     out = make({m, columns}, at::kBFloat16, packed);
     d.out = data<terna_bf16>(&out);
@@ -430,12 +473,12 @@ TERNA_FUNCTION(fused_linear, 17)
         stats_out = make({m, columns / 16, 2}, at::kFloat, packed);
         d.next_norm_weight = data<terna_bf16>(next_weight), d.stats_out = data<float>(&stats_out);
     }
-    if (PyObject_IsTrue(a[16])) {
+    if (publish) {
         xq = make({m, k}, at::kChar, packed), s = make({m}, at::kBFloat16, packed);
         d.xq_out = data<int8_t>(&xq), d.s_out = data<terna_bf16>(&s);
     }
-    if (lib.ternaspmm_fused_linear(&d, stream()) < 0) Py_RETURN_NONE;
-    return pack(std::move(out), std::move(stats_out), std::move(raw), std::move(xq), std::move(s));
+    if (lib.ternaspmm_fused_linear(&d, stream()) < 0) return none(unlocked);
+    return pack(unlocked, std::move(out), std::move(stats_out), std::move(raw), std::move(xq), std::move(s));
 }
 
 // What the attention entry points read beside a block's new rows, checked against these and each other.
@@ -485,15 +528,17 @@ TERNA_FUNCTION(prompt_attention, 11)
     const char* who = "prompt_attention";
     const at::Tensor& qkv = new_rows(who, a[0]);
     const AttentionArgs g(who, a + 1, qkv.size(0), qkv.size(1));
+    const bool attention = PyObject_IsTrue(a[10]);
+    Unlocked unlocked;
     at::Tensor q = make({g.batch, g.heads, g.t, g.head_dim}, at::kBFloat16, qkv);
     const terna_stream st = stream();
     lib.ternaspmm_rope_kv_store(TERNA_ATTENTION_INPUTS(data<terna_bf16>(&qkv), g), data<terna_bf16>(&q), data<terna_bf16>(&g.ck), data<terna_bf16>(&g.cv), g.batch, g.t, g.heads,
                                 g.kv, g.head_dim, g.slots, g.adjacent, st);
-    if (!PyObject_IsTrue(a[10])) return wrap(std::move(q));
+    if (!attention) return wrap(std::move(q), unlocked);
     at::Tensor o = make({g.batch * g.t, g.heads * g.head_dim}, at::kBFloat16, qkv);
     lib.ternaspmm_prefill_attention(data<terna_bf16>(&q), data<terna_bf16>(&g.ck), data<terna_bf16>(&g.cv), data<long long>(&g.pos), g.each,
                                     data<terna_bf16>(&o), g.batch, g.t, g.heads, g.kv, g.head_dim, g.slots, g.scale, st);
-    return wrap(std::move(o));
+    return wrap(std::move(o), unlocked);
 }
 
 // (qkv, the nine of AttentionArgs, workspace | None, norm_weight | None, partial | None, splits): RoPE, cache write and attention of one new
@@ -511,25 +556,29 @@ TERNA_FUNCTION(decode_attention, 14)
     if (partial != nullptr) {
         const long long need = lib.ternaspmm_attention_partial_bytes(g.batch, g.heads, g.head_dim);
         if (need < 0 || static_cast<long long>(partial->numel() * partial->element_size()) < need) refuse("%s: the partial buffer is too small", who);
-        lib.ternaspmm_rope_decode_attention_partial(TERNA_ATTENTION_INPUTS(data<terna_bf16>(&qkv), g), ck, cv, data<float>(partial), integer32(a[13]), g.batch, g.heads, g.kv,
+        const int splits = integer32(a[13]);
+        Unlocked unlocked;
+        lib.ternaspmm_rope_decode_attention_partial(TERNA_ATTENTION_INPUTS(data<terna_bf16>(&qkv), g), ck, cv, data<float>(partial), splits, g.batch, g.heads, g.kv,
                                                     g.head_dim, g.slots, g.scale, g.adjacent, nullptr, nullptr, nullptr, 0, st);
-        Py_RETURN_NONE;
+        return none(unlocked);
     }
+    check_numel(who, "norm_weight", weight, g.heads * g.head_dim);
+    if (weight == nullptr && workspace != nullptr &&
+        static_cast<long long>(workspace->numel() * workspace->element_size()) < lib.ternaspmm_attention_workspace_bytes(g.batch, g.heads, g.head_dim))
+        refuse("%s: the workspace is too small", who);
+    Unlocked unlocked;
     at::Tensor o = make({g.batch, g.heads * g.head_dim}, at::kBFloat16, qkv), stats;
     if (weight != nullptr) {
-        check_numel(who, "norm_weight", weight, g.heads * g.head_dim);
         stats = make({g.batch, g.heads, 2}, at::kFloat, qkv);
-        if (lib.ternaspmm_rope_decode_attention_stats(TERNA_ATTENTION_INPUTS(data<terna_bf16>(&qkv), g), ck, cv, data<terna_bf16>(&o), g.batch, g.heads, g.kv, g.head_dim, g.slots,
-                                                      g.scale, g.adjacent, data<terna_bf16>(weight), data<float>(&stats), st) != g.heads)
-            refuse("%s: ternaspmm_rope_decode_attention_stats refused the launch", who);
+        const int left = lib.ternaspmm_rope_decode_attention_stats(TERNA_ATTENTION_INPUTS(data<terna_bf16>(&qkv), g), ck, cv, data<terna_bf16>(&o), g.batch, g.heads, g.kv,
+                                                                   g.head_dim, g.slots, g.scale, g.adjacent, data<terna_bf16>(weight), data<float>(&stats), st);
+        unlocked.end();
+        if (left != g.heads) refuse("%s: ternaspmm_rope_decode_attention_stats refused the launch", who);
     } else {
-        if (workspace != nullptr && static_cast<long long>(workspace->numel() * workspace->element_size()) <
-                                        lib.ternaspmm_attention_workspace_bytes(g.batch, g.heads, g.head_dim))
-            refuse("%s: the workspace is too small", who);
         lib.ternaspmm_rope_decode_attention(TERNA_ATTENTION_INPUTS(data<terna_bf16>(&qkv), g), ck, cv, data<terna_bf16>(&o), g.batch, g.heads, g.kv, g.head_dim, g.slots, g.scale,
                                             g.adjacent, data(workspace), st);
     }
-    return pack(std::move(o), std::move(stats));
+    return pack(unlocked, std::move(o), std::move(stats));
 }
 
 // A ternary matrix of a block as four arguments: packed, ws, ws_num, out_features.
@@ -573,6 +622,7 @@ TERNA_FUNCTION(block, 35)
                                                 lib.ternaspmm_attention_workspace_bytes(g.batch, heads, head_dim))
         refuse("%s: the attention workspace is too small", who);
 
+    Unlocked unlocked;
     // scratch of this call, in one piece: int8 rows and scales; then qkv, rotated queries, attention output and its projection,
     // in whose place the gate and up outputs go
     auto up = [](int64_t bytes) { return (bytes + 255) & ~int64_t{255}; };
@@ -605,8 +655,10 @@ TERNA_FUNCTION(block, 35)
     if (!rows_in_place) linear(qkv_w, dim, qkv);
     if (rows_in_place) {
         if (!lib.ternaspmm_prefill_attention_rows(qkv, qkv_w.n, ck, cv, data<long long>(&g.pos), g.each, o, g.batch, g.t, heads, g.kv, head_dim, g.slots,
-                                                  g.scale, st))
+                                                  g.scale, st)) {
+            unlocked.end();
             refuse("%s: the attention over the projection's rows refused the launch", who);
+        }
     } else if (g.t > 1) {
         lib.ternaspmm_rope_kv_store(TERNA_ATTENTION_INPUTS(qkv, g), q, ck, cv, g.batch, g.t, heads, g.kv, head_dim, g.slots, g.adjacent, st);
         lib.ternaspmm_prefill_attention(q, ck, cv, data<long long>(&g.pos), g.each, o, g.batch, g.t, heads, g.kv, head_dim, g.slots, g.scale, st);
@@ -632,9 +684,9 @@ TERNA_FUNCTION(block, 35)
         linear(gate_w, dim, x13);
         lib.ternaspmm_relu2_mul_rmsnorm_quant(x13, data<terna_bf16>(norm[3]), eps, nullptr, xq, s, m, ffn, st);
     }
-    if (add_linear(down_w, ffn, data<terna_bf16>(&mid), data<terna_bf16>(&out))) return pack(std::move(out), at::Tensor());
+    if (add_linear(down_w, ffn, data<terna_bf16>(&mid), data<terna_bf16>(&out))) return pack(unlocked, std::move(out), at::Tensor());
     linear(down_w, ffn, data<terna_bf16>(&out));
-    return pack(std::move(mid), std::move(out));
+    return pack(unlocked, std::move(mid), std::move(out));
 }
 
 // (partial, splits, heads, head_dim, norm_weight, eps, sequences, want_output) -> (xq, s, o | None), or None
@@ -648,12 +700,14 @@ TERNA_FUNCTION(attention_merge_rmsnorm_quant, 8)
     const long long held = partial.numel() * partial.element_size(), need = lib.ternaspmm_attention_partial_bytes(sequences, heads, head_dim);
     if (sequences < 1 || need < 0 || held < need) refuse("partial buffer of %lld bytes does not hold %d sequences", held, sequences);
     if (weight.numel() != k || weight.scalar_type() != at::kBFloat16) refuse("%s: the norm weight is a bf16 vector of heads * head_dim elements", who);
+    const bool want_output = PyObject_IsTrue(a[7]);
+    Unlocked unlocked;
     at::Tensor q = make({sequences, k}, at::kChar, partial), s = make({sequences}, at::kBFloat16, partial), o;
-    if (PyObject_IsTrue(a[7])) o = make({sequences, k}, at::kBFloat16, partial);
+    if (want_output) o = make({sequences, k}, at::kBFloat16, partial);
     if (lib.ternaspmm_attention_merge_rmsnorm_quant(data<float>(&partial), splits, data<terna_bf16>(&weight), eps, o.defined() ? data<terna_bf16>(&o) : nullptr,
                                                     data<int8_t>(&q), data<terna_bf16>(&s), sequences, heads, head_dim, stream()) != 0)
-        Py_RETURN_NONE;
-    return pack(std::move(q), std::move(s), std::move(o));
+        return none(unlocked);
+    return pack(unlocked, std::move(q), std::move(s), std::move(o));
 }
 
 // (tokens, pos, embedding, rope_table, norm_weight) -> (x, stats, rope [2, B, half]); tokens / pos contiguous int64 vectors
@@ -669,15 +723,18 @@ TERNA_FUNCTION(step_inputs, 5)
     check_numel(who, "norm_weight", &weight, k);
     const int count = lib.ternaspmm_row_stats_count(k);
     if (count < 1) refuse("%s: unsupported K=%d", who, static_cast<int>(k));
+    Unlocked unlocked;
     const at::Tensor ids = tokens.contiguous(), at_slot = pos.contiguous();         // (copies only where a caller passed a strided view)
     const int64_t slots = table.size(0), half = table.size(2);
     at::Tensor x = make({b, k}, at::kBFloat16, embedding), stats = make({b, count, 2}, at::kFloat, embedding), rope = make({2, b, half}, at::kFloat, embedding);
-    if (lib.ternaspmm_step_inputs(data<long long>(&ids), data<long long>(&at_slot), pos.numel() == b && b > 1, data<terna_bf16>(&embedding), v, k,
-                                  data<float>(&table), slots, half, data<terna_bf16>(&weight), data<terna_bf16>(&x), data<float>(&stats), data<float>(&rope), b,
-                                  stream()) != count)
+    const int left = lib.ternaspmm_step_inputs(data<long long>(&ids), data<long long>(&at_slot), pos.numel() == b && b > 1, data<terna_bf16>(&embedding), v, k,
+                                               data<float>(&table), slots, half, data<terna_bf16>(&weight), data<terna_bf16>(&x), data<float>(&stats),
+                                               data<float>(&rope), b, stream());
+    unlocked.end();
+    if (left != count)
         refuse("%s: the library refused the launch (B=%d V=%d K=%d S=%d half=%d)", who, static_cast<int>(b), static_cast<int>(v), static_cast<int>(k),
                static_cast<int>(slots), static_cast<int>(half));
-    return pack(std::move(x), std::move(stats), std::move(rope));
+    return pack(unlocked, std::move(x), std::move(stats), std::move(rope));
 }
 
 // (tokens, pos, embedding, rope_table) -> (x, rope [2, positions, half]): int64 tokens [B, T] and positions of T or B T elements
@@ -692,14 +749,17 @@ TERNA_FUNCTION(prompt_inputs, 4)
     if (table.dim() != 3 || table.size(1) != 2 || tokens.scalar_type() != at::kLong || pos.scalar_type() != at::kLong || table.scalar_type() != at::kFloat ||
         embedding.scalar_type() != at::kBFloat16 || !embedding.is_contiguous() || !table.is_contiguous())
         refuse("%s: tokens / pos int64, embedding bf16 [V, K] and rope_table fp32 [S, 2, half] contiguous", who);
+    Unlocked unlocked;
     const at::Tensor ids = tokens.contiguous(), at_slot = pos.contiguous();
     const int64_t slots = table.size(0), half = table.size(2);
     at::Tensor x = make({m, k}, at::kBFloat16, embedding), rope = make({2, rows, half}, at::kFloat, embedding);
-    if (lib.ternaspmm_prompt_inputs(data<long long>(&ids), data<long long>(&at_slot), rows, data<terna_bf16>(&embedding), v, k, data<float>(&table), slots, half,
-                                    data<terna_bf16>(&x), data<float>(&rope), m, stream()) != 0)
+    const int rc = lib.ternaspmm_prompt_inputs(data<long long>(&ids), data<long long>(&at_slot), rows, data<terna_bf16>(&embedding), v, k, data<float>(&table), slots,
+                                               half, data<terna_bf16>(&x), data<float>(&rope), m, stream());
+    unlocked.end();
+    if (rc != 0)
         refuse("%s: the library refused the launch (M=%d V=%d K=%d S=%d half=%d)", who, static_cast<int>(m), static_cast<int>(v), static_cast<int>(k),
                static_cast<int>(slots), static_cast<int>(half));
-    return pack(std::move(x), std::move(rope));
+    return pack(unlocked, std::move(x), std::move(rope));
 }
 
 // (path of libternaspmm.so)

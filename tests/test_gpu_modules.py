@@ -252,3 +252,47 @@ def test_infinite_bf16_activations_at_the_end_of_a_row(m, n, k):
     whole = torch.isfinite(want)
     if whole.any():
         assert (got[whole] - want[whole]).abs().max() <= 1e-2 * want[whole].abs().max()
+
+
+def test_other_threads_run_while_a_module_call_waits():
+    """The first sight of a weight waits for the device inside the module's call (the library makes its copy): meanwhile other
+    Python threads go on."""
+    import threading
+    import time
+    import ctypes
+    import ternainfer_amd as T
+    from ternainfer_amd import _lib
+    lib = _lib.load()
+    n, k, wait = 256, 320, 0.5
+    dic, _ = checkpoint_entry(make_ternary(n, k, 0.40, 970), [1.25])
+    module = T.SpBitLinear(k, n, dic, "l")
+    x = torch.ones((3, k), dtype=torch.bfloat16, device="cuda")
+    was = lib.ternaspmm_repack_cache_enable(1)
+    try:
+        module(x)                                 # whatever is loaded or allocated once
+        lib.ternaspmm_repack_cache_clear()
+        torch.cuda.synchronize()
+        print("[case] a module call that waits for the device, and another thread", flush=True)
+        done = []
+
+        def call():
+            stream = torch.cuda.current_stream()
+            lib.gpu_sleep(wait * 1e6, ctypes.c_void_p(stream.cuda_stream))
+            start = time.monotonic()
+            module(x)
+            done.append(time.monotonic() - start)
+
+        thread = threading.Thread(target=call)
+        thread.start()
+        longest, last = 0.0, time.monotonic()
+        while thread.is_alive():
+            time.sleep(0.002)
+            now = time.monotonic()
+            longest, last = max(longest, now - last), now
+        thread.join()
+        assert done and done[0] > wait / 2        # the call did wait ...
+        assert longest < wait / 2                 # ... and this thread did not
+    finally:
+        torch.cuda.synchronize()
+        lib.ternaspmm_repack_cache_clear()
+        lib.ternaspmm_repack_cache_enable(was)
