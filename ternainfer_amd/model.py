@@ -202,6 +202,12 @@ class Block:
             self.w13_interleaved = interleave_gate_up(self.w13.packed, self.w13.n, self.w13.k)
         return self.w13_interleaved
 
+    def gate_linear_reads(self, rows):
+        """Whether a block call of `rows` rows reads the interleaved matrix (a second copy of the widest one): the calls that
+        ternaspmm_gate_linear takes."""
+        n = self.w13.n
+        return rows > 16 and n != 3840 and (self.w13.ws_num == 1 or n % 256 == 0)
+
     def forward_chain(self, x, stats, cache_k, cache_v, pos_idx, cos, sin, attn_ws, next_norm, split=False):
         """One new token per sequence (up to 16 sequences), the linears chained through producer-side norm statistics:
         `x` is the residual stream INCLUDING the previous block's FFN output and `stats` its partials under this block's
@@ -344,7 +350,7 @@ class Block:
                 attn_ws, get_global_workspace(x.device) if x.shape[0] > 64 else None, self.attention_norm, self.attn_sub_norm, self.ffn_norm,
                 self.ffn_sub_norm, wqkv.packed, wqkv.ws, wqkv.ws_num, wqkv.n, wo.packed, wo.ws, wo.ws_num, wo.n, w13.packed, w13.ws, w13.ws_num, w13.n,
                 w2.packed, w2.ws, w2.ws_num, w2.n,
-                self.gate_up_interleaved())
+                self.gate_up_interleaved() if self.gate_linear_reads(x.shape[0]) else None)
         qkv, x = self._norm_linear(self.wqkv, x, self.attention_norm, residual=pending, name="wqkv")
         rep = a.n_heads // a.n_kv_heads
         native = _lib.native()

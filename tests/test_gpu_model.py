@@ -353,3 +353,26 @@ def test_token_ids_are_indices(batch, tokens):
         wrong[0, 0] = outside
         got = logits(wrong)
         assert torch.isnan(got[0]).all() and torch.equal(got[1:], want[1:])
+
+
+@pytest.mark.parametrize("ffn_dim,tokens,reads", [(384, 9, False), (384, 16, False), (384, 17, True), (320, 17, False), (1920, 17, False)])
+def test_interleaved_copy_is_made_where_it_is_read(ffn_dim, tokens, reads):
+    """The interleaved gate+up matrix is a second copy of the widest weight: a prompt pass makes it exactly where
+    ternaspmm_gate_linear takes the call."""
+    import ctypes
+    from ternainfer_amd.model import ModelArgs, Transformer
+    args = ModelArgs(dim=256, n_layers=1, n_heads=4, n_kv_heads=2, vocab_size=512, ffn_dim=ffn_dim)
+    model = Transformer(args, seed=33)
+    layer = model.layers[0]
+    print(f"[case] interleaved copy ffn={ffn_dim} tokens={tokens}", flush=True)
+    with torch.inference_mode():
+        model.forward(torch.zeros((1, tokens), dtype=torch.int64, device="cuda"), model.make_cache(1, tokens), torch.arange(tokens, device="cuda"))
+    assert (layer.w13_interleaved is not None) == reads == layer.gate_linear_reads(tokens)
+    w, lib = layer.w13, layer.w13.lib
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    xq, s = torch.zeros((tokens, w.k), dtype=torch.int8, device="cuda"), torch.ones(tokens, dtype=torch.bfloat16, device="cuda")
+    out = torch.empty((tokens, w.n // 2), dtype=torch.bfloat16, device="cuda")
+    taken = lib.ternaspmm_gate_linear(p(xq), p(layer.gate_up_interleaved()), p(out), p(s), p(w.ws), w.ws_num, tokens, w.n, w.k,
+                                      ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert bool(taken) == reads
