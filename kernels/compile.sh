@@ -25,7 +25,7 @@ compile() {  # compile <source> <object> [extra flags]
 compile ternaspmm.hip ternaspmm.o
 compile launch_reference.hip launch_reference.o
 compile launch_decode_packed.hip launch_decode_packed.o
-compile launch_prefill_packed.hip launch_prefill_packed_i8.o -DTERNA_PREFILL_ACT=int8_t
+compile launch_prefill_packed.hip launch_prefill_packed_i8.o -DTERNA_PREFILL_ACT=int8_t -DTERNA_PREFILL_PRODUCERS
 compile launch_prefill_packed.hip launch_prefill_packed_bf16.o -DTERNA_PREFILL_ACT=uint16_t
 compile launch_mid.hip launch_mid.o
 compile abi_fused.hip abi_fused.o

@@ -1,5 +1,6 @@
 // Launchers of the MFMA-tiled kernels on the P2 layout (prefill_packed_kernel.h).  Compiled once per activation
-// type (-DTERNA_PREFILL_ACT=int8_t | uint16_t): the two sets of instantiations build in parallel.
+// type (-DTERNA_PREFILL_ACT=int8_t | uint16_t): the two sets of instantiations build in parallel.  The producing epilogues
+// belong to the int8 family (-DTERNA_PREFILL_PRODUCERS).
 #include "launchers.h"
 #include "host_util.h"
 #include "prefill_deep_kernel.h"
@@ -188,41 +189,31 @@ bool launch_prefill_packed(const Act* x, const uint32_t* packed, uint16_t* out, 
     return false;
 }
 
-template <int EPI, typename Act>
-bool launch_prefill_producer(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, const PackedExtra<EPI>* extra,
-                             hipStream_t st, void* scratch = nullptr, size_t scratch_bytes = 0)
+#ifdef TERNA_PREFILL_PRODUCERS
+template <int EPI>
+static bool launch_prefill_producer(const int8_t* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K,
+                                    const PackedExtra<EPI>* extra, hipStream_t st, void* scratch = nullptr, size_t scratch_bytes = 0)
 {
-    if constexpr (sizeof(Act) == 1) {
-        const PrefillPlan plan = plan_prefill_packed<Act>(x, M, N, K, scratch, scratch_bytes);
-        if (!plan.direct_lds || plan.bm != 64) return false;
-        if (plan.bn == 128) launch_prefill_packed_dma_as<Act, 2, 1, EPI>(x, packed, out, ep, M, N, K, plan, scratch, st, extra);
-        else launch_prefill_packed_dma_as<Act, 2, 2, EPI>(x, packed, out, ep, M, N, K, plan, scratch, st, extra);
-        return true;
-    }
-    return false;
+    const PrefillPlan plan = plan_prefill_packed<int8_t>(x, M, N, K, scratch, scratch_bytes);
+    if (!plan.direct_lds || plan.bm != 64) return false;
+    if (plan.bn == 128) launch_prefill_packed_dma_as<int8_t, 2, 1, EPI>(x, packed, out, ep, M, N, K, plan, scratch, st, extra);
+    else launch_prefill_packed_dma_as<int8_t, 2, 2, EPI>(x, packed, out, ep, M, N, K, plan, scratch, st, extra);
+    return true;
 }
-template <typename Act>
-bool launch_prefill_gate(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, hipStream_t st)
+bool launch_prefill_gate(const int8_t* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, hipStream_t st)
 {
     return launch_prefill_producer<PACKED_GATE>(x, packed, out, ep, M, N, K, nullptr, st);
 }
-template <typename Act>
-bool launch_prefill_rope(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, const RopeStore& rope, hipStream_t st)
+bool launch_prefill_rope(const int8_t* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, const RopeStore& rope, hipStream_t st)
 {
     return launch_prefill_producer<PACKED_ROPE>(x, packed, out, ep, M, N, K, &rope, st);
 }
-template <typename Act>
-bool launch_prefill_residual(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, const ResidualRows& stream,
+bool launch_prefill_residual(const int8_t* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, const ResidualRows& stream,
                              void* scratch, size_t scratch_bytes, hipStream_t st)
 {
     return launch_prefill_producer<PACKED_RESIDUAL>(x, packed, out, ep, M, N, K, &stream, st, scratch, scratch_bytes);
 }
-
-template bool launch_prefill_residual<TERNA_PREFILL_ACT>(const TERNA_PREFILL_ACT*, const uint32_t*, uint16_t*, const Epilogue&, int, int, int,
-                                                         const ResidualRows&, void*, size_t, hipStream_t);
-template bool launch_prefill_gate<TERNA_PREFILL_ACT>(const TERNA_PREFILL_ACT*, const uint32_t*, uint16_t*, const Epilogue&, int, int, int, hipStream_t);
-template bool launch_prefill_rope<TERNA_PREFILL_ACT>(const TERNA_PREFILL_ACT*, const uint32_t*, uint16_t*, const Epilogue&, int, int, int, const RopeStore&,
-                                                     hipStream_t);
+#endif
 
 template bool launch_prefill_packed<TERNA_PREFILL_ACT>(const TERNA_PREFILL_ACT*, const uint32_t*, uint16_t*, const Epilogue&, int, int, int,
                                                        void*, size_t, hipStream_t, const RepackGuard*);

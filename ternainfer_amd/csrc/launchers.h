@@ -48,17 +48,14 @@ void launch_mid(const Act* x, const uint32_t* packed, uint16_t* out, const Epilo
                 const RepackGuard* guard = nullptr);
 // The gate+up matrix with its gate (bands of w1 and w3 interleaved, int8 activations, out [M][N / 2]): the kernels of more than 16 rows.
 void launch_mid_gate(const int8_t* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, hipStream_t st);
-template <typename Act>
-bool launch_prefill_gate(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, hipStream_t st);
+bool launch_prefill_gate(const int8_t* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, hipStream_t st);
 // The QKV projection of a prompt pass with RoPE and the cache write: the same kernels.
 void launch_mid_rope(const int8_t* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, const RopeStore& rope, hipStream_t st);
-template <typename Act>
-bool launch_prefill_rope(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, const RopeStore& rope, hipStream_t st);
+bool launch_prefill_rope(const int8_t* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, const RopeStore& rope, hipStream_t st);
 // Output + residual stream (O and down projection), more than 16 rows.
 void launch_mid_residual(const int8_t* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, const ResidualRows& stream,
                          hipStream_t st);
-template <typename Act>
-bool launch_prefill_residual(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, const ResidualRows& stream,
+bool launch_prefill_residual(const int8_t* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, const ResidualRows& stream,
                              void* scratch, size_t scratch_bytes, hipStream_t st);
 // Fingerprint of the reference-format tensors named by `guard` into *out / the check of it as a launch of its own.
 void launch_repack_fingerprint(const RepackGuard& guard, unsigned long long* out, hipStream_t st);

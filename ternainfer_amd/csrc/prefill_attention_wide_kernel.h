@@ -27,11 +27,6 @@ constexpr int kWideRing = 4;                                           // tiles 
 constexpr int kWideTile = kPrefillAttnKeys * 256;                      // bytes of one
 constexpr int kWideLds = 2 * kWideRing * kWideTile;
 
-__device__ __forceinline__ void wide_dma_b128(const void* sbase, uint32_t voff, uint32_t lds_addr)
-{
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_addr), "v"(voff), "s"(sbase) : "memory");
-}
-
 // key_groups_reduce as statements that may be scheduled among others (all lanes are active wherever it stands)
 template <bool IS_MAX>
 __device__ __forceinline__ float wide_groups_reduce(float v)
@@ -109,7 +104,7 @@ __global__ __launch_bounds__(256, 2) void terna_prefill_attention_wide_kernel(
     auto load_rows = [&](const uint8_t* base, uint32_t piece, int step, int i, uint32_t lds) __attribute__((always_inline)) {
         const int k0 = step * KB < n_keys ? step * KB : n_keys - 1;    // uniform
         const int row = min(ROWS * wave + 4 * i + r4, n_keys - 1 - k0);
-        wide_dma_b128(base + static_cast<size_t>(k0) * 256, row * 256 + piece, lds + i * 1024);
+        lds_dma_b128(base + static_cast<size_t>(k0) * 256, row * 256 + piece, lds + i * 1024);
     };
     auto load_keys_at = [&](int step, int slot4, int i) __attribute__((always_inline)) { load_rows(kbase, k_piece[i], step, i, lds0 + slot4 * kWideTile); };
     auto load_values_at = [&](int step, int slot4, int i) __attribute__((always_inline)) {

@@ -57,22 +57,10 @@ struct OutTile {
     __device__ static constexpr int swizzle(int row) { return (row >> (NA == 2 ? 1 : 2)) & (kPieces - 1); }
 };
 
-// Fused epilogue of one wave's NA x MB accumulator tiles (v_mfma_f32_32x32x16 layout: lane holds
-// column m = L % 32 and rows n = (v&3) + 8(v>>2) + 4(L/32) of each tile).  A float accumulator is
-// twice the true sum (weights were +-2; x0.5 is exact); an integer one is the sum times 64 (weights were +-64; >> 6 is exact).
-// `tile`: this wave's OutTile<NA>::kBytes of LDS (results leave as whole rows; needs out and N * 2 to be multiples of
-// 16 bytes), or nullptr (every lane stores its 8-byte pieces itself).
-// One weight-group scale per 32-feature tile: always under the per-128-column rule of the prefill epilogue and with one
-// group, otherwise when the group boundaries fall on multiples of 32.  (Host and device: the launcher picks a kernel by it.)
-__host__ __device__ inline bool epilogue_scales_per_tile(const Epilogue& ep, int N)
-{
-    return ep.kind == EP_I8_PREFILL || ep.ws_num == 1 || (N == 3840 && ep.ws_num == 3) || (N / ep.ws_num) % 32 == 0;
-}
-
 // The gate of a feed-forward layer on the matrix whose w1 and w3 bands are interleaved (ternaspmm_interleave_gate_up): rows 0 .. 15 of a
 // 32-feature tile are x1, rows 16 .. 31 the x3 of the same features, and a lane holds both (its values v and v + 8).  Every product is
 // rounded to bf16 where the separate launches store it.  out [M][N / 2]: half the bytes here, a quarter in the norm that
-// follows (it read both halves).  int8 family, one scale per half: see gate_linear_takes.
+// follows (it read both halves).  int8 family, one scale per half: see ternaspmm_gate_linear.
 template <int MB, int NA, typename AccV>
 __device__ __forceinline__ void packed_prefill_gate_epilogue(AccV (&acc)[NA][MB], uint16_t* __restrict__ out, const Epilogue& ep, int M, int N,
                                                              int n_wave, int m0, int lane, uint8_t* tile)
@@ -186,6 +174,11 @@ enum PackedEpilogue { PACKED_STORE, PACKED_GATE, PACKED_ROPE, PACKED_RESIDUAL };
 template <int EPI>
 using PackedExtra = typename std::conditional<EPI == PACKED_ROPE, RopeStore, typename std::conditional<EPI == PACKED_RESIDUAL, ResidualRows, RepackGuard>::type>::type;
 
+// Fused epilogue of one wave's NA x MB accumulator tiles (v_mfma_f32_32x32x16 layout: lane holds
+// column m = L % 32 and rows n = (v&3) + 8(v>>2) + 4(L/32) of each tile).  A float accumulator is
+// twice the true sum (weights were +-2; x0.5 is exact); an integer one is the sum times 64 (weights were +-64; >> 6 is exact).
+// `tile`: this wave's OutTile<NA>::kBytes of LDS (results leave as whole rows; needs out and N * 2 to be multiples of
+// 16 bytes), or nullptr (every lane stores its 8-byte pieces itself).
 // COLS = false leaves out the per-column path (scales that change inside a 32-feature tile): unrolled next to 64 - 128 live
 // accumulators it spilled up to 88 registers, so every launch of the larger tiles carried scratch memory for a path that
 // almost no call takes.  The launcher sends such calls to the 128 x 64 instantiation, which keeps the path.
@@ -547,11 +540,6 @@ __global__ __launch_bounds__(256, MB == 8 ? 1 : (MB == 3 ? 3 : 2)) void terna_pr
 constexpr int kXSwizzleShift = 1;
 __device__ __forceinline__ constexpr int x_swizzle(int row) { return (row >> kXSwizzleShift) & 7; }
 
-// LDS[lds_addr + 16*lane .. +15] <- global[sbase + voff .. +15]; completion is counted by vmcnt.
-__device__ __forceinline__ void lds_dma_b128(const void* sbase, uint32_t voff, uint32_t lds_addr)
-{
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_addr), "v"(voff), "s"(sbase) : "memory");
-}
 // d <- global[sbase + voff .. +15] without a compiler-generated wait: d may be read only after a
 // later wait_loads<>() and a landed(d).
 __device__ __forceinline__ void global_load_b128_nowait(u32x4& d, const void* sbase, uint32_t voff)

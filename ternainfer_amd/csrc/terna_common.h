@@ -63,6 +63,13 @@ struct Epilogue {
     int             kind;
 };
 
+// One weight-group scale per 32-feature tile: always under the per-128-column rule of the prefill epilogue and with one
+// group, otherwise when the group boundaries fall on multiples of 32.  (Host and device: the launcher picks a kernel by it.)
+__host__ __device__ inline bool epilogue_scales_per_tile(const Epilogue& ep, int N)
+{
+    return ep.kind == EP_I8_PREFILL || ep.ws_num == 1 || (N == 3840 && ep.ws_num == 3) || (N / ep.ws_num) % 32 == 0;
+}
+
 __device__ __forceinline__ float bf16_bits_to_float(uint16_t h)
 {
     return __uint_as_float(static_cast<uint32_t>(h) << 16);
@@ -161,6 +168,12 @@ constexpr int kBufferOutOfRange = static_cast<int>(0x80000000u);   // a lane off
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_raw_buffer(const void* base, uint32_t bytes)
 {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, static_cast<int>(bytes), kBufferRsrcFlags);
+}
+
+// LDS[lds_addr + 16*lane .. +15] <- global[sbase + voff .. +15]; completion is counted by vmcnt.
+__device__ __forceinline__ void lds_dma_b128(const void* sbase, uint32_t voff, uint32_t lds_addr)
+{
+    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_addr), "v"(voff), "s"(sbase) : "memory");
 }
 
 // Makes the value live in registers at this point of the program: a load that produced it cannot be sunk

@@ -529,16 +529,10 @@ int ternaspmm_gate_linear(const int8_t* x, const void* packed, terna_bf16* out, 
     const uint32_t* p = static_cast<const uint32_t*>(packed);
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (mid_kernel_takes(x, M, N, K, sizeof(int8_t))) launch_mid_gate(x, p, out, ep, M, N, K, st);
-    else if (!launch_prefill_gate<int8_t>(x, p, out, ep, M, N, K, st)) return 0;
+    else if (!launch_prefill_gate(x, p, out, ep, M, N, K, st)) return 0;
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) die("ternaspmm_gate_linear", e, __LINE__);
     return 1;
-}
-
-// one weight scale per 32 features
-static bool scale_per_32(const Epilogue& ep, int N)
-{
-    return ep.kind == EP_I8_PREFILL || ep.ws_num == 1 || (N == 3840 && ep.ws_num == 3) || (N / ep.ws_num) % 32 == 0;
 }
 
 int ternaspmm_residual_linear(const int8_t* x, const void* packed, terna_bf16* out, const terna_bf16* s, const terna_bf16* ws, int ws_num,
@@ -549,12 +543,12 @@ int ternaspmm_residual_linear(const int8_t* x, const void* packed, terna_bf16* o
         return 0;
     if (!shape_ok(M, N, K) || !groups_ok(ws_num) || !i8_depth_ok(K)) return 0;
     const Epilogue ep{s, ws, nullptr, ws_num, M <= 64 ? EP_I8_DECODE : EP_I8_PREFILL};
-    if (!scale_per_32(ep, N)) return 0;
+    if (!epilogue_scales_per_tile(ep, N)) return 0;
     const uint32_t* p = static_cast<const uint32_t*>(packed);
     const ResidualRows rows{residual};
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (mid_kernel_takes(x, M, N, K, sizeof(int8_t))) launch_mid_residual(x, p, out, ep, M, N, K, rows, st);
-    else if (!launch_prefill_residual<int8_t>(x, p, out, ep, M, N, K, rows, workspace, workspace_bytes > 0 ? static_cast<size_t>(workspace_bytes) : 0, st)) return 0;
+    else if (!launch_prefill_residual(x, p, out, ep, M, N, K, rows, workspace, workspace_bytes > 0 ? static_cast<size_t>(workspace_bytes) : 0, st)) return 0;
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) die("ternaspmm_residual_linear", e, __LINE__);
     return 1;
@@ -570,12 +564,12 @@ int ternaspmm_qkv_rope_linear(const int8_t* x, const void* packed, terna_bf16* o
         return 0;
     if (!shape_ok(M, N, K) || !groups_ok(ws_num) || !i8_depth_ok(K)) return 0;
     const Epilogue ep{s, ws, nullptr, ws_num, M <= 64 ? EP_I8_DECODE : EP_I8_PREFILL};
-    if (!scale_per_32(ep, N)) return 0;
+    if (!epilogue_scales_per_tile(ep, N)) return 0;
     const RopeStore rope{cos, sin, pos, cache_k, cache_v, per_sequence != 0, T, H, KV, D, S};
     const uint32_t* p = static_cast<const uint32_t*>(packed);
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (mid_kernel_takes(x, M, N, K, sizeof(int8_t))) launch_mid_rope(x, p, out, ep, M, N, K, rope, st);
-    else if (!launch_prefill_rope<int8_t>(x, p, out, ep, M, N, K, rope, st)) return 0;
+    else if (!launch_prefill_rope(x, p, out, ep, M, N, K, rope, st)) return 0;
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) die("ternaspmm_qkv_rope_linear", e, __LINE__);
     return 1;

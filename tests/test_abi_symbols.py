@@ -136,3 +136,17 @@ def test_python_wrappers_refuse_mismatched_tensors_on_the_host():
     with pytest.raises(ValueError, match="does not hold"):
         L.attention_merge_rmsnorm_linear_packed(torch.zeros(1000, dtype=torch.float32), 4, 20, 128, w, 1e-5, packed, ws, 1, 2560,
                                                 sequences=8)
+
+
+def test_fused_linear_descriptor_is_laid_out_as_the_header_declares_it(tmp_path):
+    """`FusedLinearDesc`, what a ctypes caller of ternaspmm_fused_linear fills in, against the struct as a C compiler lays it out."""
+    import shutil
+    import subprocess
+    from ternainfer_amd.linear import FusedLinearDesc
+    names = [name for name, _ in FusedLinearDesc._fields_]
+    source = tmp_path / "layout.c"
+    source.write_text('#include <stddef.h>\n#include <stdio.h>\n#include "ternaspmm.h"\nint main(void)\n{\n    printf("%zu", sizeof(ternaspmm_fused_linear_desc));\n' +
+                      "".join(f'    printf(" %zu", offsetof(ternaspmm_fused_linear_desc, {name}));\n' for name in names) + "    return 0;\n}\n")
+    subprocess.run([shutil.which("gcc") or "cc", "-I", os.path.dirname(HEADER), str(source), "-o", str(tmp_path / "layout")], check=True, timeout=60)
+    said = subprocess.run([str(tmp_path / "layout")], capture_output=True, text=True, check=True, timeout=60).stdout
+    assert [int(v) for v in said.split()] == [ctypes.sizeof(FusedLinearDesc)] + [getattr(FusedLinearDesc, name).offset for name in names]
