@@ -138,6 +138,19 @@ def test_python_wrappers_refuse_mismatched_tensors_on_the_host():
                                                 sequences=8)
 
 
+def test_prompt_inputs_refuses_what_its_kernel_does_not_take():
+    """Shapes, missing and misaligned pointers are refused on the host, nothing is enqueued (so this runs without a GPU)."""
+    from ternainfer_amd import _lib
+    lib = _lib.load()
+    p = lambda address: ctypes.c_void_p(address)
+    good = dict(tokens=p(64), pos=p(64), rows=4, emb=p(64), v=10, k=64, table=p(64), s=8, half=32, x=p(64), rope=p(64), m=4)
+    order = ("tokens", "pos", "rows", "emb", "v", "k", "table", "s", "half", "x", "rope", "m")
+    for wrong in (dict(m=0), dict(rows=0), dict(rows=5), dict(v=0), dict(s=0), dict(k=60), dict(k=0), dict(half=6), dict(half=0), dict(half=516), dict(emb=p(72)),
+                  dict(table=p(68)), dict(x=p(66)), dict(rope=p(65)), *({name: None} for name in ("tokens", "pos", "emb", "table", "x", "rope"))):
+        arguments = {**good, **wrong}
+        assert lib.ternaspmm_prompt_inputs(*(arguments[name] for name in order), None) == -1, wrong
+
+
 def test_fused_linear_descriptor_is_laid_out_as_the_header_declares_it(tmp_path):
     """`FusedLinearDesc`, what a ctypes caller of ternaspmm_fused_linear fills in, against the struct as a C compiler lays it out."""
     import shutil
