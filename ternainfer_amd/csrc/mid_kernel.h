@@ -95,13 +95,14 @@ __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
     RawW rw;
     auto issue = [&](int at_chunk) __attribute__((always_inline)) {
         const int chunk = __builtin_amdgcn_readfirstlane(at_chunk);
-        // columns past K (a partial last chunk): loads pulled back into the row, one of the operands zeroed when they are used
+        // columns past K (a partial last chunk): loads pulled back into the row, zeros in place of their activations before these are used
         const int tile0 = chunk * 4;
         const int left = ktiles - 1 - tile0;
         const uint32_t woff = static_cast<uint32_t>(tile0 * 256 + (g < left ? g : left) * 256 + i * 16);
 #pragma unroll
         for (int b = 0; b < FB; ++b) global_load_b128_nowait(rw.w[b], wbase + static_cast<size_t>(b) * ktiles * 256, woff);
-        const int col = chunk * S::kRowBytes, last = rowbytes - 16 - col;
+        const int col = chunk * S::kRowBytes;
+        const int last = left < 3 ? rowbytes - 16 - col : S::kRowBytes;
 #pragma unroll
         for (int j = 0; j < XI; ++j) {
             const int at = (piece0 ^ ((ROWS_PER_LOAD * j) & 15)) * 16;
@@ -115,29 +116,38 @@ __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
 #pragma unroll
         for (int b = 0; b < FB; ++b) acc[r][b] = Acc{0, 0, 0, 0};
 
-    auto multiply = [&](int chunk) __attribute__((always_inline)) {
+    // Tiles that do not exist: what was loaded in their place are other activations of the row, which may be infinite, and zero weights
+    // would make NaN of them.  Each lane clears what it is going to read.
+    auto clear_past_end = [&](int chunk) __attribute__((always_inline)) {
+        if (chunk * 4 + 4 <= ktiles) return;             // uniform
+        if (chunk * 4 + g < ktiles) return;
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+            for (int p = 0; p < 4 * SZ; ++p)
+                *reinterpret_cast<u32x4*>(mine + (16 * r + i) * S::kRowBytes + (((4 * SZ * g + p) ^ i) * 16)) = u32x4{0u, 0u, 0u, 0u};
+    };
+    // the activations that MFMA number c of a chunk (bf16: numbers 2 c and 2 c + 1) takes, read one c ahead of their use
+    constexpr int HALVES = BF16 ? 2 : 1;
+    struct Ops { u32x4 v[RT][HALVES]; };
+    auto read = [&](int c, Ops& o) __attribute__((always_inline)) {
+        const uint8_t* src = mine + i * S::kRowBytes;
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+            for (int h = 0; h < HALVES; ++h)
+                o.v[r][h] = *reinterpret_cast<const u32x4*>(src + 16 * r * S::kRowBytes + (((4 * HALVES * g + HALVES * c + h) ^ i) * 16));
+    };
+    auto multiply = [&] __attribute__((always_inline)) {
+        Ops ops[2];
+        read(0, ops[0]);
 #pragma unroll
         for (int b = 0; b < FB; ++b) landed(rw.w[b]);
-        uint8_t* src = mine + i * S::kRowBytes;
-        if (chunk * 4 + 4 > ktiles) {                    // uniform
-            const bool exists = chunk * 4 + g < ktiles;  // this lane's tile
-            if constexpr (BF16) {
-                // the activations in the place of a tile that does not exist are others of the row, which may be infinite: they are
-                // overwritten (each lane what it will read), zero weights would make NaN of them
-                if (!exists) {
-#pragma unroll
-                    for (int r = 0; r < RT; ++r)
-#pragma unroll
-                        for (int p = 0; p < 8; ++p) *reinterpret_cast<u32x4*>(src + 16 * r * S::kRowBytes + (((8 * g + p) ^ i) * 16)) = u32x4{0u, 0u, 0u, 0u};
-                }
-            } else {
-                const uint32_t keep = exists ? ~0u : 0u;
-#pragma unroll
-                for (int b = 0; b < FB; ++b) rw.w[b] = u32x4{rw.w[b].x & keep, rw.w[b].y & keep, rw.w[b].z & keep, rw.w[b].w & keep};
-            }
-        }
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
+            __builtin_amdgcn_sched_barrier(0);                           // keeps the reads ahead
+            if (c < 3) read(c + 1, ops[(c + 1) & 1]);
+            const Ops& now = ops[c & 1];
             if constexpr (BF16) {
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
@@ -145,22 +155,20 @@ __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
 #pragma unroll
                     for (int b = 0; b < FB; ++b) a[b] = __builtin_bit_cast(bf16x8, expand_chunk_bf16(h ? rw.w[b][c] : rw.w[b][c] << 4));
 #pragma unroll
-                    for (int r = 0; r < RT; ++r) {
-                        const bf16x8 v = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(src + 16 * r * S::kRowBytes + (((8 * g + 2 * c + h) ^ i) * 16)));
+                    for (int r = 0; r < RT; ++r)
 #pragma unroll
-                        for (int b = 0; b < FB; ++b) acc[r][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[b], v, acc[r][b], 0, 0, 0);
-                    }
+                        for (int b = 0; b < FB; ++b)
+                            acc[r][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[b], __builtin_bit_cast(bf16x8, now.v[r][h]), acc[r][b], 0, 0, 0);
                 }
             } else {
                 i32x4 a[FB];
 #pragma unroll
                 for (int b = 0; b < FB; ++b) a[b] = expand_word_i8(rw.w[b][c]);
 #pragma unroll
-                for (int r = 0; r < RT; ++r) {
-                    const i32x4 v = *reinterpret_cast<const i32x4*>(src + 16 * r * S::kRowBytes + (((4 * g + c) ^ i) * 16));
+                for (int r = 0; r < RT; ++r)
 #pragma unroll
-                    for (int b = 0; b < FB; ++b) acc[r][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[b], v, acc[r][b], 0, 0, 0);
-                }
+                    for (int b = 0; b < FB; ++b)
+                        acc[r][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[b], __builtin_bit_cast(i32x4, now.v[r][0]), acc[r][b], 0, 0, 0);
             }
         }
     };
@@ -193,7 +201,8 @@ __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
     for (int chunk = wave;;) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
-        multiply(chunk);
+        clear_past_end(chunk);
+        multiply();
         __builtin_amdgcn_sched_barrier(0);
         chunk += waves;
         if (chunk >= chunks) break;

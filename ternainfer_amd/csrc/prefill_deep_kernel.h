@@ -73,9 +73,11 @@ __global__ __launch_bounds__(256 * KS) void terna_prefill_deep_kernel(
     const int n0 = n_tile * BN, m0 = m_tile * BM;
     const int ktiles = K >> 6, steps = (ktiles + 1) >> 1;
     const bool half_tail = ktiles & 1;                                    // the last stage has one 64-column tile only
-    const int turns = (steps + KS - 1) / KS;                              // steps of a part (the last one's last may not exist)
-    const int k_begin = part * turns;
-    const int k_end = k_begin + turns < steps ? k_begin + turns : steps;
+    // steps of a part; of an odd number the first part's last does not exist, so that the last step of all is a part's last
+    const int turns = (steps + KS - 1) / KS;
+    const int k_begin = part == 0 ? 0 : steps - turns;
+    const int k_end = part == KS - 1 ? steps : steps - turns;
+    const int k_last = k_end > 0 ? k_end - 1 : 0;                         // (of one step in all the first part has none: it loads that step's stage)
     const int last_band = (N >> 4) - 1;
     const int kb = lane >> 5, l32 = lane & 31;
 
@@ -102,7 +104,7 @@ __global__ __launch_bounds__(256 * KS) void terna_prefill_deep_kernel(
     uint8_t* const stages = smem + part * S::kBytes;
     const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(stages));
     auto issue = [&](int kk, int st) __attribute__((always_inline)) {
-        const int k = kk < k_end - 1 ? kk : k_end - 1;
+        const int k = kk < k_last ? kk : k_last;
         const bool back = half_tail && k == steps - 1;
         const uint8_t* xs = x_base + static_cast<size_t>(k) * S::kRow;
         const uint8_t* ws = w_base + static_cast<size_t>(k) * 512;
@@ -136,11 +138,7 @@ __global__ __launch_bounds__(256 * KS) void terna_prefill_deep_kernel(
         }
     };
     const int wshift = 4 - 4 * kb;
-    // Of a last stage with one tile: int8 multiplies both by weights that are 0 where the lane's tile does not exist; bf16 leaves the
-    // groups of the other one out (its activations are the first tile's, which may be infinite: 0 times that is NaN).
-    uint32_t wmask = kTopFieldMask;
-    bool upper = true;
-    auto mma = [&](const Ops& v, auto qc) __attribute__((always_inline)) {
+    auto mma = [&](const Ops& v, auto qc, uint32_t wmask = kTopFieldMask) __attribute__((always_inline)) {
         constexpr int q = decltype(qc)::value;
 #pragma unroll
         for (int a = 0; a < NA; ++a) {
@@ -163,34 +161,28 @@ __global__ __launch_bounds__(256 * KS) void terna_prefill_deep_kernel(
     int st_next = S::kStage, st_dma = (D - 1) * S::kStage;
     Ops even, odd;
     static_for<0, GROUPS>([&](auto qc) { load(0, qc, even); });
-    auto set_mask = [&](int k) __attribute__((always_inline)) {
-        if constexpr (I8) wmask = (half_tail && k == steps - 1 && kb) ? 0u : kTopFieldMask;
-        else upper = !(half_tail && k == steps - 1);
-    };
-    constexpr int LOWER = I8 ? GROUPS : GROUPS / 2;                       // groups of the first tile (int8: of both)
     auto step = [&](int k, const Ops& cur, Ops& nxt) __attribute__((always_inline)) {
-        set_mask(k);
         // own part of stage k + 1 landed; everybody's, and everybody is past the operand reads of stage k - 1
         asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((D - 3) * PER) : "memory");
         issue(k + D - 1, st_dma);                                         // into the stage of step k - 1
-        auto group = [&](auto qc) __attribute__((always_inline)) {
+        static_for<0, GROUPS>([&](auto qc) {
             __builtin_amdgcn_sched_barrier(0);                            // keeps the reads between the groups
             load(st_next, qc, nxt);
             mma(cur, qc);
-        };
-        static_for<0, LOWER>(group);
-        if (I8 || upper) static_for<LOWER, GROUPS>(group);                // uniform
-        else static_for<LOWER, GROUPS>([&](auto qc) { load(st_next, qc, nxt); });
+        });
         __builtin_amdgcn_sched_barrier(0);
         st_next = next(st_next);
         st_dma = next(st_dma);
     };
-    // the last turn multiplies what is in registers
+    // The last turn multiplies what is in registers.  A last stage with one tile: int8 multiplies both by weights that are 0 where the
+    // lane's tile does not exist; bf16 leaves the groups of the other one out (its activations are the first tile's, which may be
+    // infinite: 0 times that is NaN).
     auto last_step = [&](int k, const Ops& cur) __attribute__((always_inline)) {
         if (k >= k_end) return;                                           // uniform over the part
-        set_mask(k);
-        static_for<0, LOWER>([&](auto qc) { mma(cur, qc); });
-        if (I8 || upper) static_for<LOWER, GROUPS>([&](auto qc) { mma(cur, qc); });
+        const bool half = half_tail && k == steps - 1;
+        constexpr int LOWER = I8 ? GROUPS : GROUPS / 2;                   // groups of the first tile (int8: of both)
+        static_for<0, LOWER>([&](auto qc) { mma(cur, qc, half && kb ? 0u : kTopFieldMask); });
+        if (!half) static_for<LOWER, GROUPS>([&](auto qc) { mma(cur, qc); });
     };
     int t = 0;
     for (; t + 2 < turns; t += 2) {
