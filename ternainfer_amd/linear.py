@@ -345,6 +345,7 @@ def quant_input(input: torch.Tensor, mode: Optional[int] = None):
                       quotient multiplies, the returned s is its bf16 rounding;
       QUANT_EAGER     the same lines without torch.compile on a bf16 tensor: every op rounds to bf16.
     The three differ from each other on a few percent of the elements, by one step (two at most).
+    A NaN in a row makes its s NaN, an infinity makes it 0; the integers of such rows are 0 in every mode.
     Returns (x_q int8, s bf16 [..., 1])."""
     if mode is None:
         mode = _lib.load().ternaspmm_quant_mode(-1)
