@@ -162,16 +162,10 @@ __global__ __launch_bounds__(256) void terna_quant_stats_kernel(const uint16_t* 
     const float s = quant_scale(fabsf(round_bf16(__fmul_rn(pmax, rstd))), quant_mode, &sb);
     if (blockIdx.y == 0 && threadIdx.x == 0) s_out[row] = sb;
     if (!in) return;
-    float f[8], w[8];
-    unpack_bf16x8(hv, f);
-    unpack_bf16x8(wv, w);
-    uint32_t d[2] = {0u, 0u};
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const float y = round_bf16(__fmul_rn(__fmul_rn(f[e], w[e]), rstd));
-        d[e >> 2] = __builtin_amdgcn_cvt_pk_u8_f32(quant_value(y, s, quant_mode) + 128.0f, e & 3, d[e >> 2]);
-    }
-    *reinterpret_cast<u32x2*>(xq_out + row * K + c) = u32x2{d[0] ^ 0x80808080u, d[1] ^ 0x80808080u};
+    const uint32_t hd[4] = {hv.x, hv.y, hv.z, hv.w}, wd[4] = {wv.x, wv.y, wv.z, wv.w};
+    uint32_t d[2];
+    chain_quantise<8>(hd, wd, rstd, s, quant_mode, d);
+    *reinterpret_cast<u32x2*>(xq_out + row * K + c) = u32x2{d[0], d[1]};
 }
 
 // One launch of terna_decode_fused_kernel<WAVES, TMAX, MODE, MP, NB, ASP, AHD, EPI> with MP picked by M (1, 2, 4, 8).

@@ -80,22 +80,26 @@ __device__ __forceinline__ void chain_quantise(const uint32_t (&hraw)[NE / 2], c
     float f[NE];
 #pragma unroll
     for (int j = 0; j < NE / 2; ++j) {
-        f[2 * j] = __uint_as_float(hraw[j] << 16);
-        f[2 * j + 1] = __uint_as_float(hraw[j] & 0xffff0000u);
-        if constexpr (NORM) {
-            f[2 * j] = round_bf16(__fmul_rn(__fmul_rn(f[2 * j], __uint_as_float(wraw[j] << 16)), rstd));
-            f[2 * j + 1] = round_bf16(__fmul_rn(__fmul_rn(f[2 * j + 1], __uint_as_float(wraw[j] & 0xffff0000u)), rstd));
-        }
+        uint32_t pair = hraw[j];
+        if constexpr (NORM)
+            pair = pack_bf16x2(__fmul_rn(__fmul_rn(__uint_as_float(hraw[j] << 16), __uint_as_float(wraw[j] << 16)), rstd),
+                               __fmul_rn(__fmul_rn(__uint_as_float(hraw[j] & 0xffff0000u), __uint_as_float(wraw[j] & 0xffff0000u)), rstd));
+        f[2 * j] = __uint_as_float(pair << 16);
+        f[2 * j + 1] = __uint_as_float(pair & 0xffff0000u);
+    }
+    if (quant_mode == QUANT_ROUNDED) {                       // uniform: one branch, not one per element
+#pragma unroll
+        for (int j = 0; j < NE / 4; ++j) d[j] = quant_rounded4(f[4 * j], f[4 * j + 1], f[4 * j + 2], f[4 * j + 3], s_mul);
+        return;
     }
 #pragma unroll
     for (int j = 0; j < NE / 4; ++j) d[j] = 0u;
-    const bool eager = quant_mode == QUANT_EAGER;            // uniform: one branch, not one per element
-    if (eager) {
+    if (quant_mode == QUANT_EAGER) {
 #pragma unroll
         for (int e = 0; e < NE; ++e) d[e >> 2] = __builtin_amdgcn_cvt_pk_u8_f32(quant_value(f[e], s_mul, QUANT_EAGER) + 128.0f, e & 3, d[e >> 2]);
     } else {
 #pragma unroll
-        for (int e = 0; e < NE; ++e) d[e >> 2] = __builtin_amdgcn_cvt_pk_u8_f32(quant_value(f[e], s_mul, QUANT_ROUNDED) + 128.0f, e & 3, d[e >> 2]);
+        for (int e = 0; e < NE; ++e) d[e >> 2] = __builtin_amdgcn_cvt_pk_u8_f32(quant_value(f[e], s_mul, QUANT_COMPILED) + 128.0f, e & 3, d[e >> 2]);
     }
 #pragma unroll
     for (int j = 0; j < NE / 4; ++j) d[j] ^= 0x80808080u;

@@ -122,10 +122,15 @@ __device__ __forceinline__ void quant_pass(const float (&h)[NV][8], float amax, 
         const int v = tid + i * kNormThreads;
         if (v < nvec) {
             uint32_t q[2] = {0u, 0u};
+            if (quant_mode == QUANT_ROUNDED) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float r = quant_value(h[i][j], s, quant_mode);
-                q[j >> 2] |= (static_cast<uint32_t>(static_cast<int>(r)) & 0xffu) << (8 * (j & 3));
+                for (int j = 0; j < 2; ++j) q[j] = quant_rounded4(h[i][4 * j], h[i][4 * j + 1], h[i][4 * j + 2], h[i][4 * j + 3], s);
+            } else {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const float r = quant_value(h[i][j], s, quant_mode);
+                    q[j >> 2] |= (static_cast<uint32_t>(static_cast<int>(r)) & 0xffu) << (8 * (j & 3));
+                }
             }
             *reinterpret_cast<u32x2*>(xq_out + row * K + 8 * v) = u32x2{q[0], q[1]};
         }

@@ -136,6 +136,24 @@ def _with_broken_rows(x_bits, kind):
     return x, [0, m - 1], [1, 2]
 
 
+@pytest.mark.parametrize("m", [1, 2, 5, 8, 9, 70])
+def test_every_half_is_quantised_to_its_even_neighbour(m):
+    """Rows of all multiples of a half up to 127 times a power of two, whose scale is that power's inverse: half of the products
+    are ties.  Through an identity matrix the outputs are the integers themselves (up to 8 rows quantised inside the linear, above
+    in front of it): exact."""
+    import ternainfer_amd as T
+    k = 512
+    entry, _ = checkpoint_entry(np.eye(k, dtype=np.int8), [1.0])
+    module = T.SpBitLinear(k, k, entry, "l")
+    halves = torch.zeros(k)
+    halves[:509] = torch.arange(-254, 255) / 2
+    power = 2.0 ** (torch.arange(m) % 7 - 3)[:, None]
+    x = torch.stack([halves.roll(37 * i) for i in range(m)]) * power
+    want = torch.round(x / power) * power                                     # torch.round: ties to even
+    got = module(x.to(torch.bfloat16).cuda())
+    assert torch.equal(got.float().cpu(), want)
+
+
 @pytest.mark.parametrize("m,kind", [(1, "nan"), (1, "inf"), (1, "-inf"), (2, "nan"), (3, "inf"), (4, ""), (8, ""), (9, ""), (64, ""), (65, ""), (300, "")])
 @pytest.mark.parametrize("k", [192, 2560])
 def test_spbitlinear_broken_activations_show_in_the_output(m, kind, k):
