@@ -358,6 +358,39 @@ int ternaspmm_step_inputs(const long long* tokens, const long long* pos, int per
 int ternaspmm_prompt_inputs(const long long* tokens, const long long* pos, int pos_rows, const terna_bf16* embedding, int V, int K,
                             const float* rope_table, int S, int rope_half, terna_bf16* x_out, float* rope_out, int M, terna_stream stream);
 
+/* A decode step of one to four sequences -- embedding rows, every block, everything up to the final norm -- in two launches:
+ * one that forms the inputs (as ternaspmm_step_inputs) and clears `scratch`, and one whose workgroups stay for all blocks and hand
+ * the rows from phase to phase in `scratch` (up to 32 blocks; more take one more launch each).  The same bits as the launches it
+ * stands for: ternaspmm_fused_linear with the partial statistics of the producers, and between them
+ * ternaspmm_rope_decode_attention_partial of `splits` splits (one sequence) or ternaspmm_rope_decode_attention_stats (more), with
+ * ternaspmm_quant_from_stats in front of the down projection from two sequences on.
+ *   blocks   host array of `layers` entries: P2 matrices (w13 as ternaspmm_interleave_gate_up leaves it), bf16 weight scales (ws_13
+ *            two, the others ws_num_*), bf16 norm weights, caches bf16 [M][kv_heads][slots][head_dim]; RoPE pairs are adjacent
+ *   tokens, pos   int64 in device memory, M of them (pos: one for all unless per_sequence); clamped to their tables
+ *   x_out    bf16 [M][dim]: the residual stream behind the last block
+ * Takes head_dim 128, dim and heads * head_dim up to 2560, ffn up to 7168 (multiples of 64), at most 4096 QKV columns; one sequence: two,
+ * four or eight splits of up to 1024 slots; more: splits = 1 and up to 640 slots, not in quant mode 2.
+ * The workgroups wait for each other, so all of them have to be resident: the call is refused where the device (or the
+ * stream's mask of CUs) does not hold four such grids at once -- as many as the runtime's default of four hardware queues runs
+ * side by side; GPU_MAX_HW_QUEUES above that raises the bound.  (More than four such steps at once from several processes, or from
+ * streams of several priorities, are not foreseen.)  A wait that lasts four seconds ends the step with NaN rows.
+ * ternaspmm_decode_step_bytes: bytes of `scratch` (256-byte aligned, its contents do not matter), or -1 for a shape that is not
+ * taken.  ternaspmm_decode_step: 0, or -1 (nothing enqueued).  Only enqueues; calls that overlap need scratch of their own. */
+typedef struct ternaspmm_step_block {
+    const void *wqkv, *wo, *w13, *w2;
+    const terna_bf16 *ws_qkv, *ws_o, *ws_13, *ws_down;
+    const terna_bf16 *attention_norm, *attn_sub_norm, *ffn_norm, *ffn_sub_norm;
+    terna_bf16 *cache_k, *cache_v;
+} ternaspmm_step_block;
+typedef struct ternaspmm_step_desc {
+    int layers, M, dim, ffn, heads, kv_heads, head_dim, slots, splits, per_sequence, vocab;
+    int ws_num_qkv, ws_num_o, ws_num_down;
+    float eps, scale;
+} ternaspmm_step_desc;
+long long ternaspmm_decode_step_bytes(const ternaspmm_step_desc* desc);
+int ternaspmm_decode_step(const ternaspmm_step_desc* desc, const ternaspmm_step_block* blocks, const long long* tokens, const long long* pos,
+                          const terna_bf16* embedding, const float* rope_table, void* scratch, terna_bf16* x_out, terna_stream stream);
+
 /* Load time: band permutation of a P2 gate+up matrix [w1; w3] ([N][K], N = 2F) for TERNASPMM_EPILOGUE_GATE -- band 2j <-
  * rows 16j .. 16j+15 of w1, band 2j+1 <- the same rows of w3.  packed_out: N*K/4 bytes, not `packed`.  Returns 0 / -1. */
 int ternaspmm_interleave_gate_up(const void* packed, void* packed_out, int N, int K, terna_stream stream);

@@ -93,6 +93,8 @@ PROTOTYPES = {
     "ternaspmm_interleave_gate_up": ([_vp, _vp, _ci, _ci, _vp], _ci),
     "ternaspmm_step_inputs": ([_vp, _vp, _ci, _vp, _ci, _ci, _vp, _ci, _ci, _vp, _vp, _vp, _vp, _ci, _vp], _ci),
     "ternaspmm_prompt_inputs": ([_vp, _vp, _ci, _vp, _ci, _ci, _vp, _ci, _ci, _vp, _vp, _ci, _vp], _ci),
+    "ternaspmm_decode_step_bytes": ([_vp], ctypes.c_longlong),
+    "ternaspmm_decode_step": ([_vp] * 9, _ci),
     "ternaspmm_version": ([], ctypes.c_char_p),
 }
 

@@ -18,6 +18,7 @@
 
 #include <algorithm>
 #include <cstdarg>
+#include <vector>
 
 #include "../../include/ternaspmm.h"
 
@@ -51,7 +52,9 @@ namespace {
     X(ternaspmm_attention_merge_rmsnorm_quant)                                                                         \
     X(ternaspmm_row_stats_count)                                                                                       \
     X(ternaspmm_step_inputs)                                                                                           \
-    X(ternaspmm_prompt_inputs)
+    X(ternaspmm_prompt_inputs)                                                                                         \
+    X(ternaspmm_decode_step_bytes)                                                                                     \
+    X(ternaspmm_decode_step)
 struct Library {
 #define X(name) decltype(&::name) name = nullptr;
     TERNA_ENTRY_POINTS(X)
@@ -762,6 +765,67 @@ TERNA_FUNCTION(prompt_inputs, 4)
     return pack(unlocked, std::move(x), std::move(rope));
 }
 
+// (tokens, pos, embedding, rope_table, heads, head_dim, scale, eps, splits, blocks) -> the residual stream behind the last block, bf16 [B, dim],
+// or None where the step is not one for this launch (the launches it stands for have the checks that raise).  blocks: a sequence of tuples (wqkv, ws, ws_num, out_features, wo [4], interleaved
+// w13 [4], w2 [4], attention_norm, attn_sub_norm, ffn_norm, ffn_sub_norm, cache_k, cache_v).
+TERNA_FUNCTION(decode_step, 10)
+{
+    const char* who = "decode_step";
+    const at::Tensor &tokens = tensor(a[0]), &pos = tensor(a[1]), &embedding = tensor(a[2]), &table = tensor(a[3]);
+    check_matrix(who, embedding);
+    const int64_t b = tokens.numel(), v = embedding.size(0), dim = embedding.size(1);
+    const int64_t heads = integer32(a[4]), head_dim = integer32(a[5]), wide = heads * head_dim;
+    if (table.dim() != 3 || table.size(1) != 2 || 2 * table.size(2) != head_dim || tokens.scalar_type() != at::kLong || pos.scalar_type() != at::kLong ||
+        (pos.numel() != 1 && pos.numel() != b) || table.scalar_type() != at::kFloat || embedding.scalar_type() != at::kBFloat16 || !embedding.is_contiguous() ||
+        !table.is_contiguous() || !embedding.is_cuda())
+        Py_RETURN_NONE;
+    if (!PyTuple_Check(a[9]) && !PyList_Check(a[9])) refuse("%s: blocks is a list", who);
+    const Py_ssize_t layers = PySequence_Fast_GET_SIZE(a[9]);
+    if (b < 1 || b > 64 || layers < 1 || layers > 1024) Py_RETURN_NONE;
+    ternaspmm_step_desc d{};
+    d.layers = layers, d.M = b, d.dim = dim, d.heads = heads, d.head_dim = head_dim, d.slots = table.size(0);
+    d.splits = integer32(a[8]), d.per_sequence = pos.numel() == b && b > 1, d.vocab = v;
+    d.scale = real(a[6]), d.eps = real(a[7]);
+    std::vector<ternaspmm_step_block> blocks(layers);
+    for (Py_ssize_t n = 0; n < layers; ++n) {
+        PyObject* item = PySequence_Fast_GET_ITEM(a[9], n);
+        if (!PyTuple_Check(item) || PyTuple_GET_SIZE(item) != 22) refuse("%s: a block is a tuple of 22", who);
+        PyObject* const* p = reinterpret_cast<PyTupleObject*>(item)->ob_item;
+        const int64_t qkv_n = integer32(p[3]), gate_n = integer32(p[11]), ffn = gate_n / 2;
+        const BlockLinear qkv_w(who, p, dim), o_w(who, p + 4, wide), gate_w(who, p + 8, dim), down_w(who, p + 12, ffn);
+        const at::Tensor* norm[4] = {&tensor(p[16]), &tensor(p[17]), &tensor(p[18]), &tensor(p[19])};
+        const int64_t want[4] = {dim, wide, dim, ffn};
+        for (int i = 0; i < 4; ++i)
+            if (norm[i]->numel() != want[i] || norm[i]->scalar_type() != at::kBFloat16 || !norm[i]->is_contiguous()) Py_RETURN_NONE;
+        const at::Tensor &ck = tensor(p[20]), &cv = tensor(p[21]);
+        if (ck.dim() != 4 || ck.sizes() != cv.sizes() || ck.size(0) != b || ck.size(2) != d.slots || ck.size(3) != head_dim || !ck.is_contiguous() ||
+            !cv.is_contiguous() || ck.scalar_type() != at::kBFloat16 || cv.scalar_type() != at::kBFloat16)
+            Py_RETURN_NONE;
+        const int kv = ck.size(1);
+        if (o_w.n != dim || down_w.n != dim || qkv_n != (heads + 2 * kv) * head_dim) Py_RETURN_NONE;
+        if (n == 0) {
+            d.kv_heads = kv, d.ffn = ffn, d.ws_num_qkv = qkv_w.ws_num, d.ws_num_o = o_w.ws_num, d.ws_num_down = down_w.ws_num;
+        } else if (d.kv_heads != kv || d.ffn != ffn || d.ws_num_qkv != qkv_w.ws_num || d.ws_num_o != o_w.ws_num || d.ws_num_down != down_w.ws_num) {
+            Py_RETURN_NONE;                      // blocks of different shapes
+        }
+        if (gate_w.ws_num != 2 || ffn * 2 != gate_n) Py_RETURN_NONE;
+        blocks[n] = ternaspmm_step_block{data(&qkv_w.packed), data(&o_w.packed), data(&gate_w.packed), data(&down_w.packed),
+                                         data<terna_bf16>(&qkv_w.ws), data<terna_bf16>(&o_w.ws), data<terna_bf16>(&gate_w.ws), data<terna_bf16>(&down_w.ws),
+                                         data<terna_bf16>(norm[0]), data<terna_bf16>(norm[1]), data<terna_bf16>(norm[2]), data<terna_bf16>(norm[3]),
+                                         data<terna_bf16>(&ck), data<terna_bf16>(&cv)};
+    }
+    const long long bytes = lib.ternaspmm_decode_step_bytes(&d);
+    if (bytes < 0) Py_RETURN_NONE;
+    Unlocked unlocked;
+    const at::Tensor ids = tokens.contiguous(), at_slot = pos.contiguous();
+    at::Tensor x = make({b, dim}, at::kBFloat16, embedding);
+    const c10::DataPtr scratch = device_allocator()->allocate(bytes);
+    if (lib.ternaspmm_decode_step(&d, blocks.data(), data<long long>(&ids), data<long long>(&at_slot), data<terna_bf16>(&embedding), data<float>(&table), scratch.get(),
+                                  data<terna_bf16>(&x), stream()) != 0)
+        return none(unlocked);
+    return wrap(std::move(x), unlocked);
+}
+
 // (path of libternaspmm.so)
 TERNA_FUNCTION(init, 1)
 {
@@ -786,7 +850,7 @@ TERNA_FUNCTION(init, 1)
 PyMethodDef methods[] = {METHOD(init), METHOD(bit_linear), METHOD(bit_linear_bf16), METHOD(quant_input), METHOD(linear_packed),
                          METHOD(linear_bf16_packed), METHOD(rmsnorm_quant), METHOD(relu2_mul_rmsnorm_quant), METHOD(quant_from_stats),
                          METHOD(fused_linear), METHOD(prompt_attention), METHOD(decode_attention), METHOD(block),
-                         METHOD(attention_merge_rmsnorm_quant), METHOD(step_inputs), METHOD(prompt_inputs), {nullptr, nullptr, 0, nullptr}};
+                         METHOD(attention_merge_rmsnorm_quant), METHOD(step_inputs), METHOD(prompt_inputs), METHOD(decode_step), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

@@ -414,6 +414,12 @@ class Block:
         return x, ffn
 
 
+#: switches of the chained step whose other settings ask for its launches one by one (Transformer.whole_step)
+_STEP_SWITCHES = (("step_inputs", True), ("deferred_attention_merge", True), ("attention_splits", None), ("split_merge_quant", False), ("defer_above", 640),
+                  ("chain_rows", 4))
+_CHAIN_SWITCHES = (("o_norm_rows", 4), ("attention_stats_chain", True), ("attention_stats", True), ("merge_quant", True), ("chain_down_rows", 2))
+
+
 class Transformer:
     """Random-init decoder; `act` selects int8-quantised (reference semantics) or bf16 activations."""
 
@@ -549,6 +555,34 @@ class Transformer:
             held[bsz] = torch.zeros(nbytes, dtype=torch.int8, device="cuda")
         return held[bsz]
 
+    # the step as one launch of resident workgroups (whole_step), where the library takes it
+    one_launch_step = True
+
+    def whole_step(self, tokens, cache, pos_idx, max_seq):
+        """The residual stream behind the last block of a single-token step of up to four sequences, all blocks in one launch
+        (ternaspmm_decode_step), or None: where the library does not take the shape, and where something asks for the launches it
+        stands for -- a recording block, a prefetch, a switch of the chain that is not at its default.  The same bits as
+        those launches (Block.forward_chain with `split` False)."""
+        a = self.args
+        bsz = tokens.shape[0]
+        if bsz > self.chain_rows or bsz > 4 or not self.one_launch_step or not a.rope_adjacent or a.head_dim != 128 or \
+                any(getattr(self, name, default) != default for name, default in _STEP_SWITCHES) or \
+                any(getattr(Block, name) != default for name, default in _CHAIN_SWITCHES) or \
+                any(blk.capture is not None or blk.prefetch is not None or not blk.fused or blk.act != "int8" or type(blk) is not Block for blk in self.layers):
+            return None
+        splits = 1
+        if bsz == 1:
+            splits = _lib.load().ternaspmm_attention_partial_splits_kv(1, a.n_heads, a.n_kv_heads, max_seq)
+            if splits < 2:
+                return None
+        elif max_seq > self.defer_above:
+            return None
+        lin = lambda w, packed: (packed, w.ws, w.ws_num, w.n)
+        blocks = [lin(b.wqkv, b.wqkv.packed) + lin(b.wo, b.wo.packed) + lin(b.w13, b.gate_up_interleaved()) + lin(b.w2, b.w2.packed) +
+                  (b.attention_norm, b.attn_sub_norm, b.ffn_norm, b.ffn_sub_norm, ck, cv) for b, (ck, cv) in zip(self.layers, cache)]
+        return _lib.native().decode_step(tokens, pos_idx.reshape(-1), self.tok_embeddings, self.rope_tables(max_seq, tokens.device), a.n_heads, a.head_dim,
+                                         a.head_dim ** -0.5, a.norm_eps, splits, blocks)
+
     def make_cache(self, bsz: int, max_seq: int):
         a = self.args
         shape = (bsz, a.n_kv_heads, max_seq, a.head_dim)
@@ -572,6 +606,10 @@ class Transformer:
         # one new token for a few sequences: the linears chained through producer-side norm statistics (forward_chain)
         chain = one_launch_attention and self.layers[0].act == "int8" and bsz <= max(self.chain_rows, self.split_rows) and getattr(self, "chain", True) and self.chain_supported()
         stats = None
+        if chain and trace is None and last_idx is None:
+            x = self.whole_step(tokens, cache, pos_idx, max_seq)
+            if x is not None:                                                 # the blocks of the step in one launch
+                return self.head(x, None, bsz)
         if chain and getattr(self, "step_inputs", True):
             # embedding rows, their partials under the first block's norm and the RoPE rows of the positions: one launch
             x, stats, cos, sin = step_inputs(tokens, pos_idx.reshape(-1), self.tok_embeddings, self.rope_tables(max_seq, dev), self.layers[0].attention_norm)
@@ -614,6 +652,11 @@ class Transformer:
             x, pending = x.index_select(0, pick), None if pending is None else pending.index_select(0, pick)
         elif t > 1:                                                           # only the last new token feeds the head
             x, pending = x.view(bsz, t, a.dim)[:, -1].contiguous(), None if pending is None else pending.view(bsz, t, a.dim)[:, -1].contiguous()
+        return self.head(x, pending, bsz)
+
+    def head(self, x, pending, bsz):
+        """Logits of the rows x (+ pending): last residual add, final norm, LM head."""
+        a = self.args
         if self.layers[0].fused and x.is_cuda:                                # last residual add + final norm: one launch
             x, _ = rmsnorm_quant(x, self.norm, a.norm_eps, residual=pending, quant=False)     # (pending None: the stream has it)
         else:
