@@ -532,7 +532,7 @@ void ternaspmm_rope_decode_attention_prefetch(const terna_bf16* qkv, const float
  * ternaspmm_attention_partial_splits_kv(B, H, KV, S) is the recommendation for that form: it splits from 512 slots on. */
 long long ternaspmm_attention_partial_bytes(int B, int H, int D);
 int ternaspmm_attention_partial_splits(int B, int H, int S);
-int ternaspmm_attention_partial_splits_kv(int B, int H, int KV, int S);   /* the same, knowing the kv heads: see below */
+int ternaspmm_attention_partial_splits_kv(int B, int H, int KV, int S);   /* the same, knowing the kv heads: see above */
 void ternaspmm_rope_decode_attention_partial(const terna_bf16* qkv, const float* cos, const float* sin, const long long* pos,
                                              int per_sequence, terna_bf16* cache_k, terna_bf16* cache_v, float* partial, int splits,
                                              int B, int H, int KV, int D, int S, float scale, int adjacent,
@@ -547,6 +547,17 @@ void ternaspmm_attention_merge(const float* partial, int splits, terna_bf16* out
  * returns 0, or -1 for anything else (nothing enqueued). */
 int ternaspmm_attention_merge_rmsnorm_quant(const float* partial, int splits, const terna_bf16* norm_weight, float eps, terna_bf16* o_out,
                                             int8_t* xq_out, terna_bf16* s_out, int B, int H, int D, terna_stream stream);
+/* The pair for any split count from 1 to 8, as a decode step of several sequences launches it: ternaspmm_step_attention is
+ * ternaspmm_rope_decode_attention_partial, ternaspmm_step_attention_merge is ternaspmm_attention_merge_rmsnorm_quant;
+ * both return 0, or -1 with nothing enqueued.  ternaspmm_step_attention_splits(B, H, KV, S): the count that fills the chip
+ * (one sequence, or other than 2 or 4 heads per kv head: ternaspmm_attention_partial_splits_kv). */
+int ternaspmm_step_attention_splits(int B, int H, int KV, int S);
+int ternaspmm_step_attention(const terna_bf16* qkv, const float* cos, const float* sin, const long long* pos, int per_sequence,
+                             terna_bf16* cache_k, terna_bf16* cache_v, float* partial, int splits, int B, int H, int KV, int D, int S,
+                             float scale, int adjacent, const void* const* pf_ptr, const long long* pf_bytes, const long long* pf_unit_bytes,
+                             int pf_count, terna_stream stream);
+int ternaspmm_step_attention_merge(const float* partial, int splits, const terna_bf16* norm_weight, float eps, terna_bf16* o_out,
+                                   int8_t* xq_out, terna_bf16* s_out, int B, int H, int D, terna_stream stream);
 
 /* The bookkeeping of one greedy decode step in one launch (generate.py:283-305: argmax, tokens[:, pos] = next_token,
  * the position counters): tok[b] = argmax(logits[b]) as above; if history != NULL and counters[1] < history_len,

@@ -125,33 +125,36 @@ void launch_attention_deferred(const uint16_t* qkv, uint16_t* ck, uint16_t* cv, 
 
 int prefetch_workgroups(const AttentionPrefetch& pf, int slots);
 
-// The deferred-merge launch with one workgroup per (sequence, kv head, split) (attention_grouped_kernel.h).  Returns false
-// where that form does not apply: one head per kv head, a group size other than 2 or 4, a score buffer beyond the LDS.
-template <int D, bool ADJ>
+// One workgroup per (sequence, kv head, split) (attention_grouped_kernel.h): the deferred merge, or -- WHOLE, one split -- the output
+// itself.  Returns false where that form does not apply: one head per kv head, a group size other than 2 or 4, a score buffer
+// beyond the LDS.
+// Up to 256 workgroups eight waves each; more of them four, so that two or three share a CU (64 sequences, 1024 slots filled to 60 %: step
+// 2198 -> 2069 us; 32 sequences, 160 workgroups: 1531 with eight, 1614 with four).
+template <int D, bool ROPE, bool ADJ, bool WHOLE>
 bool launch_attention_grouped(const uint16_t* qkv, uint16_t* ck, uint16_t* cv, const float* cos, const float* sin, const long long* pos,
-                              int per_seq, float* partial, int splits, int B, int H, int KV, int S, float scale,
+                              int per_seq, float* partial, uint16_t* out, int splits, int B, int H, int KV, int S, float scale,
                               const AttentionPrefetch& pf_in, hipStream_t st)
 {
-    static const int waves = [] {
-        // 8 waves: measured ahead of 4 at 2 - 8 sequences with caches of 1528 slots (8 sequences: 1.351 against 1.410 ms
-        // per decode step), level with them at 384 slots
+    static const int forced = [] {
         const char* v = tuning_env("TERNASPMM_ATTN_GROUPED_WAVES");
-        return v && std::atoi(v) == 4 ? 4 : 8;
+        const int n = v ? std::atoi(v) : 0;
+        return n == 4 || n == 8 ? n : 0;
     }();
     if (KV < 1 || H % KV != 0) return false;
     const int gq = H / KV;
     if (gq != 2 && gq != 4) return false;
+    const int slots = B * KV * splits;
+    const int waves = forced ? forced : slots <= 256 ? 8 : 4;
     const size_t lds = grouped_attention_lds_bytes(D, waves, gq, S);
     if (lds > 159 * 1024) return false;          // (160 KB per workgroup, the kernel's static LDS included)
     AttentionPrefetch pf = pf_in;
-    const int slots = B * KV * splits;
     pf.workgroups = prefetch_workgroups(pf, slots);
 #define TERNA_GROUPED(NWAVES, GQ)                                                                                          \
     do {                                                                                                                   \
-        auto kernel = terna_decode_attention_grouped_kernel<D, ADJ, NWAVES, GQ>;                                            \
+        auto kernel = terna_decode_attention_grouped_kernel<D, ROPE, ADJ, NWAVES, GQ, WHOLE>;                                    \
         if (lds > 64 * 1024) allow_dynamic_lds(kernel, 159 * 1024, "hipFuncSetAttribute(decode attention, kv groups)", __LINE__); \
         kernel<<<dim3(slots + pf.workgroups), dim3(64 * NWAVES), lds, st>>>(qkv, ck, cv, pos, KV, S, splits, slots, per_seq, scale, cos, sin, \
-                                                                            partial, pf);                                  \
+                                                                            partial, out, pf);                             \
     } while (0)
     if (waves == 8) {
         if (gq == 4) TERNA_GROUPED(8, 4);
@@ -171,6 +174,14 @@ void launch_attention(const uint16_t* q, uint16_t* ck, uint16_t* cv, const float
                              AttentionStats stats = AttentionStats{nullptr, nullptr})
 {
     const int splits = attention_splits(B, H, S, scratch);
+    // More heads than two a CU: the heads of a kv group in one workgroup, which loads their keys and values once instead of four times
+    // (32 sequences, 512 slots: launch 12.8 -> 10.5 us; 48, 1024 slots: step 2046 -> 1790; 64, 512 slots: 2104 -> 1866).  Fewer heads fill
+    // the chip by themselves (20 sequences, 512 slots: 1607 us a step either way).
+    {
+        const bool crowded = splits == 1 && stats.out == nullptr && static_cast<long>(B) * H > 512;
+        if (crowded && D == 128 && launch_attention_grouped<128, ROPE, ADJ, true>(q, ck, cv, cos, sin, pos, per_seq, nullptr, out, 1, B, H, KV, S, scale, pf, st)) return;
+        if (crowded && D == 64 && launch_attention_grouped<64, ROPE, ADJ, true>(q, ck, cv, cos, sin, pos, per_seq, nullptr, out, 1, B, H, KV, S, scale, pf, st)) return;
+    }
     const int nw = splits > 1 ? 4 : attention_waves(B, H);       // a split is a short prefix: the narrow workgroup
 #define TERNA_ATTN(DIM, NWAVES, SPLIT) \
     launch_attention_as<DIM, ROPE, ADJ, NWAVES, SPLIT>(q, ck, cv, cos, sin, pos, per_seq, out, B, H, KV, S, scale, splits, scratch, pf, st, stats)
@@ -436,6 +447,26 @@ int ternaspmm_attention_partial_splits_kv(int B, int H, int KV, int S)
     return ternaspmm_attention_partial_splits(B, H, S);
 }
 
+int ternaspmm_step_attention_splits(int B, int H, int KV, int S)
+{
+    if (B < 1 || H < 1 || KV < 1 || H % KV != 0 || S < 1) return -1;
+    const int gq = H / KV;
+    // The grid of the grouped kernel is B * KV * splits workgroups that each have a CU to themselves, so as many splits as the chip
+    // holds -- the tiles go round, whatever their number -- of 160 slots at least, below which another one costs the merge more than
+    // it saves (16 sequences, 384 slots: two 1225 us, three 1238).  The 2B shape, us a step, powers of two -> this: 16 sequences, 1528
+    // slots 1455 (two) -> 1385 (three); 8 1253 (four) -> 1239 (six); 7 1243 (four) -> 1234 (seven).
+    // Kv heads for more than half the CUs are split from 1024 slots on, over four waves each and as many as make two workgroups a CU (unsplit
+    // -> two -> three, caches filled to 60 %: 32 sequences, 1024 slots 1683 -> 1665 -> 1646, 768 slots 1593 -> 1632 -> 1605; 40 sequences, 1528
+    // slots 1908 -> 1851 -> 1957; 51, 1528 slots 2056 -> 2043; 64, 2048 slots 2963 -> 3044).
+    if (B >= 2 && (gq == 2 || gq == 4)) {
+        const long groups = static_cast<long>(B) * KV;
+        long sp = groups <= 128 ? 256 / groups : S >= 1024 ? 512 / groups : 1;
+        if (sp > S / 160) sp = S / 160;
+        return sp < 1 ? 1 : sp > kAttentionMaxSplits ? kAttentionMaxSplits : static_cast<int>(sp);
+    }
+    return ternaspmm_attention_partial_splits_kv(B, H, KV, S);
+}
+
 void ternaspmm_rope_decode_attention_partial(const terna_bf16* qkv, const float* cos, const float* sin, const long long* pos,
                                              int per_sequence, terna_bf16* cache_k, terna_bf16* cache_v, float* partial, int splits,
                                              int B, int H, int KV, int D, int S, float scale, int adjacent,
@@ -443,11 +474,19 @@ void ternaspmm_rope_decode_attention_partial(const terna_bf16* qkv, const float*
                                              int pf_count, terna_stream stream)
 {
     if (!attention_args_ok("ternaspmm_rope_decode_attention_partial", B, H, KV, D, S)) return;
-    if (splits < 1 || splits > kAttentionMaxSplits || (splits & (splits - 1)) || partial == nullptr ||
-        static_cast<long>(B) * H * splits > 65536) {
+    if (splits < 1 || (splits & (splits - 1)) ||
+        ternaspmm_step_attention(qkv, cos, sin, pos, per_sequence, cache_k, cache_v, partial, splits, B, H, KV, D, S, scale, adjacent, pf_ptr, pf_bytes,
+                                 pf_unit_bytes, pf_count, stream) != 0)
         std::fprintf(stderr, "ternaspmm_rope_decode_attention_partial: unsupported splits=%d (1, 2, 4 or 8) or no partial buffer\n", splits);
-        return;
-    }
+}
+
+int ternaspmm_step_attention(const terna_bf16* qkv, const float* cos, const float* sin, const long long* pos, int per_sequence,
+                             terna_bf16* cache_k, terna_bf16* cache_v, float* partial, int splits, int B, int H, int KV, int D, int S, float scale,
+                             int adjacent, const void* const* pf_ptr, const long long* pf_bytes, const long long* pf_unit_bytes, int pf_count,
+                             terna_stream stream)
+{
+    if (!attention_args_ok("ternaspmm_step_attention", B, H, KV, D, S)) return -1;
+    if (splits < 1 || splits > kAttentionMaxSplits || partial == nullptr || static_cast<long>(B) * H * splits > 65536) return -1;
     AttentionPrefetch pf = prefetch_regions(pf_ptr, pf_bytes, pf_unit_bytes, pf_count);
     hipStream_t st = static_cast<hipStream_t>(stream);
     // several sequences: the heads of a kv group share a workgroup (TERNASPMM_ATTN_GROUPED=0|1 forces either form)
@@ -457,14 +496,14 @@ void ternaspmm_rope_decode_attention_partial(const terna_bf16* qkv, const float*
     }();
     if (forced_grouped >= 0 ? forced_grouped != 0 : B >= 2) {
         bool done;
-        if (D == 128) done = adjacent ? launch_attention_grouped<128, true>(qkv, cache_k, cache_v, cos, sin, pos, per_sequence != 0, partial, splits, B, H, KV, S, scale, pf, st)
-                                      : launch_attention_grouped<128, false>(qkv, cache_k, cache_v, cos, sin, pos, per_sequence != 0, partial, splits, B, H, KV, S, scale, pf, st);
-        else done = adjacent ? launch_attention_grouped<64, true>(qkv, cache_k, cache_v, cos, sin, pos, per_sequence != 0, partial, splits, B, H, KV, S, scale, pf, st)
-                             : launch_attention_grouped<64, false>(qkv, cache_k, cache_v, cos, sin, pos, per_sequence != 0, partial, splits, B, H, KV, S, scale, pf, st);
+        if (D == 128) done = adjacent ? launch_attention_grouped<128, true, true, false>(qkv, cache_k, cache_v, cos, sin, pos, per_sequence != 0, partial, nullptr, splits, B, H, KV, S, scale, pf, st)
+                                      : launch_attention_grouped<128, true, false, false>(qkv, cache_k, cache_v, cos, sin, pos, per_sequence != 0, partial, nullptr, splits, B, H, KV, S, scale, pf, st);
+        else done = adjacent ? launch_attention_grouped<64, true, true, false>(qkv, cache_k, cache_v, cos, sin, pos, per_sequence != 0, partial, nullptr, splits, B, H, KV, S, scale, pf, st)
+                             : launch_attention_grouped<64, true, false, false>(qkv, cache_k, cache_v, cos, sin, pos, per_sequence != 0, partial, nullptr, splits, B, H, KV, S, scale, pf, st);
         if (done) {
             const hipError_t e = hipGetLastError();
-            if (e != hipSuccess) die("ternaspmm_rope_decode_attention_partial", e, __LINE__);
-            return;
+            if (e != hipSuccess) die("ternaspmm_step_attention", e, __LINE__);
+            return 0;
         }
     }
     const bool grouped = attention_groups_on(H, KV);
@@ -481,7 +520,8 @@ void ternaspmm_rope_decode_attention_partial(const terna_bf16* qkv, const float*
     }
 #undef TERNA_DEFER
     const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) die("ternaspmm_rope_decode_attention_partial", e, __LINE__);
+    if (e != hipSuccess) die("ternaspmm_step_attention", e, __LINE__);
+    return 0;
 }
 
 void ternaspmm_attention_merge(const float* partial, int splits, terna_bf16* out, int B, int H, int D, terna_stream stream)
@@ -500,8 +540,15 @@ void ternaspmm_attention_merge(const float* partial, int splits, terna_bf16* out
 int ternaspmm_attention_merge_rmsnorm_quant(const float* partial, int splits, const terna_bf16* norm_weight, float eps, terna_bf16* o_out,
                                             int8_t* xq_out, terna_bf16* s_out, int B, int H, int D, terna_stream stream)
 {
+    if (splits < 1 || (splits & (splits - 1))) return -1;
+    return ternaspmm_step_attention_merge(partial, splits, norm_weight, eps, o_out, xq_out, s_out, B, H, D, stream);
+}
+
+int ternaspmm_step_attention_merge(const float* partial, int splits, const terna_bf16* norm_weight, float eps, terna_bf16* o_out,
+                                   int8_t* xq_out, terna_bf16* s_out, int B, int H, int D, terna_stream stream)
+{
     const long long K = static_cast<long long>(H) * D;
-    if (B < 1 || H < 1 || (D != 64 && D != 128) || (splits != 1 && splits != 2 && splits != 4 && splits != 8) || K > 2048 * 2 ||
+    if (B < 1 || H < 1 || (D != 64 && D != 128) || splits < 1 || splits > kAttentionMaxSplits || K > 2048 * 2 ||
         partial == nullptr || norm_weight == nullptr || xq_out == nullptr || s_out == nullptr)
         return -1;
     hipStream_t st = static_cast<hipStream_t>(stream);
@@ -517,17 +564,23 @@ int ternaspmm_attention_merge_rmsnorm_quant(const float* partial, int splits, co
     } while (0)
 #define TERNA_MERGE_NQ_D(DIM)                                                                                             \
     do {                                                                                                                  \
-        if (splits == 1) TERNA_MERGE_NQ(DIM, 1);                                                                          \
-        else if (splits == 2) TERNA_MERGE_NQ(DIM, 2);                                                                     \
-        else if (splits == 4) TERNA_MERGE_NQ(DIM, 4);                                                                     \
-        else TERNA_MERGE_NQ(DIM, 8);                                                                                      \
+        switch (splits) {                                                                                                 \
+            case 1: TERNA_MERGE_NQ(DIM, 1); break;                                                                        \
+            case 2: TERNA_MERGE_NQ(DIM, 2); break;                                                                        \
+            case 3: TERNA_MERGE_NQ(DIM, 3); break;                                                                        \
+            case 4: TERNA_MERGE_NQ(DIM, 4); break;                                                                        \
+            case 5: TERNA_MERGE_NQ(DIM, 5); break;                                                                        \
+            case 6: TERNA_MERGE_NQ(DIM, 6); break;                                                                        \
+            case 7: TERNA_MERGE_NQ(DIM, 7); break;                                                                        \
+            default: TERNA_MERGE_NQ(DIM, 8); break;                                                                       \
+        }                                                                                                                 \
     } while (0)
     if (D == 128) TERNA_MERGE_NQ_D(128);
     else TERNA_MERGE_NQ_D(64);
 #undef TERNA_MERGE_NQ_D
 #undef TERNA_MERGE_NQ
     const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) die("ternaspmm_attention_merge_rmsnorm_quant", e, __LINE__);
+    if (e != hipSuccess) die("ternaspmm_step_attention_merge", e, __LINE__);
     return 0;
 }
 

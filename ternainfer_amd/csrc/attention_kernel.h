@@ -345,7 +345,7 @@ constexpr size_t decode_attention_lds_bytes(int D, int NW, int S)
 // as its scores are out, and the second round of value rows right after the last scores, in the registers that held keys; no byte
 // more is read (the requests are bounded by the prefix).  The branch stands in front of the whole pass: within it the number of requests in
 // flight is known at every wait.  The price is twice the code, which every launch fetches anew: 1.2 us at prefixes of one or two rounds.
-// Measured, us per decode step of the 2B shape, caches filled to 60 %, plain -> rounds: 32 sequences x 512 slots 1630 -> 1680, x 768
+// Measured, us per decode step of the 2B shape one workgroup a head, caches filled to 60 %, plain -> rounds: 32 sequences x 512 slots 1630 -> 1680, x 768
 // 1730 -> 1777, x 1024 1847 -> 1829, x 2048 2401 -> 2184; 48 x 1024 2254 -> 2100; 64 x 1024 2434 -> 2327.
 template <int KT, int STEP, typename Load, typename Score, typename Tile>
 __device__ __forceinline__ void key_rounds(int first, int tiles, Tile (&k)[KT], Load load, Score score)

@@ -46,9 +46,11 @@ namespace {
     X(ternaspmm_prefill_attention)                                                                                     \
     X(ternaspmm_rope_decode_attention)                                                                                 \
     X(ternaspmm_rope_decode_attention_stats)                                                                           \
-    X(ternaspmm_rope_decode_attention_partial)                                                                         \
+    X(ternaspmm_step_attention)                                                                                        \
+    X(ternaspmm_step_attention_merge)                                                                                  \
     X(ternaspmm_attention_partial_bytes)                                                                               \
     X(ternaspmm_attention_workspace_bytes)                                                                             \
+    X(ternaspmm_attention_merge)                                                                                       \
     X(ternaspmm_attention_merge_rmsnorm_quant)                                                                         \
     X(ternaspmm_row_stats_count)                                                                                       \
     X(ternaspmm_step_inputs)                                                                                           \
@@ -561,8 +563,12 @@ TERNA_FUNCTION(decode_attention, 14)
         if (need < 0 || static_cast<long long>(partial->numel() * partial->element_size()) < need) refuse("%s: the partial buffer is too small", who);
         const int splits = integer32(a[13]);
         Unlocked unlocked;
-        lib.ternaspmm_rope_decode_attention_partial(TERNA_ATTENTION_INPUTS(data<terna_bf16>(&qkv), g), ck, cv, data<float>(partial), splits, g.batch, g.heads, g.kv,
-                                                    g.head_dim, g.slots, g.scale, g.adjacent, nullptr, nullptr, nullptr, 0, st);
+        const int left = lib.ternaspmm_step_attention(TERNA_ATTENTION_INPUTS(data<terna_bf16>(&qkv), g), ck, cv, data<float>(partial), splits, g.batch, g.heads, g.kv,
+                                                      g.head_dim, g.slots, g.scale, g.adjacent, nullptr, nullptr, nullptr, 0, st);
+        if (left != 0) {
+            unlocked.end();
+            refuse("%s: one to eight splits, 65536 of all heads", who);
+        }
         return none(unlocked);
     }
     check_numel(who, "norm_weight", weight, g.heads * g.head_dim);
@@ -595,7 +601,7 @@ struct BlockLinear {
     }
 };
 
-// (x, pending | None, cos, sin, pos, cache_k, cache_v, heads, head_dim, scale, adjacent, eps, attention workspace | None, linear workspace | None,
+// (x, pending | None, cos, sin, pos, cache_k, cache_v, heads, head_dim, scale, adjacent, eps, attention workspace | (partial results, splits) | None, linear workspace | None,
 //  attention_norm, attn_sub_norm, ffn_norm, ffn_sub_norm, wqkv [4], wo [4], w13 [4], w2 [4], interleaved w13 | None) -> (stream, pending; None where the stream has it): a whole block on int8
 // activations with its norms as launches of their own (prompt pass, decode steps of many sequences): the nine launches and nothing
 // else.  Called one by one from Python they cost 53 us of host time, more than they take on the device up to a hundred tokens.
@@ -603,7 +609,15 @@ TERNA_FUNCTION(block, 35)
 {
     const char* who = "block";
     const at::Tensor& x = tensor(a[0]);
-    const at::Tensor *pending = optional(a[1]), *attn_work = optional(a[12]), *work = optional(a[13]), *interleaved = optional(a[34]);
+    const at::Tensor *pending = optional(a[1]), *attn_work = nullptr, *partial = nullptr, *work = optional(a[13]), *interleaved = optional(a[34]);
+    int splits = 1;
+    if (PyTuple_Check(a[12])) {
+        if (PyTuple_GET_SIZE(a[12]) != 2) refuse("%s: (partial results, splits)", who);
+        partial = &tensor(PyTuple_GET_ITEM(a[12], 0));
+        splits = integer32(PyTuple_GET_ITEM(a[12], 1));
+    } else {
+        attn_work = optional(a[12]);
+    }
     const at::Tensor *norm[4] = {&tensor(a[14]), &tensor(a[15]), &tensor(a[16]), &tensor(a[17])};
     const int64_t heads = integer32(a[7]), head_dim = integer32(a[8]);
     const float eps = real(a[11]);
@@ -624,6 +638,9 @@ TERNA_FUNCTION(block, 35)
     if (g.t == 1 && attn_work != nullptr && static_cast<long long>(attn_work->numel() * attn_work->element_size()) <
                                                 lib.ternaspmm_attention_workspace_bytes(g.batch, heads, head_dim))
         refuse("%s: the attention workspace is too small", who);
+    if (partial != nullptr && (g.t != 1 || splits < 1 || splits > 8 || g.batch * heads * splits > 65536 ||
+                               static_cast<long long>(partial->numel() * partial->element_size()) < lib.ternaspmm_attention_partial_bytes(g.batch, heads, head_dim)))
+        refuse("%s: split attention takes one new token, one to eight splits and a buffer that holds their results", who);
 
     Unlocked unlocked;
     // scratch of this call, in one piece: int8 rows and scales; then qkv, rotated queries, attention output and its projection,
@@ -665,6 +682,9 @@ TERNA_FUNCTION(block, 35)
     } else if (g.t > 1) {
         lib.ternaspmm_rope_kv_store(TERNA_ATTENTION_INPUTS(qkv, g), q, ck, cv, g.batch, g.t, heads, g.kv, head_dim, g.slots, g.adjacent, st);
         lib.ternaspmm_prefill_attention(q, ck, cv, data<long long>(&g.pos), g.each, o, g.batch, g.t, heads, g.kv, head_dim, g.slots, g.scale, st);
+    } else if (partial != nullptr) {
+        lib.ternaspmm_step_attention(TERNA_ATTENTION_INPUTS(qkv, g), ck, cv, data<float>(partial), splits, g.batch, heads, g.kv, head_dim, g.slots, g.scale, g.adjacent,
+                                     nullptr, nullptr, nullptr, 0, st);
     } else {
         lib.ternaspmm_rope_decode_attention(TERNA_ATTENTION_INPUTS(qkv, g), ck, cv, o, g.batch, heads, g.kv, head_dim, g.slots, g.scale, g.adjacent,
                                             data(attn_work), st);
@@ -674,7 +694,11 @@ TERNA_FUNCTION(block, 35)
         return lib.ternaspmm_residual_linear(xq, data(&w.packed), to, s, data<terna_bf16>(&w.ws), w.ws_num, stream_in, m, w.n, k, data(work),
                                              work != nullptr ? work->numel() : 0, st) == 1;
     };
-    lib.ternaspmm_rmsnorm_quant(o, nullptr, nullptr, data<terna_bf16>(norm[1]), eps, nullptr, xq, s, m, wide, st);
+    if (partial == nullptr || lib.ternaspmm_step_attention_merge(data<float>(partial), splits, data<terna_bf16>(norm[1]), eps, nullptr, xq, s, g.batch, heads,
+                                                                 head_dim, st) != 0) {
+        if (partial != nullptr) lib.ternaspmm_attention_merge(data<float>(partial), splits, o, g.batch, heads, head_dim, st);
+        lib.ternaspmm_rmsnorm_quant(o, nullptr, nullptr, data<terna_bf16>(norm[1]), eps, nullptr, xq, s, m, wide, st);
+    }
     if (add_linear(o_w, wide, in, data<terna_bf16>(&mid))) {
         lib.ternaspmm_rmsnorm_quant(data<terna_bf16>(&mid), nullptr, nullptr, data<terna_bf16>(norm[2]), eps, nullptr, xq, s, m, dim, st);
     } else {
@@ -692,10 +716,8 @@ TERNA_FUNCTION(block, 35)
     return pack(unlocked, std::move(mid), std::move(out));
 }
 
-// (partial, splits, heads, head_dim, norm_weight, eps, sequences, want_output) -> (xq, s, o | None), or None
-TERNA_FUNCTION(attention_merge_rmsnorm_quant, 8)
+PyObject* merge_norm_quant(const char* who, decltype(lib.ternaspmm_step_attention_merge) merge, PyObject* const* a)
 {
-    const char* who = "attention_merge_rmsnorm_quant";
     const at::Tensor &partial = tensor(a[0]), &weight = tensor(a[4]);
     const int splits = integer32(a[1]), heads = integer32(a[2]), head_dim = integer32(a[3]), sequences = integer32(a[6]);
     const float eps = real(a[5]);
@@ -707,11 +729,16 @@ TERNA_FUNCTION(attention_merge_rmsnorm_quant, 8)
     Unlocked unlocked;
     at::Tensor q = make({sequences, k}, at::kChar, partial), s = make({sequences}, at::kBFloat16, partial), o;
     if (want_output) o = make({sequences, k}, at::kBFloat16, partial);
-    if (lib.ternaspmm_attention_merge_rmsnorm_quant(data<float>(&partial), splits, data<terna_bf16>(&weight), eps, o.defined() ? data<terna_bf16>(&o) : nullptr,
-                                                    data<int8_t>(&q), data<terna_bf16>(&s), sequences, heads, head_dim, stream()) != 0)
+    if (merge(data<float>(&partial), splits, data<terna_bf16>(&weight), eps, o.defined() ? data<terna_bf16>(&o) : nullptr, data<int8_t>(&q), data<terna_bf16>(&s),
+              sequences, heads, head_dim, stream()) != 0)
         return none(unlocked);
     return pack(unlocked, std::move(q), std::move(s), std::move(o));
 }
+
+// (partial, splits, heads, head_dim, norm_weight, eps, sequences, want_output) -> (xq, s, o | None), or None
+TERNA_FUNCTION(attention_merge_rmsnorm_quant, 8) { return merge_norm_quant("attention_merge_rmsnorm_quant", lib.ternaspmm_attention_merge_rmsnorm_quant, a); }
+// the same for any split count up to eight
+TERNA_FUNCTION(step_attention_merge, 8) { return merge_norm_quant("step_attention_merge", lib.ternaspmm_step_attention_merge, a); }
 
 // (tokens, pos, embedding, rope_table, norm_weight) -> (x, stats, rope [2, B, half]); tokens / pos contiguous int64 vectors
 TERNA_FUNCTION(step_inputs, 5)
@@ -850,7 +877,7 @@ TERNA_FUNCTION(init, 1)
 PyMethodDef methods[] = {METHOD(init), METHOD(bit_linear), METHOD(bit_linear_bf16), METHOD(quant_input), METHOD(linear_packed),
                          METHOD(linear_bf16_packed), METHOD(rmsnorm_quant), METHOD(relu2_mul_rmsnorm_quant), METHOD(quant_from_stats),
                          METHOD(fused_linear), METHOD(prompt_attention), METHOD(decode_attention), METHOD(block),
-                         METHOD(attention_merge_rmsnorm_quant), METHOD(step_inputs), METHOD(prompt_inputs), METHOD(decode_step), {nullptr, nullptr, 0, nullptr}};
+                         METHOD(attention_merge_rmsnorm_quant), METHOD(step_attention_merge), METHOD(step_inputs), METHOD(prompt_inputs), METHOD(decode_step), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

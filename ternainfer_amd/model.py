@@ -22,7 +22,7 @@ import torch
 from torch.nn import functional as F
 
 from . import _lib
-from .linear import (EPILOGUE_GATE, EPILOGUE_RESIDUAL, argmax_rows, attention_merge_rmsnorm_linear_packed, attention_merge_rmsnorm_quant, fused_linear, get_global_workspace, greedy_step,
+from .linear import (EPILOGUE_GATE, EPILOGUE_RESIDUAL, argmax_rows, attention_merge_rmsnorm_linear_packed, fused_linear, get_global_workspace, greedy_step,
                      greedy_step_state, interleave_gate_up, lm_head, prompt_inputs, quant_from_stats, quant_input, row_stats, relu2_mul_rmsnorm_linear_packed, relu2_mul_rmsnorm_quant, step_inputs,
                      repack_weight, rmsnorm_linear_packed, rmsnorm_quant)
 
@@ -253,7 +253,7 @@ class Block:
             # (weights of the next launches through the caches meanwhile: only next to a short attention -- with caches of
             # 1528 slots the prefetch cost 2 % of the step, at 728 slots it gains 0.5 %)
             if split and self.prefetch is not None and cache_k.shape[2] <= 1024:
-                lib.ternaspmm_rope_decode_attention_partial(
+                lib.ternaspmm_step_attention(
                     _p(qkv), _p(cos), _p(sin), _p(pos_idx), per_seq, _p(cache_k), _p(cache_v), _p(partial), splits, bsz, a.n_heads,
                     a.n_kv_heads, a.head_dim, cache_k.shape[2], a.head_dim ** -0.5, int(a.rope_adjacent), *self.prefetch, stream)
             else:
@@ -261,7 +261,7 @@ class Block:
             r = None
             if split or (bsz > 1 and self.merge_quant):
                 # merge + sub-norm + quantisation once per sequence, then the O projection on the quantised rows
-                mq = attention_merge_rmsnorm_quant(partial, splits, a.n_heads, a.head_dim, self.attn_sub_norm, a.norm_eps, bsz, want_output=pub)
+                mq = native.step_attention_merge(partial, splits, a.n_heads, a.head_dim, self.attn_sub_norm, a.norm_eps, bsz, pub)
                 if mq is not None:
                     if pub:
                         cap.append(("attention", None, None, mq[2]))
@@ -343,7 +343,7 @@ class Block:
         one_token = mask is None           # the caller's rule: fused, one new token, a head size the kernel has
         # more rows than _norm_linear's one-launch forms take: the launches of the block as one native call
         if x.shape[0] > 8 and self.fused and self.act == "int8" and self.capture is None and \
-                (mask is KERNEL_ATTENTION or (one_token and self.prefetch is None and not isinstance(attn_ws, tuple))):
+                (mask is KERNEL_ATTENTION or (one_token and self.prefetch is None)):
             wqkv, wo, w13, w2 = self.wqkv, self.wo, self.w13, self.w2
             return _lib.native().block(
                 x, pending, cos, sin, pos_idx, cache_k, cache_v, a.n_heads, a.head_dim, a.head_dim ** -0.5, int(a.rope_adjacent), a.norm_eps,
@@ -535,7 +535,7 @@ class Transformer:
             return None
         a = self.args
         lib = _lib.load()
-        splits = getattr(self, "attention_splits", None) or lib.ternaspmm_attention_partial_splits_kv(bsz, a.n_heads, a.n_kv_heads, max_seq)
+        splits = getattr(self, "attention_splits", None) or lib.ternaspmm_step_attention_splits(bsz, a.n_heads, a.n_kv_heads, max_seq)
         if splits < 1 or (splits == 1 and not single_split):
             return None
         # one buffer per batch size, kept while the model lives: a captured decode graph holds the raw pointer
@@ -634,7 +634,10 @@ class Transformer:
         # (in the split chain that merge launch also norms and quantises the O projection's input; with short caches
         # the unsplit launch + the O projection with the norm inside stay ahead there too: 8 sequences, slot 255 of 384,
         # 1.198 against 1.218 ms per step -- `split_merge_quant` forces the split form)
-        if one_launch_attention and self.layers[0].act == "int8" and (bsz == 1 or max_seq > (512 if split else self.defer_above)):
+        # With more heads than CUs already from 256 slots on (14 sequences, 384 slots: 1303 -> 1217 us a step; 20, 512: 1607 -> 1500; at 256 slots
+        # level), where the chip holds two splits of every kv head and more.
+        short = 256 if bsz * a.n_heads > 256 else 512 if split else self.defer_above
+        if one_launch_attention and self.layers[0].act == "int8" and (bsz == 1 or max_seq > short):
             attn_ws = self.attention_partial(bsz, max_seq) or attn_ws
         elif split and getattr(self, "split_merge_quant", False):
             attn_ws = self.attention_partial(bsz, max_seq, single_split=True) or attn_ws

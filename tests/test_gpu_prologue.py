@@ -901,6 +901,57 @@ def test_rope_decode_attention_partial_and_merge(lib, b, h, kv, d, s_max, n, spl
     assert torch.equal(o2, o3) and torch.equal(ck2, ck3) and torch.equal(cv2, cv3)
 
 
+# The one-workgroup-per-kv-head kernel over the edges of its tiles (16 slots), of its rounds (8 waves: 128 slots of keys and of values; 4 waves:
+# 128 and 128) and of its split counts: splits 0 = ternaspmm_rope_decode_attention, which takes it from 513 heads on.
+_EDGE_LENS = (1, 16, 17, 127, 128, 129, 256, 257, 300)
+
+
+@pytest.mark.parametrize("b,h,kv,d,s_max,splits,adjacent", [
+    (9, 20, 5, 128, 300, 3, 1), (9, 8, 4, 128, 301, 5, 0), (9, 16, 4, 64, 300, 6, 0), (9, 8, 4, 64, 304, 7, 1), (30, 20, 5, 128, 300, 2, 1),
+    (27, 20, 5, 128, 300, 0, 1), (60, 20, 5, 128, 300, 0, 0), (35, 16, 8, 128, 303, 0, 1), (36, 16, 4, 64, 300, 0, 1), (72, 8, 4, 64, 300, 0, 0)])
+def test_attention_of_a_kv_group_against_the_oracle(lib, b, h, kv, d, s_max, splits, adjacent):
+    """The tolerance: the output is one bf16 rounding (2^-9 of it) away from float32 sums over probabilities whose scores carry the bf16
+    products' float32 rounding; 2^-7 of the head's largest output, as for the other attention kernels."""
+    lens = [_EDGE_LENS[i % len(_EDGE_LENS)] for i in range(b)]
+    qkv = make_bf16_activations(b, (h + 2 * kv) * d, 1851 + b)
+    k0 = make_bf16_activations(b * kv * s_max, d, 1852 + b).reshape(b, kv, s_max, d)
+    v0 = make_bf16_activations(b * kv * s_max, d, 1853 + b, outlier_frac=0.01).reshape(b, kv, s_max, d)
+    pos = np.array(lens, np.int64) - 1
+    for i, n in enumerate(lens):                                     # slots past a prefix hold anything
+        k0[i, :, n:], v0[i, :, n:] = 0x7FC0, 0x7F80
+    cos, sin = _angles(pos, d)
+    xd, cd, sd, pd, ck, cv = _dev(qkv), _dev(cos), _dev(sin), _dev(pos), _dev(k0), _dev(v0)
+    out = torch.zeros((b, h * d), dtype=torch.int16, device="cuda")
+    print(f"[case] attention of a kv group b={b} h={h} kv={kv} d={d} S={s_max} splits={splits} adjacent={adjacent}", flush=True)
+    rotate = O.rope_adjacent if adjacent else O.rope_rotate_half
+    if splits:
+        part = _partial_buffer(lib, b, h, d)
+        assert lib.ternaspmm_step_attention(_vp(xd), _vp(cd), _vp(sd), _vp(pd), 1, _vp(ck), _vp(cv), _vp(part), splits,
+                                            b, h, kv, d, s_max, float(d) ** -0.5, adjacent, None, None, None, 0, None) == 0
+        lib.ternaspmm_attention_merge(_vp(part), splits, _vp(out), b, h, d, None)
+        if h * d <= 4096:                                            # the merge with norm and quantisation behind it, at every split count
+            norm_w, merged = _dev(_weight(h * d, 1854)), torch.zeros_like(out)
+            xq, s = torch.zeros((2, b, h * d), dtype=torch.int8, device="cuda"), torch.zeros((2, b), dtype=torch.int16, device="cuda")
+            assert lib.ternaspmm_step_attention_merge(_vp(part), splits, _vp(norm_w), 1e-5, _vp(merged), _vp(xq[0]), _vp(s[0]), b, h, d, None) == 0
+            lib.ternaspmm_rmsnorm_quant(_vp(out), None, None, _vp(norm_w), 1e-5, None, _vp(xq[1]), _vp(s[1]), b, h * d, None)
+            assert torch.equal(merged, out) and torch.equal(xq[0], xq[1]) and torch.equal(s[0], s[1])
+    else:
+        lib.ternaspmm_rope_decode_attention(_vp(xd), _vp(cd), _vp(sd), _vp(pd), 1, _vp(ck), _vp(cv), _vp(out), b, h, kv, d, s_max,
+                                            float(d) ** -0.5, adjacent, None, None)
+    torch.cuda.synchronize()
+    got = O.bf16_bits_to_f32(out.cpu().numpy().view(np.uint16)).reshape(b, h, d).astype(np.float64)
+    kc, vc = ck.cpu().numpy().view(np.uint16), cv.cpu().numpy().view(np.uint16)
+    x = qkv.reshape(b, h + 2 * kv, d)
+    for i in range(b):
+        c, sn = cos[i][None, None], sin[i][None, None]
+        assert (kc[i][:, pos[i]] == rotate(x[i:i + 1, h:h + kv], c, sn)[0]).all() and (vc[i][:, pos[i]] == x[i, h + kv:]).all()
+        untouched = np.setdiff1d(np.arange(s_max), pos[i])
+        assert (kc[i][:, untouched] == k0[i][:, untouched]).all() and (vc[i][:, untouched] == v0[i][:, untouched]).all()
+        want = O.attention_one_token(rotate(x[i:i + 1, :h], c, sn), kc[i:i + 1], vc[i:i + 1], lens[i], float(d) ** -0.5)[0]
+        tol = 2.0 ** -7 * np.abs(want).max(axis=-1, keepdims=True) + 1e-6
+        assert (np.abs(got[i] - want) <= tol).all(), (i, float((np.abs(got[i] - want) / tol).max()))
+
+
 def test_attention_partial_against_the_oracle(lib):
     """Every sequence against attention_one_token at its own length, 8 splits over a 2B-shaped cache."""
     b, h, kv, d, s_max, lens = 2, 20, 5, 128, 1024, (1000, 333)
