@@ -547,9 +547,23 @@ void ternaspmm_attention_merge(const float* partial, int splits, terna_bf16* out
  * returns 0, or -1 for anything else (nothing enqueued). */
 int ternaspmm_attention_merge_rmsnorm_quant(const float* partial, int splits, const terna_bf16* norm_weight, float eps, terna_bf16* o_out,
                                             int8_t* xq_out, terna_bf16* s_out, int B, int H, int D, terna_stream stream);
+/* The launches that norm and quantise the rows of an int8 linear, with the weights of that linear fetched into the caches by workgroups
+ * they have to spare (no counterpart in the reference): the entries without `_ahead`, and their results.  next (may be NULL):
+ * packed weights [N][K] that the next launch of the stream reads with the rows of this one; gate != 0: a gate+up matrix in the
+ * interleaved band order. */
+typedef struct ternaspmm_next_linear {
+    const void* packed;
+    int N, K, gate;
+} ternaspmm_next_linear;
+void ternaspmm_rmsnorm_quant_ahead(const terna_bf16* x, const terna_bf16* residual, terna_bf16* sum_out,
+                                   const terna_bf16* weight, float eps, terna_bf16* y_out, int8_t* xq_out,
+                                   terna_bf16* s_out, int M, int K, const ternaspmm_next_linear* next, terna_stream stream);
+void ternaspmm_relu2_mul_rmsnorm_quant_ahead(const terna_bf16* x13, const terna_bf16* weight, float eps, terna_bf16* y_out,
+                                             int8_t* xq_out, terna_bf16* s_out, int M, int F, const ternaspmm_next_linear* next, terna_stream stream);
+
 /* The pair for any split count from 1 to 8, as a decode step of several sequences launches it: ternaspmm_step_attention is
  * ternaspmm_rope_decode_attention_partial, ternaspmm_step_attention_merge is ternaspmm_attention_merge_rmsnorm_quant;
- * both return 0, or -1 with nothing enqueued.  ternaspmm_step_attention_splits(B, H, KV, S): the count that fills the chip
+ * both return 0, or -1 with nothing enqueued (next: as above).  ternaspmm_step_attention_splits(B, H, KV, S): the count that fills the chip
  * (one sequence, or other than 2 or 4 heads per kv head: ternaspmm_attention_partial_splits_kv). */
 int ternaspmm_step_attention_splits(int B, int H, int KV, int S);
 int ternaspmm_step_attention(const terna_bf16* qkv, const float* cos, const float* sin, const long long* pos, int per_sequence,
@@ -557,7 +571,7 @@ int ternaspmm_step_attention(const terna_bf16* qkv, const float* cos, const floa
                              float scale, int adjacent, const void* const* pf_ptr, const long long* pf_bytes, const long long* pf_unit_bytes,
                              int pf_count, terna_stream stream);
 int ternaspmm_step_attention_merge(const float* partial, int splits, const terna_bf16* norm_weight, float eps, terna_bf16* o_out,
-                                   int8_t* xq_out, terna_bf16* s_out, int B, int H, int D, terna_stream stream);
+                                   int8_t* xq_out, terna_bf16* s_out, int B, int H, int D, const ternaspmm_next_linear* next, terna_stream stream);
 
 /* The bookkeeping of one greedy decode step in one launch (generate.py:283-305: argmax, tokens[:, pos] = next_token,
  * the position counters): tok[b] = argmax(logits[b]) as above; if history != NULL and counters[1] < history_len,

@@ -41,7 +41,9 @@ PROTOTYPES = {
     "bitlinear_TernaSpMM_bf16_packed_ws": ([_vp, _vp, _vp, _vp, _ci, _ci, _ci, _ci, _ci, _vp, ctypes.c_longlong, _vp], None),
     "bitlinear_TernaSpMM_packed_ws": ([_vp, _vp, _vp, _vp, _vp, _ci, _ci, _ci, _ci, _ci, _vp, ctypes.c_longlong, _vp], None),
     "ternaspmm_rmsnorm_quant": ([_vp, _vp, _vp, _vp, ctypes.c_float, _vp, _vp, _vp, _ci, _ci, _vp], None),
+    "ternaspmm_rmsnorm_quant_ahead": ([_vp, _vp, _vp, _vp, ctypes.c_float, _vp, _vp, _vp, _ci, _ci, _vp, _vp], None),
     "ternaspmm_relu2_mul_rmsnorm_quant": ([_vp, _vp, ctypes.c_float, _vp, _vp, _vp, _ci, _ci, _vp], None),
+    "ternaspmm_relu2_mul_rmsnorm_quant_ahead": ([_vp, _vp, ctypes.c_float, _vp, _vp, _vp, _ci, _ci, _vp, _vp], None),
     "bitlinear_TernaSpMM_packed_fused": ([_vp, _vp, _vp, _vp, ctypes.c_float, _vp, _vp, _vp, _ci, _vp, _vp, _ci, _ci, _ci, _vp],
                                          ctypes.c_int),
     "bitlinear_TernaSpMM_packed_fused_attn": ([_vp, _ci, _ci, _vp, ctypes.c_float, _vp, _vp, _vp, _ci, _vp, _vp, _ci, _ci, _ci, _vp],
@@ -61,7 +63,7 @@ PROTOTYPES = {
     "ternaspmm_attention_merge": ([_vp, _ci, _vp, _ci, _ci, _ci, _vp], None),
     "ternaspmm_attention_merge_rmsnorm_quant": ([_vp, _ci, _vp, ctypes.c_float, _vp, _vp, _vp, _ci, _ci, _ci, _vp], ctypes.c_int),
     "ternaspmm_step_attention": ([_vp] * 4 + [_ci] + [_vp] * 3 + [_ci] * 6 + [ctypes.c_float, _ci, _vp, _vp, _vp, _ci, _vp], ctypes.c_int),
-    "ternaspmm_step_attention_merge": ([_vp, _ci, _vp, ctypes.c_float, _vp, _vp, _vp, _ci, _ci, _ci, _vp], ctypes.c_int),
+    "ternaspmm_step_attention_merge": ([_vp, _ci, _vp, ctypes.c_float, _vp, _vp, _vp, _ci, _ci, _ci, _vp, _vp], ctypes.c_int),
     "ternaspmm_rope_kv_store": ([_vp] * 4 + [_ci] + [_vp] * 3 + [_ci] * 7 + [_vp], None),
     "ternaspmm_rope_decode_attention_stats": ([_vp] * 4 + [_ci] + [_vp] * 3 + [_ci] * 5 + [ctypes.c_float, _ci, _vp, _vp, _vp], ctypes.c_int),
     "ternaspmm_rope_decode_attention": ([_vp] * 4 + [_ci] + [_vp] * 3 + [_ci] * 5 + [ctypes.c_float, _ci, _vp, _vp], None),

@@ -10,6 +10,7 @@
 
 #include "../../include/ternaspmm.h"
 #include "host_util.h"
+#include "launchers.h"
 #include "attention_kernel.h"
 #include "attention_grouped_kernel.h"
 
@@ -541,11 +542,11 @@ int ternaspmm_attention_merge_rmsnorm_quant(const float* partial, int splits, co
                                             int8_t* xq_out, terna_bf16* s_out, int B, int H, int D, terna_stream stream)
 {
     if (splits < 1 || (splits & (splits - 1))) return -1;
-    return ternaspmm_step_attention_merge(partial, splits, norm_weight, eps, o_out, xq_out, s_out, B, H, D, stream);
+    return ternaspmm_step_attention_merge(partial, splits, norm_weight, eps, o_out, xq_out, s_out, B, H, D, nullptr, stream);
 }
 
 int ternaspmm_step_attention_merge(const float* partial, int splits, const terna_bf16* norm_weight, float eps, terna_bf16* o_out,
-                                   int8_t* xq_out, terna_bf16* s_out, int B, int H, int D, terna_stream stream)
+                                   int8_t* xq_out, terna_bf16* s_out, int B, int H, int D, const ternaspmm_next_linear* next, terna_stream stream)
 {
     const long long K = static_cast<long long>(H) * D;
     if (B < 1 || H < 1 || (D != 64 && D != 128) || splits < 1 || splits > kAttentionMaxSplits || K > 2048 * 2 ||
@@ -553,14 +554,15 @@ int ternaspmm_step_attention_merge(const float* partial, int splits, const terna
         return -1;
     hipStream_t st = static_cast<hipStream_t>(stream);
     const int qmode = quant_mode();
+    const NextWeights ahead = next != nullptr ? next_weights(next->packed, next->N, next->K, next->gate != 0, B) : NextWeights{};
 #define TERNA_MERGE_NQ(DIM, SP)                                                                                           \
     do {                                                                                                                  \
         if (K <= 2048)                                                                                                    \
-            terna_attention_merge_norm_quant_kernel<DIM, SP, 1><<<dim3(B), dim3(kNormThreads), 0, st>>>(                   \
-                partial, norm_weight, H, B * H, eps, o_out, nullptr, xq_out, s_out, qmode);                               \
+            terna_attention_merge_norm_quant_kernel<DIM, SP, 1><<<dim3(B + ahead.workgroups), dim3(kNormThreads), 0, st>>>( \
+                partial, norm_weight, H, B * H, eps, o_out, nullptr, xq_out, s_out, qmode, B, ahead);                     \
         else                                                                                                              \
-            terna_attention_merge_norm_quant_kernel<DIM, SP, 2><<<dim3(B), dim3(kNormThreads), 0, st>>>(                   \
-                partial, norm_weight, H, B * H, eps, o_out, nullptr, xq_out, s_out, qmode);                               \
+            terna_attention_merge_norm_quant_kernel<DIM, SP, 2><<<dim3(B + ahead.workgroups), dim3(kNormThreads), 0, st>>>( \
+                partial, norm_weight, H, B * H, eps, o_out, nullptr, xq_out, s_out, qmode, B, ahead);                     \
     } while (0)
 #define TERNA_MERGE_NQ_D(DIM)                                                                                             \
     do {                                                                                                                  \

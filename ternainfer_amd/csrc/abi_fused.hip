@@ -13,11 +13,25 @@
 
 using namespace terna;
 
+namespace {
+NextWeights next_of(const ternaspmm_next_linear* next, int M)
+{
+    return next != nullptr ? next_weights(next->packed, next->N, next->K, next->gate != 0, M) : NextWeights{};
+}
+}  // namespace
+
 extern "C" {
 
 void ternaspmm_rmsnorm_quant(const terna_bf16* x, const terna_bf16* residual, terna_bf16* sum_out,
                              const terna_bf16* weight, float eps, terna_bf16* y_out, int8_t* xq_out,
                              terna_bf16* s_out, int M, int K, terna_stream stream)
+{
+    ternaspmm_rmsnorm_quant_ahead(x, residual, sum_out, weight, eps, y_out, xq_out, s_out, M, K, nullptr, stream);
+}
+
+void ternaspmm_rmsnorm_quant_ahead(const terna_bf16* x, const terna_bf16* residual, terna_bf16* sum_out,
+                                   const terna_bf16* weight, float eps, terna_bf16* y_out, int8_t* xq_out,
+                                   terna_bf16* s_out, int M, int K, const ternaspmm_next_linear* next, terna_stream stream)
 {
     if (M < 1 || K < 8 || (K & 7) || K > 8 * kNormThreads * kNormMaxVecs || (xq_out != nullptr) != (s_out != nullptr)) {
         std::fprintf(stderr, "ternaspmm_rmsnorm_quant: unsupported arguments (M=%d K=%d)\n", M, K);
@@ -25,10 +39,11 @@ void ternaspmm_rmsnorm_quant(const terna_bf16* x, const terna_bf16* residual, te
     }
     // as many 8-element vectors per thread as the row needs (1, 2 or 4), the residual's loads only where there is one
     const int nv = (K / 8 + kNormThreads - 1) / kNormThreads;
-    const dim3 grid(M), block(kNormThreads);
+    const NextWeights ahead = next_of(next, M);
+    const dim3 grid(M + ahead.workgroups), block(kNormThreads);
     hipStream_t st = static_cast<hipStream_t>(stream);
     const int qm = quant_mode();
-#define TERNA_NORM(NV, SECOND) terna_norm_quant_kernel<false, NV, SECOND><<<grid, block, 0, st>>>(x, residual, weight, K, eps, sum_out, y_out, xq_out, s_out, qm)
+#define TERNA_NORM(NV, SECOND) terna_norm_quant_kernel<false, NV, SECOND><<<grid, block, 0, st>>>(x, residual, weight, K, eps, sum_out, y_out, xq_out, s_out, qm, M, ahead)
     if (residual != nullptr) {
         if (nv <= 1) TERNA_NORM(1, true);
         else if (nv <= 2) TERNA_NORM(2, true);
@@ -46,15 +61,22 @@ void ternaspmm_rmsnorm_quant(const terna_bf16* x, const terna_bf16* residual, te
 void ternaspmm_relu2_mul_rmsnorm_quant(const terna_bf16* x13, const terna_bf16* weight, float eps, terna_bf16* y_out,
                                        int8_t* xq_out, terna_bf16* s_out, int M, int F, terna_stream stream)
 {
+    ternaspmm_relu2_mul_rmsnorm_quant_ahead(x13, weight, eps, y_out, xq_out, s_out, M, F, nullptr, stream);
+}
+
+void ternaspmm_relu2_mul_rmsnorm_quant_ahead(const terna_bf16* x13, const terna_bf16* weight, float eps, terna_bf16* y_out,
+                                             int8_t* xq_out, terna_bf16* s_out, int M, int F, const ternaspmm_next_linear* next, terna_stream stream)
+{
     if (M < 1 || F < 8 || (F & 7) || F > 8 * kNormThreads * kNormMaxVecs || (xq_out != nullptr) != (s_out != nullptr)) {
         std::fprintf(stderr, "ternaspmm_relu2_mul_rmsnorm_quant: unsupported arguments (M=%d F=%d)\n", M, F);
         return;
     }
     const int nv = (F / 8 + kNormThreads - 1) / kNormThreads;
-    const dim3 grid(M), block(kNormThreads);
+    const NextWeights ahead = next_of(next, M);
+    const dim3 grid(M + ahead.workgroups), block(kNormThreads);
     hipStream_t st = static_cast<hipStream_t>(stream);
     const int qm = quant_mode();
-#define TERNA_NORM(NV) terna_norm_quant_kernel<true, NV, true><<<grid, block, 0, st>>>(x13, nullptr, weight, F, eps, nullptr, y_out, xq_out, s_out, qm)
+#define TERNA_NORM(NV) terna_norm_quant_kernel<true, NV, true><<<grid, block, 0, st>>>(x13, nullptr, weight, F, eps, nullptr, y_out, xq_out, s_out, qm, M, ahead)
     if (nv <= 1) TERNA_NORM(1);
     else if (nv <= 2) TERNA_NORM(2);
     else TERNA_NORM(4);

@@ -175,8 +175,13 @@ __global__ __launch_bounds__(D) void terna_attention_merge_kernel(const float* _
 template <int D, int SP, int NV>
 __global__ __launch_bounds__(kNormThreads) void terna_attention_merge_norm_quant_kernel(
     const float* __restrict__ partial, const uint16_t* __restrict__ weight, int H, int heads_total, float eps,
-    uint16_t* __restrict__ o_out, uint16_t* __restrict__ y_out, int8_t* __restrict__ xq_out, uint16_t* __restrict__ s_out, int quant_mode)
+    uint16_t* __restrict__ o_out, uint16_t* __restrict__ y_out, int8_t* __restrict__ xq_out, uint16_t* __restrict__ s_out, int quant_mode,
+    int rows, NextWeights next)
 {
+    if (static_cast<int>(blockIdx.x) >= rows) {
+        fetch_next_weights(next, rows);
+        return;
+    }
     static_assert(D % 8 == 0 && SP >= 1 && SP <= kAttentionMaxSplits && kAttentionMaxSplits == 8, "a vector lies inside one head");
     const int tid = threadIdx.x;
     const size_t row = blockIdx.x;

@@ -103,6 +103,24 @@ void launch_mid_residual(const int8_t* x, const uint32_t* packed, uint16_t* out,
     launch_mid_tile<int8_t, PACKED_RESIDUAL>(x, packed, out, ep, M, N, K, st, &stream);
 }
 
+// Up to 2048 rows (a launch of 4000 has no spare moments: 11361 against 11380 us a prompt), and up to half of every L2 (4 MiB an XCD).
+NextWeights next_weights(const void* packed, int N, int K, bool gate, int M)
+{
+    NextWeights next{};
+    const long bytes = static_cast<long>(N) * K / 4;
+    if (packed == nullptr || N < 64 || K < 64 || (N & 63) || (K & 63) || M > 2048 || bytes > (16l << 20)) return next;
+    int bands;                                           // of one workgroup of the launch that will run
+    if (M <= 16) bands = gate || N / 16 > 256 ? 4 : 1;
+    else if (mid_kernel_takes(nullptr, M, N, K, 1)) bands = choose_tile(M, N, K, 1).fb;
+    else bands = plan_prefill_packed<int8_t>(nullptr, M, N, K, nullptr, 0).bn / 16;
+    next.base = static_cast<const uint8_t*>(packed);
+    next.lines = static_cast<uint32_t>(bytes / 128);
+    next.tile_lines = static_cast<uint32_t>(bands * K / 32);
+    next.workgroups = static_cast<int>(next.lines / 256 + 7) / 8 * 8;
+    if (next.workgroups > 192) next.workgroups = 192;
+    return next;
+}
+
 template void launch_mid<int8_t>(const int8_t*, const uint32_t*, uint16_t*, const Epilogue&, int, int, int, hipStream_t, const RepackGuard*);
 template void launch_mid<uint16_t>(const uint16_t*, const uint32_t*, uint16_t*, const Epilogue&, int, int, int, hipStream_t, const RepackGuard*);
 

@@ -46,6 +46,9 @@ bool mid_kernel_takes(const void* x, int M, int N, int K, size_t act_bytes);
 template <typename Act>
 void launch_mid(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, hipStream_t st,
                 const RepackGuard* guard = nullptr);
+// For a launch that quantises the M rows of an int8 linear on `packed` (NULL: none) (gate: the interleaved gate+up matrix): what its
+// spare workgroups fetch.
+NextWeights next_weights(const void* packed, int N, int K, bool gate, int M);
 // The gate+up matrix with its gate (bands of w1 and w3 interleaved, int8 activations, out [M][N / 2]): the kernels of more than 16 rows.
 void launch_mid_gate(const int8_t* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, hipStream_t st);
 bool launch_prefill_gate(const int8_t* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, hipStream_t st);

@@ -13,7 +13,7 @@
 //        which of the reference's ways of evaluating these two lines is reproduced: QuantMode in terna_common.h)
 //
 // The row stays in registers between the three passes; HBM sees each input element once and each
-// output element once.  Rows are independent, so the grid is M workgroups of 256 threads.
+// output element once.  Rows are independent, so the grid is M workgroups of 256 threads (and those of fetch_next_weights).
 #pragma once
 
 #include "terna_common.h"
@@ -184,6 +184,32 @@ __device__ __forceinline__ void norm_quant_passes(float (&h)[NV][8], const u32x4
     quant_pass<NV>(h, amax, K, row, xq_out, s_out, quant_mode);
 }
 
+// Spare workgroups of a launch that norms and quantises rows bring the packed weights of the linear behind it into the L2s while its few
+// workgroups wait for memory and each other: the linear then starts on data that is one L2 trip away instead of one to HBM (a model's
+// weights are read once per pass and twice the size of the last cache).  A load of four bytes fetches a line; nobody waits for it but
+// the end of the launch.  Measured, us, without -> with: decode step of 32 sequences x 512 slots 1540 -> 1494, of 64 1815 -> 1735, prompts of 100, 300,
+// 1000 and 1920 tokens 1616 -> 1575, 2324 -> 2225, 4307 -> 4195, 6549 -> 6434; 8 sequences x 1528 slots, in the launch that also merges
+// the attention's splits, 1249 -> 1243.  Tried: weights of the launch after next as well, or instead (32 sequences 1505 - 1531), 64 workgroups
+// (1525) and 384 (1508); in the shorter launch that quantises from a producer's statistics (up to 16 rows) it costs 5 - 20 us
+// a step, in the quantisation in front of a linear module's call it is level.
+__device__ __forceinline__ void fetch_next_weights(const NextWeights& next, int first)
+{
+    const uint32_t xcd = blockIdx.x & 7, per_xcd = next.workgroups >> 3;
+    const uint32_t rank = (blockIdx.x - first - ((xcd - (first & 7) + 8) & 7)) >> 3;    // among the fetching workgroups of this XCD
+    const uint32_t step = per_xcd * blockDim.x;
+    const __amdgpu_buffer_rsrc_t lines = make_raw_buffer(next.base, next.lines << 7);      // a load past them fetches nothing
+    auto line_of = [&](uint32_t g) {                     // of this XCD's lines, tile by tile: ascending
+        const uint32_t tile = g / next.tile_lines;
+        return (8 * tile + xcd) * next.tile_lines + (g - tile * next.tile_lines);
+    };
+    for (uint32_t g = rank * blockDim.x + threadIdx.x; line_of(g) < next.lines; g += 4 * step) {
+        uint32_t d[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) d[j] = __builtin_amdgcn_raw_buffer_load_b32(lines, line_of(g + j * step) << 7, 0, 0);
+        asm volatile("" ::"v"(d[0]), "v"(d[1]), "v"(d[2]), "v"(d[3]));
+    }
+}
+
 // GLU = false: x [M][K], optional residual [M][K] and sum_out [M][K].
 // GLU = true : x [M][2K] holding x1 | x3; residual / sum_out unused.
 // NV = 8-element vectors per thread (K <= 2048 NV); SECOND = there is a second operand (the residual, or x3).
@@ -191,9 +217,13 @@ template <bool GLU, int NV = kNormMaxVecs, bool SECOND = true>
 __global__ __launch_bounds__(kNormThreads) void terna_norm_quant_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ residual, const uint16_t* __restrict__ weight, int K,
     float eps, uint16_t* __restrict__ sum_out, uint16_t* __restrict__ y_out, int8_t* __restrict__ xq_out,
-    uint16_t* __restrict__ s_out, int quant_mode)
+    uint16_t* __restrict__ s_out, int quant_mode, int rows, NextWeights next)
 {
     static_assert(!GLU || SECOND, "the gate has two operands");
+    if (static_cast<int>(blockIdx.x) >= rows) {
+        fetch_next_weights(next, rows);
+        return;
+    }
     const int tid = threadIdx.x;
     const size_t row = blockIdx.x;
     const int nvec = K >> 3;

@@ -39,7 +39,9 @@ namespace {
     X(ternaspmm_residual_linear)                                                                                       \
     X(ternaspmm_quant_input)                                                                                           \
     X(ternaspmm_rmsnorm_quant)                                                                                         \
+    X(ternaspmm_rmsnorm_quant_ahead)                                                                                   \
     X(ternaspmm_relu2_mul_rmsnorm_quant)                                                                               \
+    X(ternaspmm_relu2_mul_rmsnorm_quant_ahead)                                                                         \
     X(ternaspmm_fused_linear)                                                                                          \
     X(ternaspmm_quant_from_stats)                                                                                      \
     X(ternaspmm_rope_kv_store)                                                                                         \
@@ -657,6 +659,10 @@ TERNA_FUNCTION(block, 35)
 
     at::Tensor mid = make({m, dim}, at::kBFloat16, x), out = make({m, dim}, at::kBFloat16, x), first;
     if (pending != nullptr) first = make({m, dim}, at::kBFloat16, x);
+    const auto next = [](const BlockLinear& w, int64_t k) { return ternaspmm_next_linear{data(&w.packed), static_cast<int>(w.n), static_cast<int>(k), 0}; };
+    const ternaspmm_next_linear next_qkv = next(qkv_w, dim), next_o = next(o_w, wide), next_down = next(down_w, ffn);
+    ternaspmm_next_linear next_gate = next(gate_w, dim);
+    if (interleaved != nullptr) next_gate.packed = data(interleaved), next_gate.gate = 1;
     const terna_bf16* in = data<terna_bf16>(&x);
     const terna_stream st = stream();
     terna_bf16 *ck = data<terna_bf16>(&g.ck), *cv = data<terna_bf16>(&g.cv);
@@ -664,8 +670,8 @@ TERNA_FUNCTION(block, 35)
         lib.bitlinear_TernaSpMM_packed_ws(xq, data(&w.packed), to, s, data<terna_bf16>(&w.ws), w.ws_num, m, w.n, k, 0, data(work),
                                           work != nullptr ? work->numel() : 0, st);
     };
-    lib.ternaspmm_rmsnorm_quant(in, data<terna_bf16>(pending), pending != nullptr ? data<terna_bf16>(&first) : nullptr, data<terna_bf16>(norm[0]), eps, nullptr,
-                                xq, s, m, dim, st);
+    lib.ternaspmm_rmsnorm_quant_ahead(in, data<terna_bf16>(pending), pending != nullptr ? data<terna_bf16>(&first) : nullptr, data<terna_bf16>(norm[0]), eps, nullptr,
+                                      xq, s, m, dim, &next_qkv, st);
     if (pending != nullptr) in = data<terna_bf16>(&first);
     // RoPE and the cache write in the projection's epilogue, for the attention that reads its rows
     const bool rows_in_place =
@@ -695,28 +701,40 @@ TERNA_FUNCTION(block, 35)
                                              work != nullptr ? work->numel() : 0, st) == 1;
     };
     if (partial == nullptr || lib.ternaspmm_step_attention_merge(data<float>(partial), splits, data<terna_bf16>(norm[1]), eps, nullptr, xq, s, g.batch, heads,
-                                                                 head_dim, st) != 0) {
+                                                                 head_dim, &next_o, st) != 0) {
         if (partial != nullptr) lib.ternaspmm_attention_merge(data<float>(partial), splits, o, g.batch, heads, head_dim, st);
-        lib.ternaspmm_rmsnorm_quant(o, nullptr, nullptr, data<terna_bf16>(norm[1]), eps, nullptr, xq, s, m, wide, st);
+        lib.ternaspmm_rmsnorm_quant_ahead(o, nullptr, nullptr, data<terna_bf16>(norm[1]), eps, nullptr, xq, s, m, wide, &next_o, st);
     }
     if (add_linear(o_w, wide, in, data<terna_bf16>(&mid))) {
-        lib.ternaspmm_rmsnorm_quant(data<terna_bf16>(&mid), nullptr, nullptr, data<terna_bf16>(norm[2]), eps, nullptr, xq, s, m, dim, st);
+        lib.ternaspmm_rmsnorm_quant_ahead(data<terna_bf16>(&mid), nullptr, nullptr, data<terna_bf16>(norm[2]), eps, nullptr, xq, s, m, dim, &next_gate, st);
     } else {
         linear(o_w, wide, attn);
-        lib.ternaspmm_rmsnorm_quant(in, attn, data<terna_bf16>(&mid), data<terna_bf16>(norm[2]), eps, nullptr, xq, s, m, dim, st);
+        lib.ternaspmm_rmsnorm_quant_ahead(in, attn, data<terna_bf16>(&mid), data<terna_bf16>(norm[2]), eps, nullptr, xq, s, m, dim, &next_gate, st);
     }
     if (interleaved != nullptr && lib.ternaspmm_gate_linear(xq, data(interleaved), x13, s, data<terna_bf16>(&gate_w.ws), gate_w.ws_num, m, gate_w.n, dim, st)) {
-        lib.ternaspmm_rmsnorm_quant(x13, nullptr, nullptr, data<terna_bf16>(norm[3]), eps, nullptr, xq, s, m, ffn, st);
+        lib.ternaspmm_rmsnorm_quant_ahead(x13, nullptr, nullptr, data<terna_bf16>(norm[3]), eps, nullptr, xq, s, m, ffn, &next_down, st);
     } else {
         linear(gate_w, dim, x13);
-        lib.ternaspmm_relu2_mul_rmsnorm_quant(x13, data<terna_bf16>(norm[3]), eps, nullptr, xq, s, m, ffn, st);
+        lib.ternaspmm_relu2_mul_rmsnorm_quant_ahead(x13, data<terna_bf16>(norm[3]), eps, nullptr, xq, s, m, ffn, &next_down, st);
     }
     if (add_linear(down_w, ffn, data<terna_bf16>(&mid), data<terna_bf16>(&out))) return pack(unlocked, std::move(out), at::Tensor());
     linear(down_w, ffn, data<terna_bf16>(&out));
     return pack(unlocked, std::move(mid), std::move(out));
 }
 
-PyObject* merge_norm_quant(const char* who, decltype(lib.ternaspmm_step_attention_merge) merge, PyObject* const* a)
+// (packed, out_features, in_features, gate) | None: the linear behind a launch
+ternaspmm_next_linear next_linear(const char* who, PyObject* o)
+{
+    if (o == Py_None) return ternaspmm_next_linear{};
+    if (!PyTuple_Check(o) || PyTuple_GET_SIZE(o) != 4) refuse("%s: the next linear is (packed, out_features, in_features, gate)", who);
+    const at::Tensor& packed = tensor(PyTuple_GET_ITEM(o, 0));
+    const int n = integer32(PyTuple_GET_ITEM(o, 1)), k = integer32(PyTuple_GET_ITEM(o, 2));
+    if (n < 1 || k < 1 || static_cast<int64_t>(packed.numel() * packed.element_size()) < static_cast<int64_t>(n) * k / 4)
+        refuse("%s: the next linear's weight is too small", who);
+    return ternaspmm_next_linear{data(&packed), n, k, PyObject_IsTrue(PyTuple_GET_ITEM(o, 3))};
+}
+
+PyObject* merge_norm_quant(const char* who, bool any_splits, const ternaspmm_next_linear& next, PyObject* const* a)
 {
     const at::Tensor &partial = tensor(a[0]), &weight = tensor(a[4]);
     const int splits = integer32(a[1]), heads = integer32(a[2]), head_dim = integer32(a[3]), sequences = integer32(a[6]);
@@ -729,16 +747,19 @@ PyObject* merge_norm_quant(const char* who, decltype(lib.ternaspmm_step_attentio
     Unlocked unlocked;
     at::Tensor q = make({sequences, k}, at::kChar, partial), s = make({sequences}, at::kBFloat16, partial), o;
     if (want_output) o = make({sequences, k}, at::kBFloat16, partial);
-    if (merge(data<float>(&partial), splits, data<terna_bf16>(&weight), eps, o.defined() ? data<terna_bf16>(&o) : nullptr, data<int8_t>(&q), data<terna_bf16>(&s),
-              sequences, heads, head_dim, stream()) != 0)
+    terna_bf16* const o_out = o.defined() ? data<terna_bf16>(&o) : nullptr;
+    if ((any_splits ? lib.ternaspmm_step_attention_merge(data<float>(&partial), splits, data<terna_bf16>(&weight), eps, o_out, data<int8_t>(&q), data<terna_bf16>(&s),
+                                                         sequences, heads, head_dim, &next, stream())
+                    : lib.ternaspmm_attention_merge_rmsnorm_quant(data<float>(&partial), splits, data<terna_bf16>(&weight), eps, o_out, data<int8_t>(&q),
+                                                                  data<terna_bf16>(&s), sequences, heads, head_dim, stream())) != 0)
         return none(unlocked);
     return pack(unlocked, std::move(q), std::move(s), std::move(o));
 }
 
 // (partial, splits, heads, head_dim, norm_weight, eps, sequences, want_output) -> (xq, s, o | None), or None
-TERNA_FUNCTION(attention_merge_rmsnorm_quant, 8) { return merge_norm_quant("attention_merge_rmsnorm_quant", lib.ternaspmm_attention_merge_rmsnorm_quant, a); }
-// the same for any split count up to eight
-TERNA_FUNCTION(step_attention_merge, 8) { return merge_norm_quant("step_attention_merge", lib.ternaspmm_step_attention_merge, a); }
+TERNA_FUNCTION(attention_merge_rmsnorm_quant, 8) { return merge_norm_quant("attention_merge_rmsnorm_quant", false, ternaspmm_next_linear{}, a); }
+// (..., next linear | None): the same for any split count up to eight
+TERNA_FUNCTION(step_attention_merge, 9) { return merge_norm_quant("step_attention_merge", true, next_linear("step_attention_merge", a[8]), a); }
 
 // (tokens, pos, embedding, rope_table, norm_weight) -> (x, stats, rope [2, B, half]); tokens / pos contiguous int64 vectors
 TERNA_FUNCTION(step_inputs, 5)

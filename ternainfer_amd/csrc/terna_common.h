@@ -460,4 +460,11 @@ struct RopeStore {
     }
 };
 
+// The packed weights that the next launch reads (fetch_next_weights).
+struct NextWeights {
+    const uint8_t* base;
+    uint32_t lines, tile_lines;   // 128-byte lines of the matrix, and of a workgroup's tile of it: tile t is read on XCD t mod 8
+    int workgroups;               // that fetch, a multiple of 8 (0: none)
+};
+
 }  // namespace terna

@@ -261,7 +261,8 @@ class Block:
             r = None
             if split or (bsz > 1 and self.merge_quant):
                 # merge + sub-norm + quantisation once per sequence, then the O projection on the quantised rows
-                mq = native.step_attention_merge(partial, splits, a.n_heads, a.head_dim, self.attn_sub_norm, a.norm_eps, bsz, pub)
+                mq = native.step_attention_merge(partial, splits, a.n_heads, a.head_dim, self.attn_sub_norm, a.norm_eps, bsz, pub,
+                                                 (self.wo.packed, self.wo.n, self.wo.k, False))
                 if mq is not None:
                     if pub:
                         cap.append(("attention", None, None, mq[2]))

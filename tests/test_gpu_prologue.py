@@ -901,6 +901,30 @@ def test_rope_decode_attention_partial_and_merge(lib, b, h, kv, d, s_max, n, spl
     assert torch.equal(o2, o3) and torch.equal(ck2, ck3) and torch.equal(cv2, cv3)
 
 
+class _NextLinear(ctypes.Structure):
+    _fields_ = [("packed", ctypes.c_void_p), ("N", ctypes.c_int), ("K", ctypes.c_int), ("gate", ctypes.c_int)]
+
+
+@pytest.mark.parametrize("m", [1, 9, 17, 100, 2048, 2049])
+@pytest.mark.parametrize("n,k,gate", [(64, 64, 0), (2560, 2560, 0), (13824, 2560, 1), (320, 6912, 0), (32768, 8192, 0)])
+def test_quantising_launches_that_fetch_the_next_weights(lib, m, n, k, gate):
+    """The launches whose spare workgroups load the weights of the linear behind them: the bits of the launches without, for weights of
+    less than a tile on every XCD, of every kernel's tiles, and beyond what is fetched."""
+    print(f"[case] next weights m={m} n={n} k={k}", flush=True)
+    next_linear = _NextLinear(torch.zeros(n * k // 16, dtype=torch.int32, device="cuda").data_ptr(), n, k, gate)
+    x, w = _dev(make_bf16_activations(m, k, 1861 + m)), _dev(_weight(k, 1862))
+    x13 = _dev(make_bf16_activations(m, 2 * k, 1863 + m))
+    xq, s = torch.zeros((2, m, k), dtype=torch.int8, device="cuda"), torch.zeros((2, m), dtype=torch.int16, device="cuda")
+    for plain, ahead in ((lambda q, t: lib.ternaspmm_rmsnorm_quant(_vp(x), None, None, _vp(w), 1e-5, None, _vp(q), _vp(t), m, k, None),
+                          lambda q, t: lib.ternaspmm_rmsnorm_quant_ahead(_vp(x), None, None, _vp(w), 1e-5, None, _vp(q), _vp(t), m, k, ctypes.byref(next_linear), None)),
+                         (lambda q, t: lib.ternaspmm_relu2_mul_rmsnorm_quant(_vp(x13), _vp(w), 1e-5, None, _vp(q), _vp(t), m, k, None),
+                          lambda q, t: lib.ternaspmm_relu2_mul_rmsnorm_quant_ahead(_vp(x13), _vp(w), 1e-5, None, _vp(q), _vp(t), m, k, ctypes.byref(next_linear), None))):
+        xq.zero_(), s.zero_()
+        plain(xq[0], s[0])
+        ahead(xq[1], s[1])
+        assert torch.equal(xq[0], xq[1]) and torch.equal(s[0], s[1]) and bool(xq[0].any())
+
+
 # The one-workgroup-per-kv-head kernel over the edges of its tiles (16 slots), of its rounds (8 waves: 128 slots of keys and of values; 4 waves:
 # 128 and 128) and of its split counts: splits 0 = ternaspmm_rope_decode_attention, which takes it from 513 heads on.
 _EDGE_LENS = (1, 16, 17, 127, 128, 129, 256, 257, 300)
@@ -932,7 +956,7 @@ def test_attention_of_a_kv_group_against_the_oracle(lib, b, h, kv, d, s_max, spl
         if h * d <= 4096:                                            # the merge with norm and quantisation behind it, at every split count
             norm_w, merged = _dev(_weight(h * d, 1854)), torch.zeros_like(out)
             xq, s = torch.zeros((2, b, h * d), dtype=torch.int8, device="cuda"), torch.zeros((2, b), dtype=torch.int16, device="cuda")
-            assert lib.ternaspmm_step_attention_merge(_vp(part), splits, _vp(norm_w), 1e-5, _vp(merged), _vp(xq[0]), _vp(s[0]), b, h, d, None) == 0
+            assert lib.ternaspmm_step_attention_merge(_vp(part), splits, _vp(norm_w), 1e-5, _vp(merged), _vp(xq[0]), _vp(s[0]), b, h, d, None, None) == 0
             lib.ternaspmm_rmsnorm_quant(_vp(out), None, None, _vp(norm_w), 1e-5, None, _vp(xq[1]), _vp(s[1]), b, h * d, None)
             assert torch.equal(merged, out) and torch.equal(xq[0], xq[1]) and torch.equal(s[0], s[1])
     else:
