@@ -369,7 +369,7 @@ int ternaspmm_prompt_inputs(const long long* tokens, const long long* pos, int p
  *   tokens, pos   int64 in device memory, M of them (pos: one for all unless per_sequence); clamped to their tables
  *   x_out    bf16 [M][dim]: the residual stream behind the last block
  * Takes head_dim 128, dim and heads * head_dim up to 2560, ffn up to 7168 (multiples of 64), at most 4096 QKV columns; one sequence: two,
- * four or eight splits of up to 1024 slots; more: splits = 1 and up to 640 slots, not in quant mode 2.
+ * four or eight splits of up to 1024 slots; more: splits = 1 and up to 1024 slots (two: 1280), not in quant mode 2.
  * The workgroups wait for each other, so all of them have to be resident: the call is refused where the device (or the
  * stream's mask of CUs) does not hold four such grids at once -- as many as the runtime's default of four hardware queues runs
  * side by side; GPU_MAX_HW_QUEUES above that raises the bound.  (More than four such steps at once from several processes, or from

@@ -111,7 +111,7 @@ bool step_shape_ok(const ternaspmm_step_desc& d)
     if (d.M == 1) {
         if ((d.splits != 2 && d.splits != 4 && d.splits != 8) || d.slots > d.splits * kStepMaxSplitSlots) return false;
     } else {
-        if (d.splits != 1 || d.slots > kStepMaxSlots) return false;
+        if (d.splits != 1 || d.slots > step_max_slots(d.M)) return false;
     }
     return d.M == 1 || quant_mode() != QUANT_EAGER;          // (the int8 words that are handed over need one value no integer takes)
 }

@@ -9,7 +9,7 @@
 // and no second trip for the data.  A handover alone: 1.44 us from one poll to the next (160 workgroups, 32-byte slices, 5 KB;
 // 256 writers of 20 bytes each, which share lines, 1.95).
 // Measured, us a step of 30 blocks of the 2B shape with the LM head, launches -> this: one sequence, 384 slots 809 -> 643, 4096 slots
-// 1022 -> 837; two, 384 slots 890 -> 725; three, 101 slots 882 -> 798; four, 384 slots 936 -> 855, 640 slots 996 -> 908.
+// 1022 -> 837; two, 384 slots 890 -> 725; three, 101 slots 882 -> 795; four, 384 slots 936 -> 846.
 //
 // Bound: what is left of the handovers (0.7 - 1.3 us each, five or six a block), and behind each wait the instructions of one wave per
 // SIMD, 4 - 8 cycles apiece: 1.6 - 2.7 us a phase.  Hence, in the order of what they gave:
@@ -46,7 +46,12 @@ constexpr int kStepMaxBlocks = 32;               // blocks per launch: their poi
 constexpr int kStepHeadDim = 128;
 constexpr int kStepMaxSplits = 8;                // splits of the cache, one sequence; four at a time are merged
 constexpr int kStepRecord = (kStepHeadDim + 4) * 4;      // bytes a (head, split) hands over: 128 sums, maximum, sum of numerators
-constexpr int kStepMaxSlots = 640, kStepMaxSplitSlots = 1024;    // of a cache that is not split; of a split
+// Slots of a cache that is not split; of a split.  Every (sequence, head, half) walks its whole prefix, so the lines lie where that takes as
+// long as the launches with the attention split over the chip (us a step, caches filled to 90 %, those -> this: two sequences, 700 slots
+// 1004 -> 833, 1024 1012 -> 915, 1528 1033 -> 1052; three, 1024 1044 -> 1018, 1528 1066 -> 1145; four, 700 1044 -> 966, 1024 1058 -> 1043,
+// 1528 1078 -> 1174; filled to half 15 - 23 % ahead at two, 6 - 12 % at four).
+constexpr int step_max_slots(int M) { return M == 2 ? 1280 : 1024; }
+constexpr int kStepMaxSplitSlots = 1024;
 constexpr int kStepWideTiles = 112;              // tiles of the down projection's K: ffn <= 7168
 constexpr int kStepTiles = 40;                   // tiles of the other linears' K: <= 2560
 constexpr uint32_t kStepEmpty = 0xffffffffu;
@@ -136,7 +141,7 @@ struct StepLds {
     static constexpr int kPartialBytes = (MR * kPartials > kStepWideTiles * 4 ? MR * kPartials : kStepWideTiles * 4) * 8;
     static constexpr int kLinear = kStepWaves * kSlab + kPartialBytes;
     // attention: slices and groups of output dimensions, scores
-    static constexpr int kScores = (MR == 1 ? kStepMaxSplitSlots : kStepMaxSlots) + 32;
+    static constexpr int kScores = (MR == 1 ? kStepMaxSplitSlots : step_max_slots(MR)) + 32;
     static constexpr int kAttention = ((16 + 2) * kStepHeadDim + kScores) * 4;             // (slices and groups: the same number of floats split or not)
     static constexpr int kBytes = kLinear > kAttention ? kLinear : kAttention;
     static_assert(4 * MR * 64 <= kSlab, "the accumulators of four bands fit a wave's slab");

@@ -563,7 +563,7 @@ class Transformer:
         """The residual stream behind the last block of a single-token step of up to four sequences, all blocks in one launch
         (ternaspmm_decode_step), or None: where the library does not take the shape, and where something asks for the launches it
         stands for -- a recording block, a prefetch, a switch of the chain that is not at its default.  The same bits as
-        those launches (Block.forward_chain with `split` False)."""
+        those launches (Block.forward_chain with `split` False, for two sequences and more with the attention in one piece)."""
         a = self.args
         bsz = tokens.shape[0]
         if bsz > self.chain_rows or bsz > 4 or not self.one_launch_step or not a.rope_adjacent or a.head_dim != 128 or \
@@ -576,8 +576,6 @@ class Transformer:
             splits = _lib.load().ternaspmm_attention_partial_splits_kv(1, a.n_heads, a.n_kv_heads, max_seq)
             if splits < 2:
                 return None
-        elif max_seq > self.defer_above:
-            return None
         lin = lambda w, packed: (packed, w.ws, w.ws_num, w.n)
         blocks = [lin(b.wqkv, b.wqkv.packed) + lin(b.wo, b.wo.packed) + lin(b.w13, b.gate_up_interleaved()) + lin(b.w2, b.w2.packed) +
                   (b.attention_norm, b.attn_sub_norm, b.ffn_norm, b.ffn_sub_norm, ck, cv) for b, (ck, cv) in zip(self.layers, cache)]
