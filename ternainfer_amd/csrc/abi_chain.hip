@@ -92,6 +92,7 @@ __global__ __launch_bounds__(256) void terna_interleave_gate_up_kernel(const uin
 // for row counts at which every consuming workgroup repeating the element-wise work costs more than this launch.
 // Grid (M, ceil(K / 2048)); every wave adds up the partials of its row in the same fixed order as the FUSED_STATS
 // prologue, so the (xq, s) written here are the ones that prologue would have formed.
+template <int PT>
 __global__ __launch_bounds__(256) void terna_quant_stats_kernel(const uint16_t* __restrict__ h, const float2* __restrict__ stats, int count,
                                                                  const uint16_t* __restrict__ norm_w, int K, float eps,
                                                                  int8_t* __restrict__ xq_out, uint16_t* __restrict__ s_out, int quant_mode)
@@ -102,7 +103,6 @@ __global__ __launch_bounds__(256) void terna_quant_stats_kernel(const uint16_t* 
     const bool in = c < K;                                       // K is a multiple of 8
     const u32x4 hv = *reinterpret_cast<const u32x4*>(h + row * K + (in ? c : 0));
     const u32x4 wv = *reinterpret_cast<const u32x4*>(norm_w + (in ? c : 0));
-    constexpr int PT = kStatsMaxPartials / 64;
     float2 part[PT];
 #pragma unroll
     for (int t = 0; t < PT; ++t) {
@@ -191,7 +191,7 @@ template <int NBANDS, int EPI, int UNIT_BANDS = (NBANDS == 4 ? 2 : 1)>
 bool launch_chunk_by_rows(const ChainArgs& a, int units)
 {
     const ChainIo io{a.out, a.ws, a.xq_out, a.s_out, a.ex.epi_residual, a.ex.epi_next_w, a.ex.stats_out, a.ex.raw_out};
-    const int workers = kChunkWaves - a.M;
+    const int workers = kChunkWaves - chain_reducers(a.M, units);
     const int ct = (units + workers - 1) / workers;
     if (ct > 3) return false;
 #define TERNA_CHAIN_CHUNK(CT, MR)                                                                                       \
@@ -424,7 +424,8 @@ int ternaspmm_quant_from_stats(const terna_bf16* h, const float* stats, int stat
         std::fprintf(stderr, "ternaspmm_quant_from_stats: unsupported arguments (M=%d K=%d partials=%d)\n", M, K, stats_count);
         return -1;
     }
-    terna_quant_stats_kernel<<<dim3(M, (K + 2047) / 2048), dim3(256), 0, static_cast<hipStream_t>(stream)>>>(
+    auto kernel = stats_count <= 192 ? terna_quant_stats_kernel<3> : terna_quant_stats_kernel<kStatsMaxPartials / 64>;      // partials a lane
+    kernel<<<dim3(M, (K + 2047) / 2048), dim3(256), 0, static_cast<hipStream_t>(stream)>>>(
         h, reinterpret_cast<const float2*>(stats), stats_count, norm_weight, K, eps, xq_out, s_out, quant_mode());
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) die("ternaspmm_quant_from_stats", e, __LINE__);

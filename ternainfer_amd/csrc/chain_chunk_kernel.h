@@ -49,12 +49,13 @@ constexpr int kChainSlabPitch = 256 + 16;
 
 // Row statistics from the producer's partials: wave r < M, all its lanes.  Leaves rstd / the multiplier / the bf16 scale
 // of row r in LDS (lane 0) and publishes the scale when asked to.
-__device__ __forceinline__ void chain_reduce_partials(const float2 (&part)[kStatsMaxPartials / 64], int row, int K, float eps, int quant_mode,
+template <int PN>
+__device__ __forceinline__ void chain_reduce_partials(const float2 (&part)[PN], int row, int K, float eps, int quant_mode,
                                                       float* rstd_s, float* smul_s, float* sval_s, uint16_t* s_out, int lane)
 {
     float sum = 0.0f, pmax = 0.0f;
 #pragma unroll
-    for (int t = 0; t < kStatsMaxPartials / 64; ++t) {      // entries past the count were out of range: zeros
+    for (int t = 0; t < PN; ++t) {                          // entries past the count were out of range: zeros
         sum += part[t].x;
         pmax = max_keep_nan(pmax, part[t].y);
     }
@@ -110,13 +111,20 @@ __device__ __forceinline__ void chain_quantise(const uint32_t (&hraw)[NE / 2], c
 //             w3), two gate / up pairs per workgroup so that one round of workgroups covers 864 bands; CEPI_GATE.  A unit of
 //             work is (chunk, pair) -- unit u is chunk u of pair 0 for u < chunks, chunk u - chunks of pair 1 behind it --
 //             or, UNIT_BANDS = 4, a chunk with all four bands: its activations are then normed and quantised once.
-// The 16 - M working waves take the units round robin, CT each at most.
+// A wave reduces a row's partials; the others take the units round robin, CT each at most.  From 5 rows on a wave reduces two
+// rows where the units then take one round (chain_reducers).
 // MR = 1, 2, 4 or 8 >= M: rows of the wave's LDS slot.  One row: 64 lanes x 4 columns; more: 32 lanes x 8 columns, two rows
 // per load.
 // XQ: the activations are quantised already (`hin` is int8 [M][K], io.s_in their scales; a launch of
 // terna_quant_stats_kernel or of the norm kernel made them): no reducing waves, no statistics, no barrier ahead of the
 // matmul; all 16 waves share the units and a chunk's rows go from the load to the LDS slot as they are (16 bytes per lane,
 // four rows per load).  The producing epilogues are the same.  MR = 16 exists in this form only.
+// Reducing waves of M rows: 7 or 8 rows and 10 units (K = 2560) are 6 waves that reduce and one round of 10, not 7 or 8 and two rounds
+// (decode step, 384 slots: 7 sequences 1082 -> 1026 us, 8 1072 -> 1034).
+__host__ __device__ inline int chain_reducers(int M, int units)
+{
+    return M <= 4 || units <= kChunkWaves - M || units > kChunkWaves - (M + 1) / 2 ? M : kChunkWaves - units;
+}
 template <int NBANDS, int CT, int MR, int EPI, int UNIT_BANDS = (NBANDS == 4 ? 2 : 1), bool XQ = false>
 __global__ __launch_bounds__(kChunkWaves * 64) void terna_chain_chunk_kernel(
     const void* __restrict__ hin, const uint16_t* __restrict__ norm_w, const uint32_t* __restrict__ packed,
@@ -151,7 +159,7 @@ __global__ __launch_bounds__(kChunkWaves * 64) void terna_chain_chunk_kernel(
     const bool writer = blockIdx.x == 0;
 
     // this wave's units of work
-    const int reducers = XQ ? 0 : M;
+    const int reducers = XQ ? 0 : (MR == 8 ? chain_reducers(M, chunks * UPAIRS) : M);
     const bool reducer = wave < reducers;
     const int workers = WAVES - reducers;
     int upair[CT], uchunk[CT];
@@ -173,15 +181,25 @@ __global__ __launch_bounds__(kChunkWaves * 64) void terna_chain_chunk_kernel(
 
     // What a wave requests: a reducing wave its row's partials; a working wave the weights, then the activations and norm
     // weights of its chunks; a finishing wave the epilogue's operands on top.
-    float2 part[PT];
-    auto request_partials = [&]() {
+    // ROWS rows of this wave, PN partials a lane: K = 2560 fills three of the seven loads there can
+    // be, and all other waves wait for these (decode step of five sequences, 384 slots: seven loads 1002 us, three 997; fourteen 1040).
+    auto reduce_rows = [&](auto rows, auto pn, auto meanwhile) {
+        constexpr int ROWS = decltype(rows)::value, PN = decltype(pn)::value;
         const __amdgpu_buffer_rsrc_t rs = make_raw_buffer(stats_in, static_cast<uint32_t>(M) * stats_count * 8u);
+        float2 part[ROWS][PN];
 #pragma unroll
-        for (int t = 0; t < PT; ++t) {
-            const int idx = lane + 64 * t;
-            const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, idx < stats_count ? (wave * stats_count + idx) * 8 : kBufferOutOfRange, 0, 0));
-            part[t] = float2{__uint_as_float(v.x), __uint_as_float(v.y)};
-        }
+        for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+            for (int t = 0; t < PN; ++t) {
+                const int row = wave + reducers * r, idx = lane + 64 * t;
+                const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, row < M && idx < stats_count ? (row * stats_count + idx) * 8 : kBufferOutOfRange, 0, 0));
+                part[r][t] = float2{__uint_as_float(v.x), __uint_as_float(v.y)};
+            }
+        meanwhile();
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r)
+            if (wave + reducers * r < M)         // uniform
+                chain_reduce_partials<PN>(part[r], wave + reducers * r, K, eps, quant_mode, rstd_s, smul_s, sval_s, writer ? io.s_out : nullptr, lane);
     };
     // Finishing: the accumulators of a band lie in LDS as a [batch row][column] matrix; task (p, q) = band (pair) p, batch
     // rows 4q .. 4q+3 goes to wave p FW + q: lane l has row 4q + (l >> 4), column l & 15.
@@ -269,9 +287,21 @@ __global__ __launch_bounds__(kChunkWaves * 64) void terna_chain_chunk_kernel(
         for (int o = MR * kChainSlabPitch + lane * 16; o < (MR + 1) * kChainSlabPitch; o += 64 * 16) *reinterpret_cast<u32x4*>(slab + o) = u32x4{0u, 0u, 0u, 0u};
     } else {
         if (reducer) {
-            request_partials();
-            if (finisher) request_epilogue();
-            chain_reduce_partials(part, wave, K, eps, quant_mode, rstd_s, smul_s, sval_s, writer ? io.s_out : nullptr, lane);
+            auto meanwhile = [&]() {
+                if (finisher) request_epilogue();
+            };
+            using One = std::integral_constant<int, 1>;
+            using Two = std::integral_constant<int, 2>;
+            using Few = std::integral_constant<int, 3>;
+            using All = std::integral_constant<int, PT>;
+            const bool two = MR == 8 && reducers < M;
+            if (stats_count <= 64 * Few::value) {
+                if (two) reduce_rows(Two{}, Few{}, meanwhile);
+                else reduce_rows(One{}, Few{}, meanwhile);
+            } else {
+                if (two) reduce_rows(Two{}, All{}, meanwhile);
+                else reduce_rows(One{}, All{}, meanwhile);
+            }
         } else if (finisher) {
             request_epilogue();
         }

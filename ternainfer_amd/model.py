@@ -113,9 +113,9 @@ KERNEL_ATTENTION = object()    # in place of a mask: several new tokens, attenti
 
 class Block:
     # forward_chain: up to this many rows the O projection takes the sub-norm's statistics inside; above, the norm kernel
-    # and the O projection on its quantised rows (measured: 4 sequences 3917 against 3769 tokens/s, 5 sequences 4285
-    # against 4343, 8 sequences 6708 against 6849)
-    o_norm_rows = 4
+    # and the O projection on its quantised rows (measured, us a step of 384 slots with the O projection so: 5 sequences 1022 -> 1002, 6 1030 -> 1014,
+    # 8 1071 -> 1066)
+    o_norm_rows = 8
     attention_stats_chain = True   # the same for 2 .. o_norm_rows sequences, consumed by the O projection's STATS prologue (+1 - 1.6 %)
     attention_stats = True         # ... and the unsplit attention launch leaves the sub-norm's partial statistics (see forward_chain)
     merge_quant = True             # forward_chain, several sequences, deferred attention merge: the merge launch also norms and quantises
@@ -417,8 +417,8 @@ class Block:
 
 #: switches of the chained step whose other settings ask for its launches one by one (Transformer.whole_step)
 _STEP_SWITCHES = (("step_inputs", True), ("deferred_attention_merge", True), ("attention_splits", None), ("split_merge_quant", False), ("defer_above", 640),
-                  ("chain_rows", 4))
-_CHAIN_SWITCHES = (("o_norm_rows", 4), ("attention_stats_chain", True), ("attention_stats", True), ("merge_quant", True), ("chain_down_rows", 2))
+                  ("chain_rows", 8))
+_CHAIN_SWITCHES = (("o_norm_rows", 8), ("attention_stats_chain", True), ("attention_stats", True), ("merge_quant", True), ("chain_down_rows", 2))
 
 
 class Transformer:
@@ -426,9 +426,10 @@ class Transformer:
 
     # Up to this many sequences a one-token step chains its linears with the norm + quantisation inside the consuming
     # linear (Block.forward_chain).  Every workgroup of such a linear normalises and quantises the whole activation matrix
-    # again, and one of its waves per row only adds up partials; from five rows on that costs more than a launch that does
-    # it once (measured at 5, 6 and 8 rows).
-    chain_rows = 4
+    # again, and some of its waves only add up partials: at four instructions an element still less than a launch that does
+    # it once (us a step of 384 slots, launches -> inside: 5 sequences 1070 -> 997, 6 1079 -> 1008, 7 1082 -> 1026, 8 1088 -> 1034; 8 with
+    # 1528 slots 1237 -> 1204).
+    chain_rows = 8
     # Above that, up to this many sequences, the producing epilogues stay (residual add, gate, partial statistics) and a
     # small element-wise launch forms the quantised rows from the partials (Block.forward_chain, split): lighter than the
     # norm kernels, which reduce over the row twice, and the gate+up launch writes F columns instead of 2F.
@@ -635,7 +636,7 @@ class Transformer:
         # 1.198 against 1.218 ms per step -- `split_merge_quant` forces the split form)
         # With more heads than CUs already from 256 slots on (14 sequences, 384 slots: 1303 -> 1217 us a step; 20, 512: 1607 -> 1500; at 256 slots
         # level), where the chip holds two splits of every kv head and more.
-        short = 256 if bsz * a.n_heads > 256 else 512 if split else self.defer_above
+        short = 256 if bsz * a.n_heads > 256 else 512 if chain and bsz > 4 else self.defer_above
         if one_launch_attention and self.layers[0].act == "int8" and (bsz == 1 or max_seq > short):
             attn_ws = self.attention_partial(bsz, max_seq) or attn_ws
         elif split and getattr(self, "split_merge_quant", False):

@@ -426,3 +426,24 @@ def test_unsupported_combinations_are_declined():
                           next_norm_weight=_bf(_weight(n // 2, 1254))) is None                              # GATE on quantised rows: up to 16
     assert L.fused_linear(xq9, None, 1e-5, packed, _bf(WS), 1, n, k, quantised=s9) is None                 # QUANTISED + STORE: bitlinear_TernaSpMM_packed
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("m,k,count", [(5, 2560, 160), (6, 2560, 192), (7, 2560, 160), (8, 2560, 160), (8, 2560, 193), (7, 2304, 144), (8, 2112, 1), (8, 2048, 128), (7, 6912, 432),
+                                       (8, 6976, 436), (8, 192, 12)])
+def test_reducing_waves_of_five_to_eight_rows(m, k, count):
+    """One or two rows a reducing wave, few partials or all: the integers and scales of the launch that quantises from the same
+    partials, and with them the same outputs."""
+    n = 256
+    w = make_ternary(n, k, 0.4, 1251 + k)
+    packed, ws = _packed(w), _bf(WS)
+    h, g, nxt, res = _bf(make_bf16_activations(m, k, 1252)), _bf(_weight(k, 1253)), _bf(_weight(n, 1254)), _bf(make_bf16_activations(m, n, 1255))
+    rng = np.random.default_rng(1256)
+    stats = torch.from_numpy(rng.uniform(0.1, 1.0, (m, count, 2)).astype(np.float32) * np.array([k / count, 8.0], np.float32)).cuda()
+    print(f"[case] reducing waves m={m} k={k} count={count}", flush=True)
+    kw = dict(epilogue=L.EPILOGUE_RESIDUAL, residual=res, next_norm_weight=nxt, want_raw=True)
+    inside = L.fused_linear(h, g, 1e-5, packed, ws, 1, n, k, stats=stats, publish=True, **kw)
+    xq, s = L.quant_from_stats(h, stats, g, 1e-5)
+    outside = L.fused_linear(xq, None, 1e-5, packed, ws, 1, n, k, quantised=s, **kw)
+    assert torch.equal(inside[3], xq) and torch.equal(inside[4].view(torch.int16), s.view(torch.int16)) and bool(xq.any())
+    for a, b in zip(inside[:3], outside[:3]):
+        assert torch.equal(a, b)
