@@ -477,7 +477,7 @@ class Transformer:
     def enable_prefetch(self, on: bool = True, which=("wo", "w13", "w2", "next_wqkv", "norms")) -> None:
         """Single-token steps: while a block's attention runs (one workgroup per head), extra workgroups of that
         launch prefetch the weights of its O, gate+up and down projections and of the next block's QKV projection
-        (`which` picks among them).  Measured on MI355X with the unsplit attention launch: +6 % tokens/s at batch 1 with
+        (`which` picks among them).  A step that one launch takes (whole_step) does without.  Measured on MI355X with the unsplit attention launch: +6 % tokens/s at batch 1 with
         all four.  With the step as it is now -- one sequence runs the split attention, which passes no regions -- it pays
         for two sequences (+1 %); from three on the step is 1.4 - 1.7 % faster without, and where few CUs are left idle the
         prefetching workgroups become the launch's critical path (nine to eleven sequences: 10 - 20 % slower)."""
@@ -563,14 +563,15 @@ class Transformer:
     def whole_step(self, tokens, cache, pos_idx, max_seq):
         """The residual stream behind the last block of a single-token step of up to four sequences, all blocks in one launch
         (ternaspmm_decode_step), or None: where the library does not take the shape, and where something asks for the launches it
-        stands for -- a recording block, a prefetch, a switch of the chain that is not at its default.  The same bits as
+        stands for -- a recording block, a switch of the chain that is not at its default.  (Not `enable_prefetch`: the step fetches its
+        weights ahead by itself; one sequence, 384 slots, with prefetching launches 819 us, so 653, bookkeeping included.)  The same bits as
         those launches (Block.forward_chain with `split` False, for two sequences and more with the attention in one piece)."""
         a = self.args
         bsz = tokens.shape[0]
         if bsz > self.chain_rows or bsz > 4 or not self.one_launch_step or not a.rope_adjacent or a.head_dim != 128 or \
                 any(getattr(self, name, default) != default for name, default in _STEP_SWITCHES) or \
                 any(getattr(Block, name) != default for name, default in _CHAIN_SWITCHES) or \
-                any(blk.capture is not None or blk.prefetch is not None or not blk.fused or blk.act != "int8" or type(blk) is not Block for blk in self.layers):
+                any(blk.capture is not None or not blk.fused or blk.act != "int8" or type(blk) is not Block for blk in self.layers):
             return None
         splits = 1
         if bsz == 1:
