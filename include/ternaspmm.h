@@ -282,10 +282,9 @@ int bitlinear_TernaSpMM_packed_fused_glu(const terna_bf16* x13, const terna_bf16
  *             TERNASPMM_PROLOGUE_QUANTISED  x = int8 [M][K] with its scales s_in bf16 [M] (ternaspmm_quant_from_stats,
  *                                           ternaspmm_rmsnorm_quant): no prologue; with TERNASPMM_EPILOGUE_RESIDUAL
  *                                           (M <= 16, any K the int8 kernels take) or TERNASPMM_EPILOGUE_GATE (M <= 16,
- *                                           K <= 6144).  From five rows on this pair -- the element-wise quantise launch,
- *                                           then the linear on its rows -- is the faster way to consume a producer's
- *                                           partials (measured, 2B shapes, 8 rows: 6706 against 6498 tokens/s for the
- *                                           norm kernels + plain linears, 6322 for the STATS prologue)
+ *                                           K <= 6144).  From nine rows on (K = 6912: three) this pair -- the element-wise
+ *                                           quantise launch, then the linear on its rows -- is the faster way to consume a
+ *                                           producer's partials
  *   epilogue  TERNASPMM_EPILOGUE_STORE      out bf16 [M][N] = the linear's output (decode rule, Reduction_Kernel.cuh:60)
  *             TERNASPMM_EPILOGUE_RESIDUAL   out bf16 [M][N] = bf16(residual + output): the residual stream after this
  *                                           linear (model.py:330, :334); stats_out fp32 [M][N/16][2] = its partials under
@@ -329,7 +328,7 @@ int ternaspmm_fused_linear(const ternaspmm_fused_linear_desc* desc, terna_stream
 /* Norm + quant_input of h bf16 [M][K] as a launch of its own, from partials a producer left: xq_out int8 [M][K], s_out bf16 [M]
  * -- the values the TERNASPMM_PROLOGUE_STATS prologue forms inside its launch (same order of additions), for row counts at
  * which every consuming workgroup repeating the element-wise work costs more than one more launch (measured on MI355X: the
- * down projection, K = 6912, from five rows on).  Returns 0 / -1.  Only enqueues. */
+ * down projection, K = 6912, from three rows on; K = 2560 from nine on).  Returns 0 / -1.  Only enqueues. */
 int ternaspmm_quant_from_stats(const terna_bf16* h, const float* stats, int stats_count, const terna_bf16* norm_weight, float eps,
                                int8_t* xq_out, terna_bf16* s_out, int M, int K, terna_stream stream);
 

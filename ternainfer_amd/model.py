@@ -540,12 +540,8 @@ class Transformer:
         splits = getattr(self, "attention_splits", None) or lib.ternaspmm_step_attention_splits(bsz, a.n_heads, a.n_kv_heads, max_seq)
         if splits < 1 or (splits == 1 and not single_split):
             return None
-        # one buffer per batch size, kept while the model lives: a captured decode graph holds the raw pointer
-        held = self.__dict__.setdefault("_attn_partial", {})
-        if bsz not in held:
-            nbytes = lib.ternaspmm_attention_partial_bytes(bsz, a.n_heads, a.head_dim)
-            held[bsz] = torch.empty(nbytes // 4, dtype=torch.float32, device="cuda")
-        return held[bsz], splits
+        # of this step: steps of several streams may overlap (a captured one's lies in its graph's pool)
+        return torch.empty(lib.ternaspmm_attention_partial_bytes(bsz, a.n_heads, a.head_dim) // 4, dtype=torch.float32, device="cuda"), splits
 
     def attention_workspace(self, bsz: int):
         """Zero-filled scratch of the single-token attention (split over the cache); one per batch size, kept while

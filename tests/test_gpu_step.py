@@ -163,3 +163,30 @@ def test_steps_on_several_streams_at_once():
                 assert same(logits, want)
                 logits.zero_()
         torch.cuda.synchronize()
+
+
+def test_split_attention_steps_of_two_streams_at_once():
+    """Two captured steps of one model and one batch size whose launches leave partial attention results, side by side: each has
+    its own."""
+    model = build(WIDE, 4)
+    runs = []
+    for i in range(2):
+        whole, tokens, pos = state(model, 6, 700, [690 - 30 * i], seed=40 + i)
+        assert model.attention_partial(6, 700)[1] > 1 and model.whole_step(tokens, [(whole[n, 0], whole[n, 1]) for n in range(4)], pos, 700) is None
+        cache = [(whole[n, 0], whole[n, 1]) for n in range(4)]
+        stream = torch.cuda.Stream()
+        with torch.inference_mode():
+            want = model.forward(tokens, cache, pos).clone()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                logits = model.forward(tokens, cache, pos)
+        runs.append((stream, graph, logits, want, cache, tokens, pos))
+    torch.cuda.synchronize()
+    for _ in range(3):
+        for _ in range(8):
+            for stream, graph, *_ in runs:
+                with torch.cuda.stream(stream):
+                    graph.replay()
+        torch.cuda.synchronize()
+        for _, _, logits, want, *_ in runs:
+            assert same(logits, want)
