@@ -434,7 +434,7 @@ class Transformer:
     # small element-wise launch forms the quantised rows from the partials (Block.forward_chain, split): lighter than the
     # norm kernels, which reduce over the row twice, and the gate+up launch writes F columns instead of 2F.
     split_rows = 16
-    # Cache slots from which on a chained step of 2 .. chain_rows sequences splits its attention and leaves the merge to a
+    # Cache slots from which on a chained step of two to four sequences (more: 512) splits its attention and leaves the merge to a
     # launch of its own (measured, 4 sequences: 428 slots 1.041 ms per step unsplit against 1.115, 728 slots 1.154 against 1.120)
     defer_above = 640
 
