@@ -357,9 +357,9 @@ int ternaspmm_step_inputs(const long long* tokens, const long long* pos, int per
 int ternaspmm_prompt_inputs(const long long* tokens, const long long* pos, int pos_rows, const terna_bf16* embedding, int V, int K,
                             const float* rope_table, int S, int rope_half, terna_bf16* x_out, float* rope_out, int M, terna_stream stream);
 
-/* A decode step of one to four sequences -- embedding rows, every block, everything up to the final norm -- in two launches:
- * one that forms the inputs (as ternaspmm_step_inputs) and clears `scratch`, and one whose workgroups stay for all blocks and hand
- * the rows from phase to phase in `scratch` (up to 32 blocks; more take one more launch each).  The same bits as the launches it
+/* A decode step of one to four sequences -- embedding rows, every block, everything up to the final norm -- in three launches:
+ * one that forms the inputs (as ternaspmm_step_inputs) and clears `scratch`, one whose workgroups stay for all blocks and hand
+ * the rows from phase to phase in `scratch` (up to 32 blocks; more take one more launch each), and one as a rule empty (below).  The same bits as the launches it
  * stands for: ternaspmm_fused_linear with the partial statistics of the producers, and between them
  * ternaspmm_rope_decode_attention_partial of `splits` splits (one sequence) or ternaspmm_rope_decode_attention_stats (more), with
  * ternaspmm_quant_from_stats in front of the down projection from two sequences on.
@@ -369,10 +369,12 @@ int ternaspmm_prompt_inputs(const long long* tokens, const long long* pos, int p
  *   x_out    bf16 [M][dim]: the residual stream behind the last block
  * Takes head_dim 128, dim and heads * head_dim up to 2560, ffn up to 7168 (multiples of 64), at most 4096 QKV columns; one sequence: two,
  * four or eight splits of up to 1024 slots; more: splits = 1 and up to 1024 slots (two: 1280), not in quant mode 2.
- * The workgroups wait for each other, so all of them have to be resident: the call is refused where the device (or the
- * stream's mask of CUs) does not hold four such grids at once -- as many as the runtime's default of four hardware queues runs
- * side by side; GPU_MAX_HW_QUEUES above that raises the bound.  (More than four such steps at once from several processes, or from
- * streams of several priorities, are not foreseen.)  A wait that lasts four seconds ends the step with NaN rows.
+ * The workgroups wait for each other, so all of them should be resident: the call is refused where the device (or the
+ * stream's mask of CUs at the time of the call) does not hold four such grids at once -- as many as the runtime's default of
+ * four hardware queues runs side by side; GPU_MAX_HW_QUEUES above that raises the bound.  A step whose workgroups are not
+ * resident together all the same -- more than four at once, from several processes or on streams of several priorities; a captured one
+ * replayed on a stream with a narrower mask -- gives up after 20 ms and more and is done again by a launch behind it that needs none
+ * of that, in three or four milliseconds: the same results, later.  (Programs that share a GPU like that are better off with the launches.)
  * ternaspmm_decode_step_bytes: bytes of `scratch` (256-byte aligned, its contents do not matter), or -1 for a shape that is not
  * taken.  ternaspmm_decode_step: 0, or -1 (nothing enqueued).  Only enqueues; calls that overlap need scratch of their own. */
 typedef struct ternaspmm_step_block {
@@ -656,6 +658,9 @@ int ternaspmm_plan_reference_call(int int8_activations, int route, int M, int N,
  *                            far): what a persistent kernel would pay between two dependent phases.  Every wait is
  *                            bounded; uint32 word 512 of `state` counts workgroups that gave up (0 after a good run).
  *                            Returns 0, or -1 when the arguments are refused.
+ *   ternaspmm_probe_decode_step  ternaspmm_decode_step with `workgroups` (1 .. 256) of the 256 that wait for each other and
+ *                            waits of `polls` polls (0 .. 131072; looked at every 256): the step where the device does not hold them
+ *                            all, which is done again in order.
  * All only enqueue; time them with events on `stream`. */
 void ternaspmm_probe_empty(terna_stream stream);
 int ternaspmm_probe_empty_shape(int workgroups, int threads, int lds_bytes, terna_stream stream);
@@ -663,6 +668,9 @@ void ternaspmm_probe_read(const void* src, long long bytes, void* sink, terna_st
 int ternaspmm_probe_read_grid(const void* src, long long bytes, void* sink, int workgroups, terna_stream stream);
 void ternaspmm_probe_copy(const void* src, void* dst, long long bytes, terna_stream stream);
 size_t ternaspmm_probe_barrier_state_bytes(void);
+int ternaspmm_probe_decode_step(const ternaspmm_step_desc* desc, const ternaspmm_step_block* blocks, const long long* tokens, const long long* pos,
+                                const terna_bf16* embedding, const float* rope_table, void* scratch, terna_bf16* x_out, int workgroups, int polls,
+                                terna_stream stream);
 int ternaspmm_probe_barrier(void* state, int workgroups, int rounds, unsigned first_tag, terna_stream stream);
 
 /* Library version string, e.g. "ternaspmm-gfx950 0.1". */

@@ -78,6 +78,7 @@ PROTOTYPES = {
     "ternaspmm_probe_copy": ([_vp, _vp, ctypes.c_longlong, _vp], None),
     "ternaspmm_probe_barrier_state_bytes": ([], ctypes.c_size_t),
     "ternaspmm_probe_barrier": ([_vp, _ci, _ci, ctypes.c_uint, _vp], ctypes.c_int),
+    "ternaspmm_probe_decode_step": ([_vp] * 8 + [_ci, _ci, _vp], _ci),
     "ternaspmm_repack_cache_clear": ([], None),
     "ternaspmm_repack_cache_enable": ([_ci], _ci),
     "ternaspmm_repack_cache_limit": ([ctypes.c_longlong], ctypes.c_longlong),

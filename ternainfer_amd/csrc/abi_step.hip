@@ -5,6 +5,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <mutex>
+#include <type_traits>
 
 #include "../../include/ternaspmm.h"
 #include "host_util.h"
@@ -54,12 +55,13 @@ StepExchange exchange_of(const ternaspmm_step_desc& d)
 
 const void* step_kernel_of(int M)
 {
-    return M == 1 ? reinterpret_cast<const void*>(terna_decode_step_kernel<1>)
-                  : M == 2 ? reinterpret_cast<const void*>(terna_decode_step_kernel<2>) : reinterpret_cast<const void*>(terna_decode_step_kernel<4>);
+    return M == 1 ? reinterpret_cast<const void*>(terna_decode_step_kernel<1, false>)
+                  : M == 2 ? reinterpret_cast<const void*>(terna_decode_step_kernel<2, false>) : reinterpret_cast<const void*>(terna_decode_step_kernel<4, false>);
 }
 
-// Whether as many grids as the runtime runs side by side are resident together, whatever their order: the workgroups of a
-// step wait for each other.  A queue with a mask of CUs has to hold them with those.
+// Whether as many grids as the runtime runs side by side for a process are resident together, whatever their order: the workgroups
+// of a step wait for each other, and one whose do not come loses the time of the waits and of doing it in order.  A
+// queue with a mask of CUs has to hold them with those.
 bool grids_fit(int M, hipStream_t st)
 {
     static const int queues = [] {               // hardware queues per process (HIP's default: 4)
@@ -116,19 +118,9 @@ bool step_shape_ok(const ternaspmm_step_desc& d)
     return d.M == 1 || quant_mode() != QUANT_EAGER;          // (the int8 words that are handed over need one value no integer takes)
 }
 
-}  // namespace
-
-extern "C" {
-
-long long ternaspmm_decode_step_bytes(const ternaspmm_step_desc* d)
-{
-    if (d == nullptr || !step_shape_ok(*d)) return -1;
-    const long long count = ternaspmm_row_stats_count(d->dim);
-    return 256 + static_cast<long long>(d->layers) * exchange_of(*d).bytes + up(2ll * d->M * d->dim) + up(8ll * d->M * count) + up(4ll * d->M * d->head_dim);
-}
-
-int ternaspmm_decode_step(const ternaspmm_step_desc* d, const ternaspmm_step_block* blocks, const long long* tokens, const long long* pos,
-                          const terna_bf16* embedding, const float* rope_table, void* scratch, terna_bf16* x_out, terna_stream stream)
+// groups, patience: of the resident launches.
+int enqueue_step(const ternaspmm_step_desc* d, const ternaspmm_step_block* blocks, const long long* tokens, const long long* pos, const terna_bf16* embedding,
+                 const float* rope_table, void* scratch, terna_bf16* x_out, int groups, int patience, terna_stream stream)
 {
     const long long bytes = ternaspmm_decode_step_bytes(d);
     if (bytes < 0 || blocks == nullptr || tokens == nullptr || pos == nullptr || embedding == nullptr || rope_table == nullptr || scratch == nullptr ||
@@ -150,7 +142,7 @@ int ternaspmm_decode_step(const ternaspmm_step_desc* d, const ternaspmm_step_blo
     StepArgs a{};
     a.at = exchange_of(*d);
     char* base = static_cast<char*>(scratch);
-    const long long cleared = 256 + static_cast<long long>(d->layers) * a.at.bytes;
+    const long long cleared = kStepControlBytes + static_cast<long long>(d->layers) * a.at.bytes;
     uint16_t* x = reinterpret_cast<uint16_t*>(base + cleared);
     float2* stats = reinterpret_cast<float2*>(base + cleared + up(2ll * d->M * d->dim));
     float* rope = reinterpret_cast<float*>(base + cleared + up(2ll * d->M * d->dim) + up(8ll * d->M * count));
@@ -164,26 +156,58 @@ int ternaspmm_decode_step(const ternaspmm_step_desc* d, const ternaspmm_step_blo
     a.M = d->M, a.dim = d->dim, a.ffn = d->ffn, a.H = d->heads, a.KV = d->kv_heads, a.S = d->slots, a.SP = d->splits, a.per_seq = d->per_sequence != 0;
     a.stats_count = count, a.quant_mode = quant_mode(), a.ws_qkv = d->ws_num_qkv, a.ws_o = d->ws_num_o, a.ws_2 = d->ws_num_down;
     a.eps = d->eps, a.scale = d->scale;
-    for (int first = 0; first < d->layers; first += kStepMaxBlocks) {
-        a.blocks = d->layers - first < kStepMaxBlocks ? d->layers - first : kStepMaxBlocks;
-        a.exchange = base + 256 + static_cast<size_t>(first) * a.at.bytes;
-        a.x = first == 0 ? x : reinterpret_cast<const uint16_t*>(a.exchange - a.at.bytes + a.at.out);
-        a.stats = first == 0 ? stats : nullptr;
-        // (behind the last block of a launch that is not the last: where that block's consumers look for it)
-        a.x_out = first + a.blocks == d->layers ? x_out : reinterpret_cast<uint16_t*>(a.exchange + static_cast<size_t>(a.blocks - 1) * a.at.bytes + a.at.out);
-        for (int n = 0; n < a.blocks; ++n) {
-            const ternaspmm_step_block& b = blocks[first + n];
-            a.block[n] = StepBlock{static_cast<const uint32_t*>(b.wqkv), static_cast<const uint32_t*>(b.wo), static_cast<const uint32_t*>(b.w13),
-                                   static_cast<const uint32_t*>(b.w2), b.ws_qkv, b.ws_o, b.ws_13, b.ws_down, b.attention_norm, b.attn_sub_norm, b.ffn_norm,
-                                   b.ffn_sub_norm, b.cache_k, b.cache_v};
+    a.patience = patience;
+    auto launches = [&](auto ordered) {
+        constexpr bool ORDERED = decltype(ordered)::value;
+        const dim3 grid(ORDERED ? kStepOrderedGroups : groups), threads(kStepThreads);
+        for (int first = 0; first < d->layers; first += kStepMaxBlocks) {
+            a.blocks = d->layers - first < kStepMaxBlocks ? d->layers - first : kStepMaxBlocks;
+            a.tickets = a.alive + 1 + 2 * (first / kStepMaxBlocks);
+            a.exchange = base + kStepControlBytes + static_cast<size_t>(first) * a.at.bytes;
+            a.x = first == 0 ? x : reinterpret_cast<const uint16_t*>(a.exchange - a.at.bytes + a.at.out);
+            a.stats = first == 0 ? stats : nullptr;
+            // (behind the last block of a launch that is not the last: where that block's consumers look for it)
+            a.x_out = first + a.blocks == d->layers ? x_out : reinterpret_cast<uint16_t*>(a.exchange + static_cast<size_t>(a.blocks - 1) * a.at.bytes + a.at.out);
+            for (int n = 0; n < a.blocks; ++n) {
+                const ternaspmm_step_block& b = blocks[first + n];
+                a.block[n] = StepBlock{static_cast<const uint32_t*>(b.wqkv), static_cast<const uint32_t*>(b.wo), static_cast<const uint32_t*>(b.w13),
+                                       static_cast<const uint32_t*>(b.w2), b.ws_qkv, b.ws_o, b.ws_13, b.ws_down, b.attention_norm, b.attn_sub_norm, b.ffn_norm,
+                                       b.ffn_sub_norm, b.cache_k, b.cache_v};
+            }
+            if (d->M == 1) terna_decode_step_kernel<1, ORDERED><<<grid, threads, 0, st>>>(a);
+            else if (d->M == 2) terna_decode_step_kernel<2, ORDERED><<<grid, threads, 0, st>>>(a);
+            else terna_decode_step_kernel<4, ORDERED><<<grid, threads, 0, st>>>(a);
         }
-        if (d->M == 1) terna_decode_step_kernel<1><<<dim3(kStepGroups), dim3(kStepThreads), 0, st>>>(a);
-        else if (d->M == 2) terna_decode_step_kernel<2><<<dim3(kStepGroups), dim3(kStepThreads), 0, st>>>(a);
-        else terna_decode_step_kernel<4><<<dim3(kStepGroups), dim3(kStepThreads), 0, st>>>(a);
-    }
+    };
+    launches(std::false_type{});
+    launches(std::true_type{});                  // (behind all of them: one that gave up left nothing for the next)
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) die("ternaspmm_decode_step", e, __LINE__);
     return 0;
+}
+
+}  // namespace
+
+extern "C" {
+
+long long ternaspmm_decode_step_bytes(const ternaspmm_step_desc* d)
+{
+    if (d == nullptr || !step_shape_ok(*d)) return -1;
+    const long long count = ternaspmm_row_stats_count(d->dim);
+    return kStepControlBytes + static_cast<long long>(d->layers) * exchange_of(*d).bytes + up(2ll * d->M * d->dim) + up(8ll * d->M * count) + up(4ll * d->M * d->head_dim);
+}
+
+int ternaspmm_decode_step(const ternaspmm_step_desc* d, const ternaspmm_step_block* blocks, const long long* tokens, const long long* pos,
+                          const terna_bf16* embedding, const float* rope_table, void* scratch, terna_bf16* x_out, terna_stream stream)
+{
+    return enqueue_step(d, blocks, tokens, pos, embedding, rope_table, scratch, x_out, kStepGroups, kStepPatience, stream);
+}
+
+int ternaspmm_probe_decode_step(const ternaspmm_step_desc* d, const ternaspmm_step_block* blocks, const long long* tokens, const long long* pos,
+                                const terna_bf16* embedding, const float* rope_table, void* scratch, terna_bf16* x_out, int workgroups, int polls, terna_stream stream)
+{
+    if (workgroups < 1 || workgroups > kStepGroups || polls < 0 || polls > kStepPatience) return -1;
+    return enqueue_step(d, blocks, tokens, pos, embedding, rope_table, scratch, x_out, workgroups, polls, stream);
 }
 
 }  // extern "C"

@@ -20,11 +20,15 @@
 //   * the weights come into the XCD's L2 two phases ahead (step_prefetch) and into registers, partly expanded, during the wait;
 //   * an element takes four instructions to its int8 byte (quant_rounded4).
 //
-// Waiting is safe.  All workgroups are resident together: a workgroup takes a quarter of a CU at most (four waves of up
-// to 128 registers, 40 KB of LDS), the launcher checks that the device holds four grids at once, and the runtime runs kernels
-// of at most four queues side by side -- so also when several streams run such steps.  Every wait ends all the same: after
-// kStepPatience of wall clock a wave gives up, says so to all others (StepControl::alive), and the rest of the launch runs
-// through without waiting, on what it finds: NaN, which reaches the outputs.
+// Waiting is safe.  All workgroups are resident together as a rule: a workgroup takes a quarter of a CU at most (four waves of
+// up to 128 registers, 40 KB of LDS), the launcher checks that the device holds four grids at once, and the runtime runs
+// kernels of at most four queues of a process side by side.  Where they are not -- more steps at once, of several processes or
+// on streams of several priorities; a captured step replayed on a stream with few CUs -- the waits end: after kStepPatience
+// polls a wave gives up, says so to all others (StepControl::alive), and the rest of the launch runs through without
+// waiting, on what it finds.  The launch behind it (ORDERED) then does the step again, from the same inputs and over everything the
+// first wrote, in a way that needs no workgroups side by side: a few of them take the units of work one by one in the order
+// in which they depend on each other (step_ticket), so that whatever one waits for is held by a workgroup that runs (30 blocks of
+// the 2B shape, 384 slots: 3 ms with one sequence, 4 with four).  Where nobody gave up it ends at once, 3 us.
 //
 // Every result has the bits of the launches this replaces: integer sums, and for all that is rounded the same operations in
 // the same order (the partial statistics of 16 columns are formed by the consumer instead of the producer).
@@ -38,12 +42,11 @@
 
 #include "attention_kernel.h"
 #include "chain_chunk_kernel.h"
+#include "step_layout.h"
 
 namespace terna {
 
-constexpr int kStepWaves = 4, kStepThreads = 64 * kStepWaves, kStepGroups = 256;
 constexpr int kStepMaxBlocks = 32;               // blocks per launch: their pointers travel as arguments (4 KB)
-constexpr int kStepHeadDim = 128;
 constexpr int kStepMaxSplits = 8;                // splits of the cache, one sequence; four at a time are merged
 constexpr int kStepRecord = (kStepHeadDim + 4) * 4;      // bytes a (head, split) hands over: 128 sums, maximum, sum of numerators
 // Slots of a cache that is not split; of a split.  Every (sequence, head, half) walks its whole prefix, so the lines lie where that takes as
@@ -55,7 +58,12 @@ constexpr int kStepMaxSplitSlots = 1024;
 constexpr int kStepWideTiles = 112;              // tiles of the down projection's K: ffn <= 7168
 constexpr int kStepTiles = 40;                   // tiles of the other linears' K: <= 2560
 constexpr uint32_t kStepEmpty = 0xffffffffu;
-constexpr int kStepPatience = 4 * 1526;           // 4 s, in 65536 ticks of the 100 MHz clock
+// Polls of one wait before a wave gives up: 20 ms where they take 0.15 us (an idle chip), more on a busy one -- longer than the kernels
+// of other streams hold a part of the grid back.  Polls and not wall clock: a process that was suspended has not waited.
+constexpr int kStepPatience = 1 << 17;
+constexpr int kStepOrderedGroups = 64;           // workgroups that do a step in order
+constexpr int kStepOrderedPolls = 1 << 26;       // ... whose waits end too (10 s and more, for work of microseconds)
+constexpr int kStepControlBytes = 512;           // scratch in front of the exchange: word 0 StepArgs::alive, 1 + 2 i and 2 + 2 i the tickets of launch i
 constexpr int kDeviceScope = 16;                 // cache policy of a raw buffer access: sc1
 
 struct StepBlock {
@@ -73,12 +81,13 @@ struct StepExchange {
 struct StepArgs {
     char* exchange;                              // [blocks][StepExchange::bytes]
     uint32_t* alive;                             // 0xffffffff, 0 once a wave has given up
+    uint32_t* tickets;                           // ORDERED: [0] taken, [1] done, both from 0xffffffff
     const uint16_t* x;                           // the stream in front of the first block, no word 0xffffffff
     const float2* stats;                         // its partials under the first block's norm, [M][stats_count]; nullptr: formed here
     uint16_t* x_out;                             // the stream behind the last block
     const long long* pos;
     const float *cosv, *sinv;
-    int blocks, M, dim, ffn, H, KV, S, SP, per_seq, stats_count, quant_mode, ws_qkv, ws_o, ws_2;
+    int blocks, M, dim, ffn, H, KV, S, SP, per_seq, stats_count, quant_mode, ws_qkv, ws_o, ws_2, patience;
     float eps, scale;
     StepExchange at;
     StepBlock block[kStepMaxBlocks];
@@ -91,14 +100,13 @@ __device__ __forceinline__ uint32_t step_word(uint32_t v) { return v < kStepEmpt
 
 struct StepControl {
     uint32_t* alive;
+    int patience;
     bool gave_up;
 
     // every 256 polls of a wave
-    __device__ void check(int& since)
+    __device__ void check(int polls)
     {
-        const int now = __builtin_amdgcn_readfirstlane(static_cast<int>(__builtin_amdgcn_s_memrealtime() >> 16));
-        if (since == 0) since = now;
-        const bool late = now - since > kStepPatience;
+        const bool late = polls > patience;
         if (late) __hip_atomic_store(alive, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         gave_up = late || __builtin_amdgcn_readfirstlane(__hip_atomic_load(alive, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0;
     }
@@ -106,7 +114,6 @@ struct StepControl {
     template <typename Load, typename There, typename Meanwhile>
     __device__ __forceinline__ void await(Load load, There there, Meanwhile meanwhile)
     {
-        int since = 0;
         load();
         asm volatile("" ::: "memory");
         meanwhile();
@@ -115,7 +122,7 @@ struct StepControl {
             asm volatile("" ::: "memory");       // the loads are made again
             load();
             all = __all(there());
-            if ((n & 255) == 0) check(since);
+            if ((n & 255) == 0) check(n);
         }
         asm volatile("" ::: "memory");
     }
@@ -456,7 +463,7 @@ __device__ __forceinline__ void step_fetch_rows(StepControl& ctl, const void* fr
 struct StepMerge {
     float w[kStepMaxSplits], sum[kStepMaxSplits];
 };
-template <typename Op, typename Meanwhile>
+template <typename Op, bool ORDERED, typename Meanwhile>
 __device__ __forceinline__ void step_fetch_merged(StepControl& ctl, const void* from, int H, int SP, u32x2 (&xr)[Op::ROUNDS], StepMerge (&merge)[8], int lane, int wave, Meanwhile meanwhile)
 {
     const int K = H * kStepHeadDim, first = wave * Op::TPW, ktiles = K >> 6, head0 = first >> 1;
@@ -469,7 +476,8 @@ __device__ __forceinline__ void step_fetch_merged(StepControl& ctl, const void* 
         ml = step_load8(rp, own_head < H && own_split < SP ? (own_head * SP + own_split) * kStepRecord + kStepHeadDim * 4 : kBufferOutOfRange);
     }, [&]() { return step_largest(ml) != kStepEmpty; }, meanwhile);
     // ... then the rest, which by now is mostly there, through the L2 that twenty workgroups share; a line that came too early
-    // shows its empty words and is loaded again past it.
+    // shows its empty words and is loaded again past it.  (ORDERED: past it at once, the words were not cleared.)
+    using First = std::integral_constant<int, ORDERED ? kDeviceScope : 0>;
     u32x4 o[Op::ROUNDS][4];
     auto load = [&](int j0, auto scope) {
 #pragma unroll
@@ -489,7 +497,7 @@ __device__ __forceinline__ void step_fetch_merged(StepControl& ctl, const void* 
             for (int j = 0; j < 4; ++j) top = step_max(top, step_largest(o[r][j]));
         return top != kStepEmpty;
     };
-    load(0, std::integral_constant<int, 0>{});
+    load(0, First{});
     {
         const float m = own_split < SP ? __uint_as_float(ml.x) : -INFINITY;
         const float w = __expf(m - group_reduce<8, true>(m));          // a split that is empty or not there: exp(-inf) = 0
@@ -514,7 +522,7 @@ __device__ __forceinline__ void step_fetch_merged(StepControl& ctl, const void* 
     };
     add(0);
     if (SP > 4) {
-        load(4, std::integral_constant<int, 0>{});
+        load(4, First{});
         if (!__all(there())) ctl.await([&]() { load(4, std::integral_constant<int, kDeviceScope>{}); }, there);
         add(4);
     }
@@ -526,20 +534,6 @@ __device__ __forceinline__ void step_fetch_merged(StepControl& ctl, const void* 
         for (int e = 0; e < 4; ++e) merged[e] = t < Op::TPW && first + t < ktiles ? num[r][e] / den[r] : 0.0f;
         xr[r] = u32x2{pack_bf16x2(merged[0], merged[1]), pack_bf16x2(merged[2], merged[3])};
     }
-}
-
-// Attention units over the workgroups, from the last one downwards: the H / KV heads of a kv group read the same keys and values
-// and sit on one XCD (workgroups go to the eight of them round robin).  A group is a (sequence, kv head), or (one sequence) a
-// (kv head, split); per: its workgroups.  group < 0: no unit.
-struct StepUnit {
-    int group, head;                             // head within the group (several sequences: 2 head + half)
-};
-__host__ __device__ inline int step_unit_groups(int groups, int per) { return 8 * per * ((groups + 7) / 8); }      // workgroups they take
-__device__ __forceinline__ StepUnit step_unit(int w, int groups, int per)
-{
-    const int u = kStepGroups - 1 - w;
-    const int q = u >> 3, group = 8 * (q / per) + (u & 7);
-    return {u < step_unit_groups(groups, per) && group < groups ? group : -1, q % per};
 }
 
 // RoPE, cache write and attention of one unit: terna_decode_attention_kernel's arithmetic -- unsplit with eight waves (several
@@ -792,9 +786,12 @@ __device__ __forceinline__ void step_prefetch(const void* base, int bytes, int l
     asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"s"(lds_words), "v"((line + lane) * 128), "s"(range) : "memory");
 }
 
-template <int MR>
-__global__ __launch_bounds__(kStepThreads, 4) void terna_decode_step_kernel(const StepArgs a)
+template <int MR, bool ORDERED>
+__global__ __launch_bounds__(kStepThreads, ORDERED ? 2 : 4) void terna_decode_step_kernel(const StepArgs a)
 {
+    if constexpr (ORDERED) {
+        if (__hip_atomic_load(a.alive, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return;     // the step is done
+    }
     using Lds = StepLds<MR>;
     constexpr bool QUANT = MR >= 2;              // the down projection's rows quantised by a phase of its own
     __shared__ __align__(16) uint8_t lds[Lds::kBytes];
@@ -806,16 +803,19 @@ __global__ __launch_bounds__(kStepThreads, 4) void terna_decode_step_kernel(cons
     __shared__ uint16_t weight_s[kStepMaxBlocks][16];             // QKV, O, gate+up, down: four each
     __shared__ uint32_t dummy_s[64];
     __shared__ float2 nowhere_s;
+    __shared__ StepTicket ticket_s[1];           // (ORDERED)
     // What the lanes of wave 0 keep for the columns they finish -- row lane >> 4, column lane & 15 of band w: the residual stream, and the
     // weight-scale groups of QKV, O and down.  (In registers they would be spilled, and a load of a spilled register waits behind
     // the prefetches like any other.)
     __shared__ float stream_s[64];
     __shared__ uint8_t group_s[3][64];
     __shared__ __align__(16) StepShape shape_s;
-    static_assert(sizeof(lds) + sizeof(scale_s) + sizeof(red) + sizeof(merge_s) + sizeof(block_s) + sizeof(weight_s) + sizeof(dummy_s) + sizeof(stream_s) + sizeof(group_s) + 64 <= 40 * 1024, "a quarter of a CU");
-    const int wave0 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), w0 = blockIdx.x;
+    static_assert(sizeof(lds) + sizeof(scale_s) + sizeof(red) + sizeof(merge_s) + sizeof(block_s) + sizeof(weight_s) + sizeof(dummy_s) + sizeof(stream_s) + sizeof(group_s) + 96 <= 40 * 1024, "a quarter of a CU");
+    const int wave0 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int w0 = blockIdx.x;                         // (ORDERED: of the unit that is being done)
     if (threadIdx.x == 0) shape_s = StepShape{a.M, a.dim, a.ffn, a.H, a.KV, a.SP, a.quant_mode, a.eps};
     __syncthreads();
+    auto uniform = [](int v) { return ORDERED ? __builtin_amdgcn_readfirstlane(v) : v; };      // (what take() changes)
     auto phase = [&]() {
         StepPhase p;
         p.M = __builtin_amdgcn_readfirstlane(shape_s.M);
@@ -828,7 +828,7 @@ __global__ __launch_bounds__(kStepThreads, 4) void terna_decode_step_kernel(cons
         p.eps = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(shape_s.eps)));
         p.lane = step_lane();
         p.wave = step_uniform(wave0);
-        p.w = step_uniform(w0);
+        p.w = step_uniform(uniform(w0));
         p.wide = p.H * kStepHeadDim;
         p.qkv_n = (p.H + 2 * p.KV) * kStepHeadDim;
         return p;
@@ -836,24 +836,32 @@ __global__ __launch_bounds__(kStepThreads, 4) void terna_decode_step_kernel(cons
     bool has_qkv, has_out, has_gate, has_unit, has_quant;
     StepUnit unit;
     int seen = 0;                                // slots of the unit's prefix; negative: the position lies outside the cache (clamped)
-    {
-        const StepPhase p = phase();
-        const int fin_n = 16 * p.w + (p.lane & 15);
+    auto find_unit = [&](const StepPhase& p) {
         unit = step_unit(p.w, MR == 1 ? p.KV * p.SP : p.M * p.KV, p.H / p.KV * (MR == 1 ? 1 : 2));
-        has_qkv = p.w < p.qkv_n >> 4;
-        has_out = p.w < p.dim >> 4;
-        has_gate = 4 * p.w < p.ffn >> 3;
         has_unit = unit.group >= 0;
         if (has_unit) {                          // (once: a load behind the prefetches would wait for them)
             const long long p0 = a.pos[MR == 1 || !a.per_seq ? 0 : unit.group / p.KV];
             seen = __builtin_amdgcn_readfirstlane(p0 < 0 ? -1 : p0 >= a.S ? -a.S : static_cast<int>(p0) + 1);
         }
-        has_quant = QUANT && kStepGroups - 1 - p.w < 4 * p.M;
-        if (p.wave == 0) {
-            group_s[0][p.lane] = has_qkv && a.ws_qkv != 1 ? ws_group_decode(fin_n, p.qkv_n, a.ws_qkv) : 0;
-            group_s[1][p.lane] = has_out && a.ws_o != 1 ? ws_group_decode(fin_n, p.dim, a.ws_o) : 0;
-            group_s[2][p.lane] = has_out && a.ws_2 != 1 ? ws_group_decode(fin_n, p.dim, a.ws_2) : 0;
-            stream_s[p.lane] = has_out && (p.lane >> 4) < p.M ? bf16_bits_to_float(a.x[(p.lane >> 4) * p.dim + fin_n]) : 0.0f;
+    };
+    auto find_groups = [&](const StepPhase& p, int fin_n) {
+        group_s[0][p.lane] = has_qkv && a.ws_qkv != 1 ? ws_group_decode(fin_n, p.qkv_n, a.ws_qkv) : 0;
+        group_s[1][p.lane] = has_out && a.ws_o != 1 ? ws_group_decode(fin_n, p.dim, a.ws_o) : 0;
+        group_s[2][p.lane] = has_out && a.ws_2 != 1 ? ws_group_decode(fin_n, p.dim, a.ws_2) : 0;
+    };
+    {
+        const StepPhase p = phase();
+        if constexpr (!ORDERED) {
+            const int fin_n = 16 * p.w + (p.lane & 15);
+            has_qkv = p.w < p.qkv_n >> 4;
+            has_out = p.w < p.dim >> 4;
+            has_gate = 4 * p.w < p.ffn >> 3;
+            find_unit(p);
+            has_quant = QUANT && kStepGroups - 1 - p.w < 4 * p.M;
+            if (p.wave == 0) {
+                find_groups(p, fin_n);
+                stream_s[p.lane] = has_out && (p.lane >> 4) < p.M ? bf16_bits_to_float(a.x[(p.lane >> 4) * p.dim + fin_n]) : 0.0f;
+            }
         }
         const int tid = 64 * p.wave + p.lane;
         const uint32_t* from = reinterpret_cast<const uint32_t*>(a.block);
@@ -870,7 +878,7 @@ __global__ __launch_bounds__(kStepThreads, 4) void terna_decode_step_kernel(cons
         }
         __syncthreads();
     }
-    StepControl ctl{a.alive, false};
+    StepControl ctl{a.alive, a.patience, false}; // (ORDERED: take() has waited, every poll finds its words)
     const uint32_t dummy = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint32_t*)dummy_s));
 
     // (operands expanded ahead of the wait: as many as the registers of the phase hold)
@@ -892,11 +900,50 @@ __global__ __launch_bounds__(kStepThreads, 4) void terna_decode_step_kernel(cons
     // The next block's matrix of this phase (this workgroup's bands of it) and its norm weights (a few lines by every workgroup of
     // the XCD), right behind a wait: in front of one its polls would return behind the lines.
     auto prefetch = [&](const StepPhase& p, const uint32_t* packed, int band0, int bands, const uint16_t* norm_w, int K) {
+        if constexpr (ORDERED) return;
         const int bytes = bands * (K >> 6) * 256;
         for (int l = p.wave; 8192 * l < bytes; l += kStepWaves) step_prefetch(packed + static_cast<size_t>(band0) * K, bytes, 64 * l, dummy, p.lane);
         if (p.wave == kStepWaves - 1) step_prefetch(norm_w, 2 * K, p.lane < 4 ? 4 * (p.w >> 3) : 1 << 20, dummy, p.lane);
     };
-    for (int n = 0; n < a.blocks; ++n) {
+    // ORDERED: the next unit, of which exactly one of the phases below is this workgroup's; its block, or all of them where
+    // there is none.  The stream of a band's columns is what its last phase handed over.
+    bool out_now = false, down_now = false;
+    auto take = [&](bool first) {
+        uint32_t* const tickets = a.tickets;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");          // this wave's outputs have arrived
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            if (!first) __hip_atomic_fetch_add(tickets + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const int mine = static_cast<int>(__hip_atomic_fetch_add(tickets, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1);
+            const StepTicket t = step_ticket(mine, a.M, a.dim, a.ffn, a.H, a.KV, a.SP);
+            bool ready = t.block >= a.blocks;
+            for (int polls = 0; !ready && polls < kStepOrderedPolls; ++polls)
+                ready = static_cast<int>(__hip_atomic_load(tickets + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1) >= t.before;
+            ticket_s[0] = StepTicket{ready ? t.block : a.blocks, t.kind, t.w, t.before};
+        }
+        __syncthreads();
+        asm volatile("" ::: "memory");
+        const int block = __builtin_amdgcn_readfirstlane(ticket_s[0].block), kind = __builtin_amdgcn_readfirstlane(ticket_s[0].kind);
+        if (block >= a.blocks) return block;
+        w0 = __builtin_amdgcn_readfirstlane(ticket_s[0].w);
+        has_qkv = kind == STEP_QKV, out_now = kind == STEP_OUT, has_gate = kind == STEP_GATE, has_quant = kind == STEP_QUANT, down_now = kind == STEP_DOWN;
+        has_out = out_now || down_now, has_unit = false;
+        const StepPhase p = phase();
+        if (kind == STEP_ATTENTION) find_unit(p);
+        if (p.wave == 0) {
+            const int fin_n = 16 * p.w + (p.lane & 15);
+            find_groups(p, fin_n);
+            const char* from = a.exchange + static_cast<size_t>(block) * a.at.bytes;
+            from = down_now ? from + a.at.mid : block == 0 ? reinterpret_cast<const char*>(a.x) : from - a.at.bytes + a.at.out;
+            const __amdgpu_buffer_rsrc_t rx = make_raw_buffer(from, static_cast<uint32_t>(p.M) * p.dim * 2u);
+            const bool mine = has_out && (p.lane >> 4) < p.M;
+            const uint16_t bits = __builtin_amdgcn_raw_buffer_load_b16(rx, mine ? ((p.lane >> 4) * p.dim + fin_n) * 2 : kBufferOutOfRange, 0, kDeviceScope);
+            stream_s[p.lane] = bf16_bits_to_float(bits);
+        }
+        __syncthreads();
+        return block;
+    };
+    for (int n = ORDERED ? take(true) : 0; n < a.blocks; n = ORDERED ? take(false) : n + 1) {
         char* ex = a.exchange + static_cast<size_t>(n) * a.at.bytes;
         const int ahead = n + 1 < a.blocks ? n + 1 : n;
         // ---- QKV
@@ -909,7 +956,7 @@ __global__ __launch_bounds__(kStepThreads, 4) void terna_decode_step_kernel(cons
             if (has_out) prefetch(p, pointer(block_s[n].wo), p.w, 1, pointer(block_s[n].attn_sub_norm), p.wide);
             if (has_gate) prefetch(p, pointer(block_s[n].w13), 4 * p.w, 4, pointer(block_s[n].ffn_norm), p.dim);
             if (!has_gate) prefetch(p, pointer(block_s[ahead].wqkv), p.w, 1, pointer(block_s[ahead].attention_norm), p.dim);
-            if (has_unit) {                      // this block's keys and values, a share by each of the workgroups that read them
+            if (!ORDERED && has_unit) {          // this block's keys and values, a share by each of the workgroups that read them
                 const int b = MR == 1 ? 0 : unit.group / p.KV, kvh = MR == 1 ? unit.group / p.SP : unit.group - b * p.KV, per = p.H / p.KV;
                 const int bytes = 2 * kStepHeadDim * (seen < 0 ? -seen : seen);
                 const size_t at = (static_cast<size_t>(b) * p.KV + kvh) * a.S * kStepHeadDim;
@@ -929,16 +976,16 @@ __global__ __launch_bounds__(kStepThreads, 4) void terna_decode_step_kernel(cons
         // ---- attention
         if (has_unit) {
             const StepPhase p = phase();
-            step_attention<MR>(ctl, a, p, pointer(block_s[n].cache_k), pointer(block_s[n].cache_v), ex + a.at.qkv, ex + a.at.attention, StepUnit{step_uniform(unit.group), step_uniform(unit.head)},
+            step_attention<MR>(ctl, a, p, pointer(block_s[n].cache_k), pointer(block_s[n].cache_v), ex + a.at.qkv, ex + a.at.attention, StepUnit{step_uniform(uniform(unit.group)), step_uniform(uniform(unit.head))},
                                seen < 0 ? -seen : seen, seen > 0, lds, red);
         }
         // ---- O projection, added to the stream
-        if (has_out) {
+        if (ORDERED ? out_now : has_out) {
             const StepPhase p = phase();
             Out op;
             op.request(pointer(block_s[n].wo), p.dim >> 4, p.w, p.wide, pointer(block_s[n].attn_sub_norm), p.lane, p.wave);
             u32x2 xr[Out::ROUNDS];
-            if constexpr (MR == 1) step_fetch_merged<Out>(ctl, ex + a.at.attention, p.H, p.SP, xr, merge_s[p.wave], p.lane, p.wave, [&] { op.expand(); });
+            if constexpr (MR == 1) step_fetch_merged<Out, ORDERED>(ctl, ex + a.at.attention, p.H, p.SP, xr, merge_s[p.wave], p.lane, p.wave, [&] { op.expand(); });
             else step_fetch_rows<MR, Out>(ctl, ex + a.at.attention, p.M, p.wide, xr, p.lane, p.wave, [&] { op.expand(); });
             prefetch(p, pointer(block_s[n].w2), p.w, 1, pointer(block_s[n].ffn_sub_norm), p.ffn);
             const float s = step_norm_linear<MR, MR == 1 ? STEP_CHUNKS : STEP_HEADS, kStepTiles, 1>(op, xr, p, p.wide, nullptr, 0, lds, &nowhere_s, scale_s);
@@ -974,7 +1021,7 @@ __global__ __launch_bounds__(kStepThreads, 4) void terna_decode_step_kernel(cons
                 step_quantise<MR>(ctl, p, pointer(block_s[n].ffn_sub_norm), ex + a.at.inner, ex + a.at.quantised, ex + a.at.scales, kStepGroups - 1 - p.w, lds, &nowhere_s);
             }
         }
-        if (has_out) {
+        if (ORDERED ? down_now : has_out) {
             const StepPhase p = phase();
             Down op;
             op.request(pointer(block_s[n].w2), p.dim >> 4, p.w, p.ffn, pointer(block_s[n].ffn_sub_norm), p.lane, p.wave);

@@ -1,0 +1,48 @@
+// Who does what in a decode step in one launch (step_kernel.h): integer rules alone, so that they can be checked without a GPU.
+#pragma once
+
+#if defined(__HIP__)
+#define TERNA_STEP_FUNCTION __host__ __device__ inline
+#else
+#define TERNA_STEP_FUNCTION inline
+#endif
+
+namespace terna {
+
+constexpr int kStepWaves = 4, kStepThreads = 64 * kStepWaves, kStepGroups = 256;
+constexpr int kStepHeadDim = 128;
+
+// Attention units over the workgroups, from the last one downwards: the H / KV heads of a kv group read the same keys and values
+// and sit on one XCD (workgroups go to the eight of them round robin).  A group is a (sequence, kv head), or (one sequence) a
+// (kv head, split); per: its workgroups.  group < 0: no unit.
+struct StepUnit {
+    int group, head;                             // head within the group (several sequences: 2 head + half)
+};
+TERNA_STEP_FUNCTION int step_unit_groups(int groups, int per) { return 8 * per * ((groups + 7) / 8); }      // workgroups they take
+TERNA_STEP_FUNCTION StepUnit step_unit(int w, int groups, int per)
+{
+    const int u = kStepGroups - 1 - w;
+    const int q = u >> 3, group = 8 * (q / per) + (u & 7);
+    return {u < step_unit_groups(groups, per) && group < groups ? group : -1, q % per};
+}
+
+// The step's units of work in the order of their dependences: those of a phase, then those of the next, block by block.  A
+// workgroup of the ORDERED launch takes one after the other from a counter; a unit may start once as many are done as stand in front of
+// its phase (a later one cannot be among them).
+enum StepKind { STEP_QKV, STEP_ATTENTION, STEP_OUT, STEP_GATE, STEP_QUANT, STEP_DOWN, STEP_KINDS };
+struct StepTicket {
+    int block, kind, w, before;                  // w: the workgroup of the other launch that does this unit; before: units in front of the phase
+};
+TERNA_STEP_FUNCTION StepTicket step_ticket(int ticket, int M, int dim, int ffn, int H, int KV, int SP)
+{
+    const int bands = (H + 2 * KV) * kStepHeadDim / 16, units = step_unit_groups(M == 1 ? KV * SP : M * KV, H / KV * (M == 1 ? 1 : 2));
+    const int count[STEP_KINDS] = {bands, units, dim >> 4, ((ffn >> 3) + 3) / 4, M == 1 ? 0 : 4 * M, dim >> 4};
+    int all = 0;
+    for (int k = 0; k < STEP_KINDS; ++k) all += count[k];
+    StepTicket t{ticket / all, 0, ticket % all, ticket / all * all};
+    while (t.w >= count[t.kind]) t.w -= count[t.kind], t.before += count[t.kind], ++t.kind;
+    if (t.kind == STEP_ATTENTION || t.kind == STEP_QUANT) t.w = kStepGroups - 1 - t.w;       // these go from the last workgroup downwards
+    return t;
+}
+
+}  // namespace terna

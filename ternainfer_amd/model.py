@@ -553,7 +553,11 @@ class Transformer:
             held[bsz] = torch.zeros(nbytes, dtype=torch.int8, device="cuda")
         return held[bsz]
 
-    # the step as one launch of resident workgroups (whole_step), where the library takes it
+    # The step as one launch of resident workgroups (whole_step), where the library takes it.  Its workgroups wait for each other, which
+    # the library makes sure of for up to four such steps side by side in a process (its hardware queues).  Where a GPU is shared by
+    # more -- five and more processes that decode at once, streams of several priorities, a captured step replayed on a stream with few CUs
+    # -- a step may find a part of its workgroups missing: it is then done again in order, with the same results, 20 ms and more
+    # later.  Set this to False there, on the class or the model: the step is the launches it stands for.
     one_launch_step = True
 
     def whole_step(self, tokens, cache, pos_idx, max_seq):

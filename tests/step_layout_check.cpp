@@ -1,0 +1,74 @@
+// The rules of ternainfer_amd/csrc/step_layout.h, over small and large shapes: built with g++ and run by test_step_layout.py.
+#include <cstdio>
+#include <set>
+#include <tuple>
+#include <vector>
+
+#include "../ternainfer_amd/csrc/step_layout.h"
+
+using namespace terna;
+
+static int failures = 0;
+#define CHECK(cond, ...)                                   \
+    do {                                                   \
+        if (!(cond) && ++failures < 20) {                  \
+            std::printf("%s:%d: %s: ", __FILE__, __LINE__, #cond); \
+            std::printf(__VA_ARGS__);                      \
+            std::printf("\n");                             \
+        }                                                  \
+    } while (0)
+
+struct Shape {
+    int M, dim, ffn, H, KV, SP;
+};
+
+// What a workgroup of the resident launch does (the conditions in its prologue).
+static bool resident_does(const Shape& s, int kind, int w)
+{
+    switch (kind) {
+        case STEP_QKV: return w < (s.H + 2 * s.KV) * kStepHeadDim / 16;
+        case STEP_ATTENTION: return step_unit(w, s.M == 1 ? s.KV * s.SP : s.M * s.KV, s.H / s.KV * (s.M == 1 ? 1 : 2)).group >= 0;
+        case STEP_GATE: return 4 * w < s.ffn >> 3;
+        case STEP_QUANT: return s.M > 1 && kStepGroups - 1 - w < 4 * s.M;
+        default: return w < s.dim >> 4;
+    }
+}
+
+// Every unit of the resident launch is a ticket, once; the tickets of a phase stand together, behind all it depends on.
+static void check_tickets(const Shape& s)
+{
+    std::set<std::tuple<int, int, int>> seen;
+    int previous = -1, start = 0, t = 0;
+    for (;; ++t) {
+        const StepTicket k = step_ticket(t, s.M, s.dim, s.ffn, s.H, s.KV, s.SP);
+        if (k.block >= 2) break;
+        const int phase = k.block * STEP_KINDS + k.kind;
+        CHECK(phase >= previous, "ticket %d: phase %d behind %d", t, phase, previous);
+        if (phase != previous) start = t;
+        previous = phase;
+        CHECK(k.before == start, "ticket %d waits for %d, its phase starts at %d", t, k.before, start);
+        CHECK(k.w >= 0 && k.w < kStepGroups, "ticket %d: workgroup %d", t, k.w);
+        CHECK(seen.insert({k.block, k.kind, k.w}).second, "ticket %d: done twice", t);
+        // (units that only fill a round of eight groups are tickets too, with nothing to do)
+        CHECK(k.kind == STEP_ATTENTION || resident_does(s, k.kind, k.w), "ticket %d: kind %d workgroup %d has none", t, k.kind, k.w);
+    }
+    for (int block = 0; block < 2; ++block)
+        for (int kind = 0; kind < STEP_KINDS; ++kind)
+            for (int w = 0; w < kStepGroups; ++w)
+                CHECK(!resident_does(s, kind, w) || seen.count({block, kind, w}), "block %d kind %d workgroup %d is no ticket", block, kind, w);
+}
+
+int main()
+{
+    std::vector<Shape> shapes;
+    for (int M = 1; M <= 4; ++M)
+        for (int SP : {1, 2, 4, 8})
+            for (const auto& [H, KV, dim, ffn] : std::vector<std::tuple<int, int, int, int>>{
+                     {20, 5, 2560, 6912}, {20, 5, 2560, 7168}, {2, 1, 256, 192}, {9, 3, 1152, 1088}, {5, 5, 640, 64}, {1, 1, 64, 64}, {16, 4, 2048, 5632}, {20, 1, 192, 6976}}) {
+                const Shape s{M, dim, ffn, H, KV, SP};
+                if ((M == 1) == (SP > 1) && step_unit_groups(M == 1 ? KV * SP : M * KV, H / KV * (M == 1 ? 1 : 2)) <= kStepGroups) shapes.push_back(s);
+            }
+    for (const Shape& s : shapes) check_tickets(s);
+    if (failures == 0) std::printf("step layout ok: %zu shapes\n", shapes.size());
+    return failures != 0;
+}

@@ -1,5 +1,7 @@
 """The decode step of one to four sequences in one launch (ternaspmm_decode_step) against the launches it stands for: the same
 bits in the logits and in the caches, whatever the shape, the prefix, the quantisation mode or the values."""
+import ctypes
+
 import pytest
 import torch
 
@@ -190,3 +192,68 @@ def test_split_attention_steps_of_two_streams_at_once():
         torch.cuda.synchronize()
         for _, _, logits, want, *_ in runs:
             assert same(logits, want)
+
+
+class StepBlock(ctypes.Structure):
+    """ternaspmm_step_block of include/ternaspmm.h."""
+    _fields_ = [(n, ctypes.c_void_p) for n in ("wqkv", "wo", "w13", "w2", "ws_qkv", "ws_o", "ws_13", "ws_down", "attention_norm", "attn_sub_norm", "ffn_norm",
+                                               "ffn_sub_norm", "cache_k", "cache_v")]
+
+
+class StepDesc(ctypes.Structure):
+    """ternaspmm_step_desc of include/ternaspmm.h."""
+    _fields_ = [(n, ctypes.c_int) for n in ("layers", "M", "dim", "ffn", "heads", "kv_heads", "head_dim", "slots", "splits", "per_sequence", "vocab",
+                                            "ws_num_qkv", "ws_num_o", "ws_num_down")] + [("eps", ctypes.c_float), ("scale", ctypes.c_float)]
+
+
+def raw_step(model, whole, tokens, pos, workgroups, polls):
+    """(call, stream behind the last block): ternaspmm_probe_decode_step on the buffers of `state`; call() enqueues it."""
+    a, lib = model.args, _lib.load()
+    m, slots = whole.shape[2], whole.shape[4]
+    b0 = model.layers[0]
+    desc = StepDesc(a.n_layers, m, a.dim, a.ffn_dim, a.n_heads, a.n_kv_heads, a.head_dim, slots,
+                    lib.ternaspmm_attention_partial_splits_kv(1, a.n_heads, a.n_kv_heads, slots) if m == 1 else 1, int(pos.numel() == m and m > 1), a.vocab_size,
+                    b0.wqkv.ws_num, b0.wo.ws_num, b0.w2.ws_num, a.norm_eps, a.head_dim ** -0.5)
+    blocks = (StepBlock * a.n_layers)(*[
+        StepBlock(*(t.data_ptr() for t in (b.wqkv.packed, b.wo.packed, b.gate_up_interleaved(), b.w2.packed, b.wqkv.ws, b.wo.ws, b.w13.ws, b.w2.ws, b.attention_norm,
+                                           b.attn_sub_norm, b.ffn_norm, b.ffn_sub_norm, whole[i, 0], whole[i, 1]))) for i, b in enumerate(model.layers)])
+    table = model.rope_tables(slots, whole.device)
+    scratch = torch.empty(lib.ternaspmm_decode_step_bytes(ctypes.byref(desc)), dtype=torch.uint8, device="cuda")
+    x = torch.zeros((m, a.dim), dtype=torch.bfloat16, device="cuda")
+    held = (blocks, table, scratch, tokens, pos)
+
+    def call():
+        assert held and lib.ternaspmm_probe_decode_step(
+            ctypes.byref(desc), blocks, tokens.data_ptr(), pos.data_ptr(), model.tok_embeddings.data_ptr(), table.data_ptr(), scratch.data_ptr(), x.data_ptr(),
+            workgroups, polls, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    return call, x
+
+
+@pytest.mark.parametrize("shape,layers,m,slots,positions,workgroups,polls", [
+    (TINY, 3, 1, 64, [40], 1, 0), (TINY, 65, 1, 64, [33], 255, 512), (TINY, 65, 3, 30, [29, 2, 11], 16, 0), (SINGLE, 2, 2, 128, [127], 255, 0),
+    (ODD, 3, 1, 200, [130], 100, 256), (ODD, 3, 4, 640, [1, 639, 127, 128], 200, 0), (ODD, 2, 1, 8192, [8191], 64, 0),
+    (WIDE, 2, 1, 384, [255], 240, 1024), (WIDE, 2, 2, 101, [100], 255, 0), (WIDE, 2, 4, 1024, [1023, 640, 0, 777], 128, 0), (WIDE, 2, 1, 384, [300], 256, 0),
+])
+def test_a_step_whose_workgroups_do_not_all_come(shape, layers, m, slots, positions, workgroups, polls):
+    """Fewer workgroups than wait for each other, and waits that end soon: the step is done again in order, with the same bits in
+    the stream and in the caches -- eager, captured, and after a step that went through."""
+    model = build(shape, layers)
+    whole, tokens, pos = state(model, m, slots, positions)
+    fresh = whole.clone()
+    call, x = raw_step(model, whole, tokens, pos, 256, 131072)
+    call()
+    want, want_cache = x.clone(), whole.clone()
+    assert torch.isfinite(want.float()).all()
+    whole.copy_(fresh)
+    short, x = raw_step(model, whole, tokens, pos, workgroups, polls)
+    short()
+    assert same(x, want) and same(whole, want_cache)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        short()
+    for _ in range(3):
+        whole.copy_(fresh)
+        x.fill_(7.0)
+        graph.replay()
+        assert same(x, want) and same(whole, want_cache)
