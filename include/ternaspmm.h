@@ -328,7 +328,8 @@ int ternaspmm_fused_linear(const ternaspmm_fused_linear_desc* desc, terna_stream
 /* Norm + quant_input of h bf16 [M][K] as a launch of its own, from partials a producer left: xq_out int8 [M][K], s_out bf16 [M]
  * -- the values the TERNASPMM_PROLOGUE_STATS prologue forms inside its launch (same order of additions), for row counts at
  * which every consuming workgroup repeating the element-wise work costs more than one more launch (measured on MI355X: the
- * down projection, K = 6912, from three rows on; K = 2560 from nine on).  Returns 0 / -1.  Only enqueues. */
+ * down projection, K = 6912, from three rows on; K = 2560 from nine on).  The scale is that of the maximum `stats` names; values
+ * above it are clamped to -128 .. 127.  Returns 0 / -1.  Only enqueues. */
 int ternaspmm_quant_from_stats(const terna_bf16* h, const float* stats, int stats_count, const terna_bf16* norm_weight, float eps,
                                int8_t* xq_out, terna_bf16* s_out, int M, int K, terna_stream stream);
 

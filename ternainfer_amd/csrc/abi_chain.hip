@@ -126,7 +126,7 @@ __global__ __launch_bounds__(256) void terna_quant_stats_kernel(const uint16_t* 
     if (!in) return;
     const uint32_t hd[4] = {hv.x, hv.y, hv.z, hv.w}, wd[4] = {wv.x, wv.y, wv.z, wv.w};
     uint32_t d[2];
-    chain_quantise<8>(hd, wd, rstd, s, quant_mode, d);
+    chain_quantise<8, true, true>(hd, wd, rstd, s, quant_mode, d);
     *reinterpret_cast<u32x2*>(xq_out + row * K + c) = u32x2{d[0], d[1]};
 }
 

@@ -73,8 +73,8 @@ __device__ __forceinline__ void chain_reduce_partials(const float2 (&part)[PN], 
     }
 }
 
-// NE (4 or 8) columns of one row: norm (NORM) + quantisation, packed int8 (NE / 4 dwords).
-template <int NE, bool NORM = true>
+// NE (4 or 8) columns of one row: norm (NORM) + quantisation, packed int8 (NE / 4 dwords).  BOUNDED: the row's maximum is a caller's.
+template <int NE, bool NORM = true, bool BOUNDED = false>
 __device__ __forceinline__ void chain_quantise(const uint32_t (&hraw)[NE / 2], const uint32_t (&wraw)[NE / 2], float rstd, float s_mul, int quant_mode,
                                                uint32_t (&d)[NE / 4])
 {
@@ -90,7 +90,7 @@ __device__ __forceinline__ void chain_quantise(const uint32_t (&hraw)[NE / 2], c
     }
     if (quant_mode == QUANT_ROUNDED) {                       // uniform: one branch, not one per element
 #pragma unroll
-        for (int j = 0; j < NE / 4; ++j) d[j] = quant_rounded4(f[4 * j], f[4 * j + 1], f[4 * j + 2], f[4 * j + 3], s_mul);
+        for (int j = 0; j < NE / 4; ++j) d[j] = quant_rounded4<BOUNDED>(f[4 * j], f[4 * j + 1], f[4 * j + 2], f[4 * j + 3], s_mul);
         return;
     }
 #pragma unroll
@@ -332,7 +332,7 @@ __global__ __launch_bounds__(kChunkWaves * 64) void terna_chain_chunk_kernel(
                 const int row = xrow0 + RPL * q;
                 const int rc = row < M ? row : 0;
                 uint32_t d[NE / 4];
-                chain_quantise<NE>(xr[t][q], nw[t], rstd_s[rc], smul_s[rc], quant_mode, d);
+                chain_quantise<NE, true, true>(xr[t][q], nw[t], rstd_s[rc], smul_s[rc], quant_mode, d);
                 const bool pub = writer && io.xq_out != nullptr && row < M && col0 + xcol < K && upair[t] == 0;
                 if constexpr (NE == 8) {
                     *reinterpret_cast<u32x2*>(slab + row * kChainSlabPitch + xcol) = u32x2{d[0], d[1]};

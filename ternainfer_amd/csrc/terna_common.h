@@ -121,15 +121,20 @@ __device__ __forceinline__ float quant_value(float x, float s_mul, int mode)
 
 // Four activations in QUANT_ROUNDED, as packed int8: quant_value's integers in half its operations.  bf16 x bf16 is exact in
 // fp32, so one fused multiply-add with 1.5 * 2^23 rounds the product to the integer that stands in the low byte of the
-// sum.  No bound is needed: |x| is at most the row's maximum and the scale within 2^-8 of 127 over it, so |x * s| < 127.5; and
-// where the scale is NaN or 0 (a row that is not finite) the sum is a NaN, whose low byte is 0 (bf16 payloads end above
-// it), or exactly the constant.  Every quantising launch and linear is a little shorter for it: decode step of one sequence 825 ->
+// sum.  No bound is needed where the kernel itself has taken the row's maximum: |x| is at most that and the scale within 2^-8 of 127
+// over it, so |x * s| < 127.5; and where the scale is NaN or 0 (a row that is not finite) the sum is a NaN, whose low byte is
+// 0 (bf16 payloads end above it), or exactly the constant.  BOUNDED: the maximum is a caller's, and a value above it gives 127 or
+// -128 as in quant_value, not the low byte of what it is (an instruction more an element: 8 sequences, 1528 slots 1198 -> 1210 us).  Every quantising launch and linear is a little shorter for it: decode step of one sequence 825 ->
 // 809 us, 1 x 1920 tokens 6741 -> 6592, 5000 x 6912 rows of a module call 101.8 -> 99.5.
+template <bool BOUNDED = false>
 __device__ __forceinline__ uint32_t quant_rounded4(float x0, float x1, float x2, float x3, float s)
 {
-    const float magic = 12582912.0f;
-    const uint32_t b0 = __float_as_uint(fmaf(x0, s, magic)), b1 = __float_as_uint(fmaf(x1, s, magic));
-    const uint32_t b2 = __float_as_uint(fmaf(x2, s, magic)), b3 = __float_as_uint(fmaf(x3, s, magic));
+    const float magic = 12582912.0f, low = s > 0.0f ? magic - 128.0f : magic;
+    auto bits = [&](float x) {
+        const float sum = fmaf(x, s, magic);
+        return __float_as_uint(BOUNDED ? __builtin_amdgcn_fmed3f(sum, low, magic + 127.0f) : sum);
+    };
+    const uint32_t b0 = bits(x0), b1 = bits(x1), b2 = bits(x2), b3 = bits(x3);
     return __builtin_amdgcn_perm(b1, b0, 0x0c0c0400u) | __builtin_amdgcn_perm(b3, b2, 0x04000c0cu);
 }
 

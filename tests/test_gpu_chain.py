@@ -447,3 +447,35 @@ def test_reducing_waves_of_five_to_eight_rows(m, k, count):
     assert torch.equal(inside[3], xq) and torch.equal(inside[4].view(torch.int16), s.view(torch.int16)) and bool(xq.any())
     for a, b in zip(inside[:3], outside[:3]):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])
+@pytest.mark.parametrize("m,k", [(1, 192), (1, 2560), (2, 2560), (4, 6912), (5, 2560), (8, 2560), (8, 6912)])
+def test_a_given_maximum_below_the_rows_own_saturates(m, k, mode):
+    """Partials are a caller's: values above the maximum they name give 127 and -128, and so do an infinity and (-128) a NaN the
+    partials do not show -- the clamp of quant_input (model.py:120-123), in every quantisation mode."""
+    lib = T._lib.load()
+    rng = np.random.default_rng(1260 + k + m)
+    n, count = 256, k // 16
+    h = torch.from_numpy(rng.standard_normal((m, k)).astype(np.float32)).cuda().to(torch.bfloat16)
+    h[:, 1], h[:, k // 2], h[:, k - 1] = float("inf"), float("nan"), float("-inf")
+    ones = torch.ones(k, dtype=torch.bfloat16, device="cuda")
+    stats = torch.zeros((m, count, 2), dtype=torch.float32, device="cuda")
+    stats[:, count // 2, 0] = k                    # the sum of squares: rstd = 1 with eps = 0, so the norm leaves h as it is
+    stats[:, count - 1, 1] = torch.linspace(0.3, 1.0, m, device="cuda")
+    before = lib.ternaspmm_quant_mode(mode)
+    try:
+        xq, s = L.quant_from_stats(h, stats, ones, 0.0)
+        packed = _packed(make_ternary(n, k, 0.4, 1261))
+        inside = L.fused_linear(h, ones, 0.0, packed, _bf(WS), 1, n, k, stats=stats, publish=True)
+    finally:
+        lib.ternaspmm_quant_mode(before)
+    # the products by hand: what multiplies is 127 / max (mode 1 in fp32, else rounded to bf16, which `s` is)
+    mul = s.float()[:, None] if mode != 1 else 127.0 * (1.0 / stats[:, count - 1, 1].to(torch.bfloat16).float())[:, None]
+    p = h.float() * mul
+    if mode == 2:
+        p = p.to(torch.bfloat16).float()
+    want = torch.where(torch.isnan(p), torch.tensor(-128.0, device="cuda"), p.round().clamp(-128, 127)).to(torch.int8)
+    assert int((want == 127).sum()) > m and int((want == -128).sum()) > 2 * m
+    assert torch.equal(xq, want)
+    assert inside is not None and torch.equal(inside[3], want) and torch.equal(inside[4].view(torch.int16), s.view(torch.int16))
