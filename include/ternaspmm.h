@@ -660,7 +660,7 @@ int ternaspmm_plan_reference_call(int int8_activations, int route, int M, int N,
  *                            bounded; uint32 word 512 of `state` counts workgroups that gave up (0 after a good run).
  *                            Returns 0, or -1 when the arguments are refused.
  *   ternaspmm_probe_decode_step  ternaspmm_decode_step with `workgroups` (1 .. 256) of the 256 that wait for each other and
- *                            waits of `polls` polls (0 .. 131072; looked at every 256): the step where the device does not hold them
+ *                            waits of `polls` polls (1 .. 131072; looked at every 256): the step where the device does not hold them
  *                            all, which is done again in order.
  * All only enqueue; time them with events on `stream`. */
 void ternaspmm_probe_empty(terna_stream stream);

@@ -33,6 +33,7 @@ compile abi_chain.hip abi_chain.o
 compile abi_attention.hip abi_attention.o
 # the step's phases share no loop-invariant worth a register that one of them would then spill
 compile abi_step.hip abi_step.o -mllvm -disable-machine-licm
+compile launch_step_ordered.hip launch_step_ordered.o -mllvm -disable-machine-licm
 # accumulators of the prompt-pass attention in ordinary vector registers (they are rescaled between matrix instructions)
 compile abi_prefill_attention.hip abi_prefill_attention.o -mllvm -amdgpu-mfma-vgpr-form
 compile abi_head.hip abi_head.o

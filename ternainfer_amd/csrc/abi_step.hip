@@ -18,8 +18,9 @@ namespace {
 
 constexpr int kClearGroups = 512;
 
-// In front of the step: its inputs (the first B workgroups), and the exchange buffer cleared to "not there yet".
-__global__ __launch_bounds__(256) void terna_step_begin_kernel(const StepInputs in, int B, u32x4* clear, long long vecs)
+// In front of the step: its inputs (the first B workgroups), and the exchange buffer cleared to "not there yet"; its first word
+// (StepArgs::alive) is what a wait may take.
+__global__ __launch_bounds__(256) void terna_step_begin_kernel(const StepInputs in, int B, u32x4* clear, long long vecs, uint32_t patience)
 {
     const int b = blockIdx.x;
     if (b < B) {
@@ -27,7 +28,7 @@ __global__ __launch_bounds__(256) void terna_step_begin_kernel(const StepInputs 
         return;
     }
     for (long long v = static_cast<long long>(b - B) * 256 + threadIdx.x; v < vecs; v += static_cast<long long>(gridDim.x - B) * 256)
-        clear[v] = u32x4{kStepEmpty, kStepEmpty, kStepEmpty, kStepEmpty};
+        clear[v] = u32x4{v == 0 ? patience : kStepEmpty, kStepEmpty, kStepEmpty, kStepEmpty};
 }
 
 uint32_t up(long long bytes) { return static_cast<uint32_t>((bytes + 255) & ~255ll); }
@@ -120,7 +121,7 @@ bool step_shape_ok(const ternaspmm_step_desc& d)
 
 // groups, patience: of the resident launches.
 int enqueue_step(const ternaspmm_step_desc* d, const ternaspmm_step_block* blocks, const long long* tokens, const long long* pos, const terna_bf16* embedding,
-                 const float* rope_table, void* scratch, terna_bf16* x_out, int groups, int patience, terna_stream stream)
+                 const float* rope_table, void* scratch, terna_bf16* x_out, int groups, uint32_t patience, terna_stream stream)
 {
     const long long bytes = ternaspmm_decode_step_bytes(d);
     if (bytes < 0 || blocks == nullptr || tokens == nullptr || pos == nullptr || embedding == nullptr || rope_table == nullptr || scratch == nullptr ||
@@ -147,7 +148,7 @@ int enqueue_step(const ternaspmm_step_desc* d, const ternaspmm_step_block* block
     float2* stats = reinterpret_cast<float2*>(base + cleared + up(2ll * d->M * d->dim));
     float* rope = reinterpret_cast<float*>(base + cleared + up(2ll * d->M * d->dim) + up(8ll * d->M * count));
     const StepInputs in{tokens, pos, d->per_sequence != 0, embedding, d->vocab, d->dim, rope_table, d->slots, half, blocks[0].attention_norm, x, stats, rope, count};
-    terna_step_begin_kernel<<<dim3(d->M + kClearGroups), dim3(256), 0, st>>>(in, d->M, reinterpret_cast<u32x4*>(base), cleared / 16);
+    terna_step_begin_kernel<<<dim3(d->M + kClearGroups), dim3(256), 0, st>>>(in, d->M, reinterpret_cast<u32x4*>(base), cleared / 16, patience);
 
     a.alive = reinterpret_cast<uint32_t*>(base);
     a.pos = pos;
@@ -156,10 +157,8 @@ int enqueue_step(const ternaspmm_step_desc* d, const ternaspmm_step_block* block
     a.M = d->M, a.dim = d->dim, a.ffn = d->ffn, a.H = d->heads, a.KV = d->kv_heads, a.S = d->slots, a.SP = d->splits, a.per_seq = d->per_sequence != 0;
     a.stats_count = count, a.quant_mode = quant_mode(), a.ws_qkv = d->ws_num_qkv, a.ws_o = d->ws_num_o, a.ws_2 = d->ws_num_down;
     a.eps = d->eps, a.scale = d->scale;
-    a.patience = patience;
     auto launches = [&](auto ordered) {
         constexpr bool ORDERED = decltype(ordered)::value;
-        const dim3 grid(ORDERED ? kStepOrderedGroups : groups), threads(kStepThreads);
         for (int first = 0; first < d->layers; first += kStepMaxBlocks) {
             a.blocks = d->layers - first < kStepMaxBlocks ? d->layers - first : kStepMaxBlocks;
             a.tickets = a.alive + 1 + 2 * (first / kStepMaxBlocks);
@@ -174,9 +173,10 @@ int enqueue_step(const ternaspmm_step_desc* d, const ternaspmm_step_block* block
                                        static_cast<const uint32_t*>(b.w2), b.ws_qkv, b.ws_o, b.ws_13, b.ws_down, b.attention_norm, b.attn_sub_norm, b.ffn_norm,
                                        b.ffn_sub_norm, b.cache_k, b.cache_v};
             }
-            if (d->M == 1) terna_decode_step_kernel<1, ORDERED><<<grid, threads, 0, st>>>(a);
-            else if (d->M == 2) terna_decode_step_kernel<2, ORDERED><<<grid, threads, 0, st>>>(a);
-            else terna_decode_step_kernel<4, ORDERED><<<grid, threads, 0, st>>>(a);
+            if constexpr (ORDERED) launch_step_ordered(a, st);
+            else if (d->M == 1) terna_decode_step_kernel<1, false><<<dim3(groups), dim3(kStepThreads), 0, st>>>(a);
+            else if (d->M == 2) terna_decode_step_kernel<2, false><<<dim3(groups), dim3(kStepThreads), 0, st>>>(a);
+            else terna_decode_step_kernel<4, false><<<dim3(groups), dim3(kStepThreads), 0, st>>>(a);
         }
     };
     launches(std::false_type{});
@@ -206,7 +206,7 @@ int ternaspmm_decode_step(const ternaspmm_step_desc* d, const ternaspmm_step_blo
 int ternaspmm_probe_decode_step(const ternaspmm_step_desc* d, const ternaspmm_step_block* blocks, const long long* tokens, const long long* pos,
                                 const terna_bf16* embedding, const float* rope_table, void* scratch, terna_bf16* x_out, int workgroups, int polls, terna_stream stream)
 {
-    if (workgroups < 1 || workgroups > kStepGroups || polls < 0 || polls > kStepPatience) return -1;
+    if (workgroups < 1 || workgroups > kStepGroups || polls < 1 || polls > kStepPatience) return -1;
     return enqueue_step(d, blocks, tokens, pos, embedding, rope_table, scratch, x_out, workgroups, polls, stream);
 }
 

@@ -28,7 +28,7 @@
 // waiting, on what it finds.  The launch behind it (ORDERED) then does the step again, from the same inputs and over everything the
 // first wrote, in a way that needs no workgroups side by side: a few of them take the units of work one by one in the order
 // in which they depend on each other (step_ticket), so that whatever one waits for is held by a workgroup that runs (30 blocks of
-// the 2B shape, 384 slots: 3 ms with one sequence, 4 with four).  Where nobody gave up it ends at once, 3 us.
+// the 2B shape, 384 slots: 3 ms with one sequence, 4 with four).  Where nobody gave up it ends at once, 2 - 4 us.
 //
 // Every result has the bits of the launches this replaces: integer sums, and for all that is rounded the same operations in
 // the same order (the partial statistics of 16 columns are formed by the consumer instead of the producer).
@@ -80,19 +80,21 @@ struct StepExchange {
 
 struct StepArgs {
     char* exchange;                              // [blocks][StepExchange::bytes]
-    uint32_t* alive;                             // 0xffffffff, 0 once a wave has given up
-    uint32_t* tickets;                           // ORDERED: [0] taken, [1] done, both from 0xffffffff
+    uint32_t* alive;                             // polls a wait may take, 0 once a wave has given up
     const uint16_t* x;                           // the stream in front of the first block, no word 0xffffffff
     const float2* stats;                         // its partials under the first block's norm, [M][stats_count]; nullptr: formed here
     uint16_t* x_out;                             // the stream behind the last block
     const long long* pos;
     const float *cosv, *sinv;
-    int blocks, M, dim, ffn, H, KV, S, SP, per_seq, stats_count, quant_mode, ws_qkv, ws_o, ws_2, patience;
+    int blocks, M, dim, ffn, H, KV, S, SP, per_seq, stats_count, quant_mode, ws_qkv, ws_o, ws_2;
     float eps, scale;
     StepExchange at;
     StepBlock block[kStepMaxBlocks];
+    uint32_t* tickets;                           // ORDERED: [0] taken, [1] done, both from 0xffffffff
 };
 static_assert(sizeof(StepArgs) <= 4096, "kernel arguments");
+
+void launch_step_ordered(const StepArgs& a, hipStream_t st);      // launch_step_ordered.hip: the ORDERED kernel
 
 // What a producer stores: never the word that stands for "not there yet" (a pair of bf16 NaNs, or an fp32 one: the last
 // bit of a NaN goes).
@@ -100,15 +102,13 @@ __device__ __forceinline__ uint32_t step_word(uint32_t v) { return v < kStepEmpt
 
 struct StepControl {
     uint32_t* alive;
-    int patience;
     bool gave_up;
 
     // every 256 polls of a wave
     __device__ void check(int polls)
     {
-        const bool late = polls > patience;
-        if (late) __hip_atomic_store(alive, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        gave_up = late || __builtin_amdgcn_readfirstlane(__hip_atomic_load(alive, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0;
+        gave_up = polls > __builtin_amdgcn_readfirstlane(static_cast<int>(__hip_atomic_load(alive, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)));
+        if (gave_up) __hip_atomic_store(alive, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     // load(): requests what the lane needs; there(): all of it has come.  meanwhile(): once, while the first requests are on their way.
     template <typename Load, typename There, typename Meanwhile>
@@ -182,10 +182,9 @@ struct StepOperands {
     {
         const int ktiles = K >> 6, first = wave * TPW, i = lane & 15, g = lane >> 4;
         const __amdgpu_buffer_rsrc_t rw = make_raw_buffer(packed, static_cast<uint32_t>(bands) * ktiles * 256u);
-        const int chunk = lane * 16, single = (4 * i + g) * 4;
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
-            const int at = ((band0 + b) * ktiles + first) * 256;
+            const int chunk = lane * 16, single = (4 * i + g) * 4, at = ((band0 + b) * ktiles + first) * 256;
 #pragma unroll
             for (int c = 0; c < CH; ++c) wc[b][c] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, chunk, at + 1024 * c, 0));
 #pragma unroll
@@ -786,6 +785,33 @@ __device__ __forceinline__ void step_prefetch(const void* base, int bytes, int l
     asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"s"(lds_words), "v"((line + lane) * 128), "s"(range) : "memory");
 }
 
+// Slots of a sequence's prefix; negative: its position lies outside the cache (clamped).
+__device__ __forceinline__ int step_seen(const StepArgs& a, int sequence)
+{
+    const long long p = a.pos[a.per_seq ? sequence : 0];
+    return __builtin_amdgcn_readfirstlane(p < 0 ? -1 : p >= a.S ? -a.S : static_cast<int>(p) + 1);
+}
+
+// ORDERED: the next unit, once it may start, for the whole workgroup; a block past the last where there is none.
+__device__ __forceinline__ StepTicket step_take(const StepArgs& a, StepTicket* shared, bool first)
+{
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");              // this wave's outputs have arrived
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        if (!first) __hip_atomic_fetch_add(a.tickets + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const int mine = static_cast<int>(__hip_atomic_fetch_add(a.tickets, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1);
+        StepTicket t = step_ticket(mine, a.M, a.dim, a.ffn, a.H, a.KV, a.SP);
+        bool ready = t.block >= a.blocks;
+        for (int polls = 0; !ready && polls < kStepOrderedPolls; ++polls)
+            ready = static_cast<int>(__hip_atomic_load(a.tickets + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1) >= t.before;
+        if (!ready) t.block = a.blocks;
+        *shared = t;
+    }
+    __syncthreads();
+    asm volatile("" ::: "memory");
+    return {__builtin_amdgcn_readfirstlane(shared->block), __builtin_amdgcn_readfirstlane(shared->kind), __builtin_amdgcn_readfirstlane(shared->w), 0};
+}
+
 template <int MR, bool ORDERED>
 __global__ __launch_bounds__(kStepThreads, ORDERED ? 2 : 4) void terna_decode_step_kernel(const StepArgs a)
 {
@@ -803,7 +829,7 @@ __global__ __launch_bounds__(kStepThreads, ORDERED ? 2 : 4) void terna_decode_st
     __shared__ uint16_t weight_s[kStepMaxBlocks][16];             // QKV, O, gate+up, down: four each
     __shared__ uint32_t dummy_s[64];
     __shared__ float2 nowhere_s;
-    __shared__ StepTicket ticket_s[1];           // (ORDERED)
+    __shared__ StepTicket ticket_s;              // (ORDERED)
     // What the lanes of wave 0 keep for the columns they finish -- row lane >> 4, column lane & 15 of band w: the residual stream, and the
     // weight-scale groups of QKV, O and down.  (In registers they would be spilled, and a load of a spilled register waits behind
     // the prefetches like any other.)
@@ -812,10 +838,10 @@ __global__ __launch_bounds__(kStepThreads, ORDERED ? 2 : 4) void terna_decode_st
     __shared__ __align__(16) StepShape shape_s;
     static_assert(sizeof(lds) + sizeof(scale_s) + sizeof(red) + sizeof(merge_s) + sizeof(block_s) + sizeof(weight_s) + sizeof(dummy_s) + sizeof(stream_s) + sizeof(group_s) + 96 <= 40 * 1024, "a quarter of a CU");
     const int wave0 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    int w0 = blockIdx.x;                         // (ORDERED: of the unit that is being done)
+    int w0 = ORDERED ? -1 : blockIdx.x;          // (ORDERED: of the unit that is being done)
     if (threadIdx.x == 0) shape_s = StepShape{a.M, a.dim, a.ffn, a.H, a.KV, a.SP, a.quant_mode, a.eps};
     __syncthreads();
-    auto uniform = [](int v) { return ORDERED ? __builtin_amdgcn_readfirstlane(v) : v; };      // (what take() changes)
+    auto uniform = [](int v) { return ORDERED ? __builtin_amdgcn_readfirstlane(v) : v; };      // (what another unit changes)
     auto phase = [&]() {
         StepPhase p;
         p.M = __builtin_amdgcn_readfirstlane(shape_s.M);
@@ -834,17 +860,11 @@ __global__ __launch_bounds__(kStepThreads, ORDERED ? 2 : 4) void terna_decode_st
         return p;
     };
     bool has_qkv, has_out, has_gate, has_unit, has_quant;
+    bool out_now, down_now;                      // ORDERED: which of has_out's two phases
     StepUnit unit;
     int seen = 0;                                // slots of the unit's prefix; negative: the position lies outside the cache (clamped)
-    auto find_unit = [&](const StepPhase& p) {
-        unit = step_unit(p.w, MR == 1 ? p.KV * p.SP : p.M * p.KV, p.H / p.KV * (MR == 1 ? 1 : 2));
-        has_unit = unit.group >= 0;
-        if (has_unit) {                          // (once: a load behind the prefetches would wait for them)
-            const long long p0 = a.pos[MR == 1 || !a.per_seq ? 0 : unit.group / p.KV];
-            seen = __builtin_amdgcn_readfirstlane(p0 < 0 ? -1 : p0 >= a.S ? -a.S : static_cast<int>(p0) + 1);
-        }
-    };
-    auto find_groups = [&](const StepPhase& p, int fin_n) {
+    auto find_groups = [&](const StepPhase& p) {
+        const int fin_n = 16 * p.w + (p.lane & 15);
         group_s[0][p.lane] = has_qkv && a.ws_qkv != 1 ? ws_group_decode(fin_n, p.qkv_n, a.ws_qkv) : 0;
         group_s[1][p.lane] = has_out && a.ws_o != 1 ? ws_group_decode(fin_n, p.dim, a.ws_o) : 0;
         group_s[2][p.lane] = has_out && a.ws_2 != 1 ? ws_group_decode(fin_n, p.dim, a.ws_2) : 0;
@@ -852,15 +872,16 @@ __global__ __launch_bounds__(kStepThreads, ORDERED ? 2 : 4) void terna_decode_st
     {
         const StepPhase p = phase();
         if constexpr (!ORDERED) {
-            const int fin_n = 16 * p.w + (p.lane & 15);
+            unit = step_unit(p.w, MR == 1 ? p.KV * p.SP : p.M * p.KV, p.H / p.KV * (MR == 1 ? 1 : 2));
             has_qkv = p.w < p.qkv_n >> 4;
             has_out = p.w < p.dim >> 4;
             has_gate = 4 * p.w < p.ffn >> 3;
-            find_unit(p);
+            has_unit = unit.group >= 0;
+            if (has_unit) seen = step_seen(a, MR == 1 ? 0 : unit.group / p.KV);        // (once: a load behind the prefetches would wait for them)
             has_quant = QUANT && kStepGroups - 1 - p.w < 4 * p.M;
             if (p.wave == 0) {
-                find_groups(p, fin_n);
-                stream_s[p.lane] = has_out && (p.lane >> 4) < p.M ? bf16_bits_to_float(a.x[(p.lane >> 4) * p.dim + fin_n]) : 0.0f;
+                find_groups(p);
+                stream_s[p.lane] = has_out && (p.lane >> 4) < p.M ? bf16_bits_to_float(a.x[(p.lane >> 4) * p.dim + 16 * p.w + (p.lane & 15)]) : 0.0f;
             }
         }
         const int tid = 64 * p.wave + p.lane;
@@ -878,7 +899,7 @@ __global__ __launch_bounds__(kStepThreads, ORDERED ? 2 : 4) void terna_decode_st
         }
         __syncthreads();
     }
-    StepControl ctl{a.alive, a.patience, false}; // (ORDERED: take() has waited, every poll finds its words)
+    StepControl ctl{a.alive, false}; // (ORDERED: step_take has waited, every poll finds its words)
     const uint32_t dummy = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint32_t*)dummy_s));
 
     // (operands expanded ahead of the wait: as many as the registers of the phase hold)
@@ -905,45 +926,32 @@ __global__ __launch_bounds__(kStepThreads, ORDERED ? 2 : 4) void terna_decode_st
         for (int l = p.wave; 8192 * l < bytes; l += kStepWaves) step_prefetch(packed + static_cast<size_t>(band0) * K, bytes, 64 * l, dummy, p.lane);
         if (p.wave == kStepWaves - 1) step_prefetch(norm_w, 2 * K, p.lane < 4 ? 4 * (p.w >> 3) : 1 << 20, dummy, p.lane);
     };
-    // ORDERED: the next unit, of which exactly one of the phases below is this workgroup's; its block, or all of them where
-    // there is none.  The stream of a band's columns is what its last phase handed over.
-    bool out_now = false, down_now = false;
-    auto take = [&](bool first) {
-        uint32_t* const tickets = a.tickets;
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");          // this wave's outputs have arrived
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            if (!first) __hip_atomic_fetch_add(tickets + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const int mine = static_cast<int>(__hip_atomic_fetch_add(tickets, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1);
-            const StepTicket t = step_ticket(mine, a.M, a.dim, a.ffn, a.H, a.KV, a.SP);
-            bool ready = t.block >= a.blocks;
-            for (int polls = 0; !ready && polls < kStepOrderedPolls; ++polls)
-                ready = static_cast<int>(__hip_atomic_load(tickets + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1) >= t.before;
-            ticket_s[0] = StepTicket{ready ? t.block : a.blocks, t.kind, t.w, t.before};
+    for (int n = 0; ORDERED || n < a.blocks; ++n) {
+        if constexpr (ORDERED) {                 // the next unit: of the phases below, its one alone is this workgroup's
+            const StepTicket t = step_take(a, &ticket_s, w0 < 0);
+            if (t.block >= a.blocks) break;
+            n = t.block;
+            w0 = t.w;
+            has_qkv = t.kind == STEP_QKV, out_now = t.kind == STEP_OUT, has_gate = t.kind == STEP_GATE, has_quant = t.kind == STEP_QUANT, down_now = t.kind == STEP_DOWN;
+            has_out = out_now || down_now, has_unit = t.kind == STEP_ATTENTION;
+            const StepPhase p = phase();
+            if (has_unit) {
+                unit = step_unit(p.w, MR == 1 ? p.KV * p.SP : p.M * p.KV, p.H / p.KV * (MR == 1 ? 1 : 2));
+                has_unit = unit.group >= 0;
+                seen = has_unit ? step_seen(a, MR == 1 ? 0 : unit.group / p.KV) : 0;
+            }
+            if (p.wave == 0) {
+                find_groups(p);
+                // the stream of the columns: what their last phase handed over
+                const char* from = a.exchange + static_cast<size_t>(n) * a.at.bytes;
+                from = down_now ? from + a.at.mid : n == 0 ? reinterpret_cast<const char*>(a.x) : from - a.at.bytes + a.at.out;
+                const __amdgpu_buffer_rsrc_t rx = make_raw_buffer(from, static_cast<uint32_t>(p.M) * p.dim * 2u);
+                const bool mine = has_out && (p.lane >> 4) < p.M;
+                const uint16_t bits = __builtin_amdgcn_raw_buffer_load_b16(rx, mine ? ((p.lane >> 4) * p.dim + 16 * p.w + (p.lane & 15)) * 2 : kBufferOutOfRange, 0, kDeviceScope);
+                stream_s[p.lane] = bf16_bits_to_float(bits);
+            }
+            __syncthreads();
         }
-        __syncthreads();
-        asm volatile("" ::: "memory");
-        const int block = __builtin_amdgcn_readfirstlane(ticket_s[0].block), kind = __builtin_amdgcn_readfirstlane(ticket_s[0].kind);
-        if (block >= a.blocks) return block;
-        w0 = __builtin_amdgcn_readfirstlane(ticket_s[0].w);
-        has_qkv = kind == STEP_QKV, out_now = kind == STEP_OUT, has_gate = kind == STEP_GATE, has_quant = kind == STEP_QUANT, down_now = kind == STEP_DOWN;
-        has_out = out_now || down_now, has_unit = false;
-        const StepPhase p = phase();
-        if (kind == STEP_ATTENTION) find_unit(p);
-        if (p.wave == 0) {
-            const int fin_n = 16 * p.w + (p.lane & 15);
-            find_groups(p, fin_n);
-            const char* from = a.exchange + static_cast<size_t>(block) * a.at.bytes;
-            from = down_now ? from + a.at.mid : block == 0 ? reinterpret_cast<const char*>(a.x) : from - a.at.bytes + a.at.out;
-            const __amdgpu_buffer_rsrc_t rx = make_raw_buffer(from, static_cast<uint32_t>(p.M) * p.dim * 2u);
-            const bool mine = has_out && (p.lane >> 4) < p.M;
-            const uint16_t bits = __builtin_amdgcn_raw_buffer_load_b16(rx, mine ? ((p.lane >> 4) * p.dim + fin_n) * 2 : kBufferOutOfRange, 0, kDeviceScope);
-            stream_s[p.lane] = bf16_bits_to_float(bits);
-        }
-        __syncthreads();
-        return block;
-    };
-    for (int n = ORDERED ? take(true) : 0; n < a.blocks; n = ORDERED ? take(false) : n + 1) {
         char* ex = a.exchange + static_cast<size_t>(n) * a.at.bytes;
         const int ahead = n + 1 < a.blocks ? n + 1 : n;
         // ---- QKV

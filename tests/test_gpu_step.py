@@ -230,9 +230,9 @@ def raw_step(model, whole, tokens, pos, workgroups, polls):
 
 
 @pytest.mark.parametrize("shape,layers,m,slots,positions,workgroups,polls", [
-    (TINY, 3, 1, 64, [40], 1, 0), (TINY, 65, 1, 64, [33], 255, 512), (TINY, 65, 3, 30, [29, 2, 11], 16, 0), (SINGLE, 2, 2, 128, [127], 255, 0),
-    (ODD, 3, 1, 200, [130], 100, 256), (ODD, 3, 4, 640, [1, 639, 127, 128], 200, 0), (ODD, 2, 1, 8192, [8191], 64, 0),
-    (WIDE, 2, 1, 384, [255], 240, 1024), (WIDE, 2, 2, 101, [100], 255, 0), (WIDE, 2, 4, 1024, [1023, 640, 0, 777], 128, 0), (WIDE, 2, 1, 384, [300], 256, 0),
+    (TINY, 3, 1, 64, [40], 1, 1), (TINY, 65, 1, 64, [33], 255, 512), (TINY, 65, 3, 30, [29, 2, 11], 16, 1), (SINGLE, 2, 2, 128, [127], 255, 1),
+    (ODD, 3, 1, 200, [130], 100, 256), (ODD, 3, 4, 640, [1, 639, 127, 128], 200, 1), (ODD, 2, 1, 8192, [8191], 64, 1),
+    (WIDE, 2, 1, 384, [255], 240, 1024), (WIDE, 2, 2, 101, [100], 255, 1), (WIDE, 2, 4, 1024, [1023, 640, 0, 777], 128, 1), (WIDE, 2, 1, 384, [300], 256, 1),
 ])
 def test_a_step_whose_workgroups_do_not_all_come(shape, layers, m, slots, positions, workgroups, polls):
     """Fewer workgroups than wait for each other, and waits that end soon: the step is done again in order, with the same bits in
