@@ -1,5 +1,5 @@
 // The launch that does a decode step in order where the resident one gave up (step_kernel.h).  A file of its own: compiled beside it, the
-// resident kernels spill more (two sequences 722 -> 736 us a step).
+// resident kernels spill more (two sequences 722 -> 730 us a step).
 #include <hip/hip_runtime.h>
 
 #include "step_kernel.h"

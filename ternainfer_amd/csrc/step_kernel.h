@@ -55,8 +55,6 @@ constexpr int kStepRecord = (kStepHeadDim + 4) * 4;      // bytes a (head, split
 // 1528 1078 -> 1174; filled to half 15 - 23 % ahead at two, 6 - 12 % at four).
 constexpr int step_max_slots(int M) { return M == 2 ? 1280 : 1024; }
 constexpr int kStepMaxSplitSlots = 1024;
-constexpr int kStepWideTiles = 112;              // tiles of the down projection's K: ffn <= 7168
-constexpr int kStepTiles = 40;                   // tiles of the other linears' K: <= 2560
 constexpr uint32_t kStepEmpty = 0xffffffffu;
 // Polls of one wait before a wave gives up: 20 ms where they take 0.15 us (an idle chip), more on a busy one -- longer than the kernels
 // of other streams hold a part of the grid back.  Polls and not wall clock: a process that was suspended has not waited.
@@ -177,18 +175,19 @@ struct StepOperands {
     // word of pair (tile t of the run, band b): in chunks a lane holds component t & 3 of one load
     __device__ __forceinline__ uint32_t word(int t, int b) const { return t < 4 * CH ? wc[b][t >> 2][t & 3] : wt[b][t - 4 * CH]; }
 
-    // (Tiles past K: words of the next band or nothing, times activations that are zero.)
+    // (Tiles past K: words of the next band or nothing, times activations that are zero.  All of the offset is the lane's, which is what
+    // the buffer's range is held against: a run of the last band may begin past the matrix.)
     __device__ __forceinline__ void request(const uint32_t* packed, int bands, int band0, int K, const uint16_t* norm_w, int lane, int wave)
     {
         const int ktiles = K >> 6, first = wave * TPW, i = lane & 15, g = lane >> 4;
         const __amdgpu_buffer_rsrc_t rw = make_raw_buffer(packed, static_cast<uint32_t>(bands) * ktiles * 256u);
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
-            const int chunk = lane * 16, single = (4 * i + g) * 4, at = ((band0 + b) * ktiles + first) * 256;
+            const int chunk = step_weight_offset(band0 + b, ktiles, first, lane * 16), single = step_weight_offset(band0 + b, ktiles, first, (4 * i + g) * 4);
 #pragma unroll
-            for (int c = 0; c < CH; ++c) wc[b][c] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, chunk, at + 1024 * c, 0));
+            for (int c = 0; c < CH; ++c) wc[b][c] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, chunk + 1024 * c, 0, 0));
 #pragma unroll
-            for (int s = 0; s < SG; ++s) wt[b][s] = __builtin_amdgcn_raw_buffer_load_b32(rw, single, at + 256 * (4 * CH + s), 0);
+            for (int s = 0; s < SG; ++s) wt[b][s] = __builtin_amdgcn_raw_buffer_load_b32(rw, single + 256 * (4 * CH + s), 0, 0);
         }
         if constexpr (NORM) {
             const __amdgpu_buffer_rsrc_t rn = make_raw_buffer(norm_w, static_cast<uint32_t>(K) * 2u);
@@ -571,10 +570,10 @@ __device__ __forceinline__ void step_attention(StepControl& ctl, const StepArgs&
     const int chunk = tid % CH, slice = tid / CH;
 
     u32x4 kr[KT][NJ], vr[VU];
-    auto load_keys = [&](int ltile, u32x4 (&dst)[NJ]) {
+    auto load_keys = [&](int ltile, u32x4 (&dst)[NJ]) {         // (tiles past the last one too: the lane's offset says so)
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
-            dst[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, (SPM * j + sl) * D * 2 + 16 * piece, 16 * (ltile * SP + sp) * D * 2, 0));
+            dst[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, (16 * (ltile * SP + sp) + SPM * j + sl) * D * 2 + 16 * piece, 0, 0));
     };
     auto load_value = [&](int l) { return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rv, (cache_slot(l) * D + chunk * DT) * 2, 0, 0)); };
 #pragma unroll

@@ -11,6 +11,11 @@ namespace terna {
 
 constexpr int kStepWaves = 4, kStepThreads = 64 * kStepWaves, kStepGroups = 256;
 constexpr int kStepHeadDim = 128;
+constexpr int kStepWideTiles = 112;              // tiles of the down projection's K: ffn <= 7168
+constexpr int kStepTiles = 40;                   // tiles of the other linears' K: <= 2560
+
+// Byte of a P2 matrix where a lane's part of a wave's run begins: tile `first` and on of a band, 256 bytes a tile.
+TERNA_STEP_FUNCTION int step_weight_offset(int band, int ktiles, int first, int lane_bytes) { return (band * ktiles + first) * 256 + lane_bytes; }
 
 // Attention units over the workgroups, from the last one downwards: the H / KV heads of a kv group read the same keys and values
 // and sit on one XCD (workgroups go to the eight of them round robin).  A group is a (sequence, kv head), or (one sequence) a

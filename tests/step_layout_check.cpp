@@ -58,6 +58,27 @@ static void check_tickets(const Shape& s)
                 CHECK(!resident_does(s, kind, w) || seen.count({block, kind, w}), "block %d kind %d workgroup %d is no ticket", block, kind, w);
 }
 
+// What a wave requests of a matrix lies in it, or wholly past its last byte, where the buffer's range check -- an unsigned
+// comparison with the lane's offset -- returns zeros; and every tile of a band is requested by the wave whose run it is in.
+static void check_weight_requests(int bands, int K, int per_workgroup, int chunks, int singles)
+{
+    const int ktiles = K / 64, run = 4 * chunks + singles, range = bands * ktiles * 256;
+    for (int band = 0; band < (bands + per_workgroup - 1) / per_workgroup * per_workgroup; ++band) {
+        std::vector<bool> read(static_cast<size_t>(ktiles) * 256);
+        auto request = [&](long long at, int size) {
+            CHECK(at >= 0 && at < 0x7fffffff && (at + size <= range || at >= range), "band %d of %d, K %d: %d bytes at %lld of %d", band, bands, K, size, at, range);
+            for (long long b = at; b < at + size; ++b)
+                if (b >= static_cast<long long>(band) * ktiles * 256 && b < static_cast<long long>(band + 1) * ktiles * 256) read[b - static_cast<long long>(band) * ktiles * 256] = true;
+        };
+        for (int wave = 0; wave < kStepWaves; ++wave)
+            for (int lane = 0; lane < 64; ++lane) {
+                for (int c = 0; c < chunks; ++c) request(step_weight_offset(band, ktiles, wave * run, lane * 16) + 1024 * c, 16);
+                for (int s = 0; s < singles; ++s) request(step_weight_offset(band, ktiles, wave * run, lane * 4) + 256 * (4 * chunks + s), 4);
+            }
+        for (size_t b = 0; b < read.size(); ++b) CHECK(band >= bands || read[b], "band %d, K %d: byte %zu is requested by no wave", band, K, b);
+    }
+}
+
 int main()
 {
     std::vector<Shape> shapes;
@@ -69,6 +90,13 @@ int main()
                 if ((M == 1) == (SP > 1) && step_unit_groups(M == 1 ? KV * SP : M * KV, H / KV * (M == 1 ? 1 : 2)) <= kStepGroups) shapes.push_back(s);
             }
     for (const Shape& s : shapes) check_tickets(s);
+    for (int ktiles : {1, 2, 3, 9, 10, 11, 30, 39, kStepTiles})
+        for (int bands : {4, 12, 160}) {
+            check_weight_requests(bands, 64 * ktiles, 1, 2, 2);
+            check_weight_requests(bands, 64 * ktiles, 4, 2, 2);
+        }
+    for (int ktiles : {1, 27, 28, 29, 85, 108, kStepWideTiles})
+        for (int bands : {4, 160}) check_weight_requests(bands, 64 * ktiles, 1, 7, 0);
     if (failures == 0) std::printf("step layout ok: %zu shapes\n", shapes.size());
     return failures != 0;
 }
