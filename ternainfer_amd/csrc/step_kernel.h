@@ -775,13 +775,13 @@ __device__ __forceinline__ void step_quantise(StepControl& ctl, const StepPhase&
 }
 
 // Lines of device memory on their way into the L2 of this XCD, without a register: a word of each goes to a place in LDS nobody
-// reads.  Line `line` + lane of 128 bytes; past the range nothing is read.  (asm: the compiler would wait for the builtin's LDS
+// reads.  The lane's line begins at byte `at`; past the range nothing is read.  (asm: the compiler would wait for the builtin's LDS
 // writes in front of the next LDS access of any kind.)
-__device__ __forceinline__ void step_prefetch(const void* base, int bytes, int line, uint32_t lds_words, int lane)
+__device__ __forceinline__ void step_prefetch(const void* base, int bytes, int at, uint32_t lds_words)
 {
-    const uint64_t at = reinterpret_cast<uint64_t>(base);
-    const i32x4 range = {static_cast<int>(at), static_cast<int>(at >> 32), bytes, kBufferRsrcFlags};
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"s"(lds_words), "v"((line + lane) * 128), "s"(range) : "memory");
+    const uint64_t from = reinterpret_cast<uint64_t>(base);
+    const i32x4 range = {static_cast<int>(from), static_cast<int>(from >> 32), bytes, kBufferRsrcFlags};
+    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"s"(lds_words), "v"(at), "s"(range) : "memory");
 }
 
 // Slots of a sequence's prefix; negative: its position lies outside the cache (clamped).
@@ -829,6 +829,7 @@ __global__ __launch_bounds__(kStepThreads, ORDERED ? 2 : 4) void terna_decode_st
     __shared__ uint32_t dummy_s[64];
     __shared__ float2 nowhere_s;
     __shared__ StepTicket ticket_s;              // (ORDERED)
+    __shared__ int sharing_s;                    // prefetch_cache: how many share a unit's keys and values << 16 | which of them this is
     // What the lanes of wave 0 keep for the columns they finish -- row lane >> 4, column lane & 15 of band w: the residual stream, and the
     // weight-scale groups of QKV, O and down.  (In registers they would be spilled, and a load of a spilled register waits behind
     // the prefetches like any other.)
@@ -878,6 +879,10 @@ __global__ __launch_bounds__(kStepThreads, ORDERED ? 2 : 4) void terna_decode_st
             has_unit = unit.group >= 0;
             if (has_unit) seen = step_seen(a, MR == 1 ? 0 : unit.group / p.KV);        // (once: a load behind the prefetches would wait for them)
             has_quant = QUANT && kStepGroups - 1 - p.w < 4 * p.M;
+            if (has_unit) {
+                const int per = p.H / p.KV * (MR == 1 ? 1 : 2), past = MR == 1 ? 0 : step_unit_past(unit, per, p.qkv_n >> 4);
+                sharing_s = (per - past) << 16 | (unit.head - past);      // (of those past the bands, with several sequences: not read)
+            }
             if (p.wave == 0) {
                 find_groups(p);
                 stream_s[p.lane] = has_out && (p.lane >> 4) < p.M ? bf16_bits_to_float(a.x[(p.lane >> 4) * p.dim + 16 * p.w + (p.lane & 15)]) : 0.0f;
@@ -922,8 +927,28 @@ __global__ __launch_bounds__(kStepThreads, ORDERED ? 2 : 4) void terna_decode_st
     auto prefetch = [&](const StepPhase& p, const uint32_t* packed, int band0, int bands, const uint16_t* norm_w, int K) {
         if constexpr (ORDERED) return;
         const int bytes = bands * (K >> 6) * 256;
-        for (int l = p.wave; 8192 * l < bytes; l += kStepWaves) step_prefetch(packed + static_cast<size_t>(band0) * K, bytes, 64 * l, dummy, p.lane);
-        if (p.wave == kStepWaves - 1) step_prefetch(norm_w, 2 * K, p.lane < 4 ? 4 * (p.w >> 3) : 1 << 20, dummy, p.lane);
+        for (int l = p.wave; 8192 * l < bytes; l += kStepWaves) step_prefetch(packed + static_cast<size_t>(band0) * K, bytes, (64 * l + p.lane) * 128, dummy);
+        if (p.wave == kStepWaves - 1) step_prefetch(norm_w, 2 * K, (p.lane < 4 ? 4 * (p.w >> 3) + p.lane : 1 << 20) * 128, dummy);
+    };
+    // A block's keys and values, what the unit's group reads of them shared out over its workgroups, right behind the wait for the
+    // stream.  Those past the bands of QKV, which do not wait there: one sequence, at any time before their attention (4096 slots, filled to 90 %, 901 -> 867 us
+    // a step, 8192 1130 -> 1048; left to the others 879 and 1102); several, nothing, the others take their shares (two, 1280 slots 986 -> 944, four,
+    // 1024 1046 -> 1016; by themselves 934 and 1021, but for the registers of a second copy of this code 5 - 9 more in short caches).
+    auto prefetch_cache = [&](const StepPhase& p, int n) {
+        if constexpr (!ORDERED) {
+            const int b = MR == 1 ? 0 : unit.group / p.KV, kvh = MR == 1 ? unit.group / p.SP : unit.group - b * p.KV;
+            const int split = MR == 1 ? unit.group % p.SP : 0, splits = MR == 1 ? p.SP : 1;
+            const int sharing = __builtin_amdgcn_readfirstlane(sharing_s), members = sharing >> 16;
+            const int bytes = 2 * kStepHeadDim * (seen < 0 ? -seen : seen);
+            const size_t at = (static_cast<size_t>(b) * p.KV + kvh) * a.S * kStepHeadDim;
+            const uint16_t *k = pointer(block_s[n].cache_k) + at, *v = pointer(block_s[n].cache_v) + at;
+#pragma unroll 1
+            for (int share = (sharing & 0xffff) + members * p.wave; step_cache_share(share, split, splits, bytes); share += members * kStepWaves) {
+                const int line = step_cache_line(share, p.lane, split, splits);
+                step_prefetch(k, bytes, line, dummy);
+                step_prefetch(v, bytes, line, dummy);
+            }
+        }
     };
     for (int n = 0; ORDERED || n < a.blocks; ++n) {
         if constexpr (ORDERED) {                 // the next unit: of the phases below, its one alone is this workgroup's
@@ -963,17 +988,7 @@ __global__ __launch_bounds__(kStepThreads, ORDERED ? 2 : 4) void terna_decode_st
             if (has_out) prefetch(p, pointer(block_s[n].wo), p.w, 1, pointer(block_s[n].attn_sub_norm), p.wide);
             if (has_gate) prefetch(p, pointer(block_s[n].w13), 4 * p.w, 4, pointer(block_s[n].ffn_norm), p.dim);
             if (!has_gate) prefetch(p, pointer(block_s[ahead].wqkv), p.w, 1, pointer(block_s[ahead].attention_norm), p.dim);
-            if (!ORDERED && has_unit) {          // this block's keys and values, a share by each of the workgroups that read them
-                const int b = MR == 1 ? 0 : unit.group / p.KV, kvh = MR == 1 ? unit.group / p.SP : unit.group - b * p.KV, per = p.H / p.KV;
-                const int bytes = 2 * kStepHeadDim * (seen < 0 ? -seen : seen);
-                const size_t at = (static_cast<size_t>(b) * p.KV + kvh) * a.S * kStepHeadDim;
-                const uint16_t *k = pointer(block_s[n].cache_k) + at, *v = pointer(block_s[n].cache_v) + at;
-                const int share = MR == 1 ? per * p.SP : 2 * per, mine = MR == 1 ? unit.head * p.SP + unit.group % p.SP : unit.head;
-                for (int l = mine + share * p.wave; 8192 * l < bytes; l += share * kStepWaves) {
-                    step_prefetch(k, bytes, 64 * l, dummy, p.lane);
-                    step_prefetch(v, bytes, 64 * l, dummy, p.lane);
-                }
-            }
+            if (has_unit) prefetch_cache(p, n);
             const float s = step_norm_linear<MR, STEP_GROUPS, kStepTiles, 1>(op, xr, p, p.dim, n == 0 ? a.stats : nullptr, a.stats_count, lds, &nowhere_s, scale_s);
             if (p.wave == 0) {
                 const uint16_t o = outputs(step_band_sum<MR>(lds, 0, p.lane), s, weight_s[n][group_s[0][p.lane]]);
@@ -982,6 +997,7 @@ __global__ __launch_bounds__(kStepThreads, ORDERED ? 2 : 4) void terna_decode_st
         }
         // ---- attention
         if (has_unit) {
+            if (MR == 1 && !has_qkv) prefetch_cache(phase(), n);
             const StepPhase p = phase();
             step_attention<MR>(ctl, a, p, pointer(block_s[n].cache_k), pointer(block_s[n].cache_v), ex + a.at.qkv, ex + a.at.attention, StepUnit{step_uniform(uniform(unit.group)), step_uniform(uniform(unit.head))},
                                seen < 0 ? -seen : seen, seen > 0, lds, red);

@@ -31,6 +31,23 @@ TERNA_STEP_FUNCTION StepUnit step_unit(int w, int groups, int per)
     return {u < step_unit_groups(groups, per) && group < groups ? group : -1, q % per};
 }
 
+// Workgroups of a group that stand past the bands of QKV: its first ones.
+TERNA_STEP_FUNCTION int step_unit_past(const StepUnit& unit, int per, int bands)
+{
+    const int q = (kStepGroups - bands - (unit.group & 7) + 7) >> 3;      // those with u = 8 q' + (group & 7) < kStepGroups - bands
+    const int past = q - per * (unit.group >> 3);
+    return past < 0 ? 0 : past > per ? per : past;
+}
+
+// Byte of a kv head's keys (or values) whose line of 128 a lane brings into the L2 of its XCD: of the split it reads itself -- tiles of 16
+// slots, split, split + splits, ... -- two tiles a share, shares dealt out over the workgroups of the group, which sit on one XCD.
+// step_cache_share: whether a share has a line within the prefix.
+TERNA_STEP_FUNCTION int step_cache_line(int share, int lane, int split, int splits)
+{
+    return (((2 * share + (lane >> 5)) * splits + split) * 16 + (lane & 31) / 2) * kStepHeadDim * 2 + (lane & 1) * 128;
+}
+TERNA_STEP_FUNCTION bool step_cache_share(int share, int split, int splits, int bytes) { return step_cache_line(share, 0, split, splits) < bytes; }
+
 // The step's units of work in the order of their dependences: those of a phase, then those of the next, block by block.  A
 // workgroup of the ORDERED launch takes one after the other from a counter; a unit may start once as many are done as stand in front of
 // its phase (a later one cannot be among them).

@@ -79,6 +79,41 @@ static void check_weight_requests(int bands, int K, int per_workgroup, int chunk
     }
 }
 
+// The lines of the keys that the workgroups of a unit's group bring into the L2 of their XCD: those the group reads, each once --
+// with several sequences by those of its workgroups that have a band of QKV, if any has.
+static void check_cache_lines(const Shape& s, int slots_seen)
+{
+    const int groups = s.M == 1 ? s.KV * s.SP : s.M * s.KV, per = s.H / s.KV * (s.M == 1 ? 1 : 2), splits = s.M == 1 ? s.SP : 1;
+    const int bytes = 2 * kStepHeadDim * slots_seen, lines = bytes / 128;
+    std::vector<std::vector<int>> fetched(groups, std::vector<int>(lines));
+    std::vector<int> xcd(groups, -1), fetching(groups);
+    const int bands = (s.H + 2 * s.KV) * kStepHeadDim / 16;
+    for (int w = 0; w < kStepGroups; ++w) {
+        const StepUnit u = step_unit(w, groups, per);
+        if (u.group < 0) continue;
+        CHECK(xcd[u.group] < 0 || xcd[u.group] == w % 8, "group %d sits on two XCDs", u.group);
+        xcd[u.group] = w % 8;
+        const int split = s.M == 1 ? u.group % s.SP : 0, past = s.M == 1 ? 0 : step_unit_past(u, per, bands);
+        CHECK(s.M == 1 || (u.head >= past) == resident_does(s, STEP_QKV, w), "workgroup %d, %d of its group past %d bands", w, past, bands);
+        if (u.head < past) continue;
+        ++fetching[u.group];
+        for (int wave = 0; wave < kStepWaves; ++wave)
+            for (int share = u.head - past + (per - past) * wave; step_cache_share(share, split, splits, bytes); share += (per - past) * kStepWaves)
+                for (int lane = 0; lane < 64; ++lane) {
+                    const int at = step_cache_line(share, lane, split, splits);
+                    CHECK(at >= 0 && at % 128 == 0, "byte %d", at);
+                    if (at >= bytes) continue;                    // (nothing is read)
+                    CHECK(at / (16 * 2 * kStepHeadDim) % splits == split, "split %d of %d fetches byte %d of another", split, splits, at);
+                    ++fetched[u.group][at / 128];
+                }
+    }
+    for (int g = 0; g < groups; ++g)
+        for (int l = 0; l < lines; ++l) {
+            const int split = s.M == 1 ? g % s.SP : 0, own = fetching[g] > 0 && l * 128 / (16 * 2 * kStepHeadDim) % splits == split;
+            CHECK(fetched[g][l] == own, "group %d, %d slots: line %d is fetched %d times", g, slots_seen, l, fetched[g][l]);
+        }
+}
+
 int main()
 {
     std::vector<Shape> shapes;
@@ -89,7 +124,10 @@ int main()
                 const Shape s{M, dim, ffn, H, KV, SP};
                 if ((M == 1) == (SP > 1) && step_unit_groups(M == 1 ? KV * SP : M * KV, H / KV * (M == 1 ? 1 : 2)) <= kStepGroups) shapes.push_back(s);
             }
-    for (const Shape& s : shapes) check_tickets(s);
+    for (const Shape& s : shapes) {
+        check_tickets(s);
+        for (int slots_seen : {1, 15, 16, 17, 100, 254, 1024}) check_cache_lines(s, slots_seen);
+    }
     for (int ktiles : {1, 2, 3, 9, 10, 11, 30, 39, kStepTiles})
         for (int bands : {4, 12, 160}) {
             check_weight_requests(bands, 64 * ktiles, 1, 2, 2);
