@@ -149,7 +149,7 @@ def attention_merge_rmsnorm_linear_packed(partial, splits, heads, head_dim, norm
     """The O projection of a decode step fed by the partial results of a split attention launch
     (ternaspmm_rope_decode_attention_partial over `sequences` sequences): for one sequence merge -> RMSNorm -> quant_input
     -> int8 TernaSpMM in one launch where the library supports the shape; for more, merge + norm + quantisation in one
-    launch (ternaspmm_attention_merge_rmsnorm_quant) and the linear on its rows; else ternaspmm_attention_merge +
+    launch (ternaspmm_step_attention_merge, any number of splits) and the linear on its rows; else ternaspmm_attention_merge +
     rmsnorm_linear_packed.  partial: fp32 device buffer of ternaspmm_attention_partial_bytes(sequences, ...);
     returns out bf16 [sequences, out_features]."""
     lib = _lib.load()
@@ -165,7 +165,7 @@ def attention_merge_rmsnorm_linear_packed(partial, splits, heads, head_dim, norm
             return out
     else:
         # several sequences: merge + norm + quantisation once per sequence in one launch, then the linear on the quantised rows
-        mq = attention_merge_rmsnorm_quant(partial, splits, heads, head_dim, norm_weight, eps, sequences)
+        mq = _lib.native().step_attention_merge(partial, splits, heads, head_dim, norm_weight, eps, sequences, False, None)
         if mq is not None:
             return TernaInfer_linear_packed(mq[0], packed, mq[1], ws, ws_num, out_features)
     o = torch.empty((sequences, k), dtype=torch.bfloat16, device=partial.device)

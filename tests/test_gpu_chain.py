@@ -479,3 +479,24 @@ def test_a_given_maximum_below_the_rows_own_saturates(m, k, mode):
     assert int((want == 127).sum()) > m and int((want == -128).sum()) > 2 * m
     assert torch.equal(xq, want)
     assert inside is not None and torch.equal(inside[3], want) and torch.equal(inside[4].view(torch.int16), s.view(torch.int16))
+
+
+@pytest.mark.parametrize("sequences,splits", [(2, 1), (3, 3), (17, 3), (9, 5), (20, 6), (2, 7), (5, 8)])
+def test_o_projection_behind_any_number_of_splits(sequences, splits, monkeypatch):
+    """Several sequences: merge, norm and quantisation in one launch whatever the number of splits, with the bits of the merge and the
+    norm as launches of their own."""
+    lib = T._lib.load()
+    heads, hd, n = 20, 128, 256
+    k = heads * hd
+    packed, ws, g = _packed(make_ternary(n, k, 0.4, 1270)), _bf(WS), _bf(_weight(k, 1271))
+    count = lib.ternaspmm_attention_partial_bytes(sequences, heads, hd) // 4
+    part = torch.from_numpy(np.random.default_rng(1272 + splits).standard_normal(count).astype(np.float32)).cuda()
+    stat_floats = count - sequences * heads * 8 * hd
+    part[:stat_floats] = part[:stat_floats].abs() + 0.5         # maxima and sums of numerators: the sums positive
+    o = torch.empty((sequences, k), dtype=torch.bfloat16, device="cuda")
+    lib.ternaspmm_attention_merge(part.data_ptr(), splits, o.data_ptr(), sequences, heads, hd, torch.cuda.current_stream().cuda_stream)
+    xq, s, _ = T.rmsnorm_quant(o, g, 1e-5)
+    want = T.TernaInfer_linear_packed(xq, packed, s, ws, 1, n)
+    monkeypatch.setattr(L, "rmsnorm_linear_packed", None)       # the way with launches of their own is not taken
+    got = L.attention_merge_rmsnorm_linear_packed(part, splits, heads, hd, g, 1e-5, packed, ws, 1, n, sequences=sequences)
+    assert torch.equal(got, want) and torch.isfinite(want.float()).all()
