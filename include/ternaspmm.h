@@ -278,7 +278,10 @@ int bitlinear_TernaSpMM_packed_fused_glu(const terna_bf16* x13, const terna_bf16
  *             TERNASPMM_PROLOGUE_ATTENTION  x = the partial results of ternaspmm_rope_decode_attention_partial
  *                                           (attention_splits, head_dim; M = 1), merged inside, statistics taken inside
  *             TERNASPMM_PROLOGUE_STATS      x = h bf16 [M][K] with its partials stats_in fp32 [M][stats_count][2]
- *                                           (stats_count <= 448), as a producing epilogue or ternaspmm_row_stats left them
+ *                                           (stats_count <= 448), as a producing epilogue or ternaspmm_row_stats left them; values
+ *                                           above the maximum they name are clamped to -128 .. 127
+ *             TERNASPMM_PROLOGUE_OWN_STATS  the same, where no value of a row lies above the maximum its partials name: saves the
+ *                                           clamp (1 % of a decode step of 5 - 8 sequences); one that does is not clamped
  *             TERNASPMM_PROLOGUE_QUANTISED  x = int8 [M][K] with its scales s_in bf16 [M] (ternaspmm_quant_from_stats,
  *                                           ternaspmm_rmsnorm_quant): no prologue; with TERNASPMM_EPILOGUE_RESIDUAL
  *                                           (M <= 16, any K the int8 kernels take) or TERNASPMM_EPILOGUE_GATE (M <= 16,
@@ -300,14 +303,15 @@ int bitlinear_TernaSpMM_packed_fused_glu(const terna_bf16* x13, const terna_bf16
  * residual.  Only enqueues.  Every workgroup of a launch with a NORM / ATTENTION / STATS prologue repeats the norm +
  * quantisation of all M rows: measured on the 2B shapes that pays up to 8 rows of K = 2560 (2 of K = 6912); above,
  * ternaspmm_quant_from_stats in front of a PROLOGUE_QUANTISED launch (or of bitlinear_TernaSpMM_packed) is faster. */
-enum { TERNASPMM_PROLOGUE_NORM = 0, TERNASPMM_PROLOGUE_ATTENTION = 1, TERNASPMM_PROLOGUE_STATS = 2, TERNASPMM_PROLOGUE_QUANTISED = 3 };
+enum { TERNASPMM_PROLOGUE_NORM = 0, TERNASPMM_PROLOGUE_ATTENTION = 1, TERNASPMM_PROLOGUE_STATS = 2, TERNASPMM_PROLOGUE_QUANTISED = 3,
+       TERNASPMM_PROLOGUE_OWN_STATS = 4 };
 enum { TERNASPMM_EPILOGUE_STORE = 0, TERNASPMM_EPILOGUE_RESIDUAL = 1, TERNASPMM_EPILOGUE_GATE = 2 };
 typedef struct ternaspmm_fused_linear_desc {
     int prologue, epilogue;
     int M, N, K;
     int ws_num;
     float eps;
-    int stats_count;                  /* PROLOGUE_STATS */
+    int stats_count;                  /* PROLOGUE_STATS, PROLOGUE_OWN_STATS */
     int attention_splits, head_dim;   /* PROLOGUE_ATTENTION */
     const void* x;
     const float* stats_in;

@@ -121,7 +121,7 @@ __global__ __launch_bounds__(256) void terna_quant_stats_kernel(const uint16_t* 
     pmax = wave_amax(pmax);
     const float rstd = rsqrtf(sum / static_cast<float>(K) + eps);
     uint16_t sb;
-    const float s = quant_scale(fabsf(round_bf16(__fmul_rn(pmax, rstd))), quant_mode, &sb);
+    const float s = quant_scale(fabsf(round_bf16(__fmul_rn(pmax, rstd))), quant_scale_mode(quant_mode), &sb);
     if (blockIdx.y == 0 && threadIdx.x == 0) s_out[row] = sb;
     if (!in) return;
     const uint32_t hd[4] = {hv.x, hv.y, hv.z, hv.w}, wd[4] = {wv.x, wv.y, wv.z, wv.w};
@@ -129,6 +129,9 @@ __global__ __launch_bounds__(256) void terna_quant_stats_kernel(const uint16_t* 
     chain_quantise<8, true, true>(hd, wd, rstd, s, quant_mode, d);
     *reinterpret_cast<u32x2*>(xq_out + row * K + c) = u32x2{d[0], d[1]};
 }
+
+// The quantisation mode of a kernel whose partials come from a caller.
+int given_mode(int mode) { return mode == QUANT_ROUNDED ? static_cast<int>(QUANT_ROUNDED_GIVEN) : mode; }
 
 // One launch of terna_decode_fused_kernel<WAVES, TMAX, MODE, MP, NB, ASP, AHD, EPI> with MP picked by M (1, 2, 4, 8).
 struct ChainArgs {
@@ -145,6 +148,7 @@ struct ChainArgs {
     int8_t* xq_out;
     uint16_t* s_out;
     int qmode;
+    bool own_stats;                              // the given partials are the rows' own
     FusedExtra ex;
     dim3 grid;
     hipStream_t st;
@@ -192,11 +196,11 @@ bool launch_chunk_by_rows(const ChainArgs& a, int units)
 {
     const ChainIo io{a.out, a.ws, a.xq_out, a.s_out, a.ex.epi_residual, a.ex.epi_next_w, a.ex.stats_out, a.ex.raw_out};
     const int workers = kChunkWaves - chain_reducers(a.M, units);
-    const int ct = (units + workers - 1) / workers;
+    const int ct = (units + workers - 1) / workers, qmode = a.own_stats ? a.qmode : given_mode(a.qmode);
     if (ct > 3) return false;
 #define TERNA_CHAIN_CHUNK(CT, MR)                                                                                       \
     terna_chain_chunk_kernel<NBANDS, CT, MR, EPI, UNIT_BANDS><<<a.grid, dim3(kChunkWaves * 64), 0, a.st>>>(                \
-        a.x, a.norm_w, a.packed, a.ex.stats_in, a.M, a.N, a.K, a.ex.stats_count, a.eps, a.ws_num, a.qmode, io)
+        a.x, a.norm_w, a.packed, a.ex.stats_in, a.M, a.N, a.K, a.ex.stats_count, a.eps, a.ws_num, qmode, io)
 #define TERNA_CHAIN_CHUNK_CT(MR)                                                                                        \
     do {                                                                                                                \
         if (ct == 1) TERNA_CHAIN_CHUNK(1, MR);                                                                          \
@@ -426,7 +430,7 @@ int ternaspmm_quant_from_stats(const terna_bf16* h, const float* stats, int stat
     }
     auto kernel = stats_count <= 192 ? terna_quant_stats_kernel<3> : terna_quant_stats_kernel<kStatsMaxPartials / 64>;      // partials a lane
     kernel<<<dim3(M, (K + 2047) / 2048), dim3(256), 0, static_cast<hipStream_t>(stream)>>>(
-        h, reinterpret_cast<const float2*>(stats), stats_count, norm_weight, K, eps, xq_out, s_out, quant_mode());
+        h, reinterpret_cast<const float2*>(stats), stats_count, norm_weight, K, eps, xq_out, s_out, given_mode(quant_mode()));
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) die("ternaspmm_quant_from_stats", e, __LINE__);
     return 0;
@@ -436,7 +440,8 @@ int ternaspmm_fused_linear(const ternaspmm_fused_linear_desc* d, terna_stream st
 {
     if (d == nullptr) return -1;
     const int M = d->M, N = d->N, K = d->K;
-    const int pro = d->prologue, epi = d->epilogue;
+    const bool own_stats = d->prologue == TERNASPMM_PROLOGUE_OWN_STATS;
+    const int pro = own_stats ? static_cast<int>(TERNASPMM_PROLOGUE_STATS) : d->prologue, epi = d->epilogue;
     if (pro == TERNASPMM_PROLOGUE_QUANTISED) {
         // activations already quantised (ternaspmm_quant_from_stats, ternaspmm_rmsnorm_quant): the matmul of
         // bitlinear_TernaSpMM_packed with a producing epilogue
@@ -503,6 +508,7 @@ int ternaspmm_fused_linear(const ternaspmm_fused_linear_desc* d, terna_stream st
     a.xq_out = d->xq_out;
     a.s_out = d->s_out;
     a.qmode = quant_mode();
+    a.own_stats = own_stats;
     a.ex = FusedExtra{reinterpret_cast<const float2*>(d->stats_in), d->stats_count, d->residual, d->next_norm_weight,
                       reinterpret_cast<float2*>(d->stats_out), d->raw_out};
     a.st = static_cast<hipStream_t>(stream);

@@ -65,7 +65,7 @@ __device__ __forceinline__ void chain_reduce_partials(const float2 (&part)[PN], 
         const float r = rsqrtf(sum / static_cast<float>(K) + eps);
         const float amax_y = fabsf(round_bf16(__fmul_rn(pmax, r)));      // = max |y| of the row, exactly
         uint16_t sb;
-        const float s_mul = quant_scale(amax_y, quant_mode, &sb);
+        const float s_mul = quant_scale(amax_y, quant_scale_mode(quant_mode), &sb);
         rstd_s[row] = r;
         smul_s[row] = s_mul;
         sval_s[row] = bf16_bits_to_float(sb);
@@ -73,8 +73,9 @@ __device__ __forceinline__ void chain_reduce_partials(const float2 (&part)[PN], 
     }
 }
 
-// NE (4 or 8) columns of one row: norm (NORM) + quantisation, packed int8 (NE / 4 dwords).  BOUNDED: the row's maximum is a caller's.
-template <int NE, bool NORM = true, bool BOUNDED = false>
+// NE (4 or 8) columns of one row: norm (NORM) + quantisation, packed int8 (NE / 4 dwords).  GIVEN: the mode may be
+// QUANT_ROUNDED_GIVEN.
+template <int NE, bool NORM = true, bool GIVEN = false>
 __device__ __forceinline__ void chain_quantise(const uint32_t (&hraw)[NE / 2], const uint32_t (&wraw)[NE / 2], float rstd, float s_mul, int quant_mode,
                                                uint32_t (&d)[NE / 4])
 {
@@ -90,7 +91,12 @@ __device__ __forceinline__ void chain_quantise(const uint32_t (&hraw)[NE / 2], c
     }
     if (quant_mode == QUANT_ROUNDED) {                       // uniform: one branch, not one per element
 #pragma unroll
-        for (int j = 0; j < NE / 4; ++j) d[j] = quant_rounded4<BOUNDED>(f[4 * j], f[4 * j + 1], f[4 * j + 2], f[4 * j + 3], s_mul);
+        for (int j = 0; j < NE / 4; ++j) d[j] = quant_rounded4(f[4 * j], f[4 * j + 1], f[4 * j + 2], f[4 * j + 3], s_mul);
+        return;
+    }
+    if (GIVEN && quant_mode == QUANT_ROUNDED_GIVEN) {
+#pragma unroll
+        for (int j = 0; j < NE / 4; ++j) d[j] = quant_rounded4<true>(f[4 * j], f[4 * j + 1], f[4 * j + 2], f[4 * j + 3], s_mul);
         return;
     }
 #pragma unroll

@@ -411,9 +411,9 @@ TERNA_FUNCTION(quant_from_stats, 4)
 }
 
 // (x, norm_weight | None, eps, packed, ws, ws_num, out_features, in_features, stats | None, attention splits (0: none), head_dim,
-//  quantised | None, epilogue, residual | None, next_norm_weight | None, want_raw, publish) -> the five tensors of
+//  quantised | None, epilogue, residual | None, next_norm_weight | None, want_raw, publish, own_stats) -> the five tensors of
 // linear.fused_linear, or None where the library does not take the combination
-TERNA_FUNCTION(fused_linear, 17)
+TERNA_FUNCTION(fused_linear, 18)
 {
     const char* who = "fused_linear";
     const at::Tensor &x = tensor(a[0]), &packed = tensor(a[3]), &ws = tensor(a[4]);
@@ -439,7 +439,7 @@ TERNA_FUNCTION(fused_linear, 17)
             if (x.scalar_type() != at::kChar || quantised->scalar_type() != at::kBFloat16)
                 refuse("%s: quantised activations are int8 with bf16 scales", who);
         } else {
-            d.prologue = stats != nullptr ? TERNASPMM_PROLOGUE_STATS : TERNASPMM_PROLOGUE_NORM;
+            d.prologue = stats == nullptr ? TERNASPMM_PROLOGUE_NORM : PyObject_IsTrue(a[17]) ? TERNASPMM_PROLOGUE_OWN_STATS : TERNASPMM_PROLOGUE_STATS;
             check_numel(who, "norm_weight", weight, k);
         }
     }

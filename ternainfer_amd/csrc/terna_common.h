@@ -53,7 +53,8 @@ struct RepackGuard {
 //   QUANT_EAGER     what the same lines give without torch.compile on bf16 tensors: every op rounds to bf16 --
 //                   s = bf16(bf16(1 / max(max|x|, bf16(1e-5))) * 127), q = rint(bf16(x * s)).
 // In every mode the s that is published (and that the epilogue divides by) is the bf16 value.
-enum QuantMode : int { QUANT_ROUNDED = 0, QUANT_COMPILED = 1, QUANT_EAGER = 2 };
+//   QUANT_ROUNDED_GIVEN   within kernels: QUANT_ROUNDED where the row's maximum is a caller's and need not be one.
+enum QuantMode : int { QUANT_ROUNDED = 0, QUANT_COMPILED = 1, QUANT_EAGER = 2, QUANT_ROUNDED_GIVEN = 3 };
 
 struct Epilogue {
     const uint16_t* s;      // bf16 [M]       (int8 family)
@@ -109,6 +110,8 @@ __device__ __forceinline__ float quant_scale(float amax, int mode, uint16_t* s_b
     *s_bits = float_to_bf16_bits(t);
     return mode == QUANT_COMPILED ? t : bf16_bits_to_float(*s_bits);
 }
+// The mode whose scale a row has that is quantised in `mode`.
+__device__ __forceinline__ int quant_scale_mode(int mode) { return mode == QUANT_ROUNDED_GIVEN ? static_cast<int>(QUANT_ROUNDED) : mode; }
 // One activation: clamp(rint(x * s_mul)), the product rounded to bf16 first in QUANT_EAGER.  Returned as a float in
 // [-128, 127].  Products are NaN only where the scale is NaN or 0 (see quant_scale), and there every integer is 0, which is what
 // the conversion of a NaN to int8 gives in torch: the median of a NaN and two bounds is the lower bound.
@@ -121,10 +124,11 @@ __device__ __forceinline__ float quant_value(float x, float s_mul, int mode)
 
 // Four activations in QUANT_ROUNDED, as packed int8: quant_value's integers in half its operations.  bf16 x bf16 is exact in
 // fp32, so one fused multiply-add with 1.5 * 2^23 rounds the product to the integer that stands in the low byte of the
-// sum.  No bound is needed where the kernel itself has taken the row's maximum: |x| is at most that and the scale within 2^-8 of 127
-// over it, so |x * s| < 127.5; and where the scale is NaN or 0 (a row that is not finite) the sum is a NaN, whose low byte is
-// 0 (bf16 payloads end above it), or exactly the constant.  BOUNDED: the maximum is a caller's, and a value above it gives 127 or
-// -128 as in quant_value, not the low byte of what it is (an instruction more an element: 8 sequences, 1528 slots 1198 -> 1210 us).  Every quantising launch and linear is a little shorter for it: decode step of one sequence 825 ->
+// sum.  No bound is needed where the maximum is the row's own: |x| is at most that and the scale within 2^-8 of 127 over
+// it, so |x * s| < 127.5; and where the scale is NaN or 0 (a row that is not finite) the sum is a NaN, whose low byte is
+// 0 (bf16 payloads end above it), or exactly the constant.  BOUNDED: the maximum may be less, and a value above it gives 127 or -128
+// as in quant_value, not the low byte of what it is (an instruction more an element: in the chained linears of 8 sequences, 1528 slots, 1198 -> 1210
+// us a step, so they say where the partials are their own).  Every quantising launch and linear is a little shorter for it: decode step of one sequence 825 ->
 // 809 us, 1 x 1920 tokens 6741 -> 6592, 5000 x 6912 rows of a module call 101.8 -> 99.5.
 template <bool BOUNDED = false>
 __device__ __forceinline__ uint32_t quant_rounded4(float x0, float x1, float x2, float x3, float s)

@@ -215,7 +215,7 @@ class FusedLinearDesc(ctypes.Structure):
                                                "next_norm_weight", "stats_out", "raw_out", "xq_out", "s_out", "s_in")]
 
 
-PROLOGUE_NORM, PROLOGUE_ATTENTION, PROLOGUE_STATS, PROLOGUE_QUANTISED = 0, 1, 2, 3
+PROLOGUE_NORM, PROLOGUE_ATTENTION, PROLOGUE_STATS, PROLOGUE_QUANTISED, PROLOGUE_OWN_STATS = 0, 1, 2, 3, 4
 EPILOGUE_STORE, EPILOGUE_RESIDUAL, EPILOGUE_GATE = 0, 1, 2
 
 
@@ -264,16 +264,17 @@ def interleave_gate_up(packed, out_features, in_features):
 
 
 def fused_linear(x, norm_weight, eps, packed, ws, ws_num, out_features, in_features, *, stats=None, attention=None, quantised=None,
-                 epilogue=EPILOGUE_STORE, residual=None, next_norm_weight=None, want_raw=False, publish=False):
+                 epilogue=EPILOGUE_STORE, residual=None, next_norm_weight=None, want_raw=False, publish=False, own_stats=False):
     """One launch of ternaspmm_fused_linear (include/ternaspmm.h): prologue -> ternary matmul on a P2 weight -> epilogue.
-    x: h bf16 [M, K], with `stats` (fp32 [M, count, 2]) when its producer left the norm statistics; or, with
+    x: h bf16 [M, K], with `stats` (fp32 [M, count, 2]) when its producer left the norm statistics (`own_stats`: no value
+    lies above the maximum they name, and none is clamped to it); or, with
     `attention` = (splits, head_dim), the fp32 partial results of a split attention launch (one sequence); or, with
     `quantised` = s (bf16 [M]), int8 activations that are quantised already (norm_weight is then not used).
     Returns (out, stats_out, raw, xq, s) -- stats_out for the producing epilogues, raw with `want_raw`, (xq, s) with
     `publish`, None otherwise -- or None when the library does not support the combination (nothing was enqueued)."""
     splits, head_dim = attention if attention is not None else (0, 0)
     return _lib.native().fused_linear(x, norm_weight, eps, packed, ws, ws_num, out_features, in_features, stats, splits, head_dim,
-                                      quantised, epilogue, residual, next_norm_weight, want_raw, publish)
+                                      quantised, epilogue, residual, next_norm_weight, want_raw, publish, own_stats)
 
 
 def lm_head(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:

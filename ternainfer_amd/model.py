@@ -242,7 +242,7 @@ class Block:
             if stats is None:                       # (recording: the first block's statistics as a launch of their own)
                 stats = row_stats(x, self.attention_norm)
             r = fused_linear(x, self.attention_norm, a.norm_eps, self.wqkv.packed, self.wqkv.ws, self.wqkv.ws_num, self.wqkv.n, self.wqkv.k,
-                             stats=stats, publish=pub)
+                             stats=stats, own_stats=True, publish=pub)
             note("wqkv", r)
             qkv = r[0]
         deferred = isinstance(attn_ws, tuple)
@@ -297,7 +297,7 @@ class Block:
             r = None
             if bsz <= self.o_norm_rows:          # the sub-norm's statistics taken inside the O projection (or given by the attention)
                 r = fused_linear(o, self.attn_sub_norm, a.norm_eps, self.wo.packed, self.wo.ws, self.wo.ws_num, self.wo.n, self.wo.k,
-                                 stats=o_stats, **o_kw)
+                                 stats=o_stats, own_stats=True, **o_kw)
             if r is None:                        # more rows: the norm kernel (or the quantise launch), then the O projection on quantised rows
                 if o_stats is not None:
                     xq, s = quant_from_stats(o, o_stats, self.attn_sub_norm, a.norm_eps)
@@ -315,7 +315,7 @@ class Block:
             r = (r[0], r[1], None, xq, s)
         else:
             r = fused_linear(h, self.ffn_norm, a.norm_eps, self.gate_up_interleaved(), self.w13.ws, self.w13.ws_num, self.w13.n, self.w13.k,
-                             stats=h_stats, epilogue=EPILOGUE_GATE, next_norm_weight=self.ffn_sub_norm, publish=pub)
+                             stats=h_stats, own_stats=True, epilogue=EPILOGUE_GATE, next_norm_weight=self.ffn_sub_norm, publish=pub)
         note("w13", r)
         inner, inner_stats = r[0], r[1]
         if split or bsz > self.chain_down_rows:
@@ -327,7 +327,7 @@ class Block:
             r = (r[0], r[1], r[2], xq, s)
         else:
             r = fused_linear(inner, self.ffn_sub_norm, a.norm_eps, self.w2.packed, self.w2.ws, self.w2.ws_num, self.w2.n, self.w2.k,
-                             stats=inner_stats, epilogue=EPILOGUE_RESIDUAL, residual=h, next_norm_weight=next_norm, want_raw=pub, publish=pub)
+                             stats=inner_stats, own_stats=True, epilogue=EPILOGUE_RESIDUAL, residual=h, next_norm_weight=next_norm, want_raw=pub, publish=pub)
         note("w2", r)
         return r[0], r[1]
 

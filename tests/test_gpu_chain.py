@@ -449,6 +449,19 @@ def test_reducing_waves_of_five_to_eight_rows(m, k, count):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("m,k", [(1, 2560), (2, 192), (5, 2560), (8, 2560), (8, 6912)])
+def test_partials_of_the_rows_own_need_no_clamp(m, k):
+    """own_stats: the same bits where the partials are those of the rows."""
+    n = 256
+    packed, ws = _packed(make_ternary(n, k, 0.4, 1280 + k)), _bf(WS)
+    h, g, nxt, res = _bf(make_bf16_activations(m, k, 1281)), _bf(_weight(k, 1282)), _bf(_weight(n, 1283)), _bf(make_bf16_activations(m, n, 1284))
+    stats = L.row_stats(h, g)
+    kw = dict(stats=stats, publish=True, epilogue=L.EPILOGUE_RESIDUAL, residual=res, next_norm_weight=nxt, want_raw=True)
+    given, own = (L.fused_linear(h, g, 1e-5, packed, ws, 1, n, k, own_stats=o, **kw) for o in (False, True))
+    for a, b in zip(given, own):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("mode", [0, 1, 2])
 @pytest.mark.parametrize("m,k", [(1, 192), (1, 2560), (2, 2560), (4, 6912), (5, 2560), (8, 2560), (8, 6912)])
 def test_a_given_maximum_below_the_rows_own_saturates(m, k, mode):
