@@ -415,7 +415,7 @@ class Block:
         return x, ffn
 
 
-#: switches of the chained step whose other settings ask for its launches one by one (Transformer.whole_step)
+#: switches of the chained step, of the model and of each block, whose other settings ask for its launches one by one (Transformer.whole_step)
 _STEP_SWITCHES = (("step_inputs", True), ("deferred_attention_merge", True), ("attention_splits", None), ("split_merge_quant", False), ("defer_above", 640),
                   ("chain_rows", 8))
 _CHAIN_SWITCHES = (("o_norm_rows", 8), ("attention_stats_chain", True), ("attention_stats", True), ("merge_quant", True), ("chain_down_rows", 2))
@@ -563,15 +563,15 @@ class Transformer:
     def whole_step(self, tokens, cache, pos_idx, max_seq):
         """The residual stream behind the last block of a single-token step of up to four sequences, all blocks in one launch
         (ternaspmm_decode_step), or None: where the library does not take the shape, and where something asks for the launches it
-        stands for -- a recording block, a switch of the chain that is not at its default.  (Not `enable_prefetch`: the step fetches its
+        stands for -- a recording block, a switch of the chain that is not at its default, on the model or on one of its blocks.  (Not `enable_prefetch`: the step fetches its
         weights ahead by itself; one sequence, 384 slots, with prefetching launches 819 us, so 653, bookkeeping included.)  The same bits as
         those launches (Block.forward_chain with `split` False, for two sequences and more with the attention in one piece)."""
         a = self.args
         bsz = tokens.shape[0]
         if bsz > self.chain_rows or bsz > 4 or not self.one_launch_step or not a.rope_adjacent or a.head_dim != 128 or \
                 any(getattr(self, name, default) != default for name, default in _STEP_SWITCHES) or \
-                any(getattr(Block, name) != default for name, default in _CHAIN_SWITCHES) or \
-                any(blk.capture is not None or not blk.fused or blk.act != "int8" or type(blk) is not Block for blk in self.layers):
+                any(blk.capture is not None or not blk.fused or blk.act != "int8" or type(blk) is not Block or
+                    any(getattr(blk, name) != default for name, default in _CHAIN_SWITCHES) for blk in self.layers):
             return None
         splits = 1
         if bsz == 1:

@@ -118,6 +118,22 @@ def test_rows_that_are_not_finite(m):
         assert same(got[1:], want[1:]) and torch.isfinite(got[1:, :7].float()).all()
 
 
+def test_a_switch_of_one_block_asks_for_the_launches():
+    """As one of the model, or of all blocks, does: whoever sets it times or checks the launches."""
+    from ternainfer_amd.model import _CHAIN_SWITCHES, Block
+    model = build(TINY, 3)
+    whole, tokens, pos = state(model, 2, 40, [11])
+    cache = [(whole[i, 0], whole[i, 1]) for i in range(3)]
+    with torch.inference_mode():
+        for name, default in _CHAIN_SWITCHES:
+            assert getattr(Block, name) == default
+            setattr(model.layers[1], name, (not default) if isinstance(default, bool) else default - 1)
+            assert model.whole_step(tokens, cache, pos, 40) is None, name
+            assert torch.isfinite(model.forward(tokens, cache, pos).float()).all()
+            delattr(model.layers[1], name)
+            assert model.whole_step(tokens, cache, pos, 40) is not None, name
+
+
 def test_more_blocks_than_a_launch_takes():
     model = build(TINY, 65)
     check(model, *state(model, 1, 64, [33]))
