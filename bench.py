@@ -244,7 +244,7 @@ def cpu_baseline(mats, torch):
 
 
 # ------------------------------------------------------------------------------------------------ model
-def measure_model(torch, batch, act="int8", prefetch=True, gen_tokens=256, check_tokens=8, model=None, prompt_tokens=128, chain=True):
+def measure_model(torch, batch, act="int8", prefetch=True, gen_tokens=256, check_tokens=8, model=None, prompt_tokens=128, chain=True, one_launch=True):
     """2B-shaped random-init model, prompt of `prompt_tokens` (128) uniform random ids, greedy decode of `gen_tokens`
     tokens; tokens/s = generated tokens / decode-phase time (as the reference's stats.py:19-27).
     Self-check of the run: the captured decode graph must produce the tokens of eager execution
@@ -255,6 +255,7 @@ def measure_model(torch, batch, act="int8", prefetch=True, gen_tokens=256, check
     if model is None:
         model = Transformer(margs, seed=20260500, act=act)
     model.chain = chain
+    model.one_launch_step = one_launch
     if os.environ.get("TERNA_BENCH_CHAIN_ROWS"):           # measurement aids
         model.chain_rows = int(os.environ["TERNA_BENCH_CHAIN_ROWS"])
     if os.environ.get("TERNA_BENCH_SPLIT_ROWS"):
@@ -295,7 +296,10 @@ def measure_model(torch, batch, act="int8", prefetch=True, gen_tokens=256, check
     assert graph_equals_eager, "decode graph and eager execution disagree"
     toks, prefill_s, decode_s = greedy_decode(model, prompt, gen_tokens)
     assert torch.equal(toks[:, :check_tokens], eager)
-    return {"batch": batch, "tokens_per_s": batch * gen_tokens / decode_s, "ms_per_step": decode_s * 1e3 / gen_tokens,
+    slots = prompt_tokens + gen_tokens
+    with torch.inference_mode():                                                # whether the decode steps were one launch each
+        in_one = chain and model.whole_step(prompt[:, :1], model.make_cache(batch, slots), torch.zeros(1, dtype=torch.int64, device="cuda"), slots) is not None
+    return {"batch": batch, "step_in_one_launch": in_one, "tokens_per_s": batch * gen_tokens / decode_s, "ms_per_step": decode_s * 1e3 / gen_tokens,
             "prefill_tokens_per_s": batch * prompt_tokens / prefill_s, "prefill_ms": prefill_s * 1e3, "decode_s": decode_s,
             "prompt_tokens": prompt_tokens,
             "generated_tokens": gen_tokens, "graph_equals_eager_first_tokens": check_tokens,
@@ -306,7 +310,8 @@ def run_model(args, torch):
     act = args.act or "int8"
     gen = 256 if args.prompt_tokens <= 128 else 128
     fig, _ = measure_model(torch, args.batch, act, not args.no_prefetch, gen_tokens=gen, prompt_tokens=args.prompt_tokens,
-                           chain=not args.no_chain)
+                           chain=not args.no_chain, one_launch=not args.no_one_launch)
+    in_one = fig["step_in_one_launch"]
     return {
         "metric": "2B-shape decode tok/s", "value": fig["tokens_per_s"], "unit": "tokens/s", "n_gpus": 1, "steps": gen, "warmup": 8,
         "ms_per_step": fig["ms_per_step"], "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
@@ -317,16 +322,17 @@ def run_model(args, torch):
                                "decode step; norms, gate, activation quantisation, RoPE, cache write, single-token "
                                "attention, the multi-token attention of the prompt pass, the bf16 LM head and greedy "
                                "sampling are library kernels; the prompt pass is one HIP graph too"
-                               + ("; one sequence: the attention is split over several workgroups per head and the O "
+                               + ("; every block of a decode step in one launch, which fetches its weights ahead by itself" if in_one else
+                                  "; one sequence: the attention is split over several workgroups per head and the O "
                                   "projection's prologue merges the partial results" if args.batch == 1 else
                                   ("" if args.no_prefetch or args.batch > 2 else "; the idle CUs of the attention launch "
                                                                                  "prefetch the weights of the launches that follow"))
-                               + ("" if args.no_chain or args.batch > 8 else
+                               + ("" if in_one or args.no_chain or args.batch > 16 else
                                   "; the linears are chained through producer-side norm statistics"
-                                  + (" (consumed inside the next linear)" if args.batch <= 4 else
-                                     " (consumed by an element-wise quantise launch in front of the next linear)")),
+                                  + (" (consumed inside the next linear; from three sequences on by a quantise launch in front of the down projection)"
+                                     if args.batch <= 8 else " (consumed by an element-wise quantise launch in front of the next linear)")),
                    "batch": args.batch, "act": act},
-        **{k: fig[k] for k in ("prefill_tokens_per_s", "prefill_ms", "decode_s", "model_build_s", "first_tokens",
+        **{k: fig[k] for k in ("prefill_tokens_per_s", "prefill_ms", "decode_s", "model_build_s", "first_tokens", "step_in_one_launch",
                                "graph_equals_eager_first_tokens")}}
 
 
@@ -746,7 +752,10 @@ def main():
                     help="packed: weights repacked once at load time to the library's P2 layout (bit-exact); "
                          "reference: kernels read the reference's compressed format directly")
     ap.add_argument("--no-prefetch", action="store_true",
-                    help="model workload: no weight prefetch by the idle CUs of the attention launch")
+                    help="model workload: no weight prefetch by the idle CUs of the attention launch (up to two sequences, where the decode step "
+                         "is launches: --no-one-launch, --no-chain, bf16, longer caches)")
+    ap.add_argument("--no-one-launch", action="store_true",
+                    help="model workload: the decode step of up to four sequences as the launches it stands for")
     ap.add_argument("--no-chain", action="store_true",
                     help="model workload: the decode step without producer-side norm statistics (every linear re-derives them)")
     ap.add_argument("--no-cpu-baseline", action="store_true")

@@ -138,6 +138,7 @@ def test_toy_model_prompts_of_different_lengths_in_one_batch(head_dim, prefetch)
     args = ModelArgs(dim=4 * head_dim, n_layers=2, n_heads=4, n_kv_heads=2, vocab_size=1024, ffn_dim=384)
     model = Transformer(args, seed=31, act="int8")
     model.enable_prefetch(prefetch)
+    model.one_launch_step = not prefetch          # (the one launch has no attention launch whose idle CUs could prefetch)
     lens = [5, 12, 9]
     gen = torch.Generator().manual_seed(32)
     prompts = [torch.randint(0, args.vocab_size, (1, n), generator=gen).cuda() for n in lens]

@@ -313,15 +313,19 @@ def test_full_size_blocks_match_cpu_twin_layer_by_layer(full_model, bsz):
             print(f"[info] batch {bsz} pass {pi} logits: {r}", flush=True)
 
 
-@pytest.mark.parametrize("bsz", [1, 8, 12, 16])
-def test_full_size_decode_graph_gives_the_tokens_of_eager_execution(full_model, bsz):
+@pytest.mark.parametrize("bsz,one_launch", [(1, True), (1, False), (4, True), (8, True), (12, True), (16, True)])
+def test_full_size_decode_graph_gives_the_tokens_of_eager_execution(full_model, bsz, one_launch):
+    """`one_launch` False: one sequence through the launches, whose attention prefetches the weights of those behind it (the step in
+    one launch, which up to four sequences take otherwise, does that by itself)."""
     from ternainfer_amd.model import greedy_decode
     args, model, _ = full_model
     prompt = torch.randint(0, args.vocab_size, (bsz, PROMPT), generator=torch.Generator().manual_seed(20260510 + bsz)).cuda()
     model.enable_prefetch(True, ("wo", "w13", "w2", "next_wqkv", "norms") if bsz == 1 else ("wo", "w13"))
-    print(f"[case] full-size greedy decode batch {bsz}: graph vs eager, 16 tokens", flush=True)
+    model.one_launch_step = one_launch
+    print(f"[case] full-size greedy decode batch {bsz} one launch {one_launch}: graph vs eager, 16 tokens", flush=True)
     a, _, _ = greedy_decode(model, prompt, 16, use_graph=True)
     b, _, _ = greedy_decode(model, prompt, 16, use_graph=False)
+    model.one_launch_step = True
     model.enable_prefetch(False)
     assert torch.equal(a, b)
     assert int(a.min()) >= 0 and int(a.max()) < args.vocab_size
