@@ -411,11 +411,10 @@ TERNA_FUNCTION(quant_from_stats, 4)
 }
 
 // (x, norm_weight | None, eps, packed, ws, ws_num, out_features, in_features, stats | None, attention splits (0: none), head_dim,
-//  quantised | None, epilogue, residual | None, next_norm_weight | None, want_raw, publish, own_stats) -> the five tensors of
+//  quantised | None, epilogue, residual | None, next_norm_weight | None, want_raw, publish) -> the five tensors of
 // linear.fused_linear, or None where the library does not take the combination
-TERNA_FUNCTION(fused_linear, 18)
+PyObject* chained_linear(const char* who, bool own_stats, PyObject* const* a)
 {
-    const char* who = "fused_linear";
     const at::Tensor &x = tensor(a[0]), &packed = tensor(a[3]), &ws = tensor(a[4]);
     const at::Tensor *weight = optional(a[1]), *stats = optional(a[8]), *quantised = optional(a[11]), *residual = optional(a[13]), *next_weight = optional(a[14]);
     const int64_t n = integer32(a[6]), k = integer32(a[7]);
@@ -439,7 +438,7 @@ TERNA_FUNCTION(fused_linear, 18)
             if (x.scalar_type() != at::kChar || quantised->scalar_type() != at::kBFloat16)
                 refuse("%s: quantised activations are int8 with bf16 scales", who);
         } else {
-            d.prologue = stats == nullptr ? TERNASPMM_PROLOGUE_NORM : PyObject_IsTrue(a[17]) ? TERNASPMM_PROLOGUE_OWN_STATS : TERNASPMM_PROLOGUE_STATS;
+            d.prologue = stats == nullptr ? TERNASPMM_PROLOGUE_NORM : own_stats ? TERNASPMM_PROLOGUE_OWN_STATS : TERNASPMM_PROLOGUE_STATS;
             check_numel(who, "norm_weight", weight, k);
         }
     }
@@ -487,6 +486,10 @@ TERNA_FUNCTION(fused_linear, 18)
     if (lib.ternaspmm_fused_linear(&d, stream()) < 0) return none(unlocked);
     return pack(unlocked, std::move(out), std::move(stats_out), std::move(raw), std::move(xq), std::move(s));
 }
+
+TERNA_FUNCTION(fused_linear, 17) { return chained_linear("fused_linear", false, a); }
+// The same where `stats` are the rows' own (TERNASPMM_PROLOGUE_OWN_STATS).
+TERNA_FUNCTION(fused_linear_own_stats, 17) { return chained_linear("fused_linear_own_stats", true, a); }
 
 // What the attention entry points read beside a block's new rows, checked against these and each other.
 struct AttentionArgs {
@@ -897,7 +900,7 @@ TERNA_FUNCTION(init, 1)
 #define METHOD(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(name)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {METHOD(init), METHOD(bit_linear), METHOD(bit_linear_bf16), METHOD(quant_input), METHOD(linear_packed),
                          METHOD(linear_bf16_packed), METHOD(rmsnorm_quant), METHOD(relu2_mul_rmsnorm_quant), METHOD(quant_from_stats),
-                         METHOD(fused_linear), METHOD(prompt_attention), METHOD(decode_attention), METHOD(block),
+                         METHOD(fused_linear), METHOD(fused_linear_own_stats), METHOD(prompt_attention), METHOD(decode_attention), METHOD(block),
                          METHOD(attention_merge_rmsnorm_quant), METHOD(step_attention_merge), METHOD(step_inputs), METHOD(prompt_inputs), METHOD(decode_step), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -273,8 +273,9 @@ def fused_linear(x, norm_weight, eps, packed, ws, ws_num, out_features, in_featu
     Returns (out, stats_out, raw, xq, s) -- stats_out for the producing epilogues, raw with `want_raw`, (xq, s) with
     `publish`, None otherwise -- or None when the library does not support the combination (nothing was enqueued)."""
     splits, head_dim = attention if attention is not None else (0, 0)
-    return _lib.native().fused_linear(x, norm_weight, eps, packed, ws, ws_num, out_features, in_features, stats, splits, head_dim,
-                                      quantised, epilogue, residual, next_norm_weight, want_raw, publish, own_stats)
+    call = _lib.native().fused_linear_own_stats if own_stats else _lib.native().fused_linear
+    return call(x, norm_weight, eps, packed, ws, ws_num, out_features, in_features, stats, splits, head_dim, quantised, epilogue, residual,
+                next_norm_weight, want_raw, publish)
 
 
 def lm_head(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:

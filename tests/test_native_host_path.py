@@ -10,7 +10,7 @@ from ternainfer_amd import _lib, linear
 ATTENTION = "TTTTTiifi"
 SIGNATURES = {
     "bit_linear": "ToTTTTTiio", "bit_linear_bf16": "TTTTTTiii", "quant_input": "T", "linear_packed": "TTTTiio", "linear_bf16_packed": "TTTiio",
-    "rmsnorm_quant": "TTfob", "relu2_mul_rmsnorm_quant": "TTfb", "quant_from_stats": "TTTf", "fused_linear": "TofTTiiioiioioobb",
+    "rmsnorm_quant": "TTfob", "relu2_mul_rmsnorm_quant": "TTfb", "quant_from_stats": "TTTf", "fused_linear": "TofTTiiioiioioobb", "fused_linear_own_stats": "TofTTiiioiioioobb",
     "prompt_attention": "T" + ATTENTION + "b", "decode_attention": "T" + ATTENTION + "oooi",
     "block": "To" + ATTENTION + "foo" + "TTTT" + "TTii" * 4 + "o", "attention_merge_rmsnorm_quant": "TiiiTfib", "step_inputs": "TTTTT",
     "prompt_inputs": "TTTT",
@@ -32,7 +32,7 @@ def _arguments(name):
         values[14:18] = [bf(64)] * 4
         for at, n in ((18, 192), (22, 64), (26, 128), (30, 64)):
             values[at:at + 4] = [torch.zeros(n * 16, dtype=torch.int8), bf(4), 1, n]
-    if name == "fused_linear":
+    if name.startswith("fused_linear"):
         values[7] = 64
     return values
 
