@@ -569,7 +569,7 @@ void ternaspmm_relu2_mul_rmsnorm_quant_ahead(const terna_bf16* x13, const terna_
 
 /* The pair for any split count from 1 to 8, as a decode step of several sequences launches it: ternaspmm_step_attention is
  * ternaspmm_rope_decode_attention_partial, ternaspmm_step_attention_merge is ternaspmm_attention_merge_rmsnorm_quant;
- * both return 0, or -1 with nothing enqueued (next: as above).  ternaspmm_step_attention_splits(B, H, KV, S): the count that fills the chip
+ * both return 0, or -1 with nothing enqueued (next: as above).  ternaspmm_step_attention_splits(B, H, KV, S): the count that fills the chip's 256 CUs
  * (one sequence, or other than 2 or 4 heads per kv head: ternaspmm_attention_partial_splits_kv). */
 int ternaspmm_step_attention_splits(int B, int H, int KV, int S);
 int ternaspmm_step_attention(const terna_bf16* qkv, const float* cos, const float* sin, const long long* pos, int per_sequence,

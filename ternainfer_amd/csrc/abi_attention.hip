@@ -175,9 +175,11 @@ void launch_attention(const uint16_t* q, uint16_t* ck, uint16_t* cv, const float
                              AttentionStats stats = AttentionStats{nullptr, nullptr})
 {
     const int splits = attention_splits(B, H, S, scratch);
-    // More heads than two a CU: the heads of a kv group in one workgroup, which loads their keys and values once instead of four times
-    // (32 sequences, 512 slots: launch 12.8 -> 10.5 us; 48, 1024 slots: step 2046 -> 1790; 64, 512 slots: 2104 -> 1866).  Fewer heads fill
-    // the chip by themselves (20 sequences, 512 slots: 1607 us a step either way).
+    // More heads than two a CU: the heads of a kv group in one workgroup, which loads their keys and values once instead of four times.
+    // Us a step, a workgroup a head -> a kv group, caches filled to 90 - 95 % unless it says otherwise: 26 sequences, 900 slots to 60 % 1901 -> 1665; 48, 1000
+    // 2980 -> 1980; 64, 512 to 60 % 2047 -> 1826, 1280 3173 -> 2561, 2048 4230 -> 3316.  From about 2700 slots on the scores of four heads leave one
+    // workgroup of four waves a CU, which is still ahead: 64, 3072 5420 -> 5185, 4096 6690 -> 6225 (to 50 % 4295 -> 4050), 7168 10340 -> 9800 (to 50 % 6300 -> 5917);
+    // 52, 6144 8700 -> 8546; 128, 4096 11161 -> 8665.  Fewer heads fill the chip by themselves (20 sequences, 512 slots: 1607 us a step either way).
     {
         const bool crowded = splits == 1 && stats.out == nullptr && static_cast<long>(B) * H > 512;
         if (crowded && D == 128 && launch_attention_grouped<128, ROPE, ADJ, true>(q, ck, cv, cos, sin, pos, per_seq, nullptr, out, 1, B, H, KV, S, scale, pf, st)) return;
@@ -452,6 +454,7 @@ int ternaspmm_step_attention_splits(int B, int H, int KV, int S)
 {
     if (B < 1 || H < 1 || KV < 1 || H % KV != 0 || S < 1) return -1;
     const int gq = H / KV;
+    // (256, 512: workgroups on a whole MI355X's 256 CUs, here and where attention is launched; a stream with a mask of fewer gives the same results.)
     // The grid of the grouped kernel is B * KV * splits workgroups that each have a CU to themselves, so as many splits as the chip
     // holds -- the tiles go round, whatever their number -- of 160 slots at least, below which another one costs the merge more than
     // it saves (16 sequences, 384 slots: two 1225 us, three 1238).  The 2B shape, us a step, powers of two -> this: 16 sequences, 1528

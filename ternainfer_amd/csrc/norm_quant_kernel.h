@@ -187,9 +187,10 @@ __device__ __forceinline__ void norm_quant_passes(float (&h)[NV][8], const u32x4
 // Spare workgroups of a launch that norms and quantises rows bring the packed weights of the linear behind it into the L2s while its few
 // workgroups wait for memory and each other: the linear then starts on data that is one L2 trip away instead of one to HBM (a model's
 // weights are read once per pass and twice the size of the last cache).  A load of four bytes fetches a line; nobody waits for it but
-// the end of the launch.  Measured, us, without -> with: decode step of 32 sequences x 512 slots 1540 -> 1494, of 64 1815 -> 1735, prompts of 100, 300,
-// 1000 and 1920 tokens 1616 -> 1575, 2324 -> 2225, 4307 -> 4195, 6549 -> 6434; 8 sequences x 1528 slots, in the launch that also merges
-// the attention's splits, 1249 -> 1243.  Tried: weights of the launch after next as well, or instead (32 sequences 1505 - 1531), 64 workgroups
+// the end of the launch.  Measured in turn, us, without -> with: decode step of 32 sequences x 512 slots of different lengths 1567 -> 1501, of one length
+// 1588 -> 1519, 64 x 512 1905 -> 1817, 64 x 1000 2159 -> 2073; prompts of 100 and 1920 tokens 1614 -> 1581 and 6576 -> 6444; in the launch that also
+// merges the attention's splits 8 x 1528 slots 1214 -> 1199, 16 x 1528 1361 -> 1354.  (Cards differ: the first of these with 1500 - 1540, the 1920 tokens with 6440 - 7050.)
+// Tried: weights of the launch after next as well, or instead (32 sequences 1505 - 1531), 64 workgroups
 // (1525) and 384 (1508); in the shorter launch that quantises from a producer's statistics (up to 16 rows) it costs 5 - 20 us
 // a step, in the quantisation in front of a linear module's call it is level.
 __device__ __forceinline__ void fetch_next_weights(const NextWeights& next, int first)

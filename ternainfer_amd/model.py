@@ -435,7 +435,8 @@ class Transformer:
     # norm kernels, which reduce over the row twice, and the gate+up launch writes F columns instead of 2F.
     split_rows = 16
     # Cache slots from which on a chained step of two to four sequences (more: 512) splits its attention and leaves the merge to a
-    # launch of its own (measured, 4 sequences: 428 slots 1.041 ms per step unsplit against 1.115, 728 slots 1.154 against 1.120)
+    # launch of its own, where the step is launches: us a step, unsplit -> split, filled to 60 and to 95 %: 2 sequences at 640 slots 949 -> 988 and 1037 ->
+    # 1006, 4 at 640 991 -> 1032 and 1077 -> 1050, at 1400 1182 -> 1062 and 1359 -> 1083
     defer_above = 640
 
     def __init__(self, args: ModelArgs, seed: int = 0, act: str = "int8", p_zero: float = 0.40):
@@ -629,14 +630,14 @@ class Transformer:
         pending = None
         attn_ws = self.attention_workspace(bsz) if one_launch_attention else None     # layers run one after another: shared
         split = chain and bsz > self.chain_rows
-        # split attention whose merge is left to its consumer: always for one sequence (the O projection's prologue merges);
-        # for more only with long caches, where the shorter attention launch pays for the merge launch (8 sequences at slot
-        # 1500: 1943 -> 1713 us per step; at slot 255 of 384 the pair of launches is 1.5 us slower than the unsplit one) --
-        # (in the split chain that merge launch also norms and quantises the O projection's input; with short caches
-        # the unsplit launch + the O projection with the norm inside stay ahead there too: 8 sequences, slot 255 of 384,
-        # 1.198 against 1.218 ms per step -- `split_merge_quant` forces the split form)
-        # With more heads than CUs already from 256 slots on (14 sequences, 384 slots: 1303 -> 1217 us a step; 20, 512: 1607 -> 1500; at 256 slots
-        # level), where the chip holds two splits of every kv head and more.
+        # Split attention whose merge is left to its consumer: always for one sequence (the O projection's prologue merges); for more, where the
+        # attention is shorter by more than the merge launch costs.  That launch also norms and quantises the O projection's rows, which unsplit
+        # up to eight sequences the projection does itself from the attention's partial statistics.  The lines lie between caches filled to
+        # 60 and to 95 %.  Us a step, unsplit -> split: two to four sequences (`defer_above`); 5 at 512 slots 1049 -> 1082 and 1080 -> 1099, at 640 1059 -> 1082
+        # and 1149 -> 1100; 8 at 512 1088 -> 1111 and 1119 -> 1128, at 640 1097 -> 1119 and 1188 -> 1138, at 1528 1303 -> 1163 and 1508 -> 1209; 12 at
+        # 512 1208 -> 1218 and 1237 -> 1234, at 640 1221 -> 1235 and 1310 -> 1250.  With more heads than the 256 CUs already from 256 slots
+        # on, where both are level: 14 at 384 1320 -> 1217 and 1409 -> 1240, 16 at 384 1331 -> 1227 and 1415 -> 1249, 20 at 512 1654 -> 1466 and 1712 ->
+        # 1516.  `split_merge_quant`: the split form of 9 to 16 sequences whatever the length.
         short = 256 if bsz * a.n_heads > 256 else 512 if chain and bsz > 4 else self.defer_above
         if one_launch_attention and self.layers[0].act == "int8" and (bsz == 1 or max_seq > short):
             attn_ws = self.attention_partial(bsz, max_seq) or attn_ws
