@@ -8,8 +8,8 @@
 // of them reads 0xffffffff any more.  That word is a pair of NaNs no producer writes (step_word).  There is no counter, no fence
 // and no second trip for the data.  A handover alone: 1.44 us from one poll to the next (160 workgroups, 32-byte slices, 5 KB;
 // 256 writers of 20 bytes each, which share lines, 1.95).
-// Measured, us a step of 30 blocks of the 2B shape with the LM head, launches -> this: one sequence, 384 slots 809 -> 643, 4096 slots
-// 1022 -> 837; two, 384 slots 890 -> 725; three, 101 slots 882 -> 795; four, 384 slots 936 -> 846.
+// Measured, us a step of 30 blocks of the 2B shape with the LM head, launches -> this: one sequence, 384 slots 813 -> 640, 4096 slots
+// filled to 50 % 920 -> 766, to 90 % 1132 -> 867; two, 384 slots 895 -> 732; three, 101 slots 885 -> 798; four, 384 slots 939 -> 856.
 //
 // Bound: what is left of the handovers (0.7 - 1.3 us each, five or six a block), and behind each wait the instructions of one wave per
 // SIMD, 4 - 8 cycles apiece: 1.6 - 2.7 us a phase.  Hence, in the order of what they gave:
@@ -50,9 +50,9 @@ constexpr int kStepMaxBlocks = 32;               // blocks per launch: their poi
 constexpr int kStepMaxSplits = 8;                // splits of the cache, one sequence; four at a time are merged
 constexpr int kStepRecord = (kStepHeadDim + 4) * 4;      // bytes a (head, split) hands over: 128 sums, maximum, sum of numerators
 // Slots of a cache that is not split; of a split.  Every (sequence, head, half) walks its whole prefix, so the lines lie where that takes as
-// long as the launches with the attention split over the chip (us a step, caches filled to 90 %, those -> this: two sequences, 700 slots
-// 1004 -> 833, 1024 1012 -> 915, 1528 1033 -> 1052; three, 1024 1044 -> 1018, 1528 1066 -> 1145; four, 700 1044 -> 966, 1024 1058 -> 1043,
-// 1528 1078 -> 1174; filled to half 15 - 23 % ahead at two, 6 - 12 % at four).
+// long as the launches with the attention split over the chip (us a step, caches filled to 90 %, those -> this: two sequences, 1280 slots
+// 1027 -> 945; three, 1024 1052 -> 985; four, 700 1054 -> 939, 1024 1064 -> 1012, filled to half 1045 -> 910.  With 1528 slots two 1033 -> 1052,
+// three 1066 -> 1145, four 1078 -> 1174, taken before each XCD fetched what its own workgroups read, which gave 30 - 40 at the lines; they are where they were).
 constexpr int step_max_slots(int M) { return M == 2 ? 1280 : 1024; }
 constexpr int kStepMaxSplitSlots = 1024;
 constexpr uint32_t kStepEmpty = 0xffffffffu;
