@@ -146,16 +146,20 @@ bool launch_attention_grouped(const uint16_t* qkv, uint16_t* ck, uint16_t* cv, c
     if (gq != 2 && gq != 4) return false;
     const int slots = B * KV * splits;
     const int waves = forced ? forced : slots <= 256 ? 8 : 4;
-    const size_t lds = grouped_attention_lds_bytes(D, waves, gq, S);
-    if (lds > 159 * 1024) return false;          // (160 KB per workgroup, the kernel's static LDS included)
     AttentionPrefetch pf = pf_in;
     pf.workgroups = prefetch_workgroups(pf, slots);
+    constexpr int kLds = 160 * 1024;
+    if (KV > 0xffff || static_cast<long long>(slots) * (KV > splits ? KV : splits) >= 1ll << 31) return false;     // (numbers the kernel divides)
+    auto inverse = [](int d) { return d > 1 ? static_cast<uint32_t>((0xffffffffull + d) / d) : 0u; };
 #define TERNA_GROUPED(NWAVES, GQ)                                                                                          \
     do {                                                                                                                   \
         auto kernel = terna_decode_attention_grouped_kernel<D, ROPE, ADJ, NWAVES, GQ, WHOLE>;                                    \
-        if (lds > 64 * 1024) allow_dynamic_lds(kernel, 159 * 1024, "hipFuncSetAttribute(decode attention, kv groups)", __LINE__); \
-        kernel<<<dim3(slots + pf.workgroups), dim3(64 * NWAVES), lds, st>>>(qkv, ck, cv, pos, KV, S, splits, slots, per_seq, scale, cos, sin, \
-                                                                            partial, out, pf);                             \
+        const int lds = GroupedShape<D, NWAVES, GQ>::bytes(16 * (((S + 15) / 16 + splits - 1) / splits));                     \
+        if (lds > kLds) return false;                                                                                          \
+        allow_dynamic_lds(kernel, kLds, "hipFuncSetAttribute(decode attention, kv groups)", __LINE__);                          \
+        const uint32_t shape = KV | splits << 16 | (per_seq != 0) << 24 | (pf.workgroups > 0) << 25;                          \
+        kernel<<<dim3(slots + pf.workgroups), dim3(64 * NWAVES), lds, st>>>(qkv, ck, cv, pos, shape, S, inverse(KV), inverse(splits), cos, sin, scale, \
+                                                                            slots, partial, out, pf);                      \
     } while (0)
     if (waves == 8) {
         if (gq == 4) TERNA_GROUPED(8, 4);

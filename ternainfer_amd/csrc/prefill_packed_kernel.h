@@ -540,13 +540,6 @@ __global__ __launch_bounds__(256, MB == 8 ? 1 : (MB == 3 ? 3 : 2)) void terna_pr
 constexpr int kXSwizzleShift = 1;
 __device__ __forceinline__ constexpr int x_swizzle(int row) { return (row >> kXSwizzleShift) & 7; }
 
-// d <- global[sbase + voff .. +15] without a compiler-generated wait: d may be read only after a
-// later wait_loads<>() and a landed(d).
-__device__ __forceinline__ void global_load_b128_nowait(u32x4& d, const void* sbase, uint32_t voff)
-{
-    asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(d) : "v"(voff), "s"(sbase) : "memory");
-}
-__device__ __forceinline__ void landed(u32x4& d) { asm volatile("" : "+v"(d)); }
 template <int VM>
 __device__ __forceinline__ void wait_loads_and_barrier()
 {

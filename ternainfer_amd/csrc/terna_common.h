@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <cfloat>
 #include <type_traits>
 
 namespace terna {
@@ -15,6 +16,7 @@ typedef __attribute__((ext_vector_type(16))) int i32x16;
 typedef __attribute__((ext_vector_type(4))) int i32x4;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
+typedef short s16x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kWave = 64;
 
@@ -199,6 +201,14 @@ __device__ __forceinline__ void lds_dma_b128(const void* sbase, uint32_t voff, u
 {
     asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_addr), "v"(voff), "s"(sbase) : "memory");
 }
+
+// d <- global[sbase + voff .. +15] without a compiler-generated wait: d may be read only after a
+// later wait for it and a landed(d).
+__device__ __forceinline__ void global_load_b128_nowait(u32x4& d, const void* sbase, uint32_t voff)
+{
+    asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(d) : "v"(voff), "s"(sbase) : "memory");
+}
+__device__ __forceinline__ void landed(u32x4& d) { asm volatile("" : "+v"(d)); }
 
 // Makes the value live in registers at this point of the program: a load that produced it cannot be sunk
 // past here (into a branch, next to its use), and is waited for here.

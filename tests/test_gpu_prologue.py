@@ -976,6 +976,43 @@ def test_attention_of_a_kv_group_against_the_oracle(lib, b, h, kv, d, s_max, spl
         assert (np.abs(got[i] - want) <= tol).all(), (i, float((np.abs(got[i] - want) / tol).max()))
 
 
+@pytest.mark.parametrize("b,h,kv,d,s_max,splits,adjacent", [(60, 20, 5, 128, 420, 1, 1), (33, 20, 5, 128, 1100, 2, 0), (40, 8, 4, 128, 300, 3, 1),
+                                                            (70, 16, 4, 64, 700, 1, 0), (36, 8, 4, 64, 900, 5, 1)])
+def test_attention_of_a_kv_group_is_the_per_head_kernel_bit_for_bit(lib, b, h, kv, d, s_max, splits, adjacent):
+    """More than 256 workgroups run four waves each, as the per-head kernel of a single sequence does: the partial results of a sequence in the
+    batch are those of the sequence alone, over prefixes around the units of keys and values (16 and 64 slots a wave and a thread's batch),
+    with infinities and NaNs among the keys and values, and whatever stands behind the prefix."""
+    lens = [1, 16, 17, 63, 64, 65, 128, 129, 192, 255, 256, 257, 300, s_max - 1, s_max]
+    lens = [min(lens[i % len(lens)], s_max) for i in range(b)]
+    qkv = make_bf16_activations(b, (h + 2 * kv) * d, 1871 + b)
+    k0 = make_bf16_activations(b * kv * s_max, d, 1872 + b).reshape(b, kv, s_max, d)
+    v0 = make_bf16_activations(b * kv * s_max, d, 1873 + b, outlier_frac=0.01).reshape(b, kv, s_max, d)
+    pos = np.array(lens, np.int64) - 1
+    for i, n in enumerate(lens):
+        k0[i, :, n:], v0[i, :, n:] = 0x7FC0, 0x7F80
+    v0[12, 0, 100, 3], v0[13, 1, 5, 9], k0[14, 0, 40, 1] = 0x7F80, 0x7FC0, 0xFF80
+    cos, sin = _angles(pos, d)
+    xd, cd, sd, pd, ck, cv = _dev(qkv), _dev(cos), _dev(sin), _dev(pos), _dev(k0), _dev(v0)
+    part = _partial_buffer(lib, b, h, d)
+    print(f"[case] kv group against one head b={b} h={h} kv={kv} d={d} S={s_max} splits={splits} adjacent={adjacent}", flush=True)
+    assert lib.ternaspmm_step_attention(_vp(xd), _vp(cd), _vp(sd), _vp(pd), 1, _vp(ck), _vp(cv), _vp(part), splits, b, h, kv, d, s_max, float(d) ** -0.5,
+                                        adjacent, None, None, None, 0, None) == 0
+    floats = lib.ternaspmm_attention_partial_bytes(1, h, d) // 4
+    stats = floats - h * 8 * d                                       # of one sequence; behind all sequences' their sums
+    for i in range(15):
+        ck1, cv1 = _dev(k0[i:i + 1]), _dev(v0[i:i + 1])
+        one = _partial_buffer(lib, 1, h, d)
+        x1, c1, s1, p1 = _dev(qkv[i:i + 1]), _dev(cos[i:i + 1]), _dev(sin[i:i + 1]), _dev(pos[i:i + 1])
+        assert lib.ternaspmm_step_attention(_vp(x1), _vp(c1), _vp(s1), _vp(p1), 0, _vp(ck1), _vp(cv1), _vp(one), splits, 1, h, kv, d, s_max, float(d) ** -0.5,
+                                            adjacent, None, None, None, 0, None) == 0
+        flat, alone = part.view(torch.float32).flatten(), one.view(torch.float32).flatten()
+        for got, want in ((flat[i * stats:(i + 1) * stats], alone[:stats]),
+                          (flat[b * stats + i * h * splits * d:b * stats + (i + 1) * h * splits * d], alone[stats:stats + h * splits * d])):
+            got, want = got.view(-1), want.view(-1)
+            assert bool(((got.view(torch.int32) == want.view(torch.int32)) | (got.isnan() & want.isnan())).all()), (i, lens[i])
+        assert torch.equal(ck[i], ck1[0]) and torch.equal(cv[i], cv1[0])
+
+
 def test_attention_partial_against_the_oracle(lib):
     """Every sequence against attention_one_token at its own length, 8 splits over a 2B-shaped cache."""
     b, h, kv, d, s_max, lens = 2, 20, 5, 128, 1024, (1000, 333)
