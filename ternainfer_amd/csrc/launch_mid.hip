@@ -14,7 +14,8 @@ struct MidTile {
 
 // A CU's load time is what a launch takes beyond its fixed part, so the tile is the one with the least of
 // (workgroups per CU, rounded up) x (bytes of one workgroup per 4 columns of K: 64 rt sz activations + 16 fb weights).
-// One workgroup per CU: as many waves as K has chunks for, evenly; more of them: four waves each, whose small LDS shares
+// One workgroup per CU: as many waves as K has chunks for, evenly (K = 6912, 27 chunks: fourteen waves take them in two rounds, twelve in three: 32 rows
+// 5.6 -> 5.0 us a launch); more of them: four waves each, whose small LDS shares
 // let four or five workgroups overlap on a CU (measured at M = 17 .. 512: within 5 % of the best of the tiles and wave counts
 // in all but two of ninety cells).
 MidTile choose_tile(int M, int N, int K, int sz)

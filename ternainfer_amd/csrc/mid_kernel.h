@@ -14,7 +14,10 @@
 //     barrier before the sum; 16-byte piece p of row r sits at p ^ (r & 15), which spreads the operand reads over all banks;
 //   * a weight is expanded once for all RT row tiles, an activation operand read once for all FB bands;
 //   * the waves' partial sums meet in LDS (each wave's in place of its activations, 16-byte units XOR-swizzled by the row)
-//     behind the only barrier, are added in wave order (bit-reproducible; integer sums exact) and leave as whole rows.
+//     behind the only barrier, are added in wave order (bit-reproducible; integer sums exact) and leave as whole rows; about 512 threads finish
+//     one to four features each, all waves' sums of them read at once.  In one to two threads per wave and one sum after the other that
+//     was 2000 - 3500 of a workgroup's 6000 - 12000 clocks, now 850 - 1700: decode step of 32 sequences x 512 slots 1461 -> 1355 us, prompt of
+//     100 tokens 1580 -> 1541.
 // Every load of the main part is issued and awaited by hand (see prefill_packed_kernel.h).
 // Measured, us per launch, weights rotating over 20 copies, ring / MFMA-tiled kernel before -> this kernel (tile choice:
 // launch_mid.hip):             QKV 2560->3840   O 2560->2560   gate+up 2560->13824   down 6912->2560
@@ -29,7 +32,7 @@
 
 namespace terna {
 
-constexpr int kMidMaxWaves = 12;
+constexpr int kMidMaxWaves = 16;
 
 template <typename Act, int RT, int FB>
 struct MidShape {
@@ -175,29 +178,63 @@ __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
 
     // ---- the wave's chunks (at least one: waves <= chunks)
     issue(wave);
-    // what the first of this thread's results needs at the end
-    constexpr int UNITS = 4 * FB;                        // 16-byte units (four features) of a result row
-    constexpr int SWZ = FB == 4 ? 0 : 1;
-    constexpr int RESULTS = 16 * RT * UNITS;
-    const int fin_m = m0 + tid / UNITS;
-    const bool fin = tid < RESULTS && fin_m < M;
-    EpilogueRaw raw = load_epilogue_raw_flat<BF16>(ep, fin ? fin_m : 0, band0 * 16 + 4 * (tid % UNITS), N);
-    float2 turn_c = {1.0f, 1.0f}, turn_s = {0.0f, 0.0f};
-    uint16_t* turn_to = nullptr;
-    auto load_turn = [&](int m, int n0) __attribute__((always_inline)) {
-        if constexpr (EPI == PACKED_ROPE) {
-            const int table_row = guard.table_row(m);
-            turn_c = guard.angles2(guard.cos, table_row, n0);
-            turn_s = guard.angles2(guard.sin, table_row, n0);
-            turn_to = guard.place(out, m, n0, N);
-        }
+    // ---- a thread's results: F neighbouring features of one row, so that about 512 threads finish at a time
+    constexpr bool GATE = EPI == PACKED_GATE;
+    constexpr int UNITS = 4 * FB;                        // 16-byte units (four features) of a row of sums
+    constexpr int OUT_UNITS = GATE ? UNITS / 2 : UNITS;  // ... of a row of results
+    constexpr int FEW = EPI == PACKED_ROPE ? 2 : 1, ALL = RT * OUT_UNITS / 8;
+    constexpr int F = ALL < FEW ? FEW : ALL;
+    constexpr int PER_ROW = OUT_UNITS * 4 / F, TASKS = 16 * RT * PER_ROW;
+    static_assert(F == 1 || F == 2 || F == 4, "features of a thread");
+    typedef AccScalar Sums __attribute__((ext_vector_type(F)));
+    // what the first of them needs at the end is requested here
+    struct Finish {
+        uint32_t s, w[GATE ? 2 : F], stream[(F + 1) / 2];
+        float turn_c[(F + 1) / 2], turn_s[(F + 1) / 2];
+        uint16_t* to;
     };
-    if (fin) load_turn(fin_m, band0 * 16 + 4 * (tid % UNITS));
-    u32x2 stream = {0u, 0u};
-    if constexpr (EPI == PACKED_RESIDUAL) {
-        const int n0 = band0 * 16 + 4 * (tid % UNITS);
-        stream = *reinterpret_cast<const u32x2*>(guard.rows + static_cast<size_t>(fin ? fin_m : 0) * N + (n0 < N ? n0 : 0));
-    }
+    const int out_n0 = band0 * (GATE ? 8 : 16);
+    auto request_finish = [&](int idx) __attribute__((always_inline)) {
+        Finish f{};
+        const int row = idx / PER_ROW, m = m0 + row < M ? m0 + row : M - 1, n0 = out_n0 + F * (idx % PER_ROW);
+        if constexpr (!BF16) f.s = ep.s[m];
+        if constexpr (GATE) {
+            f.w[0] = ep.ws[0];
+            f.w[1] = ep.ws[ep.ws_num - 1];
+        } else {
+            int group[4] = {0, 0, 0, 0};
+            if (ep.ws_num != 1) {
+                ws_group_decode4(n0, N, ep.ws_num, group);
+                if (ep.kind == EP_I8_PREFILL) {
+#pragma unroll
+                    for (int v = 0; v < F; ++v) group[v] = ws_group_prefill(n0 + v, N, ep.ws_num);
+                }
+            }
+#pragma unroll
+            for (int v = 0; v < F; ++v) f.w[v] = BF16 ? __float_as_uint(ep.scale[group[v]]) : ep.ws[group[v]];
+        }
+        if constexpr (EPI == PACKED_RESIDUAL) {
+            const uint16_t* from = guard.rows + static_cast<size_t>(m) * N + n0;
+            if constexpr (F == 1) f.stream[0] = *from;
+            else if constexpr (F == 2) f.stream[0] = *reinterpret_cast<const uint32_t*>(from);
+            else {
+                const u32x2 v = *reinterpret_cast<const u32x2*>(from);
+                f.stream[0] = v.x;
+                f.stream[1] = v.y;
+            }
+        }
+        if constexpr (EPI == PACKED_ROPE) {
+            const int at = guard.table_row(m) * (guard.D >> 1) + ((n0 % guard.D) >> 1);
+#pragma unroll
+            for (int v = 0; v < F / 2; ++v) {
+                f.turn_c[v] = guard.cos[at + v];
+                f.turn_s[v] = guard.sin[at + v];
+            }
+            f.to = guard.place(out, m, n0, N);
+        }
+        return f;
+    };
+    Finish first = request_finish(tid < TASKS ? tid : 0);
     for (int chunk = wave;;) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
@@ -211,68 +248,96 @@ __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
     }
 
     // ---- partial sums in place of the wave's activations: unit q = 4 b + g of row 16 r + i
+    constexpr int SWZ = FB == 4 ? 0 : 1;
 #pragma unroll
     for (int r = 0; r < RT; ++r)
 #pragma unroll
         for (int b = 0; b < FB; ++b)
             *reinterpret_cast<Acc*>(mine + ((16 * r + i) * UNITS + ((4 * b + g) ^ ((i >> SWZ) & (UNITS - 1)))) * 16) = acc[r][b];
-    asm volatile("" : "+v"(raw.s), "+v"(raw.w[0]), "+v"(raw.w[1]), "+v"(raw.w[2]), "+v"(raw.w[3]));
+    asm volatile("" : "+v"(first.s), "+v"(first.w[0]), "+v"(first.stream[0]));
     __syncthreads();
-    if constexpr (EPI == PACKED_GATE) {
-        for (int idx = tid; idx < RESULTS / 2; idx += waves * 64) {
-            const int row = idx / (UNITS / 2), u = idx % (UNITS / 2), m = m0 + row, q = 8 * (u >> 2) + (u & 3);
+    // All waves' sums of a result are read before the first is added (one after the other they took 2000 - 3500 of a launch's 6000 - 12000
+    // clocks); W: of the waves that the usual depths of K give, else of any number up to W.
+    auto finish = [&](auto count, auto exact) __attribute__((always_inline)) {
+        constexpr int W = decltype(count)::value;
+        constexpr bool EXACT = decltype(exact)::value;
+        for (int idx = tid; idx < TASKS; idx += waves * 64) {
+            const int row = idx / PER_ROW, n = F * (idx % PER_ROW), m = m0 + row, u = n >> 2, sub = n & 3;
             if (m >= M) break;
-            const int swz = ((row & 15) >> SWZ) & (UNITS - 1);
-            const uint8_t *from1 = smem + (row * UNITS + (q ^ swz)) * 16, *from3 = smem + (row * UNITS + ((q + 4) ^ swz)) * 16;
-            Acc x1 = *reinterpret_cast<const Acc*>(from1), x3 = *reinterpret_cast<const Acc*>(from3);
-            for (int v = 1; v < waves; ++v) {
-                x1 += *reinterpret_cast<const Acc*>(from1 + v * S::kWaveBytes);
-                x3 += *reinterpret_cast<const Acc*>(from3 + v * S::kWaveBytes);
-            }
-            EpilogueRegs e1, e3;
-            e1.s = e3.s = bf16_bits_to_float(ep.s[m]);
-            uint16_t o[4];
+            const int q = GATE ? 8 * (u >> 2) + (u & 3) : u;
+            Sums part[GATE ? 2 : 1][W], sum[GATE ? 2 : 1];
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                e1.w[v] = bf16_bits_to_float(ep.ws[0]);
-                e3.w[v] = bf16_bits_to_float(ep.ws[ep.ws_num - 1]);
-                const float r = max_keep_nan(bf16_bits_to_float(apply_epilogue<int>(ep.kind, e1, v, x1[v] >> kI8WeightShift)), 0.0f);
-                o[v] = float_to_bf16_bits(bf16_bits_to_float(float_to_bf16_bits(r * r)) *
-                                          bf16_bits_to_float(apply_epilogue<int>(ep.kind, e3, v, x3[v] >> kI8WeightShift)));
-            }
-            *reinterpret_cast<u32x2*>(out + static_cast<size_t>(m) * (N >> 1) + band0 * 8 + 4 * u) =
-                u32x2{o[0] | (static_cast<uint32_t>(o[1]) << 16), o[2] | (static_cast<uint32_t>(o[3]) << 16)};
-        }
-        return;
-    }
-    for (int idx = tid; idx < RESULTS; idx += waves * 64) {
-        const int row = idx / UNITS, q = idx % UNITS, m = m0 + row, n0 = band0 * 16 + 4 * q;
-        if (m >= M) break;
-        const uint8_t* from = smem + (row * UNITS + (q ^ (((row & 15) >> SWZ) & (UNITS - 1)))) * 16;
-        Acc sum = *reinterpret_cast<const Acc*>(from);
-        for (int v = 1; v < waves; ++v) sum += *reinterpret_cast<const Acc*>(from + v * S::kWaveBytes);
-        if (idx != tid) raw = load_epilogue_raw_flat<BF16>(ep, m, n0, N);
-        const EpilogueRegs e = finish_epilogue(ep, raw);
-        uint16_t o[4];
+            for (int x = 0; x < (GATE ? 2 : 1); ++x) {
+                const uint8_t* from = smem + (row * UNITS + ((q + 4 * x) ^ (((row & 15) >> SWZ) & (UNITS - 1)))) * 16 + sub * 4;
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            if constexpr (BF16) o[v] = apply_epilogue<float>(EP_BF16, e, v, static_cast<AccScalar>(sum[v] * kBf16WeightUndo));
-            else o[v] = apply_epilogue<int>(ep.kind, e, v, sum[v] >> kI8WeightShift);
+                for (int v = 0; v < W; ++v) part[x][v] = *reinterpret_cast<const Sums*>(from + (EXACT || v < waves ? v : 0) * S::kWaveBytes);
+            }
+            const Finish f = idx == tid ? first : request_finish(idx);
+#pragma unroll
+            for (int x = 0; x < (GATE ? 2 : 1); ++x) {
+                sum[x] = part[x][0];
+#pragma unroll
+                for (int v = 1; v < W; ++v) sum[x] += EXACT || v < waves ? part[x][v] : Sums(0);
+            }
+            // sums -> outputs rounded to bf16, as apply_epilogue has them; under the prefill rule F features of a 128-column tile share a scale
+            const float s = BF16 ? 1.0f : __uint_as_float(f.s << 16);
+            float r[GATE ? 2 : 1][F];
+#pragma unroll
+            for (int x = 0; x < (GATE ? 2 : 1); ++x)
+#pragma unroll
+                for (int v = 0; v < F; ++v) {
+                    if constexpr (BF16) r[x][v] = sum[x][v] * kBf16WeightUndo;
+                    else r[x][v] = static_cast<float>(sum[x][v] >> kI8WeightShift);
+                }
+            auto weight = [&](int x, int v) { return __uint_as_float(BF16 ? f.w[v] : f.w[GATE ? x : v] << 16); };
+            if constexpr (BF16) {
+#pragma unroll
+                for (int v = 0; v < F; ++v) r[0][v] *= weight(0, v);
+            } else if (ep.kind == EP_I8_DECODE) {
+                const RowQuotient by(s);
+#pragma unroll
+                for (int x = 0; x < (GATE ? 2 : 1); ++x) {
+                    by.of(r[x]);
+#pragma unroll
+                    for (int v = 0; v < F; ++v) r[x][v] = __fmul_rn(r[x][v], weight(x, v));
+                }
+            } else {
+#pragma unroll
+                for (int x = 0; x < (GATE ? 2 : 1); ++x) {
+                    const float coeff = s != 0.0f ? __fdiv_rn(weight(x, 0), s) : 0.0f;
+#pragma unroll
+                    for (int v = 0; v < F; ++v) r[x][v] = __fmul_rn(r[x][v], coeff);
+                }
+            }
+            uint16_t o[F];
+#pragma unroll
+            for (int v = 0; v < F; ++v) {
+                o[v] = float_to_bf16_bits(r[0][v]);
+                if constexpr (GATE) {
+                    const float x1 = max_keep_nan(bf16_bits_to_float(o[v]), 0.0f);
+                    o[v] = float_to_bf16_bits(bf16_bits_to_float(float_to_bf16_bits(x1 * x1)) * bf16_bits_to_float(float_to_bf16_bits(r[GATE][v])));
+                }
+            }
+            uint32_t pair[(F + 1) / 2];
+#pragma unroll
+            for (int v = 0; v < (F + 1) / 2; ++v) {
+                pair[v] = F == 1 ? o[0] : o[2 * v] | (static_cast<uint32_t>(o[F == 1 ? 0 : 2 * v + 1]) << 16);
+                if constexpr (EPI == PACKED_RESIDUAL) pair[v] = ResidualRows::pair(pair[v], f.stream[v]);
+                if constexpr (EPI == PACKED_ROPE) {
+                    if (guard.part(out_n0 + n) < 2) pair[v] = RopeStore::rotate(pair[v], f.turn_c[v], f.turn_s[v]);
+                }
+            }
+            uint16_t* to = EPI == PACKED_ROPE ? f.to : out + static_cast<size_t>(m) * (GATE ? N >> 1 : N) + out_n0 + n;
+            if (EPI == PACKED_ROPE && to == nullptr) continue;
+            if constexpr (F == 1) *to = static_cast<uint16_t>(pair[0]);
+            else if constexpr (F == 2) *reinterpret_cast<uint32_t*>(to) = pair[0];
+            else *reinterpret_cast<u32x2*>(to) = u32x2{pair[0], pair[1]};
         }
-        if constexpr (EPI == PACKED_ROPE) {
-            if (idx != tid) load_turn(m, n0);
-            u32x2 turned = {o[0] | (static_cast<uint32_t>(o[1]) << 16), o[2] | (static_cast<uint32_t>(o[3]) << 16)};
-            if (guard.part(n0) < 2) turned = u32x2{RopeStore::rotate(turned.x, turn_c.x, turn_s.x), RopeStore::rotate(turned.y, turn_c.y, turn_s.y)};
-            if (turn_to != nullptr) *reinterpret_cast<u32x2*>(turn_to) = turned;
-            continue;
-        }
-        u32x2 v = {o[0] | (static_cast<uint32_t>(o[1]) << 16), o[2] | (static_cast<uint32_t>(o[3]) << 16)};
-        if constexpr (EPI == PACKED_RESIDUAL) {
-            if (idx != tid) stream = *reinterpret_cast<const u32x2*>(guard.rows + static_cast<size_t>(m) * N + n0);
-            v = ResidualRows::add(v, stream);
-        }
-        *reinterpret_cast<u32x2*>(out + static_cast<size_t>(m) * N + n0) = v;
-    }
+    };
+    if (waves == 10) finish(std::integral_constant<int, 10>{}, std::true_type{});
+    else if (waves == 4) finish(std::integral_constant<int, 4>{}, std::true_type{});
+    else if (waves == 14) finish(std::integral_constant<int, 14>{}, std::true_type{});
+    else finish(std::integral_constant<int, kMidMaxWaves>{}, std::false_type{});
 }
 
 }  // namespace terna
