@@ -57,23 +57,40 @@ struct OutTile {
     __device__ static constexpr int swizzle(int row) { return (row >> (NA == 2 ? 1 : 2)) & (kPieces - 1); }
 };
 
+// What an epilogue of one 32 x 32 tile needs, for a kernel that requests it ahead of its loop (filled by request_epilogue below): the
+// loads of the scales alone keep a wave that finishes by itself waiting 600 clocks.
+struct NothingRequested {
+    static constexpr bool kHere = false;
+};
+struct RequestedEpilogue {
+    static constexpr bool kHere = true;
+    float s, w[2];                                            // of the lane's row; of the tile, or of its gate and up halves
+    u32x4 added[2];                                           // PACKED_RESIDUAL
+    f32x4 cos[2], sin[2];                                     // PACKED_ROPE
+    uint16_t* to[2];
+};
+
 // The gate of a feed-forward layer on the matrix whose w1 and w3 bands are interleaved (ternaspmm_interleave_gate_up): rows 0 .. 15 of a
 // 32-feature tile are x1, rows 16 .. 31 the x3 of the same features, and a lane holds both (its values v and v + 8).  Every product is
 // rounded to bf16 where the separate launches store it.  out [M][N / 2]: half the bytes here, a quarter in the norm that
 // follows (it read both halves).  int8 family, one scale per half: see ternaspmm_gate_linear.
-template <int MB, int NA, typename AccV>
+template <int MB, int NA, typename AccV, typename Ahead = NothingRequested>
 __device__ __forceinline__ void packed_prefill_gate_epilogue(AccV (&acc)[NA][MB], uint16_t* __restrict__ out, const Epilogue& ep, int M, int N,
-                                                             int n_wave, int m0, int lane, uint8_t* tile)
+                                                             int n_wave, int m0, int lane, uint8_t* tile, const Ahead& ahead = Ahead{})
 {
     constexpr int PIECES = 2 * NA, ROW = 16 * PIECES, PER_READ = 64 / PIECES;           // a wave's 16 NA features as rows in LDS
     const int kb = lane >> 5, l32 = lane & 31, F = N >> 1;
-    const float w1 = bf16_bits_to_float(ep.ws[0]), w3 = bf16_bits_to_float(ep.ws[ep.ws_num - 1]);
+    float w1, w3;
+    if constexpr (Ahead::kHere) w1 = ahead.w[0], w3 = ahead.w[1];
+    else w1 = bf16_bits_to_float(ep.ws[0]), w3 = bf16_bits_to_float(ep.ws[ep.ws_num - 1]);
     auto swizzle = [](int row) { return NA == 2 ? (row >> 2) & 3 : 0; };
     auto rows = [&](auto&& element) {
         static_for<0, MB>([&](auto bc) {
             constexpr int b = decltype(bc)::value;
             const int row_m = m0 + 32 * b + l32;
-            const float s = bf16_bits_to_float(ep.s[row_m < M ? row_m : M - 1]);
+            float s;
+            if constexpr (Ahead::kHere) s = ahead.s;
+            else s = bf16_bits_to_float(ep.s[row_m < M ? row_m : M - 1]);
             const float c1 = s != 0.0f ? __fdiv_rn(w1, s) : 0.0f, c3 = s != 0.0f ? __fdiv_rn(w3, s) : 0.0f;
             static_for<0, 2 * NA>([&](auto tc) {
                 constexpr int a = decltype(tc)::value >> 1, vq = decltype(tc)::value & 1;
@@ -105,9 +122,9 @@ __device__ __forceinline__ void packed_prefill_gate_epilogue(AccV (&acc)[NA][MB]
     else rows([](float x, float, float, float c) { return __fmul_rn(x, c); });
 }
 
-template <int MB, int NA, typename AccV>
+template <int MB, int NA, typename AccV, typename Ahead = NothingRequested>
 __device__ __forceinline__ void packed_prefill_rope_epilogue(AccV (&acc)[NA][MB], uint16_t* __restrict__ out, const Epilogue& ep, const RopeStore& rope,
-                                                             int M, int N, int n_wave, int m0, int lane, uint8_t* tile)
+                                                             int M, int N, int n_wave, int m0, int lane, uint8_t* tile, const Ahead& ahead = Ahead{})
 {
     using OT = OutTile<NA>;
     const int kb = lane >> 5, l32 = lane & 31;
@@ -116,8 +133,12 @@ __device__ __forceinline__ void packed_prefill_rope_epilogue(AccV (&acc)[NA][MB]
     float w_of[NA];
     static_for<0, NA>([&](auto ac) {
         constexpr int a = decltype(ac)::value;
-        const int g = ep.ws_num == 1 ? 0 : (ep.kind == EP_I8_PREFILL ? ws_group_prefill(n_wave + 32 * a, N, ep.ws_num) : ws_group_decode(n_wave + 32 * a, N, ep.ws_num));
-        w_of[a] = bf16_bits_to_float(ep.ws[g]);
+        if constexpr (Ahead::kHere) {
+            w_of[a] = ahead.w[0];
+        } else {
+            const int g = ep.ws_num == 1 ? 0 : (ep.kind == EP_I8_PREFILL ? ws_group_prefill(n_wave + 32 * a, N, ep.ws_num) : ws_group_decode(n_wave + 32 * a, N, ep.ws_num));
+            w_of[a] = bf16_bits_to_float(ep.ws[g]);
+        }
     });
     const int piece = lane & (OT::kPieces - 1), n = n_wave + 8 * piece;
     static_for<0, MB>([&](auto bc) {
@@ -128,14 +149,22 @@ __device__ __forceinline__ void packed_prefill_rope_epilogue(AccV (&acc)[NA][MB]
         uint16_t* to[OT::kReads];
 #pragma unroll
         for (int i = 0; i < OT::kReads; ++i) {
-            const int m = m0 + 32 * b + i * OT::kRowsPerRead + lane / OT::kPieces;
-            const int row = rope.table_row(m < M ? m : M - 1);
-            c[i] = rope.angles4(rope.cos, row, n);
-            sn[i] = rope.angles4(rope.sin, row, n);
-            to[i] = m < M ? rope.place(out, m, n, N) : nullptr;
+            if constexpr (Ahead::kHere) {
+                c[i] = ahead.cos[i];
+                sn[i] = ahead.sin[i];
+                to[i] = ahead.to[i];
+            } else {
+                const int m = m0 + 32 * b + i * OT::kRowsPerRead + lane / OT::kPieces;
+                const int row = rope.table_row(m < M ? m : M - 1);
+                c[i] = rope.angles4(rope.cos, row, n);
+                sn[i] = rope.angles4(rope.sin, row, n);
+                to[i] = m < M ? rope.place(out, m, n, N) : nullptr;
+            }
         }
         const int m = m0 + 32 * b + l32 < M ? m0 + 32 * b + l32 : M - 1;
-        const float s = bf16_bits_to_float(ep.s[m]);
+        float s;
+        if constexpr (Ahead::kHere) s = ahead.s;
+        else s = bf16_bits_to_float(ep.s[m]);
         static_for<0, NA>([&](auto ac) {
             constexpr int a = decltype(ac)::value;
             const float coeff = s != 0.0f ? __fdiv_rn(w_of[a], s) : 0.0f;
@@ -183,10 +212,11 @@ using PackedExtra = typename std::conditional<EPI == PACKED_ROPE, RopeStore, typ
 // accumulators it spilled up to 88 registers, so every launch of the larger tiles carried scratch memory for a path that
 // almost no call takes.  The launcher sends such calls to the 128 x 64 instantiation, which keeps the path.
 // ADD: the outputs are added to the rows of `stream` (needs the tile); a block's pieces of it are requested before its sums are scaled.
-template <int MB, int NA, typename AccV, bool COLS = true, bool ADD = false>
+template <int MB, int NA, typename AccV, bool COLS = true, bool ADD = false, typename Ahead = NothingRequested>
 __device__ __forceinline__ void packed_prefill_epilogue(AccV (&acc)[NA][MB], uint16_t* __restrict__ out,
                                                         const Epilogue& ep, int M, int N, int n_wave, int m0, int lane,
-                                                        uint8_t* tile = nullptr, const ResidualRows& stream = ResidualRows{nullptr})
+                                                        uint8_t* tile = nullptr, const ResidualRows& stream = ResidualRows{nullptr},
+                                                        const Ahead& ahead = Ahead{})
 {
     using OT = OutTile<NA>;
     const int kb = lane >> 5, l32 = lane & 31;
@@ -201,7 +231,8 @@ __device__ __forceinline__ void packed_prefill_epilogue(AccV (&acc)[NA][MB], uin
     static_for<0, MB>([&](auto bc) {
         constexpr int b = decltype(bc)::value;
         m_of[b] = m0 + 32 * b + l32;
-        s_of[b] = ep.kind == EP_BF16 ? 1.0f : bf16_bits_to_float(ep.s[m_of[b] < M ? m_of[b] : M - 1]);
+        if constexpr (Ahead::kHere) s_of[b] = ahead.s;
+        else s_of[b] = ep.kind == EP_BF16 ? 1.0f : bf16_bits_to_float(ep.s[m_of[b] < M ? m_of[b] : M - 1]);
     });
     // features 32a + 8vq + 4kb .. +3 of batch row 32b + l32
     const int tile_put = l32 * OT::kRowBytes + 8 * kb, tile_swz = OT::swizzle(l32);
@@ -221,7 +252,8 @@ __device__ __forceinline__ void packed_prefill_epilogue(AccV (&acc)[NA][MB], uin
 #pragma unroll
             for (int i = 0; i < OT::kReads; ++i) {
                 const int m = m0 + 32 * b + i * OT::kRowsPerRead + lane / OT::kPieces;
-                added[i] = *reinterpret_cast<const u32x4*>(stream.rows + static_cast<size_t>(m < M ? m : M - 1) * N + (n < N ? n : 0));
+                if constexpr (Ahead::kHere) added[i] = ahead.added[i];
+                else added[i] = *reinterpret_cast<const u32x4*>(stream.rows + static_cast<size_t>(m < M ? m : M - 1) * N + (n < N ? n : 0));
             }
         }
     };
@@ -254,11 +286,15 @@ __device__ __forceinline__ void packed_prefill_epilogue(AccV (&acc)[NA][MB], uin
         float w_of[NA];
         static_for<0, NA>([&](auto ac) {
             constexpr int a = decltype(ac)::value;
-            int n_a = n_wave + 32 * a;
-            n_a = n_a < N ? n_a : N - 4;
-            const int g = ep.ws_num == 1 ? 0 : (ep.kind == EP_I8_PREFILL ? ws_group_prefill(n_a, N, ep.ws_num)
-                                                                       : ws_group_decode(n_a, N, ep.ws_num));
-            w_of[a] = ep.kind == EP_BF16 ? ep.scale[g] : bf16_bits_to_float(ep.ws[g]);
+            if constexpr (Ahead::kHere) {
+                w_of[a] = ahead.w[0];
+            } else {
+                int n_a = n_wave + 32 * a;
+                n_a = n_a < N ? n_a : N - 4;
+                const int g = ep.ws_num == 1 ? 0 : (ep.kind == EP_I8_PREFILL ? ws_group_prefill(n_a, N, ep.ws_num)
+                                                                           : ws_group_decode(n_a, N, ep.ws_num));
+                w_of[a] = ep.kind == EP_BF16 ? ep.scale[g] : bf16_bits_to_float(ep.ws[g]);
+            }
         });
         // Separate loops under a uniform branch: written as a select, the compiler evaluates the
         // IEEE division of the decode rule for every element of every kind.
@@ -313,6 +349,44 @@ __device__ __forceinline__ void packed_prefill_epilogue(AccV (&acc)[NA][MB], uin
         });
         flush(b);
     });
+}
+
+// The loads of an epilogue of the 32 x 32 tile at (m0, n_wave), n_wave past N included.  (Scales that change inside the tile are read by
+// the epilogue itself.)
+template <int EPI>
+__device__ __forceinline__ RequestedEpilogue request_epilogue(uint16_t* out, const Epilogue& ep, const PackedExtra<EPI>& extra, int M, int N,
+                                                              int n_wave, int m0, int lane)
+{
+    using OT = OutTile<1>;
+    static_assert(OT::kReads == 2, "pieces of a lane");
+    RequestedEpilogue r{};
+    const int l32 = lane & 31, row = m0 + l32 < M ? m0 + l32 : M - 1;
+    r.s = ep.kind == EP_BF16 ? 1.0f : bf16_bits_to_float(ep.s[row]);
+    if constexpr (EPI == PACKED_GATE) {
+        r.w[0] = bf16_bits_to_float(ep.ws[0]);
+        r.w[1] = bf16_bits_to_float(ep.ws[ep.ws_num - 1]);
+    } else {
+        const int n = n_wave < N ? n_wave : N - 4;
+        const int g = ep.ws_num == 1 ? 0 : (ep.kind == EP_I8_PREFILL ? ws_group_prefill(n, N, ep.ws_num) : ws_group_decode(n, N, ep.ws_num));
+        r.w[0] = ep.kind == EP_BF16 ? ep.scale[g] : bf16_bits_to_float(ep.ws[g]);
+    }
+    if constexpr (EPI == PACKED_RESIDUAL || EPI == PACKED_ROPE) {
+        int n = n_wave + 8 * (lane & (OT::kPieces - 1));
+        n = n < N ? n : 0;
+#pragma unroll
+        for (int i = 0; i < OT::kReads; ++i) {
+            const int m = m0 + i * OT::kRowsPerRead + lane / OT::kPieces, mr = m < M ? m : M - 1;
+            if constexpr (EPI == PACKED_RESIDUAL) {
+                r.added[i] = *reinterpret_cast<const u32x4*>(extra.rows + static_cast<size_t>(mr) * N + n);
+            } else {
+                const int at = extra.table_row(mr);
+                r.cos[i] = extra.angles4(extra.cos, at, n);
+                r.sin[i] = extra.angles4(extra.sin, at, n);
+                r.to[i] = m < M ? extra.place(out, m, n, N) : nullptr;
+            }
+        }
+    }
+    return r;
 }
 
 // Raw accumulators of one wave into a [M][N] plane of split-K partial sums (same element order as the epilogue).

@@ -899,6 +899,15 @@ def test_deep_tile_kernel(lib, act, m, n, k):
         assert max_err <= 1e-2 * max_ref and med_ulp <= 1, (max_err, max_ref, med_ulp)
 
 
+@pytest.mark.parametrize("act", ["int8", "bf16"])
+@pytest.mark.parametrize("m,n", [(620, 1856), (1300, 1920)])
+@pytest.mark.parametrize("k", [256, 320, 576, 704, 1088, 1152, 1280, 1344, 1536, 1664, 2496])
+def test_deep_tile_kernel_for_every_number_of_steps(lib, act, m, n, k):
+    """The same kernel at the step counts where its loop without conditions begins, ends and hands over to the one at the edge: 2 to 20
+    steps, odd ones with one less for the first half of K, a last stage of half width, in grids of one and of two workgroups a CU."""
+    test_deep_tile_kernel(lib, act, m, n, k)
+
+
 @pytest.mark.parametrize("m,n,k,groups", [(17, 64, 64, 1), (33, 2560, 320, 1), (64, 192, 2560, 2), (65, 320, 448, 1), (100, 2560, 192, 1), (256, 2560, 6912, 1),
                                           (300, 2560, 3392, 1), (431, 2560, 128, 1), (1000, 2560, 192, 1), (1930, 2624, 64, 1), (2000, 6912, 192, 1)])
 def test_residual_linear(lib, m, n, k, groups):
