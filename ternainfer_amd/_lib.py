@@ -90,6 +90,8 @@ PROTOTYPES = {
     "ternaspmm_gate_linear": ([_vp] * 5 + [_ci] * 4 + [_vp], _ci),
     "bitlinear_TernaSpMM_quant_packed": ([_vp, _vp, _vp, _vp, _ci, _ci, _ci, _ci, _vp], _ci),
     "bitlinear_TernaSpMM_quant": ([_vp] * 7 + [_ci] * 4 + [_vp], _ci),
+    "ternaspmm_quant_rows_linear_packed": ([_vp] * 4 + [_ci] * 4 + [_vp], _ci),
+    "ternaspmm_quant_rows_linear": ([_vp] * 7 + [_ci] * 4 + [_vp], _ci),
     "ternaspmm_quant_input": ([_vp, _vp, _vp, _ci, _ci, _vp], _ci),
     "ternaspmm_quant_mode": ([_ci], _ci),
     "ternaspmm_fused_linear": ([_vp, _vp], _ci),

@@ -52,13 +52,13 @@ void launch_mid_as(const Act* x, const uint32_t* packed, uint16_t* out, const Ep
         if (extra != nullptr) {
             auto kernel = terna_mid_kernel<Act, RT, FB, true>;
             allow_dynamic_lds(kernel, 160 * 1024, "hipFuncSetAttribute(mid)", __LINE__);
-            kernel<<<dim3(grid + 1), block, lds, st>>>(x, packed, out, M, N, K, row_tiles, waves, ep, *extra);
+            kernel<<<dim3(grid + 1), block, lds, st>>>(x, packed, out, M, N, K, row_tiles, waves, ep, *extra, 0);
             return;
         }
     }
     auto kernel = terna_mid_kernel<Act, RT, FB, false, EPI>;
     allow_dynamic_lds(kernel, 160 * 1024, "hipFuncSetAttribute(mid)", __LINE__);
-    kernel<<<dim3(grid), block, lds, st>>>(x, packed, out, M, N, K, row_tiles, waves, ep, extra != nullptr ? *extra : PackedExtra<EPI>{});
+    kernel<<<dim3(grid), block, lds, st>>>(x, packed, out, M, N, K, row_tiles, waves, ep, extra != nullptr ? *extra : PackedExtra<EPI>{}, 0);
 }
 
 template <typename Act, int EPI>
@@ -71,7 +71,46 @@ void launch_mid_tile(const Act* x, const uint32_t* packed, uint16_t* out, const 
     else launch_mid_as<Act, 1, 2, EPI>(x, packed, out, ep, M, N, K, t.waves, extra, st);
 }
 
+// The quantising form: 16 rows a workgroup; the bands of a workgroup, 0 where it does not pay.  Measured at K = 2560, us of the device, two
+// launches / one: 64 x 2560 6.3 / 6.4, 64 x 3840 6.4 / 6.6, 16 x 2560 5.2 / 5.8, 16 x 13824 7.1 / 6.7; with more than one workgroup per CU
+// 128 x 2560 7.1 / 9.2; 32 rows of K = 4096, N = 4096 6.6 / 7.4.  The host's share of a module call is 10.6 / 6.9.
+int quant_tile_bands(int M, int N, int K)
+{
+    const long row_tiles = (M + 15) / 16, bands = N / 16;
+    if ((K / 64 + 3) / 4 > kMidMaxWaves) return 0;
+    return row_tiles * ((bands + 1) / 2) <= 256 ? 2 : row_tiles * ((bands + 3) / 4) <= 256 ? 4 : 0;
+}
+
+template <int FB, bool GUARD>
+void launch_mid_quant_as(const uint16_t* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, hipStream_t st,
+                         const RepackGuard& guard)
+{
+    const int feature_tiles = (N / 16 + FB - 1) / FB, row_tiles = (M + 15) / 16, waves = (K / 64 + 3) / 4;
+    auto kernel = terna_mid_kernel<int8_t, 1, FB, GUARD, PACKED_STORE, true>;
+    allow_dynamic_lds(kernel, 160 * 1024, "hipFuncSetAttribute(mid quant)", __LINE__);
+    kernel<<<dim3((feature_tiles + 7) / 8 * 8 * row_tiles + (GUARD ? 1 : 0)), dim3(waves * 64), MidQuantShape::bytes(waves), st>>>(
+        reinterpret_cast<const int8_t*>(x), packed, out, M, N, K, row_tiles, waves, ep, guard, quant_mode());
+}
+
 }  // namespace
+
+bool mid_quant_takes(const uint16_t* x, const uint16_t* out, int M, int N, int K)
+{
+    return (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(out) & 3) == 0 &&
+           (static_cast<uint64_t>(M) + 16) * K * 2 < (1ull << 31) && static_cast<uint64_t>(N) * K / 4 < (1ull << 31) && quant_tile_bands(M, N, K) != 0;
+}
+void launch_mid_quant(const uint16_t* x, const uint32_t* packed, uint16_t* out, const uint16_t* ws, int ws_num, int M, int N, int K, hipStream_t st,
+                      const RepackGuard* guard)
+{
+    const Epilogue ep{nullptr, ws, nullptr, ws_num, M <= 64 ? EP_I8_DECODE : EP_I8_PREFILL};
+    if (quant_tile_bands(M, N, K) == 2) {
+        if (guard != nullptr) launch_mid_quant_as<2, true>(x, packed, out, ep, M, N, K, st, *guard);
+        else launch_mid_quant_as<2, false>(x, packed, out, ep, M, N, K, st, RepackGuard{});
+    } else {
+        if (guard != nullptr) launch_mid_quant_as<4, true>(x, packed, out, ep, M, N, K, st, *guard);
+        else launch_mid_quant_as<4, false>(x, packed, out, ep, M, N, K, st, RepackGuard{});
+    }
+}
 
 // Up to 16 rows the small-M kernels are faster (3.1 against 3.9 us).  Upwards the MFMA-tiled kernel, whose activations are
 // shared by 128 or 256 features, catches up where the outputs fill the chip several times: measured at M N = 1.0 - 1.25 M for both

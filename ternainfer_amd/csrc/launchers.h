@@ -46,6 +46,10 @@ bool mid_kernel_takes(const void* x, int M, int N, int K, size_t act_bytes);
 template <typename Act>
 void launch_mid(const Act* x, const uint32_t* packed, uint16_t* out, const Epilogue& ep, int M, int N, int K, hipStream_t st,
                 const RepackGuard* guard = nullptr);
+// quant_input + int8 linear on a P2 weight in one launch for more rows than launch_quant_linear takes: whether, and the launch.
+bool mid_quant_takes(const uint16_t* x, const uint16_t* out, int M, int N, int K);
+void launch_mid_quant(const uint16_t* x, const uint32_t* packed, uint16_t* out, const uint16_t* ws, int ws_num, int M, int N, int K, hipStream_t st,
+                      const RepackGuard* guard);
 // For a launch that quantises the M rows of an int8 linear on `packed` (NULL: none) (gate: the interleaved gate+up matrix): what its
 // spare workgroups fetch.
 NextWeights next_weights(const void* packed, int N, int K, bool gate, int M);

@@ -28,6 +28,7 @@
 //   int8 M = 300               10.9 -> 8.8      11.1 -> 6.7    16.4 (stays)           16.3 -> 11.1
 #pragma once
 
+#include "chain_chunk_kernel.h"
 #include "prefill_packed_kernel.h"
 
 namespace terna {
@@ -41,12 +42,22 @@ struct MidShape {
     static_assert(FB == 2 || FB == 4, "result rows of 8 or 16 units: see the swizzle of the partial sums");
     static_assert(RT * FB * 1024 <= kWaveBytes, "partial sums (1 KB per 16 x 16 tile) take the place of the activations");
 };
+// A wave's LDS where the rows are quantised inside (a chunk of 16 int8 rows), and what follows all waves': every wave's row maxima, its
+// copy of the multipliers, the scales.
+struct MidQuantShape {
+    static constexpr int kWaveBytes = 16 * kChainSlabPitch;
+    static constexpr int bytes(int waves) { return waves * kWaveBytes + (16 + 16) * kMidMaxWaves * 4 + 16 * 4; }
+};
 
+// QUANT (RT = 1, Act = int8_t, a wave for every chunk): x is bf16 and quantised inside -- quant_input and the linear of a module call in
+// one launch, for the host's sake: a call of two launches takes it 10.6 us, one 6.9.  A wave holds its chunk of 16 rows in registers; their
+// maxima meet in LDS, every wave forms the 16 scales for itself and writes int8 rows where the other form has them by direct loads.  Two
+// chunks a wave (K = 6912) were 10 us of the device, where the two launches are 7.
 // EPI: plain outputs, the sum with the stream, the feed-forward gate or the rotary embedding and cache write (see the epilogues of prefill_packed_kernel.h)
-template <typename Act, int RT, int FB, bool GUARD, int EPI = PACKED_STORE>
+template <typename Act, int RT, int FB, bool GUARD, int EPI = PACKED_STORE, bool QUANT = false>
 __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
     const Act* __restrict__ x, const uint32_t* __restrict__ packed, uint16_t* __restrict__ out,
-    int M, int N, int K, int row_tiles, int waves, Epilogue ep, PackedExtra<EPI> guard)
+    int M, int N, int K, int row_tiles, int waves, Epilogue ep, PackedExtra<EPI> guard, int quant_mode)
 {
     if constexpr (GUARD) {
         if (blockIdx.x == 0) {
@@ -60,6 +71,8 @@ __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
     using S = MidShape<Act, RT, FB>;
     constexpr bool BF16 = sizeof(Act) == 2;
     constexpr int SZ = static_cast<int>(sizeof(Act));
+    static_assert(!QUANT || (RT == 1 && !BF16 && EPI == PACKED_STORE && FB * 1024 <= MidQuantShape::kWaveBytes), "see above");
+    constexpr int WAVE_BYTES = QUANT ? MidQuantShape::kWaveBytes : S::kWaveBytes;
     constexpr int PIECES = 16 * SZ;                      // 16-byte pieces of a chunk row
     constexpr int ROWS_PER_LOAD = 64 / PIECES;           // rows one direct load fills
     constexpr int XI = 16 * RT / ROWS_PER_LOAD;          // direct loads per chunk
@@ -91,7 +104,7 @@ __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
         const int m = m0 + r0 + ROWS_PER_LOAD * j;
         xrow[j] = static_cast<uint32_t>(m < M ? m : M - 1) * static_cast<uint32_t>(rowbytes);
     }
-    uint8_t* mine = smem + wave * S::kWaveBytes;
+    uint8_t* mine = smem + wave * WAVE_BYTES;
     const uint32_t lds_mine = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(mine));
 
     struct RawW { u32x4 w[FB]; };
@@ -177,7 +190,27 @@ __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
     };
 
     // ---- the wave's chunks (at least one: waves <= chunks)
-    issue(wave);
+    u32x4 xr[8];                                         // QUANT: rows 2 q + (lane >> 5), columns 8 (lane & 31) .. +7
+    const int l32 = lane & 31, odd = lane >> 5;
+    if constexpr (QUANT) {
+        // what is in the caches first: requested behind the weights it would arrive with them
+        const __amdgpu_buffer_rsrc_t rx = make_raw_buffer(x, static_cast<uint32_t>(M) * K * 2u);
+        const int col = wave * 256 + 8 * l32;
+        int at = ((m0 + odd) * K + col) * 2;                             // (a row past M is past the buffer)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            xr[q] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, col < K ? at : kBufferOutOfRange, 0, 0));
+            at += 4 * K;
+        }
+        __builtin_amdgcn_s_barrier();
+        const __amdgpu_buffer_rsrc_t rb = make_raw_buffer(packed, static_cast<uint32_t>(N >> 4) * static_cast<uint32_t>(ktiles) * 256u);
+#pragma unroll
+        for (int b = 0; b < FB; ++b)
+            rw.w[b] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                rb, wave * 4 + g < ktiles ? ((band0 + b) * ktiles + wave * 4) * 256 + lane * 16 : kBufferOutOfRange, 0, 0));
+    } else {
+        issue(wave);
+    }
     // ---- a thread's results: F neighbouring features of one row, so that about 512 threads finish at a time
     constexpr bool GATE = EPI == PACKED_GATE;
     constexpr int UNITS = 4 * FB;                        // 16-byte units (four features) of a row of sums
@@ -197,7 +230,7 @@ __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
     auto request_finish = [&](int idx) __attribute__((always_inline)) {
         Finish f{};
         const int row = idx / PER_ROW, m = m0 + row < M ? m0 + row : M - 1, n0 = out_n0 + F * (idx % PER_ROW);
-        if constexpr (!BF16) f.s = ep.s[m];
+        if constexpr (!BF16 && !QUANT) f.s = ep.s[m];
         if constexpr (GATE) {
             f.w[0] = ep.ws[0];
             f.w[1] = ep.ws[ep.ws_num - 1];
@@ -235,7 +268,53 @@ __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
         return f;
     };
     Finish first = request_finish(tid < TASKS ? tid : 0);
-    for (int chunk = wave;;) {
+    float* const maxima = reinterpret_cast<float*>(smem + waves * WAVE_BYTES);          // [row][wave]
+    float* const multiplier = maxima + 16 * kMidMaxWaves + 16 * wave;                    // of row r: at 8 (r & 1) + r / 2
+    float* const scale = maxima + 32 * kMidMaxWaves;
+    if constexpr (QUANT) {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            float most = 0.0f;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                most = max_keep_nan(max_keep_nan(most, fabsf(__uint_as_float(xr[q][j] << 16))), fabsf(__uint_as_float(xr[q][j] & 0xffff0000u)));
+            most = group_amax<32>(most);
+            if (l32 == 0) maxima[(2 * q + odd) * kMidMaxWaves + wave] = most;
+        }
+        __syncthreads();
+        {
+            const int row = lane >> 2;
+            float most = 0.0f;
+            for (int w = lane & 3; w < waves; w += 4) most = max_keep_nan(most, maxima[row * kMidMaxWaves + w]);
+            most = group_amax<4>(most);
+            uint16_t bits;
+            const float mul = quant_scale(most, quant_mode, &bits);
+            if ((lane & 3) == 0) {
+                multiplier[8 * (row & 1) + (row >> 1)] = mul;
+                if (wave == 0) scale[row] = bf16_bits_to_float(bits);
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        const f32x4 mul_lo = *reinterpret_cast<const f32x4*>(multiplier + 8 * odd), mul_hi = *reinterpret_cast<const f32x4*>(multiplier + 8 * odd + 4);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            landed(xr[q]);                                               // (unpacked again, not kept unpacked: twice the registers)
+            const uint32_t pairs[4] = {xr[q].x, xr[q].y, xr[q].z, xr[q].w}, none[4] = {};
+            uint32_t d[2];
+            chain_quantise<8, false>(pairs, none, 0.0f, q < 4 ? mul_lo[q & 3] : mul_hi[q & 3], quant_mode, d);
+            *reinterpret_cast<u32x2*>(mine + (2 * q + odd) * kChainSlabPitch + 8 * l32) = u32x2{d[0], d[1]};
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const i32x4 v = *reinterpret_cast<const i32x4*>(mine + i * kChainSlabPitch + 64 * g + 16 * c);
+#pragma unroll
+            for (int b = 0; b < FB; ++b) acc[0][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(expand_word_i8(rw.w[b][c]), v, acc[0][b], 0, 0, 0);
+        }
+    }
+    for (int chunk = wave; !QUANT;) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
         clear_past_end(chunk);
@@ -271,7 +350,7 @@ __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
             for (int x = 0; x < (GATE ? 2 : 1); ++x) {
                 const uint8_t* from = smem + (row * UNITS + ((q + 4 * x) ^ (((row & 15) >> SWZ) & (UNITS - 1)))) * 16 + sub * 4;
 #pragma unroll
-                for (int v = 0; v < W; ++v) part[x][v] = *reinterpret_cast<const Sums*>(from + (EXACT || v < waves ? v : 0) * S::kWaveBytes);
+                for (int v = 0; v < W; ++v) part[x][v] = *reinterpret_cast<const Sums*>(from + (EXACT || v < waves ? v : 0) * WAVE_BYTES);
             }
             const Finish f = idx == tid ? first : request_finish(idx);
 #pragma unroll
@@ -281,7 +360,7 @@ __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
                 for (int v = 1; v < W; ++v) sum[x] += EXACT || v < waves ? part[x][v] : Sums(0);
             }
             // sums -> outputs rounded to bf16, as apply_epilogue has them; under the prefill rule F features of a 128-column tile share a scale
-            const float s = BF16 ? 1.0f : __uint_as_float(f.s << 16);
+            const float s = BF16 ? 1.0f : QUANT ? scale[row] : __uint_as_float(f.s << 16);
             float r[GATE ? 2 : 1][F];
 #pragma unroll
             for (int x = 0; x < (GATE ? 2 : 1); ++x)

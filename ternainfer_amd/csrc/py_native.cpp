@@ -33,6 +33,8 @@ namespace {
     X(bitlinear_TernaSpMM_bf16_packed_ws)                                                                              \
     X(bitlinear_TernaSpMM_quant)                                                                                       \
     X(bitlinear_TernaSpMM_quant_packed)                                                                                \
+    X(ternaspmm_quant_rows_linear)                                                                                     \
+    X(ternaspmm_quant_rows_linear_packed)                                                                              \
     X(ternaspmm_qkv_rope_linear)                                                                                       \
     X(ternaspmm_prefill_attention_rows)                                                                                \
     X(ternaspmm_gate_linear)                                                                                           \
@@ -251,6 +253,14 @@ TERNA_FUNCTION(bit_linear, 10)
                                            : lib.bitlinear_TernaSpMM_quant(data<terna_bf16>(&rows), data<uint64_t>(&bitmap), data<int>(&offsets),
                                                                            data<uint16_t>(&median), data<uint32_t>(&signs), data<terna_bf16>(&out),
                                                                            data<terna_bf16>(&ws), ws_num, m, n, k, st);
+        if (done) return wrap(std::move(out), unlocked);
+    }
+    {                                   // ... or of more rows, where one round of workgroups covers the matrix
+        const int done = packed != nullptr ? lib.ternaspmm_quant_rows_linear_packed(data<terna_bf16>(&rows), data(packed), data<terna_bf16>(&out),
+                                                                                    data<terna_bf16>(&ws), ws_num, m, n, k, st)
+                                           : lib.ternaspmm_quant_rows_linear(data<terna_bf16>(&rows), data<uint64_t>(&bitmap), data<int>(&offsets),
+                                                                             data<uint16_t>(&median), data<uint32_t>(&signs), data<terna_bf16>(&out),
+                                                                             data<terna_bf16>(&ws), ws_num, m, n, k, st);
         if (done) return wrap(std::move(out), unlocked);
     }
     QuantRows q = make_quant_rows(m, k);

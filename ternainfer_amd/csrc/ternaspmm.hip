@@ -585,6 +585,45 @@ int bitlinear_TernaSpMM_quant_packed(const terna_bf16* x, const void* packed, te
     return 1;
 }
 
+// Whether a module call's quantisation and linear are one launch: not while a graph is recorded -- a replay is not bound by the host, and the two
+// are up to 1.2 us shorter there.
+static bool quant_rows_taken(const terna_bf16* x, const terna_bf16* out, int ws_num, int M, int N, int K, hipStream_t st)
+{
+    if (!shape_ok(M, N, K) || !groups_ok(ws_num) || !mid_quant_takes(x, out, M, N, K)) return false;
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &capturing) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return capturing == hipStreamCaptureStatusNone;
+}
+
+int ternaspmm_quant_rows_linear_packed(const terna_bf16* x, const void* packed, terna_bf16* out, const terna_bf16* ws, int ws_num,
+                                       int M, int N, int K, terna_stream stream)
+{
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (!quant_rows_taken(x, out, ws_num, M, N, K, st)) return 0;
+    launch_mid_quant(x, static_cast<const uint32_t*>(packed), out, ws, ws_num, M, N, K, st, nullptr);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) die("ternaspmm_quant_rows_linear_packed", e, __LINE__);
+    return 1;
+}
+
+int ternaspmm_quant_rows_linear(const terna_bf16* x, const uint64_t* bitmap, const int* tile_off, const uint16_t* median_off,
+                                const uint32_t* sign_words, terna_bf16* out, const terna_bf16* ws, int ws_num, int M, int N, int K,
+                                terna_stream stream)
+{
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (!quant_rows_taken(x, out, ws_num, M, N, K, st)) return 0;
+    const Weights w{bitmap, tile_off, median_off, sign_words};
+    RepackLaunch cached{};
+    if (!cached_packed(w, N, K, st, &cached, __LINE__)) return 0;
+    launch_mid_quant(x, cached.packed, out, ws, ws_num, M, N, K, st, &cached.guard);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) die("ternaspmm_quant_rows_linear", e, __LINE__);
+    return 1;
+}
+
 int bitlinear_TernaSpMM_quant(const terna_bf16* x, const uint64_t* bitmap, const int* tile_off, const uint16_t* median_off,
                               const uint32_t* sign_words, terna_bf16* out, const terna_bf16* ws, int ws_num, int M, int N, int K,
                               terna_stream stream)

@@ -908,6 +908,60 @@ def test_deep_tile_kernel_for_every_number_of_steps(lib, act, m, n, k):
     test_deep_tile_kernel(lib, act, m, n, k)
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 64, 64), (9, 2560, 2560), (16, 13824, 2560), (17, 704, 320), (33, 192, 4096), (64, 3840, 2560), (65, 2560, 2560),
+                                   (96, 2560, 2304), (250, 256, 1088), (1040, 192, 576)])
+def test_quantisation_and_linear_in_one_launch(lib, m, n, k):
+    """ternaspmm_quant_rows_linear (mid_kernel.h, QUANT) against quant_input and the linear it stands for, bit for bit in every quantisation mode: both of
+    its tiles, one to sixteen waves, partial last chunks and rows, rows of zeros, with an infinity or a NaN; what it does not take (the reference
+    format without a cached copy, a stream that is being captured) enqueues nothing."""
+    from ternainfer_amd import repack_weight
+    fmt = DeviceFormat(make_ternary(n, k, 0.40, 6000 + m + n + k))
+    packed = repack_weight(fmt.vals, fmt.off, fmt.med, fmt.bm, n, k)
+    groups = 3 if n == 3840 else 1
+    ws = torch.tensor([1.25, 0.75, 1.5], dtype=torch.bfloat16, device="cuda")
+    x = torch.from_numpy(make_bf16_activations(m, k, 6100 + m, outlier_frac=0.01).view(np.int16)).cuda().view(torch.bfloat16)
+    if m > 4:
+        x[1], x[2, k // 2], x[m - 1, k - 1] = 0.0, float("inf"), float("nan")
+    xq, s = torch.empty((m, k), dtype=torch.int8, device="cuda"), torch.empty(m, dtype=torch.bfloat16, device="cuda")
+    want, got, again = [torch.full((m, n), 7.0, dtype=torch.bfloat16, device="cuda") for _ in range(3)]
+    formats, cached = (vp(fmt.bm), vp(fmt.off), vp(fmt.med), vp(fmt.vals)), int(os.environ["TERNASPMM_REPACK_CACHE"] == "1")
+    try:
+        for mode in (0, 1, 2):
+            print(f"[case] quantised inside M={m} N={n} K={k} mode={mode}", flush=True)
+            lib.ternaspmm_quant_mode(mode)
+            assert lib.ternaspmm_quant_input(vp(x), vp(xq), vp(s), m, k, _stream()) == 0
+            lib.bitlinear_TernaSpMM_packed(vp(xq), vp(packed), vp(want), vp(s), vp(ws), groups, m, n, k, 0, _stream())
+            assert lib.ternaspmm_quant_rows_linear_packed(vp(x), vp(packed), vp(got), vp(ws), groups, m, n, k, _stream()) == 1
+            assert lib.ternaspmm_quant_rows_linear(vp(x), *formats, vp(again), vp(ws), groups, m, n, k, _stream()) == cached
+            torch.cuda.synchronize()
+            for out in (got, again)[:1 + cached]:
+                assert torch.equal(torch.isnan(out), torch.isnan(want))
+                assert torch.equal(torch.nan_to_num(out.float(), nan=0.0), torch.nan_to_num(want.float(), nan=0.0))
+    finally:
+        lib.ternaspmm_quant_mode(0)
+    got.fill_(7.0)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        taken = lib.ternaspmm_quant_rows_linear_packed(vp(x), vp(packed), vp(got), vp(ws), groups, m, n, k, _stream())
+        got.add_(0.0)
+    assert taken == 0
+    for refused in ((x.data_ptr() + 2, m, n, k), (x.data_ptr(), 4096, 2560, k), (x.data_ptr(), m, n, 4160), (x.data_ptr(), 0, n, k), (x.data_ptr(), m, 72, k)):
+        assert lib.ternaspmm_quant_rows_linear_packed(refused[0], vp(packed), vp(got), vp(ws), groups, *refused[1:], _stream()) == 0
+    torch.cuda.synchronize()
+    assert bool((got == 7.0).all())
+
+
+def test_quantisation_and_linear_in_one_launch_on_the_reference_format():
+    """The same with cached copies of the weights (TERNASPMM_REPACK_CACHE=1 is read once per process, hence a child process)."""
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    run = ("from tests import test_gpu_parity as t; from ternainfer_amd import _lib\n"
+           "for m, n, k in ((9, 2560, 2560), (17, 704, 320), (65, 2560, 1088)): t.test_quantisation_and_linear_in_one_launch(_lib.load(), m, n, k)\nprint('all the same')")
+    r = subprocess.run([sys.executable, "-u", "-c", run], cwd=root, env={**os.environ, "TERNASPMM_REPACK_CACHE": "1"}, capture_output=True, text=True, timeout=110)
+    assert r.returncode == 0 and "all the same" in r.stdout, r.stdout[-2000:] + r.stderr[-2000:]
+
+
 @pytest.mark.parametrize("m,n,k,groups", [(17, 64, 64, 1), (33, 2560, 320, 1), (64, 192, 2560, 2), (65, 320, 448, 1), (100, 2560, 192, 1), (256, 2560, 6912, 1),
                                           (300, 2560, 3392, 1), (431, 2560, 128, 1), (1000, 2560, 192, 1), (1930, 2624, 64, 1), (2000, 6912, 192, 1)])
 def test_residual_linear(lib, m, n, k, groups):
