@@ -112,13 +112,16 @@ void launch_mid_quant(const uint16_t* x, const uint32_t* packed, uint16_t* out, 
     }
 }
 
-// Up to 16 rows the small-M kernels are faster (3.1 against 3.9 us).  Upwards the MFMA-tiled kernel, whose activations are
-// shared by 128 or 256 features, catches up where the outputs fill the chip several times: measured at M N = 1.0 - 1.25 M for both
-// types and every matrix (gate+up: M = 80, QKV: M = 300, O and down projection: M = 420 - 450).
+// Up to 16 rows the small-M kernels are faster (3.1 against 3.9 us).  Upwards the MFMA-tiled kernel, whose activations are shared by 128
+// features, is ahead where the tiles of 32 x 64 are more than two a CU -- counted as they lie on the XCDs, in eights of feature
+// tiles (N = 256 leaves half of the XCDs without one).  Measured, us, MFMA-tiled / this kernel, int8; bf16: QKV M = 250 (480 tiles) 7.7 / 6.8;
+// 10.8 / 9.6, M = 280 (576) 7.7 / 8.1; 10.9 / 12.7; gate+up M = 64 (432) 8.2 / 7.1; 10.7 / 9.8, M = 70 (648) 8.0 / 8.4; 11.8 / 12.8; down M = 350
+// (440) 13.2 / 11.2; 22.2 / 18.3, M = 430 (560) 13.4 / 14.2; 22.3 / 28.2; N = 1024 = K, M = 1000 (512) 5.2 / 4.6; 6.3 / 5.5, M = 1200 (608) 5.3 / 5.4;
+// 6.6 / 7.3; N = 256, M = 1000 (256) 6.9 / 5.0; 11.5 / 9.3, M = 4000 (1000) 7.7 / 13.2; 12.1 / 23.8; N = 704, K = 320, M = 1500 (752) 4.4 / 6.0; 4.6 / 7.5.
 bool mid_kernel_takes(const void* x, int M, int N, int K, size_t act_bytes)
 {
-    const long outputs = static_cast<long>(M) * N, most = 1100000;
-    return M > 16 && outputs <= most && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
+    const long tiles = static_cast<long>((M + 31) / 32) * ((N / 16 + 31) / 32 * 8);
+    return M > 16 && tiles <= 512 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
            static_cast<uint64_t>(M) * K * act_bytes < (1ull << 31) && static_cast<uint64_t>(N) * K / 4 < (1ull << 31);
 }
 

@@ -869,6 +869,14 @@ def test_mid_kernel_against_the_forced_kernels(lib, act, m, n, k):
 
 
 @pytest.mark.parametrize("act", ["int8", "bf16"])
+@pytest.mark.parametrize("m,n,k", [(64, 13824, 192), (70, 13824, 192), (256, 3840, 320), (257, 3840, 320), (1024, 960, 128), (1025, 960, 128), (2048, 256, 320),
+                                   (2049, 256, 320), (1500, 704, 320)])
+def test_calls_on_both_sides_of_the_mid_kernels_limit(lib, act, m, n, k):
+    """The last rows that the kernel of a few hundred rows takes and the first that the MFMA-tiled one does, wide, narrow and odd matrices."""
+    test_mid_kernel_against_the_forced_kernels(lib, act, m, n, k)
+
+
+@pytest.mark.parametrize("act", ["int8", "bf16"])
 @pytest.mark.parametrize("m,n,k", [(641, 2112, 64), (1100, 1280, 128), (520, 2560, 448), (97, 13824, 192), (750, 1792, 960), (1340, 1088, 832),
                                    (900, 3328, 192), (1300, 2560, 448)])
 def test_deep_tile_kernel(lib, act, m, n, k):
