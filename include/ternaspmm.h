@@ -212,8 +212,8 @@ int bitlinear_TernaSpMM_quant(const terna_bf16* x, const uint64_t* bitmap, const
                               const uint16_t* tile_offsets_median, const uint32_t* sign_words, terna_bf16* out,
                               const terna_bf16* ws, int ws_num, int M, int N, int K, terna_stream stream);
 
-/* The same for more rows, with the epilogue that the two calls choose by M: up to 256 workgroups of 16 rows x 32 or 64 features
- * (ceil(M / 16) * ceil(N / 64) <= 256), K <= 4096, 16-byte aligned x, 4-byte aligned out, a stream that is not being captured (a replay is
+/* The same for more rows, with the epilogue that the two calls choose by M: up to 256 workgroups of 16 rows x 32 or 64 features (512
+ * for K <= 2048; ceil(M / 16) * 8 ceil(N / 512)), K <= 4096, 16-byte aligned x, 4-byte aligned out, a stream that is not being captured (a replay is
  * not bound by the host, and there the two launches are shorter).  1, or 0 with nothing enqueued. */
 int ternaspmm_quant_rows_linear_packed(const terna_bf16* x, const void* packed, terna_bf16* out, const terna_bf16* ws, int ws_num,
                                        int M, int N, int K, terna_stream stream);

@@ -336,8 +336,8 @@ bool launch_quant_linear(const uint16_t* x, const uint32_t* packed, uint16_t* ou
     const dim3 grid(N / 16 + (guard != nullptr ? 1 : 0)), block(kChunkWaves * 64);
 #define TERNA_QUANT_LINEAR(CT, MR)                                                                                                     \
     do {                                                                                                                              \
-        if (guard != nullptr) terna_quant_linear_kernel<CT, MR, true><<<grid, block, 0, st>>>(x, packed, out, ws, M, N, K, ws_num, qm, *guard); \
-        else terna_quant_linear_kernel<CT, MR, false><<<grid, block, 0, st>>>(x, packed, out, ws, M, N, K, ws_num, qm, RepackGuard{});         \
+        if (guard != nullptr) launch(terna_quant_linear_kernel<CT, MR, true>, grid, block, 0, st, x, packed, out, ws, M, N, K, ws_num, qm, *guard); \
+        else launch(terna_quant_linear_kernel<CT, MR, false>, grid, block, 0, st, x, packed, out, ws, M, N, K, ws_num, qm, RepackGuard{});         \
     } while (0)
 #define TERNA_QUANT_LINEAR_CT(MR)                                                                                                      \
     do {                                                                                                                              \

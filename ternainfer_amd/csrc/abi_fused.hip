@@ -93,9 +93,9 @@ int ternaspmm_quant_input(const terna_bf16* x, int8_t* xq_out, terna_bf16* s_out
     const dim3 grid(M), block(kNormThreads);
     hipStream_t st = static_cast<hipStream_t>(stream);
     const int qm = quant_mode();
-    if (nv <= 1) terna_quant_input_kernel<1><<<grid, block, 0, st>>>(x, K, xq_out, s_out, qm);
-    else if (nv <= 2) terna_quant_input_kernel<2><<<grid, block, 0, st>>>(x, K, xq_out, s_out, qm);
-    else terna_quant_input_kernel<4><<<grid, block, 0, st>>>(x, K, xq_out, s_out, qm);
+    if (nv <= 1) launch(terna_quant_input_kernel<1>, grid, block, 0, st, x, K, xq_out, s_out, qm);
+    else if (nv <= 2) launch(terna_quant_input_kernel<2>, grid, block, 0, st, x, K, xq_out, s_out, qm);
+    else launch(terna_quant_input_kernel<4>, grid, block, 0, st, x, K, xq_out, s_out, qm);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) die("ternaspmm_quant_input", e, __LINE__);
     return 0;

@@ -21,9 +21,9 @@ void launch_decode_packed_as(const Act* x, const uint32_t* packed, uint16_t* out
 {
     const dim3 grid(N / 16 / NB + (guard != nullptr ? 1 : 0), (M + 16 * MB - 1) / (16 * MB));
     if (guard != nullptr)
-        terna_decode_packed_kernel<Act, WAVES, MB, DEPTH, NB, true><<<grid, dim3(WAVES * 64), 0, st>>>(x, packed, out, M, N, K, ep, *guard, PackedProducer{});
+        launch(terna_decode_packed_kernel<Act, WAVES, MB, DEPTH, NB, true>, grid, dim3(WAVES * 64), 0, st, x, packed, out, M, N, K, ep, *guard, PackedProducer{});
     else
-        terna_decode_packed_kernel<Act, WAVES, MB, DEPTH, NB, false><<<grid, dim3(WAVES * 64), 0, st>>>(x, packed, out, M, N, K, ep, RepackGuard{}, PackedProducer{});
+        launch(terna_decode_packed_kernel<Act, WAVES, MB, DEPTH, NB, false>, grid, dim3(WAVES * 64), 0, st, x, packed, out, M, N, K, ep, RepackGuard{}, PackedProducer{});
 }
 
 template <typename Act, int WAVES, int TMAX, int NB>
@@ -32,9 +32,9 @@ void launch_decode_flat_as(const Act* x, const uint32_t* packed, uint16_t* out, 
 {
     const dim3 grid(N / 16 / NB + (guard != nullptr ? 1 : 0));
     if (guard != nullptr)
-        terna_decode_flat_kernel<Act, WAVES, TMAX, NB, true><<<grid, dim3(WAVES * 64), 0, st>>>(x, packed, out, M, N, K, ep, *guard);
+        launch(terna_decode_flat_kernel<Act, WAVES, TMAX, NB, true>, grid, dim3(WAVES * 64), 0, st, x, packed, out, M, N, K, ep, *guard);
     else
-        terna_decode_flat_kernel<Act, WAVES, TMAX, NB, false><<<grid, dim3(WAVES * 64), 0, st>>>(x, packed, out, M, N, K, ep, RepackGuard{});
+        launch(terna_decode_flat_kernel<Act, WAVES, TMAX, NB, false>, grid, dim3(WAVES * 64), 0, st, x, packed, out, M, N, K, ep, RepackGuard{});
 }
 
 // Up to 16 rows and a K whose tiles one workgroup holds in flight: the straight-line kernel (decode_flat_kernel.h).
@@ -64,9 +64,9 @@ void launch_decode_chunk_as(const Act* x, const uint32_t* packed, uint16_t* out,
 {
     const dim3 grid(N / 16 + (guard != nullptr ? 1 : 0));
     if (guard != nullptr)
-        terna_decode_chunk_kernel<Act, CT, MR, true><<<grid, dim3(kChunkWaves * 64), 0, st>>>(x, packed, out, M, N, K, ep, *guard);
+        launch(terna_decode_chunk_kernel<Act, CT, MR, true>, grid, dim3(kChunkWaves * 64), 0, st, x, packed, out, M, N, K, ep, *guard);
     else
-        terna_decode_chunk_kernel<Act, CT, MR, false><<<grid, dim3(kChunkWaves * 64), 0, st>>>(x, packed, out, M, N, K, ep, RepackGuard{});
+        launch(terna_decode_chunk_kernel<Act, CT, MR, false>, grid, dim3(kChunkWaves * 64), 0, st, x, packed, out, M, N, K, ep, RepackGuard{});
 }
 
 template <typename Act, int MR>
@@ -75,9 +75,9 @@ void launch_decode_chunk4_as(const Act* x, const uint32_t* packed, uint16_t* out
 {
     const dim3 grid(N / 64 + (guard != nullptr ? 1 : 0));
     if (guard != nullptr)
-        terna_decode_chunk4_kernel<Act, MR, true><<<grid, dim3(kChunkWaves * 64), 0, st>>>(x, packed, out, M, N, K, ep, *guard);
+        launch(terna_decode_chunk4_kernel<Act, MR, true>, grid, dim3(kChunkWaves * 64), 0, st, x, packed, out, M, N, K, ep, *guard);
     else
-        terna_decode_chunk4_kernel<Act, MR, false><<<grid, dim3(kChunkWaves * 64), 0, st>>>(x, packed, out, M, N, K, ep, RepackGuard{});
+        launch(terna_decode_chunk4_kernel<Act, MR, false>, grid, dim3(kChunkWaves * 64), 0, st, x, packed, out, M, N, K, ep, RepackGuard{});
 }
 
 // Up to 16 rows, up to 32 chunks of four tiles (K <= 8192): the kernel with four band-tiles per load (decode_chunk_kernel.h).
@@ -154,9 +154,9 @@ void launch_decode_packed_producer(const int8_t* x, const uint32_t* packed, uint
     const PackedProducer prod{residual, next_w, reinterpret_cast<float2*>(stats_out), raw_out};
     const dim3 grid(N / 16, 1);
     if (N / 16 <= 256)
-        terna_decode_packed_kernel<int8_t, 16, 1, 3, 1, false, true><<<grid, dim3(16 * 64), 0, st>>>(x, packed, out, M, N, K, ep, RepackGuard{}, prod);
+        launch(terna_decode_packed_kernel<int8_t, 16, 1, 3, 1, false, true>, grid, dim3(16 * 64), 0, st, x, packed, out, M, N, K, ep, RepackGuard{}, prod);
     else
-        terna_decode_packed_kernel<int8_t, 8, 1, 2, 1, false, true><<<grid, dim3(8 * 64), 0, st>>>(x, packed, out, M, N, K, ep, RepackGuard{}, prod);
+        launch(terna_decode_packed_kernel<int8_t, 8, 1, 2, 1, false, true>, grid, dim3(8 * 64), 0, st, x, packed, out, M, N, K, ep, RepackGuard{}, prod);
 }
 
 // one wave each: record the fingerprint of a weight's reference-format tensors / check it as a launch of its own

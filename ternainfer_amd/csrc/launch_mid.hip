@@ -51,14 +51,14 @@ void launch_mid_as(const Act* x, const uint32_t* packed, uint16_t* out, const Ep
     if constexpr (EPI == PACKED_STORE) {
         if (extra != nullptr) {
             auto kernel = terna_mid_kernel<Act, RT, FB, true>;
-            allow_dynamic_lds(kernel, 160 * 1024, "hipFuncSetAttribute(mid)", __LINE__);
-            kernel<<<dim3(grid + 1), block, lds, st>>>(x, packed, out, M, N, K, row_tiles, waves, ep, *extra, 0);
+            if (lds > kPlainLds) allow_dynamic_lds(kernel, 160 * 1024, "hipFuncSetAttribute(mid)", __LINE__);
+            launch(kernel, dim3(grid + 1), block, lds, st, x, packed, out, M, N, K, row_tiles, waves, ep, *extra, 0);
             return;
         }
     }
     auto kernel = terna_mid_kernel<Act, RT, FB, false, EPI>;
-    allow_dynamic_lds(kernel, 160 * 1024, "hipFuncSetAttribute(mid)", __LINE__);
-    kernel<<<dim3(grid), block, lds, st>>>(x, packed, out, M, N, K, row_tiles, waves, ep, extra != nullptr ? *extra : PackedExtra<EPI>{}, 0);
+    if (lds > kPlainLds) allow_dynamic_lds(kernel, 160 * 1024, "hipFuncSetAttribute(mid)", __LINE__);
+    launch(kernel, dim3(grid), block, lds, st, x, packed, out, M, N, K, row_tiles, waves, ep, extra != nullptr ? *extra : PackedExtra<EPI>{}, 0);
 }
 
 template <typename Act, int EPI>
@@ -71,14 +71,16 @@ void launch_mid_tile(const Act* x, const uint32_t* packed, uint16_t* out, const 
     else launch_mid_as<Act, 1, 2, EPI>(x, packed, out, ep, M, N, K, t.waves, extra, st);
 }
 
-// The quantising form: 16 rows a workgroup; the bands of a workgroup, 0 where it does not pay.  Measured at K = 2560, us of the device, two
-// launches / one: 64 x 2560 6.3 / 6.4, 64 x 3840 6.4 / 6.6, 16 x 2560 5.2 / 5.8, 16 x 13824 7.1 / 6.7; with more than one workgroup per CU
-// 128 x 2560 7.1 / 9.2; 32 rows of K = 4096, N = 4096 6.6 / 7.4.  The host's share of a module call is 10.6 / 6.9.
+// The quantising form: 16 rows a workgroup; the bands of a workgroup, 0 where it does not pay: up to one workgroup a CU, two where K is short,
+// feature tiles counted in eights as they lie on the XCDs.  us of the device, two launches / one: K = 2560, 64 x 2560 6.3 / 6.4, 64 x 3840
+// 6.4 / 6.6, 16 x 2560 5.2 / 5.8, 16 x 13824 7.1 / 6.7, two workgroups a CU 128 x 2560 7.1 / 9.2; 32 rows of K = 4096, N = 4096 6.6 / 7.4; two
+// workgroups a CU, K = 1024, 512 x 1024 6.9 / 6.0, K = 2048 8.0 / 8.0.  The host's share of a module call is 10.6 / 6.9.
 int quant_tile_bands(int M, int N, int K)
 {
     const long row_tiles = (M + 15) / 16, bands = N / 16;
-    if ((K / 64 + 3) / 4 > kMidMaxWaves) return 0;
-    return row_tiles * ((bands + 1) / 2) <= 256 ? 2 : row_tiles * ((bands + 3) / 4) <= 256 ? 4 : 0;
+    const int chunks = (K / 64 + 3) / 4;
+    if (chunks > kMidMaxWaves) return 0;
+    return row_tiles * ((bands + 15) / 16 * 8) <= 256 ? 2 : row_tiles * ((bands + 31) / 32 * 8) <= (chunks <= 8 ? 512 : 256) ? 4 : 0;
 }
 
 template <int FB, bool GUARD>
@@ -87,9 +89,10 @@ void launch_mid_quant_as(const uint16_t* x, const uint32_t* packed, uint16_t* ou
 {
     const int feature_tiles = (N / 16 + FB - 1) / FB, row_tiles = (M + 15) / 16, waves = (K / 64 + 3) / 4;
     auto kernel = terna_mid_kernel<int8_t, 1, FB, GUARD, PACKED_STORE, true>;
-    allow_dynamic_lds(kernel, 160 * 1024, "hipFuncSetAttribute(mid quant)", __LINE__);
-    kernel<<<dim3((feature_tiles + 7) / 8 * 8 * row_tiles + (GUARD ? 1 : 0)), dim3(waves * 64), MidQuantShape::bytes(waves), st>>>(
-        reinterpret_cast<const int8_t*>(x), packed, out, M, N, K, row_tiles, waves, ep, guard, quant_mode());
+    const int lds = MidQuantShape::bytes(waves);
+    if (lds > kPlainLds) allow_dynamic_lds(kernel, 160 * 1024, "hipFuncSetAttribute(mid quant)", __LINE__);
+    launch(kernel, dim3((feature_tiles + 7) / 8 * 8 * row_tiles + (GUARD ? 1 : 0)), dim3(waves * 64), lds, st,
+           reinterpret_cast<const int8_t*>(x), packed, out, M, N, K, row_tiles, waves, ep, guard, quant_mode());
 }
 
 }  // namespace

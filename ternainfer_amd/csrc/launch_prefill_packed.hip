@@ -21,7 +21,7 @@ void launch_prefill_packed_as(const Act* x, const uint32_t* packed, uint16_t* ou
     allow_dynamic_lds(kernel, S::kBytes, "hipFuncSetAttribute(prefill packed)", __LINE__);
     constexpr int BN = 128 * NA;
     const dim3 grid((N + BN - 1) / BN, (M + S::BM - 1) / S::BM);
-    kernel<<<grid, dim3(256), S::kBytes, st>>>(x, packed, out, ep, M, N, K);
+    launch(kernel, grid, dim3(256), S::kBytes, st, x, packed, out, ep, M, N, K);
 }
 
 // Split-K: with few output tiles for the chip (small M x N) every workgroup walks all of K alone and most CUs idle.
@@ -75,7 +75,7 @@ void launch_prefill_packed_dma_as(const Act* x, const uint32_t* packed, uint16_t
             }
         }
     }
-    allow_dynamic_lds(kernel, lds, "hipFuncSetAttribute(prefill packed dma)", __LINE__);
+    if (lds > kPlainLds) allow_dynamic_lds(kernel, lds, "hipFuncSetAttribute(prefill packed dma)", __LINE__);
     const int splits = plan.splits;
     // The check of a cached copy rides in the launch: as one more row of workgroups in y, or -- with split-K planes, whose
     // workgroup -> XCD pattern an extra row per plane would shift -- as the first workgroup of the reduce launch.
@@ -90,7 +90,7 @@ void launch_prefill_packed_dma_as(const Act* x, const uint32_t* packed, uint16_t
     // TERNASPMM_PREFILL_XCD_MAP=0|1 forces it off / on (tuning aid).
     const bool big_x = static_cast<size_t>(M) * K * sizeof(Act) > (4u << 20);
     const int xcd_map = (plan.grid_y % 8 == 0) && (xcd_forced < 0 ? big_x : xcd_forced != 0);
-    kernel<<<grid, dim3(threads), lds, st>>>(x, packed, out, ep, M, N, K, xcd_map, splits, splits > 1 ? scratch : nullptr,
+    launch(kernel, grid, dim3(threads), lds, st, x, packed, out, ep, M, N, K, xcd_map, splits, splits > 1 ? scratch : nullptr,
                                                guard_row ? 1 : 0, guard_row || (EPI != PACKED_STORE && guard != nullptr) ? *guard : PackedExtra<EPI>{});
     if constexpr (EPI == PACKED_STORE || EPI == PACKED_RESIDUAL) if (splits > 1) {
         using AccT = typename std::conditional<sizeof(Act) == 1, int, float>::type;
@@ -100,7 +100,7 @@ void launch_prefill_packed_dma_as(const Act* x, const uint32_t* packed, uint16_t
         if constexpr (EPI == PACKED_RESIDUAL) stream = *guard;
         else if (guard != nullptr) check = *guard;
         const bool guard_first = EPI == PACKED_STORE && guard != nullptr;
-        terna_splitk_reduce_kernel<AccT><<<dim3(static_cast<unsigned>((quads + 255) / 256) + (guard_first ? 1 : 0)), dim3(256), 0, st>>>(
+        launch(terna_splitk_reduce_kernel<AccT>, dim3(static_cast<unsigned>((quads + 255) / 256) + (guard_first ? 1 : 0)), dim3(256), 0, st, 
             static_cast<const AccT*>(scratch), out, ep, M, N, splits, guard_first ? 1 : 0, check, stream);
     }
 }

@@ -917,7 +917,7 @@ def test_deep_tile_kernel_for_every_number_of_steps(lib, act, m, n, k):
 
 
 @pytest.mark.parametrize("m,n,k", [(1, 64, 64), (9, 2560, 2560), (16, 13824, 2560), (17, 704, 320), (33, 192, 4096), (64, 3840, 2560), (65, 2560, 2560),
-                                   (96, 2560, 2304), (250, 256, 1088), (1040, 192, 576)])
+                                   (96, 2560, 2304), (250, 256, 1088), (1000, 192, 576), (505, 1024, 2048)])
 def test_quantisation_and_linear_in_one_launch(lib, m, n, k):
     """ternaspmm_quant_rows_linear (mid_kernel.h, QUANT) against quant_input and the linear it stands for, bit for bit in every quantisation mode: both of
     its tiles, one to sixteen waves, partial last chunks and rows, rows of zeros, with an infinity or a NaN; what it does not take (the reference
