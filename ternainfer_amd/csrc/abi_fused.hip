@@ -43,6 +43,14 @@ void ternaspmm_rmsnorm_quant_ahead(const terna_bf16* x, const terna_bf16* residu
     const dim3 grid(M + ahead.workgroups), block(kNormThreads);
     hipStream_t st = static_cast<hipStream_t>(stream);
     const int qm = quant_mode();
+    if (residual == nullptr && xq_out != nullptr && nv > 1 && M <= kNormWideRows) {
+        const dim3 threads((K / 8 + 63) / 64 * 64);
+        auto kernel = nv <= 2 ? terna_norm_quant_wide_kernel<2> : terna_norm_quant_wide_kernel<4>;
+        kernel<<<grid, threads, 0, st>>>(x, weight, K, eps, M, qm, xq_out, s_out, y_out, ahead);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) die("ternaspmm_rmsnorm_quant", e, __LINE__);
+        return;
+    }
 #define TERNA_NORM(NV, SECOND) terna_norm_quant_kernel<false, NV, SECOND><<<grid, block, 0, st>>>(x, residual, weight, K, eps, sum_out, y_out, xq_out, s_out, qm, M, ahead)
     if (residual != nullptr) {
         if (nv <= 1) TERNA_NORM(1, true);

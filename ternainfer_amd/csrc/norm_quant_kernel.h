@@ -279,6 +279,92 @@ __global__ __launch_bounds__(kNormThreads) void terna_norm_quant_kernel(
     norm_quant_passes<NV>(h, raw_w, K, eps, row, y_out, xq_out, s_out, quant_mode);
 }
 
+// The plain form for few rows: a thread for every eight-element vector (up to sixteen waves).  The sum of squares is defined by 256
+// threads that take the vectors t, t + 256, ... in turn: the first four waves read those as well and add them up so; everything behind
+// the sum is one vector a thread.  A row's launch is what one wave does in a row: of 4000 clocks (K = 2560; 5900 for K = 6912) the request took 900,
+// the data 600, the sum 550, norm and maximum 1100, quantisation 700, and the first wave had two vectors in each (four).  Blocks of a pass
+// in a graph, us, the form above -> this: 32 sequences 41.4 -> 40.9, a prompt of 100 tokens 47.5 -> 46.9; of 256 65.5 -> 65.5, 600 102.6 -> 104.3, 1920 216 ->
+// 224: many rows fill the chip either way, and the sums read twice.
+constexpr int kNormWideRows = 128;
+template <int NV>
+__global__ __launch_bounds__(1024) void terna_norm_quant_wide_kernel(
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ weight, int K, float eps, int rows, int quant_mode,
+    int8_t* __restrict__ xq_out, uint16_t* __restrict__ s_out, uint16_t* __restrict__ y_out, NextWeights next)
+{
+    if (static_cast<int>(blockIdx.x) >= rows) {
+        fetch_next_weights(next, rows);
+        return;
+    }
+    __shared__ float sums[kNormThreads / 64];
+    __shared__ __align__(16) float maxima[16];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const size_t row = blockIdx.x;
+    const int nvec = K >> 3, vc = tid < nvec ? tid : nvec - 1;
+    const uint16_t* xr = x + row * static_cast<size_t>(K);
+    u32x4 raw = *reinterpret_cast<const u32x4*>(xr + 8 * vc);
+    u32x4 raw_w;
+    if (wave < kNormThreads / 64) {
+        u32x4 more[NV];
+#pragma unroll
+        for (int i = 1; i < NV; ++i) {
+            const int v = tid + i * kNormThreads;
+            more[i] = *reinterpret_cast<const u32x4*>(xr + 8 * (v < nvec ? v : nvec - 1));
+        }
+        raw_w = *reinterpret_cast<const u32x4*>(weight + 8 * vc);
+        if (tid < 16) maxima[tid] = 0.0f;
+        more[0] = raw;
+        float ssq = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            float f[8];
+            unpack_bf16x8(more[i], f);
+            if (tid + i * kNormThreads < nvec) {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) ssq = fmaf(f[j], f[j], ssq);
+            }
+        }
+        ssq = wave_sum(ssq);
+        if (lane == 0) sums[wave] = ssq;
+    } else {
+        raw_w = *reinterpret_cast<const u32x4*>(weight + 8 * vc);
+    }
+    __syncthreads();
+    const float total = (sums[0] + sums[1]) + (sums[2] + sums[3]);
+    const float rstd = rsqrtf(total / static_cast<float>(K) + eps);
+    float h[8], w[8], amax = 0.0f;
+    unpack_bf16x8(raw, h);
+    unpack_bf16x8(raw_w, w);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {                                    // (a clamped vector is one of the row's: the maximum may see it twice)
+        h[j] = round_bf16(h[j] * rstd * w[j]);
+        amax = max_keep_nan(amax, fabsf(h[j]));
+    }
+    amax = wave_amax(amax);
+    if (lane == 0) maxima[wave] = amax;
+    if (y_out != nullptr && tid < nvec) *reinterpret_cast<u32x4*>(y_out + row * K + 8 * tid) = pack_bf16x8(h);
+    __syncthreads();
+    amax = 0.0f;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const f32x4 m = *reinterpret_cast<const f32x4*>(&maxima[4 * q]);
+        amax = max_keep_nan(max_keep_nan(amax, max_keep_nan(m[0], m[1])), max_keep_nan(m[2], m[3]));
+    }
+    uint16_t s_bits;
+    const float s = quant_scale(amax, quant_mode, &s_bits);
+    if (tid == 0) s_out[row] = s_bits;
+    if (tid >= nvec) return;
+    uint32_t q[2] = {0u, 0u};
+    if (quant_mode == QUANT_ROUNDED) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) q[j] = quant_rounded4(h[4 * j], h[4 * j + 1], h[4 * j + 2], h[4 * j + 3], s);
+    } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) q[j >> 2] |= (static_cast<uint32_t>(static_cast<int>(quant_value(h[j], s, quant_mode))) & 0xffu) << (8 * (j & 3));
+    }
+    *reinterpret_cast<u32x2*>(xq_out + row * K + 8 * tid) = u32x2{q[0], q[1]};
+}
+
 // quant_input of rows that no norm precedes (SpBitLinear on its own): x [M][K] -> (xq, s), one workgroup per row.
 // Bound: HBM on many rows, the launch on few.  It stands for the eleven elementwise and reduction launches of the same
 // lines in PyTorch (5000 x 6912: 350 us there, 21 us here; one row: 75 us of host time there, 2 us).

@@ -1266,3 +1266,34 @@ def test_quant_input_kernel(lib, m, k, mode):
         assert lib.ternaspmm_quant_input(_vp(xd), _vp(xd), _vp(xd), m, 60, None) == -1
     finally:
         lib.ternaspmm_quant_mode(O.QUANT_ROUNDED)
+
+
+@pytest.mark.parametrize("k", [2056, 2560, 4096, 4104, 6144, 6912, 8192])
+def test_norm_of_few_rows_has_the_bits_of_many(lib, k):
+    """Up to 128 rows are normed with a thread for every eight elements, more with 256 threads a row: the same rows both ways give the same integers,
+    scales and normed rows in every quantisation mode, rows of zeros, with an infinity or a NaN included."""
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    x = (torch.randn((200, k), generator=gen, device="cuda") * torch.rand((200, 1), generator=gen, device="cuda") * 20).bfloat16()
+    x[3], x[5, k // 3], x[7, k - 1], x[120, 0] = 0.0, float("inf"), float("nan"), 3e38
+    g = torch.randn(k, generator=gen, device="cuda").bfloat16()
+    def norm(rows):
+        m = rows.shape[0]
+        y, xq, s = torch.empty_like(rows), torch.empty((m, k), dtype=torch.int8, device="cuda"), torch.empty(m, dtype=torch.bfloat16, device="cuda")
+        lib.ternaspmm_rmsnorm_quant(_vp(rows), None, None, _vp(g), 1e-5, _vp(y), _vp(xq), _vp(s), m, k, None)
+        return y, xq, s
+
+    was = lib.ternaspmm_quant_mode(-1)
+    try:
+        for mode in (0, 1, 2):
+            lib.ternaspmm_quant_mode(mode)
+            many = norm(x)
+            few = [norm(x[at:at + rows].contiguous()) for at, rows in ((0, 1), (1, 71), (72, 128))]
+            torch.cuda.synchronize()
+            for want, got in zip(many, [torch.cat(parts) for parts in zip(*few)]):
+                if want.dtype == torch.int8:
+                    assert torch.equal(want, got)
+                else:
+                    assert torch.equal(torch.isnan(want), torch.isnan(got))
+                    assert torch.equal(torch.nan_to_num(want.float(), nan=0.0), torch.nan_to_num(got.float(), nan=0.0))
+    finally:
+        lib.ternaspmm_quant_mode(was)
