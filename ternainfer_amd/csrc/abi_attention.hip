@@ -562,15 +562,9 @@ int ternaspmm_step_attention_merge(const float* partial, int splits, const terna
     hipStream_t st = static_cast<hipStream_t>(stream);
     const int qmode = quant_mode();
     const NextWeights ahead = next != nullptr ? next_weights(next->packed, next->N, next->K, next->gate != 0, B) : NextWeights{};
+    const dim3 grid(B + ahead.workgroups), threads(static_cast<unsigned>((K / 8 + 63) / 64 * 64));
 #define TERNA_MERGE_NQ(DIM, SP)                                                                                           \
-    do {                                                                                                                  \
-        if (K <= 2048)                                                                                                    \
-            terna_attention_merge_norm_quant_kernel<DIM, SP, 1><<<dim3(B + ahead.workgroups), dim3(kNormThreads), 0, st>>>( \
-                partial, norm_weight, H, B * H, eps, o_out, nullptr, xq_out, s_out, qmode, B, ahead);                     \
-        else                                                                                                              \
-            terna_attention_merge_norm_quant_kernel<DIM, SP, 2><<<dim3(B + ahead.workgroups), dim3(kNormThreads), 0, st>>>( \
-                partial, norm_weight, H, B * H, eps, o_out, nullptr, xq_out, s_out, qmode, B, ahead);                     \
-    } while (0)
+    terna_attention_merge_norm_quant_kernel<DIM, SP><<<grid, threads, 0, st>>>(partial, norm_weight, H, B * H, eps, B, qmode, xq_out, s_out, o_out, ahead)
 #define TERNA_MERGE_NQ_D(DIM)                                                                                             \
     do {                                                                                                                  \
         switch (splits) {                                                                                                 \

@@ -171,83 +171,130 @@ __global__ __launch_bounds__(D) void terna_attention_merge_kernel(const float* _
 // terna_attention_merge_kernel and the norm kernel behind it (norm_quant_kernel.h) as one launch: one workgroup per
 // sequence forms its merged row -- H * D columns, rounded to bf16: the bits the merge kernel stores -- in registers and
 // runs the norm kernel's passes on it.  Everything a thread reads (its heads' statistics, SP partial results of eight
-// columns per vector, the norm weights) is requested before the first use.  o_out (optional): the merged row.
-template <int D, int SP, int NV>
-__global__ __launch_bounds__(kNormThreads) void terna_attention_merge_norm_quant_kernel(
-    const float* __restrict__ partial, const uint16_t* __restrict__ weight, int H, int heads_total, float eps,
-    uint16_t* __restrict__ o_out, uint16_t* __restrict__ y_out, int8_t* __restrict__ xq_out, uint16_t* __restrict__ s_out, int quant_mode,
-    int rows, NextWeights next)
+// columns, the norm weights) is requested before the first use.  o_out (optional): the merged row.
+// A thread for every eight columns (H * D <= 4096: up to eight waves): what bounds the launch is what one wave does in a row, and with 256
+// threads the first had two vectors of K = 2560 to fetch, merge and norm while the others fetched a vector for nothing.  The sum of squares is
+// that of 256 threads with the vectors t and t + 256: the latter ones' columns go to
+// them through LDS.  A step of 8 sequences, 1528 slots, 1155 -> 1145 us, of 7 with 1995 slots 1127 -> 1107.
+template <int D, int SP>
+__global__ __launch_bounds__(512) void terna_attention_merge_norm_quant_kernel(
+    const float* __restrict__ partial, const uint16_t* __restrict__ weight, int H, int heads_total, float eps, int rows, int quant_mode,
+    int8_t* __restrict__ xq_out, uint16_t* __restrict__ s_out, uint16_t* __restrict__ o_out, NextWeights next)
 {
     if (static_cast<int>(blockIdx.x) >= rows) {
         fetch_next_weights(next, rows);
         return;
     }
     static_assert(D % 8 == 0 && SP >= 1 && SP <= kAttentionMaxSplits && kAttentionMaxSplits == 8, "a vector lies inside one head");
-    const int tid = threadIdx.x;
+    __shared__ __align__(16) float later[kNormThreads][8];            // vectors 256 ..
+    __shared__ float sums[kNormThreads / 64];
+    __shared__ __align__(16) float maxima[8];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const size_t row = blockIdx.x;
-    const int K = H * D, nvec = K >> 3;
-    u32x4 raw_w[NV];
-    f32x4 st[NV][4], po[NV][SP][2];
+    const int K = H * D, nvec = K >> 3, vc = tid < nvec ? tid : nvec - 1;
+    const int head = (8 * vc) / D, d = (8 * vc) % D;
+    const size_t bh = row * H + head;
+    u32x4 raw_w;
+    f32x4 st[4], po[SP][2];
+    const f32x4* sp = reinterpret_cast<const f32x4*>(partial + bh * kAttentionStatFloats);
 #pragma unroll
-    for (int i = 0; i < NV; ++i) {
-        const int v = tid + i * kNormThreads;
-        const int vc = v < nvec ? v : nvec - 1;
-        const int head = (8 * vc) / D, d = (8 * vc) % D;
-        const size_t bh = row * H + head;
-        raw_w[i] = *reinterpret_cast<const u32x4*>(weight + 8 * vc);
-        const f32x4* sp = reinterpret_cast<const f32x4*>(partial + bh * kAttentionStatFloats);
+    for (int q = 0; q < 4; ++q) st[q] = sp[q];
+    const float* op = partial + attention_stat_floats(static_cast<size_t>(heads_total)) + bh * SP * D + d;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) st[i][q] = sp[q];
-        const float* op = partial + attention_stat_floats(static_cast<size_t>(heads_total)) + bh * SP * D + d;
-#pragma unroll
-        for (int j = 0; j < SP; ++j) {
-            po[i][j][0] = *reinterpret_cast<const f32x4*>(op + j * D);
-            po[i][j][1] = *reinterpret_cast<const f32x4*>(op + j * D + 4);
-        }
+    for (int j = 0; j < SP; ++j) {
+        po[j][0] = *reinterpret_cast<const f32x4*>(op + j * D);
+        po[j][1] = *reinterpret_cast<const f32x4*>(op + j * D + 4);
     }
+    raw_w = *reinterpret_cast<const u32x4*>(weight + 8 * vc);
 #pragma unroll
-    for (int i = 0; i < NV; ++i) {
-        pin_registers(raw_w[i]);
+    for (int q = 0; q < 4; ++q) pin_registers(st[q]);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) pin_registers(st[i][q]);
-#pragma unroll
-        for (int j = 0; j < SP; ++j) {
-            pin_registers(po[i][j][0]);
-            pin_registers(po[i][j][1]);
-        }
+    for (int j = 0; j < SP; ++j) {
+        pin_registers(po[j][0]);
+        pin_registers(po[j][1]);
     }
-    float h[NV][8];
+    // attention_merge's arithmetic on the values in registers
+    float mx[SP], dn[SP];
 #pragma unroll
-    for (int i = 0; i < NV; ++i) {
-        const int v = tid + i * kNormThreads;
-        if (v < nvec) {
-            // attention_merge's arithmetic on the values in registers
-            float mx[SP], dn[SP];
-#pragma unroll
-            for (int j = 0; j < SP; ++j) {
-                mx[j] = st[i][j >> 2][j & 3];
-                dn[j] = st[i][2 + (j >> 2)][j & 3];
-            }
-            float m_all = -INFINITY;
-#pragma unroll
-            for (int j = 0; j < SP; ++j) m_all = fmaxf(m_all, mx[j]);
-            float wj[SP], den = 0.0f;
-#pragma unroll
-            for (int j = 0; j < SP; ++j) {
-                wj[j] = __expf(mx[j] - m_all);
-                den = fmaf(wj[j], dn[j], den);
-            }
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                float num = 0.0f;
-#pragma unroll
-                for (int j = 0; j < SP; ++j) num = fmaf(wj[j], po[i][j][e >> 2][e & 3], num);
-                h[i][e] = round_bf16(num / den);
-            }
-            if (o_out != nullptr) *reinterpret_cast<u32x4*>(o_out + row * K + 8 * v) = pack_bf16x8(h[i]);
-        }
+    for (int j = 0; j < SP; ++j) {
+        mx[j] = st[j >> 2][j & 3];
+        dn[j] = st[2 + (j >> 2)][j & 3];
     }
-    norm_quant_passes<NV>(h, raw_w, K, eps, row, y_out, xq_out, s_out, quant_mode);
+    float m_all = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < SP; ++j) m_all = fmaxf(m_all, mx[j]);
+    float wj[SP], den = 0.0f;
+#pragma unroll
+    for (int j = 0; j < SP; ++j) {
+        wj[j] = __expf(mx[j] - m_all);
+        den = fmaf(wj[j], dn[j], den);
+    }
+    float h[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        float num = 0.0f;
+#pragma unroll
+        for (int j = 0; j < SP; ++j) num = fmaf(wj[j], po[j][e >> 2][e & 3], num);
+        h[e] = round_bf16(num / den);
+    }
+    if (o_out != nullptr && tid < nvec) *reinterpret_cast<u32x4*>(o_out + row * K + 8 * tid) = pack_bf16x8(h);
+
+    const bool two = nvec > kNormThreads;                                // uniform
+    if (tid < 8) maxima[tid] = 0.0f;
+    if (two) {
+        if (tid >= kNormThreads) {
+            *reinterpret_cast<f32x4*>(&later[tid - kNormThreads][0]) = f32x4{h[0], h[1], h[2], h[3]};
+            *reinterpret_cast<f32x4*>(&later[tid - kNormThreads][4]) = f32x4{h[4], h[5], h[6], h[7]};
+        }
+        __syncthreads();
+    }
+    if (wave < kNormThreads / 64) {
+        float ssq = 0.0f;
+        if (tid < nvec) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) ssq = fmaf(h[e], h[e], ssq);
+        }
+        if (tid + kNormThreads < nvec) {
+            const f32x4 lo = *reinterpret_cast<const f32x4*>(&later[tid][0]), hi = *reinterpret_cast<const f32x4*>(&later[tid][4]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) ssq = fmaf(lo[e], lo[e], ssq);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) ssq = fmaf(hi[e], hi[e], ssq);
+        }
+        ssq = wave_sum(ssq);
+        if (lane == 0) sums[wave] = ssq;
+    }
+    __syncthreads();
+    // (waves that a short row does not have: their sums are zeros)
+    const int waves = static_cast<int>(blockDim.x) >> 6;
+    const float total = (sums[0] + (waves > 1 ? sums[1] : 0.0f)) + ((waves > 2 ? sums[2] : 0.0f) + (waves > 3 ? sums[3] : 0.0f));
+    const float rstd = rsqrtf(total / static_cast<float>(K) + eps);
+    float w[8], amax = 0.0f;
+    unpack_bf16x8(raw_w, w);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {                                        // (a clamped vector is one of the row's: the maximum may see it twice)
+        h[e] = round_bf16(h[e] * rstd * w[e]);
+        amax = max_keep_nan(amax, fabsf(h[e]));
+    }
+    amax = wave_amax(amax);
+    if (lane == 0) maxima[wave] = amax;
+    __syncthreads();
+    const f32x4 lo = *reinterpret_cast<const f32x4*>(&maxima[0]), hi = *reinterpret_cast<const f32x4*>(&maxima[4]);
+    amax = max_keep_nan(max_keep_nan(max_keep_nan(lo[0], lo[1]), max_keep_nan(lo[2], lo[3])), max_keep_nan(max_keep_nan(hi[0], hi[1]), max_keep_nan(hi[2], hi[3])));
+    uint16_t s_bits;
+    const float s = quant_scale(amax, quant_mode, &s_bits);
+    if (tid == 0) s_out[row] = s_bits;
+    if (tid >= nvec) return;
+    uint32_t q[2] = {0u, 0u};
+    if (quant_mode == QUANT_ROUNDED) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) q[j] = quant_rounded4(h[4 * j], h[4 * j + 1], h[4 * j + 2], h[4 * j + 3], s);
+    } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) q[j >> 2] |= (static_cast<uint32_t>(static_cast<int>(quant_value(h[j], s, quant_mode))) & 0xffu) << (8 * (j & 3));
+    }
+    *reinterpret_cast<u32x2*>(xq_out + row * K + 8 * tid) = u32x2{q[0], q[1]};
 }
 
 // Extra workgroups of the attention launch (blockIdx.x >= heads) that pull up to kAttentionPrefetchRegions regions of
