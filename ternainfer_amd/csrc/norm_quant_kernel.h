@@ -137,7 +137,7 @@ __device__ __forceinline__ void quant_pass(const float (&h)[NV][8], float amax, 
     }
 }
 
-// The passes behind the formation of a row, for every kernel that holds one in registers (h[i][j] = element
+// The passes behind the formation of a row in registers (h[i][j] = element
 // 8 (tid + kNormThreads i) + j, vectors past K / 8 unused; raw_w the norm weights of the same elements): sum of squares
 // -- per thread in element order, the lanes of a wave by group_reduce, the four waves pairwise -- then the norm, the row
 // maximum, the scale and the int8 values.  y_out / xq_out + s_out: optional outputs.
