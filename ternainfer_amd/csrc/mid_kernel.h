@@ -35,6 +35,23 @@ namespace terna {
 
 constexpr int kMidMaxWaves = 16;
 
+// f(std::integral_constant<int, n>{}) for n = 1 .. MOST: a uniform branch to code that knows the number.
+template <int MOST, typename Function>
+__device__ __forceinline__ void with_constant(int n, Function&& f)
+{
+    static_assert(MOST >= 1 && MOST <= 16, "cases below");
+    switch (n) {
+#define TERNA_CASE(V) \
+    case V: \
+        if constexpr (V <= MOST) f(std::integral_constant<int, V>{}); \
+        break
+        TERNA_CASE(1); TERNA_CASE(2); TERNA_CASE(3); TERNA_CASE(4); TERNA_CASE(5); TERNA_CASE(6); TERNA_CASE(7); TERNA_CASE(8);
+        TERNA_CASE(9); TERNA_CASE(10); TERNA_CASE(11); TERNA_CASE(12); TERNA_CASE(13); TERNA_CASE(14); TERNA_CASE(15); TERNA_CASE(16);
+#undef TERNA_CASE
+    default: __builtin_unreachable();
+    }
+}
+
 template <typename Act, int RT, int FB>
 struct MidShape {
     static constexpr int kRowBytes = 256 * static_cast<int>(sizeof(Act));    // a chunk's piece of one activation row
@@ -73,6 +90,7 @@ __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
     constexpr int SZ = static_cast<int>(sizeof(Act));
     static_assert(!QUANT || (RT == 1 && !BF16 && EPI == PACKED_STORE && FB * 1024 <= MidQuantShape::kWaveBytes), "see above");
     constexpr int WAVE_BYTES = QUANT ? MidQuantShape::kWaveBytes : S::kWaveBytes;
+    constexpr int MOST_WAVES = 160 * 1024 / WAVE_BYTES < kMidMaxWaves ? 160 * 1024 / WAVE_BYTES : kMidMaxWaves;
     constexpr int PIECES = 16 * SZ;                      // 16-byte pieces of a chunk row
     constexpr int ROWS_PER_LOAD = 64 / PIECES;           // rows one direct load fills
     constexpr int XI = 16 * RT / ROWS_PER_LOAD;          // direct loads per chunk
@@ -211,25 +229,34 @@ __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
     } else {
         issue(wave);
     }
-    // ---- a thread's results: F neighbouring features of one row, so that about 512 threads finish at a time
+    // ---- a thread's results: 2^f neighbouring features of one row, as few as give every thread of the workgroup some (four are a unit of sums)
     constexpr bool GATE = EPI == PACKED_GATE;
+    constexpr int X = GATE ? 2 : 1;
     constexpr int UNITS = 4 * FB;                        // 16-byte units (four features) of a row of sums
-    constexpr int OUT_UNITS = GATE ? UNITS / 2 : UNITS;  // ... of a row of results
-    constexpr int FEW = EPI == PACKED_ROPE ? 2 : 1, ALL = RT * OUT_UNITS / 8;
-    constexpr int F = ALL < FEW ? FEW : ALL;
-    constexpr int PER_ROW = OUT_UNITS * 4 / F, TASKS = 16 * RT * PER_ROW;
-    static_assert(F == 1 || F == 2 || F == 4, "features of a thread");
-    typedef AccScalar Sums __attribute__((ext_vector_type(F)));
-    // what the first of them needs at the end is requested here
+    constexpr int OUT_UNITS = UNITS / X;                 // ... of a row of results
+    constexpr int RESULTS = 16 * RT * OUT_UNITS * 4;
+    constexpr auto log_features = [](int of_waves) {
+        const int few = EPI == PACKED_ROPE ? 2 : 1, f = RESULTS / (64 * (of_waves >= 8 ? 8 : of_waves >= 4 ? 4 : 1)), n = f < few ? few : f;
+        return n >= 4 ? 2 : n == 2 ? 1 : 0;
+    };
+    constexpr int MANY = 1 << log_features(8);           // of eight waves or more
+    // (One wave of K <= 256 with a feature a thread went eight times through its results, each time waiting for their scales: 17 x 704 x 192 4.6 us int8,
+    // 4.1 bf16; four features a thread 3.6, 3.0.)
+    // What they need at the end, the first of them requested here.  Values on the way must not be moved, not even to where two branches meet: that
+    // waits for every load before them (two ways of requesting them, by the number of waves, cost every launch 0.3 us).  So there is
+    // one way, and the scales that only threads with more features have are in branches that nothing else ends in.
     struct Finish {
-        uint32_t s, w[GATE ? 2 : F], stream[(F + 1) / 2];
-        float turn_c[(F + 1) / 2], turn_s[(F + 1) / 2];
+        uint32_t s, w[4];
+        u32x2 stream;                                    // the unit of four
+        float2 turn_c, turn_s;                           // "
         uint16_t* to;
     };
     const int out_n0 = band0 * (GATE ? 8 : 16);
-    auto request_finish = [&](int idx) __attribute__((always_inline)) {
-        Finish f{};
-        const int row = idx / PER_ROW, m = m0 + row < M ? m0 + row : M - 1, n0 = out_n0 + F * (idx % PER_ROW);
+    auto request_finish = [&](int idx, auto log_f) __attribute__((always_inline)) {
+        Finish f;
+        constexpr int LOG_ROW = __builtin_ctz(OUT_UNITS * 4);
+        const int shift = LOG_ROW - log_f, row = idx >> shift, m = m0 + row < M ? m0 + row : M - 1;
+        const int n0 = out_n0 + ((idx & ((1 << shift) - 1)) << log_f);
         if constexpr (!BF16 && !QUANT) f.s = ep.s[m];
         if constexpr (GATE) {
             f.w[0] = ep.ws[0];
@@ -238,36 +265,26 @@ __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
             int group[4] = {0, 0, 0, 0};
             if (ep.ws_num != 1) {
                 ws_group_decode4(n0, N, ep.ws_num, group);
-                if (ep.kind == EP_I8_PREFILL) {
-#pragma unroll
-                    for (int v = 0; v < F; ++v) group[v] = ws_group_prefill(n0 + v, N, ep.ws_num);
-                }
+                if (ep.kind == EP_I8_PREFILL) group[0] = group[1] = group[2] = group[3] = ws_group_prefill(n0, N, ep.ws_num);
             }
+            auto scale_of = [&](int v) -> uint32_t { return BF16 ? __float_as_uint(ep.scale[group[v]]) : ep.ws[group[v]]; };
 #pragma unroll
-            for (int v = 0; v < F; ++v) f.w[v] = BF16 ? __float_as_uint(ep.scale[group[v]]) : ep.ws[group[v]];
+            for (int v = 0; v < MANY; ++v) f.w[v] = scale_of(v);
+#pragma unroll
+            for (int v = MANY; v < 4; ++v)
+                if (v < 1 << log_f) f.w[v] = scale_of(v);                // uniform
         }
-        if constexpr (EPI == PACKED_RESIDUAL) {
-            const uint16_t* from = guard.rows + static_cast<size_t>(m) * N + n0;
-            if constexpr (F == 1) f.stream[0] = *from;
-            else if constexpr (F == 2) f.stream[0] = *reinterpret_cast<const uint32_t*>(from);
-            else {
-                const u32x2 v = *reinterpret_cast<const u32x2*>(from);
-                f.stream[0] = v.x;
-                f.stream[1] = v.y;
-            }
-        }
+        if constexpr (EPI == PACKED_RESIDUAL) f.stream = *reinterpret_cast<const u32x2*>(guard.rows + static_cast<size_t>(m) * N + (n0 & ~3));
         if constexpr (EPI == PACKED_ROPE) {
-            const int at = guard.table_row(m) * (guard.D >> 1) + ((n0 % guard.D) >> 1);
-#pragma unroll
-            for (int v = 0; v < F / 2; ++v) {
-                f.turn_c[v] = guard.cos[at + v];
-                f.turn_s[v] = guard.sin[at + v];
-            }
+            const int at = guard.table_row(m);
+            f.turn_c = guard.angles2(guard.cos, at, n0 & ~3);
+            f.turn_s = guard.angles2(guard.sin, at, n0 & ~3);
             f.to = guard.place(out, m, n0, N);
         }
         return f;
     };
-    Finish first = request_finish(tid < TASKS ? tid : 0);
+    const int log_first = waves >= 8 ? log_features(8) : waves >= 4 ? log_features(4) : log_features(1);
+    Finish first = request_finish(tid < (RESULTS >> log_first) ? tid : 0, log_first);
     float* const maxima = reinterpret_cast<float*>(smem + waves * WAVE_BYTES);          // [row][wave]
     float* const multiplier = maxima + 16 * kMidMaxWaves + 16 * wave;                    // of row r: at 8 (r & 1) + r / 2
     float* const scale = maxima + 32 * kMidMaxWaves;
@@ -333,37 +350,39 @@ __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
 #pragma unroll
         for (int b = 0; b < FB; ++b)
             *reinterpret_cast<Acc*>(mine + ((16 * r + i) * UNITS + ((4 * b + g) ^ ((i >> SWZ) & (UNITS - 1)))) * 16) = acc[r][b];
-    asm volatile("" : "+v"(first.s), "+v"(first.w[0]), "+v"(first.stream[0]));
+    asm volatile("" : "+v"(first.w[0]));
+    if constexpr (!BF16 && !QUANT) asm volatile("" : "+v"(first.s));
+    if constexpr (EPI == PACKED_RESIDUAL) asm volatile("" : "+v"(first.stream));
     __syncthreads();
     // All waves' sums of a result are read before the first is added (one after the other they took 2000 - 3500 of a launch's 6000 - 12000
-    // clocks); W: of the waves that the usual depths of K give (bf16, K = 6912 and 32 rows a tile: nine), else of any number up to W: read up to
-    // sixteen, a module call of 114 rows of that was 11.4 us, 10.9 so.
-    auto finish = [&](auto count, auto exact) __attribute__((always_inline)) {
-        constexpr int W = decltype(count)::value;
-        constexpr bool EXACT = decltype(exact)::value;
-        for (int idx = tid; idx < TASKS; idx += waves * 64) {
+    // clocks), by code of its own for every number of waves.  Read as up to eight or sixteen, the ones that are not there cost, us a launch, int8; bf16:
+    // 32 rows of N = 2560 K = 4096 3.9 (sixteen by number) / 4.3; 300 rows of N = 704 K = 320 (two) 3.5 / 3.9; 4.0 / 4.6.
+    with_constant<MOST_WAVES>(waves, [&](auto count) __attribute__((always_inline)) {
+        constexpr int W = decltype(count)::value, LOG_F = log_features(W), F = 1 << LOG_F, PER_ROW = OUT_UNITS * 4 / F;
+        typedef AccScalar Sums __attribute__((ext_vector_type(F)));
+        for (int idx = tid; idx < RESULTS / F; idx += W * 64) {
             const int row = idx / PER_ROW, n = F * (idx % PER_ROW), m = m0 + row, u = n >> 2, sub = n & 3;
             if (m >= M) break;
             const int q = GATE ? 8 * (u >> 2) + (u & 3) : u;
-            Sums part[GATE ? 2 : 1][W], sum[GATE ? 2 : 1];
+            Sums part[X][W], sum[X];
 #pragma unroll
-            for (int x = 0; x < (GATE ? 2 : 1); ++x) {
+            for (int x = 0; x < X; ++x) {
                 const uint8_t* from = smem + (row * UNITS + ((q + 4 * x) ^ (((row & 15) >> SWZ) & (UNITS - 1)))) * 16 + sub * 4;
 #pragma unroll
-                for (int v = 0; v < W; ++v) part[x][v] = *reinterpret_cast<const Sums*>(from + (EXACT || v < waves ? v : 0) * WAVE_BYTES);
+                for (int v = 0; v < W; ++v) part[x][v] = *reinterpret_cast<const Sums*>(from + v * WAVE_BYTES);
             }
-            const Finish f = idx == tid ? first : request_finish(idx);
+            const Finish f = idx == tid ? first : request_finish(idx, std::integral_constant<int, LOG_F>{});
 #pragma unroll
-            for (int x = 0; x < (GATE ? 2 : 1); ++x) {
+            for (int x = 0; x < X; ++x) {
                 sum[x] = part[x][0];
 #pragma unroll
-                for (int v = 1; v < W; ++v) sum[x] += EXACT || v < waves ? part[x][v] : Sums(0);
+                for (int v = 1; v < W; ++v) sum[x] += part[x][v];
             }
             // sums -> outputs rounded to bf16, as apply_epilogue has them; under the prefill rule F features of a 128-column tile share a scale
             const float s = BF16 ? 1.0f : QUANT ? scale[row] : __uint_as_float(f.s << 16);
-            float r[GATE ? 2 : 1][F];
+            float r[X][F];
 #pragma unroll
-            for (int x = 0; x < (GATE ? 2 : 1); ++x)
+            for (int x = 0; x < X; ++x)
 #pragma unroll
                 for (int v = 0; v < F; ++v) {
                     if constexpr (BF16) r[x][v] = sum[x][v] * kBf16WeightUndo;
@@ -376,14 +395,14 @@ __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
             } else if (ep.kind == EP_I8_DECODE) {
                 const RowQuotient by(s);
 #pragma unroll
-                for (int x = 0; x < (GATE ? 2 : 1); ++x) {
+                for (int x = 0; x < X; ++x) {
                     by.of(r[x]);
 #pragma unroll
                     for (int v = 0; v < F; ++v) r[x][v] = __fmul_rn(r[x][v], weight(x, v));
                 }
             } else {
 #pragma unroll
-                for (int x = 0; x < (GATE ? 2 : 1); ++x) {
+                for (int x = 0; x < X; ++x) {
                     const float coeff = s != 0.0f ? __fdiv_rn(weight(x, 0), s) : 0.0f;
 #pragma unroll
                     for (int v = 0; v < F; ++v) r[x][v] = __fmul_rn(r[x][v], coeff);
@@ -402,9 +421,14 @@ __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
 #pragma unroll
             for (int v = 0; v < (F + 1) / 2; ++v) {
                 pair[v] = F == 1 ? o[0] : o[2 * v] | (static_cast<uint32_t>(o[F == 1 ? 0 : 2 * v + 1]) << 16);
-                if constexpr (EPI == PACKED_RESIDUAL) pair[v] = ResidualRows::pair(pair[v], f.stream[v]);
+                // (of a unit's two pairs, or of a pair's two features, this thread's first)
+                if constexpr (EPI == PACKED_RESIDUAL) {
+                    const uint32_t word = F == 4 ? f.stream[v] : sub < 2 ? f.stream[0] : f.stream[1];
+                    pair[v] = ResidualRows::pair(pair[v], F == 1 && (sub & 1) ? word >> 16 : word);
+                }
                 if constexpr (EPI == PACKED_ROPE) {
-                    if (guard.part(out_n0 + n) < 2) pair[v] = RopeStore::rotate(pair[v], f.turn_c[v], f.turn_s[v]);
+                    const bool second = F == 4 ? v == 1 : sub >= 2;
+                    if (guard.part(out_n0 + n) < 2) pair[v] = RopeStore::rotate(pair[v], second ? f.turn_c.y : f.turn_c.x, second ? f.turn_s.y : f.turn_s.x);
                 }
             }
             uint16_t* to = EPI == PACKED_ROPE ? f.to : out + static_cast<size_t>(m) * (GATE ? N >> 1 : N) + out_n0 + n;
@@ -413,15 +437,7 @@ __global__ __launch_bounds__(kMidMaxWaves * 64) void terna_mid_kernel(
             else if constexpr (F == 2) *reinterpret_cast<uint32_t*>(to) = pair[0];
             else *reinterpret_cast<u32x2*>(to) = u32x2{pair[0], pair[1]};
         }
-    };
-    using Exact = std::true_type;
-    using UpTo = std::false_type;
-    if (waves == 10) finish(std::integral_constant<int, 10>{}, Exact{});
-    else if (waves == 4) finish(std::integral_constant<int, 4>{}, Exact{});
-    else if (BF16 && waves == 9) finish(std::integral_constant<int, 9>{}, Exact{});
-    else if (waves == 14) finish(std::integral_constant<int, 14>{}, Exact{});
-    else if (waves <= 8) finish(std::integral_constant<int, 8>{}, UpTo{});
-    else finish(std::integral_constant<int, kMidMaxWaves>{}, UpTo{});
+    });
 }
 
 }  // namespace terna

@@ -868,6 +868,52 @@ def test_mid_kernel_against_the_forced_kernels(lib, act, m, n, k):
         assert max_err <= 1e-2 * max_ref and med_ulp <= 1, (max_err, max_ref, med_ulp)
 
 
+@pytest.mark.parametrize("k", [64, 320, 768, 896, 1280, 1408, 1792, 1920, 2304, 2560, 2752, 3072, 3328, 3584, 3776, 4096, 6912])
+def test_mid_kernel_with_every_number_of_waves(lib, k):
+    """The same kernel's last sums, whose code is one for each of its 1 to 16 waves: all three tiles with a workgroup a CU, and many workgroups of up to four
+    waves; plain outputs of both types, the residual, gate and rotary epilogues.  int8 bit for bit against the small-M kernel (and what the
+    epilogues stand for on its outputs), bf16 within the family's bar of products in float64."""
+    from ternainfer_amd import repack_weight
+    from ternainfer_amd.linear import interleave_gate_up
+    n, h, kv, d = 2560, 12, 4, 128
+    fmt = DeviceFormat(make_ternary(n, k, 0.40, 4400 + k))
+    packed = repack_weight(fmt.vals, fmt.off, fmt.med, fmt.bm, n, k)
+    gated = interleave_gate_up(packed, n, k)
+    dense = torch.from_numpy(fmt.w).cuda().double()
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    ws = torch.tensor([1.25, 0.75], dtype=torch.bfloat16, device="cuda")
+    bits = lambda a: a.contiguous().view(torch.int16)
+    for m in (20, 61, 90, 150, 430):
+        print(f"[case] mid kernel, every number of waves M={m} K={k}", flush=True)
+        x = torch.randint(-127, 128, (m, k), generator=gen, device="cuda", dtype=torch.int8)
+        s = (torch.rand(m, generator=gen, device="cuda") * 20 + 5).bfloat16()
+        out, want, added, two = torch.zeros((4, m, n), dtype=torch.bfloat16, device="cuda")
+        for route, o in ((0, out), (4, want)):
+            lib.bitlinear_TernaSpMM_packed(vp(x), vp(packed), vp(o), vp(s), vp(ws), 2, m, n, k, route, None)
+        stream = torch.randn((m, n), generator=gen, device="cuda").bfloat16() * want.float().std().bfloat16()
+        assert lib.ternaspmm_residual_linear(vp(x), vp(packed), vp(added), vp(s), vp(ws), 2, vp(stream), m, n, k, None, 0, None) == 1
+        gate = torch.zeros((m, n // 2), dtype=torch.bfloat16, device="cuda")
+        assert lib.ternaspmm_gate_linear(vp(x), vp(gated), vp(gate), vp(s), vp(ws), 2, m, n, k, None) == 1
+        pos, caches = torch.arange(m, device="cuda") + 2, torch.zeros((4, kv, m + 2, d), dtype=torch.bfloat16, device="cuda")
+        angle = torch.rand((m, d // 2), generator=gen, device="cuda") * 6
+        cos, sin, q = angle.cos().contiguous(), angle.sin().contiguous(), torch.zeros((h, m, d), dtype=torch.bfloat16, device="cuda")
+        assert lib.ternaspmm_qkv_rope_linear(vp(x), vp(packed), vp(two), vp(s), vp(ws), 2, m, n, k, vp(cos), vp(sin), vp(pos), 0, vp(caches[0]), vp(caches[1]),
+                                             m, h, kv, d, m + 2, None) == 1
+        lib.ternaspmm_rope_kv_store(vp(want), vp(cos), vp(sin), vp(pos), 0, vp(q), vp(caches[2]), vp(caches[3]), 1, m, h, kv, d, m + 2, 1, None)
+        torch.cuda.synchronize()
+        assert torch.equal(bits(out), bits(want))
+        assert torch.equal(added, stream + want)
+        assert torch.equal(gate, torch.relu(want[:, :n // 2]).square() * want[:, n // 2:])
+        assert torch.equal(bits(two[:, :h * d]), bits(q.transpose(0, 1).reshape(m, h * d)))
+        assert torch.equal(bits(caches[0]), bits(caches[2])) and torch.equal(bits(caches[1]), bits(caches[3]))
+        xb, sc = torch.randn((m, k), generator=gen, device="cuda").bfloat16(), ws.float()
+        lib.bitlinear_TernaSpMM_bf16_packed(vp(xb), vp(packed), vp(out), vp(sc), 2, m, n, k, 0, None)
+        torch.cuda.synchronize()
+        exact = (xb.double() @ dense.T) * sc.double().repeat_interleave(n // 2)
+        assert float((out.double() - exact).abs().max()) <= 1e-2 * float(exact.abs().max())
+        assert float((out.double() - exact).norm() / exact.norm()) <= 2.0 ** -8               # of a rounding to bf16: 2^-9 at most
+
+
 @pytest.mark.parametrize("act", ["int8", "bf16"])
 @pytest.mark.parametrize("m,n,k", [(64, 13824, 192), (70, 13824, 192), (256, 3840, 320), (257, 3840, 320), (1024, 960, 128), (1025, 960, 128), (2048, 256, 320),
                                    (2049, 256, 320), (1500, 704, 320)])
