@@ -8,7 +8,6 @@ namespace {
 
 struct MidTile {
     int rt, fb;                  // 16-row tiles, 16-feature bands of a workgroup
-    long tiles;
     int waves;
 };
 
@@ -16,8 +15,10 @@ struct MidTile {
 // (workgroups per CU, rounded up) x (bytes of one workgroup per 4 columns of K: 64 rt sz activations + 16 fb weights).
 // One workgroup per CU: as many waves as K has chunks for, evenly (K = 6912, 27 chunks: fourteen waves take them in two rounds, twelve in three: 32 rows
 // 5.6 -> 5.0 us a launch); more of them: four waves each, whose small LDS shares
-// let four or five workgroups overlap on a CU (measured at M = 17 .. 512: within 5 % of the best of the tiles and wave counts
-// in all but two of ninety cells).
+// let four or five workgroups overlap on a CU.  How many a CU has is counted with feature tiles in eights, as they lie on the XCDs (N = 128: a workgroup per
+// CU by their number, four on the CUs that have any; sixteen waves' LDS each then run one after the other: 1500 rows, K = 6912, int8 15.7 -> 12.2 us,
+// bf16 26.1 -> 21.2; 1000 rows, N = 256, K = 4096, bf16 12.4 -> 11.2; 1224 launches of N = 64 - 1536, geometric mean 0.978).  The tile is chosen by their number: counted
+// in eights for that too, the mean is 0.94, but 32-row tiles of short K come out up to 1.3 times as slow (850 rows, N = 704, K = 64: 4.6 -> 5.7 us).
 MidTile choose_tile(int M, int N, int K, int sz)
 {
     const int chunks = (K / 64 + 3) / 4;
@@ -28,14 +29,15 @@ MidTile choose_tile(int M, int N, int K, int sz)
         const long tiles = static_cast<long>((M + 16 * t[0] - 1) / (16 * t[0])) * ((N / 16 + t[1] - 1) / t[1]);
         const long cost = (tiles + 255) / 256 * (64 * t[0] * sz + 16 * t[1]);
         if (best.rt == 0 || cost < best_cost) {
-            best = MidTile{t[0], t[1], tiles, 0};
+            best = MidTile{t[0], t[1], 0};
             best_cost = cost;
         }
     }
+    const bool shared = static_cast<long>((M + 16 * best.rt - 1) / (16 * best.rt)) * ((N / 16 + 8 * best.fb - 1) / (8 * best.fb) * 8) > 256;
     const int fit = 160 * 1024 / (16 * best.rt * 256 * sz);                // LDS of a workgroup
-    const int most = best.tiles > 256 ? 4 : (fit < kMidMaxWaves ? fit : kMidMaxWaves);
+    const int most = shared ? 4 : (fit < kMidMaxWaves ? fit : kMidMaxWaves);
     const int rounds = (chunks + most - 1) / most;
-    best.waves = best.tiles > 256 ? (chunks < most ? chunks : most) : (chunks + rounds - 1) / rounds;
+    best.waves = shared ? (chunks < most ? chunks : most) : (chunks + rounds - 1) / rounds;
     return best;
 }
 

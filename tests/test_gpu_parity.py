@@ -834,7 +834,7 @@ def test_gpu_sleep_and_error_check(lib):
 
 @pytest.mark.parametrize("act", ["int8", "bf16"])
 @pytest.mark.parametrize("m,n,k", [(17, 64, 64), (32, 128, 192), (33, 2560, 320), (37, 192, 6912), (48, 3840, 2560), (100, 2560, 1088),
-                                   (64, 13824, 128), (113, 704, 2560), (300, 2560, 512), (1000, 192, 832)])
+                                   (64, 13824, 128), (113, 704, 2560), (300, 2560, 512), (1000, 192, 832), (1500, 128, 2304), (1030, 320, 1280)])
 def test_mid_kernel_against_the_forced_kernels(lib, act, m, n, k):
     """The kernel between the small-M and the MFMA-tiled one (mid_kernel.h), which serves these calls when the library chooses:
     each tile it has, partial last chunks, row and feature tiles that hang over, one to three scale groups; int8 bit for bit
