@@ -123,10 +123,16 @@ void launch_mid_quant(const uint16_t* x, const uint32_t* packed, uint16_t* out, 
 // 10.8 / 9.6, M = 280 (576) 7.7 / 8.1; 10.9 / 12.7; gate+up M = 64 (432) 8.2 / 7.1; 10.7 / 9.8, M = 70 (648) 8.0 / 8.4; 11.8 / 12.8; down M = 350
 // (440) 13.2 / 11.2; 22.2 / 18.3, M = 430 (560) 13.4 / 14.2; 22.3 / 28.2; N = 1024 = K, M = 1000 (512) 5.2 / 4.6; 6.3 / 5.5, M = 1200 (608) 5.3 / 5.4;
 // 6.6 / 7.3; N = 256, M = 1000 (256) 6.9 / 5.0; 11.5 / 9.3, M = 4000 (1000) 7.7 / 13.2; 12.1 / 23.8; N = 704, K = 320, M = 1500 (752) 4.4 / 6.0; 4.6 / 7.5.
+// Few rows of a wide matrix stay here up to four tiles a CU: a tile of the MFMA-tiled kernel has 64 rows, half of them and more for nothing, and up to 32 rows the
+// small-M kernel takes what this one leaves.  The other kernel / this one: 17 rows, N = 65536 (1024 tiles) K = 1024 9.1 / 7.7; 11.5 / 11.1, K = 4096 20.7 / 15.4; 30.5 / 23.9;
+// 32 rows, N = 40960 K = 4096 15.8 / 12.7; 22.9 / 17.6; 33 - 48 rows, N = 20480 (640) K = 1024 6.4 / 5.0; 7.0 / 6.1, K = 4096 10.5 / 9.2; 15.1 / 14.1, N = 32768 (1024)
+// 11.9 / 12.2; 16.3 / 19.3; 64 rows, N = 20480 10.8 / 11.5; 15.4 / 16.9.  Where K is short the others are ahead: 32 rows, N = 49152 K = 64 4.4 / 6.7;
+// 5.4 / 6.1, K = 320 5.4 / 6.4; 6.8 / 6.8, K = 512 6.2 / 6.5; 7.1 / 6.9; 40 rows, N = 20480, K = 320 5.4 / 4.7; 4.9 / 5.3.
 bool mid_kernel_takes(const void* x, int M, int N, int K, size_t act_bytes)
 {
     const long tiles = static_cast<long>((M + 31) / 32) * ((N / 16 + 31) / 32 * 8);
-    return M > 16 && tiles <= 512 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
+    const long most = M > 48 ? 512 : M > 32 ? (K >= 512 ? 640 : 512) : K * act_bytes >= 1024 ? 1024 : 512;
+    return M > 16 && tiles <= most && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
            static_cast<uint64_t>(M) * K * act_bytes < (1ull << 31) && static_cast<uint64_t>(N) * K / 4 < (1ull << 31);
 }
 

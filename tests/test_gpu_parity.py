@@ -916,7 +916,7 @@ def test_mid_kernel_with_every_number_of_waves(lib, k):
 
 @pytest.mark.parametrize("act", ["int8", "bf16"])
 @pytest.mark.parametrize("m,n,k", [(64, 13824, 192), (70, 13824, 192), (256, 3840, 320), (257, 3840, 320), (1024, 960, 128), (1025, 960, 128), (2048, 256, 320),
-                                   (2049, 256, 320), (1500, 704, 320)])
+                                   (2049, 256, 320), (1500, 704, 320), (32, 49152, 512), (32, 49152, 448), (20, 40960, 1024), (17, 66048, 512), (48, 20480, 512), (49, 20480, 512)])
 def test_calls_on_both_sides_of_the_mid_kernels_limit(lib, act, m, n, k):
     """The last rows that the kernel of a few hundred rows takes and the first that the MFMA-tiled one does, wide, narrow and odd matrices."""
     test_mid_kernel_against_the_forced_kernels(lib, act, m, n, k)
