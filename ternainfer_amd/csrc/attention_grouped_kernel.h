@@ -20,6 +20,8 @@
 // trip, behind it the third pass and the sums.  Measured, the launch alone in a graph, us, keys and values in registers with vector multiply-adds ->
 // this: 32 sequences x 512 slots of different lengths filled to 60 % 10.6 -> 9.3, of one length 11.1 -> 9.8, 8 x 1528 to 90 % over six splits 10.5 -> 8.8,
 // 16 x 512 over three 8.6 -> 7.1, 48 x 400 10.5 -> 9.1, 64 x 1000 21.6 -> 20.9; a decode step of 8 x 1528 1200 -> 1157, of 32 x 512 1500 -> 1461.
+// The last batch of values apart from the others, its rows behind the prefix not weighed, the slices' sums read ahead, us before -> after (in registers):
+// 6 sequences x 64 slots, D = 64, 8 heads on 4 6.0 -> 4.9 (4.7), 8 x 200 to 10 % 6.0 -> 5.4 (5.8); 32 x 512 9.0 -> 8.4 (9.5), 64 x 2048 to 95 % 54.5 -> 51.5 (50.9).
 // Tried: four units of a wave under way, from the start or once the keys are in (level to 7 % slower).
 #pragma once
 
@@ -288,36 +290,43 @@ __global__ __launch_bounds__(64 * NW) void terna_decode_attention_grouped_kernel
         for (int e = 0; e < 8; ++e) acc[e] = __builtin_amdgcn_mfma_f32_4x4x1f32(p, v[e], acc[e], 0, 0, 0);
     };
     const int lslot = wave * RPL + lrow;
-    for (int k = 0; k < batches; ++k) {
-        const bool final = k + 1 == batches;                 // uniform: of the others every row stands in front of the last tile
-        await_all_but(!final);
+    float p[LOADS];
+    u32x4 row[LOADS];
+    auto read_batch = [&](int k, int most) __attribute__((always_inline)) {                // (numerators past local slot `most`: slot 0's)
         const uint8_t* const from = mine + buffer_of(keys + k) + lane * 16;
-        float p[LOADS];
-        u32x4 row[LOADS];
 #pragma unroll
         for (int i = 0; i < LOADS; ++i) {
             const int l = (k * LOADS + i) * STEP + lslot;
             row[i] = *reinterpret_cast<const u32x4*>(from + i * 1024);
-            p[i] = score[(final && l >= nl ? 0 : l) * GQ + (lane & (GQ - 1))];
+            p[i] = score[(l >= most ? 0 : l) * GQ + (lane & (GQ - 1))];
         }
-        if (final) {
-            // slots past the prefix hold anything, also what times 0 is no number; the new token's value row is in LDS
-            const u32x4 vnew = *reinterpret_cast<const u32x4*>(qrows + (GQ + 1) * ROW + piece * 16);
-#pragma unroll
-            for (int i = 0; i < LOADS; ++i) {
-                const int l = (k * LOADS + i) * STEP + lslot, s = cache_slot(l);
-                const bool ok = l < nl && s < n;
-                if (ROPE) row[i] = s == n - 1 ? vnew : row[i];
-                row[i] = ok ? row[i] : u32x4{0u, 0u, 0u, 0u};
-                p[i] = ok ? p[i] : 0.0f;
-            }
-        }
+    };
+    int k = 0;
+    for (; k + 1 < batches; ++k) {                           // every row stands in front of the last tile
+        await_all_but(true);
+        read_batch(k, 1 << 30);
         if (k + 2 < batches) {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             load_values(keys + k + 2, k + 2, n - 1);
         }
 #pragma unroll
         for (int i = 0; i < LOADS; ++i) weigh(p[i], row[i]);
+    }
+    if (k < batches) {
+        await_all_but(false);
+        read_batch(k, nl);
+        // slots past the prefix hold anything, also what times 0 is no number; the new token's value row is in LDS
+        const u32x4 vnew = *reinterpret_cast<const u32x4*>(qrows + (GQ + 1) * ROW + piece * 16);
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) {
+            // (uniform; weighing rows that are not there, with zeros, made launches of 20 - 60 slots 0.3 - 0.4 us longer)
+            if ((k * LOADS + i) * STEP >= nl) break;
+            const int l = (k * LOADS + i) * STEP + lslot, s = cache_slot(l);
+            const bool ok = l < nl && s < n;
+            if (ROPE) row[i] = s == n - 1 ? vnew : row[i];
+            row[i] = ok ? row[i] : u32x4{0u, 0u, 0u, 0u};
+            weigh(ok ? p[i] : 0.0f, row[i]);
+        }
     }
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");            // (a wave without keys: what it requested ahead)
 
@@ -333,15 +342,16 @@ __global__ __launch_bounds__(64 * NW) void terna_decode_attention_grouped_kernel
     for (int idx = tid; idx < GQ * D; idx += NT) {
         const int h = idx / D, d = idx - h * D;
         const uint8_t* const from = smem + (h * D + 4 * sum_at(d >> 2) + (d & 3)) * 4;
-        float o = 0.0f;
+        // (all read ahead of the first addition: a pair at a time as they were added, the launch was 0.1 us longer, 0.2 with the 64 slices of D = 64)
+        float of[STEP], o = 0.0f;
+#pragma unroll
+        for (int slice = 0; slice < STEP; ++slice) of[slice] = *reinterpret_cast<const float*>(from + (slice / RPL) * Shape::kWave + (slice % RPL) * GQ * D * 4);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int grp = 0; grp < STEP / GROUP; ++grp) {
             float part = 0.0f;
 #pragma unroll
-            for (int i = 0; i < GROUP; ++i) {
-                const int slice = grp * GROUP + i;
-                part += *reinterpret_cast<const float*>(from + (slice / RPL) * Shape::kWave + (slice % RPL) * GQ * D * 4);
-            }
+            for (int i = 0; i < GROUP; ++i) part += of[grp * GROUP + i];
             o += part;
         }
         float all = red_s[h];

@@ -925,18 +925,20 @@ def test_quantising_launches_that_fetch_the_next_weights(lib, m, n, k, gate):
         assert torch.equal(xq[0], xq[1]) and torch.equal(s[0], s[1]) and bool(xq[0].any())
 
 
-# The one-workgroup-per-kv-head kernel over the edges of its tiles (16 slots), of its rounds (8 waves: 128 slots of keys and of values; 4 waves:
-# 128 and 128) and of its split counts: splits 0 = ternaspmm_rope_decode_attention, which takes it from 513 heads on.
+# The one-workgroup-per-kv-head kernel over the edges of its tiles (16 slots), of its rounds (of keys, and of values: 128 slots with eight waves, 64 with
+# four; D = 64: 256, 128) and of its split counts: splits 0 = ternaspmm_rope_decode_attention, which takes it from 513 heads on.
 _EDGE_LENS = (1, 16, 17, 127, 128, 129, 256, 257, 300)
+_EDGE_LENS_OF_SPLITS = (1, 639, 640, 641, 1280, 1281, 1400, 1527, 1528)          # about 128, 256 and 300 slots of each of five splits
 
 
 @pytest.mark.parametrize("b,h,kv,d,s_max,splits,adjacent", [
     (9, 20, 5, 128, 300, 3, 1), (9, 8, 4, 128, 301, 5, 0), (9, 16, 4, 64, 300, 6, 0), (9, 8, 4, 64, 304, 7, 1), (30, 20, 5, 128, 300, 2, 1),
-    (27, 20, 5, 128, 300, 0, 1), (60, 20, 5, 128, 300, 0, 0), (35, 16, 8, 128, 303, 0, 1), (36, 16, 4, 64, 300, 0, 1), (72, 8, 4, 64, 300, 0, 0)])
+    (9, 20, 5, 128, 1528, 5, 1), (9, 16, 4, 64, 1528, 2, 0), (27, 20, 5, 128, 300, 0, 1), (60, 20, 5, 128, 300, 0, 0), (35, 16, 8, 128, 303, 0, 1), (36, 16, 4, 64, 300, 0, 1), (72, 8, 4, 64, 300, 0, 0)])
 def test_attention_of_a_kv_group_against_the_oracle(lib, b, h, kv, d, s_max, splits, adjacent):
     """The tolerance: the output is one bf16 rounding (2^-9 of it) away from float32 sums over probabilities whose scores carry the bf16
     products' float32 rounding; 2^-7 of the head's largest output, as for the other attention kernels."""
-    lens = [_EDGE_LENS[i % len(_EDGE_LENS)] for i in range(b)]
+    edges = _EDGE_LENS if s_max < 1528 else _EDGE_LENS_OF_SPLITS
+    lens = [edges[i % len(edges)] for i in range(b)]
     qkv = make_bf16_activations(b, (h + 2 * kv) * d, 1851 + b)
     k0 = make_bf16_activations(b * kv * s_max, d, 1852 + b).reshape(b, kv, s_max, d)
     v0 = make_bf16_activations(b * kv * s_max, d, 1853 + b, outlier_frac=0.01).reshape(b, kv, s_max, d)
@@ -974,6 +976,38 @@ def test_attention_of_a_kv_group_against_the_oracle(lib, b, h, kv, d, s_max, spl
         want = O.attention_one_token(rotate(x[i:i + 1, :h], c, sn), kc[i:i + 1], vc[i:i + 1], lens[i], float(d) ** -0.5)[0]
         tol = 2.0 ** -7 * np.abs(want).max(axis=-1, keepdims=True) + 1e-6
         assert (np.abs(got[i] - want) <= tol).all(), (i, float((np.abs(got[i] - want) / tol).max()))
+
+
+@pytest.mark.parametrize("b,h,kv,d,s_max,adjacent", [(16, 20, 5, 128, 900, 1), (17, 8, 4, 128, 300, 0), (16, 16, 4, 64, 700, 0), (18, 8, 4, 64, 64, 1)])
+def test_attention_of_a_kv_group_with_eight_waves_is_the_per_head_kernel_bit_for_bit(lib, b, h, kv, d, s_max, adjacent):
+    """Up to 256 workgroups run eight waves each, as the unsplit kernel of a single sequence does: one split's merged results are that kernel's
+    outputs, over prefixes of a part of a thread's rows (32 slots apart, 64 for D = 64), of one and of several units, with infinities and NaNs among
+    the values, and whatever stands behind the prefix."""
+    lens = [1, 16, 17, 31, 33, 64, 65, 95, 97, 128, 129, 192, 193, 256, 257, s_max - 1, s_max, 300]
+    lens = [min(n, s_max) for n in lens[:b]]
+    qkv = make_bf16_activations(b, (h + 2 * kv) * d, 1881 + b)
+    k0 = make_bf16_activations(b * kv * s_max, d, 1882 + b).reshape(b, kv, s_max, d)
+    v0 = make_bf16_activations(b * kv * s_max, d, 1883 + b, outlier_frac=0.01).reshape(b, kv, s_max, d)
+    pos = np.array(lens, np.int64) - 1
+    for i, n in enumerate(lens):
+        k0[i, :, n:], v0[i, :, n:] = 0x7FC0, 0x7F80
+    v0[12, 0, 30, 3], v0[13, 1, 5, 9] = 0x7F80, 0x7FC0
+    cos, sin = _angles(pos, d)
+    xd, cd, sd, pd, ck, cv = _dev(qkv), _dev(cos), _dev(sin), _dev(pos), _dev(k0), _dev(v0)
+    part, out = _partial_buffer(lib, b, h, d), torch.zeros((b, h * d), dtype=torch.int16, device="cuda")
+    print(f"[case] kv group of eight waves against one head b={b} h={h} kv={kv} d={d} S={s_max} adjacent={adjacent}", flush=True)
+    assert lib.ternaspmm_step_attention(_vp(xd), _vp(cd), _vp(sd), _vp(pd), 1, _vp(ck), _vp(cv), _vp(part), 1, b, h, kv, d, s_max, float(d) ** -0.5,
+                                        adjacent, None, None, None, 0, None) == 0
+    lib.ternaspmm_attention_merge(_vp(part), 1, _vp(out), b, h, d, None)
+    for i in range(b):
+        ck1, cv1, one = _dev(k0[i:i + 1]), _dev(v0[i:i + 1]), torch.zeros((1, h * d), dtype=torch.int16, device="cuda")
+        x1, c1, s1, p1 = _dev(qkv[i:i + 1]), _dev(cos[i:i + 1]), _dev(sin[i:i + 1]), _dev(pos[i:i + 1])
+        lib.ternaspmm_rope_decode_attention(_vp(x1), _vp(c1), _vp(s1), _vp(p1), 0, _vp(ck1), _vp(cv1), _vp(one), 1, h, kv, d, s_max, float(d) ** -0.5,
+                                            adjacent, None, None)
+        torch.cuda.synchronize()
+        got, want = out[i].view(torch.bfloat16), one[0].view(torch.bfloat16)
+        assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.nan_to_num(got.float()), torch.nan_to_num(want.float())), (i, lens[i])
+        assert torch.equal(ck[i], ck1[0]) and torch.equal(cv[i], cv1[0])
 
 
 @pytest.mark.parametrize("b,h,kv,d,s_max,splits,adjacent", [(60, 20, 5, 128, 420, 1, 1), (33, 20, 5, 128, 1100, 2, 0), (40, 8, 4, 128, 300, 3, 1),
