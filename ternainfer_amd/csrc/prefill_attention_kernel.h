@@ -217,6 +217,7 @@ __global__ __launch_bounds__(64) void terna_prefill_attention_kernel(
 //     most rounds once the maxima have settled).
 // Arithmetic, order of the sums and therefore the bits of the result are those of the one-wave kernel.
 // Workgroups are numbered from the last query block down: under a causal mask those have the most keys to walk.
+typedef short s16x4 __attribute__((ext_vector_type(4)));
 
 // d <- global[sbase + voff .. +15] with no compiler-generated wait: d may be read only after attn_wait_loads<N>() with
 // N = the number of such loads issued after this one, followed by attn_landed(d).

@@ -4,8 +4,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include <cfloat>
 #include <type_traits>
+
+#include "row_quotient.h"
 
 namespace terna {
 
@@ -16,7 +17,6 @@ typedef __attribute__((ext_vector_type(16))) int i32x16;
 typedef __attribute__((ext_vector_type(4))) int i32x4;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
-typedef short s16x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kWave = 64;
 
@@ -394,31 +394,6 @@ __device__ __forceinline__ uint16_t apply_epilogue(int kind, const EpilogueRegs&
     }
     return float_to_bf16_bits(r);
 }
-
-// Quotients of sums by one row's scale, the IEEE ones: an estimate by the scale's reciprocal and one correction by its exact remainder (Markstein) for
-// scales whose products and remainders are normal numbers -- every row's but one of absurd or no finite numbers -- three
-// operations instead of a division's dozen.  (All mantissas of a bf16 scale times all sums up to 2^22 and a sample beyond: the same bits.)
-struct RowQuotient {
-    float s, inverse;
-    bool plain;
-    __device__ explicit RowQuotient(float scale) : s(scale), inverse(__fdiv_rn(1.0f, scale)), plain(scale >= 0x1p-60f && scale <= 0x1p60f) {}
-    template <int F>
-    __device__ void of(float (&x)[F]) const
-    {
-        float q[F];
-#pragma unroll
-        for (int v = 0; v < F; ++v) {
-            q[v] = __fmul_rn(x[v], inverse);
-            q[v] = fmaf(fmaf(-q[v], s, x[v]), inverse, q[v]);
-        }
-        if (!plain) {
-#pragma unroll
-            for (int v = 0; v < F; ++v) q[v] = __fdiv_rn(x[v], s);
-        }
-#pragma unroll
-        for (int v = 0; v < F; ++v) x[v] = q[v];
-    }
-};
 
 // Expansion tables: index = (nonzero nibble << 4) | (next 4 sign bits of the stream).
 // The j-th set bit of the nibble takes sign bit number popcount(nibble below j).
