@@ -963,15 +963,15 @@ def test_deep_tile_kernel_for_every_number_of_steps(lib, act, m, n, k):
 
 
 @pytest.mark.parametrize("m,n,k", [(1, 64, 64), (9, 2560, 2560), (16, 13824, 2560), (17, 704, 320), (33, 192, 4096), (64, 3840, 2560), (65, 2560, 2560),
-                                   (96, 2560, 2304), (250, 256, 1088), (1000, 192, 576), (505, 1024, 2048)])
+                                   (96, 2560, 2304), (250, 256, 1088), (1000, 192, 576), (505, 1024, 2048), (96, 3840, 1024), (100, 960, 576)])
 def test_quantisation_and_linear_in_one_launch(lib, m, n, k):
     """ternaspmm_quant_rows_linear (mid_kernel.h, QUANT) against quant_input and the linear it stands for, bit for bit in every quantisation mode: both of
-    its tiles, one to sixteen waves, partial last chunks and rows, rows of zeros, with an infinity or a NaN; what it does not take (the reference
+    its tiles, one to sixteen waves, one and three weight scales under the rules of up to 64 rows and of more, partial last chunks and rows, rows of zeros, with an infinity or a NaN; what it does not take (the reference
     format without a cached copy, a stream that is being captured) enqueues nothing."""
     from ternainfer_amd import repack_weight
     fmt = DeviceFormat(make_ternary(n, k, 0.40, 6000 + m + n + k))
     packed = repack_weight(fmt.vals, fmt.off, fmt.med, fmt.bm, n, k)
-    groups = 3 if n == 3840 else 1
+    groups = 3 if n in (960, 3840) else 1
     ws = torch.tensor([1.25, 0.75, 1.5], dtype=torch.bfloat16, device="cuda")
     x = torch.from_numpy(make_bf16_activations(m, k, 6100 + m, outlier_frac=0.01).view(np.int16)).cuda().view(torch.bfloat16)
     if m > 4:
