@@ -158,9 +158,9 @@ int64_t ternaspmm_packed_bytes(int N, int K);
 void ternaspmm_repack(const uint64_t* bitmap, const int* tile_offsets_global, const uint16_t* tile_offsets_median,
                       const uint32_t* sign_words, void* packed, int N, int K, terna_stream stream);
 
-/* bf16-activation linear on a P2 buffer.  route: 0 = the library picks the kernel (by measurement: the small-M kernel up
- * to 32 rows for matrices of more than 512 bands, up to 64 - 256 rows otherwise, depending on K, the activation type
- * and whether scratch memory for split-K is at hand), 1 = MFMA-tiled kernel, 2 = small-M kernel. */
+/* bf16-activation linear on a P2 buffer.  route: 0 = the library picks the kernel (by measurement: small-M kernels up to 16 rows,
+ * from there a kernel for a few rows to a few hundred or the MFMA-tiled one, by the tiles of 32 x 64 outputs; where x is not
+ * 16-byte aligned one of the first and the last), 1 = MFMA-tiled kernel, 2 = small-M kernel. */
 void bitlinear_TernaSpMM_bf16_packed(const terna_bf16* x, const void* packed, terna_bf16* out, const float* scale,
                                      int ws_num, int M, int N, int K, int route, terna_stream stream);
 

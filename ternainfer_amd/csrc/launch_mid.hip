@@ -117,12 +117,13 @@ void launch_mid_quant(const uint16_t* x, const uint32_t* packed, uint16_t* out, 
     }
 }
 
-// Up to 16 rows the small-M kernels are faster (3.1 against 3.9 us).  Upwards the MFMA-tiled kernel, whose activations are shared by 128
+// Up to 16 rows the small-M kernels are faster (16 rows, us, small-M / this kernel, int8; bf16: O 2.9 / 3.3; 3.3 / 3.7, QKV 3.1 / 3.3; 3.5 / 3.8, down
+// 4.1 / 4.7; 5.5 / 6.1; wide and shallow matrices are level or the other way round: gate+up 4.7 / 4.5; 5.7 / 5.4).  Upwards the MFMA-tiled kernel, whose activations are shared by 128
 // features, is ahead where the tiles of 32 x 64 are more than two a CU -- counted as they lie on the XCDs, in eights of feature
-// tiles (N = 256 leaves half of the XCDs without one).  Measured, us, MFMA-tiled / this kernel, int8; bf16: QKV M = 250 (480 tiles) 7.7 / 6.8;
-// 10.8 / 9.6, M = 280 (576) 7.7 / 8.1; 10.9 / 12.7; gate+up M = 64 (432) 8.2 / 7.1; 10.7 / 9.8, M = 70 (648) 8.0 / 8.4; 11.8 / 12.8; down M = 350
-// (440) 13.2 / 11.2; 22.2 / 18.3, M = 430 (560) 13.4 / 14.2; 22.3 / 28.2; N = 1024 = K, M = 1000 (512) 5.2 / 4.6; 6.3 / 5.5, M = 1200 (608) 5.3 / 5.4;
-// 6.6 / 7.3; N = 256, M = 1000 (256) 6.9 / 5.0; 11.5 / 9.3, M = 4000 (1000) 7.7 / 13.2; 12.1 / 23.8; N = 704, K = 320, M = 1500 (752) 4.4 / 6.0; 4.6 / 7.5.
+// tiles (N = 256 leaves half of the XCDs without one).  Measured, us, MFMA-tiled / this kernel, int8; bf16: QKV M = 250 (480 tiles) 7.7 / 7.0;
+// 10.9 / 9.7, M = 280 (576) 7.7 / 8.2; 10.9 / 12.0; gate+up M = 64 (432) 8.1 / 7.2; 10.9 / 9.8, M = 70 (648) 7.8 / 8.4; 11.2 / 12.1; down M = 350
+// (440) 13.0 / 11.4; 22.0 / 18.2, M = 430 (560) 13.5 / 14.3; 22.1 / 27.2; N = 1024 = K, M = 1000 (512) 5.2 / 4.7; 6.4 / 5.8, M = 1200 (608) 5.4 / 5.6;
+// 6.6 / 6.9; N = 256, M = 1000 (256) 6.9 / 4.8; 11.3 / 8.2, M = 4000 (1000) 7.6 / 13.8; 11.8 / 24.0; N = 704, K = 320, M = 1500 (752) 4.4 / 5.3; 4.6 / 6.7.
 // Few rows of a wide matrix stay here up to four tiles a CU: a tile of the MFMA-tiled kernel has 64 rows, half of them and more for nothing, and up to 32 rows the
 // small-M kernel takes what this one leaves.  The other kernel / this one: 17 rows, N = 65536 (1024 tiles) K = 1024 9.1 / 7.7; 11.5 / 11.1, K = 4096 20.7 / 15.4; 30.5 / 23.9;
 // 32 rows, N = 40960 K = 4096 15.8 / 12.7; 22.9 / 17.6; 33 - 48 rows, N = 20480 (640) K = 1024 6.4 / 5.0; 7.0 / 6.1, K = 4096 10.5 / 9.2; 15.1 / 14.1, N = 32768 (1024)

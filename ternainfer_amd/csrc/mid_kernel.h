@@ -14,18 +14,19 @@
 //     barrier before the sum; 16-byte piece p of row r sits at p ^ (r & 15), which spreads the operand reads over all banks;
 //   * a weight is expanded once for all RT row tiles, an activation operand read once for all FB bands;
 //   * the waves' partial sums meet in LDS (each wave's in place of its activations, 16-byte units XOR-swizzled by the row)
-//     behind the only barrier, are added in wave order (bit-reproducible; integer sums exact) and leave as whole rows; about 512 threads finish
-//     one to four features each, all waves' sums of them read at once.  In one to two threads per wave and one sum after the other that
+//     behind the only barrier, are added in wave order (bit-reproducible; integer sums exact) and leave as whole rows; every thread finishes
+//     one to four features at a time, all waves' sums of them read at once.  In one to two threads per wave and one sum after the other that
 //     was 2000 - 3500 of a workgroup's 6000 - 12000 clocks, now 850 - 1700: decode step of 32 sequences x 512 slots 1461 -> 1355 us, prompt of
 //     100 tokens 1580 -> 1541.
 // Every load of the main part is issued and awaited by hand (see prefill_packed_kernel.h).
-// Measured, us per launch, weights rotating over 20 copies, ring / MFMA-tiled kernel before -> this kernel (tile choice:
-// launch_mid.hip):             QKV 2560->3840   O 2560->2560   gate+up 2560->13824   down 6912->2560
-//   bf16 M = 37                6.9 -> 5.0       6.8 -> 4.1     16.5 -> 8.6            13.3 -> 6.4
-//   bf16 M = 100               12.1 -> 6.3      11.5 -> 6.1    16.7 -> 14.3           15.3 -> 10.5
-//   int8 M = 37                5.5 -> 4.5       5.4 -> 3.9     11.4 -> 6.8            9.4 -> 5.2
-//   int8 M = 100               7.7 -> 5.3       7.5 -> 5.2     11.4 -> 10.0           12.9 -> 7.8
-//   int8 M = 300               10.9 -> 8.8      11.1 -> 6.7    16.4 (stays)           16.3 -> 11.1
+// Measured, us per launch, weights rotating over 8 copies, the ring / MFMA-tiled kernel that such calls had before -> this kernel (tile choice
+// and what is left to the MFMA-tiled one, "-": launch_mid.hip):
+//                              QKV 2560->3840   O 2560->2560   gate+up 2560->13824   down 6912->2560
+//   bf16 M = 37                6.9 -> 4.8       6.8 -> 3.9     16.5 -> 9.0            13.3 -> 6.2
+//   bf16 M = 100               12.1 -> 6.2      11.5 -> 5.8    -                      15.3 -> 11.0
+//   int8 M = 37                5.5 -> 3.8       5.4 -> 3.3     11.4 -> 6.3            9.4 -> 4.6
+//   int8 M = 100               7.7 -> 4.6       7.5 -> 4.4     -                      12.9 -> 7.2
+//   int8 M = 300               -                11.1 -> 5.7    -                      16.3 -> 11.1
 #pragma once
 
 #include "chain_chunk_kernel.h"

@@ -13,7 +13,8 @@
 //        which of the reference's ways of evaluating these two lines is reproduced: QuantMode in terna_common.h)
 //
 // The row stays in registers between the three passes; HBM sees each input element once and each
-// output element once.  Rows are independent, so the grid is M workgroups of 256 threads (and those of fetch_next_weights).
+// output element once.  Rows are independent, so the grid is M workgroups of 256 threads, or of one for every
+// eight elements (terna_norm_quant_wide_kernel: few rows), and those of fetch_next_weights.
 #pragma once
 
 #include "terna_common.h"
